@@ -877,6 +877,27 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
     }
 }
 
+// Merges attention_partial_kernel's states in slice order, for consumers that take the context as fp16 rows.  grid (query heads, rows).
+template <int HD>
+__global__ __launch_bounds__(HD) void attention_partial_merge_kernel(const float *head_partials, int n_head, uint16_t *ctx_f16) {
+    const size_t row = (size_t)blockIdx.y * n_head + blockIdx.x;
+    const float *ps = head_partials + row * kAttentionHeadSplits * (HD + 4);
+    float pm[kAttentionHeadSplits], pl[kAttentionHeadSplits], pa[kAttentionHeadSplits], M = -INFINITY, L = 0.0f, A = 0.0f;
+#pragma unroll
+    for (int sp = 0; sp < kAttentionHeadSplits; sp++) {
+        pm[sp] = ps[sp * (HD + 4) + HD]; pl[sp] = ps[sp * (HD + 4) + HD + 1]; pa[sp] = ps[sp * (HD + 4) + threadIdx.x];
+    }
+#pragma unroll
+    for (int sp = 0; sp < kAttentionHeadSplits; sp++) M = fmaxf(M, pm[sp]);
+#pragma unroll
+    for (int sp = 0; sp < kAttentionHeadSplits; sp++) {
+        const float f = pm[sp] == -INFINITY ? 0.0f : expf(pm[sp] - M);
+        L = __builtin_fmaf(pl[sp], f, L);
+        A = __builtin_fmaf(pa[sp], f, A);
+    }
+    ctx_f16[row * HD + threadIdx.x] = to_half_bits(L > 0.0f ? A / L : 0.0f);
+}
+
 template <int HD, int G>
 hipError_t launch_attention_gqa(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s) {
     // enough workgroups to spread a long prefix over the chip; fixed per runtime so that a captured
@@ -1352,6 +1373,15 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
             if (group == 2) return launch_attention_gqa<64, 2>(a, rows, kv_f16, s);
             if (group == 4) return launch_attention_gqa<64, 4>(a, rows, kv_f16, s);
         }
+    }
+    // other head groups: the kernel of the single-row step and a merge launch
+    if (a.n_head % a.n_kv_head == 0 && (a.head_dim == 128 || a.head_dim == 64) && a.head_partials && rows <= kMaxStepRows &&
+        a.cache_seq_stride <= 0xFFFFFFFFull && a.n_head <= 0xFFFF) {
+        const hipError_t e = launch_attention_partials(a, rows, kv_f16, s);
+        if (e != hipSuccess) return e;
+        if (a.head_dim == 128) hipLaunchKernelGGL(attention_partial_merge_kernel<128>, dim3(a.n_head, rows), dim3(128), 0, s, a.head_partials, a.n_head, a.ctx_f16);
+        else hipLaunchKernelGGL(attention_partial_merge_kernel<64>, dim3(a.n_head, rows), dim3(64), 0, s, a.head_partials, a.n_head, a.ctx_f16);
+        return hipGetLastError();
     }
     if (a.head_dim > kBlock && a.head_dim % kBlock != 0) return hipErrorInvalidValue;
     if (a.head_dim < kBlock && kBlock % a.head_dim != 0) return hipErrorInvalidValue;

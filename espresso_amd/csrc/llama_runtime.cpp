@@ -1,5 +1,7 @@
 #include "llama_runtime.h"
 
+#include "kernels/span_attention.h"
+
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -355,7 +357,9 @@ int LlamaRuntime::finalize() {
     }
     {
         const char *pa = getenv("ESPRESSO_HIP_PROMPT_ATTENTION");   // "0": prompt blocks keep the single-query attention kernel
-        prompt_attention_ = attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim) && !(pa && pa[0] == '0');
+        const bool block_attention = !(pa && pa[0] == '0');
+        prompt_attention_ = block_attention && attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
+        span_attention_ = block_attention && !prompt_attention_ && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
         const char *fh = getenv("ESPRESSO_HIP_FUSED_HEAD_ARGMAX");   // "0": the head stores logits and separate launches pick the token
         fused_head_argmax_ = !(fh && fh[0] == '0');
         const char *sa = getenv("ESPRESSO_HIP_SPLIT_ACTIVATIONS");   // "0": activations rounded to fp16 once
@@ -491,12 +495,12 @@ int LlamaRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int b
     const int rc = upload_block_rows(seq, tokens, rows, base);
     if (rc != ESP_OK) return rc;
     ESP_HIP_TRY(launch_embed(embedding_, embedding_f16_, d_tokens_, rows, c_.d_model, hidden_, context().stream));
-    return enqueue_layers_matrix(rows, true);
+    return enqueue_layers_matrix(rows, base + rows);
 }
 
 // The layer loop over `rows` rows whose embeddings sit in hidden_ and whose (position, sequence) sit in
 // d_pos_/d_seq_, every projection as one dequant-fused MFMA GEMM.  Rows that are one sequence at consecutive positions
-// (a prompt block) take the matrix-core attention kernel, others the single-query one.
+// (a prompt block) take a matrix-core attention kernel, others the single-query one.
 // Prompt blocks of Q4_K models: every projection with exact weights and split activations (launch_gemm_split), queries and softmax
 // weights split in the attention: the block then stays as close to the fp32 CPU walk as the decode steps do.
 bool LlamaRuntime::split_blocks_supported() const {
@@ -554,8 +558,9 @@ int LlamaRuntime::enqueue_layers_split(int rows) {
     return ESP_OK;
 }
 
-int LlamaRuntime::enqueue_layers_matrix(int rows, bool one_sequence_consecutive) {
-    if (one_sequence_consecutive && split_blocks_supported()) return enqueue_layers_split(rows);
+// block_keys: the keys that the last row of a prompt block sees; 0 for rows that are not one sequence at consecutive positions.
+int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
+    if (block_keys && split_blocks_supported()) return enqueue_layers_split(rows);
     hipStream_t s = context().stream;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const bool kv16 = c_.kv_format == FMT_F16;
@@ -592,8 +597,9 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, bool one_sequence_consecutive)
         AttentionArgs aa{};
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
-        aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_;
-        if (one_sequence_consecutive && prompt_attention_) ESP_HIP_TRY(launch_attention_prompt(aa, rows, kv16, s));
+        aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_; aa.head_partials = attn_scratch_;
+        if (block_keys && prompt_attention_) ESP_HIP_TRY(launch_attention_prompt(aa, rows, kv16, s));
+        else if (block_keys && span_attention_) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, kv16, s));
         else ESP_HIP_TRY(launch_attention(aa, rows, kv16, s));
         g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_;
         { int rc = project_and_norm(L.rms_ffn); if (rc != ESP_OK) return rc; }

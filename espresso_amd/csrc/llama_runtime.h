@@ -91,7 +91,7 @@ class LlamaRuntime : public DecoderRuntime {
     int prefill_block(int seq, const uint32_t *tokens, int rows, int base) override;
     int clear_state() override;
     unsigned tuning_epoch() const override { return gemv_tuning_epoch(); }
-    int enqueue_layers_matrix(int rows, bool one_sequence_consecutive = false);
+    int enqueue_layers_matrix(int rows, int block_keys = 0);
     bool matrix_prefill_supported() const override;
     bool wo_merges_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);
@@ -120,6 +120,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool merged_attention_ = true;
     bool split_activations_ = true;
     bool prompt_attention_ = false;   // prompt blocks run attention on the matrix cores
+    bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for
     float *gemm_workspace_ = nullptr;
     GemmSplitSharedK gemm_shared_k_;   // the device's pool for launch_gemm_split's hand-over between workgroups (not owned)
 };
