@@ -333,13 +333,16 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
+            auto row_of = [&](int r) { return m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); };
+            if (!split && a.residual) {
+                float res[16];   // requested together: y may be the residual's own memory, and a load behind each store is a trip to memory each
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (m < a.M && n < a.N) {
-                    const size_t o = (size_t)m * a.N + n;
-                    out[o] = (!split && a.residual) ? a.residual[o] + acc[i][j][r] : acc[i][j][r];
-                }
+                for (int r = 0; r < 16; r++) res[r] = a.residual[(size_t)(row_of(r) < a.M ? row_of(r) : a.M - 1) * a.N + (n < a.N ? n : a.N - 1)];
+#pragma unroll
+                for (int r = 0; r < 16; r++) if (row_of(r) < a.M && n < a.N) out[(size_t)row_of(r) * a.N + n] = res[r] + acc[i][j][r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; r++) if (row_of(r) < a.M && n < a.N) out[(size_t)row_of(r) * a.N + n] = acc[i][j][r];
             }
         }
 }
