@@ -121,6 +121,9 @@ struct GemmParams {
     float *y = nullptr;               // fp32 out [rows][w.rows]
     const float *residual = nullptr;  // optional [rows][w.rows], may alias y
     int rows = 0;
+    // few rows may take the kernel that keeps every weight exact (rows_gemm.hip) instead of the tile kernels, which round each
+    // dequantised weight to fp16 once: esp_gemv promises those results for its row counts, the runtimes do not
+    bool unrounded = false;
     float *workspace = nullptr;       // split-K partial sums for short row counts (optional)
     size_t workspace_floats = 0;
     // optional fp16 [rows][w.rows / 2]: silu(y[2i]) * y[2i + 1] for a matrix whose rows are (gate, up) pairs; y is then

@@ -24,6 +24,7 @@
 //     adds the partial sums in split order (deterministic, no atomics).
 #include "../common.h"
 #include "decode_ops.h"
+#include "rows_gemm.h"
 #include <atomic>
 #include <type_traits>
 
@@ -854,12 +855,13 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t stream) {
     if (!w.qs || !p.x || !p.y || p.rows <= 0 || w.rows <= 0 || w.cols <= 0 || w.cols % KT != 0 || w.qs_row_bytes % 16 != 0) return hipErrorInvalidValue;
     if ((w.format == FMT_Q8_0 || w.format == FMT_Q4_0) && !w.scales) return hipErrorInvalidValue;
     if (w.format == FMT_Q4_K && w.cols % 256 != 0) return hipErrorInvalidValue;
+    if (p.deferred_splits) *p.deferred_splits = 1;
+    if (rows_gemm_takes(p)) return launch_rows_gemm(p, stream);
     GemmArgs a{};
     a.qs = w.qs; a.scales = w.scales; a.qs_row_bytes = w.qs_row_bytes; a.N = w.rows; a.K = w.cols; a.M = p.rows;
     a.x = p.x; a.y = p.y; a.residual = p.residual;
     bool fused = false;
     hipError_t e;
-    if (p.deferred_splits) *p.deferred_splits = 1;
     switch (w.format) {
     case FMT_Q4_K: e = launch_format<FMT_Q4_K>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;
     case FMT_Q4_0: e = launch_format<FMT_Q4_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;

@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "../common.h"
+#include "rows_gemm.h"
 
 #include <hip/hip_ext.h>
 #include "gemv_device.h"
@@ -2551,6 +2552,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "q4k_mfma_rows8_max") { g_q4k_mfma_rows8_max = value; return true; }
     if (k == "q4k_long_row_waves") { g_q4k_long_row_waves = value; return true; }
     if (k == "q4k_wide") { g_q4k_wide_mode = value; return true; }
+    if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
     if (k == "split_gemm_shared_k") { gemm_split_set_shared_k(value); return true; }
     if (k == "prompt_attention_key_sets") { attention_prompt_set_key_sets(value); return true; }
     return false;

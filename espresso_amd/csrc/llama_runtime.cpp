@@ -566,7 +566,7 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
     const bool kv16 = c_.kv_format == FMT_F16;
     const size_t cache_seq_stride = (size_t)kd * c_.max_seq;
     GemmParams g;
-    g.rows = rows; g.workspace = gemm_workspace_; g.workspace_floats = kGemmWorkspaceFloats;
+    g.rows = rows; g.unrounded = true; g.workspace = gemm_workspace_; g.workspace_floats = kGemmWorkspaceFloats;
     // The RMSNorm that follows a projection with a residual reads that projection's result; when the GEMM ran split-K the
     // norm kernel adds the partial sums itself (one launch instead of reduce + norm).
     const bool fuse_norm = rmsnorm_reduce_supported(d);
@@ -633,7 +633,7 @@ int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits
         // batched rows: final RMSNorm, then the head as one MFMA GEMM
         ESP_HIP_TRY(launch_rmsnorm(hidden_rows, final_norm_, c_.norm_eps, count, c_.d_model, xn_, nullptr, s));
         GemmParams m;
-        m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.workspace = gemm_workspace_; m.workspace_floats = kGemmWorkspaceFloats;
+        m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = kGemmWorkspaceFloats;
         ESP_HIP_TRY(launch_gemm(m, s));
         ESP_HIP_TRY(launch_argmax(logits_, count, c_.vocab, d_out_tokens_, nullptr, argmax_scratch_, s));
         return ESP_OK;
