@@ -104,6 +104,8 @@ struct GemvParams {
     // The products then carry the activations to about 22 bits instead of 11.  split_out: EPI_SWIGLU_F16 writes such row pairs,
     // out_f16 = [2 * batch][rows / 2].
     bool split_x = false, split_out = false;
+    // one launch for up to sixteen rows of fp16 activations given (gemv_takes_sixteen_rows), every epilogue but the arg-max
+    bool sixteen_rows = false;
     // measurement only: device buffer of four wall-clock stamps (100 MHz) per wavefront of the launch, room for stamp_capacity
     // wavefronts (matrix-core Q4_K kernel, fp16 activations given, one or two rows)
     unsigned long long *stamps = nullptr;
@@ -198,6 +200,7 @@ constexpr int kAttentionHeadSplits = ESP_ATTENTION_HEAD_SPLITS;
 bool gemv_set_tuning(const char *key, int value);
 // True when launch_gemv handles `batch` rows without re-reading the weights per pair of rows (always for one or two rows).
 bool gemv_takes_rows(const DeviceMatrix &w, int batch);
+bool gemv_takes_sixteen_rows(const DeviceMatrix &w, int batch);
 // True when launch_gemv has the EPI_ARGMAX epilogue for this matrix (every format; Q4_K rows of 8192 or more columns, which
 // several wavefronts share, keep the separate argmax launches).
 bool gemv_supports_argmax(const DeviceMatrix &w);

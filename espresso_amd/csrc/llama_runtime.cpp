@@ -389,7 +389,7 @@ int LlamaRuntime::enqueue_trunk(int M, bool embedded, float *final_out) {
         if ((rc = time_end()) != ESP_OK) return rc;
     }
     // more than two rows (batched sequences, batched verify): one pass over the weights on the matrix cores
-    if (M > 2 && matrix_prefill_ && matrix_prefill_supported()) return enqueue_layers_matrix(M);
+    if (M > 2 && matrix_prefill_ && matrix_prefill_supported()) return sixteen_rows_supported(M) ? enqueue_layers_sixteen(M) : enqueue_layers_matrix(M);
     for (Layer &L : layers_) {
         // both RMSNorms of the layer run inside the staging of the GEMV that consumes them
         GemvParams g;
@@ -613,6 +613,44 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
     return ESP_OK;
 }
 
+// Up to sixteen rows (a batch of sequences): every projection as one launch with its epilogue (launch_gemv, sixteen_rows).
+bool LlamaRuntime::sixteen_rows_supported(int rows) const {
+    for (const Layer &L : layers_)
+        if (L.q_norm || !gemv_takes_sixteen_rows(L.wqkv, rows) || !gemv_takes_sixteen_rows(L.wo, rows) || !gemv_takes_sixteen_rows(L.w13, rows) || !gemv_takes_sixteen_rows(L.w2, rows))
+            return false;
+    return true;
+}
+
+int LlamaRuntime::enqueue_layers_sixteen(int rows) {
+    hipStream_t s = context().stream;
+    const int d = c_.d_model, kd = c_.kv_dim();
+    const bool kv16 = c_.kv_format == FMT_F16;
+    for (Layer &L : layers_) {
+        GemvParams g;
+        g.batch = rows; g.sixteen_rows = true;
+        ESP_HIP_TRY(launch_rmsnorm(hidden_, L.rms_att, c_.norm_eps, rows, d, xn_, nullptr, s));
+        g.w = L.wqkv; g.x = xn_; g.epilogue = EPI_QKV_ROPE;
+        g.qkv.n_head = c_.n_head; g.qkv.n_kv_head = c_.n_kv_head; g.qkv.head_dim = c_.head_dim; g.qkv.max_seq = c_.max_seq;
+        g.qkv.rope_cos = rope_cos_; g.qkv.rope_sin = rope_sin_; g.qkv.pos = d_pos_; g.qkv.seq = d_seq_;
+        g.qkv.q_out = q_; g.qkv.k_cache = L.k_cache; g.qkv.v_cache = L.v_cache;
+        g.qkv.cache_seq_stride = (size_t)kd * c_.max_seq; g.qkv.kv_f16 = kv16 ? 1 : 0;
+        ESP_HIP_TRY(launch_gemv(g, s));
+        AttentionArgs aa{};
+        aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = (size_t)kd * c_.max_seq;
+        aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
+        aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_; aa.head_partials = attn_scratch_;
+        ESP_HIP_TRY(launch_attention(aa, rows, kv16, s));
+        g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL;
+        ESP_HIP_TRY(launch_gemv(g, s));
+        ESP_HIP_TRY(launch_rmsnorm(hidden_, L.rms_ffn, c_.norm_eps, rows, d, xn_, nullptr, s));
+        g.w = L.w13; g.x = xn_; g.y = nullptr; g.residual = nullptr; g.out_f16 = act_; g.epilogue = EPI_SWIGLU_F16;
+        ESP_HIP_TRY(launch_gemv(g, s));
+        g.w = L.w2; g.x = act_; g.out_f16 = nullptr; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL;
+        ESP_HIP_TRY(launch_gemv(g, s));
+    }
+    return ESP_OK;
+}
+
 int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits) {
     hipStream_t s = context().stream;
     if (count <= 2 && !want_logits && head_fuses_argmax()) {
@@ -632,6 +670,13 @@ int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits
     if (count > 2 && matrix_prefill_ && lm_head_.format != FMT_F32 && lm_head_.cols % 64 == 0) {
         // batched rows: final RMSNorm, then the head as one MFMA GEMM
         ESP_HIP_TRY(launch_rmsnorm(hidden_rows, final_norm_, c_.norm_eps, count, c_.d_model, xn_, nullptr, s));
+        if (gemv_takes_sixteen_rows(lm_head_, count)) {
+            GemvParams g;
+            g.w = lm_head_; g.x = xn_; g.y = logits_; g.batch = count; g.sixteen_rows = true; g.epilogue = EPI_STORE_F32;
+            ESP_HIP_TRY(launch_gemv(g, s));
+            ESP_HIP_TRY(launch_argmax(logits_, count, c_.vocab, d_out_tokens_, nullptr, argmax_scratch_, s));
+            return ESP_OK;
+        }
         GemmParams m;
         m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = kGemmWorkspaceFloats;
         ESP_HIP_TRY(launch_gemm(m, s));

@@ -92,6 +92,8 @@ class LlamaRuntime : public DecoderRuntime {
     int clear_state() override;
     unsigned tuning_epoch() const override { return gemv_tuning_epoch(); }
     int enqueue_layers_matrix(int rows, int block_keys = 0);
+    bool sixteen_rows_supported(int rows) const;
+    int enqueue_layers_sixteen(int rows);
     bool matrix_prefill_supported() const override;
     bool wo_merges_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);

@@ -1,0 +1,42 @@
+"""Steps of a few rows: batches of up to sixteen sequences in one launch per projection."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from test_gpu_full_size import oracle_from_packed
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mods():
+    import espresso_amd.llama as ll
+    import espresso_amd.ops as ops
+    import espresso_amd.synthetic as syn
+    ops.init()
+    return ll, ops, syn
+
+
+# column counts of the sixteen-row kernel: d_model and attention width, hidden size
+@pytest.mark.parametrize("fmt,d,hidden,kv_fp16", [(orc.FMT_Q4_K, 1024, 2048, True), (orc.FMT_Q4_K, 2048, 3072, False), (orc.FMT_Q4_K, 3072, 8192, True),
+                                                  (orc.FMT_Q4_K, 4096, 14336, True), (orc.FMT_Q4_0, 4096, 14336, False)])
+def test_batches_match_oracle(mods, fmt, d, hidden, kv_fp16):
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=1, n_head=d // 128, n_kv_head=d // 512, d_model=d, head_dim=128, hidden_dim=hidden, vocab=520 if fmt != orc.FMT_Q4_K else 512, max_seq=64)
+    g, packed = syn.build_runtime(cfg, fmt, seed=d, keep_packed=True, max_sequences=16, kv_format=orc.FMT_F16 if kv_fp16 else orc.FMT_F32)
+    o = oracle_from_packed(cfg, packed, fmt, 1, kv_fp16, 64)
+    prompts = [np.random.default_rng(s).integers(0, cfg.vocab, 1 + s % 5).astype(np.uint32) for s in range(16)]
+    for n in (3, 8, 9, 16):
+        g.reset()
+        got, _ = ll.generate_batch(g, prompts[:n], 5)
+        for s in (0, n // 2, n - 1):
+            o.reset()
+            o.prefill([int(t) for t in prompts[s]])
+            for t in got[s]:   # a near tie may fall either way: the chosen token's logit is what has to match
+                logits = o.logits()
+                assert logits.max() - logits[t] <= 2e-2, (n, s)
+                o.advance(int(t))
+        # the caches hold what the steps wrote
+        logits = g.append([int(got[n - 1][-1])], want=[0], sequence=n - 1)[0]
+        assert np.abs(logits - o.logits()).max() <= 2e-2
+    g.close()
