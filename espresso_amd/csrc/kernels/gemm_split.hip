@@ -23,6 +23,7 @@
 #include "decode_ops.h"
 #include <atomic>
 #include <mutex>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 #include <utility>
@@ -410,9 +411,19 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_kernel(SplitGemmArgs 
 // MFMAs instead of four: gate|up of a 512-row block 356 -> 324 us (the kernel above: 421 on the same boxes).  The activation tiles
 // rotate through four LDS buffers so that one barrier serves two tiles (318 -> 313 us, old and new alternating on one box).
 __device__ __forceinline__ void store_subblock_sum(uint16_t *sums, size_t row, int cols, int group, float s);
-constexpr int NT2 = 256;
 constexpr int kRegBBufs = 4;   // activation tiles in LDS: with four, one barrier serves two tiles
-constexpr size_t kLdsBytesRegB = 2 * kRegBBufs * kTileHalfs * 2 + 2 * 128 * 16 * 2;
+// Whole forms (RB x CB = 4 x 2, 2 x 4): 128 activation rows x 256 weight rows per workgroup.  Narrow forms (CB 1): the four wavefronts side by
+// side along 128 weight rows, each on all 32 RB activation rows, for short blocks and for matrices too small to give every compute
+// unit a whole tile.
+constexpr int regb_waves_n(int rb, int cb) { return rb * cb == 8 ? 8 / cb : 4; }
+constexpr int regb_tile_m(int rb, int cb) { return 32 * rb * (4 / regb_waves_n(rb, cb)); }
+constexpr int regb_tile_n(int rb, int cb) { return 32 * cb * regb_waves_n(rb, cb); }
+constexpr size_t regb_lds_bytes(int rb, int cb) {
+    const size_t x = 2 * kRegBBufs * (size_t)regb_tile_m(rb, cb) * LDK * 2 + 2 * (size_t)regb_tile_m(rb, cb) * 16 * 2;
+    const size_t act = 2 * (size_t)regb_tile_m(rb, cb) * (regb_tile_n(rb, cb) / 2 + 16) * 2;
+    return x > act ? x : act;
+}
+constexpr size_t kLdsBytesRegB = regb_lds_bytes(4, 2);
 
 // RB x CB = 32-row blocks of activations x 32-row blocks of weights per wavefront (eight in all: 128 accumulator registers).
 //
@@ -433,14 +444,17 @@ constexpr size_t kLdsBytesRegB = 2 * kRegBBufs * kTileHalfs * 2 + 2 * 128 * 16 *
 // hand the totals over, 6.3 us to take them; the launch 295 against 310 us for the plain grid on the same box.
 template <int RB, int CB, bool SK = false>
 __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemmArgs a) {
-    static_assert(RB * CB == 8 && (RB == 2 || RB == 4), "a wavefront owns eight 32 x 32 tiles");
+    static_assert((RB * CB == 8 && (RB == 2 || RB == 4)) || (!SK && CB == 1 && (RB == 1 || RB == 2 || RB == 4)), "whole tiles, or a narrow form");
     __shared__ int sk_flag_seen;
-    constexpr int THREADS = kThreads, XP = 1024 / THREADS;   // sixteen-byte pieces of a plane's tile per thread
-    constexpr int NW = 8 / CB;                               // wavefronts along the weight rows
+    constexpr int THREADS = kThreads;
+    constexpr int NW = regb_waves_n(RB, CB);                 // wavefronts along the weight rows
+    constexpr int MT = regb_tile_m(RB, CB), NT2 = regb_tile_n(RB, CB);
+    constexpr size_t kTileHalfs = (size_t)MT * LDK;
+    constexpr int XP = MT * 8 / THREADS;                     // sixteen-byte pieces of a plane's tile per thread
     extern __shared__ uint4 smem_raw[];
-    _Float16 *xh = reinterpret_cast<_Float16 *>(smem_raw);     // [kRegBBufs][128 * LDK]
-    _Float16 *xl = xh + kRegBBufs * kTileHalfs;                  // [kRegBBufs][128 * LDK]
-    _Float16 *xs = xl + kRegBBufs * kTileHalfs;                        // [2][128][16]   (hi of S_0..S_7, lo of S_0..S_7) of the row
+    _Float16 *xh = reinterpret_cast<_Float16 *>(smem_raw);     // [kRegBBufs][MT * LDK]
+    _Float16 *xl = xh + kRegBBufs * kTileHalfs;                  // [kRegBBufs][MT * LDK]
+    _Float16 *xs = xl + kRegBBufs * kTileHalfs;                        // [2][MT][16]   (hi of S_0..S_7, lo of S_0..S_7) of the row
     const int tiles = a.K / KT, sbs = a.K / 256;
     floatx16 tot[RB][CB], acc[RB][CB];   // acc starts every super-block from the zero C operand of its first MFMAs
     int sk_unit = SK ? (int)blockIdx.x * a.sk_units : 0;
@@ -480,7 +494,8 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         WRaw r;
         const size_t o = (size_t)(tile >> 2) * 2304 + 256 + 256 * (tile & 3) + 8 * kg;
         r.a0 = *reinterpret_cast<const uint2 *>(wrow[0] + o); r.b0 = *reinterpret_cast<const uint2 *>(wrow[0] + o + 1024);
-        r.a1 = *reinterpret_cast<const uint2 *>(wrow[1] + o); r.b1 = *reinterpret_cast<const uint2 *>(wrow[1] + o + 1024);
+        if constexpr (CB > 1) { r.a1 = *reinterpret_cast<const uint2 *>(wrow[1] + o); r.b1 = *reinterpret_cast<const uint2 *>(wrow[1] + o + 1024); }
+        else { r.a1 = r.a0; r.b1 = r.b0; }
         if constexpr (CB > 2) {
             r.a2 = *reinterpret_cast<const uint2 *>(wrow[2] + o); r.b2 = *reinterpret_cast<const uint2 *>(wrow[2] + o + 1024);
             r.a3 = *reinterpret_cast<const uint2 *>(wrow[3] + o); r.b3 = *reinterpret_cast<const uint2 *>(wrow[3] + o + 1024);
@@ -491,7 +506,7 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
     auto fetch_hdr = [&](int sb) __attribute__((always_inline)) {
         Hdrs h;
         const size_t o = (size_t)(sb < sbs ? sb : sbs - 1) * 2304;
-        h.h0 = *reinterpret_cast<const uint4 *>(wrow[0] + o); h.h1 = *reinterpret_cast<const uint4 *>(wrow[1] + o);
+        h.h0 = *reinterpret_cast<const uint4 *>(wrow[0] + o); h.h1 = CB > 1 ? *reinterpret_cast<const uint4 *>(wrow[1] + o) : h.h0;
         if constexpr (CB > 2) { h.h2 = *reinterpret_cast<const uint4 *>(wrow[2] + o); h.h3 = *reinterpret_cast<const uint4 *>(wrow[3] + o); }
         else { h.h2 = h.h3 = h.h0; }
         return h;
@@ -504,34 +519,34 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         const int row = (tid >> 3) + XSTEP * i;
         return (unsigned)(m0 + row < a.M ? m0 + row : a.M - 1) * (unsigned)a.K + x_col;
     };
-    const unsigned xo0 = x_row_offset(0), xo1 = x_row_offset(1), xo2 = x_row_offset(XP > 2 ? 2 : 0), xo3 = x_row_offset(XP > 2 ? 3 : 0);
+    const unsigned xo0 = x_row_offset(0), xo1 = x_row_offset(XP > 1 ? 1 : 0), xo2 = x_row_offset(XP > 2 ? 2 : 0), xo3 = x_row_offset(XP > 2 ? 3 : 0);
     struct XTile { uint4 h0, h1, h2, h3, l0, l1, l2, l3; };
     auto fetch_x = [&](int tile) __attribute__((always_inline)) {
         const unsigned t = (unsigned)tile * KT;
         XTile x;
         x.h0 = *reinterpret_cast<const uint4 *>(a.xh + (xo0 + t)); x.l0 = *reinterpret_cast<const uint4 *>(a.xl + (xo0 + t));
-        x.h1 = *reinterpret_cast<const uint4 *>(a.xh + (xo1 + t)); x.l1 = *reinterpret_cast<const uint4 *>(a.xl + (xo1 + t));
+        if constexpr (XP > 1) { x.h1 = *reinterpret_cast<const uint4 *>(a.xh + (xo1 + t)); x.l1 = *reinterpret_cast<const uint4 *>(a.xl + (xo1 + t)); }
         if constexpr (XP > 2) {
             x.h2 = *reinterpret_cast<const uint4 *>(a.xh + (xo2 + t)); x.l2 = *reinterpret_cast<const uint4 *>(a.xl + (xo2 + t));
             x.h3 = *reinterpret_cast<const uint4 *>(a.xh + (xo3 + t)); x.l3 = *reinterpret_cast<const uint4 *>(a.xl + (xo3 + t));
         }
         return x;
     };
-    const int xs_row = m0 + ((tid & 255) >> 1) < a.M ? m0 + ((tid & 255) >> 1) : a.M - 1;
+    const int xs_row = m0 + (tid >> 1) < a.M ? m0 + (tid >> 1) : a.M - 1;   // two threads per row (those beyond the tile fetch and drop)
     auto fetch_sums = [&](int sb) __attribute__((always_inline)) {
         return reinterpret_cast<const uint4 *>(a.xs + ((size_t)xs_row * sbs + (sb < sbs ? sb : sbs - 1)) * 16)[tid & 1];
     };
     auto store_x = [&](const XTile &x, int buf) __attribute__((always_inline)) {
         const int o = buf * (int)kTileHalfs + (tid >> 3) * LDK + (tid & 7) * 8;
         *reinterpret_cast<uint4 *>(xh + o) = x.h0; *reinterpret_cast<uint4 *>(xl + o) = x.l0;
-        *reinterpret_cast<uint4 *>(xh + o + XSTEP * LDK) = x.h1; *reinterpret_cast<uint4 *>(xl + o + XSTEP * LDK) = x.l1;
+        if constexpr (XP > 1) { *reinterpret_cast<uint4 *>(xh + o + XSTEP * LDK) = x.h1; *reinterpret_cast<uint4 *>(xl + o + XSTEP * LDK) = x.l1; }
         if constexpr (XP > 2) {
             *reinterpret_cast<uint4 *>(xh + o + 64 * LDK) = x.h2; *reinterpret_cast<uint4 *>(xl + o + 64 * LDK) = x.l2;
             *reinterpret_cast<uint4 *>(xh + o + 96 * LDK) = x.h3; *reinterpret_cast<uint4 *>(xl + o + 96 * LDK) = x.l3;
         }
     };
-    auto store_sums = [&](const uint4 &v, int sb) __attribute__((always_inline)) {   // with 512 threads both halves write the same values
-        *reinterpret_cast<uint4 *>(xs + (sb & 1) * 128 * 16 + ((tid & 255) >> 1) * 16 + 8 * (tid & 1)) = v;
+    auto store_sums = [&](const uint4 &v, int sb) __attribute__((always_inline)) {
+        if (2 * MT == THREADS || tid < 2 * MT) *reinterpret_cast<uint4 *>(xs + (sb & 1) * MT * 16 + (tid >> 1) * 16 + 8 * (tid & 1)) = v;
     };
 
     if (!SK || !sk_resume_from) {
@@ -609,7 +624,7 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         if (u == 3) {
             const int sbuf = (t >> 2) & 1;
 #pragma unroll
-            for (int i = 0; i < RB; i++) fs[i] = *reinterpret_cast<const half8 *>(xs + (size_t)sbuf * 128 * 16 + ((wm * RB + i) * 32 + bn) * 16 + 8 * kg);
+            for (int i = 0; i < RB; i++) fs[i] = *reinterpret_cast<const half8 *>(xs + (size_t)sbuf * MT * 16 + ((wm * RB + i) * 32 + bn) * 16 + 8 * kg);
         }
         auto fold = [&](int cb) __attribute__((always_inline)) {
             const float mscale = kg ? kUnscale : 1.0f;
@@ -751,12 +766,12 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
     }
     // accumulator r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of the 32 x 32 tile
     if (a.sw_hi) {
-        // SiLU(gate) * up of the workgroup's 128 x 128 units as the two fp16 planes, through LDS (free now) so that the planes leave
-        // in whole 16-byte pieces of a row: [plane][128 rows][kActLd].  SiLU as g / (1 + exp(-g)) (the form of Sources/CPUOps/SiLU.swift:5-8):
+        // SiLU(gate) * up of the workgroup's units (128 x 128 for a whole tile) as the two fp16 planes, through LDS (free now) so that the planes leave
+        // in whole 16-byte pieces of a row: [plane][MT rows][kActLd].  SiLU as g / (1 + exp(-g)) (the form of Sources/CPUOps/SiLU.swift:5-8):
         // the same function as the 0.5 g (1 + tanh(0.5 g)) of RealModelInferenceEngine.swift:6825-6827 that the single-row kernels keep, a fifth of the instructions (this epilogue measured 10 us per
         // output tile with tanhf and two-byte stores, a fifteenth of the tile's time).
-        constexpr int kActLd = 144;   // halfs per staged row: consecutive rows eight LDS banks apart
-        uint16_t *act_hi = reinterpret_cast<uint16_t *>(smem_raw), *act_lo = act_hi + 128 * kActLd;
+        constexpr int UN = NT2 / 2, RP = UN / 8, kActLd = UN + 16;   // units and pieces of a row; halfs per staged row: consecutive rows eight LDS banks apart
+        uint16_t *act_hi = reinterpret_cast<uint16_t *>(smem_raw), *act_lo = act_hi + MT * kActLd;
         const bool odd = lane & 1;
 #pragma unroll
         for (int i = 0; i < RB; i++)
@@ -783,8 +798,8 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         const int units_n = a.N / 2, unit0 = n0 / 2;
         const bool whole_pieces = units_n % 8 == 0;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int piece = q * THREADS + tid, row = piece >> 4, c8 = (piece & 15) * 8;
+        for (int q = 0; q < MT * RP / THREADS; q++) {
+            const int piece = q * THREADS + tid, row = piece / RP, c8 = (piece % RP) * 8;
             const int m = m0 + row;
             if (m >= a.M || unit0 + c8 >= units_n) continue;
             const size_t o = (size_t)m * units_n + unit0 + c8;
@@ -1017,7 +1032,72 @@ hipError_t gemm_split_shared_k_pool(GemmSplitSharedK *out) {
 }
 void gemm_split_set_shared_k(int mode) { g_shared_k_mode = mode < 0 ? 1 : mode; }
 
+static int regb_shape_setting() {
+    static const int shape = [] { const char *e = getenv("ESPRESSO_HIP_SPLIT_GEMM_SHAPE"); return e ? atoi(e) : 4; }();
+    return shape;
+}
+// Which form of the register-B kernel a launch takes (row blocks of a narrow form, 0 = a whole one), and over how many workgroups K is split.
+//
+// The forms do the same work per weight and activation; they differ in how much of it one workgroup does at a time.  Measured per K tile
+// of 64 (us, launches without split K over 14336 x 4096 pairs): a workgroup alone on its compute unit 0.75 / 0.9 / 1.3 / 1.95 for 32, 64, 128
+// rows x 128 and 128 x 256 (2.35 once more than half of the units have one); several of them on one (three, two, one and one are resident)
+// 0.39 / 0.64 / 1.42 / 2.35 each.  A launch is its longest compute unit's share, a start of about 3 us, and with split K the planes' way to
+// memory and back at about 4 TB/s plus a little.  Where shared K ranges apply, every unit has the same share of whole tiles: those launches keep them.
+// The rule takes the cheapest by that account (us per launch, whole form with splits of at least 1024 columns -> the rule's choice):
+//   8B, gate|up 32 / 64 / 128 / 192 rows 122 / 123 / 126 / 140 -> 48 / 56 / 85 / 127, q|k|v 37 / 38 / 41 / 44 -> 14 / 19 / 25 / 34,
+//   whole layers of 33 / 64 / 128 / 256 / 512 rows 249 / 257 / 270 / 322 / 558 -> 141 / 150 / 196 / 314 / 558
+//   1B, gate|up 64 / 128 / 256 / 512 rows 66 / 66 / 68 / 80 -> 26 / 31 / 48 / 76, whole layers 152 / 171 / 186 / 232 -> 83 / 99 / 135 / 210
+// (whole layers: the whole form with splits of 256 columns and more, which is already faster than the splits of 1024 it had before:
+// 1B 64 / 512 rows 200 / 265)
+struct RegBForm { int narrow, splits; };
+static int g_regb_narrow = -1;   // -1: the rule; 0: never narrow; 1, 2, 4: always that form (tests, measurements)
+void gemm_split_set_narrow(int form) { g_regb_narrow = form == 0 || form == 1 || form == 2 || form == 4 ? form : -1; }
+static RegBForm regb_form(int rows, int n, int k, bool may_split, size_t workspace_floats, bool shares_k) {
+    struct Form { int rb, cb; float alone, shared; };
+    static const Form forms[] = {{1, 1, 0.75f, 0.39f}, {2, 1, 0.9f, 0.64f}, {4, 1, 1.3f, 1.42f}, {4, 2, 1.95f, 2.35f}};
+    const int tiles = k / KT;
+    RegBForm best{0, 1};
+    if (shares_k && g_regb_narrow <= 0) return best;
+    float best_us = INFINITY;
+    for (const Form &f : forms) {
+        const int narrow = f.cb == 1 ? f.rb : 0;
+        if (g_regb_narrow >= 0 && narrow != g_regb_narrow) continue;
+        const int nt = regb_tile_n(f.rb, f.cb), mt = regb_tile_m(f.rb, f.cb);
+        const long blocks = (long)((n + nt - 1) / nt) * ((rows + mt - 1) / mt);
+        for (int splits = 1; splits <= (may_split ? tiles / 4 : 1); splits++) {
+            if (splits > 1 && (size_t)splits * rows * n > workspace_floats) break;
+            const int per = ((tiles + splits - 1) / splits + 3) & ~3;
+            const long groups = blocks * ((tiles + per - 1) / per), on_one = (groups + 255) / 256;
+            float tile_us = on_one > 1 || (!narrow && groups > 128) ? on_one * f.shared : f.alone;
+            if (narrow && tile_us < f.alone + 0.12f * (on_one - 1)) tile_us = f.alone + 0.12f * (on_one - 1);
+            const float us = 3.0f + per * tile_us + (splits > 1 ? 1.0f + (float)splits * rows * n * 8 / 4e6f : 0.0f);
+            if (us < best_us) { best_us = us; best = {narrow, splits}; }
+            if (on_one > 4) break;   // more splits only add planes
+        }
+    }
+    return best;
+}
+
 bool gemm_split_supported(const DeviceMatrix &w) { return w.format == FMT_Q4_K && w.qs && w.cols % 256 == 0 && w.qs_row_bytes % 16 == 0; }
+
+// Shared K ranges for the SiLU(gate) * up launch when the whole form's output tiles do not fill whole rounds of the chip: one workgroup
+// per compute unit, each with the same number of K tiles.  Their number, or 0 where they do not apply.
+static int shared_k_workgroups_for(const GemmSplitParams &p, int tiles) {
+    if (regb_shape_setting() != 4 || shared_k_mode() == 0 || !p.shared_k || !p.shared_k->flags || !p.shared_k->partial) return 0;
+    static std::atomic<int> cus[64];
+    int device = 0, n = 0;
+    if (hipGetDevice(&device) != hipSuccess) return 0;
+    n = cus[device & 63].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+        cus[device & 63].store(n, std::memory_order_relaxed);
+    }
+    const int blocks = ((p.w.rows + regb_tile_n(4, 2) - 1) / regb_tile_n(4, 2)) * ((p.rows + regb_tile_m(4, 2) - 1) / regb_tile_m(4, 2));
+    const long long units = (long long)blocks * tiles;
+    const bool applies = n > 0 && n <= kStreamKMaxWorkgroups && blocks > n && blocks % n != 0 && units % n == 0 && (units / n) % 4 == 0 && units / n >= tiles &&
+                         (size_t)n * 128 * kThreads <= p.shared_k->partial_floats;
+    return applies ? n : 0;
+}
 
 hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     const DeviceMatrix &w = p.w;
@@ -1033,11 +1113,14 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     // restores the kernel that stages them
     static const bool lds_weights = [] { const char *e = getenv("ESPRESSO_HIP_SPLIT_GEMM_LDS_WEIGHTS"); return e && atoi(e) != 0; }();
     const bool regb = w.tiled != nullptr && !lds_weights;
-    const int nt = regb ? NT2 : NT;
-    const int tiles = a.K / KT, blocks = ((a.N + nt - 1) / nt) * ((a.M + MT - 1) / MT);
-    // split K until the grid fills the chip (one workgroup per compute unit is resident), whole super-blocks per split
-    int splits = 1;
-    if (!swiglu && p.workspace) {
+    const int tiles = a.K / KT;
+    RegBForm form{0, 1};
+    if (regb && regb_shape_setting() == 4) form = regb_form(a.M, a.N, a.K, !swiglu && p.workspace, p.workspace_floats, swiglu && shared_k_workgroups_for(p, tiles) > 0);
+    const int nt = !regb ? NT : form.narrow ? regb_tile_n(form.narrow, 1) : regb_tile_n(4, 2), mt = form.narrow ? regb_tile_m(form.narrow, 1) : MT;
+    const int blocks = ((a.N + nt - 1) / nt) * ((a.M + mt - 1) / mt);
+    int splits = form.splits;
+    if (!(regb && regb_shape_setting() == 4) && !swiglu && p.workspace) {
+        // the other kernels: split K until the grid fills the chip (one workgroup per compute unit is resident), whole super-blocks per split
         const int target = 256;
         splits = blocks >= target ? 1 : (target + blocks - 1) / blocks;
         if (splits > tiles / 16) splits = tiles / 16;
@@ -1052,27 +1135,12 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (device & 63);
-    static const int regb_shape = [] { const char *e = getenv("ESPRESSO_HIP_SPLIT_GEMM_SHAPE"); return e ? atoi(e) : 4; }();
-    // Shared K ranges for the SiLU(gate) * up launch when its output tiles do not fill whole rounds of the chip: one workgroup
-    // per compute unit, each with the same number of K tiles.
-    const int shared_k = shared_k_mode();
-    int shared_k_workgroups = 0;
-    if (swiglu && regb && regb_shape == 4 && shared_k != 0 && p.shared_k && p.shared_k->flags && p.shared_k->partial) {
-        static std::atomic<int> cus[64];
-        int n = cus[device & 63].load(std::memory_order_relaxed);
-        if (n == 0) {
-            e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device);
-            if (e != hipSuccess) return e;
-            cus[device & 63].store(n, std::memory_order_relaxed);
-        }
-        const long long units = (long long)blocks * tiles;
-        if (n > 0 && n <= kStreamKMaxWorkgroups && blocks > n && blocks % n != 0 && units % n == 0 && (units / n) % 4 == 0 && units / n >= tiles &&
-            (size_t)n * 128 * kThreads <= p.shared_k->partial_floats) {
-            shared_k_workgroups = n;
-            a.sk_units = (int)(units / n); a.sk_tiles_n = (a.N + nt - 1) / nt;
-            a.sk_flags = p.shared_k->flags; a.sk_partial = p.shared_k->partial;
-            a.sk_spin_limit = shared_k == 2 ? 0u : kStreamKSpinLimit;
-        }
+    const int regb_shape = regb_shape_setting();
+    const int shared_k_workgroups = swiglu && regb && !form.narrow ? shared_k_workgroups_for(p, tiles) : 0;
+    if (shared_k_workgroups) {
+        a.sk_units = (int)((long long)blocks * tiles / shared_k_workgroups); a.sk_tiles_n = (a.N + nt - 1) / nt;
+        a.sk_flags = p.shared_k->flags; a.sk_partial = p.shared_k->partial;
+        a.sk_spin_limit = shared_k_mode() == 2 ? 0u : kStreamKSpinLimit;
     }
     if (!(raised.load(std::memory_order_acquire) & bit)) {
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_split_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
@@ -1082,11 +1150,18 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_split_regb_kernel<4, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytesRegB);
         if (e == hipSuccess)
             e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_split_regb_kernel<4, 2, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytesRegB);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_split_regb_kernel<2, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)regb_lds_bytes(2, 1));
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q4k_split_regb_kernel<4, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)regb_lds_bytes(4, 1));
         if (e != hipSuccess) return e;
         raised.fetch_or(bit, std::memory_order_release);
     }
-    dim3 grid((a.N + nt - 1) / nt, splits, (a.M + MT - 1) / MT);
+    dim3 grid((a.N + nt - 1) / nt, splits, (a.M + mt - 1) / mt);
     if (shared_k_workgroups) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<4, 2, true>), dim3(shared_k_workgroups), dim3(kThreads), kLdsBytesRegB, stream, a);
+    else if (form.narrow == 1) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<1, 1>), grid, dim3(kThreads), regb_lds_bytes(1, 1), stream, a);
+    else if (form.narrow == 2) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<2, 1>), grid, dim3(kThreads), regb_lds_bytes(2, 1), stream, a);
+    else if (form.narrow == 4) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<4, 1>), grid, dim3(kThreads), regb_lds_bytes(4, 1), stream, a);
     else if (regb && regb_shape == 4) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<4, 2>), grid, dim3(kThreads), kLdsBytesRegB, stream, a);
     else if (regb) hipLaunchKernelGGL((gemm_q4k_split_regb_kernel<2, 4>), grid, dim3(kThreads), kLdsBytesRegB, stream, a);
     else hipLaunchKernelGGL(gemm_q4k_split_kernel<2>, grid, dim3(kThreads), kLdsBytes, stream, a);

@@ -1,7 +1,9 @@
-"""Steps of a few rows: batches of up to sixteen sequences in one launch per projection."""
+"""Steps and blocks of a few rows: the narrow forms of the exact Q4_K GEMM and batches of up to
+sixteen sequences in one launch per projection."""
 import numpy as np
 import pytest
 
+import espresso_amd._lib as lib
 from oracle import oracle as orc
 from test_gpu_full_size import oracle_from_packed
 
@@ -15,6 +17,31 @@ def mods():
     import espresso_amd.synthetic as syn
     ops.init()
     return ll, ops, syn
+
+
+@pytest.mark.parametrize("form", [1, 2, 4])
+@pytest.mark.parametrize("rows,cols", [(130, 1024), (384, 2048), (40, 3072)])
+def test_narrow_split_gemm_matches_float64(mods, form, rows, cols):
+    _, ops, _ = mods
+    m = ops.Matrix(lib.FORMAT_Q4_K, ops.synth_weights(lib.FORMAT_Q4_K, rows, 0.02, rows * cols), rows, cols)
+    w = m.dequantize().astype(np.float64)
+    try:
+        ops.set_tuning("split_gemm_narrow", form)
+        for n in (3, 31, 32, 33, 64, 65, 129):
+            x = np.random.default_rng(n).normal(0, 1, (n, cols)).astype(np.float32)
+            res = np.random.default_rng(n + 1).normal(0, 1, (n, rows)).astype(np.float32)
+            want = x.astype(np.float64) @ w.T + res
+            # the bound test_gpu_split_gemm.py holds the whole form to: the split leaves 2^-22 per activation, the sums are fp32
+            assert np.abs(m.matmul_f32(x, res) - want).max() <= 4e-6 * (want - res).std() + 1e-6, n
+            if rows % 8:
+                continue
+            g = x.astype(np.float64) @ w.T
+            gate, up = g[:, 0::2], g[:, 1::2]
+            act = gate / (1 + np.exp(-gate)) * up
+            assert (np.abs(m.matmul_f32_swiglu(x) - act) <= 5e-6 * g.std() * (np.abs(up) + np.abs(gate) + 1.0)).all(), n
+    finally:
+        ops.set_tuning("split_gemm_narrow", -1)
+    m.close()
 
 
 # column counts of the sixteen-row kernel: d_model and attention width, hidden size
