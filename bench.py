@@ -545,7 +545,7 @@ def main() -> None:
                             "again after a reset; fp16_operands: the same with esp_llama_set_split_activations(0), every operand rounded to fp16 once",
                     "path": ("blocks of up to 512 rows; Q4_K: MFMA GEMM with exact integer weights and activations as hi/lo fp16 pairs (twice the "
                              "MFMA work of the fp16-operand GEMM, logits within 2e-2 of the fp32 CPU walk at 32 layers); other formats: "
-                             "dequant-fused fp16 MFMA GEMM") if w["prompt"] >= 32 else "Q4_K: exact blocks from four tokens on; other formats: single steps"},
+                             "dequant-fused fp16 MFMA GEMM") if w["prompt"] >= 32 else "Q4_K: exact blocks from four tokens on; other formats: two tokens per step"},
     }
     if not args.no_cpu_baseline:
         result["cpu_baseline"] = cpu_baseline(args.workload, gpu)

@@ -1,5 +1,5 @@
-"""Steps and blocks of a few rows: the narrow forms of the exact Q4_K GEMM and batches of up to
-sixteen sequences in one launch per projection."""
+"""Steps and blocks of a few rows: the narrow forms of the exact Q4_K GEMM, batches of up to sixteen sequences in one launch per
+projection, and short prompts two tokens per step."""
 import numpy as np
 import pytest
 
@@ -66,4 +66,27 @@ def test_batches_match_oracle(mods, fmt, d, hidden, kv_fp16):
         # the caches hold what the steps wrote
         logits = g.append([int(got[n - 1][-1])], want=[0], sequence=n - 1)[0]
         assert np.abs(logits - o.logits()).max() <= 2e-2
+    g.close()
+
+
+@pytest.mark.parametrize("fmt,d,hidden", [("q8_0", 256, 512), ("f16", 576, 1536), ("q4_0", 768, 2048), ("q4_k", 1024, 3072)])
+def test_short_prompts_in_pairs_match_single_steps(mods, fmt, d, hidden):
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=d // 64, n_kv_head=d // 64, d_model=d, head_dim=64, hidden_dim=hidden, vocab=512, max_seq=64)
+    g, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=5, std=0.05)   # fp32 caches: no block form takes prompts this short
+    tokens = np.random.default_rng(d).integers(0, cfg.vocab, 12)
+    want = []
+    for t in tokens:
+        g.advance(int(t))
+        want.append(g.logits())
+    want = np.array(want)
+    for portions in ([12], [2, 3, 7], [1, 11], [5, 2, 2, 3]):
+        g.reset()
+        got = []
+        for n in portions:
+            at = g.visible()
+            got.append(g.append(tokens[at:at + n], want=range(n)))
+        # one and two rows take the same products in another order of their fp32 sums; activations are rounded to fp16 in between
+        assert np.abs(np.concatenate(got) - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max()), portions
+        assert np.abs(g.logits() - want[-1]).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max())
     g.close()
