@@ -75,13 +75,13 @@ __device__ __forceinline__ void byte_dword(u32 w, h2 x02, h2 x13, float &d) {
 template <int FMT>
 struct Traits;
 template <>
-struct Traits<FMT_Q4_0> { static constexpr int kItemElems = 32; static constexpr bool kPermuteX = true; static constexpr bool kXSums = false; };
+struct Traits<FMT_Q4_0> { static constexpr int kItemElems = 32; static constexpr bool kPermuteX = true; };
 template <>
-struct Traits<FMT_Q8_0> { static constexpr int kItemElems = 16; static constexpr bool kPermuteX = true; static constexpr bool kXSums = false; };
+struct Traits<FMT_Q8_0> { static constexpr int kItemElems = 16; static constexpr bool kPermuteX = true; };
 template <>
-struct Traits<FMT_F32> { static constexpr int kItemElems = 4; static constexpr bool kPermuteX = false; static constexpr bool kXSums = false; };
+struct Traits<FMT_F32> { static constexpr int kItemElems = 4; static constexpr bool kPermuteX = false; };
 template <>
-struct Traits<FMT_F16> { static constexpr int kItemElems = 8; static constexpr bool kPermuteX = false; static constexpr bool kXSums = false; };
+struct Traits<FMT_F16> { static constexpr int kItemElems = 8; static constexpr bool kPermuteX = false; };
 
 struct KernelArgs {
     QkvEpilogue qkv;
@@ -212,9 +212,51 @@ __device__ __forceinline__ uint4 activation_group(const KernelArgs &a, int b, in
     return normalized_group(x4[2 * g], x4[2 * g + 1], w4[2 * g], w4[2 * g + 1], inv);
 }
 
-// What a wavefront does with the two row sums (rows 2p and 2p+1) of each batch column.
+// What a lane's epilogue reads, requested before the arithmetic (EarlyEpilogue): the two residual values, or the position and then its
+// RoPE factors, are a memory round trip (two, for RoPE) that nothing hides where a wavefront has one round of rows and a compute unit one or
+// two workgroups.
 template <int B>
-__device__ __forceinline__ void pair_epilogue(const KernelArgs &a, int pair, const float va[B], const float vb[B]) {
+struct EarlyEpilogue {
+    float r0[B], r1[B];   // residual values, or RoPE cosine and sine, of the pair in each batch row
+    int pos[B], seq[B];
+};
+// First half: the position and sequence of each row, before anything else is requested.
+template <int B>
+__device__ __forceinline__ void early_positions(const KernelArgs &a, EarlyEpilogue<B> &e) {
+    if (a.epilogue != EPI_QKV_ROPE) return;
+    unsigned o = 0;
+    asm volatile("" : "+v"(o));   // a vector load: scalar loads are waited for with the first LDS access
+#pragma unroll
+    for (int b = 0; b < B; b++) { e.pos[b] = a.qkv.pos[b + o]; e.seq[b] = a.qkv.seq[b + o]; }
+}
+// Second half, after the staging (the positions have arrived by then).
+template <int B>
+__device__ __forceinline__ void early_operands(const KernelArgs &a, int pair, EarlyEpilogue<B> &e) {
+    unsigned o = 0;
+    asm volatile("" : "+v"(o));
+    if (a.epilogue == EPI_QKV_ROPE) {
+        const QkvEpilogue &q = a.qkv;
+        const int half = q.head_dim / 2, ad = q.n_head * q.head_dim, kd = q.n_kv_head * q.head_dim;
+        if (2 * pair >= ad + kd) return;
+        const int pr = 2 * pair < ad ? pair : pair - ad / 2, j = pr % half;
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            e.r0[b] = q.rope_cos[(size_t)e.pos[b] * half + j + o];
+            e.r1[b] = q.rope_sin[(size_t)e.pos[b] * half + j + o];
+        }
+    } else if (a.epilogue == EPI_ADD_RESIDUAL) {
+        const int r0 = 2 * pair < a.rows ? 2 * pair : a.rows - 1, r1 = 2 * pair + 1 < a.rows ? 2 * pair + 1 : a.rows - 1;
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            e.r0[b] = a.residual[(size_t)b * a.rows + r0 + o];
+            e.r1[b] = a.residual[(size_t)b * a.rows + r1 + o];
+        }
+    }
+}
+
+// What a wavefront does with the two row sums (rows 2p and 2p+1) of each batch column.  EARLY: `e` holds what the epilogue reads.
+template <int B, bool EARLY = false>
+__device__ __forceinline__ void pair_epilogue(const KernelArgs &a, int pair, const float va[B], const float vb[B], const EarlyEpilogue<B> *e = nullptr) {
     const int r0 = 2 * pair, r1 = 2 * pair + 1;
     if (a.epilogue == EPI_SWIGLU_F16) {
         // rows are (gate_i, up_i): act_i = silu_tanh(gate) * up, rounded to fp16 for the next GEMV
@@ -246,13 +288,13 @@ __device__ __forceinline__ void pair_epilogue(const KernelArgs &a, int pair, con
         if (r1 >= a.rows) return;
 #pragma unroll
         for (int b = 0; b < B; b++) {
-            const int pos = q.pos[b];
-            const size_t seq_base = (size_t)q.seq[b] * q.cache_seq_stride;
+            const int pos = EARLY ? e->pos[b] : q.pos[b];
+            const size_t seq_base = (size_t)(EARLY ? e->seq[b] : q.seq[b]) * q.cache_seq_stride;
             if (r0 < ad + kd) {
                 const bool is_q = r0 < ad;
                 const int pr = is_q ? pair : pair - ad / 2;
                 const int h = pr / half, j = pr - h * half;
-                const float c = q.rope_cos[(size_t)pos * half + j], sn = q.rope_sin[(size_t)pos * half + j];
+                const float c = EARLY ? e->r0[b] : q.rope_cos[(size_t)pos * half + j], sn = EARLY ? e->r1[b] : q.rope_sin[(size_t)pos * half + j];
                 const float o0 = __fsub_rn(__fmul_rn(va[b], c), __fmul_rn(vb[b], sn));
                 const float o1 = __fadd_rn(__fmul_rn(va[b], sn), __fmul_rn(vb[b], c));
                 if (is_q) {
@@ -290,11 +332,11 @@ __device__ __forceinline__ void pair_epilogue(const KernelArgs &a, int pair, con
     for (int b = 0; b < B; b++) {
         if (r0 < a.rows) {
             const size_t o = (size_t)b * a.rows + r0;
-            a.y[o] = a.epilogue == EPI_ADD_RESIDUAL ? a.residual[o] + va[b] : va[b];
+            a.y[o] = a.epilogue == EPI_ADD_RESIDUAL ? (EARLY ? e->r0[b] : a.residual[o]) + va[b] : va[b];
         }
         if (r1 < a.rows) {
             const size_t o = (size_t)b * a.rows + r1;
-            a.y[o] = a.epilogue == EPI_ADD_RESIDUAL ? a.residual[o] + vb[b] : vb[b];
+            a.y[o] = a.epilogue == EPI_ADD_RESIDUAL ? (EARLY ? e->r1[b] : a.residual[o]) + vb[b] : vb[b];
         }
     }
 }
@@ -324,18 +366,56 @@ inline const void *leading_activations(const KernelArgs &a) {
 }
 inline int leading_mode(const KernelArgs &a) { return a.merge_partials ? (2 | (a.merge_head_dim << 8)) : a.norm_x ? 1 : 0; }
 
-template <int FMT, int B, int R>
+// Dot products, any column count.  Bound by its chain of memory round trips, not by bytes (576 x 576 fp16: 0.7 MB in 5 us), so everything whose
+// address is known is requested at once: the first DEPTH (x 64) items of the wavefront's R rows, the values and norm weights of up to
+// two groups per thread, what the epilogue reads.  MODE as in with_leading_args.  Measured against one item ahead, activations read twice
+// and the epilogue's operands read at the end (us per launch of a decode step): 576 columns fp16 q|k|v 5.1 -> 4.0, wo 5.2 -> 3.4, gate|up
+// 5.3 -> 4.1, down 5.2 -> 3.1; the smol model's prompt and 24 steps 15.5 -> 14.66 ms, 32 steps of the 1B model with Q4_0 weights 18.27 -> 17.59 ms.
+template <int FMT, int B, int R, int MODE, int DEPTH>
 __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const uint16_t *scales, const void *activations, const float *norm_w, int rows,
                                                         int cols_arg, int row_bytes, int mode, float norm_eps, KernelArgs rest) {
-    const KernelArgs a = with_leading_args(rest, qs, scales, activations, norm_w, rows, cols_arg, row_bytes, mode, norm_eps);
+    const KernelArgs a = with_leading_args(rest, qs, scales, activations, norm_w, rows, cols_arg, row_bytes, (mode & ~0xFF) | MODE, norm_eps);
     using T = Traits<FMT>;
     extern __shared__ uint4 smem_raw[];
     uint16_t *xs = reinterpret_cast<uint16_t *>(smem_raw);                 // [B][cols] fp16
-    float *xsum = reinterpret_cast<float *>(xs + (size_t)B * a.cols);      // [B][cols/16] (Q4_K)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cols = a.cols;
 
-    // ---- the wavefront's rows and the first 128 bits of weights per lane: in flight while the activations are staged ----
+    // ---- positions and activations: requested first (memory returns in order) ----
+    EarlyEpilogue<B> early;
+    if constexpr (R == 2) early_positions<B>(a, early);
+    constexpr int KS = 2;                                                  // groups of eight per thread in registers (MODE 0 and 1)
+    const int per_row = cols / 8;
+    float4 nv0[MODE == 1 ? B : 1][KS], nv1[MODE == 1 ? B : 1][KS], ng0[KS], ng1[KS];
+    uint4 xv0[MODE == 0 ? B : 1][KS];
+    if constexpr (MODE != 2) {
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            const int g = tid + k * kThreads < per_row ? tid + k * kThreads : per_row - 1;
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                if constexpr (MODE == 1) {
+                    const float4 *x4 = reinterpret_cast<const float4 *>(a.norm_x + (size_t)b * cols);
+                    nv0[b][k] = x4[2 * g]; nv1[b][k] = x4[2 * g + 1];
+                } else {
+                    xv0[b][k] = reinterpret_cast<const uint4 *>(a.x)[(size_t)b * per_row + g];
+                }
+            }
+            if constexpr (MODE == 1) {
+                const float4 *w4 = reinterpret_cast<const float4 *>(a.norm_w);
+                ng0[k] = w4[2 * g]; ng1[k] = w4[2 * g + 1];
+            }
+        }
+    }
+
+    float2 mml[B][kMergeSplits];
+    float4 mm0[B][kMergeSplits], mm1[B][kMergeSplits];
+    if constexpr (MODE == 2) {
+#pragma unroll
+        for (int b = 0; b < B; b++) merge_group_load(a, b, tid < per_row ? tid : per_row - 1, cols, mml[b], mm0[b], mm1[b]);
+    }
+
+    // ---- the wavefront's rows ----
     const int row0 = (blockIdx.x * kWaves + wave) * R;
     const int items = cols / T::kItemElems;
     const uint8_t *rowp[R];
@@ -348,6 +428,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     }
     struct Item { uint4 q[R]; uint16_t d[R]; };
     auto load_item = [&](int item) {
+        if (item >= items) item = items - 1;
         Item it;
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -358,36 +439,58 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
         }
         return it;
     };
-    Item cur = load_item(lane < items ? lane : items - 1);
+    Item ring[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) ring[d] = load_item(lane + 64 * d);
 
     // ---- stage activations: 128-bit loads (or the fused RMSNorm), middle elements of each group of
     // four swapped for the integer formats ----
     {
         __shared__ float norm_red[B * kWaves];
         uint4 *dst = reinterpret_cast<uint4 *>(xs);
-        const int per_row = cols / 8;
+        auto put = [&](int b, int g, const uint4 &v) { dst[(size_t)b * per_row + g] = T::kPermuteX ? swap_middle(v) : v; };
 #pragma unroll
         for (int b = 0; b < B; b++) {
-            const float inv = a.norm_x ? row_inverse_rms(a, b, cols, norm_red + b * kWaves) : 0.0f;
-            for (int g = tid; g < per_row; g += kThreads) {
-                const uint4 v = activation_group(a, b, g, cols, inv);
-                dst[(size_t)b * per_row + g] = T::kPermuteX ? swap_middle(v) : v;
+            float inv = 0.0f;
+            if constexpr (MODE == 1) {
+                float s = 0.0f;
+#pragma unroll
+                for (int k = 0; k < KS; k++)
+                    if (tid + k * kThreads < per_row) s += sum_squares(nv0[b][k], nv1[b][k]);
+                const float4 *x4 = reinterpret_cast<const float4 *>(a.norm_x + (size_t)b * cols);
+                for (int g = tid + KS * kThreads; g < per_row; g += kThreads) s += sum_squares(x4[2 * g], x4[2 * g + 1]);
+                inv = 1.0f / sqrtf(workgroup_sum(s, norm_red + b * kWaves) / (float)cols + a.norm_eps);
+            }
+            if constexpr (MODE != 2) {
+#pragma unroll
+                for (int k = 0; k < KS; k++)
+                    if (tid + k * kThreads < per_row) {
+                        if constexpr (MODE == 1) put(b, tid + k * kThreads, normalized_group(nv0[b][k], nv1[b][k], ng0[k], ng1[k], inv));
+                        else put(b, tid + k * kThreads, xv0[b][k]);
+                    }
+            }
+            if constexpr (MODE == 0) {
+                // the others four per thread at a time
+                const uint4 *xr = reinterpret_cast<const uint4 *>(a.x) + (size_t)b * per_row;
+                for (int g0 = KS * kThreads + tid; g0 < per_row; g0 += 4 * kThreads) {
+                    uint4 t[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) t[k] = xr[g0 + k * kThreads < per_row ? g0 + k * kThreads : per_row - 1];
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        if (g0 + k * kThreads < per_row) put(b, g0 + k * kThreads, t[k]);
+                }
+            } else {
+                if constexpr (MODE == 2) {
+                    if (tid < per_row) put(b, tid, merge_group(mml[b], mm0[b], mm1[b]));
+                }
+                for (int g = tid + (MODE == 1 ? KS : 1) * kThreads; g < per_row; g += kThreads) put(b, g, activation_group(a, b, g, cols, inv));
             }
         }
     }
     __syncthreads();
-    if (T::kXSums) {
-        const int groups = B * cols / 16;
-        for (int g = tid; g < groups; g += kThreads) {
-            const h2 *p = reinterpret_cast<const h2 *>(xs + (size_t)g * 16);
-            float s = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; i++) s += (float)p[i].x + (float)p[i].y;
-            xsum[g] = s;
-        }
-        __syncthreads();
-    }
 
+    if constexpr (R == 2) early_operands<B>(a, row0 / 2, early);
     if (row0 >= a.rows && a.epilogue != EPI_ARGMAX) return;   // (the arg-max epilogue ends with a workgroup barrier)
 
     float acc[R][B];
@@ -396,9 +499,14 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
 #pragma unroll
         for (int b = 0; b < B; b++) acc[r][b] = 0.0f;
 
-    for (int item = lane; item < items; item += 64) {
-        Item nxt = cur;
-        if (item + 64 < items) nxt = load_item(item + 64);   // one step ahead of the arithmetic
+    for (int base = 0; base < items; base += 64 * DEPTH) {
+        const bool more = base + 64 * DEPTH < items;
+#pragma unroll
+        for (int slot = 0; slot < DEPTH; slot++) {
+        const int item = base + 64 * slot + lane;
+        const Item cur = ring[slot];
+        if (more) ring[slot] = load_item(item + 64 * DEPTH);
+        if (item >= items) continue;
         if constexpr (FMT == FMT_Q4_0) {
             const int e_lo = item * 32;
             uint4 xl[B][2], xh[B][2];
@@ -487,7 +595,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
                 }
             }
         }
-        cur = nxt;
+        }
     }
 
 #pragma unroll
@@ -519,7 +627,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
             float va[B], vb[B];
 #pragma unroll
             for (int b = 0; b < B; b++) { va[b] = acc[2 * p][b]; vb[b] = acc[2 * p + 1][b]; }
-            pair_epilogue<B>(a, row0 / 2 + p, va, vb);
+            pair_epilogue<B, R == 2>(a, row0 / 2 + p, va, vb, &early);
         }
     }
 }
@@ -2413,12 +2521,11 @@ hipError_t launch_q4k(const KernelArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <int FMT, int B, int R>
+template <int FMT, int B, int R, int MODE, int DEPTH>
 hipError_t launch_one(const KernelArgs &a, hipStream_t stream) {
-    using T = Traits<FMT>;
-    size_t lds = (size_t)B * a.cols * 2 + (T::kXSums ? (size_t)B * (a.cols / 16) * 4 : 0);
+    const size_t lds = (size_t)B * a.cols * 2;
     if (lds > 160 * 1024) return hipErrorInvalidValue;
-    auto kernel = gemv_kernel<FMT, B, R>;
+    auto kernel = gemv_kernel<FMT, B, R, MODE, DEPTH>;
     static size_t configured_lds = 0;  // per instantiation
     if (lds > 48 * 1024 && lds > configured_lds) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -2433,15 +2540,28 @@ hipError_t launch_one(const KernelArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// DEPTH: one, two rounds of 64 items in flight cover the row, four the longer rows.
+template <int FMT, int B, int R>
+hipError_t launch_mode(const KernelArgs &a, hipStream_t stream) {
+    const int mode = leading_mode(a) & 0xFF;
+    if constexpr (R == 2) {
+        if (a.cols / Traits<FMT>::kItemElems <= 64)
+            return mode == 1 ? launch_one<FMT, B, R, 1, 1>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 1>(a, stream) : launch_one<FMT, B, R, 0, 1>(a, stream);
+        if (a.cols / Traits<FMT>::kItemElems > 128)
+            return mode == 1 ? launch_one<FMT, B, R, 1, 4>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 4>(a, stream) : launch_one<FMT, B, R, 0, 4>(a, stream);
+    }
+    return mode == 1 ? launch_one<FMT, B, R, 1, 2>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 2>(a, stream) : launch_one<FMT, B, R, 0, 2>(a, stream);
+}
+
 template <int FMT>
 hipError_t launch_fmt(const KernelArgs &a, int batch, hipStream_t stream) {
     if (batch == 1) {
         // tall matrices (an output head): four rows per wavefront, so that one wave of workgroups covers the matrix (32000 x 768 Q8_0:
         // 2000 workgroups instead of 4000, 8.8 against 10.1 us; eight rows measure the same as four)
-        if (a.rows >= 16384) return launch_one<FMT, 1, 4>(a, stream);
-        return launch_one<FMT, 1, 2>(a, stream);
+        if (a.rows >= 16384) return launch_mode<FMT, 1, 4>(a, stream);
+        return launch_mode<FMT, 1, 2>(a, stream);
     }
-    if (batch == 2) return a.rows >= 16384 ? launch_one<FMT, 2, 4>(a, stream) : launch_one<FMT, 2, 2>(a, stream);
+    if (batch == 2) return a.rows >= 16384 ? launch_mode<FMT, 2, 4>(a, stream) : launch_mode<FMT, 2, 2>(a, stream);
     return hipErrorInvalidValue;
 }
 
