@@ -2361,11 +2361,13 @@ hipError_t try_q40_wide(const KernelArgs &a, int batch, hipStream_t stream, bool
     return hipSuccess;
 }
 
+inline bool q40_mfma_width(int cols) { return cols == 2048 || cols == 3072 || cols == 4096 || cols == 8192 || cols == 14336; }
+
 // Up to sixteen rows, every epilogue but the arg-max: bound by the weights' tiled copies.  A batch of sixteen sequences on the 8B model spends
 // 82 us per layer here (gate|up 24.6 us against 12 for the bytes alone) and 135 us as fp16-operand tile products of 64 columns with K
 // splits and their reductions, whose weights are rounded to fp16 on top (logits 4.2e-4 -> 3.6e-4 off the exact ones).
 bool wide16_width(int format, int cols) {
-    return format == FMT_Q4_K ? cols == 4096 || cols == 14336 || q4k_registry_width(cols) : format == FMT_Q4_0 && (cols == 4096 || cols == 14336);
+    return format == FMT_Q4_K ? cols == 4096 || cols == 14336 || q4k_registry_width(cols) : format == FMT_Q4_0 && q40_mfma_width(cols);
 }
 template <int COLS, bool Q40>
 hipError_t launch_wide16_cols(const KernelArgs &a, int batch, hipStream_t stream, bool *launched) {
@@ -2385,6 +2387,9 @@ hipError_t launch_wide16(const KernelArgs &a, int format, int batch, hipStream_t
         if (a.cols == 8192) e = launch_wide16_cols<8192, false>(a, batch, stream, &launched);
         if (a.cols == 14336) e = launch_wide16_cols<14336, false>(a, batch, stream, &launched);
     } else {
+        if (a.cols == 2048) e = launch_wide16_cols<2048, true>(a, batch, stream, &launched);
+        if (a.cols == 3072) e = launch_wide16_cols<3072, true>(a, batch, stream, &launched);
+        if (a.cols == 8192) e = launch_wide16_cols<8192, true>(a, batch, stream, &launched);
         if (a.cols == 4096) e = launch_wide16_cols<4096, true>(a, batch, stream, &launched);
         if (a.cols == 14336) e = launch_wide16_cols<14336, true>(a, batch, stream, &launched);
     }
@@ -2630,6 +2635,26 @@ hipError_t try_q40_mfma(const KernelArgs &a, hipStream_t stream, bool *launched)
 #undef ESP_Q40_CASE
         return hipSuccess;
     }
+    if constexpr (NB <= 2) {
+#define ESP_Q40_WIDTH(COLS_, W_, KS_)                                                                            \
+        if (a.cols == COLS_ && waves == W_ && ks == KS_) {                                                       \
+            if (mode == 0) return launch_q40_mfma<NB, COLS_ / 512, W_, KS_, 0>(a, stream, launched);             \
+            if (mode == 1) return launch_q40_mfma<NB, COLS_ / 512, W_, KS_, 1>(a, stream, launched);             \
+            return launch_q40_mfma<NB, COLS_ / 512, W_, KS_, 2>(a, stream, launched);                            \
+        }
+        // measured (us, one row, dot-product / four or six wavefronts per block / two or three blocks sharing them): 2048 columns: 3072 rows
+        // 3.25 / 3.12 / 3.47, 16384 rows 6.5 / 5.3 / 4.9, 128256 rows 39.2 / 28.8 / 28.1; 3072 columns: 3072 rows 4.1 / 3.2 / 3.7, 5120 rows
+        // 5.1 / 4.9 / 3.7, 16384 rows 9.3 / 7.9 / 6.4, 128256 rows 54 / 42.5 / 43.5 (4 x 2: 40.9, 16384 rows 6.4); 8192 columns: 2048 rows 5.3 / 3.8
+        if (a.cols == 2048) { if (waves == 0) waves = 4; if (ks == 0) ks = a.rows <= 4096 ? 4 : 2; }
+        if (a.cols == 3072) { if (waves == 0) waves = a.rows <= 16384 ? 6 : 4; if (ks == 0) ks = a.rows <= 4096 ? 6 : a.rows <= 16384 ? 3 : 2; }
+        ESP_Q40_WIDTH(2048, 4, 4)
+        ESP_Q40_WIDTH(2048, 4, 2)
+        ESP_Q40_WIDTH(3072, 6, 6)
+        ESP_Q40_WIDTH(3072, 6, 3)
+        ESP_Q40_WIDTH(3072, 4, 2)
+        if (a.cols == 8192 && mode == 0 && (waves == 0 || waves == 8) && (ks == 0 || ks == 8)) return launch_q40_mfma<NB, 16, 8, 8, 0>(a, stream, launched);
+#undef ESP_Q40_WIDTH
+    }
     if constexpr (NB <= 4) if (a.cols == 14336 && mode == 0) {
         // 4096 rows: 14 x 14 10.5 / 11.4 / 13.7, 7 x 7 10.4 / 11.6 / 14.6; the dot-product kernel 10.8 / 14.2 / 25.1
         if (waves == 0) waves = 14;
@@ -2813,7 +2838,7 @@ bool gemv_wants_tiled_copy(int format, int cols) {
     static const int enabled = env_int("ESPRESSO_HIP_TILED_COPIES", 1);
     if (!enabled) return false;
     if (format == FMT_Q4_K) return cols == 4096 || cols == 14336 || q4k_registry_width(cols);
-    if (format == FMT_Q4_0) return cols == 4096 || cols == 14336;
+    if (format == FMT_Q4_0) return q40_mfma_width(cols);
     if (format == FMT_Q8_0) return q80_mfma_width(cols);
     if (format == FMT_F16) return cols == 768 || cols == 2048;
     return false;

@@ -46,7 +46,8 @@ def test_narrow_split_gemm_matches_float64(mods, form, rows, cols):
 
 # column counts of the sixteen-row kernel: d_model and attention width, hidden size
 @pytest.mark.parametrize("fmt,d,hidden,kv_fp16", [(orc.FMT_Q4_K, 1024, 2048, True), (orc.FMT_Q4_K, 2048, 3072, False), (orc.FMT_Q4_K, 3072, 8192, True),
-                                                  (orc.FMT_Q4_K, 4096, 14336, True), (orc.FMT_Q4_0, 4096, 14336, False)])
+                                                  (orc.FMT_Q4_K, 4096, 14336, True), (orc.FMT_Q4_0, 4096, 14336, False),
+                                                  (orc.FMT_Q4_0, 2048, 8192, True), (orc.FMT_Q4_0, 3072, 8192, False)])
 def test_batches_match_oracle(mods, fmt, d, hidden, kv_fp16):
     ll, ops, syn = mods
     cfg = ll.MultiModelConfig(n_layer=1, n_head=d // 128, n_kv_head=d // 512, d_model=d, head_dim=128, hidden_dim=hidden, vocab=520 if fmt != orc.FMT_Q4_K else 512, max_seq=64)
@@ -89,4 +90,46 @@ def test_short_prompts_in_pairs_match_single_steps(mods, fmt, d, hidden):
         # one and two rows take the same products in another order of their fp32 sums; activations are rounded to fp16 in between
         assert np.abs(np.concatenate(got) - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max()), portions
         assert np.abs(g.logits() - want[-1]).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max())
+    g.close()
+
+
+@pytest.mark.parametrize("cols", [2048, 3072, 8192])
+@pytest.mark.parametrize("rows", [16, 130, 4097, 16400, 33000])
+def test_q4_0_matrix_core_widths_match_float64(mods, rows, cols):
+    _, ops, _ = mods
+    m = ops.Matrix(lib.FORMAT_Q4_0, ops.synth_weights(lib.FORMAT_Q4_0, rows, 0.02, rows * cols), rows, cols)
+    w = m.dequantize().astype(np.float64).reshape(rows, cols)
+    try:
+        ops.set_tuning("q40_mfma", 1)
+        for batch in (1, 2):
+            x = np.random.default_rng(batch).normal(0, 1, (batch, cols)).astype(np.float16)
+            res = np.random.default_rng(rows).normal(0, 1, (batch, rows)).astype(np.float32)
+            want = x.astype(np.float64) @ w.T
+            # exact products, fp32 sums: the bound test_gpu_q40_mfma.py holds the other widths to
+            tol = 2e-5 * np.abs(w).max() * np.sqrt(cols) + 1e-6
+            assert np.abs(m.gemv(x) - want).max() <= tol, batch
+            assert np.abs(m.gemv(x, res) - (want + res)).max() <= tol + 1e-5, batch
+    finally:
+        ops.set_tuning("q40_mfma", -1)
+    m.close()
+
+
+@pytest.mark.parametrize("d,heads,kv,hidden", [(2048, 32, 8, 8192), (3072, 24, 8, 8192)])
+def test_q4_0_decode_matches_oracle(mods, d, heads, kv, hidden):
+    """Norm, RoPE / cache, merged attention, SwiGLU, residual and arg-max forms, then the two-row steps of a short prompt."""
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=1, n_head=heads, n_kv_head=kv, d_model=d, head_dim=d // heads, hidden_dim=hidden, vocab=9000, max_seq=48)
+    g, packed = syn.build_runtime(cfg, orc.FMT_Q4_0, seed=d, kv_format=orc.FMT_F16, keep_packed=True)
+    o = oracle_from_packed(cfg, packed, orc.FMT_Q4_0, 1, True, 48)
+    prompt = [1, 8999, 777, 16, 5]
+    o.prefill(prompt)
+    g.prefill(np.asarray(prompt, np.uint32))
+    for _ in range(5):
+        want = o.logits()
+        assert np.abs(want - g.logits()).max() <= 2e-2
+        tok = o.select_greedy()
+        if o.top2_margin() > 1e-3:
+            assert g.select_greedy() == tok
+        o.advance(tok)
+        g.advance(tok)
     g.close()
