@@ -821,29 +821,34 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
         // every load above is issued before the first use below: one memory round trip for all U chunks
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        // the scores of all U chunks before their one maximum and their exponentials, which then do not wait for each other (chunks wholly
+        // beyond the prefix give p = 0: no branch, so the loop unrolls and all U chunks stay in registers)
+        float sc[U], cm = -INFINITY;
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int t = t0 + u * stride + slot;
-            const bool valid = t < visible;
-            // a chunk wholly beyond the prefix changes nothing (alpha = 1, p = 0): no branch, so the loop unrolls and
-            // all U chunks stay in registers
-            float k[8], v[8];
+            float k[8], d = 0.0f;
             unpack8(kr[u], k);
-            unpack8(vr[u], v);
-            float d = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; i++) d = __builtin_fmaf(q[i], k[i], d);
-            d = group_sum<LPT>(d);                                  // all lanes of the token
-            const float sc = valid ? __fmul_rn(d, scale) : -INFINITY;
-            const float cm = max_over_groups<LPT>(sc);              // over the chunk's tokens
-            const float m_new = fmaxf(mx, cm);         // finite: the chunk holds at least one visible token
-            const float alpha = expf(mx - m_new);      // exp(-inf) = 0 on the first chunk
-            const float p = valid ? expf(sc - m_new) : 0.0f;
-            l = __builtin_fmaf(l, alpha, p);
-#pragma unroll
-            for (int i = 0; i < 8; i++) acc[i] = __builtin_fmaf(p, v[i], __fmul_rn(acc[i], alpha));
-            mx = m_new;
+            d = group_sum<LPT>(d);                                      // all lanes of the token
+            sc[u] = t0 + u * stride + slot < visible ? __fmul_rn(d, scale) : -INFINITY;
+            cm = fmaxf(cm, sc[u]);
         }
+        const float m_new = fmaxf(mx, max_over_groups<LPT>(cm));       // finite: the first chunk holds at least one visible token
+        const float alpha = expf(mx - m_new);                          // exp(-inf) = 0 in the first pass
+        l = __fmul_rn(l, alpha);
+#pragma unroll
+        for (int i = 0; i < 8; i++) acc[i] = __fmul_rn(acc[i], alpha);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            float v[8];
+            unpack8(vr[u], v);
+            const float p = t0 + u * stride + slot < visible ? expf(sc[u] - m_new) : 0.0f;
+            l += p;
+#pragma unroll
+            for (int i = 0; i < 8; i++) acc[i] = __builtin_fmaf(p, v[i], acc[i]);
+        }
+        mx = m_new;
     }
     // ---- the wavefront's token slots share one m: their sums and accumulators add up across the lanes that differ in the slot
     // index only, and the wavefront publishes one state ----
