@@ -75,7 +75,7 @@ hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, bool kv_f16
 // the context merges them (GemvParams::merge_partials).  attention_head_splits: slices per query head.
 int attention_head_splits(int max_seq);
 hipError_t launch_attention_partials(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s);
-hipError_t launch_swiglu(const float *gu, int rows, int hidden, uint16_t *act_f16, hipStream_t s);
+hipError_t launch_swiglu(const float *gu, int splits, size_t plane, int rows, int hidden, uint16_t *act_f16, hipStream_t s);
 // Scratch of the two-launch argmax: kMaxStepRows x 128 partial (value, index) pairs.
 struct ArgmaxScratch {
     float *part_value = nullptr;

