@@ -1383,7 +1383,12 @@ int attention_split_count(int max_seq, int head_dim) {
 hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s) {
     // grouped-query kernel for the common head shapes; everything else takes the general kernel
     const int group = a.n_head / a.n_kv_head;
-    if (a.n_head % a.n_kv_head == 0) {
+    const bool by_head = a.head_partials && (a.head_dim == 128 || a.head_dim == 64) && a.n_head % a.n_kv_head == 0 && rows <= kMaxStepRows &&
+                         a.cache_seq_stride <= 0xFFFFFFFFull && a.n_head <= 0xFFFF;
+    // Contexts of up to 512 tokens: the kernel of the single-row step, whose four slices of a head cover them in two passes (sixteen
+    // sequences of the 8B model, attention + merge of a layer: prefix 60-84 of 512 8.4 + 6.6 -> 6.4 + 4.8 us, 384 of 512 14.4 + 6.6 -> 12.7 + 4.9;
+    // 768 of 1024 19.5 + 6.7 against 21.4 + 4.9, 3072 of 4096 55.7 + 6.6 against 65.9 + 4.9: those keep the kernel that reads a key once per group).
+    if (a.n_head % a.n_kv_head == 0 && !(by_head && a.max_seq <= 512)) {
         if (a.head_dim == 128) {
             if (group == 1) return launch_attention_gqa<128, 1>(a, rows, kv_f16, s);
             if (group == 2) return launch_attention_gqa<128, 2>(a, rows, kv_f16, s);
@@ -1394,9 +1399,8 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
             if (group == 4) return launch_attention_gqa<64, 4>(a, rows, kv_f16, s);
         }
     }
-    // other head groups: the kernel of the single-row step and a merge launch
-    if (a.n_head % a.n_kv_head == 0 && (a.head_dim == 128 || a.head_dim == 64) && a.head_partials && rows <= kMaxStepRows &&
-        a.cache_seq_stride <= 0xFFFFFFFFull && a.n_head <= 0xFFFF) {
+    // short contexts and other head groups: the kernel of the single-row step and a merge launch
+    if (by_head) {
         const hipError_t e = launch_attention_partials(a, rows, kv_f16, s);
         if (e != hipSuccess) return e;
         if (a.head_dim == 128) hipLaunchKernelGGL(attention_partial_merge_kernel<128>, dim3(a.n_head, rows), dim3(128), 0, s, a.head_partials, a.n_head, a.ctx_f16);
