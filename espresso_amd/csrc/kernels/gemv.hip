@@ -385,13 +385,13 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     EarlyEpilogue<B> early;
     if constexpr (R == 2) early_positions<B>(a, early);
     constexpr int KS = 2;                                                  // groups of eight per thread in registers (MODE 0 and 1)
-    const int per_row = cols / 8;
+    const int per_row = cols / 8, last_group = per_row > 1 ? per_row - 1 : 0;   // (four fp32 columns: no whole group)
     float4 nv0[MODE == 1 ? B : 1][KS], nv1[MODE == 1 ? B : 1][KS], ng0[KS], ng1[KS];
     uint4 xv0[MODE == 0 ? B : 1][KS];
     if constexpr (MODE != 2) {
 #pragma unroll
         for (int k = 0; k < KS; k++) {
-            const int g = tid + k * kThreads < per_row ? tid + k * kThreads : per_row - 1;
+            const int g = tid + k * kThreads < per_row ? tid + k * kThreads : last_group;
 #pragma unroll
             for (int b = 0; b < B; b++) {
                 if constexpr (MODE == 1) {
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     float4 mm0[B][kMergeSplits], mm1[B][kMergeSplits];
     if constexpr (MODE == 2) {
 #pragma unroll
-        for (int b = 0; b < B; b++) merge_group_load(a, b, tid < per_row ? tid : per_row - 1, cols, mml[b], mm0[b], mm1[b]);
+        for (int b = 0; b < B; b++) merge_group_load(a, b, tid < per_row ? tid : last_group, cols, mml[b], mm0[b], mm1[b]);
     }
 
     // ---- the wavefront's rows ----
