@@ -39,6 +39,9 @@ class DecoderRuntime {
     // Rollback = lower the visible length.  Runtimes with recurrent state (can_roll_back() false) take only 0 and the length
     // the sequence has.
     int set_visible(int seq, int count);
+    // A generation loop has run `count` more tokens of the sequence through its own rows (forward_rows, enqueue_device_rows), so the caches
+    // and states hold them: recurrent runtimes included, whose visible length set_visible() does not raise.
+    void add_consumed(int seq, int count) { visible_[seq] += count; }
     virtual bool can_roll_back() const { return true; }
     // whether one step may hold several rows of one sequence (draft verification)
     virtual bool takes_rows_of_one_sequence() const { return true; }

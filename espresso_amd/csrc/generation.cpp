@@ -180,7 +180,7 @@ int generate_greedy_batch(DecoderRuntime &rt, const uint32_t *const *prompts, co
             if ((rc = hip_ok(hipStreamSynchronize(st), "greedy batch")) != ESP_OK) return rc;
             for (int s = 0; s < n_seq; s++) {
                 for (int i = 0; i < steps; i++) (*out)[s].push_back((uint32_t)log[(size_t)i * n_seq + s]);
-                rt.set_visible(s, rt.visible(s) + steps);
+                rt.add_consumed(s, steps);
             }
             first_host_step = eff;
         }
@@ -192,7 +192,7 @@ int generate_greedy_batch(DecoderRuntime &rt, const uint32_t *const *prompts, co
             if ((rc = rt.forward_rows(rows)) != ESP_OK) return rc;
             if ((rc = rt.head_rows(n_seq, next)) != ESP_OK) return rc;
             for (int s = 0; s < n_seq; s++) {
-                rt.set_visible(s, rows.pos[s] + 1);
+                rt.add_consumed(s, 1);
                 current[s] = next[s];
                 (*out)[s].push_back(next[s]);
             }

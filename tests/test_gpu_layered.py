@@ -292,6 +292,22 @@ def test_batches_of_unequal_prompts(mixed):
         assert g == mixed.greedy(p, 20)
 
 
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("new", [1, 2, 5])
+def test_a_batch_leaves_sequences_that_go_on(mixed, new, graphs):
+    """Steps of a batch with and without a captured graph: the tokens, the visible lengths and what the sequences hold afterwards."""
+    rt = mixed.runtime("f32", max_seq=160, sequences=3)
+    ll.set_graph_replay(rt, graphs)
+    prompts = [lu.tokens(mixed.cfg, n, 70 + n) for n in (5, 41, 12)]
+    got, _ = ll.generate_batch(rt, prompts, new)
+    for s, (p, g) in enumerate(zip(prompts, got)):
+        assert g == mixed.greedy(p, new)
+        assert rt.visible(s) == len(p) + new - 1   # the last token is chosen and not consumed
+        more = g[-1:] + lu.tokens(mixed.cfg, 3, 80 + s)
+        out = rt.append(more, list(range(len(more))), sequence=s)
+        assert lu.error(out, mixed.logits(p + g[:-1] + more)[len(p) + new - 1:]) < lu.F32_LIMIT
+
+
 def marked_attention(tmp_path, window, kv_from):
     """Grouped attention whose queries match only the keys of token 1, by far: a query's logits say whether token 1 stands in its window."""
     layers = [lu.attention(window=window, ff=0, scale=0.5, dims=4)]
