@@ -384,10 +384,14 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     // ---- positions and activations: requested first (memory returns in order) ----
     EarlyEpilogue<B> early;
     if constexpr (R == 2) early_positions<B>(a, early);
-    constexpr int KS = 2;                                                  // groups of eight per thread in registers (MODE 0 and 1)
-    const int per_row = cols / 8, last_group = per_row > 1 ? per_row - 1 : 0;   // (four fp32 columns: no whole group)
+    // Groups a row is staged in: eight activations; of fp32 matrices given fp16 activations four, since their rows may be whole groups of
+    // four columns only (fused norms and merges see whole groups of eight).
+    constexpr bool kFours = FMT == FMT_F32 && MODE == 0;
+    using Group = std::conditional_t<kFours, uint2, uint4>;
+    constexpr int KS = kFours ? 4 : 2;                                     // groups per thread in registers (MODE 0 and 1)
+    const int per_row = cols / (kFours ? 4 : 8), last_group = per_row - 1;
     float4 nv0[MODE == 1 ? B : 1][KS], nv1[MODE == 1 ? B : 1][KS], ng0[KS], ng1[KS];
-    uint4 xv0[MODE == 0 ? B : 1][KS];
+    Group xv0[MODE == 0 ? B : 1][KS];
     if constexpr (MODE != 2) {
 #pragma unroll
         for (int k = 0; k < KS; k++) {
@@ -398,7 +402,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
                     const float4 *x4 = reinterpret_cast<const float4 *>(a.norm_x + (size_t)b * cols);
                     nv0[b][k] = x4[2 * g]; nv1[b][k] = x4[2 * g + 1];
                 } else {
-                    xv0[b][k] = reinterpret_cast<const uint4 *>(a.x)[(size_t)b * per_row + g];
+                    xv0[b][k] = reinterpret_cast<const Group *>(a.x)[(size_t)b * per_row + g];
                 }
             }
             if constexpr (MODE == 1) {
@@ -447,8 +451,11 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     // four swapped for the integer formats ----
     {
         __shared__ float norm_red[B * kWaves];
-        uint4 *dst = reinterpret_cast<uint4 *>(xs);
-        auto put = [&](int b, int g, const uint4 &v) { dst[(size_t)b * per_row + g] = T::kPermuteX ? swap_middle(v) : v; };
+        Group *dst = reinterpret_cast<Group *>(xs);
+        auto put = [&](int b, int g, const Group &v) {
+            if constexpr (T::kPermuteX) dst[(size_t)b * per_row + g] = swap_middle(v);
+            else dst[(size_t)b * per_row + g] = v;
+        };
 #pragma unroll
         for (int b = 0; b < B; b++) {
             float inv = 0.0f;
@@ -471,9 +478,9 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
             }
             if constexpr (MODE == 0) {
                 // the others four per thread at a time
-                const uint4 *xr = reinterpret_cast<const uint4 *>(a.x) + (size_t)b * per_row;
+                const Group *xr = reinterpret_cast<const Group *>(a.x) + (size_t)b * per_row;
                 for (int g0 = KS * kThreads + tid; g0 < per_row; g0 += 4 * kThreads) {
-                    uint4 t[4];
+                    Group t[4];
 #pragma unroll
                     for (int k = 0; k < 4; k++) t[k] = xr[g0 + k * kThreads < per_row ? g0 + k * kThreads : per_row - 1];
 #pragma unroll

@@ -51,6 +51,25 @@ def test_rounds_of_items(mods, fmt, items):
         m.close()
 
 
+@pytest.mark.parametrize("cols", [4, 8, 12, 252, 260, 1028, 4092, 5124])
+def test_fp32_rows_of_whole_fours(mods, cols):
+    """Every multiple of four columns is taken: rows of the activations start at any multiple of eight bytes, and the last four columns count."""
+    _, ops, _ = mods
+    rng = np.random.default_rng(cols)
+    for rows in (1, 6, 9):
+        w = rng.normal(0, 0.02, (rows, cols)).astype(np.float32)
+        w[:, -4:] *= 50
+        m = ops.Matrix(orc.FMT_F32, w.view(np.uint8), rows, cols)
+        for batch in (1, 2, 3):
+            x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
+            res = rng.normal(0, 1, (batch, rows)).astype(np.float32)
+            want = x.astype(np.float64) @ w.astype(np.float64).T
+            bound = 2.0 ** -23 * (np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T) * (8 + cols / 64) + 1e-6   # as above
+            assert (np.abs(m.gemv(x) - want) <= bound).all(), (rows, batch)
+            assert (np.abs(m.gemv(x, res) - (want + res)) <= bound + 2.0 ** -22 * np.abs(want + res)).all(), (rows, batch)
+        m.close()
+
+
 # norm rows of up to 512 groups of eight stay in registers; attention states beyond one group per thread; odd pair counts
 @pytest.mark.parametrize("fmt,d,heads,kv,hidden", [(orc.FMT_F16, 576, 9, 3, 1536), (orc.FMT_Q8_0, 4352, 34, 2, 608), (orc.FMT_Q4_0, 2304, 18, 2, 4224),
                                                    (orc.FMT_F16, 64, 1, 1, 72)])
