@@ -253,7 +253,7 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
         return ESP_OK;
     }
     for (int i = 0; i < count; i++) {
-        if (i + 1 < count && takes_rows_of_one_sequence()) {
+        if (i + 1 < count && matrix_prefill_ && takes_rows_of_one_sequence()) {
             // two tokens per pass over the weights: the second row sees the first one's keys and values, which the projection wrote
             // before either row's attention.  Such a step is bound by the weights' bytes and the launches, both shared by the rows:
             // ten tokens of the smol model 6.6 -> 4.4 ms.

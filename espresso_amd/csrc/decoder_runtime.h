@@ -17,7 +17,7 @@ class LayeredRuntime;
 
 constexpr int kPrefillBlockRows = 512;        // rows per MFMA prefill block
 constexpr int kStepsPerGraph = 8;             // greedy steps in the longer of the two captured step graphs
-constexpr int kMatrixPrefillMinTokens = 32;   // shorter prompts take the exact per-token path
+constexpr int kMatrixPrefillMinTokens = 32;   // shorter prompts take the steps' kernels, two tokens at a time where a step takes two rows
 constexpr size_t kGemmWorkspaceFloats = (size_t)8 << 20;
 
 struct DecoderShape {
@@ -72,7 +72,8 @@ class DecoderRuntime {
     // consumed.  The step graph notices it on the device; the host looks once per 32 replays.
     int continue_greedy_until_stop(int seq, int steps, uint32_t *out_tokens, int *produced);
     void set_use_graph(bool enabled) { use_graph_ = enabled; }
-    // Prompts of matrix_prefill_min_tokens() or more run in blocks through the MFMA kernels (default on).
+    // Prompts of matrix_prefill_min_tokens() or more run in blocks through the MFMA kernels, shorter ones two tokens per step (default on;
+    // off: one token per step, whatever the prompt's length).
     void set_matrix_prefill(bool enabled) { matrix_prefill_ = enabled; }
     int read_last_hidden(int seq, float *out);
     int read_logits(int seq, float *out);         // runs the head on the kept hidden state

@@ -234,8 +234,8 @@ int esp_llama_continue_greedy(ESPLlamaRuntime *runtime, int sequence, int steps,
 int esp_llama_set_graph_replay(ESPLlamaRuntime *runtime, int enabled);
 /* Prompts of 32 tokens or more (Q4_K models on the exact block kernels: of four or more) are prefilled in blocks of up to 512 rows with every projection as one
  * dequant-fused MFMA GEMM (fp16 weights after dequantisation, fp32 accumulation), instead of the
- * reference's token-by-token walk (RealModelInferenceEngine.swift:6365-6375).  enabled = 0 restores the
- * per-token path, whose arithmetic keeps the dequantised weights in fp32.  Default: enabled. */
+ * reference's token-by-token walk (RealModelInferenceEngine.swift:6365-6375); shorter ones walk two tokens per step.
+ * enabled = 0 restores the per-token path for every length, whose arithmetic keeps the dequantised weights in fp32.  Default: enabled. */
 int esp_llama_set_matrix_prefill(ESPLlamaRuntime *runtime, int enabled);
 /* Decode steps of one or two rows run attention (decodeContextFromCaches, :6774-6823) as one launch that leaves
  * per-head partial softmax states, and the wo GEMV merges them while it stages its input, where the shapes allow

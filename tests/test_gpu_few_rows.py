@@ -93,6 +93,21 @@ def test_short_prompts_in_pairs_match_single_steps(mods, fmt, d, hidden):
     g.close()
 
 
+def test_without_matrix_prefill_every_token_is_a_step(mods):
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=4, n_kv_head=4, d_model=256, head_dim=64, hidden_dim=512, vocab=512, max_seq=64)
+    g, _ = syn.build_runtime(cfg, lib.FORMAT_Q8_0, seed=5, std=0.05)
+    tokens = np.random.default_rng(1).integers(0, cfg.vocab, 43).astype(np.uint32)
+    ll.set_kernel_timing(g, True)
+    for enabled, count, steps in [(False, 43, 43), (False, 7, 7), (True, 7, 4)]:
+        ll.set_matrix_prefill(g, enabled)
+        g.reset()
+        ll.kernel_times(g)
+        g.prefill(tokens[:count])
+        assert ll.kernel_times(g)["qkv"]["launches"] == cfg.n_layer * steps, (enabled, count)
+    g.close()
+
+
 @pytest.mark.parametrize("cols", [2048, 3072, 8192])
 @pytest.mark.parametrize("rows", [16, 130, 4097, 16400, 33000])
 def test_q4_0_matrix_core_widths_match_float64(mods, rows, cols):
