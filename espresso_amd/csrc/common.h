@@ -202,6 +202,8 @@ bool gemv_set_tuning(const char *key, int value);
 // True when launch_gemv handles `batch` rows without re-reading the weights per pair of rows (always for one or two rows).
 bool gemv_takes_rows(const DeviceMatrix &w, int batch);
 bool gemv_takes_sixteen_rows(const DeviceMatrix &w, int batch);
+// Whether two rows of activations fit the LDS of the kernel launch_gemv picks for them (very long rows fit one at a time only).
+bool gemv_holds_two_rows(const DeviceMatrix &w);
 // True when launch_gemv has the EPI_ARGMAX epilogue for this matrix (every format; Q4_K rows of 8192 or more columns, which
 // several wavefronts share, keep the separate argmax launches).
 bool gemv_supports_argmax(const DeviceMatrix &w);

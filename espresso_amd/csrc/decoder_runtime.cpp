@@ -252,8 +252,9 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
         visible_[seq] = start + count;
         return ESP_OK;
     }
+    const bool pairs = matrix_prefill_ && takes_rows_of_one_sequence() && steps_hold_two_rows();
     for (int i = 0; i < count; i++) {
-        if (i + 1 < count && matrix_prefill_ && takes_rows_of_one_sequence()) {
+        if (i + 1 < count && pairs) {
             // two tokens per pass over the weights: the second row sees the first one's keys and values, which the projection wrote
             // before either row's attention.  Such a step is bound by the weights' bytes and the launches, both shared by the rows:
             // ten tokens of the smol model 6.6 -> 4.4 ms.

@@ -45,6 +45,8 @@ class DecoderRuntime {
     virtual bool can_roll_back() const { return true; }
     // whether one step may hold several rows of one sequence (draft verification)
     virtual bool takes_rows_of_one_sequence() const { return true; }
+    // whether the step's kernels hold two rows of every matrix at once
+    virtual bool steps_hold_two_rows() const { return true; }
     // Sequence slots for callers with requests that come and go: the lowest free slot, and its return.  A slot that is taken
     // again starts as an empty sequence.
     int acquire_sequence(int *seq);

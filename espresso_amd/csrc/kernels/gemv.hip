@@ -2159,8 +2159,10 @@ inline void launch_kernel(K kernel, dim3 grid, dim3 block, size_t lds, hipStream
     else hipLaunchKernelGGL(kernel, grid, block, lds, stream, args...);
 }
 
+constexpr size_t kMaxLds = 160 * 1024;
+constexpr size_t q4k_generic_lds(int batch, int cols) { return (size_t)batch * 8 * ((cols / 64) | 1) * 16 + (size_t)batch * (cols / 32) * 4 + (size_t)batch * kWaves * 4; }
 inline hipError_t ensure_lds(const void *kernel, size_t lds, size_t *configured) {
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
+    if (lds > kMaxLds) return hipErrorInvalidValue;
     if (lds > 48 * 1024 && lds > *configured) {
         hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
@@ -2270,7 +2272,7 @@ hipError_t launch_q4k_mfma(const KernelArgs &a, hipStream_t stream, bool *launch
     *launched = false;
     const size_t lds = ((size_t)NBX * (cols / 8) + 8) * 16 + (size_t)NB * (cols / 32) * 4 + (KS > 1 ? (size_t)kMfmaRounds * WAVES * NB * 16 * 4 : 0) +
                        (size_t)2 * NB * WAVES * 4;
-    if (lds > 160 * 1024) return hipSuccess;   // not launched
+    if (lds > kMaxLds) return hipSuccess;   // not launched
     auto kernel = gemv_q4k_mfma_kernel<NB, IPR, WAVES, KS, MODE, SPLIT, STAMPS>;
     static size_t configured_lds = 0;
     hipError_t e = ensure_lds(reinterpret_cast<const void *>(kernel), lds, &configured_lds);
@@ -2522,7 +2524,7 @@ hipError_t launch_q4k(const KernelArgs &a, hipStream_t stream) {
         break;
     default: break;
     }
-    const size_t lds = (size_t)B * 8 * ((a.cols / 64) | 1) * 16 + (size_t)B * (a.cols / 32) * 4 + (size_t)B * kWaves * 4;
+    const size_t lds = q4k_generic_lds(B, a.cols);
     auto kernel = gemv_q4k_generic_kernel<B>;
     static size_t configured_lds = 0;
     hipError_t e = ensure_lds(reinterpret_cast<const void *>(kernel), lds, &configured_lds);
@@ -2536,7 +2538,7 @@ hipError_t launch_q4k(const KernelArgs &a, hipStream_t stream) {
 template <int FMT, int B, int R, int MODE, int DEPTH>
 hipError_t launch_one(const KernelArgs &a, hipStream_t stream) {
     const size_t lds = (size_t)B * a.cols * 2;
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
+    if (lds > kMaxLds) return hipErrorInvalidValue;
     auto kernel = gemv_kernel<FMT, B, R, MODE, DEPTH>;
     static size_t configured_lds = 0;  // per instantiation
     if (lds > 48 * 1024 && lds > configured_lds) {
@@ -2584,7 +2586,7 @@ hipError_t launch_q40_mfma(const KernelArgs &a, hipStream_t stream, bool *launch
     *launched = false;
     const size_t lds = ((size_t)NB * (cols / 8) + 8) * 16 + (size_t)NB * (cols / 32) * 4 + (KS > 1 ? (size_t)q40_rounds(TPR) * WAVES * NB * 16 * 4 : 0) +
                        (size_t)2 * NB * WAVES * 4;
-    if (lds > 160 * 1024) return hipSuccess;   // not launched
+    if (lds > kMaxLds) return hipSuccess;   // not launched
     auto kernel = gemv_q40_mfma_kernel<NB, TPR, WAVES, KS, MODE>;
     static size_t configured_lds = 0;
     hipError_t e = ensure_lds(reinterpret_cast<const void *>(kernel), lds, &configured_lds);
@@ -2822,6 +2824,11 @@ bool gemv_takes_rows(const DeviceMatrix &w, int batch) {
         return true;
     if (batch > 8) return false;
     return batch <= 4 ? (w.cols == 4096 || w.cols == 14336) : (w.cols == 4096 && w.rows <= q4k_mfma_rows8_max());
+}
+
+// Only the kernels for any column count stage rows without a bound of their own; their static arrays take less than a kilobyte.
+bool gemv_holds_two_rows(const DeviceMatrix &w) {
+    return (w.format == FMT_Q4_K ? q4k_generic_lds(2, w.cols) : (size_t)2 * w.cols * 2) <= kMaxLds - 1024;
 }
 
 bool gemv_takes_sixteen_rows(const DeviceMatrix &w, int batch) {

@@ -488,6 +488,12 @@ bool LlamaRuntime::matrix_prefill_supported() const {
     return true;
 }
 
+bool LlamaRuntime::steps_hold_two_rows() const {
+    for (const Layer &L : layers_)
+        if (!gemv_holds_two_rows(L.wqkv) || !gemv_holds_two_rows(L.wo) || !gemv_holds_two_rows(L.w13) || !gemv_holds_two_rows(L.w2)) return false;
+    return true;
+}
+
 // `rows` prompt tokens at positions base.. of one sequence: the layer loop of forwardToken (:6221-6347) over
 // a block of rows, every projection as one dequant-fused MFMA GEMM.  Rows of the block see each other's
 // keys and values causally because the whole block's K/V is written before its attention runs.

@@ -95,6 +95,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool sixteen_rows_supported(int rows) const;
     int enqueue_layers_sixteen(int rows);
     bool matrix_prefill_supported() const override;
+    bool steps_hold_two_rows() const override;
     int matrix_prefill_min_tokens() const override;
     bool wo_merges_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);

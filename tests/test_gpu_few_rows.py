@@ -93,6 +93,21 @@ def test_short_prompts_in_pairs_match_single_steps(mods, fmt, d, hidden):
     g.close()
 
 
+@pytest.mark.parametrize("fmt,hidden", [("q8_0", 53248), ("f16", 40960), ("f16", 40448), ("q4_0", 53248), ("q4_k", 53248)])
+def test_short_prompts_of_feed_forwards_too_wide_for_pairs(mods, fmt, hidden):
+    """Two rows of 40960 columns and more do not fit the LDS of a workgroup: such prompts walk one token per step."""
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=1, n_head=4, n_kv_head=4, d_model=256, head_dim=64, hidden_dim=hidden, vocab=512, max_seq=16)
+    g, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=5, std=0.05)
+    tokens = np.random.default_rng(hidden).integers(0, cfg.vocab, 5).astype(np.uint32)
+    for t in tokens:
+        g.advance(int(t))
+    want = g.logits()
+    g.prefill(tokens)
+    assert np.abs(g.logits() - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max())   # as above
+    g.close()
+
+
 def test_without_matrix_prefill_every_token_is_a_step(mods):
     ll, ops, syn = mods
     cfg = ll.MultiModelConfig(n_layer=2, n_head=4, n_kv_head=4, d_model=256, head_dim=64, hidden_dim=512, vocab=512, max_seq=64)
