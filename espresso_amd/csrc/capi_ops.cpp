@@ -8,6 +8,7 @@
 #include "context.h"
 #include "host/model_support.h"
 #include "kernels/decode_ops.h"
+#include "kernels/span_attention.h"
 
 using namespace esp;
 
@@ -196,6 +197,88 @@ int esp_matmul_f32(const ESPMatrix *matrix, const float *x, int rows, float *y, 
     if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
     release();
     return e == hipSuccess ? ESP_OK : fail_hip(e, "matmul_f32");
+}
+
+int esp_block_attention(int kernel, const float *q, const void *k, const void *v, int kv_f16, int rows, int first, int heads, int kv_heads, int head_dim,
+                        int split_rows, float *ctx, int iters, double *mean_us) {
+    if (!q || !k || !v || !ctx) return fail(ESP_ERR_INVALID_ARGUMENT, "block_attention: null pointer");
+    if (rows < 1 || rows > 512 || first < 0 || heads < 1 || kv_heads < 1 || heads > 4096 || kv_heads > heads || head_dim < 1 || iters < 1 || first > (1 << 20))
+        return fail(ESP_ERR_INVALID_ARGUMENT, "block_attention: %d rows behind %d, %d heads over %d of %d", rows, first, heads, kv_heads, head_dim);
+    AttentionArgs a{};
+    a.n_head = heads; a.n_kv_head = kv_heads; a.head_dim = head_dim; a.max_seq = first + rows;
+    const size_t nq = (size_t)rows * heads * head_dim, nk = (size_t)a.max_seq * kv_heads * head_dim;
+    a.cache_seq_stride = nk;
+    const bool takes = kernel == ESP_ATTENTION_SINGLE_ROW ? heads % kv_heads == 0 && (head_dim == 64 || head_dim == 128) && !split_rows
+                       : kernel == ESP_ATTENTION_PROMPT ? attention_prompt_supported(heads, kv_heads, head_dim) && (!split_rows || (kv_f16 && heads * head_dim % 256 == 0))
+                       : kernel == ESP_ATTENTION_SPAN ? span_attention_supported(heads, kv_heads, head_dim) && (!split_rows || heads * head_dim % 256 == 0) : false;
+    if (!takes) return fail(ESP_ERR_UNSUPPORTED, "block_attention: kernel %d does not take this shape", kernel);
+    int rc = ensure_init();
+    if (rc != ESP_OK) return rc;
+    Context &c = context();
+    float *d_q = nullptr, *d_scratch = nullptr;
+    uint8_t *d_k = nullptr, *d_v = nullptr;
+    int *d_at = nullptr;
+    uint16_t *d_hi = nullptr, *d_lo = nullptr, *d_sums = nullptr;
+    hipEvent_t start = nullptr, stop = nullptr;
+    auto release = [&] {
+        void *ptrs[] = {d_q, d_k, d_v, d_at, d_hi, d_lo, d_sums, d_scratch};
+        for (void *p : ptrs) if (p) (void)hipFree(p);
+        if (start) (void)hipEventDestroy(start);
+        if (stop) (void)hipEventDestroy(stop);
+    };
+    const size_t each = kv_f16 ? 2 : 4, partials = (size_t)rows * heads * kAttentionMaxSplits * (head_dim + 4);
+    if ((rc = device_alloc(&d_q, nq)) != ESP_OK || (rc = device_alloc(&d_k, nk * each)) != ESP_OK || (rc = device_alloc(&d_v, nk * each)) != ESP_OK ||
+        (rc = device_alloc(&d_at, (size_t)2 * rows)) != ESP_OK || (rc = device_alloc(&d_hi, nq)) != ESP_OK || (rc = device_alloc(&d_lo, nq)) != ESP_OK ||
+        (rc = device_alloc(&d_sums, nq / 16 + 16)) != ESP_OK || (kernel == ESP_ATTENTION_SINGLE_ROW && (rc = device_alloc(&d_scratch, partials)) != ESP_OK)) {
+        release();
+        return rc;
+    }
+    std::vector<int> at(2 * rows, 0);   // positions, sequences
+    for (int i = 0; i < rows; i++) at[i] = first + i;
+    hipError_t e = hipMemcpy(d_q, q, nq * 4, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_k, k, nk * each, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_v, v, nk * each, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_at, at.data(), at.size() * sizeof(int), hipMemcpyHostToDevice);
+    a.q = d_q; a.k_cache = d_k; a.v_cache = d_v; a.pos = d_at; a.seq = d_at + rows; a.split_scratch = d_scratch;
+    if (split_rows) { a.ctx_hi = d_hi; a.ctx_lo = d_lo; a.ctx_sums = d_sums; }
+    else a.ctx_f16 = d_hi;
+    auto launch = [&] {
+        if (kernel == ESP_ATTENTION_PROMPT) return launch_attention_prompt(a, rows, kv_f16 != 0, c.stream);
+        if (kernel == ESP_ATTENTION_SPAN) return launch_span_attention(a, rows, a.max_seq, kv_f16 != 0, c.stream);
+        return launch_attention(a, rows, kv_f16 != 0, c.stream);
+    };
+    if (e == hipSuccess) e = hipEventCreate(&start);
+    if (e == hipSuccess) e = hipEventCreate(&stop);
+    if (e == hipSuccess) e = launch();
+    if (e == hipSuccess) e = hipEventRecord(start, c.stream);
+    for (int i = 1; i < iters && e == hipSuccess; i++) e = launch();
+    if (e == hipSuccess) e = hipEventRecord(stop, c.stream);
+    std::vector<uint16_t> hi(nq), lo(nq), sums(nq / 16);
+    if (e == hipSuccess) e = hipMemcpyAsync(hi.data(), d_hi, nq * 2, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(lo.data(), d_lo, nq * 2, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(sums.data(), d_sums, sums.size() * 2, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    float ms = 0.0f;
+    if (e == hipSuccess && iters > 1) e = hipEventElapsedTime(&ms, start, stop);
+    release();
+    if (e != hipSuccess) return fail_hip(e, "block_attention");
+    if (mean_us) *mean_us = iters > 1 ? 1e3 * ms / (iters - 1) : 0.0;
+    for (size_t i = 0; i < nq; i++) {   // the planes' order inside fours is 0, 2, 1, 3
+        const size_t p = split_rows ? (i & ~(size_t)3) + ((i & 1) << 1 | (i >> 1 & 1)) : i;
+        ctx[i] = split_rows ? half_to_float(hi[p]) + half_to_float(lo[p]) / 2048.0f : half_to_float(hi[p]);
+    }
+    // the sub-block sums that accompany the planes must be the planes' own, to rounding
+    const size_t cols = (size_t)heads * head_dim;
+    for (size_t sub = 0; split_rows && sub < nq / 32; sub++) {
+        double want = 0.0;
+        for (size_t i = 32 * sub; i < 32 * sub + 32; i++) want += ctx[i];
+        const size_t row = 32 * sub / cols, in_row = sub - row * (cols / 32);
+        const uint16_t *p = sums.data() + (row * (cols / 256) + (in_row >> 3)) * 16 + (in_row & 7);
+        const double got = (double)half_to_float(p[0]) + (double)half_to_float(p[8]) / 2048.0;
+        if (std::isfinite(want) && std::fabs(got - want) > 1e-5 * (1.0 + std::fabs(want)))
+            return fail(ESP_ERR_LAUNCH_FAILED, "block_attention: sum of sub-block %zu is %g, its columns add up to %g", sub, got, want);
+    }
+    return ESP_OK;
 }
 
 int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, float *act) {

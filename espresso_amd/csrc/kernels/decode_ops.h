@@ -49,7 +49,7 @@ struct AttentionArgs {
     float *split_scratch;
     // partial results of attention_partial_kernel: [rows][heads][attention_head_splits][head_dim + 4] floats
     float *head_partials;
-    // launch_attention_prompt only, all three or none: the context as split rows (hi = fp16(v), lo = fp16((v - hi) * 2048),
+    // launch_attention_prompt and launch_span_attention only, all three or none: the context as split rows (hi = fp16(v), lo = fp16((v - hi) * 2048),
     // sub-block sums; SplitRowsView) instead of ctx_f16, with the queries and the softmax weights split the same way
     uint16_t *ctx_hi, *ctx_lo, *ctx_sums;
 };

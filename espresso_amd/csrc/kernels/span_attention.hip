@@ -1,20 +1,25 @@
-// Causal attention of a prompt block on the matrix cores for any number of query heads per key/value head, with 32-bit queries, caches
-// and softmax weights kept to 22 bits: the block form of models whose heads attention_prompt_kernel (decode_ops.hip) is not written
-// for (three or eight query heads per key/value head, say).  Those took the general single-query kernel, in which every row reads its
-// whole prefix by itself; per layer, 512 rows of 24 heads of 128 up to position 1535: 782 -> 37 us; 93 rows of 32 heads of 64 behind
-// 700 tokens: 123 -> 13.4 us.
+// Causal attention of a prompt block on the matrix cores with 32-bit arithmetic, for any number of query heads per key/value head: the
+// block form of models whose heads attention_prompt_kernel (decode_ops.hip) is not written for (three or eight query heads per key/value
+// head, say), and of short blocks that must be as exact as the single-row steps.
 //
-// grid (query heads, tiles of 32 rows); a workgroup is KP wavefronts that share the 32 queries and deal the tiles of 32 keys among
-// themselves (wavefront p takes tiles p, p + KP, ...).  A wavefront runs by itself from its first tile to its last: its value tile is its
-// own stretch of LDS, so there is no barrier in the loop; the KP states (maximum, sum, context) are merged pairwise through the same LDS
-// at the end.  KP fills the chip where heads x row tiles do not (launch_span_attention).  What bounds it: the chain of a tile (scores,
-// maximum, exponentials, transposed values) with one or two wavefronts per SIMD; keys and values come from the L2 a tile ahead.
-//   * S^T = K Q^T with v_mfma_f32_32x32x16_f16: keys are the A rows, queries the B columns, so a lane's 16 accumulators are 16 keys of
-//     one query.  Queries go in as hi + lo / 2048 (two products), fp32 keys as well (three: hi hi, lo hi, hi lo).
-//   * O^T += V^T P: a lane's softmax weights are its B fragment as they are.  They go in times 2^15 as a pair hi + lo at one scale (a
-//     weight is at most 1, so nothing overflows and what the pair leaves is below 2^-40), which needs one accumulator; fp32 values as hi + lo.
+// grid (query heads, tiles of 32 rows); a workgroup is KP wavefronts that share the 32 queries (in LDS) and deal the tiles of 32 keys
+// among themselves (wavefront p takes tiles p, p + KP, ...).  A wavefront runs by itself from its first tile to its last, without a barrier; the
+// KP states (maximum, sum, context) are merged pairwise through LDS at the end.  KP fills the chip where heads x row tiles do not
+// (launch_span_attention).
+//   * S^T = K Q^T and O^T += V^T P on 32 x 32 tiles: keys are the A rows, queries the B columns, so a lane's 16 accumulators are 16 keys of
+//     one query, and its softmax weights are the B operand of the second product as they are.
+//   * fp32 caches: v_mfma_f32_32x32x2_f32, fp32 fused multiply-adds throughout.  A lane's 16 bytes of a key row feed four products (the order of k
+//     is free as long as both operands agree); values come straight from memory, 32 dims of one key per half wavefront.  Bound by those
+//     products: 8192 cycles per tile of 128 dims.
+//   * fp16 caches hold keys and values exactly, so only the fp32 operands are split, each into three fp16 parts that add up to its 24 bits: a query scaled
+//     by a power of two that takes its largest value to 2^14..2^15, a softmax weight times 2^15 (parts end at 2^-25, so what they leave is below
+//     2^-39 of the largest).  Three v_mfma_f32_32x32x16_f16 into one fp32 sum take 96 cycles where the fp32 form takes 512.
+// A row whose result is not finite is done again from the keys it sees alone (plain_attention_row).
+// 512 rows of 24 heads of 128 (8 key/value heads) behind 1024: 70 us with fp16 caches, 160 with fp32 ones; row by row 780 (fp16).  Pairs of fp16 parts
+// (22 bits) in the place of the three took 53 and 98, but were less exact than the row by row kernel.
 // Query heads of a key/value head are x, x + kv_heads, ...: with eight key/value heads they share one L2.
 #include "../common.h"
+#include "attention_rows.h"
 #include "span_attention.h"
 
 namespace esp {
@@ -24,34 +29,24 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr float kMostHalf = 65504.0f;
-
-// v = hi + lo / 2048 (fp16 each); what fp16 cannot hold is cut to its largest value
-__device__ __forceinline__ void split8(const float4 &x0, const float4 &x1, half8 &hi, half8 &lo) {
-    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float c = __builtin_amdgcn_fmed3f(v[e], -kMostHalf, kMostHalf);
-        hi[e] = (_Float16)c;
-        lo[e] = (_Float16)__fmul_rn(__fsub_rn(c, (float)hi[e]), 2048.0f);
-    }
-}
-// the same without a scale on the second part: v = hi + lo to 22 bits or 2^-25, whichever is coarser
-__device__ __forceinline__ void split8_plain(const float4 &x0, const float4 &x1, half8 &hi, half8 &lo) {
-    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        hi[e] = (_Float16)v[e];
-        lo[e] = (_Float16)__fsub_rn(v[e], (float)hi[e]);
-    }
+// v = p[0] + p[1] + p[2] in element e, for |v| up to 2^15
+__device__ __forceinline__ void split3(float v, half8 (&p)[3], int e) {
+    p[0][e] = (_Float16)v;
+    const float rest = __fsub_rn(v, (float)p[0][e]);
+    p[1][e] = (_Float16)rest;
+    p[2][e] = (_Float16)__fsub_rn(rest, (float)p[1][e]);
 }
 
 template <int HD, bool KV_F16, int KP>
 __global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a, int rows) {
-    constexpr int KS = HD / 16, MT = HD / 32, LDV = 32 + 8, PLANES = KV_F16 ? 1 : 2, VP = HD / 16;   // VP: 8-dim pieces of a value tile per lane
-    constexpr int kTile = PLANES * HD * LDV;                                   // fp16 per wavefront
-    constexpr int kValueBytes = KP * kTile * 2, kMergeBytes = (KP / 2) * MT * 16 * 64 * 4;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kValueBytes > kMergeBytes ? kValueBytes : kMergeBytes];
+    constexpr int KS = HD / 16, MT = HD / 32, LDV = 32 + 8, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane
+    constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
+    constexpr int kQueryBytes = KV_F16 ? 3 * 32 * LDQ * 2 : 32 * LDQ * 4;
+    constexpr int kWave = KV_F16 ? HD * LDV * 2 : 0;                        // a value tile per wavefront
+    constexpr int kMergeBytes = KP > 1 ? (KP / 2) * MT * 16 * 64 * 4 : 16;
+    __shared__ __attribute__((aligned(16))) unsigned char query_mem[kQueryBytes];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[KP * kWave > kMergeBytes ? KP * kWave : kMergeBytes];
+    __shared__ int not_finite;
     __shared__ float state[KP][2][64];
     const int lane = threadIdx.x & 63, phase = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
     const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head;
@@ -60,35 +55,70 @@ __global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a
     const int pos0 = a.pos[m0], t_max = pos0 + last_row, kd = a.n_kv_head * HD;
     const size_t base = (size_t)a.seq[m0] * a.cache_seq_stride + (size_t)kvh * HD;
     const float scale = 1.0f / sqrtf((float)HD);
-    _Float16 *vt = reinterpret_cast<_Float16 *>(smem) + phase * kTile;
+    const int qpos = pos0 + col;
 
-    // queries: column = query `col` (rows beyond the block repeat its last row, never stored), dims 16 ks + 8 half ..
-    half8 qh[KS], ql[KS];
+    // query `col` (rows beyond the block repeat its last row, never stored)
+    const float *query = a.q + (size_t)(m0 + (col <= last_row ? col : last_row)) * a.n_head * HD + (size_t)head * HD;
+    _Float16 *q16 = reinterpret_cast<_Float16 *>(query_mem);                   // [3][32][LDQ]
+    float *q32 = reinterpret_cast<float *>(query_mem);                         // [32][LDQ]
+    int q_exp = 0;
     {
-        const float *qp = a.q + (size_t)(m0 + (col <= last_row ? col : last_row)) * a.n_head * HD + (size_t)head * HD + 8 * half;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) split8(*reinterpret_cast<const float4 *>(qp + 16 * ks), *reinterpret_cast<const float4 *>(qp + 16 * ks + 4), qh[ks], ql[ks]);
-    }
-    // A tile on its way: fp16 caches 8 values per 128-bit load, fp32 caches two loads.  Keys beyond t_max are clamped to it: in bounds, and masked.
-    constexpr int W = KV_F16 ? 1 : 2;
-    float4 kr[KS * W], vr[VP * W];
-    auto load = [&](int t0) {
-        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd + 8 * half;
+        float4 x[KS][2];   // dims 16 ks + 8 half ..
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-            for (int w = 0; w < W; w++)
-                kr[ks * W + w] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + kt + 16 * ks)
-                                        : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 16 * ks + 4 * w);
-        // a value tile's piece: key = lane % 32, dims 8 (lane / 32 + 2 i) ..: the transposed two-byte writes spread over the banks
+            for (int w = 0; w < 2; w++) x[ks][w] = *reinterpret_cast<const float4 *>(query + 16 * ks + 8 * half + 4 * w);
+        if constexpr (KV_F16) {
+            float most = 0.0f;
 #pragma unroll
-        for (int i = 0; i < VP; i++)
+            for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-            for (int w = 0; w < W; w++) {
-                const size_t o = kt - 8 * half + 8 * (half + 2 * i);
-                vr[i * W + w] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + o)
-                                       : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.v_cache) + o + 4 * w);
+                for (int w = 0; w < 2; w++) most = fmaxf(fmaxf(most, fmaxf(fabsf(x[ks][w].x), fabsf(x[ks][w].y))), fmaxf(fabsf(x[ks][w].z), fabsf(x[ks][w].w)));
+            most = fmaxf(most, __shfl_xor(most, 32));
+            q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks % KP != phase) continue;   // the wavefronts share the work; each has read the row for its exponent
+            if constexpr (KV_F16) {
+                const float v[8] = {x[ks][0].x, x[ks][0].y, x[ks][0].z, x[ks][0].w, x[ks][1].x, x[ks][1].y, x[ks][1].z, x[ks][1].w};
+                half8 p[3];
+#pragma unroll
+                for (int e = 0; e < 8; e++) split3(__builtin_amdgcn_ldexpf(v[e], q_exp), p, e);
+#pragma unroll
+                for (int i = 0; i < 3; i++) *reinterpret_cast<half8 *>(q16 + (i * 32 + col) * LDQ + 16 * ks + 8 * half) = p[i];
+            } else {
+#pragma unroll
+                for (int w = 0; w < 2; w++) *reinterpret_cast<float4 *>(q32 + col * LDQ + 16 * ks + 8 * half + 4 * w) = x[ks][w];
             }
+        }
+    }
+    __syncthreads();
+
+    // Keys beyond t_max are clamped to it: in bounds, and masked.  A lane's keys: row `col` of the tile, dims 16 ks + 8 half .. (fp16), 8 j + 4 half .. (fp32)
+    constexpr int NK = KV_F16 ? KS : HD / 8;
+    float4 kr[NK];
+    auto load_keys = [&](int t0) {
+        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
+#pragma unroll
+        for (int j = 0; j < NK; j++)
+            kr[j] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + kt + 16 * j + 8 * half)
+                           : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 8 * j + 4 * half);
+    };
+    // an fp16 value tile on its way to LDS: key = lane % 32, dims 8 (lane / 32 + 2 i) ..: the transposed two-byte writes spread over the banks
+    uint4 vr[KV_F16 ? VP : 1];
+    auto load_values = [&](int t0) {
+        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
+#pragma unroll
+        for (int i = 0; i < (KV_F16 ? VP : 0); i++) vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + kt + 8 * (half + 2 * i));
+    };
+    // fp32 values of dims 32 mt .. for the product's 16 steps: step r takes key 8 (r / 4) + 4 half + r % 4, the key of accumulator r
+    auto load_value_dims = [&](int t0, int mt, float (&v)[16]) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int t = t0 + 8 * (r >> 2) + 4 * half + (r & 3);
+            v[r] = reinterpret_cast<const float *>(a.v_cache)[base + (size_t)(t < t_max ? t : t_max) * kd + 32 * mt + col];
+        }
     };
 
     floatx16 o[MT];
@@ -97,82 +127,97 @@ __global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a
 #pragma unroll
         for (int r = 0; r < 16; r++) o[mt][r] = 0.0f;
     float mx = -INFINITY, l = 0.0f;
-    const int qpos = pos0 + col;
-    if (32 * phase <= t_max) load(32 * phase);
+    _Float16 *vt = reinterpret_cast<_Float16 *>(smem + phase * kWave);
+
+    if (32 * phase <= t_max) { load_keys(32 * phase); load_values(32 * phase); }
     for (int t0 = 32 * phase; t0 <= t_max; t0 += 32 * KP) {
-        floatx16 sc, sl;
+        float vd[KV_F16 ? 1 : 2][16];
+        if constexpr (!KV_F16) load_value_dims(t0, 0, vd[0]);
+        floatx16 s0;
 #pragma unroll
-        for (int r = 0; r < 16; r++) sc[r] = sl[r] = 0.0f;
+        for (int r = 0; r < 16; r++) s0[r] = 0.0f;
+        if constexpr (KV_F16) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            half8 kh, kl;
-            if constexpr (KV_F16) kh = __builtin_bit_cast(half8, kr[ks]);
-            else split8(kr[2 * ks], kr[2 * ks + 1], kh, kl);
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[ks], sc, 0, 0, 0);
-            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[ks], sl, 0, 0, 0);
-            if constexpr (!KV_F16) sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[ks], sl, 0, 0, 0);
-        }
-        // values of this tile into LDS, transposed; nobody else reads this stretch, and a wavefront's LDS operations keep their order
+            for (int ks = 0; ks < KS; ks++) {
+                const half8 k = __builtin_bit_cast(half8, kr[ks]);
+                const _Float16 *qp = q16 + col * LDQ + 16 * ks + 8 * half;
 #pragma unroll
-        for (int i = 0; i < VP; i++) {
-            half8 vh, vl;
-            if constexpr (KV_F16) vh = __builtin_bit_cast(half8, vr[i]);
-            else split8_plain(vr[2 * i], vr[2 * i + 1], vh, vl);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                vt[(8 * (half + 2 * i) + e) * LDV + col] = vh[e];
-                if constexpr (!KV_F16) vt[HD * LDV + (8 * (half + 2 * i) + e) * LDV + col] = vl[e];
+                for (int p = 2; p >= 0; p--) s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, *reinterpret_cast<const half8 *>(qp + p * 32 * LDQ), s0, 0, 0, 0);
+                if (KP == 8 && ks % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // two wavefronts per SIMD: query parts of two steps at a time
             }
+            // values of this tile into LDS, transposed; nobody else reads this stretch, and a wavefront's LDS operations keep their order
+#pragma unroll
+            for (int i = 0; i < VP; i++) {
+                const half8 v = __builtin_bit_cast(half8, vr[i]);
+#pragma unroll
+                for (int e = 0; e < 8; e++) vt[(8 * (half + 2 * i) + e) * LDV + col] = v[e];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            load_keys(t0 + 32 * KP);   // clamped beyond the last tile
+            load_values(t0 + 32 * KP);
+#pragma unroll
+            for (int r = 0; r < 16; r++) s0[r] = __builtin_amdgcn_ldexpf(s0[r], -q_exp);
+        } else {
+#pragma unroll
+            for (int j = 0; j < HD / 8; j++) {
+                const float4 q = *reinterpret_cast<const float4 *>(q32 + col * LDQ + 8 * j + 4 * half);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].x, q.x, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].y, q.y, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].z, q.z, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].w, q.w, s0, 0, 0, 0);
+            }
+            load_keys(t0 + 32 * KP);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        load(t0 + 32 * KP);   // clamped beyond the last tile
         // accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`
         float tile_max = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const int key = t0 + 8 * (r >> 2) + 4 * half + (r & 3);
-            const float s = __builtin_fmaf(sl[r], 1.0f / 2048.0f, sc[r]);
-            sc[r] = key <= qpos ? __fmul_rn(s, scale) : -INFINITY;
-            tile_max = fmaxf(tile_max, sc[r]);
+            s0[r] = t0 + 8 * (r >> 2) + 4 * half + (r & 3) <= qpos ? __fmul_rn(s0[r], scale) : -INFINITY;
+            tile_max = fmaxf(tile_max, s0[r]);
         }
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
         // a wavefront may see only masked keys of a query for a while: its state stays (-inf, 0, 0), exponents taken against 0
         const float m_new = fmaxf(mx, tile_max), m_ref = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = __expf(mx - m_ref);      // exp(-inf) = 0 on the first tile
-        float psum = 0.0f;
-        half8 ph[2], pl[2];
+        const float alpha = expf(mx - m_ref);      // exp(-inf) = 0 on the first tile
+        float psum = 0.0f, pr[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const float pr = __expf(sc[r] - m_ref);  // masked keys: exp(-inf) = 0
-            psum += pr;
-            const float big = __fmul_rn(pr, 32768.0f);
-            ph[r >> 3][r & 7] = (_Float16)big;
-            pl[r >> 3][r & 7] = (_Float16)__fsub_rn(big, (float)ph[r >> 3][r & 7]);
+            pr[r] = expf(s0[r] - m_ref);           // masked keys: exp(-inf) = 0
+            psum += pr[r];
         }
         l = __builtin_fmaf(l, alpha, psum);
         mx = m_new;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
+        if constexpr (KV_F16) {
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                // k slot (lane / 32, i) is key 16 j + 8 (i / 4) + 4 (lane / 32) + i % 4, the key of accumulator 8 j + i
-                const _Float16 *vrow = vt + (32 * mt + col) * LDV + 16 * j + 4 * half;
-                const half4 lo = *reinterpret_cast<const half4 *>(vrow), hi = *reinterpret_cast<const half4 *>(vrow + 8);
-                const half8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, ph[j], o[mt], 0, 0, 0);
-                o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[j], o[mt], 0, 0, 0);
-                if constexpr (!KV_F16) {
-                    const half4 lo2 = *reinterpret_cast<const half4 *>(vrow + HD * LDV), hi2 = *reinterpret_cast<const half4 *>(vrow + HD * LDV + 8);
-                    const half8 vf2 = {lo2[0], lo2[1], lo2[2], lo2[3], hi2[0], hi2[1], hi2[2], hi2[3]};
-                    o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf2, ph[j], o[mt], 0, 0, 0);
+                half8 p[3];
+#pragma unroll
+                for (int i = 0; i < 8; i++) split3(__fmul_rn(pr[8 * j + i], 32768.0f), p, i);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+                    // k slot (lane / 32, i) is key 16 j + 8 (i / 4) + 4 (lane / 32) + i % 4, the key of accumulator 8 j + i
+                    const _Float16 *vrow = vt + (32 * mt + col) * LDV + 16 * j + 4 * half;
+                    const half4 lo = *reinterpret_cast<const half4 *>(vrow), hi = *reinterpret_cast<const half4 *>(vrow + 8);
+                    const half8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+                    for (int i = 2; i >= 0; i--) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[i], o[mt], 0, 0, 0);
                 }
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                if (mt + 1 < MT) load_value_dims(t0, mt + 1, vd[(mt + 1) & 1]);
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vd[mt & 1][r], pr[r], o[mt], 0, 0, 0);
+            }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
     }
     l += __shfl_xor(l, 32);
     // the upper half of the wavefronts hands its states to the lower half, until wavefront 0 holds the sum of all
@@ -192,7 +237,7 @@ __global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a
         if (phase < s) {
             const float m1 = state[phase + s][0][lane], l1 = state[phase + s][1][lane];
             const float m_all = fmaxf(mx, m1), m_ref = m_all == -INFINITY ? 0.0f : m_all;
-            const float f0 = __expf(mx - m_ref), f1 = __expf(m1 - m_ref);
+            const float f0 = expf(mx - m_ref), f1 = expf(m1 - m_ref);
             l = __builtin_fmaf(l, f0, __fmul_rn(l1, f1));
             mx = m_all;
 #pragma unroll
@@ -201,16 +246,35 @@ __global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a
                 for (int r = 0; r < 16; r++) o[mt][r] = __builtin_fmaf(o[mt][r], f0, __fmul_rn(merge[((phase * MT + mt) * 16 + r) * 64 + lane], f1));
         }
     }
-    if (phase == 0 && col <= last_row) {
-        const float inv = 1.0f / __fmul_rn(l, 32768.0f);   // key 0 is visible to every query: l > 0
-        uint16_t *out = a.ctx_f16 + (size_t)(m0 + col) * a.n_head * HD + (size_t)head * HD;
+    if (phase == 0) {
+        float check = 0.0f;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; q4++)
-                *reinterpret_cast<half4 *>(out + 32 * mt + 8 * q4 + 4 * half) = half4{(_Float16)__fmul_rn(o[mt][4 * q4], inv), (_Float16)__fmul_rn(o[mt][4 * q4 + 1], inv),
-                                                                                       (_Float16)__fmul_rn(o[mt][4 * q4 + 2], inv), (_Float16)__fmul_rn(o[mt][4 * q4 + 3], inv)};
+            for (int r = 0; r < 16; r++) check = __builtin_fmaf(o[mt][r], 0.0f, check);
+        const bool odd = __any(!(check == 0.0f && l < INFINITY));   // NaN wherever an infinity or a NaN went in
+        if (lane == 0) not_finite = odd;
+        if (!odd) {
+            const float inv = 1.0f / (KV_F16 ? __fmul_rn(l, 32768.0f) : l);   // key 0 is visible to every query: l > 0
+            const size_t row = (size_t)(m0 + (col <= last_row ? col : last_row));
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                float s = 0.0f;
+#pragma unroll
+                for (int q4 = 0; q4 < 4; q4++) {
+                    const float v[4] = {__fmul_rn(o[mt][4 * q4], inv), __fmul_rn(o[mt][4 * q4 + 1], inv), __fmul_rn(o[mt][4 * q4 + 2], inv), __fmul_rn(o[mt][4 * q4 + 3], inv)};
+                    if (col <= last_row) s += store_context4(a, row * a.n_head * HD + (size_t)head * HD + 32 * mt + 8 * q4 + 4 * half, v);
+                }
+                if (a.ctx_hi) {
+                    s += __shfl_xor(s, 32);
+                    if (half == 0 && col <= last_row) store_context_sum(a, row, a.n_head * HD, head * (HD / 32) + mt, s);
+                }
+            }
+        }
     }
+    __syncthreads();
+    if (not_finite)
+        for (int i = phase; i <= last_row; i += KP) plain_attention_row<HD, KV_F16>(a, m0 + i, head);
 }
 
 template <int HD, bool KV_F16>
@@ -218,8 +282,8 @@ void launch_shape(const AttentionArgs &a, int rows, int sets, hipStream_t s) {
     const dim3 grid(a.n_head, (rows + 31) / 32);
     if (sets == 1) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 1>), grid, dim3(64), 0, s, a, rows);
     else if (sets == 2) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 2>), grid, dim3(128), 0, s, a, rows);
-    else if (sets == 4 || (!KV_F16 && HD == 128)) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 4>), grid, dim3(256), 0, s, a, rows);
-    else hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, (!KV_F16 && HD == 128) ? 4 : 8>), grid, dim3(512), 0, s, a, rows);
+    else if (sets == 4) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 4>), grid, dim3(256), 0, s, a, rows);
+    else hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 8>), grid, dim3(512), 0, s, a, rows);
 }
 
 }  // namespace
@@ -229,9 +293,10 @@ bool span_attention_supported(int n_head, int n_kv_head, int head_dim) {
 }
 
 hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, bool kv_f16, hipStream_t s) {
-    if (rows <= 0 || !a.ctx_f16 || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
+    if (rows <= 0 || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
+    if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
-    // A 512-row block of 24 heads gets four (36.9 us), its 241-row rest eight (36.3), 93 rows of 32 heads eight (13.4).
+    // 512 rows of 24 heads get four, 241 rows of them eight, 93 rows of 32 heads eight (fp16: 70 us behind 1024, 43 behind 1536, 15.7 of 64 dims behind 700).
     const int tiles = (keys + 31) / 32, groups = a.n_head * ((rows + 31) / 32);
     int sets = 1;
     while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;

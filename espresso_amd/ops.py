@@ -201,6 +201,21 @@ def hbm_read_probe_pairs(bytes_per_launch: int, pair_bytes: int = 2304, workgrou
     return {"mean_us": us.value, "gbps": gbps.value}
 
 
+ATTENTION_KERNELS = ("single_row", "prompt", "span")
+
+
+def block_attention(kernel: str, q: np.ndarray, k: np.ndarray, v: np.ndarray, split_rows: bool = False, iters: int = 1) -> tuple[np.ndarray, float]:
+    """(context, mean microseconds) of rows q [rows, heads, size] that follow each other behind the first keys of k, v [keys, kv heads, size], fp32 or
+    fp16 (esp_block_attention; test aid)."""
+    q, k, v = np.ascontiguousarray(q, dtype=np.float32), np.ascontiguousarray(k), np.ascontiguousarray(v)
+    if k.dtype != v.dtype or k.dtype not in (np.float32, np.float16) or k.shape != v.shape or k.shape[2] != q.shape[2] or k.shape[0] < q.shape[0]:
+        raise ValueError("block_attention: keys and values")
+    ctx, us = np.empty(q.shape, dtype=np.float32), C.c_double(0)
+    _lib.check(_lib.load_library().esp_block_attention(ATTENTION_KERNELS.index(kernel), _ptr(q), _ptr(k), _ptr(v), int(k.dtype == np.float16), q.shape[0],
+                                                       k.shape[0] - q.shape[0], q.shape[1], k.shape[1], q.shape[2], int(split_rows), _ptr(ctx), iters, C.byref(us)))
+    return ctx, us.value
+
+
 def synth_weights(fmt: int, seed: int, std: float, elements: int) -> np.ndarray:
     """Seeded N(0, std) weights quantised on the GPU into GGUF-layout blocks (uint8 array)."""
     L = _lib.load_library()

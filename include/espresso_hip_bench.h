@@ -55,6 +55,15 @@ long long esp_matrix_read_tiled(const ESPMatrix *matrix, void *out, size_t capac
  * (a mismatch fails the call); tuning key split_gemm_shared_k selects how
  * workgroups share an output tile's K range (0 never, 1 where it applies, 2 as 1 with the finishing workgroup never waiting). */
 int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, float *act);
+/* Test aid: causal attention of `rows` (up to 512) consecutive rows of one sequence at positions first, first + 1, ... by one of the kernels a model's
+ * layers use.  q [rows][heads][head_dim] fp32; k, v [first + rows][kv_heads][head_dim] fp32, or fp16 bits with kv_f16; ctx [rows][heads][head_dim]
+ * as fp32: the fp16 context, or with split_rows the two fp16 planes added back together (hi + lo / 2048).  Host pointers.  `iters` launches;
+ * *mean_us (may be NULL) is their mean time.  ESP_ERR_UNSUPPORTED for a shape the kernel is not written for. */
+#define ESP_ATTENTION_SINGLE_ROW 0   /* every row by itself */
+#define ESP_ATTENTION_PROMPT 1       /* prompt blocks, one, two or four query heads per key/value head */
+#define ESP_ATTENTION_SPAN 2         /* blocks of any head group */
+int esp_block_attention(int kernel, const float *q, const void *k, const void *v, int kv_f16, int rows, int first, int heads, int kv_heads, int head_dim,
+                        int split_rows, float *ctx, int iters, double *mean_us);
 int esp_hbm_read_probe(size_t bytes, int iters, double *gb_per_s);
 /* The ceiling for ONE GEMV launch: a kernel with a persistent Q4_K GEMV's grid (`workgroups` of `wavefronts` = 4 or 8) and its
  * loads (a wavefront takes items of `pair_bytes`, a 2304-byte weight tile of the matrix-core kernel or a pair of rows of the

@@ -1,0 +1,136 @@
+"""The block attention kernels by themselves, against 64 bits: how exact they are, and that a row meets only the keys it sees."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import espresso_amd.ops as ops
+    ops.init()
+    yield ops
+    ops.set_tuning("prompt_attention_key_sets", 0)
+
+
+def inputs(rows, first, heads, kv_heads, size, dtype, seed, sharp=1.0):
+    rng = np.random.default_rng(seed)
+    q = rng.normal(0, sharp, (rows, heads, size)).astype(np.float32)
+    return q, rng.normal(0, 1, (first + rows, kv_heads, size)).astype(dtype), rng.normal(0, 1, (first + rows, kv_heads, size)).astype(dtype)
+
+
+def exact(q, k, v):
+    rows, heads, size = q.shape
+    first, share = k.shape[0] - rows, heads // k.shape[1]
+    out = np.empty(q.shape)
+    for h in range(heads):
+        s = q[:, h].astype(np.float64) @ k[:, h // share].astype(np.float64).T / np.sqrt(size)
+        s[np.arange(k.shape[0])[None, :] > first + np.arange(rows)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = p / p.sum(1, keepdims=True) @ v[:, h // share].astype(np.float64)
+    return out
+
+
+# tiles of 32 rows and keys, prefixes that are whole tiles and not, one to eight wavefronts per tile
+SHAPES = [(1, 0, 3, 1, 128), (4, 0, 8, 8, 64), (31, 1, 8, 1, 64), (32, 32, 9, 3, 64), (33, 31, 6, 2, 128), (93, 700, 8, 2, 64), (97, 33, 4, 1, 128), (300, 0, 6, 2, 128), (512, 45, 6, 2, 128),
+          (256, 257, 32, 8, 64)]
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("rows,first,heads,kv_heads,size", SHAPES)
+def test_span_attention_is_as_exact_as_fp32(ops, rows, first, heads, kv_heads, size, dtype):
+    """Split rows carry 22 bits, so a context that fp32 sums are behind shows.  Scores of hundreds: rounding queries or keys to 22 bits moves a weight by
+    2^-23 times the score's terms, rounding them to fp16 by 2^-11."""
+    planes = heads * size % 256 == 0
+    for sharp in (1.0, 60.0):
+        q, k, v = inputs(rows, first, heads, kv_heads, size, dtype, rows + first, sharp)
+        want = exact(q, k, v)
+        got, _ = ops.block_attention("span", q, k, v, split_rows=planes)
+        one, _ = ops.block_attention("single_row", q, k, v)
+        # an fp32 sum of `size` products is off by about 2^-24 sqrt(size) of their root of squares, which is sharp after the scale 1 / sqrt(size); a weight by that much of
+        # itself, and the context by that much of the values' spread; planes end at 2^-22, fp16 at 2^-11 of the result
+        def off(c):
+            return np.sqrt(np.mean((c - want) ** 2))
+        assert off(got) <= 2.0 ** -24 * (np.sqrt(size) * sharp + 8) + 2.0 ** (-22 if planes else -11) * np.sqrt(np.mean(want ** 2)), sharp
+        if not planes:   # the same fp16 rounding on both sides: no worse than the kernel that does every row by itself
+            assert off(got) <= 1.02 * off(one) + 1e-9, sharp
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("scale", [2.0 ** -40, 2.0 ** -12, 2.0 ** 14, 2.0 ** 60])
+def test_span_attention_takes_queries_of_any_size(ops, scale, dtype):
+    q, k, v = inputs(40, 50, 6, 2, 128, dtype, 5)
+    k = (k / 64).astype(dtype)
+    if dtype == np.float32:
+        k = (k / np.float32(scale)).astype(np.float32)   # products of the same size as before
+        want = exact(q * np.float32(scale), k, v)
+    else:
+        want = exact(np.float32(q * np.float32(scale)), k, v)
+    got, _ = ops.block_attention("span", q * np.float32(scale), k, v, split_rows=True)
+    if dtype == np.float32 or scale < 1:
+        assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
+    else:   # one key takes everything, and which one hangs on a score's last bits where two are near: as many rows as with fp32 sums
+        one, _ = ops.block_attention("single_row", q * np.float32(scale), k, v)
+        near = [(np.abs(c - want).max(-1) <= 2.0 ** -11 * np.abs(want).max(-1)).mean() for c in (got, one)]
+        assert near[0] >= near[1] - 0.02 > 0.9
+
+
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("magnitude", [3e-7, 1e-3, 3e4, 3e8])
+def test_span_attention_takes_values_of_any_size(ops, magnitude, dtype):
+    if dtype == np.float16 and magnitude > 65504:
+        pytest.skip("beyond the cache's type")
+    q, k, v = inputs(70, 10, 6, 2, 128, dtype, 6)
+    v = np.clip(v * magnitude / 2, -65504 if dtype == np.float16 else None, 65504 if dtype == np.float16 else None).astype(dtype)
+    if magnitude > 65504:   # what adds up to a finite fp16 context
+        v[0::2, :, :] = v[0, :, :]
+        v[1::2, :, :] = -v[0, :, :]
+        q[:] = 0.0
+    want = exact(q, k, v)
+    fits = np.abs(want) < 65000
+    got, _ = ops.block_attention("span", q, k, v)
+    assert np.isfinite(got[fits]).all() and fits.mean() > 0.3
+    # fp16 ends at 2^-25 below its normal numbers; values cancel to an fp32 sum's 2^-22 of their size
+    assert (np.abs(got - want)[fits] <= 2.0 ** -11 * np.abs(want)[fits] + 2.0 ** -25 + 2.0 ** -22 * np.abs(v).max()).all()
+
+
+@pytest.mark.parametrize("kernel,heads,kv_heads,size,sets", [("span", 6, 2, 128, 0), ("span", 8, 1, 64, 0)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_what_a_row_does_not_see_does_not_reach_it(ops, kernel, heads, kv_heads, size, sets, dtype, bad):
+    """A value that is not finite poisons the rows that see it and no others; so does a key."""
+    rows, first, at = 75, 13, 60
+    ops.set_tuning("prompt_attention_key_sets", sets)
+    q, k, v = inputs(rows, first, heads, kv_heads, size, dtype, 7)
+    clean = exact(q, k, v)
+    limit = 2e-3 if kernel == "prompt" else 2.0 ** -11   # that kernel rounds operands to fp16
+    for which in (v, k):
+        kept = which[at, 0, 5]
+        which[at, 0, 5] = bad
+        for planes in ([False, True] if heads * size % 256 == 0 and (kernel == "span" or dtype == np.float16) else [False]):
+            got, _ = ops.block_attention(kernel, q, k, v, split_rows=planes)
+            unseen = got[:at - first]
+            assert np.isfinite(unseen).all()
+            assert np.abs(unseen - clean[:at - first]).max() <= limit * np.abs(clean).max()
+            share = heads // kv_heads
+            if which is v:
+                assert not np.isfinite(got[at - first:, :share, 5]).any()
+                rest = got[at - first:, :share, :5]
+                assert np.abs(rest - clean[at - first:, :share, :5]).max() <= limit * np.abs(clean).max()
+            else:   # a score of -inf is a key that counts for nothing; any other poisons
+                with np.errstate(all="ignore"):
+                    want = exact(q[at - first:, :share], k[:, :1], v[:, :1])
+                assert (np.isfinite(got[at - first:, :share]) == np.isfinite(want)).all()
+        which[at, 0, 5] = kept
+
+
+@pytest.mark.parametrize("kernel", ["span"])
+def test_fp32_values_beyond_fp16_that_add_up(ops, kernel):
+    """fp32 caches hold more than fp16: rows whose weighted sum fits come out finite."""
+    q, k, v = inputs(40, 9, 4, 2, 64, np.float32, 8)
+    q[:] = 0.0
+    v[:] = np.where(np.arange(49)[:, None, None] % 2 == 0, 9e4, -9e4)
+    want = exact(q, k, v)
+    got, _ = ops.block_attention(kernel, q, k, v)
+    assert np.abs(want).max() < 65504 and np.isfinite(got).all()
+    assert np.abs(got - want).max() <= 2.0 ** -11 * np.abs(want).max()

@@ -31,7 +31,7 @@ def test_prompt_block_matches_oracle(head_dim, n_head, n_kv, kv_fp16, prompt_len
     o = oracle()
     o.prefill([int(t) for t in prompt])
     g.prefill(prompt)
-    # fp16 activations into every product on both sides; the attention's own error (22-bit pairs) is far below their rounding
+    # fp16 activations into every product on both sides; the attention's own error (fp32 sums) is far below their rounding
     for _ in range(2):
         ho, hg = o.last_hidden(), g.last_hidden()
         assert np.abs(ho - hg).max() <= 2e-3 * max(1.0, np.abs(ho).max())
