@@ -6,6 +6,7 @@
 // inputs.  Products that the reference rounds separately are never contracted into fused
 // multiply-adds here (__fmul_rn / __fadd_rn / __fsub_rn).
 #include "../common.h"
+#include "attention_rows.h"
 #include "decode_ops.h"
 
 namespace esp {
@@ -500,8 +501,10 @@ typedef float attn_floatx16 __attribute__((ext_vector_type(16)));
 // KP = 2: the workgroup has two sets of G wavefronts; set p takes the key tiles p, p + 2, ... with value tiles of its own, and the two
 // (maximum, sum, context) states of a head are merged through LDS at the end.  A workgroup's time is the length of its chain of key
 // tiles (a tile of arithmetic is shorter than the trip to memory behind it), and the last row tile of a 512-row block has sixteen.
+// Heads of 64 dims ask for two wavefronts per SIMD: without it the compiler spreads over accumulator registers past what two share (512 rows of 32
+// heads behind 512, split rows: 49 us, 44 with it).
 template <int HD, int G, bool KV_F16, bool SPLIT, int KP>
-__global__ __launch_bounds__(G * KP * 64) void attention_prompt_kernel(AttentionArgs a, int rows) {
+__global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_prompt_kernel(AttentionArgs a, int rows) {
     constexpr int THREADS = G * 64, QT = 32, KS = HD / 16, MTILES = HD / 32, LDV = 32 + 8;   // THREADS: of one set; LDV: fp16 per row of V^T
     constexpr int VP = 32 * (HD / 8) / THREADS;                                            // 8-dim pieces of V per thread
     static_assert(VP >= 1 && 32 * (HD / 8) % THREADS == 0, "value tile divides over a set of wavefronts");
@@ -705,6 +708,16 @@ __global__ __launch_bounds__(G * KP * 64) void attention_prompt_kernel(Attention
         if (phase == 1) return;
     }
     l += __shfl_xor(l, 32);
+    // A masked key takes part with weight 0, and fp16 ends at 65504: where something was not finite, the rows once more from the keys they see alone
+    float check = 0.0f;
+#pragma unroll
+    for (int mt = 0; mt < MTILES; mt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) check = __builtin_fmaf(SPLIT ? o[mt][r] + ol[mt][r] : o[mt][r], 0.0f, check);
+    if (__any(!(check == 0.0f && l < INFINITY))) {
+        for (int i = 0; i <= last_row; i++) plain_attention_row<HD, KV_F16>(a, m0 + i, head);
+        return;
+    }
     if constexpr (SPLIT) {
         // context = (o + ol / 2048) / l as split rows; dims 32 mt .. 32 mt + 31 of a head are one sub-block of the row, half of it in
         // this lane and half in lane ^ 32
@@ -716,28 +729,13 @@ __global__ __launch_bounds__(G * KP * 64) void attention_prompt_kernel(Attention
             float s = 0.0f;
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
-                attn_half4 vh, vl;
+                float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float v = __fmul_rn(__builtin_fmaf(ol[mt][4 * q4 + e], 1.0f / 2048.0f, o[mt][4 * q4 + e]), inv);
-                    vh[e] = (_Float16)v;
-                    vl[e] = (_Float16)__fmul_rn(__fsub_rn(v, (float)vh[e]), 2048.0f);
-                    s += __builtin_fmaf((float)vl[e], 1.0f / 2048.0f, (float)vh[e]);
-                }
-                if (col <= last_row) {   // the planes' order inside fours: (0, 2, 1, 3)
-                    const size_t o16 = row * ad + (size_t)head * HD + 32 * mt + 8 * q4 + 4 * half;
-                    *reinterpret_cast<attn_half4 *>(a.ctx_hi + o16) = attn_half4{vh[0], vh[2], vh[1], vh[3]};
-                    *reinterpret_cast<attn_half4 *>(a.ctx_lo + o16) = attn_half4{vl[0], vl[2], vl[1], vl[3]};
-                }
+                for (int e = 0; e < 4; e++) v[e] = __fmul_rn(__builtin_fmaf(ol[mt][4 * q4 + e], 1.0f / 2048.0f, o[mt][4 * q4 + e]), inv);
+                if (col <= last_row) s += store_context4(a, row * ad + (size_t)head * HD + 32 * mt + 8 * q4 + 4 * half, v);
             }
             s += __shfl_xor(s, 32);
-            if (half == 0 && col <= last_row) {
-                const int sub = head * (HD / 32) + mt;
-                uint16_t *p = a.ctx_sums + (row * (size_t)(ad / 256) + (sub >> 3)) * 16 + (sub & 7);
-                const _Float16 h = (_Float16)s;
-                p[0] = __builtin_bit_cast(uint16_t, h);
-                p[8] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(__fsub_rn(s, (float)h), 2048.0f));
-            }
+            if (half == 0 && col <= last_row) store_context_sum(a, row, ad, head * (HD / 32) + mt, s);
         }
         return;
     }

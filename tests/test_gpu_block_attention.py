@@ -94,7 +94,8 @@ def test_span_attention_takes_values_of_any_size(ops, magnitude, dtype):
     assert (np.abs(got - want)[fits] <= 2.0 ** -11 * np.abs(want)[fits] + 2.0 ** -25 + 2.0 ** -22 * np.abs(v).max()).all()
 
 
-@pytest.mark.parametrize("kernel,heads,kv_heads,size,sets", [("span", 6, 2, 128, 0), ("span", 8, 1, 64, 0)])
+@pytest.mark.parametrize("kernel,heads,kv_heads,size,sets", [("span", 6, 2, 128, 0), ("span", 8, 1, 64, 0), ("prompt", 8, 2, 128, 1), ("prompt", 8, 2, 128, 2), ("prompt", 2, 2, 64, 1),
+                                                             ("prompt", 4, 2, 64, 1)])
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 def test_what_a_row_does_not_see_does_not_reach_it(ops, kernel, heads, kv_heads, size, sets, dtype, bad):
@@ -124,7 +125,7 @@ def test_what_a_row_does_not_see_does_not_reach_it(ops, kernel, heads, kv_heads,
         which[at, 0, 5] = kept
 
 
-@pytest.mark.parametrize("kernel", ["span"])
+@pytest.mark.parametrize("kernel", ["span", "prompt"])
 def test_fp32_values_beyond_fp16_that_add_up(ops, kernel):
     """fp32 caches hold more than fp16: rows whose weighted sum fits come out finite."""
     q, k, v = inputs(40, 9, 4, 2, 64, np.float32, 8)
