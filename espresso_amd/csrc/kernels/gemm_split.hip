@@ -21,6 +21,7 @@
 // Per 256 k a wavefront issues 128 + 4 MFMAs and about 200 fold operations.
 #include "../common.h"
 #include "decode_ops.h"
+#include "silu.h"
 #include <atomic>
 #include <mutex>
 #include <cmath>
@@ -366,8 +367,7 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_kernel(SplitGemmArgs 
                     const int r = 2 * k + (odd ? 1 : 0);
                     const int m = m0 + (wm * 2 + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     if (m < a.M && (n | 1) < a.N) {
-                        const float silu = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));   // = 0.5 g (1 + tanh(0.5 g)), a fifth of tanhf's instructions
-                        const float act = __fmul_rn(silu, up);
+                        const float act = __fmul_rn(silu(g), up);
                         const _Float16 hi = (_Float16)act;
                         const int unit = n / 2, slot = unit & 3;   // the planes' order inside fours: (0, 2, 1, 3)
                         const size_t o = (size_t)m * (a.N / 2) + (unit & ~3) + (slot == 1 ? 2 : slot == 2 ? 1 : slot);
@@ -767,9 +767,8 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
     // accumulator r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of the 32 x 32 tile
     if (a.sw_hi) {
         // SiLU(gate) * up of the workgroup's units (128 x 128 for a whole tile) as the two fp16 planes, through LDS (free now) so that the planes leave
-        // in whole 16-byte pieces of a row: [plane][MT rows][kActLd].  SiLU as g / (1 + exp(-g)) (the form of Sources/CPUOps/SiLU.swift:5-8):
-        // the same function as the 0.5 g (1 + tanh(0.5 g)) of RealModelInferenceEngine.swift:6825-6827 that the single-row kernels keep, a fifth of the instructions (this epilogue measured 10 us per
-        // output tile with tanhf and two-byte stores, a fifteenth of the tile's time).
+        // in whole 16-byte pieces of a row: [plane][MT rows][kActLd] (this epilogue measured 10 us per output tile with tanhf and two-byte stores, a
+        // fifteenth of the tile's time).
         constexpr int UN = NT2 / 2, RP = UN / 8, kActLd = UN + 16;   // units and pieces of a row; halfs per staged row: consecutive rows eight LDS banks apart
         uint16_t *act_hi = reinterpret_cast<uint16_t *>(smem_raw), *act_lo = act_hi + MT * kActLd;
         const bool odd = lane & 1;
@@ -786,8 +785,7 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
                     const float p0 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, a0), 0xB1, 0xF, 0xF, false));
                     const float p1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, a1), 0xB1, 0xF, 0xF, false));
                     const float g = odd ? p1 : a0, up = odd ? a1 : p0;
-                    const float silu = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
-                    const float act = __fmul_rn(silu, up);
+                    const float act = __fmul_rn(silu(g), up);
                     const _Float16 hi = (_Float16)act;
                     const int o = (row0 + 8 * (k >> 1) + 2 * (k & 1)) * kActLd + col;   // row 8 (r / 4) + r % 4 of the block, r = 2 k (+ 1)
                     act_hi[o] = __builtin_bit_cast(uint16_t, hi);

@@ -15,6 +15,7 @@
 //     Q8_0, Q4_K: 32 p + 16 h + 8 i; fp16 and (after the two halves of a wavefront exchanged half of two blocks) Q4_0: 32 p + 16 i + 8 h.
 #include "../common.h"
 #include "rows_gemm.h"
+#include "silu.h"
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
@@ -295,8 +296,7 @@ __global__ __launch_bounds__(kWaves * 64) void rows_gemm_kernel(RowsArgs a) {
             const float g = odd ? p1 : sum[k], up = odd ? sum[k + 1] : p0;
             const int q = wave * kShare + k + (odd ? 1 : 0), r = q & 15, m = m0 + 32 * (q >> 4) + 8 * (r >> 2) + 4 * h + (r & 3);
             if (m < a.M && (n | 1) < a.N) {
-                const float silu = g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));   // = 0.5 g (1 + tanh(0.5 g))
-                a.act[(size_t)m * (a.N / 2) + n / 2] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(silu, up));
+                a.act[(size_t)m * (a.N / 2) + n / 2] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(silu(g), up));
             }
         }
         return;

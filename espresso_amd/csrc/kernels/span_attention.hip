@@ -38,7 +38,7 @@ __device__ __forceinline__ void split3(float v, half8 (&p)[3], int e) {
 }
 
 template <int HD, bool KV_F16, int KP>
-__global__ __launch_bounds__(KP * 64) void span_attention_kernel(AttentionArgs a, int rows) {
+__global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kernel(AttentionArgs a, int rows) {
     constexpr int KS = HD / 16, MT = HD / 32, LDV = 32 + 8, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane
     constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
     constexpr int kQueryBytes = KV_F16 ? 3 * 32 * LDQ * 2 : 32 * LDQ * 4;

@@ -44,6 +44,34 @@ def test_narrow_split_gemm_matches_float64(mods, form, rows, cols):
     m.close()
 
 
+@pytest.mark.parametrize("cols", [256, 1024])   # weights staged through LDS, and read in the tiled order
+@pytest.mark.parametrize("form", [0, 1, 2, 4])
+def test_silu_is_exact_to_its_split_rows(mods, cols, form):
+    """Gates and ups that the product holds exactly (weights 0 and 1), so that only SiLU and the 22 bits of the planes are left."""
+    _, ops, _ = mods
+    units, n = 64, 31
+    block = np.zeros((2 * units, cols // 256, 144), np.uint8)
+    block[:, :, 0:2] = np.frombuffer(np.float16(0.125).tobytes(), np.uint8)
+    block[:, :, 4:8] = block[:, :, 12:16] = 1                      # every sub-block's scale 1, every minimum 0
+    for u in range(units):
+        block[2 * u, 0, 16 + u % 32] = 8 << 4 * (u // 32)          # gate = x[u]
+        block[2 * u + 1, 0, 16 + 127] = 8 << 4                     # up = x[255]
+    m = ops.Matrix(lib.FORMAT_Q4_K, block, 2 * units, cols)
+    x = np.zeros((n, cols), np.float32)
+    x[:, :units] = np.round(np.linspace(-16, 16, n * units) * 1024).reshape(n, units) / 1024
+    x[:, 255] = 1024
+    g = x[:, :units].astype(np.float64)
+    want = 1024 * g / (1 + np.exp(-g))
+    try:
+        ops.set_tuning("split_gemm_narrow", form)
+        got = m.matmul_f32_swiglu(x)
+    finally:
+        ops.set_tuning("split_gemm_narrow", -1)
+    # expf 2^-23, sum, quotient and product 2^-24 each, planes 2^-23
+    assert (np.abs(got - want) <= 3.5 * 2.0 ** -23 * np.abs(want) + 1e-12).all(), np.nanmax(np.abs(got - want) / np.maximum(np.abs(want), 1e-9))
+    m.close()
+
+
 # column counts of the sixteen-row kernel: d_model and attention width, hidden size
 @pytest.mark.parametrize("fmt,d,hidden,kv_fp16", [(orc.FMT_Q4_K, 1024, 2048, True), (orc.FMT_Q4_K, 2048, 3072, False), (orc.FMT_Q4_K, 3072, 8192, True),
                                                   (orc.FMT_Q4_K, 4096, 14336, True), (orc.FMT_Q4_0, 4096, 14336, False),
