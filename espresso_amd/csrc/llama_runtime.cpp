@@ -508,7 +508,8 @@ int LlamaRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int b
 // d_pos_/d_seq_, every projection as one dequant-fused MFMA GEMM.  Rows that are one sequence at consecutive positions
 // (a prompt block) take a matrix-core attention kernel, others the single-query one.
 // Prompt blocks of Q4_K models: every projection with exact weights and split activations (launch_gemm_split), queries and softmax
-// weights split in the attention: the block then stays as close to the fp32 CPU walk as the decode steps do.
+// weights as pairs (in short blocks, which single-row steps could walk as well, 32-bit) in the attention: the block then stays as close to the fp32 CPU walk as
+// the decode steps do.
 bool LlamaRuntime::split_blocks_supported() const {
     if (!split_activations_ || !xn_lo_ || !prompt_attention_ || c_.kv_format != FMT_F16 || c_.d_model > 8192) return false;
     for (const Layer &L : layers_)
@@ -516,11 +517,13 @@ bool LlamaRuntime::split_blocks_supported() const {
     return true;
 }
 
-// Blocks that carry activations and weights as exactly as the single-row steps do pay from the fourth token on (8B: a block of 4..32 tokens
-// costs 3.4 steps per layer, 1B: 3); blocks of the other formats round what the steps do not, so short prompts keep the steps.
+// Short blocks that carry activations, weights and attention as exactly as the single-row steps do pay from the fourth token on (8B: a block of 4..32
+// tokens costs 3.4 steps per layer, 1B: 3); blocks of the other formats round what the steps do not, so short prompts keep the steps.  Distance of the last hidden
+// row from 64 bits, 5 / 13 / 24 / 31 tokens, 1B: blocks 8.3 / 5.8 / 4.6 / 4.0e-5, steps 8.4 / 6.2 / 4.9 / 4.9e-5; four layers of 8B: 2.37 / 2.16 / 2.01 / 1.85e-4 and
+// 2.40 / 2.22 / 2.03 / 1.88e-4 (fp16 caches and contexts).
 int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : kMatrixPrefillMinTokens; }
 
-int LlamaRuntime::enqueue_layers_split(int rows) {
+int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
     hipStream_t s = context().stream;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const size_t cache_seq_stride = (size_t)kd * c_.max_seq;
@@ -552,7 +555,8 @@ int LlamaRuntime::enqueue_layers_split(int rows) {
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_hi = ctx.hi; aa.ctx_lo = ctx.lo; aa.ctx_sums = ctx.sums;
-        ESP_HIP_TRY(launch_attention_prompt(aa, rows, true, s));
+        if (rows < kMatrixPrefillMinTokens) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, true, s));
+        else ESP_HIP_TRY(launch_attention_prompt(aa, rows, true, s));
         g.w = L.wo; g.x = ctx; g.y = hidden_; g.residual = hidden_; splits = 1;
         ESP_HIP_TRY(launch_gemm_split(g, s));
         ESP_HIP_TRY(norm(L.rms_ffn, splits));
@@ -570,7 +574,7 @@ int LlamaRuntime::enqueue_layers_split(int rows) {
 
 // block_keys: the keys that the last row of a prompt block sees; 0 for rows that are not one sequence at consecutive positions.
 int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
-    if (block_keys && split_blocks_supported()) return enqueue_layers_split(rows);
+    if (block_keys && split_blocks_supported()) return enqueue_layers_split(rows, block_keys);
     hipStream_t s = context().stream;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const bool kv16 = c_.kv_format == FMT_F16;

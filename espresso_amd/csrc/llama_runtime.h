@@ -116,7 +116,7 @@ class LlamaRuntime : public DecoderRuntime {
     // prompt blocks with split activations: the lo planes and sub-block sums beside xn_, ctx_ and act_ (SplitRowsView)
     uint16_t *xn_lo_ = nullptr, *ctx_lo_ = nullptr, *act_lo_ = nullptr, *xn_sums_ = nullptr, *ctx_sums_ = nullptr, *act_sums_ = nullptr;
     bool split_blocks_supported() const;
-    int enqueue_layers_split(int rows);
+    int enqueue_layers_split(int rows, int block_keys);
     size_t weight_bytes_ = 0, resident_weight_bytes_ = 0;
     DeviceLoopSession loop_session_;
     bool fused_head_argmax_ = true;      // ESPRESSO_HIP_FUSED_HEAD_ARGMAX=0: head GEMV stores logits, separate arg-max launches
