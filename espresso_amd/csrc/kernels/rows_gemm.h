@@ -1,4 +1,4 @@
-// Products of a few to about a hundred activation rows in one launch (kernels/rows_gemm.hip).
+// Small products in one launch (kernels/rows_gemm.hip).
 #pragma once
 
 #include "../common.h"

@@ -25,7 +25,9 @@ def test_products_match_float64(ops, fmt, rows, cols):
     f = lib.FORMAT_NAMES[fmt]
     m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
     w = m.dequantize().astype(np.float64)
+    rounded = m.dequantize().astype(np.float16).astype(np.float64)
     rng = np.random.default_rng(cols)
+    off, off_rounded = [], []
     for batch in (3, 8, 9, 16, 17, 32, 33, 65):
         x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
         residual = rng.normal(0, 1, (batch, rows)).astype(np.float32) if batch % 2 else None
@@ -36,6 +38,18 @@ def test_products_match_float64(ops, fmt, rows, cols):
         if fmt == "q4_k":   # scale * q and the minimum are summed apart: up to twice 63 * 15 steps of the super-block's scale each
             bound = bound * 16
         assert (np.abs(m.gemv(x, residual) - want) <= bound).all(), batch
+        # relative to the products' root of squares, which is what rounding each of them adds up to
+        spread = np.sqrt((x.astype(np.float64) ** 2) @ (w ** 2).T) + 1e-30
+        x64 = x.astype(np.float64)
+        off.append(((m.gemv(x) - x64 @ w.T) / spread).ravel())
+        off_rounded.append(((x64 @ rounded.T - x64 @ w.T) / spread).ravel())
+    # No weight is rounded: what is left is the fp32 sums' 2^-24 per addition (a lane's chain is an eighth of the row and one sum per block), eight times
+    # that in Q4_K's two opposite sums.  fp16-rounded weights are off by 2^-12 / sqrt(3) each, 2^8 times the bound, wherever a weight has more than fp16's bits.
+    rms = lambda parts: np.sqrt(np.mean(np.concatenate(parts) ** 2))  # noqa: E731
+    limit = 2.0 ** -20 if fmt == "q4_k" else 2.0 ** -22
+    assert rms(off) <= limit, rms(off)
+    if fmt != "f16":
+        assert rms(off_rounded) > 8 * limit, rms(off_rounded)
     m.close()
 
 
