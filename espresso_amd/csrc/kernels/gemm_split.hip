@@ -1065,13 +1065,24 @@ static int regb_shape_setting() {
 //   1B, gate|up 64 / 128 / 256 / 512 rows 66 / 66 / 68 / 80 -> 26 / 31 / 48 / 76, whole layers 152 / 171 / 186 / 232 -> 83 / 99 / 135 / 210
 // (whole layers: the whole form with splits of 256 columns and more, which is already faster than the splits of 1024 it had before:
 // 1B 64 / 512 rows 200 / 265)
+static int device_compute_units() {   // 0: the device does not say
+    static std::atomic<int> cus[64];
+    int device = 0, n = 0;
+    if (hipGetDevice(&device) != hipSuccess) return 0;
+    n = cus[device & 63].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+        cus[device & 63].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
 struct RegBForm { int narrow, splits; };
 static int g_regb_narrow = -1;   // -1: the rule; 0: never narrow; 1, 2, 4: always that form (tests, measurements)
 void gemm_split_set_narrow(int form) { g_regb_narrow = form == 0 || form == 1 || form == 2 || form == 4 ? form : -1; }
 static RegBForm regb_form(int rows, int n, int k, bool may_split, size_t workspace_floats, bool shares_k) {
     struct Form { int rb, cb; float alone, shared; };
     static const Form forms[] = {{1, 1, 0.75f, 0.39f}, {2, 1, 0.9f, 0.64f}, {4, 1, 1.3f, 1.42f}, {4, 2, 1.95f, 2.35f}};
-    const int tiles = k / KT;
+    const int tiles = k / KT, cus = device_compute_units() > 0 ? device_compute_units() : 256;
     RegBForm best{0, 1};
     if (shares_k && g_regb_narrow <= 0) return best;
     float best_us = INFINITY;
@@ -1083,8 +1094,8 @@ static RegBForm regb_form(int rows, int n, int k, bool may_split, size_t workspa
         for (int splits = 1; splits <= (may_split ? tiles / 4 : 1); splits++) {
             if (splits > 1 && (size_t)splits * rows * n > workspace_floats) break;
             const int per = ((tiles + splits - 1) / splits + 3) & ~3;
-            const long groups = blocks * ((tiles + per - 1) / per), on_one = (groups + 255) / 256;
-            float tile_us = on_one > 1 || (!narrow && groups > 128) ? on_one * f.shared : f.alone;
+            const long groups = blocks * ((tiles + per - 1) / per), on_one = (groups + cus - 1) / cus;
+            float tile_us = on_one > 1 || (!narrow && 2 * groups > cus) ? on_one * f.shared : f.alone;
             if (narrow && tile_us < f.alone + 0.12f * (on_one - 1)) tile_us = f.alone + 0.12f * (on_one - 1);
             const float us = 3.0f + per * tile_us + (splits > 1 ? 1.0f + (float)splits * rows * n * 8 / 4e6f : 0.0f);
             if (us < best_us) { best_us = us; best = {narrow, splits}; }
@@ -1100,14 +1111,7 @@ bool gemm_split_supported(const DeviceMatrix &w) { return w.format == FMT_Q4_K &
 // per compute unit, each with the same number of K tiles.  Their number, or 0 where they do not apply.
 static int shared_k_workgroups_for(const GemmSplitParams &p, int tiles) {
     if (regb_shape_setting() != 4 || shared_k_mode() == 0 || !p.shared_k || !p.shared_k->flags || !p.shared_k->partial) return 0;
-    static std::atomic<int> cus[64];
-    int device = 0, n = 0;
-    if (hipGetDevice(&device) != hipSuccess) return 0;
-    n = cus[device & 63].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
-        cus[device & 63].store(n, std::memory_order_relaxed);
-    }
+    const int n = device_compute_units();
     const int blocks = ((p.w.rows + regb_tile_n(4, 2) - 1) / regb_tile_n(4, 2)) * ((p.rows + regb_tile_m(4, 2) - 1) / regb_tile_m(4, 2));
     const long long units = (long long)blocks * tiles;
     const bool applies = n > 0 && n <= kStreamKMaxWorkgroups && blocks > n && blocks % n != 0 && units % n == 0 && (units / n) % 4 == 0 && units / n >= tiles &&
