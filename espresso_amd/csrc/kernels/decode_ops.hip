@@ -1385,7 +1385,9 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
                          a.cache_seq_stride <= 0xFFFFFFFFull && a.n_head <= 0xFFFF;
     // Contexts of up to 512 tokens: the kernel of the single-row step, whose four slices of a head cover them in two passes (sixteen
     // sequences of the 8B model, attention + merge of a layer: prefix 60-84 of 512 8.4 + 6.6 -> 6.4 + 4.8 us, 384 of 512 14.4 + 6.6 -> 12.7 + 4.9;
-    // 768 of 1024 19.5 + 6.7 against 21.4 + 4.9, 3072 of 4096 55.7 + 6.6 against 65.9 + 4.9: those keep the kernel that reads a key once per group).
+    // 768 of 1024 19.5 + 6.7 against 21.4 + 4.9, 3072 of 4096 55.7 + 6.6 against 65.9 + 4.9: those keep the kernel that reads a key once per group).  Whole layers of
+    // three to sixteen sequences, contexts of 128, 256 and 512, fp16 and fp32 caches: 12 over 12 heads of 64 2 to 3 us less of 36 to 50, 32 over 8 of 64 0.5 to 4 of 43 to 58, 16 over 16 and
+    // over 8 of 128 1.5 to 4 of 43 to 70, 32 over 8 of 128 3 to 7 of 93 to 124.  The line lies at the context's size, not at the prefix's: a captured step replays the kernel.
     if (a.n_head % a.n_kv_head == 0 && !(by_head && a.max_seq <= 512)) {
         if (a.head_dim == 128) {
             if (group == 1) return launch_attention_gqa<128, 1>(a, rows, kv_f16, s);
