@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     constexpr bool kFours = FMT == FMT_F32 && MODE == 0;
     using Group = std::conditional_t<kFours, uint2, uint4>;
     constexpr int KS = kFours ? 4 : 2;                                     // groups per thread in registers (MODE 0 and 1)
-    const int per_row = cols / (kFours ? 4 : 8), last_group = per_row - 1;
+    const int per_row = cols / (kFours ? 4 : 8), last_group = per_row > 1 ? per_row - 1 : 0;
     float4 nv0[MODE == 1 ? B : 1][KS], nv1[MODE == 1 ? B : 1][KS], ng0[KS], ng1[KS];
     Group xv0[MODE == 0 ? B : 1][KS];
     if constexpr (MODE != 2) {
@@ -452,10 +452,11 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     {
         __shared__ float norm_red[B * kWaves];
         Group *dst = reinterpret_cast<Group *>(xs);
-        auto put = [&](int b, int g, const Group &v) {
-            if constexpr (T::kPermuteX) dst[(size_t)b * per_row + g] = swap_middle(v);
-            else dst[(size_t)b * per_row + g] = v;
+        auto ordered = [](const Group &v) -> Group {
+            if constexpr (T::kPermuteX) return swap_middle(v);
+            else return v;
         };
+        auto put = [&](int b, int g, const Group &v) { dst[(size_t)b * per_row + g] = ordered(v); };
 #pragma unroll
         for (int b = 0; b < B; b++) {
             float inv = 0.0f;
