@@ -15,7 +15,7 @@
 //     by a power of two that takes its largest value to 2^14..2^15, a softmax weight times 2^15 (parts end at 2^-25, so what they leave is below
 //     2^-39 of the largest).  Three v_mfma_f32_32x32x16_f16 into one fp32 sum take 96 cycles where the fp32 form takes 512.
 // A row whose result is not finite is done again from the keys it sees alone (plain_attention_row).
-// 512 rows of 24 heads of 128 (8 key/value heads) behind 1024: 70 us with fp16 caches, 160 with fp32 ones; row by row 780 (fp16).  Pairs of fp16 parts
+// 512 rows of 24 heads of 128 (8 key/value heads) behind 1024: 58 us with fp16 caches, 137 with fp32 ones; row by row 780 (fp16).  Pairs of fp16 parts
 // (22 bits) in the place of the three took 53 and 98, but were less exact than the row by row kernel.
 // Query heads of a key/value head are x, x + kv_heads, ...: with eight key/value heads they share one L2.
 #include "../common.h"
@@ -37,8 +37,21 @@ __device__ __forceinline__ void split3(float v, half8 (&p)[3], int e) {
     p[2][e] = (_Float16)__fsub_rn(rest, (float)p[1][e]);
 }
 
+// e^x for x <= 0: the hardware's 2^t at the rounded t = x log2(e), times 1 + what the rounding left of it.  Within 2^-22 of e^x for results above 2^-126 (smaller ones are
+// 0, and count for nothing beside the largest weight's 1); e^-inf = 0, e^NaN = NaN.  Half of expf's instructions, of which a tile has sixteen a lane.
+__device__ __forceinline__ float exp_weight(float x) {
+    const float c = x < -128.0f ? -128.0f : x;
+    const float log2e = 1.44269504f, t = __fmul_rn(c, log2e), left = __builtin_fmaf(c, 1.92596299e-8f, __builtin_fmaf(c, log2e, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(e, __fmul_rn(left, 0.693147181f), e);
+}
+
+// Two wavefronts per SIMD where the registers (without copies to accumulator registers) and the LDS of one wavefront allow it: a tile of an fp16 cache is more vector work
+// than matrix work, and one wavefront's hides under the other's.
+constexpr int span_waves_per_simd(int hd, bool kv_f16, int kp) { return hd == 64 || (kv_f16 && kp > 1) ? 2 : 1; }
+
 template <int HD, bool KV_F16, int KP>
-__global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kernel(AttentionArgs a, int rows) {
+__global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void span_attention_kernel(AttentionArgs a, int rows) {
     constexpr int KS = HD / 16, MT = HD / 32, LDV = 32 + 8, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane
     constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
     constexpr int kQueryBytes = KV_F16 ? 3 * 32 * LDQ * 2 : 32 * LDQ * 4;
@@ -54,16 +67,37 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
     const int last_row = rows - 1 - m0 < 31 ? rows - 1 - m0 : 31;
     const int pos0 = a.pos[m0], t_max = pos0 + last_row, kd = a.n_kv_head * HD;
     const size_t base = (size_t)a.seq[m0] * a.cache_seq_stride + (size_t)kvh * HD;
-    const float scale = 1.0f / sqrtf((float)HD);
+    float scale = 1.0f / sqrtf((float)HD);   // fp16 caches: of the scaled queries
     const int qpos = pos0 + col;
+
+    // Keys beyond t_max are clamped to it: in bounds, and masked.  A lane's keys: row `col` of the tile, dims 16 ks + 8 half .. (fp16), 8 j + 4 half .. (fp32)
+    constexpr int NK = KV_F16 ? KS : HD / 8;
+    float4 kr[NK];
+    auto load_keys = [&](int t0) {
+        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
+#pragma unroll
+        for (int j = 0; j < NK; j++)
+            kr[j] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + kt + 16 * j + 8 * half)
+                           : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 8 * j + 4 * half);
+    };
+    // an fp16 value tile on its way to LDS: key = lane % 32, dims 8 (lane / 32 + 2 i) ..: the transposed two-byte writes spread over the banks
+    uint4 vr[KV_F16 ? VP : 1];
+    auto load_values = [&](int t0) {
+        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
+#pragma unroll
+        for (int i = 0; i < (KV_F16 ? VP : 0); i++) vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + kt + 8 * (half + 2 * i));
+    };
+    // The first tile's keys: ahead of the queries from fp32 caches (512 rows behind 1024: 152 -> 137 us), behind them from fp16 ones, whose queries take longer to lay out
+    // and then come first (93 rows of 64 dims behind 700: 15.3 us against 16.3).
+    if (!KV_F16 && 32 * phase <= t_max) load_keys(32 * phase);
 
     // query `col` (rows beyond the block repeat its last row, never stored)
     const float *query = a.q + (size_t)(m0 + (col <= last_row ? col : last_row)) * a.n_head * HD + (size_t)head * HD;
     _Float16 *q16 = reinterpret_cast<_Float16 *>(query_mem);                   // [3][32][LDQ]
     float *q32 = reinterpret_cast<float *>(query_mem);                         // [32][LDQ]
-    int q_exp = 0;
     {
         float4 x[KS][2];   // dims 16 ks + 8 half ..
+        int q_exp = 0;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
@@ -75,7 +109,10 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
 #pragma unroll
                 for (int w = 0; w < 2; w++) most = fmaxf(fmaxf(most, fmaxf(fabsf(x[ks][w].x), fabsf(x[ks][w].y))), fmaxf(fabsf(x[ks][w].z), fabsf(x[ks][w].w)));
             most = fmaxf(most, __shfl_xor(most, 32));
+            // where the power of two would not be a float (scores are 0 or beyond every type there), some other will do
             q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
+            q_exp = q_exp < -100 ? -100 : q_exp > 100 ? 100 : q_exp;
+            scale = __builtin_amdgcn_ldexpf(scale, -q_exp);
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
@@ -95,23 +132,6 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
     }
     __syncthreads();
 
-    // Keys beyond t_max are clamped to it: in bounds, and masked.  A lane's keys: row `col` of the tile, dims 16 ks + 8 half .. (fp16), 8 j + 4 half .. (fp32)
-    constexpr int NK = KV_F16 ? KS : HD / 8;
-    float4 kr[NK];
-    auto load_keys = [&](int t0) {
-        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
-#pragma unroll
-        for (int j = 0; j < NK; j++)
-            kr[j] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + kt + 16 * j + 8 * half)
-                           : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 8 * j + 4 * half);
-    };
-    // an fp16 value tile on its way to LDS: key = lane % 32, dims 8 (lane / 32 + 2 i) ..: the transposed two-byte writes spread over the banks
-    uint4 vr[KV_F16 ? VP : 1];
-    auto load_values = [&](int t0) {
-        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
-#pragma unroll
-        for (int i = 0; i < (KV_F16 ? VP : 0); i++) vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + kt + 8 * (half + 2 * i));
-    };
     // fp32 values of dims 32 mt .. for the product's 16 steps: step r takes key 8 (r / 4) + 4 half + r % 4, the key of accumulator r
     auto load_value_dims = [&](int t0, int mt, float (&v)[16]) {
 #pragma unroll
@@ -129,7 +149,7 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
     float mx = -INFINITY, l = 0.0f;
     _Float16 *vt = reinterpret_cast<_Float16 *>(smem + phase * kWave);
 
-    if (32 * phase <= t_max) { load_keys(32 * phase); load_values(32 * phase); }
+    if (KV_F16 && 32 * phase <= t_max) { load_keys(32 * phase); load_values(32 * phase); }
     for (int t0 = 32 * phase; t0 <= t_max; t0 += 32 * KP) {
         float vd[KV_F16 ? 1 : 2][16];
         if constexpr (!KV_F16) load_value_dims(t0, 0, vd[0]);
@@ -156,8 +176,6 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
             __builtin_amdgcn_wave_barrier();
             load_keys(t0 + 32 * KP);   // clamped beyond the last tile
             load_values(t0 + 32 * KP);
-#pragma unroll
-            for (int r = 0; r < 16; r++) s0[r] = __builtin_amdgcn_ldexpf(s0[r], -q_exp);
         } else {
 #pragma unroll
             for (int j = 0; j < HD / 8; j++) {
@@ -179,19 +197,21 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
         // a wavefront may see only masked keys of a query for a while: its state stays (-inf, 0, 0), exponents taken against 0
         const float m_new = fmaxf(mx, tile_max), m_ref = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = expf(mx - m_ref);      // exp(-inf) = 0 on the first tile
+        const float alpha = exp_weight(mx - m_ref);      // exp(-inf) = 0 on the first tile
         float psum = 0.0f, pr[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            pr[r] = expf(s0[r] - m_ref);           // masked keys: exp(-inf) = 0
+            pr[r] = exp_weight(s0[r] - m_ref);           // masked keys: exp(-inf) = 0
             psum += pr[r];
         }
         l = __builtin_fmaf(l, alpha, psum);
         mx = m_new;
+        if (!KV_F16 || __any(alpha != 1.0f)) {   // the maximum has moved (beside fp32 products it makes no difference)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
+                for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
+        }
         if constexpr (KV_F16) {
 #pragma unroll
             for (int j = 0; j < 2; j++) {
@@ -237,7 +257,7 @@ __global__ __launch_bounds__(KP * 64, HD == 64 ? 2 : 1) void span_attention_kern
         if (phase < s) {
             const float m1 = state[phase + s][0][lane], l1 = state[phase + s][1][lane];
             const float m_all = fmaxf(mx, m1), m_ref = m_all == -INFINITY ? 0.0f : m_all;
-            const float f0 = expf(mx - m_ref), f1 = expf(m1 - m_ref);
+            const float f0 = exp_weight(mx - m_ref), f1 = exp_weight(m1 - m_ref);
             l = __builtin_fmaf(l, f0, __fmul_rn(l1, f1));
             mx = m_all;
 #pragma unroll
@@ -296,7 +316,7 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     if (rows <= 0 || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
-    // 512 rows of 24 heads get four, 241 rows of them eight, 93 rows of 32 heads eight (fp16: 70 us behind 1024, 43 behind 1536, 15.7 of 64 dims behind 700).
+    // 512 rows of 24 heads get four, 241 rows of them eight, 93 rows of 32 heads eight (fp16: 58 us behind 1024, 44 behind 1536, 15.3 of 64 dims behind 700).
     const int tiles = (keys + 31) / 32, groups = a.n_head * ((rows + 31) / 32);
     int sets = 1;
     while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
