@@ -34,6 +34,7 @@ int fail(int code, const char *fmt, ...) {
 }
 
 int fail_hip(hipError_t e, const char *what) {
+    (void)hipGetLastError();   // reported here: the next launch's check must not find it again
     int code = e == hipErrorOutOfMemory ? ESP_ERR_OUT_OF_MEMORY
                : (e == hipErrorNoDevice || e == hipErrorInvalidDevice) ? ESP_ERR_NO_DEVICE
                                                                         : ESP_ERR_LAUNCH_FAILED;

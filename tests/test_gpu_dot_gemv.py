@@ -51,6 +51,23 @@ def test_rounds_of_items(mods, fmt, items):
         m.close()
 
 
+def test_a_refused_product_leaves_nothing_to_the_next(mods):
+    """Two rows of 40960 columns do not fit a workgroup's LDS; the call that follows the refusal is not blamed for it."""
+    _, ops, _ = mods
+    from espresso_amd._lib import EspressoError
+    wide = ops.Matrix(orc.FMT_F16, np.zeros((2, 40960), np.float16).view(np.uint8), 2, 40960)
+    w = np.random.default_rng(0).normal(0, 1, (8, 64)).astype(np.float16)
+    m = ops.Matrix(orc.FMT_F16, w.view(np.uint8), 8, 64)
+    x = np.random.default_rng(1).normal(0, 1, (1, 64)).astype(np.float16)
+    for _ in range(2):
+        with pytest.raises(EspressoError):
+            wide.gemv(np.zeros((2, 40960), np.float16))
+        assert np.abs(m.gemv(x) - x.astype(np.float64) @ w.astype(np.float64).T).max() <= 1e-4
+    assert (wide.gemv(np.zeros((1, 40960), np.float16)) == 0).all()
+    m.close()
+    wide.close()
+
+
 @pytest.mark.parametrize("cols", [4, 8, 12, 252, 260, 1028, 4092, 5124])
 def test_fp32_rows_of_whole_fours(mods, cols):
     """Every multiple of four columns is taken: rows of the activations start at any multiple of eight bytes, and the last four columns count."""
