@@ -771,14 +771,19 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         // fifteenth of the tile's time).
         constexpr int UN = NT2 / 2, RP = UN / 8, kActLd = UN + 16;   // units and pieces of a row; halfs per staged row: consecutive rows eight LDS banks apart
         uint16_t *act_hi = reinterpret_cast<uint16_t *>(smem_raw), *act_lo = act_hi + MT * kActLd;
-        const bool odd = lane & 1;
+        // Formed anew: what hangs on the thread alone would be held in registers across the tiles, and the compiler spills for it (gate|up of a 512-row block
+        // of the 8B model 273 us, 268 so; 281 with expf and a division as well, 266 with the bare hardware functions, which are ten times as far off).
+        int et = tid;
+        asm volatile("" : "+v"(et));
+        const int el = et & 63, en = el & 31, eg = el >> 5;
+        const bool odd = el & 1;
 #pragma unroll
         for (int i = 0; i < RB; i++)
 #pragma unroll
             for (int j = 0; j < CB; j++) {
-                const int unit = (32 * CB * wn + 32 * j + bn) >> 1, slot = unit & 3;   // the planes' order inside fours: (0, 2, 1, 3)
+                const int unit = (32 * CB * wn + 32 * j + en) >> 1, slot = unit & 3;   // the planes' order inside fours: (0, 2, 1, 3)
                 const int col = (unit & ~3) + (slot == 1 ? 2 : slot == 2 ? 1 : slot);
-                const int row0 = (wm * RB + i) * 32 + 4 * kg + (odd ? 1 : 0);
+                const int row0 = (wm * RB + i) * 32 + 4 * eg + (odd ? 1 : 0);
 #pragma unroll
                 for (int k = 0; k < 8; k++) {
                     const float a0 = tot[i][j][2 * k], a1 = tot[i][j][2 * k + 1];
@@ -797,7 +802,7 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_regb_kernel(SplitGemm
         const bool whole_pieces = units_n % 8 == 0;
 #pragma unroll
         for (int q = 0; q < MT * RP / THREADS; q++) {
-            const int piece = q * THREADS + tid, row = piece / RP, c8 = (piece % RP) * 8;
+            const int piece = q * THREADS + et, row = piece / RP, c8 = (piece % RP) * 8;
             const int m = m0 + row;
             if (m >= a.M || unit0 + c8 >= units_n) continue;
             const size_t o = (size_t)m * units_n + unit0 + c8;
