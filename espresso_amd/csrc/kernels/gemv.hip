@@ -2565,18 +2565,18 @@ hipError_t launch_mode(const KernelArgs &a, hipStream_t stream) {
         if (a.cols / Traits<FMT>::kItemElems > 128)
             return mode == 1 ? launch_one<FMT, B, R, 1, 4>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 4>(a, stream) : launch_one<FMT, B, R, 0, 4>(a, stream);
     }
-    return mode == 1 ? launch_one<FMT, B, R, 1, 2>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 2>(a, stream) : launch_one<FMT, B, R, 0, 2>(a, stream);
+    if constexpr (R == 2) if (mode == 2) return launch_one<FMT, B, R, 2, 2>(a, stream);
+    return mode == 1 ? launch_one<FMT, B, R, 1, 2>(a, stream) : launch_one<FMT, B, R, 0, 2>(a, stream);
 }
 
 template <int FMT>
 hipError_t launch_fmt(const KernelArgs &a, int batch, hipStream_t stream) {
-    if (batch == 1) {
-        // tall matrices (an output head): four rows per wavefront, so that one wave of workgroups covers the matrix (32000 x 768 Q8_0:
-        // 2000 workgroups instead of 4000, 8.8 against 10.1 us; eight rows measure the same as four)
-        if (a.rows >= 16384) return launch_mode<FMT, 1, 4>(a, stream);
-        return launch_mode<FMT, 1, 2>(a, stream);
-    }
-    if (batch == 2) return a.rows >= 16384 ? launch_mode<FMT, 2, 4>(a, stream) : launch_mode<FMT, 2, 2>(a, stream);
+    // tall matrices (an output head): four rows per wavefront, so that one wave of workgroups covers the matrix (32000 x 768 Q8_0:
+    // 2000 workgroups instead of 4000, 8.8 against 10.1 us; eight rows measure the same as four).  A product that merges attention states has as many rows
+    // as the model is wide and keeps two.
+    const bool tall = a.rows >= 16384 && !a.merge_partials;
+    if (batch == 1) return tall ? launch_mode<FMT, 1, 4>(a, stream) : launch_mode<FMT, 1, 2>(a, stream);
+    if (batch == 2) return tall ? launch_mode<FMT, 2, 4>(a, stream) : launch_mode<FMT, 2, 2>(a, stream);
     return hipErrorInvalidValue;
 }
 
