@@ -39,10 +39,16 @@ __device__ __forceinline__ void store_context_sum(const AttentionArgs &a, size_t
 // split operand may be zero, or overflow, where the operand does not.  Rare, so nothing here is fast.
 template <int HD, bool KV_F16>
 __device__ void plain_attention_row(const AttentionArgs &a, int row, int head) {
-    const int lane = threadIdx.x & 63, kvh = head / (a.n_head / a.n_kv_head), kd = a.n_kv_head * HD, visible = a.pos[row] + 1;
+    const int lane = threadIdx.x & 63, kvh = head / (a.n_head / a.n_kv_head), kd = a.n_kv_head * HD;
     const size_t base = (size_t)a.seq[row] * a.cache_seq_stride + (size_t)kvh * HD;
     const float *q = a.q + (size_t)row * a.n_head * HD + (size_t)head * HD;
     const float scale = 1.0f / sqrtf((float)HD);
+    // A query that is not finite has no score that is, so its context is NaN whatever the keys: no key at all, and 0 / 0.  Once a model's hidden state is NaN every row of
+    // every layer comes here, and this loop would take a hundred times the block's own time.
+    float check = 0.0f;
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++) check = __builtin_fmaf(q[64 * i + lane], 0.0f, check);
+    const int visible = __any(!(check == 0.0f)) ? 0 : a.pos[row] + 1;
     auto cached = [&](const void *cache, size_t at) {
         return KV_F16 ? (float)reinterpret_cast<const _Float16 *>(cache)[at] : reinterpret_cast<const float *>(cache)[at];
     };

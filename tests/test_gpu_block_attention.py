@@ -125,6 +125,19 @@ def test_what_a_row_does_not_see_does_not_reach_it(ops, kernel, heads, kv_heads,
         which[at, 0, 5] = kept
 
 
+@pytest.mark.parametrize("size,planes", [(128, False), (64, True)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_a_query_that_is_not_finite_is_its_own_row_alone(ops, size, planes, dtype, bad):
+    q, k, v = inputs(45, 20, 8, 1, size, dtype, 9)
+    want = exact(q, k, v)
+    q[33, 5, size - 1] = q[2, 0, 0] = bad
+    got, _ = ops.block_attention("span", q, k, v, split_rows=planes)
+    assert np.isnan(got[33, 5]).all() and np.isnan(got[2, 0]).all()
+    got[33, 5], got[2, 0] = want[33, 5], want[2, 0]
+    assert np.abs(got - want).max() <= 2.0 ** -11 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("kernel", ["span", "prompt"])
 def test_fp32_values_beyond_fp16_that_add_up(ops, kernel):
     """fp32 caches hold more than fp16: rows whose weighted sum fits come out finite."""
