@@ -1,0 +1,424 @@
+// y[m][n] = sum_k x[m][k] * W[n][k] for blocks of activation rows, W in Q4_K, Q4_0, Q8_0 or fp16: fp16 operands (every dequantised weight is rounded to fp16
+// once), fp32 sums.
+//
+// A workgroup is eight wavefronts, two on every SIMD, so that one unpacks weights while the other multiplies.  NW of them lie side by side along 32 NW weight rows and
+// 8 / NW groups share K; each wavefront owns 32 weight rows and all 32 TM activation rows of the workgroup's tile.
+//   * The weights never enter LDS: a lane unpacks eight k of its own row into the B operand of v_mfma_f32_32x32x16_f16, which then serves TM products.
+//   * Four lanes cover 64 bytes of a row (sixteen rows a load), and v_permlane16_swap brings each lane the two pieces of its own row: a quarter to a half of the cache
+//     accesses of lanes that read their own rows.
+//   * Loads are spread over the step, one step of 128 k ahead: more in flight only blocks the wavefronts that issue them (two steps ahead, requested in one go:
+//     11264 x 2048 Q8_0, 512 rows 38.8 us, 16 rows 11.9 against 37.8 and 11.6; 3072 x 8192 Q4_0, 512 rows 35.9 against 33.9).
+//   * Activations go through LDS, two buffers and one barrier a step, fragment g + 1 read while g is multiplied (left to the compiler: 3 to 5 % slower).
+//   * Q4_K's n s - dm is one v_fma_mix a weight (a nibble alone in sixteen bits is the fp16 number n 2^-24), rounded once as before; v_cvt_f32_ubyte, an fp32
+//     multiply-add and a conversion take almost twice the instructions.
+// What bounds it: at 512 rows the matrix cores, the unpacking beside them and the power both draw (the same kernel without loads and unpacking: 37 us of the 62 below); at 100 rows
+// and less the weights' way from memory and the steps' latencies.  Against the kernel of 128 x 128 tiles whose weights go through LDS (gemm.hip), us:
+//   16384 x 3072 Q4_0, 512 / 229 / 93 rows 93 / 58 / 39 -> 62 / 32 / 20;  3072 x 8192 Q4_0 53 / 30 / 20 -> 34 / 22 / 14;  11264 x 2048 Q8_0 64 / 39 / 26 -> 38 / 24 / 16;
+//   11264 x 2048 Q4_K 60 / 39 / 28 -> 36 / 22 / 14.  62 us are 830 TFLOP/s.
+#include "../common.h"
+#include "block_gemm.h"
+#include "silu.h"
+#include <atomic>
+#include <type_traits>
+
+namespace esp {
+namespace {
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32;
+
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
+constexpr int kStep = 128;     // k per step: four blocks of Q8_0 / Q4_0, half a super-block of Q4_K
+
+struct BlockArgs {
+    const uint8_t *qs;
+    const uint16_t *scales;
+    size_t row_bytes;
+    int N, K, M;
+    const uint16_t *x;
+    float *y;
+    const float *residual;
+    float *partial;
+    uint16_t *swiglu_out;
+    int per, splits, n_tiles, m_tiles;   // per: steps of one group of wavefronts
+};
+
+__device__ __forceinline__ h2 as_h2(u32 v) { return __builtin_bit_cast(h2, v); }
+__device__ __forceinline__ u32 as_u32(h2 v) { return __builtin_bit_cast(u32, v); }
+__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
+__device__ __forceinline__ float half_bits_to_float(u32 bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
+__device__ __forceinline__ h2 splat_bits(u32 bits16) { return as_h2(__builtin_amdgcn_perm(bits16, bits16, 0x01000100u)); }
+__device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
+    return make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
+                      __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
+}
+constexpr int pairs_of(int fmt) { return fmt == FMT_F16 ? 4 : fmt == FMT_Q8_0 ? 2 : 1; }   // 64-byte stretches of a row in a step
+
+constexpr int kRow = kStep + 8;   // fp16 between the staged activation rows: 272 bytes, sixteen-byte reads of neighbouring rows fall on different banks
+template <int TM, int NW>
+constexpr int block_buffers() { return 2 * (kWaves / NW) * 32 * TM * kRow * 2 <= 160 * 1024 ? 2 : 1; }
+template <int TM, int NW>
+constexpr size_t block_lds_bytes() {
+    const size_t x = (size_t)block_buffers<TM, NW>() * (kWaves / NW) * 32 * TM * kRow * 2, sums = kWaves / NW > 1 ? (size_t)kWaves * TM * 16 * 64 * 4 : 0;
+    return x > sums ? x : sums;
+}
+
+template <int FMT, int TM, int NW>
+__global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
+    constexpr int KW = kWaves / NW, MT = 32 * TM, GT = 64 * NW, BUFS = block_buffers<TM, NW>();
+    constexpr int XP = MT * (kStep / 8) / GT;       // sixteen-byte pieces of the activations per thread and step
+    static_assert(MT * (kStep / 8) % GT == 0 && XP >= 1, "whole pieces");
+    extern __shared__ uint4 smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, col = lane & 31;
+    const int wn = wave % NW, wk = wave / NW, gtid = wn * 64 + lane;
+    // workgroups of one die take neighbouring output tiles: the row tiles of one block of weights first
+    const int total = gridDim.x, die = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
+    const int unit = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
+    const int m_tile = unit % a.m_tiles, rest = unit / a.m_tiles, n_tile = rest % a.n_tiles, split = rest / a.n_tiles;
+    const int m0 = m_tile * MT, n0 = (n_tile * NW + wn) * 32, n = n0 + col;
+    const int row0 = n0 < a.N ? n0 : a.N - 1;
+    auto row_of = [&](int r) { return row0 + r < a.N ? r : a.N - 1 - row0; };   // rows from row0 on, clamped: those beyond are never stored
+    // every group of wavefronts passes the same barriers and has steps of its own
+    const int all = a.K / kStep, s0 = (split * KW + wk) * a.per, own = all - s0 < a.per ? (all > s0 ? all - s0 : 0) : a.per;
+    auto at = [&](int s) { return s0 + s < all ? s0 + s : all - 1; };          // steps past the end repeat the last: in bounds, never used
+
+    _Float16 *xt = reinterpret_cast<_Float16 *>(smem) + wk * BUFS * MT * kRow;   // [BUFS][MT][kRow]
+    uint4 xv[XP];
+    u32 xo[XP];                                // elements from row m0 on
+#pragma unroll
+    for (int i = 0; i < XP; i++) {
+        const int piece = gtid + i * GT, r = piece >> 4, part = piece & 15;
+        xo[i] = (u32)(m0 + r < a.M ? r : a.M - 1 - m0) * (u32)a.K + part * 8;
+    }
+    const uint16_t *xbase = a.x + (size_t)m0 * a.K;
+    auto load_x = [&](int s) __attribute__((always_inline)) {
+        const uint16_t *p = xbase + (size_t)at(s) * kStep;
+#pragma unroll
+        for (int i = 0; i < XP; i++) xv[i] = *reinterpret_cast<const uint4 *>(p + xo[i]);
+    };
+    auto store_x = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < XP; i++) {
+            const int piece = gtid + i * GT, r = piece >> 4, part = piece & 15;
+            *reinterpret_cast<uint4 *>(xt + buf * MT * kRow + r * kRow + part * 8) = FMT == FMT_Q4_0 ? swap_middle(xv[i]) : xv[i];
+        }
+    };
+    // Weights: lane 16 p + r of a load takes piece p of row r (of row 16 + r in the next), so that four lanes cover 64 bytes of a row; v_permlane16_swap
+    // then leaves pieces 2 h and 2 h + 1 of row lane % 32 in each lane.
+    const int piece = lane >> 4;
+    const uint8_t *wbase = a.qs + (size_t)row0 * a.row_bytes;
+    const u32 wlo = (u32)row_of(lane & 15) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + (lane & 15)) * (u32)a.row_bytes + piece * 16;
+    const uint16_t *sbase = a.scales + (size_t)row0 * (a.K / 32);
+    const u32 so = (u32)row_of(col) * (u32)(a.K / 32) + (FMT == FMT_Q4_0 ? 2 * h : 0), ho = (u32)row_of(col) * (u32)a.row_bytes;
+    constexpr int PAIRS = pairs_of(FMT);
+    uint4 raw[2 * PAIRS], q[2];                 // the next step's stretches as they were loaded; the stretch in use, of the lane's own row
+    auto load_pair = [&](int s, int j) __attribute__((always_inline)) {
+        const uint8_t *from = wbase + (FMT == FMT_Q4_K ? (size_t)(at(s) >> 1) * 144 + 16 + (at(s) & 1) * 64 : (size_t)at(s) * (64 * PAIRS)) + 64 * j;
+        raw[2 * j] = *reinterpret_cast<const uint4 *>(from + wlo);
+        raw[2 * j + 1] = *reinterpret_cast<const uint4 *>(from + whi);
+    };
+    auto use_pair = [&](int j) __attribute__((always_inline)) {
+        auto swap = [](u32 x, u32 y, u32 &u, u32 &v) __attribute__((always_inline)) { const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false); u = p[0]; v = p[1]; };
+        swap(raw[2 * j].x, raw[2 * j + 1].x, q[0].x, q[1].x);
+        swap(raw[2 * j].y, raw[2 * j + 1].y, q[0].y, q[1].y);
+        swap(raw[2 * j].z, raw[2 * j + 1].z, q[0].z, q[1].z);
+        swap(raw[2 * j].w, raw[2 * j + 1].w, q[0].w, q[1].w);
+    };
+    auto load_scales = [&](int s) __attribute__((always_inline)) {   // Q4_0: blocks 2 h, 2 h + 1; Q8_0: all four
+        uint2 d = {0, 0};
+        if constexpr (FMT == FMT_Q4_0) d.x = *reinterpret_cast<const u32 *>(sbase + 4 * at(s) + so);
+        if constexpr (FMT == FMT_Q8_0) d = *reinterpret_cast<const uint2 *>(sbase + 4 * at(s) + so);
+        return d;
+    };
+    auto load_hdr = [&](int s) __attribute__((always_inline)) { return *reinterpret_cast<const uint4 *>(wbase + (size_t)(at(s) >> 1) * 144 + ho); };
+    // where fragment g (0..7) of a step begins among its 128 k
+    auto koff = [&](int g) {
+        return FMT == FMT_Q4_0 ? 64 * h + 8 * g : FMT == FMT_Q4_K ? 64 * h + 32 * (g & 1) + 8 * (g >> 1) : FMT == FMT_Q8_0 ? 64 * (g >> 2) + 32 * h + 8 * (g & 3) : 32 * (g >> 1) + 16 * h + 8 * (g & 1);
+    };
+
+    floatx16 acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+
+    uint4 hdr[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};   // of this super-block and the next, by turns
+    uint2 scale[2];                                // of this step and the next, by turns
+    load_x(0);
+#pragma unroll
+    for (int j = 0; j < PAIRS; j++) load_pair(0, j);
+    if constexpr (FMT == FMT_Q4_K) { hdr[0] = load_hdr(0); hdr[1] = load_hdr(2); }
+    scale[0] = load_scales(0);
+    store_x(0);
+    load_x(1);
+    scale[1] = load_scales(1);
+    __syncthreads();
+
+    // eight weights of the lane's row as fp16
+    auto decode = [&](const uint4 &head, const uint2 &scales, auto odd, int g) __attribute__((always_inline)) {
+        if constexpr (FMT == FMT_Q4_K) {
+            // Sub-block 4 odd + 2 h + g % 2.  A nibble alone in sixteen bits is the fp16 number n 2^-24 (or 16 n 2^-24): n s - dm with product and
+            // subtraction in fp32 and one rounding to fp16, as one v_fma_mix a weight.
+            const float d = half_bits_to_float(head.x & 0xFFFFu), dmin = half_bits_to_float(head.x >> 16);
+            const int sh = 16 * h + 8 * (g & 1);
+            u32 sc, m;
+            if constexpr (decltype(odd)::value == 0) { sc = (head.y >> sh) & 63u; m = (head.z >> sh) & 63u; }
+            else {
+                sc = ((head.w >> sh) & 0xFu) | (((head.y >> sh) & 0xC0u) >> 2);
+                m = ((head.w >> (sh + 4)) & 0xFu) | (((head.z >> sh) & 0xC0u) >> 2);
+            }
+            const float s = d * (float)sc * (g & 1 ? 1048576.0f : 16777216.0f), dm = dmin * (float)m;
+            const uint4 &v = q[g >> 2];
+            const u32 w[2] = {g & 2 ? v.z : v.x, g & 2 ? v.w : v.y};
+            const u32 mask = g & 1 ? 0x00F000F0u : 0x000F000Fu;
+            u32 o[4];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const h2 even = as_h2(w[j] & mask), uneven = as_h2((w[j] >> 8) & mask);
+                o[2 * j] = as_u32(h2{(_Float16)__builtin_fmaf((float)even.x, s, -dm), (_Float16)__builtin_fmaf((float)uneven.x, s, -dm)});
+                o[2 * j + 1] = as_u32(h2{(_Float16)__builtin_fmaf((float)even.y, s, -dm), (_Float16)__builtin_fmaf((float)uneven.y, s, -dm)});
+            }
+            return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
+        } else if constexpr (FMT == FMT_Q4_0) {
+            // (n - 8) * d from n under an fp16 exponent; elements of every four come out as 0, 2, 1, 3, like the activations'
+            const h2 sc = splat_bits(g >> 2 ? scales.x >> 16 : scales.x & 0xFFFFu);
+            const uint4 &v = q[g >> 2];
+            const u32 w[2] = {g & 1 ? v.z : v.x, g & 1 ? v.w : v.y};
+            const u32 mask = g & 2 ? 0x00F000F0u : 0x000F000Fu, magic = g & 2 ? 0x54005400u : 0x64006400u;
+            const h2 off = g & 2 ? h2{(_Float16)72.0f, (_Float16)72.0f} : h2{(_Float16)1032.0f, (_Float16)1032.0f};
+            u32 o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = as_u32((as_h2(((j & 1 ? w[j >> 1] >> 8 : w[j >> 1]) & mask) | magic) - off) * sc);
+            return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
+        } else if constexpr (FMT == FMT_Q8_0) {
+            const u32 pair = g >> 2 ? scales.y : scales.x;
+            const h2 sc = splat_bits(h ? pair >> 16 : pair & 0xFFFFu), off = {(_Float16)1152.0f, (_Float16)1152.0f};   // 1024 + 128
+            const uint4 &v = q[(g >> 1) & 1];
+            const u32 w[2] = {(g & 1 ? v.z : v.x) ^ 0x80808080u, (g & 1 ? v.w : v.y) ^ 0x80808080u};
+            u32 o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, w[j >> 1], j & 1 ? 0x04030402u : 0x04010400u)) - off) * sc);
+            return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
+        } else {
+            return as_half8(q[g & 1]);
+        }
+    };
+    constexpr int VALU = FMT == FMT_F16 ? 2 : 16;   // of a fragment, to be spread over its products
+    auto step = [&](auto slot_c, int s) __attribute__((always_inline)) {   // slot: s % 4: the buffers by turns, half of a super-block, super-blocks by turns
+        constexpr int S = decltype(slot_c)::value & 1, H = decltype(slot_c)::value >> 1;
+        constexpr std::integral_constant<int, S> odd{};
+        constexpr int B = BUFS == 2 ? S : 0;
+        const _Float16 *xb = xt + B * MT * kRow + col * kRow;
+        half8 xf[2][TM], wf[2];
+        auto fragments = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) xf[g & 1][i] = *reinterpret_cast<const half8 *>(xb + 32 * i * kRow + koff(g));
+            if (g % (8 / PAIRS) == 0) {   // a stretch is taken into use, the next step's goes on its way
+                use_pair(g / (8 / PAIRS));
+                load_pair(s + 1, g / (8 / PAIRS));
+            }
+            wf[g & 1] = decode(hdr[H], scale[S], odd, g);
+        };
+        fragments(0);
+        if constexpr (BUFS == 2) {
+            store_x(S ^ 1);        // the next step's activations; that buffer was last read before the last barrier
+            load_x(s + 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            if (g + 1 < 8) fragments(g + 1);
+#pragma unroll
+            for (int i = 0; i < TM; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][i], wf[g & 1], acc[i], 0, 0, 0);
+            if (g + 1 < 8) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) {   // in this order: a product, a read, a share of the unpacking
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, (VALU + TM - 1) / TM, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        scale[S] = load_scales(s + 2);
+        if constexpr (FMT == FMT_Q4_K && S == 1) hdr[H] = load_hdr(s + 3);
+        __syncthreads();
+        if constexpr (BUFS == 1) {
+            store_x(0);
+            load_x(s + 2);
+            __syncthreads();
+        }
+    };
+    int s = 0;
+    for (; s + 4 <= own; s += 4) {
+        step(std::integral_constant<int, 0>{}, s);
+        step(std::integral_constant<int, 1>{}, s + 1);
+        step(std::integral_constant<int, 2>{}, s + 2);
+        step(std::integral_constant<int, 3>{}, s + 3);
+    }
+    if (s < own) step(std::integral_constant<int, 0>{}, s);
+    if (s + 1 < own) step(std::integral_constant<int, 1>{}, s + 1);
+    if (s + 2 < own) step(std::integral_constant<int, 2>{}, s + 2);
+    for (s = own; s < a.per; s++) {
+        __syncthreads();
+        if constexpr (BUFS == 1) __syncthreads();
+    }
+
+    // accumulator r of a lane: activation row 8 (r / 4) + 4 h + r % 4 of its 32, weight row lane % 32
+    auto out_row = [&](int r) { return m0 + 32 * (r >> 4) + 8 * ((r & 15) >> 2) + 4 * h + (r & 3); };
+    constexpr int SHARE = TM * 16 / KW;        // accumulators that a wavefront finishes
+    float v[SHARE];
+    int r0 = 0;
+    if constexpr (KW == 1) {
+#pragma unroll
+        for (int r = 0; r < SHARE; r++) v[r] = acc[r >> 4][r & 15];
+    } else {   // the groups' sums meet in LDS (the last barrier is behind everybody's last read of it), in their order
+        float *red = reinterpret_cast<float *>(smem);
+#pragma unroll
+        for (int r = 0; r < TM * 16; r++) red[((size_t)wave * TM * 16 + r) * 64 + lane] = acc[r >> 4][r & 15];
+        __syncthreads();
+        r0 = wk * SHARE;
+#pragma unroll
+        for (int r = 0; r < SHARE; r++) {
+            float sum = red[((size_t)wn * TM * 16 + r0 + r) * 64 + lane];
+#pragma unroll
+            for (int g = 1; g < KW; g++) sum += red[((size_t)(g * NW + wn) * TM * 16 + r0 + r) * 64 + lane];
+            v[r] = sum;
+        }
+    }
+    if (a.swiglu_out) {   // weight rows are (gate, up) pairs, neighbouring lanes: the even lane finishes the even accumulators, the odd lane the odd ones
+#pragma unroll
+        for (int k = 0; k < SHARE / 2; k++) {
+            const float p0 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k]), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+            const float p1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k + 1]), 0xB1, 0xF, 0xF, false));
+            const bool odd = lane & 1;
+            const float g = odd ? p1 : v[2 * k], u = odd ? v[2 * k + 1] : p0;
+            const int m = out_row(r0 + 2 * k + (odd ? 1 : 0));
+            if (m < a.M && (n | 1) < a.N) {
+                a.swiglu_out[(size_t)m * (a.N / 2) + n / 2] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(silu(g), u));
+            }
+        }
+        return;
+    }
+    float *out = a.splits > 1 ? a.partial + (size_t)split * a.M * a.N : a.y;
+    const bool whole = m0 + MT <= a.M && n0 + 32 <= a.N;
+    if (a.splits == 1 && a.residual) {
+        // requested together: y may be the residual's own memory, and a load behind each store is a trip to memory each
+#pragma unroll
+        for (int r = 0; r < SHARE; r++) v[r] += a.residual[(size_t)(out_row(r0 + r) < a.M ? out_row(r0 + r) : a.M - 1) * a.N + (n < a.N ? n : a.N - 1)];
+    }
+    if (whole) {
+#pragma unroll
+        for (int r = 0; r < SHARE; r++) out[(size_t)out_row(r0 + r) * a.N + n] = v[r];
+    } else {
+#pragma unroll
+        for (int r = 0; r < SHARE; r++) if (out_row(r0 + r) < a.M && n < a.N) out[(size_t)out_row(r0 + r) * a.N + n] = v[r];
+    }
+}
+
+template <int FMT, int TM, int NW>
+hipError_t launch(const BlockArgs &a, hipStream_t stream) {
+    static std::atomic<uint64_t> raised{0};   // the limit of dynamic LDS is raised once per kernel and device
+    constexpr size_t lds = block_lds_bytes<TM, NW>();
+    if (lds > 64 * 1024) {
+        int device = 0;
+        hipError_t err = hipGetDevice(&device);
+        if (err != hipSuccess) return err;
+        const uint64_t bit = 1ull << (device & 63);
+        if (!(raised.load(std::memory_order_acquire) & bit)) {
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (err != hipSuccess) return err;
+            raised.fetch_or(bit, std::memory_order_release);
+        }
+    }
+    hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
+    return hipGetLastError();
+}
+
+template <int FMT, int TM>
+hipError_t launch_width(int nw, const BlockArgs &a, hipStream_t stream) {
+    if (nw == 8) return launch<FMT, TM, 8>(a, stream);
+    if (nw == 4) return launch<FMT, TM, 4>(a, stream);
+    if constexpr (TM < 4) return launch<FMT, TM, 2>(a, stream);   // 128 activation rows for each of four groups: more registers than there are
+    return hipErrorInvalidValue;
+}
+template <int FMT>
+hipError_t launch_format(int tm, int nw, const BlockArgs &a, hipStream_t stream) {
+    switch (tm) {
+    case 1: return launch_width<FMT, 1>(nw, a, stream);
+    case 2: return launch_width<FMT, 2>(nw, a, stream);
+    case 3: return launch_width<FMT, 3>(nw, a, stream);
+    default: return launch_width<FMT, 4>(nw, a, stream);
+    }
+}
+
+struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
+
+// The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of 256 workgroups, a step of a round growing with the tile's rows and
+// with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, a kernel of its own).  The
+// constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows, the four formats) and are off by 6 % at the
+// median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst but for fp16.
+Form choose_form(const GemmParams &p) {
+    const int fmt = p.w.format, N = p.w.rows, M = p.rows, unit = fmt == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit);
+    const bool f16 = fmt == FMT_F16;
+    const float start = 2.25f, fill = f16 ? 1.84f : 1.34f, step = f16 ? 1.98f : 0.743f, row_tile = f16 ? 0.0f : 0.149f, staged = 0.1f, join = f16 ? 0.47f : 0.383f;
+    const float plane_us = f16 ? 0.233f : 0.28f, again_us = 0.2f;   // per MB
+    static const int kSplits[] = {1, 2, 3, 4, 6, 8};
+    Form best;
+    float best_us = 0.0f;
+    for (int tm = 1; tm <= 4 && tm <= (M + 31) / 32; tm++)
+        for (int nw = tm < 4 ? 2 : 4; nw <= 8; nw *= 2)
+            for (int want : kSplits) {
+                const int kw = 8 / nw, per = (units + want * kw - 1) / (want * kw), splits = (units + per * kw - 1) / (per * kw);
+                const float mb = (float)splits * (float)M * (float)N * 4e-6f;
+                if (splits != want || (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
+                const long wgs = (long)((N + 32 * nw - 1) / (32 * nw)) * ((M + 32 * tm - 1) / (32 * tm)) * splits;
+                const float rounds = (float)((wgs + 255) / 256);
+                float us = start + rounds * (per * unit * (step + tm * (row_tile + staged * kw)) + fill + (kw > 1 ? join * tm : 0.0f)) + plane_us * mb;
+                if (splits > 1) us += again_us * mb + (p.swiglu_out ? 3.0f : 1.0f);
+                if (!best.tm || us < best_us) { best = Form{tm, nw, per * unit, splits}; best_us = us; }
+            }
+    return best;
+}
+
+}  // namespace
+
+static std::atomic<int> g_block_gemm_form{0};
+void block_gemm_set_form(int form) {
+    const int tm = form / 100, nw = form / 10 % 10, shares = form % 10;
+    const bool known = tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
+    g_block_gemm_form.store(known ? form : 0);
+}
+
+bool block_gemm_takes(const GemmParams &p) {
+    const int fmt = p.w.format;
+    if (fmt != FMT_Q4_K && fmt != FMT_Q4_0 && fmt != FMT_Q8_0 && fmt != FMT_F16) return false;
+    if (p.w.cols % (fmt == FMT_Q4_K ? 256 : kStep) != 0) return false;
+    if (fmt != FMT_F16 || g_block_gemm_form.load() > 0) return true;
+    // fp16 weights are four times the bytes and nothing to unpack, and planes cost them more than they give: 3072 x 3072, 12 / 128 rows 9.0 / 14.4 us in the tile kernel, 11.2 / 17
+    // here; tall matrices do without planes: 11264 x 2048, 93 / 229 / 512 rows 26 / 39 / 61 -> 21 / 31 / 47
+    return p.rows > 64 && p.w.rows >= 8192 && choose_form(p).splits == 1;
+}
+
+hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {
+    Form f = choose_form(p);
+    if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
+        f.tm = forced / 100; f.nw = forced / 10 % 10;
+        const int want = forced % 10, kw = 8 / f.nw, unit = p.w.format == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit), per = (units + want * kw - 1) / (want * kw);
+        f.per = per * unit; f.splits = (units + per * kw - 1) / (per * kw);
+        if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;
+    }
+    BlockArgs a{p.w.qs, p.w.scales, p.w.qs_row_bytes, p.w.rows, p.w.cols, p.rows, p.x, p.y, p.residual, p.workspace, f.splits == 1 && p.w.rows % 2 == 0 ? p.swiglu_out : nullptr, f.per, f.splits,
+                (p.w.rows + 32 * f.nw - 1) / (32 * f.nw), (p.rows + 32 * f.tm - 1) / (32 * f.tm)};
+    *splits = f.splits;
+    switch (p.w.format) {
+    case FMT_Q4_K: return launch_format<FMT_Q4_K>(f.tm, f.nw, a, stream);
+    case FMT_Q4_0: return launch_format<FMT_Q4_0>(f.tm, f.nw, a, stream);
+    case FMT_Q8_0: return launch_format<FMT_Q8_0>(f.tm, f.nw, a, stream);
+    default: return launch_format<FMT_F16>(f.tm, f.nw, a, stream);
+    }
+}
+
+}  // namespace esp

@@ -5,15 +5,16 @@
 // (RealModelInferenceEngine.swift:6674-6697 inside the prefill loop :6365-6375) by one pass over the
 // packed weights per block of rows.
 //
-// Shape of the kernel (gfx950, wave64)
+// launch_gemm chooses: few rows or small matrices with exact weights (rows_gemm.hip), up to eight rows of Q4_K / Q4_0 (gemm_rows_kernel below), blocks of rows
+// (block_gemm.hip), and for what is left - columns that are no multiple of 128, most fp16 matrices - gemm_kernel:
 //   * a workgroup of four wavefronts owns 128 weight rows (n) x MT activation rows (m) and walks K in
 //     tiles of 64;
 //   * per K tile every thread fetches the packed bytes of (one weight row, one half of the tile) with
 //     128-bit loads, turns them into 32 fp16 weights in registers (nibble / byte exponent tricks, one
 //     packed fp16 multiply-add with the block's scale and minimum) and writes them to LDS; the fp16
 //     activations of the tile are copied to LDS next to them;
-//   * every weight reaches the matrix core as its dequantised value rounded to fp16 exactly once (Q4_K:
-//     n * d*sc - dmin*m in fp32 first; Q4_0 / Q8_0: one exact packed fp16 product);
+//   * every weight reaches the matrix core as its dequantised value rounded to fp16 exactly once
+//     (one exact packed fp16 product);
 //   * the Q4_0 / Q8_0 exponent tricks yield elements in (0,2,1,3) order inside every group of four; the
 //     activations are stored with the same swap, which costs nothing because a dot product does not care
 //     about the order of k as long as both operands agree;
@@ -24,6 +25,7 @@
 //     adds the partial sums in split order (deterministic, no atomics).
 #include "../common.h"
 #include "decode_ops.h"
+#include "block_gemm.h"
 #include "rows_gemm.h"
 #include <atomic>
 #include <type_traits>
@@ -57,6 +59,7 @@ struct GemmArgs {
 __device__ __forceinline__ h2 as_h2(u32 v) { return __builtin_bit_cast(h2, v); }
 __device__ __forceinline__ u32 as_u32(h2 v) { return __builtin_bit_cast(u32, v); }
 __device__ __forceinline__ float half_bits_to_float(u32 bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
+__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
 __device__ __forceinline__ h2 splat(float v) { const _Float16 h = (_Float16)v; return h2{h, h}; }
 __device__ __forceinline__ u32 dword_of(const uint4 &v, int k) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; }
 __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
@@ -72,8 +75,6 @@ __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
 template <int FMT>
 struct Raw;
 template <>
-struct Raw<FMT_Q4_K> { uint4 q, hdr; };          // 16 bytes of nibbles + the super-block header
-template <>
 struct Raw<FMT_Q4_0> { uint4 q; u32 d; };        // one block
 template <>
 struct Raw<FMT_Q8_0> { uint4 q0, q1; u32 d; };   // one block
@@ -84,11 +85,7 @@ template <int FMT>
 __device__ __forceinline__ Raw<FMT> fetch_raw(const GemmArgs &a, int row, int tile, int h) {
     Raw<FMT> r;
     const uint8_t *base = a.qs + (size_t)row * a.qs_row_bytes;
-    if constexpr (FMT == FMT_Q4_K) {
-        const uint8_t *blk = base + (size_t)(tile >> 2) * 144;
-        r.hdr = *reinterpret_cast<const uint4 *>(blk);
-        r.q = *reinterpret_cast<const uint4 *>(blk + 16 + (tile & 3) * 32 + h * 16);
-    } else if constexpr (FMT == FMT_Q4_0) {
+    if constexpr (FMT == FMT_Q4_0) {
         const int block = tile * 2 + h;
         r.q = *reinterpret_cast<const uint4 *>(base + (size_t)block * 16);
         r.d = a.scales[(size_t)row * (a.K / 32) + block];
@@ -131,43 +128,11 @@ __device__ __forceinline__ uint2 nibbles_to_half(u32 w, bool high, h2 s, h2 dm) 
     return make_uint2(as_u32(__builtin_elementwise_fma(n02, s, -dm)), as_u32(__builtin_elementwise_fma(n13, s, -dm)));
 }
 
-// Q4_K: four nibbles spread over the bytes of `b` -> fp16(n * s - dm) with the product and the subtraction in
-// fp32, so each weight is the dequantised value rounded to fp16 once (n * s and dm can both be several
-// times larger than their difference; rounding them separately in fp16 would cost two more bits).
-__device__ __forceinline__ uint2 q4k_bytes_to_half(u32 b, float s, float dm) {
-    // The empty statement hides where `b` came from: otherwise the compiler folds the caller's nibble mask into four
-    // bit-field extracts followed by byte conversions, two operations per weight where v_cvt_f32_ubyte0..3 on the masked
-    // word need one.
-    asm volatile("" : "+v"(b));
-    const float w0 = __builtin_fmaf((float)(b & 0xFFu), s, -dm), w1 = __builtin_fmaf((float)((b >> 8) & 0xFFu), s, -dm);
-    const float w2 = __builtin_fmaf((float)((b >> 16) & 0xFFu), s, -dm), w3 = __builtin_fmaf((float)(b >> 24), s, -dm);
-    return make_uint2(as_u32(h2{(_Float16)w0, (_Float16)w1}), as_u32(h2{(_Float16)w2, (_Float16)w3}));
-}
-
 // Writes the thread's 32 fp16 weights into its LDS row (`wrow` points at k = 0 of the tile).
-// Element order inside each group of four is (0,2,1,3) for Q4_0 and Q8_0, natural for Q4_K and F16.
-// `c` = tile % 4, the pair of Q4_K sub-blocks the tile covers (a constant where the caller's loop is unrolled by four).
+// Element order inside each group of four is (0,2,1,3) for Q4_0 and Q8_0, natural for F16.
 template <int FMT>
-__device__ __forceinline__ void dequant_to_lds(const Raw<FMT> &r, int c, int h, _Float16 *wrow) {
-    if constexpr (FMT == FMT_Q4_K) {
-        // low nibbles: sub-block 2c, elements 16h..16h+15 (k = 16h..); high nibbles: sub-block 2c+1 (k = 32+16h..)
-        const float d = half_bits_to_float(r.hdr.x & 0xFFFFu), dmin = half_bits_to_float(r.hdr.x >> 16);
-        float sc_lo, m_lo, sc_hi, m_hi;
-        q4k_scale_min(r.hdr, 2 * c, sc_lo, m_lo);
-        q4k_scale_min(r.hdr, 2 * c + 1, sc_hi, m_hi);
-        const float s_lo = d * sc_lo, dm_lo = dmin * m_lo, s_hi = d * sc_hi, dm_hi = dmin * m_hi;
-        uint2 lo[4], hi[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            lo[k] = q4k_bytes_to_half(dword_of(r.q, k) & 0x0F0F0F0Fu, s_lo, dm_lo);
-            hi[k] = q4k_bytes_to_half((dword_of(r.q, k) >> 4) & 0x0F0F0F0Fu, s_hi, dm_hi);
-        }
-        uint4 *plo = reinterpret_cast<uint4 *>(wrow + 16 * h), *phi = reinterpret_cast<uint4 *>(wrow + 32 + 16 * h);
-        plo[0] = make_uint4(lo[0].x, lo[0].y, lo[1].x, lo[1].y);
-        plo[1] = make_uint4(lo[2].x, lo[2].y, lo[3].x, lo[3].y);
-        phi[0] = make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y);
-        phi[1] = make_uint4(hi[2].x, hi[2].y, hi[3].x, hi[3].y);
-    } else if constexpr (FMT == FMT_Q4_0) {
+__device__ __forceinline__ void dequant_to_lds(const Raw<FMT> &r, int h, _Float16 *wrow) {
+    if constexpr (FMT == FMT_Q4_0) {
         // byte j: low nibble = element j, high nibble = element j + 16; w = (n - 8) * d
         const h2 s = splat(half_bits_to_float(r.d)), dm = splat(8.0f * half_bits_to_float(r.d));
         uint2 lo[4], hi[4];
@@ -262,8 +227,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
         fetch_x(tile, xv[d]);
     }
     static_assert(4 % DEPTH == 0, "the main loop is unrolled by four");
-    auto stage = [&](int S, int c, int tile, int buf) {   // S and c are constants after unrolling
-        dequant_to_lds<FMT>(raw[S], c, wh, wt[buf] + wr * LDK);
+    auto stage = [&](int S, int tile, int buf) {   // S is a constant after unrolling
+        dequant_to_lds<FMT>(raw[S], wh, wt[buf] + wr * LDK);
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int piece = tid + i * THREADS, row = piece >> 3, part = piece & 7;
@@ -273,7 +238,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
         raw[S] = fetch_raw<FMT>(a, w_row, ahead, wh);
         fetch_x(ahead, xv[S]);
     };
-    stage(0, 0, t_begin, 0);   // t_begin is a multiple of four
+    stage(0, t_begin, 0);
     __syncthreads();
     for (int t0 = t_begin; t0 < t_end; t0 += 4) {
 #pragma unroll
@@ -295,7 +260,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
 #pragma unroll
                         for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
                 }
-                stage((u + 1) % DEPTH, (u + 1) & 3, t + 1, buf ^ 1);
+                stage((u + 1) % DEPTH, t + 1, buf ^ 1);
                 __syncthreads();
             }
         }
@@ -348,205 +313,19 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
         }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Short M (at most 64 activation rows): the weights never touch LDS.  In v_mfma_f32_32x32x16_f16 a lane
-// of the B operand holds eight consecutive k of ONE column, so a lane can load 16 packed bytes of its
-// own weight row, dequantise them in registers and feed them to the matrix core directly; lanes 0..31
-// and 32..63 of a wavefront take the two halves of each 64-k tile of the same 32 weight rows.  A
-// wavefront owns 32 weight rows, a workgroup 128.  Only the activations go through LDS, 256 k at a
-// time and double-buffered, so there is one barrier per 256 k.  Packed weights for DEPTH chunks of
-// 256 k are in flight per lane.
-constexpr int CK = 256;        // k per activation stage
-constexpr int LDX = CK + 8;    // fp16 per LDS row of activations
-
-template <int FMT>
-struct RawChunk;
-template <>
-struct RawChunk<FMT_Q4_K> { uint4 hdr, q[4]; };
-template <>
-struct RawChunk<FMT_Q4_0> { uint4 q[4]; u32 d[4]; };
-template <>
-struct RawChunk<FMT_Q8_0> { uint4 q[8]; u32 d[4]; };
-
-template <int FMT>
-__device__ __forceinline__ RawChunk<FMT> fetch_chunk(const GemmArgs &a, int row, int chunk, int h) {
-    RawChunk<FMT> r;
-    const uint8_t *base = a.qs + (size_t)row * a.qs_row_bytes;
-    if constexpr (FMT == FMT_Q4_K) {
-        const uint8_t *blk = base + (size_t)chunk * 144;
-        r.hdr = *reinterpret_cast<const uint4 *>(blk);
-#pragma unroll
-        for (int c = 0; c < 4; c++) r.q[c] = *reinterpret_cast<const uint4 *>(blk + 16 + c * 32 + h * 16);
-    } else if constexpr (FMT == FMT_Q4_0) {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int block = chunk * 8 + t * 2 + h;
-            r.q[t] = *reinterpret_cast<const uint4 *>(base + (size_t)block * 16);
-            r.d[t] = a.scales[(size_t)row * (a.K / 32) + block];
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int block = chunk * 8 + t * 2 + h;
-            const uint4 *q = reinterpret_cast<const uint4 *>(base + (size_t)block * 32);
-            r.q[2 * t] = q[0];
-            r.q[2 * t + 1] = q[1];
-            r.d[t] = a.scales[(size_t)row * (a.K / 32) + block];
-        }
-    }
-    return r;
-}
-
-__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
-
-// The four B fragments (eight fp16 each) a lane contributes to 64-k tile `t` of its chunk, and the k offset
-// inside the tile at which the matching activations start.  Element order inside groups of four matches
-// the activations' LDS copy (natural for Q4_K, (0,2,1,3) for Q4_0 and Q8_0).
-template <int FMT>
-__device__ __forceinline__ void tile_fragments(const RawChunk<FMT> &r, int t, int h, half8 frag[4], int koff[4]) {
-    if constexpr (FMT == FMT_Q4_K) {
-        const float d = half_bits_to_float(r.hdr.x & 0xFFFFu), dmin = half_bits_to_float(r.hdr.x >> 16);
-        float sc_lo, m_lo, sc_hi, m_hi;
-        q4k_scale_min(r.hdr, 2 * t, sc_lo, m_lo);
-        q4k_scale_min(r.hdr, 2 * t + 1, sc_hi, m_hi);
-        const float s_lo = d * sc_lo, dm_lo = dmin * m_lo, s_hi = d * sc_hi, dm_hi = dmin * m_hi;
-        uint2 lo[4], hi[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            lo[k] = q4k_bytes_to_half(dword_of(r.q[t], k) & 0x0F0F0F0Fu, s_lo, dm_lo);
-            hi[k] = q4k_bytes_to_half((dword_of(r.q[t], k) >> 4) & 0x0F0F0F0Fu, s_hi, dm_hi);
-        }
-        frag[0] = as_half8(make_uint4(lo[0].x, lo[0].y, lo[1].x, lo[1].y));
-        frag[1] = as_half8(make_uint4(lo[2].x, lo[2].y, lo[3].x, lo[3].y));
-        frag[2] = as_half8(make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y));
-        frag[3] = as_half8(make_uint4(hi[2].x, hi[2].y, hi[3].x, hi[3].y));
-        koff[0] = 16 * h; koff[1] = 16 * h + 8; koff[2] = 32 + 16 * h; koff[3] = 40 + 16 * h;
-    } else if constexpr (FMT == FMT_Q4_0) {
-        const h2 s = splat(half_bits_to_float(r.d[t])), dm = splat(8.0f * half_bits_to_float(r.d[t]));
-        uint2 lo[4], hi[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            lo[k] = nibbles_to_half(dword_of(r.q[t], k), false, s, dm);
-            hi[k] = nibbles_to_half(dword_of(r.q[t], k), true, s, dm);
-        }
-        frag[0] = as_half8(make_uint4(lo[0].x, lo[0].y, lo[1].x, lo[1].y));
-        frag[1] = as_half8(make_uint4(lo[2].x, lo[2].y, lo[3].x, lo[3].y));
-        frag[2] = as_half8(make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y));
-        frag[3] = as_half8(make_uint4(hi[2].x, hi[2].y, hi[3].x, hi[3].y));
-#pragma unroll
-        for (int f = 0; f < 4; f++) koff[f] = 32 * h + 8 * f;
-    } else {
-        const h2 s = splat(half_bits_to_float(r.d[t])), off = h2{(_Float16)1152.0f, (_Float16)1152.0f};
-#pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const uint4 &q = r.q[2 * t + half];
-            u32 out[8];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const u32 b = dword_of(q, k) ^ 0x80808080u;
-                const h2 f02 = as_h2(__builtin_amdgcn_perm(0x64646464u, b, 0x04020400u)) - off;
-                const h2 f13 = as_h2(__builtin_amdgcn_perm(0x64646464u, b, 0x04030401u)) - off;
-                out[2 * k] = as_u32(f02 * s);
-                out[2 * k + 1] = as_u32(f13 * s);
-            }
-            frag[2 * half] = as_half8(make_uint4(out[0], out[1], out[2], out[3]));
-            frag[2 * half + 1] = as_half8(make_uint4(out[4], out[5], out[6], out[7]));
-        }
-#pragma unroll
-        for (int f = 0; f < 4; f++) koff[f] = 32 * h + 8 * f;
-    }
-}
-
-template <int FMT, int TM, int DEPTH>
-__global__ __launch_bounds__(kThreads) void gemm_skinny_kernel(GemmArgs a) {
-    constexpr int MT = 32 * TM;
-    constexpr int XV = MT * CK / 8 / kThreads;   // 128-bit pieces of x per thread per chunk (4 per 32 rows)
-    __shared__ _Float16 xt[2][MT * LDX];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
-    const int n = blockIdx.x * NT + wave * 32 + (lane & 31);
-    const int w_row = n < a.N ? n : a.N - 1;     // clamped, the result is never stored
-    const int chunks = a.K / CK;
-    const int c_begin = blockIdx.y * a.tiles_per_split;   // split granularity is a chunk here
-    const int c_end = c_begin + a.tiles_per_split < chunks ? c_begin + a.tiles_per_split : chunks;
-
-    floatx16 acc[TM];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
-
-    auto fetch_x = [&](int chunk, uint4 (&xv)[XV]) {
-#pragma unroll
-        for (int i = 0; i < XV; i++) {
-            const int piece = tid + i * kThreads, row = piece >> 5, part = piece & 31;   // 32 pieces per row
-            xv[i] = row < a.M ? reinterpret_cast<const uint4 *>(a.x + (size_t)row * a.K + (size_t)chunk * CK)[part] : make_uint4(0, 0, 0, 0);
-        }
-    };
-
-    RawChunk<FMT> raw[DEPTH];
-    uint4 xv[XV];
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++)
-        if (c_begin + d < c_end) raw[d] = fetch_chunk<FMT>(a, w_row, c_begin + d, h);
-    if (c_begin < c_end) fetch_x(c_begin, xv);
-
-    for (int c0 = c_begin; c0 < c_end; c0 += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
-            const int c = c0 + d, buf = d & 1;   // DEPTH is even
-            if (c < c_end) {
-#pragma unroll
-                for (int i = 0; i < XV; i++) {
-                    const int piece = tid + i * kThreads, row = piece >> 5, part = piece & 31;
-                    *reinterpret_cast<uint4 *>(xt[buf] + row * LDX + part * 8) = FMT == FMT_Q4_K ? xv[i] : swap_middle(xv[i]);
-                }
-                if (c + 1 < c_end) fetch_x(c + 1, xv);
-            }
-            __syncthreads();
-            if (c < c_end) {
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    half8 frag[4];
-                    int koff[4];
-                    tile_fragments<FMT>(raw[d], t, h, frag, koff);
-#pragma unroll
-                    for (int f = 0; f < 4; f++)
-#pragma unroll
-                        for (int i = 0; i < TM; i++) {
-                            const half8 af = *reinterpret_cast<const half8 *>(xt[buf] + (i * 32 + (lane & 31)) * LDX + t * KT + koff[f]);
-                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, frag[f], acc[i], 0, 0, 0);
-                        }
-                }
-                if (c + DEPTH < c_end) raw[d] = fetch_chunk<FMT>(a, w_row, c + DEPTH, h);
-            }
-        }
-    }
-
-    const bool split = gridDim.y > 1;
-    float *out = split ? a.partial + (size_t)blockIdx.y * a.M * a.N : a.y;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int m = i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            if (m < a.M && n < a.N) {
-                const size_t o = (size_t)m * a.N + n;
-                out[o] = (!split && a.residual) ? a.residual[o] + acc[i][r] : acc[i][r];
-            }
-        }
-}
+constexpr int CK = 256;        // k per activation stage of the kernel below
 
 // ---------------------------------------------------------------------------------------------
-// Up to eight activation rows against Q4_K weights without dequantising them.  With so few rows the
-// register-B kernel above is bound by the exact dequantisation (three vector operations per weight however few rows
-// there are).  Here the B operand is the nibble itself under an fp16 exponent, as in the GEMV kernels: one
+// Up to eight activation rows against Q4_K or Q4_0 weights without dequantising them (three vector operations per weight however few rows
+// there are).  The weights never touch LDS: a lane of the B operand of v_mfma_f32_32x32x16_f16 holds eight consecutive k of ONE column, so a lane loads packed bytes of its
+// own weight row; lanes 0..31 and 32..63 of a wavefront take the two halves of each 64-k tile of the same 32 weight rows.  The B operand is the nibble itself under an fp16 exponent, as in the GEMV kernels: one
 // v_and_or_b32 turns two low nibbles into (64 + n/16, 64 + n/16) and two high nibbles into (4 + n/16, 4 + n/16),
 // exactly; two MFMAs contract a 32-weight sub-block into sum (offset + n/16) x with exact products, and scale and
 // minimum of the sub-block are folded into the few accumulator registers that hold real rows afterwards:
 //     sum_k (d sc n_k - dmin m) x_k = (16 d sc) raw - (16 d sc offset + dmin m) sum_k x_k,
 // with the sums of the activations over each sub-block computed once per workgroup while they are staged.
-// Lane mapping, loads, LDS staging of the activations (in (0,2,1,3) order inside fours, which is how the masked
-// nibble pairs come out) are those of gemm_skinny_kernel; the rows 0..7 are accumulator registers 0..3 of a lane.
+// Only the activations go through LDS, in (0,2,1,3) order inside fours, which is how the masked nibble pairs come out; the rows 0..7 are
+// accumulator registers 0..3 of a lane.
 __device__ __forceinline__ float quad_sum(float v) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
     v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
@@ -572,7 +351,7 @@ template <int WAVES, int SPAN> constexpr size_t rows_lds_bytes() {
 template <int FMT>
 struct RowsChunk;
 template <>
-struct RowsChunk<FMT_Q4_K> { RawChunk<FMT_Q4_K> r; };
+struct RowsChunk<FMT_Q4_K> { uint4 hdr, q[4]; };
 template <>
 struct RowsChunk<FMT_Q4_0> { uint2 q[8]; uint4 d; };   // eight bytes of each of the chunk's eight blocks, their eight fp16 scales
 
@@ -580,7 +359,10 @@ template <int FMT>
 __device__ __forceinline__ RowsChunk<FMT> fetch_rows_chunk(const GemmArgs &a, int row, int chunk, int h) {
     RowsChunk<FMT> c;
     if constexpr (FMT == FMT_Q4_K) {
-        c.r = fetch_chunk<FMT_Q4_K>(a, row, chunk, h);
+        const uint8_t *blk = a.qs + (size_t)row * a.qs_row_bytes + (size_t)chunk * 144;
+        c.hdr = *reinterpret_cast<const uint4 *>(blk);
+#pragma unroll
+        for (int t = 0; t < 4; t++) c.q[t] = *reinterpret_cast<const uint4 *>(blk + 16 + t * 32 + h * 16);
     } else {
         const uint8_t *base = a.qs + (size_t)row * a.qs_row_bytes + (size_t)chunk * 128 + 8 * h;
 #pragma unroll
@@ -657,7 +439,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void gemm_rows_kern
                 // rows of x beyond MR alias real ones: they only reach accumulator registers that are never read
                 const _Float16 *xchunk = xt + ((lane & 31) & (MR - 1)) * LDW + local * CK;
                 if constexpr (FMT == FMT_Q4_K) {
-                    const RawChunk<FMT_Q4_K> &r = rc.r;
+                    const RowsChunk<FMT_Q4_K> &r = rc;
                     const float dd = half_bits_to_float(r.hdr.x & 0xFFFFu), dmin = half_bits_to_float(r.hdr.x >> 16);
 #pragma unroll
                     for (int t = 0; t < 4; t++) {
@@ -785,7 +567,8 @@ int choose_splits(int blocks, int units, int min_units, int target, const GemmAr
 
 // `swiglu_out` (may be null) is handed to the tile kernel when it runs without split-K; *fused tells the caller.
 template <int FMT>
-hipError_t launch_format(GemmArgs a, float *workspace, size_t workspace_floats, uint16_t *swiglu_out, bool *fused, int *deferred_splits, hipStream_t stream) {
+hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *deferred_splits, hipStream_t stream) {
+    uint16_t *const swiglu_out = p.swiglu_out;
     *fused = false;
     // split-K partial sums are added by gemm_reduce_kernel, or left to the caller's next kernel when it asked for that
     auto finish = [&](hipError_t err, int used_splits) {
@@ -794,7 +577,7 @@ hipError_t launch_format(GemmArgs a, float *workspace, size_t workspace_floats, 
         return launch_reduce(a, used_splits, stream);
     };
     const int n_blocks = (a.N + NT - 1) / NT;
-    a.partial = workspace;
+    a.partial = p.workspace;
     hipError_t e;
     int splits;
     if constexpr (FMT == FMT_Q4_K || FMT == FMT_Q4_0) {
@@ -821,24 +604,18 @@ hipError_t launch_format(GemmArgs a, float *workspace, size_t workspace_floats, 
             return go(gemm_rows_kernel<FMT, 4, 4>, 4, rows_lds_bytes<4, 4>(), raised4);
         }
     }
-    if constexpr (FMT != FMT_F16) {
-        if (a.M <= 64 && a.K % CK == 0) {
-            const int chunks = a.K / CK;
-            splits = choose_splits(n_blocks, chunks, 2, 1024, a, workspace_floats);
-            a.tiles_per_split = (chunks + splits - 1) / splits;
-            splits = (chunks + a.tiles_per_split - 1) / a.tiles_per_split;
-            dim3 grid(n_blocks, splits, 1);
-            if (a.M <= 32) hipLaunchKernelGGL((gemm_skinny_kernel<FMT, 1, 2>), grid, dim3(kThreads), 0, stream, a);
-            else hipLaunchKernelGGL((gemm_skinny_kernel<FMT, 2, 2>), grid, dim3(kThreads), 0, stream, a);
-            e = hipGetLastError();
-            return finish(e, splits);
-        }
+    if (block_gemm_takes(p)) {
+        e = launch_block_gemm(p, &splits, stream);
+        *fused = splits == 1 && swiglu_out && a.N % 2 == 0;
+        return finish(e, splits);
     }
+    if constexpr (FMT == FMT_Q4_K) return hipErrorInvalidValue;   // whole super-blocks: the kernel above takes them all
+    else {
     const int tiles = a.K / KT;
     const int mt = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
     // (eight wavefronts on a 128 x 256 tile measure 2-5 % faster at 4096 and more weight rows and 10 % slower at 1024;
     //  a 256 x 256 tile is 25 % slower: not instantiated)
-    splits = choose_splits(n_blocks * ((a.M + mt - 1) / mt), tiles, 8, 1024, a, workspace_floats);
+    splits = choose_splits(n_blocks * ((a.M + mt - 1) / mt), tiles, 8, 1024, a, p.workspace_floats);
     a.tiles_per_split = ((tiles + splits - 1) / splits + 3) & ~3;   // every split starts on a multiple of four tiles
     splits = (tiles + a.tiles_per_split - 1) / a.tiles_per_split;
     if (splits == 1 && swiglu_out && a.N % 2 == 0) { a.swiglu_out = swiglu_out; *fused = true; }
@@ -846,6 +623,7 @@ hipError_t launch_format(GemmArgs a, float *workspace, size_t workspace_floats, 
     else if (mt == 64) e = launch_tile<FMT, 1, 4, 2, 1, 4>(a, splits, stream);
     else e = launch_tile<FMT, 2, 2, 2, 2, 2>(a, splits, stream);
     return finish(e, splits);
+    }
 }
 
 }  // namespace
@@ -866,10 +644,10 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t stream) {
     int *const deferred = p.swiglu_out ? &splits : p.deferred_splits;
     hipError_t e;
     switch (w.format) {
-    case FMT_Q4_K: e = launch_format<FMT_Q4_K>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
-    case FMT_Q4_0: e = launch_format<FMT_Q4_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
-    case FMT_Q8_0: e = launch_format<FMT_Q8_0>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
-    case FMT_F16: e = launch_format<FMT_F16>(a, p.workspace, p.workspace_floats, p.swiglu_out, &fused, deferred, stream); break;
+    case FMT_Q4_K: e = launch_format<FMT_Q4_K>(p, a, &fused, deferred, stream); break;
+    case FMT_Q4_0: e = launch_format<FMT_Q4_0>(p, a, &fused, deferred, stream); break;
+    case FMT_Q8_0: e = launch_format<FMT_Q8_0>(p, a, &fused, deferred, stream); break;
+    case FMT_F16: e = launch_format<FMT_F16>(p, a, &fused, deferred, stream); break;
     default: return hipErrorInvalidValue;   // fp32 matrices stay on the GEMV path
     }
     if (e != hipSuccess || !p.swiglu_out || fused) return e;

@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "../common.h"
+#include "block_gemm.h"
 #include "rows_gemm.h"
 
 #include <hip/hip_ext.h>
@@ -2800,6 +2801,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "q4k_mfma_rows8_max") { g_q4k_mfma_rows8_max = value; return true; }
     if (k == "q4k_long_row_waves") { g_q4k_long_row_waves = value; return true; }
     if (k == "q4k_wide") { g_q4k_wide_mode = value; return true; }
+    if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
     if (k == "split_gemm_narrow") { gemm_split_set_narrow(value); return true; }
     if (k == "split_gemm_shared_k") { gemm_split_set_shared_k(value); return true; }
