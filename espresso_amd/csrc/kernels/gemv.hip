@@ -2478,6 +2478,17 @@ hipError_t try_q4k_mfma(const KernelArgs &a, hipStream_t stream, bool *launched)
             if (mode == 1) return launch_q4k_mfma<NB, COLS_ / 64, W_, W_, 1>(a, stream, launched);                 \
             return launch_q4k_mfma<NB, COLS_ / 64, W_, W_, 2>(a, stream, launched);                                \
         }
+        // Output heads have more row blocks than the K-splitting forms have LDS slots for rounds; a wavefront then takes whole rows, as at 4096 columns.  (2048 columns
+        // stay on the persistent dot-product kernel, which reads a 128256-row head at 5.2 TB/s.)  128256 x 3072, arg-max and what follows it: 99 us on the generic kernel (16032 workgroups, as many candidates), 46 here: the 3B step 947 -> 894 us.
+        if (!a.split_x && a.rows > 32768 && (a.cols == 1024 || a.cols == 3072)) {
+            if (a.cols == 1024) {
+                if (mode == 0) return launch_q4k_mfma<NB, 16, 4, 1, 0>(a, stream, launched);
+                if (mode == 1) return launch_q4k_mfma<NB, 16, 4, 1, 1>(a, stream, launched);
+            } else {
+                if (mode == 0) return launch_q4k_mfma<NB, 48, 4, 1, 0>(a, stream, launched);
+                if (mode == 1) return launch_q4k_mfma<NB, 48, 4, 1, 1>(a, stream, launched);
+            }
+        }
         ESP_MFMA_WIDTH(1024, 4)
         ESP_MFMA_WIDTH(2048, 8)
         ESP_MFMA_WIDTH(3072, 12)
