@@ -65,8 +65,10 @@ constexpr size_t block_lds_bytes() {
     return x > sums ? x : sums;
 }
 
-template <int FMT, int TM, int NW>
+// EXACT (Q8_0, Q4_0; one row tile): integers go to the matrix cores, a block's scale to its sums.  Every product then contracts one block, each half of a wavefront holding half of it.
+template <int FMT, int TM, int NW, bool EXACT = false>
 __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
+    static_assert(!EXACT || FMT == FMT_Q8_0 || FMT == FMT_Q4_0, "formats of one scale per block");
     constexpr int KW = kWaves / NW, MT = 32 * TM, GT = 64 * NW, BUFS = block_buffers<TM, NW>();
     constexpr int XP = MT * (kStep / 8) / GT;       // sixteen-byte pieces of the activations per thread and step
     static_assert(MT * (kStep / 8) % GT == 0 && XP >= 1, "whole pieces");
@@ -107,11 +109,11 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     };
     // Weights: lane 16 p + r of a load takes piece p of row r (of row 16 + r in the next), so that four lanes cover 64 bytes of a row; v_permlane16_swap
     // then leaves pieces 2 h and 2 h + 1 of row lane % 32 in each lane.
-    const int piece = lane >> 4;
+    const int piece = EXACT ? 2 * ((lane >> 4) & 1) + h : lane >> 4;   // exact: pieces h and 2 + h
     const uint8_t *wbase = a.qs + (size_t)row0 * a.row_bytes;
     const u32 wlo = (u32)row_of(lane & 15) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + (lane & 15)) * (u32)a.row_bytes + piece * 16;
     const uint16_t *sbase = a.scales + (size_t)row0 * (a.K / 32);
-    const u32 so = (u32)row_of(col) * (u32)(a.K / 32) + (FMT == FMT_Q4_0 ? 2 * h : 0), ho = (u32)row_of(col) * (u32)a.row_bytes;
+    const u32 so = (u32)row_of(col) * (u32)(a.K / 32) + (FMT == FMT_Q4_0 && !EXACT ? 2 * h : 0), ho = (u32)row_of(col) * (u32)a.row_bytes;
     constexpr int PAIRS = pairs_of(FMT);
     uint4 raw[2 * PAIRS], q[2];                 // the next step's stretches as they were loaded; the stretch in use, of the lane's own row
     auto load_pair = [&](int s, int j) __attribute__((always_inline)) {
@@ -125,17 +127,27 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
         swap(raw[2 * j].y, raw[2 * j + 1].y, q[0].y, q[1].y);
         swap(raw[2 * j].z, raw[2 * j + 1].z, q[0].z, q[1].z);
         swap(raw[2 * j].w, raw[2 * j + 1].w, q[0].w, q[1].w);
+        if constexpr (EXACT && FMT == FMT_Q4_0) {   // each half of a wavefront holds a block; it needs bytes 8 h .. of both
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const auto e0 = __builtin_amdgcn_permlane32_swap(q[p].x, q[p].z, false, false);
+                const auto e1 = __builtin_amdgcn_permlane32_swap(q[p].y, q[p].w, false, false);
+                q[p] = make_uint4(e0[0], e1[0], e0[1], e1[1]);
+            }
+        }
     };
-    auto load_scales = [&](int s) __attribute__((always_inline)) {   // Q4_0: blocks 2 h, 2 h + 1; Q8_0: all four
+    auto load_scales = [&](int s) __attribute__((always_inline)) {   // Q4_0: blocks 2 h, 2 h + 1; Q8_0 and exact: all four
         uint2 d = {0, 0};
-        if constexpr (FMT == FMT_Q4_0) d.x = *reinterpret_cast<const u32 *>(sbase + 4 * at(s) + so);
-        if constexpr (FMT == FMT_Q8_0) d = *reinterpret_cast<const uint2 *>(sbase + 4 * at(s) + so);
+        if constexpr (EXACT) d = *reinterpret_cast<const uint2 *>(sbase + 4 * at(s) + so);
+        else if constexpr (FMT == FMT_Q4_0) d.x = *reinterpret_cast<const u32 *>(sbase + 4 * at(s) + so);
+        else if constexpr (FMT == FMT_Q8_0) d = *reinterpret_cast<const uint2 *>(sbase + 4 * at(s) + so);
         return d;
     };
     auto load_hdr = [&](int s) __attribute__((always_inline)) { return *reinterpret_cast<const uint4 *>(wbase + (size_t)(at(s) >> 1) * 144 + ho); };
     // where fragment g (0..7) of a step begins among its 128 k
     auto koff = [&](int g) {
-        return FMT == FMT_Q4_0 ? 64 * h + 8 * g : FMT == FMT_Q4_K ? 64 * h + 32 * (g & 1) + 8 * (g >> 1) : FMT == FMT_Q8_0 ? 64 * (g >> 2) + 32 * h + 8 * (g & 3) : 32 * (g >> 1) + 16 * h + 8 * (g & 1);
+        if constexpr (EXACT) return 32 * (g >> 1) + (FMT == FMT_Q4_0 ? 16 * (g & 1) + 8 * h : 16 * h + 8 * (g & 1));
+        else return FMT == FMT_Q4_0 ? 64 * h + 8 * g : FMT == FMT_Q4_K ? 64 * h + 32 * (g & 1) + 8 * (g >> 1) : FMT == FMT_Q8_0 ? 64 * (g >> 2) + 32 * h + 8 * (g & 3) : 32 * (g >> 1) + 16 * h + 8 * (g & 1);
     };
 
     floatx16 acc[TM];
@@ -158,7 +170,24 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 
     // eight weights of the lane's row as fp16
     auto decode = [&](const uint4 &head, const uint2 &scales, auto odd, int g) __attribute__((always_inline)) {
-        if constexpr (FMT == FMT_Q4_K) {
+        if constexpr (EXACT) {   // fragment g % 2 of block g / 2: q - 8 or q
+            const uint4 &v = q[FMT == FMT_Q4_0 ? g >> 2 : (g >> 1) & 1];
+            const bool upper = FMT == FMT_Q4_0 ? g & 2 : g & 1;
+            const u32 w[2] = {upper ? v.z : v.x, upper ? v.w : v.y};
+            u32 o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (FMT == FMT_Q4_0) {
+                    const u32 mask = g & 1 ? 0x00F000F0u : 0x000F000Fu, magic = g & 1 ? 0x54005400u : 0x64006400u;
+                    const h2 off = g & 1 ? h2{(_Float16)72.0f, (_Float16)72.0f} : h2{(_Float16)1032.0f, (_Float16)1032.0f};
+                    o[j] = as_u32(as_h2(((j & 1 ? w[j >> 1] >> 8 : w[j >> 1]) & mask) | magic) - off);
+                } else {
+                    const h2 off = {(_Float16)1152.0f, (_Float16)1152.0f};   // 1024 + 128
+                    o[j] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, w[j >> 1] ^ 0x80808080u, j & 1 ? 0x04030402u : 0x04010400u)) - off);
+                }
+            }
+            return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
+        } else if constexpr (FMT == FMT_Q4_K) {
             // Sub-block 4 odd + 2 h + g % 2.  A nibble alone in sixteen bits is the fp16 number n 2^-24 (or 16 n 2^-24): n s - dm with product and
             // subtraction in fp32 and one rounding to fp16, as one v_fma_mix a weight.
             const float d = half_bits_to_float(head.x & 0xFFFFu), dmin = half_bits_to_float(head.x >> 16);
@@ -227,6 +256,26 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
             load_x(s + 2);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (EXACT) {
+            const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            floatx16 part[2][TM];   // a block's sums, scaled while the next block is multiplied
+            auto fold = [&](int b) __attribute__((always_inline)) {
+                const u32 pair = b >> 1 ? scale[S].y : scale[S].x;
+                const float d = half_bits_to_float(b & 1 ? pair >> 16 : pair & 0xFFFFu);
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[i][r] = __builtin_fmaf(d, part[b & 1][i][r], acc[i][r]);
+            };
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                if (g + 1 < 8) fragments(g + 1);
+#pragma unroll
+                for (int i = 0; i < TM; i++) part[(g >> 1) & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][i], wf[g & 1], g & 1 ? part[(g >> 1) & 1][i] : zero16, 0, 0, 0);
+                if (g >= 2 && !(g & 1)) fold((g >> 1) - 1);
+            }
+            fold(3);
+        } else
 #pragma unroll
         for (int g = 0; g < 8; g++) {
             if (g + 1 < 8) fragments(g + 1);
@@ -318,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     }
 }
 
-template <int FMT, int TM, int NW>
+template <int FMT, int TM, int NW, bool EXACT>
 hipError_t launch(const BlockArgs &a, hipStream_t stream) {
     static std::atomic<uint64_t> raised{0};   // the limit of dynamic LDS is raised once per kernel and device
     constexpr size_t lds = block_lds_bytes<TM, NW>();
@@ -328,24 +377,25 @@ hipError_t launch(const BlockArgs &a, hipStream_t stream) {
         if (err != hipSuccess) return err;
         const uint64_t bit = 1ull << (device & 63);
         if (!(raised.load(std::memory_order_acquire) & bit)) {
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (err != hipSuccess) return err;
             raised.fetch_or(bit, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW, EXACT>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
     return hipGetLastError();
 }
 
-template <int FMT, int TM>
+template <int FMT, int TM, bool EXACT = false>
 hipError_t launch_width(int nw, const BlockArgs &a, hipStream_t stream) {
-    if (nw == 8) return launch<FMT, TM, 8>(a, stream);
-    if (nw == 4) return launch<FMT, TM, 4>(a, stream);
-    if constexpr (TM < 4) return launch<FMT, TM, 2>(a, stream);   // 128 activation rows for each of four groups: more registers than there are
+    if (nw == 8) return launch<FMT, TM, 8, EXACT>(a, stream);
+    if (nw == 4) return launch<FMT, TM, 4, EXACT>(a, stream);
+    if constexpr (TM < 4) return launch<FMT, TM, 2, EXACT>(a, stream);   // 128 activation rows for each of four groups: more registers than there are
     return hipErrorInvalidValue;
 }
 template <int FMT>
-hipError_t launch_format(int tm, int nw, const BlockArgs &a, hipStream_t stream) {
+hipError_t launch_format(int tm, int nw, bool exact, const BlockArgs &a, hipStream_t stream) {
+    if constexpr (FMT == FMT_Q8_0 || FMT == FMT_Q4_0) if (exact) return launch_width<FMT, 1, true>(nw, a, stream);
     switch (tm) {
     case 1: return launch_width<FMT, 1>(nw, a, stream);
     case 2: return launch_width<FMT, 2>(nw, a, stream);
@@ -360,7 +410,7 @@ struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
 // with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, a kernel of its own).  The
 // constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows, the four formats) and are off by 6 % at the
 // median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst but for fp16.
-Form choose_form(const GemmParams &p) {
+Form choose_form(const GemmParams &p, bool exact) {
     const int fmt = p.w.format, N = p.w.rows, M = p.rows, unit = fmt == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit);
     const bool f16 = fmt == FMT_F16;
     const float start = 2.25f, fill = f16 ? 1.84f : 1.34f, step = f16 ? 1.98f : 0.743f, row_tile = f16 ? 0.0f : 0.149f, staged = 0.1f, join = f16 ? 0.47f : 0.383f;
@@ -368,7 +418,7 @@ Form choose_form(const GemmParams &p) {
     static const int kSplits[] = {1, 2, 3, 4, 6, 8};
     Form best;
     float best_us = 0.0f;
-    for (int tm = 1; tm <= 4 && tm <= (M + 31) / 32; tm++)
+    for (int tm = 1; tm <= (exact ? 1 : 4) && tm <= (M + 31) / 32; tm++)
         for (int nw = tm < 4 ? 2 : 4; nw <= 8; nw *= 2)
             for (int want : kSplits) {
                 const int kw = 8 / nw, per = (units + want * kw - 1) / (want * kw), splits = (units + per * kw - 1) / (per * kw);
@@ -392,6 +442,14 @@ void block_gemm_set_form(int form) {
     g_block_gemm_form.store(known ? form : 0);
 }
 
+// Few rows keep their weights exact where a format has one scale per block: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows).
+// 2048 x 8192 Q4_0, 4 to 31 rows 7.3 to 7.8 us, where the kernel of gemm.hip for eight rows took 15.5 and rows_gemm.hip 13 to 17.
+static bool keeps_exact(const GemmParams &p) { return (p.w.format == FMT_Q8_0 || p.w.format == FMT_Q4_0) && p.rows <= (p.unrounded ? 32 : 8); }
+
+bool block_gemm_exact(const DeviceMatrix &w, int rows) {
+    return w.format == FMT_F16 || ((w.format == FMT_Q8_0 || w.format == FMT_Q4_0) && w.cols % kStep == 0 && rows <= 32);
+}
+
 bool block_gemm_takes(const GemmParams &p) {
     const int fmt = p.w.format;
     if (fmt != FMT_Q4_K && fmt != FMT_Q4_0 && fmt != FMT_Q8_0 && fmt != FMT_F16) return false;
@@ -399,13 +457,15 @@ bool block_gemm_takes(const GemmParams &p) {
     if (fmt != FMT_F16 || g_block_gemm_form.load() > 0) return true;
     // fp16 weights are four times the bytes and nothing to unpack, and planes cost them more than they give: 3072 x 3072, 12 / 128 rows 9.0 / 14.4 us in the tile kernel, 11.2 / 17
     // here; tall matrices do without planes: 11264 x 2048, 93 / 229 / 512 rows 26 / 39 / 61 -> 21 / 31 / 47
-    return p.rows > 64 && p.w.rows >= 8192 && choose_form(p).splits == 1;
+    return p.rows > 64 && p.w.rows >= 8192 && choose_form(p, false).splits == 1;
 }
 
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {
-    Form f = choose_form(p);
+    bool exact = keeps_exact(p);
+    Form f = choose_form(p, exact);
     if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
         f.tm = forced / 100; f.nw = forced / 10 % 10;
+        exact = exact && f.tm == 1;
         const int want = forced % 10, kw = 8 / f.nw, unit = p.w.format == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit), per = (units + want * kw - 1) / (want * kw);
         f.per = per * unit; f.splits = (units + per * kw - 1) / (per * kw);
         if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;
@@ -414,10 +474,10 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
                 (p.w.rows + 32 * f.nw - 1) / (32 * f.nw), (p.rows + 32 * f.tm - 1) / (32 * f.tm)};
     *splits = f.splits;
     switch (p.w.format) {
-    case FMT_Q4_K: return launch_format<FMT_Q4_K>(f.tm, f.nw, a, stream);
-    case FMT_Q4_0: return launch_format<FMT_Q4_0>(f.tm, f.nw, a, stream);
-    case FMT_Q8_0: return launch_format<FMT_Q8_0>(f.tm, f.nw, a, stream);
-    default: return launch_format<FMT_F16>(f.tm, f.nw, a, stream);
+    case FMT_Q4_K: return launch_format<FMT_Q4_K>(f.tm, f.nw, false, a, stream);
+    case FMT_Q4_0: return launch_format<FMT_Q4_0>(f.tm, f.nw, exact, a, stream);
+    case FMT_Q8_0: return launch_format<FMT_Q8_0>(f.tm, f.nw, exact, a, stream);
+    default: return launch_format<FMT_F16>(f.tm, f.nw, false, a, stream);
     }
 }
 

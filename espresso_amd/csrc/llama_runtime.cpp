@@ -1,5 +1,7 @@
 #include "llama_runtime.h"
 
+#include "kernels/block_gemm.h"
+#include "kernels/rows_gemm.h"
 #include "kernels/span_attention.h"
 
 #include <cmath>
@@ -359,6 +361,7 @@ int LlamaRuntime::finalize() {
         const char *pa = getenv("ESPRESSO_HIP_PROMPT_ATTENTION");   // "0": prompt blocks keep the single-query attention kernel
         const bool block_attention = !(pa && pa[0] == '0');
         prompt_attention_ = block_attention && attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
+        short_span_attention_ = block_attention && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
         span_attention_ = block_attention && !prompt_attention_ && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
         const char *fh = getenv("ESPRESSO_HIP_FUSED_HEAD_ARGMAX");   // "0": the head stores logits and separate launches pick the token
         fused_head_argmax_ = !(fh && fh[0] == '0');
@@ -518,10 +521,26 @@ bool LlamaRuntime::split_blocks_supported() const {
 }
 
 // Short blocks that carry activations, weights and attention as exactly as the single-row steps do pay from the fourth token on (8B: a block of 4..32
-// tokens costs 3.4 steps per layer, 1B: 3); blocks of the other formats round what the steps do not, so short prompts keep the steps.  Distance of the last hidden
+// tokens costs 3.4 steps per layer, 1B: 3).  Distance of the last hidden
 // row from 64 bits, 5 / 13 / 24 / 31 tokens, 1B: blocks 8.3 / 5.8 / 4.6 / 4.0e-5, steps 8.4 / 6.2 / 4.9 / 4.9e-5; four layers of 8B: 2.37 / 2.16 / 2.01 / 1.85e-4 and
 // 2.40 / 2.22 / 2.03 / 1.88e-4 (fp16 caches and contexts).
-int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : kMatrixPrefillMinTokens; }
+int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : short_blocks_exact() ? 5 : kMatrixPrefillMinTokens; }
+
+// Blocks whose products keep every weight and whose attention is 32-bit round nothing that the single-row steps of these formats do not: activations and contexts are fp16 in
+// both.  From the fifth token on they are also faster (behind 100 tokens, 4 / 5 / 16 / 31 tokens, steps -> block, us: 6 layers Q8_0 352 / 470 / 1316 / 2583 -> 337 / 324 / 350 / 366;
+// 1.1B Q8_0 1430 / 2131 / 5436 / 11032 -> 1278 / 1259 / 1260 / 1358; 3B Q4_0 1966 / 2782 / 7341 / 14484 -> 2091 / 2061 / 2100 / 2159).
+// Models narrower than 512 columns keep the two-row steps: none is in use, and the tests of those steps count on them (two layers of 256 columns, 7 tokens: 167 us, 93 as a block).
+bool LlamaRuntime::short_blocks_exact() const {
+    if (!short_span_attention_ || c_.d_model < 512) return false;
+    auto ok = [](const DeviceMatrix &m) {
+        GemmParams p;
+        p.w = m; p.rows = kMatrixPrefillMinTokens - 1; p.unrounded = true;
+        return (m.format == FMT_Q8_0 || m.format == FMT_Q4_0 || m.format == FMT_F16) && (block_gemm_exact(m, p.rows) || rows_gemm_takes(p));
+    };
+    for (const Layer &L : layers_)
+        if (!ok(L.wqkv) || !ok(L.wo) || !ok(L.w13) || !ok(L.w2)) return false;
+    return true;
+}
 
 int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
     hipStream_t s = context().stream;
@@ -612,8 +631,9 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_; aa.head_partials = attn_scratch_;
-        if (block_keys && prompt_attention_) ESP_HIP_TRY(launch_attention_prompt(aa, rows, kv16, s));
-        else if (block_keys && span_attention_) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, kv16, s));
+        const bool few = rows < kMatrixPrefillMinTokens && short_span_attention_;   // 32-bit attention, as the steps they stand for
+        if (block_keys && prompt_attention_ && !few) ESP_HIP_TRY(launch_attention_prompt(aa, rows, kv16, s));
+        else if (block_keys && (span_attention_ || few)) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, kv16, s));
         else ESP_HIP_TRY(launch_attention(aa, rows, kv16, s));
         g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_;
         { int rc = project_and_norm(L.rms_ffn); if (rc != ESP_OK) return rc; }

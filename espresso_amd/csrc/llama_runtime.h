@@ -97,6 +97,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool matrix_prefill_supported() const override;
     bool steps_hold_two_rows() const override;
     int matrix_prefill_min_tokens() const override;
+    bool short_blocks_exact() const;
     bool wo_merges_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);
 
@@ -124,6 +125,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool merged_attention_ = true;
     bool split_activations_ = true;
     bool prompt_attention_ = false;   // prompt blocks run attention on the matrix cores
+    bool short_span_attention_ = false;   // span_attention_kernel for blocks of few rows
     bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for
     float *gemm_workspace_ = nullptr;
     GemmSplitSharedK gemm_shared_k_;   // the device's pool for launch_gemm_split's hand-over between workgroups (not owned)

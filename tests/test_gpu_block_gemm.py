@@ -44,6 +44,58 @@ def test_products_match_float64(ops, fmt, rows, cols):
     m.close()
 
 
+@pytest.mark.parametrize("fmt,rows,cols", [("q8_0", 256, 128), ("q8_0", 40, 2304), ("q8_0", 290, 1408), ("q4_0", 4, 128), ("q4_0", 300, 1152), ("q4_0", 72, 8320)])
+def test_few_rows_keep_their_weights(ops, fmt, rows, cols):
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    w = m.dequantize().astype(np.float64)
+    rounded = m.dequantize().astype(np.float16).astype(np.float64)
+    rng = np.random.default_rng(cols)
+    for form in (181, 182, 141, 143, 121, 128):
+        ops.set_tuning("block_gemm_form", form)
+        off, off_rounded = [], []
+        for batch in (3, 5, 8):
+            x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
+            x64 = x.astype(np.float64)
+            got = m.gemv(x)
+            # exact products (integers below 2^8 against 11-bit numbers), one rounding per addition and per scale, relative to the sum of the magnitudes
+            bound = (cols + cols / 16 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w).T + 1)
+            assert (np.abs(got - x64 @ w.T) <= bound).all(), (form, batch)
+            spread = np.sqrt((x64 ** 2) @ (w ** 2).T) + 1e-30
+            off.append(((got - x64 @ w.T) / spread).ravel())
+            off_rounded.append(((x64 @ rounded.T - x64 @ w.T) / spread).ravel())
+        # fp32 sums cost 2^-24 an addition; fp16-rounded weights are off by 2^-12 / sqrt(3) each
+        rms = lambda parts: np.sqrt(np.mean(np.concatenate(parts) ** 2))  # noqa: E731
+        assert rms(off) <= 2.0 ** -21 < rms(off_rounded) / 8, (form, rms(off), rms(off_rounded))
+    ops.set_tuning("block_gemm_form", 0)
+    m.close()
+
+
+@pytest.mark.parametrize("fmt,kv", [("q8_0", lib.FORMAT_F32), ("q4_0", lib.FORMAT_F16), ("f16", lib.FORMAT_F16)])
+@pytest.mark.parametrize("heads,kv_heads", [(12, 12), (12, 4)])
+def test_short_blocks_are_the_steps(ops, fmt, kv, heads, kv_heads):
+    """Prompts of 5 to 31 tokens as one block, behind a prefix and without one, against the same tokens one at a time."""
+    import espresso_amd.llama as ll
+    import espresso_amd.synthetic as syn
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=heads, n_kv_head=kv_heads, d_model=768, head_dim=64, hidden_dim=2304, vocab=260, max_seq=128)
+    rt, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=3, std=0.05, kv_format=kv)
+    tokens = np.random.default_rng(1).integers(0, 260, 80).astype(np.uint32)
+    for prefix, count in ((0, 5), (0, 31), (40, 9), (33, 17)):
+        rt.reset()
+        if prefix:
+            rt.prefill(tokens[:prefix])
+        block = rt.append(tokens[prefix:prefix + count], want=[0, count - 1])
+        rt.set_visible(prefix)
+        steps = []
+        for t in tokens[prefix:prefix + count]:
+            rt.advance(int(t))
+            steps.append(rt.logits())
+        # the same roundings in both: activations and contexts to fp16, where a last bit may fall either way
+        want = np.stack([steps[0], steps[-1]])
+        assert np.abs(block - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max()), (prefix, count)
+    rt.close()
+
+
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_k"])
 def test_gate_up_epilogue_matches_planes(ops, fmt):
     """Prompts through a two-layer model: SiLU(gate) * up in the product's epilogue, and by the launch that adds planes."""
