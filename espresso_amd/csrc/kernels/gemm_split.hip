@@ -21,7 +21,9 @@
 // Per 256 k a wavefront issues 128 + 4 MFMAs and about 200 fold operations.
 #include "../common.h"
 #include "decode_ops.h"
+#include "block_split.h"
 #include "silu.h"
+#include "split_rows.h"
 #include <atomic>
 #include <mutex>
 #include <cmath>
@@ -42,7 +44,9 @@ constexpr int kThreads = 256;
 constexpr int KT = 64;          // k per tile
 constexpr int LDK = KT + 8;     // fp16 per LDS row
 constexpr int NT = 128, MT = 128;
-constexpr float kUnscale = 1.0f / 2048.0f, kScale = 2048.0f;
+using split_rows::kScale;
+using split_rows::kUnscale;
+using split_rows::store_subblock_sum;
 
 struct SplitGemmArgs {
     const uint8_t *qs;
@@ -410,7 +414,6 @@ __global__ __launch_bounds__(kThreads) void gemm_q4k_split_kernel(SplitGemmArgs 
 // is the vector work per MFMA: with every wavefront on all 128 rows and 64 weight rows (RB x CB = 4 x 2) a B fragment serves eight
 // MFMAs instead of four: gate|up of a 512-row block 356 -> 324 us (the kernel above: 421 on the same boxes).  The activation tiles
 // rotate through four LDS buffers so that one barrier serves two tiles (318 -> 313 us, old and new alternating on one box).
-__device__ __forceinline__ void store_subblock_sum(uint16_t *sums, size_t row, int cols, int group, float s);
 constexpr int kRegBBufs = 4;   // activation tiles in LDS: with four, one barrier serves two tiles
 // Whole forms (RB x CB = 4 x 2, 2 x 4): 128 activation rows x 256 weight rows per workgroup.  Narrow forms (CB 1): the four wavefronts side by
 // side along 128 weight rows, each on all 32 RB activation rows, for short blocks and for matrices too small to give every compute
@@ -879,20 +882,6 @@ __device__ __forceinline__ float split_eight(const float (&c)[8], uint4 &hi, uin
     lo = make_uint4(l[0], l[1], l[2], l[3]);
     return s;
 }
-// The sum S of a sub-block (held by the first of each four lanes after the quad reduction) as the pair the GEMM's extra MFMA reads:
-// sums[(row, super-block)][j] = fp16(S), [8 + j] = fp16((S - fp16(S)) * 2048).
-__device__ __forceinline__ void store_subblock_sum(uint16_t *sums, size_t row, int cols, int group, float s) {
-    s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0xB1, 0xF, 0xF, false));
-    s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x4E, 0xF, 0xF, false));
-    if ((group & 3) == 0) {
-        const int sub = group >> 2;   // sub-block of 32 columns
-        uint16_t *p = sums + (row * (size_t)(cols / 256) + (sub >> 3)) * 16 + (sub & 7);
-        const _Float16 h = (_Float16)s;
-        p[0] = __builtin_bit_cast(uint16_t, h);
-        p[8] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(__fsub_rn(s, (float)h), kScale));
-    }
-}
-
 // rows of fp32 values -> split rows; optional RMSNorm ((x * inv) * w, RealModelInferenceEngine.swift:6724-6743) and optional sum of
 // split-K partial planes (+ residual) first, in which case the sums are also written to y.  One workgroup of 256 threads per row;
 // cols % 256 == 0 and cols <= 8192 with the norm (the row is held in registers), any multiple of 256 without.
@@ -1063,7 +1052,8 @@ static int regb_shape_setting() {
 // of 64 (us, launches without split K over 14336 x 4096 pairs): a workgroup alone on its compute unit 0.75 / 0.9 / 1.3 / 1.95 for 32, 64, 128
 // rows x 128 and 128 x 256 (2.35 once more than half of the units have one); several of them on one (three, two, one and one are resident)
 // 0.39 / 0.64 / 1.42 / 2.35 each.  A launch is its longest compute unit's share, a start of about 3 us, and with split K the planes' way to
-// memory and back at about 4 TB/s plus a little.  Where shared K ranges apply, every unit has the same share of whole tiles: those launches keep them.
+// memory and back at about 4 TB/s plus a little, and 0.3 us a plane (the kernels that add them up make a trip to memory for every two: behind 28 to 56 planes of 8 rows 10.8 us,
+// behind one 5).  Where shared K ranges apply, every unit has the same share of whole tiles: those launches keep them.
 // The rule takes the cheapest by that account (us per launch, whole form with splits of at least 1024 columns -> the rule's choice):
 //   8B, gate|up 32 / 64 / 128 / 192 rows 122 / 123 / 126 / 140 -> 48 / 56 / 85 / 127, q|k|v 37 / 38 / 41 / 44 -> 14 / 19 / 25 / 34,
 //   whole layers of 33 / 64 / 128 / 256 / 512 rows 249 / 257 / 270 / 322 / 558 -> 141 / 150 / 196 / 314 / 558
@@ -1081,14 +1071,14 @@ static int device_compute_units() {   // 0: the device does not say
     }
     return n;
 }
-struct RegBForm { int narrow, splits; };
+struct RegBForm { int narrow, splits; float us; };
 static int g_regb_narrow = -1;   // -1: the rule; 0: never narrow; 1, 2, 4: always that form (tests, measurements)
 void gemm_split_set_narrow(int form) { g_regb_narrow = form == 0 || form == 1 || form == 2 || form == 4 ? form : -1; }
 static RegBForm regb_form(int rows, int n, int k, bool may_split, size_t workspace_floats, bool shares_k) {
     struct Form { int rb, cb; float alone, shared; };
     static const Form forms[] = {{1, 1, 0.75f, 0.39f}, {2, 1, 0.9f, 0.64f}, {4, 1, 1.3f, 1.42f}, {4, 2, 1.95f, 2.35f}};
     const int tiles = k / KT, cus = device_compute_units() > 0 ? device_compute_units() : 256;
-    RegBForm best{0, 1};
+    RegBForm best{0, 1, 0.0f};
     if (shares_k && g_regb_narrow <= 0) return best;
     float best_us = INFINITY;
     for (const Form &f : forms) {
@@ -1102,8 +1092,8 @@ static RegBForm regb_form(int rows, int n, int k, bool may_split, size_t workspa
             const long groups = blocks * ((tiles + per - 1) / per), on_one = (groups + cus - 1) / cus;
             float tile_us = on_one > 1 || (!narrow && 2 * groups > cus) ? on_one * f.shared : f.alone;
             if (narrow && tile_us < f.alone + 0.12f * (on_one - 1)) tile_us = f.alone + 0.12f * (on_one - 1);
-            const float us = 3.0f + per * tile_us + (splits > 1 ? 1.0f + (float)splits * rows * n * 8 / 4e6f : 0.0f);
-            if (us < best_us) { best_us = us; best = {narrow, splits}; }
+            const float us = 3.0f + per * tile_us + (splits > 1 ? 1.0f + 0.3f * splits + (float)splits * rows * n * 8 / 4e6f : 0.0f);
+            if (us < best_us) { best_us = us; best = {narrow, splits, us}; }
             if (on_one > 4) break;   // more splits only add planes
         }
     }
@@ -1139,8 +1129,24 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     static const bool lds_weights = [] { const char *e = getenv("ESPRESSO_HIP_SPLIT_GEMM_LDS_WEIGHTS"); return e && atoi(e) != 0; }();
     const bool regb = w.tiled != nullptr && !lds_weights;
     const int tiles = a.K / KT;
-    RegBForm form{0, 1};
+    hipError_t e;
+    RegBForm form{0, 1, 0.0f};
     if (regb && regb_shape_setting() == 4) form = regb_form(a.M, a.N, a.K, !swiglu && p.workspace, p.workspace_floats, swiglu && shared_k_workgroups_for(p, tiles) > 0);
+    // Workgroups that share K among their wavefronts (block_split.hip) where they are expected to be faster, and for every matrix without a tiled copy (512 rows of
+    // 28672 x 4096 389 us in the kernel that stages its weights, 285 there).  Tests that ask for a form of this file get it.
+    if (g_regb_narrow < 0 && !lds_weights && regb_shape_setting() == 4) {
+        const BlockSplitForm f = block_split_form(p);
+        // (behind a SiLU planes cannot split K, and from some 200 rows on whole tiles and shared K ranges win: 28672 x 4096, 256 / 480 rows 138 / 259 us, 150 / 282 there)
+        if (f.tm && (f.us == 0.0f || !regb || (form.us > 0.0f && f.us < form.us && (!swiglu || p.rows <= 128)))) {
+            if (p.deferred_splits) *p.deferred_splits = 1;
+            e = launch_block_split(p, f, stream);
+            if (e != hipSuccess || f.splits == 1) return e;
+            if (p.deferred_splits) { *p.deferred_splits = f.splits; return hipSuccess; }
+            const size_t count = (size_t)a.M * a.N;
+            hipLaunchKernelGGL(split_gemm_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, a.partial, f.splits, count, a.residual, a.y);
+            return hipGetLastError();
+        }
+    }
     const int nt = !regb ? NT : form.narrow ? regb_tile_n(form.narrow, 1) : regb_tile_n(4, 2), mt = form.narrow ? regb_tile_m(form.narrow, 1) : MT;
     const int blocks = ((a.N + nt - 1) / nt) * ((a.M + mt - 1) / mt);
     int splits = form.splits;
@@ -1157,7 +1163,7 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     if (swiglu) { a.sw_hi = p.swiglu.hi; a.sw_lo = p.swiglu.lo; a.sw_sums = regb && (a.N / 2) % 32 == 0 ? p.swiglu.sums : nullptr; }
     static std::atomic<uint64_t> raised{0};
     int device = 0;
-    hipError_t e = hipGetDevice(&device);
+    e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
     const uint64_t bit = 1ull << (device & 63);
     const int regb_shape = regb_shape_setting();

@@ -34,6 +34,7 @@
 
 #include "../common.h"
 #include "block_gemm.h"
+#include "block_split.h"
 #include "rows_gemm.h"
 
 #include <hip/hip_ext.h>
@@ -2814,6 +2815,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "q4k_wide") { g_q4k_wide_mode = value; return true; }
     if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
+    if (k == "block_split_form") { block_split_set_form(value); return true; }
     if (k == "split_gemm_narrow") { gemm_split_set_narrow(value); return true; }
     if (k == "split_gemm_shared_k") { gemm_split_set_shared_k(value); return true; }
     if (k == "prompt_attention_key_sets") { attention_prompt_set_key_sets(value); return true; }

@@ -514,18 +514,25 @@ int LlamaRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int b
 // weights as pairs (in short blocks, which single-row steps could walk as well, 32-bit) in the attention: the block then stays as close to the fp32 CPU walk as
 // the decode steps do.
 bool LlamaRuntime::split_blocks_supported() const {
-    if (!split_activations_ || !xn_lo_ || !prompt_attention_ || c_.kv_format != FMT_F16 || c_.d_model > 8192) return false;
+    return prompt_attention_ && c_.kv_format == FMT_F16 && splits_every_product();
+}
+// Blocks of fewer than 32 rows take the 32-bit attention kernel, whatever the head groups and the caches' format.
+bool LlamaRuntime::short_split_blocks_supported() const { return short_span_attention_ && splits_every_product(); }
+bool LlamaRuntime::splits_every_product() const {
+    if (!split_activations_ || !xn_lo_ || c_.d_model > 8192) return false;
     for (const Layer &L : layers_)
         if (L.q_norm || !gemm_split_supported(L.wqkv) || !gemm_split_supported(L.wo) || !gemm_split_supported(L.w13) || !gemm_split_supported(L.w2)) return false;
     return true;
 }
 
 // Short blocks that carry activations, weights and attention as exactly as the single-row steps do pay from the fourth token on (8B: a block of 4..32
-// tokens costs 3.4 steps per layer, 1B: 3).  Distance of the last hidden
+// tokens costs 3 steps per layer, 1B: 2.5).  Distance of the last hidden
 // row from 64 bits, 5 / 13 / 24 / 31 tokens, 1B: blocks 8.3 / 5.8 / 4.6 / 4.0e-5, steps 8.4 / 6.2 / 4.9 / 4.9e-5; four layers of 8B: 2.37 / 2.16 / 2.01 / 1.85e-4 and
 // 2.40 / 2.22 / 2.03 / 1.88e-4 (fp16 caches and contexts).
-int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : short_blocks_exact() ? 5 : kMatrixPrefillMinTokens; }
+int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : short_split_blocks_supported() || short_blocks_exact() ? 5 : kMatrixPrefillMinTokens; }
 
+// Q4_K models whose long blocks round (three query heads to a key/value head, fp32 caches): from the fifth token on; behind 100 tokens, 4 / 5 / 8 / 31 tokens, 3B 2225 / 3095 /
+// 4272 / 16423 -> 2492 / 2474 / 2467 / 2319 us, four layers of 8B with fp32 caches 567 / 739 / 974 / 3327 -> 696 / 690 / 647 / 629.
 // Blocks whose products keep every weight and whose attention is 32-bit round nothing that the single-row steps of these formats do not: activations and contexts are fp16 in
 // both.  From the fifth token on they are also faster (behind 100 tokens, 4 / 5 / 16 / 31 tokens, steps -> block, us: 6 layers Q8_0 352 / 470 / 1316 / 2583 -> 337 / 324 / 350 / 366;
 // 1.1B Q8_0 1430 / 2131 / 5436 / 11032 -> 1278 / 1259 / 1260 / 1358; 3B Q4_0 1966 / 2782 / 7341 / 14484 -> 2091 / 2061 / 2100 / 2159).
@@ -544,6 +551,7 @@ bool LlamaRuntime::short_blocks_exact() const {
 
 int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
     hipStream_t s = context().stream;
+    const bool kv16 = c_.kv_format == FMT_F16;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const size_t cache_seq_stride = (size_t)kd * c_.max_seq;
     SplitRowsView xn{xn_, xn_lo_, xn_sums_}, ctx{ctx_, ctx_lo_, ctx_sums_}, act{act_, act_lo_, act_sums_};
@@ -569,12 +577,12 @@ int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
         qa.n_head = c_.n_head; qa.n_kv_head = c_.n_kv_head; qa.head_dim = c_.head_dim; qa.max_seq = c_.max_seq;
         qa.rope_cos = rope_cos_; qa.rope_sin = rope_sin_; qa.pos = d_pos_; qa.seq = d_seq_;
         qa.q_out = q_; qa.k_cache = L.k_cache; qa.v_cache = L.v_cache; qa.cache_seq_stride = cache_seq_stride;
-        ESP_HIP_TRY(launch_qkv_post(qa, rows, true, s));
+        ESP_HIP_TRY(launch_qkv_post(qa, rows, kv16, s));
         AttentionArgs aa{};
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_hi = ctx.hi; aa.ctx_lo = ctx.lo; aa.ctx_sums = ctx.sums;
-        if (rows < kMatrixPrefillMinTokens) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, true, s));
+        if (rows < kMatrixPrefillMinTokens) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, kv16, s));
         else ESP_HIP_TRY(launch_attention_prompt(aa, rows, true, s));
         g.w = L.wo; g.x = ctx; g.y = hidden_; g.residual = hidden_; splits = 1;
         ESP_HIP_TRY(launch_gemm_split(g, s));
@@ -593,7 +601,7 @@ int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
 
 // block_keys: the keys that the last row of a prompt block sees; 0 for rows that are not one sequence at consecutive positions.
 int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
-    if (block_keys && split_blocks_supported()) return enqueue_layers_split(rows, block_keys);
+    if (block_keys && (rows < kMatrixPrefillMinTokens ? short_split_blocks_supported() : split_blocks_supported())) return enqueue_layers_split(rows, block_keys);
     hipStream_t s = context().stream;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const bool kv16 = c_.kv_format == FMT_F16;

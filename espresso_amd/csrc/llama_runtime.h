@@ -98,6 +98,8 @@ class LlamaRuntime : public DecoderRuntime {
     bool steps_hold_two_rows() const override;
     int matrix_prefill_min_tokens() const override;
     bool short_blocks_exact() const;
+    bool short_split_blocks_supported() const;
+    bool splits_every_product() const;
     bool wo_merges_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);
 
