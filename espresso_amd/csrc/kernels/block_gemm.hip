@@ -442,9 +442,12 @@ void block_gemm_set_form(int form) {
     g_block_gemm_form.store(known ? form : 0);
 }
 
-// Few rows keep their weights exact where a format has one scale per block: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows).
-// 2048 x 8192 Q4_0, 4 to 31 rows 7.3 to 7.8 us, where the kernel of gemm.hip for eight rows took 15.5 and rows_gemm.hip 13 to 17.
-static bool keeps_exact(const GemmParams &p) { return (p.w.format == FMT_Q8_0 || p.w.format == FMT_Q4_0) && p.rows <= (p.unrounded ? 32 : 8); }
+// Few rows keep their weights exact where a format has one scale per block and the steps they stand for do: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows).  Up to
+// eight rows of Q4_0 always have: 2048 x 8192, 4 to 31 rows 7.3 to 7.8 us, where the kernel of gemm.hip for eight rows took 15.5 and rows_gemm.hip 13 to 17.
+static bool keeps_exact(const GemmParams &p) {
+    if (p.w.format == FMT_Q8_0) return p.unrounded && p.rows <= 32;
+    return p.w.format == FMT_Q4_0 && p.rows <= (p.unrounded ? 32 : 8);
+}
 
 bool block_gemm_exact(const DeviceMatrix &w, int rows) {
     return w.format == FMT_F16 || ((w.format == FMT_Q8_0 || w.format == FMT_Q4_0) && w.cols % kStep == 0 && rows <= 32);
@@ -465,7 +468,7 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
     Form f = choose_form(p, exact);
     if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
         f.tm = forced / 100; f.nw = forced / 10 % 10;
-        exact = exact && f.tm == 1;
+        exact = f.tm == 1 && (exact || (p.w.format == FMT_Q8_0 && p.rows <= 8));   // so that a chosen form reaches every kernel from a single product
         const int want = forced % 10, kw = 8 / f.nw, unit = p.w.format == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit), per = (units + want * kw - 1) / (want * kw);
         f.per = per * unit; f.splits = (units + per * kw - 1) / (per * kw);
         if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;
