@@ -17,7 +17,7 @@ class LayeredRuntime;
 
 constexpr int kPrefillBlockRows = 512;        // rows per MFMA prefill block
 constexpr int kStepsPerGraph = 8;             // greedy steps in the longer of the two captured step graphs
-constexpr int kMatrixPrefillMinTokens = 32;   // shorter prompts take the steps' kernels, two tokens at a time where a step takes two rows
+constexpr int kMatrixPrefillMinTokens = 32;   // shorter prompts take the steps' kernels, two tokens at a time where a step takes two rows, unless the runtime's short blocks are as exact
 constexpr size_t kGemmWorkspaceFloats = (size_t)8 << 20;
 
 struct DecoderShape {
