@@ -14,6 +14,7 @@
 //   * Lane (n = lane % 32, h = lane / 32) loads sixteen bytes of row n at a time.  Which k those are is matched by the activations' addresses:
 //     Q8_0, Q4_K: 32 p + 16 h + 8 i; fp16 and (after the two halves of a wavefront exchanged half of two blocks) Q4_0: 32 p + 16 i + 8 h.
 #include "../common.h"
+#include "block_gemm.h"
 #include "rows_gemm.h"
 #include "silu.h"
 #include <cstdlib>
@@ -321,9 +322,7 @@ bool rows_gemm_takes(const GemmParams &p) {
     const int steps = w.cols / kStep;
     const long groups = (long)((w.rows + 31) / 32) * ((rows + 31) / 32);
     if (w.format == FMT_F16 && w.cols > 1536 && rows <= 64) return false;
-    // up to 32 rows of 2048 columns and more: exact in shares of K that the next kernel adds (block_gemm.hip); 2560 x 2048, 4 / 31 rows q8_0 8.0 / 9.5 -> 6.2 / 6.4, q4_0 6.8 / 8.2 -> 5.3 / 5.5
-    if ((w.format == FMT_Q8_0 || w.format == FMT_Q4_0) && w.cols >= 2048 && w.cols % 128 == 0 && rows <= 32) return false;
-    return w.cols <= 3072 && groups * steps <= 8192;
+    return w.cols <= 3072 && groups * steps <= 8192 && !block_gemm_keeps(p);
 }
 
 hipError_t launch_rows_gemm(const GemmParams &p, hipStream_t stream) {

@@ -117,3 +117,25 @@ def test_gate_up_epilogue_matches_planes(ops, fmt):
     # activations are rounded to fp16 between the products, where a last bit may fall either way
     for form in (243, 481, 0):
         assert np.abs(logits[241] - logits[form]).max() <= 2.0 ** -9 * max(1.0, np.abs(logits[241]).max()), form
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_0"])
+def test_small_products_of_more_rows_keep_their_weights(ops, fmt):
+    """33 to 128 rows of 2048 columns whose weights a step keeps, in shares of K, against one launch without shares (rows_gemm = 2: always that kernel)."""
+    import espresso_amd.llama as ll
+    import espresso_amd.synthetic as syn
+    cfg = ll.MultiModelConfig(n_layer=1, n_head=32, n_kv_head=4, d_model=2048, head_dim=64, hidden_dim=256, vocab=260, max_seq=192)
+    rt, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=3, std=0.05, kv_format=lib.FORMAT_F16)
+    tokens = np.random.default_rng(1).integers(0, 260, 129).astype(np.uint32)
+    try:
+        for count in (34, 64, 65, 96, 128):
+            logits = {}
+            for mode in (1, 2):
+                ops.set_tuning("rows_gemm", mode)
+                rt.reset()
+                logits[mode] = rt.append(tokens[:count], want=[0, 31, 32, count - 1])
+            # fp32 sums in another order; activations are rounded to fp16 between the products, where a last bit may fall either way
+            assert np.abs(logits[1] - logits[2]).max() <= 2.0 ** -9 * max(1.0, np.abs(logits[2]).max()), count
+    finally:
+        ops.set_tuning("rows_gemm", 1)
+        rt.close()
