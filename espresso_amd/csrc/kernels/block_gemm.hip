@@ -444,11 +444,12 @@ void block_gemm_set_form(int form) {
 
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are
 // rounded).  Against rows_gemm.hip, whose wavefronts walk more of K each, 2560 x 2048, 4 / 31 / 93 rows: Q8_0 8.0 / 9.5 / 9.9 -> 6.2 / 6.4 / 7.8 us, Q4_0 6.8 / 8.2 / 8.4 -> 5.3 / 5.5 /
-// 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Behind a SiLU the shares cost a launch, so there only up to 32 rows.
+// 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Behind a SiLU the shares cost a launch, so there only up to 32 rows.  Matrices of
+// fewer rows gain nothing beyond 32 (768 x 2048, 40 / 128 rows Q8_0 6.1 / 6.3 both ways, Q4_0 5.1 / 5.2 against 5.2 / 5.3) and would still pay for the planes.
 bool block_gemm_keeps(const GemmParams &p) {
     if ((p.w.format != FMT_Q8_0 && p.w.format != FMT_Q4_0) || p.w.cols < 2048 || p.w.cols % kStep != 0 || !p.unrounded) return false;
     const long row_blocks = (p.rows + 31) / 32, groups = (long)((p.w.rows + 31) / 32) * row_blocks;
-    return row_blocks == 1 || (row_blocks <= 4 && !p.swiglu_out && p.w.cols <= 3072 && groups * (p.w.cols / 64) <= 8192);
+    return row_blocks == 1 || (row_blocks <= 4 && !p.swiglu_out && p.w.rows >= 2048 && p.w.cols <= 3072 && groups * (p.w.cols / 64) <= 8192);
 }
 
 // Few rows keep their weights exact where a format has one scale per block and the steps they stand for do: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows).  Up to
