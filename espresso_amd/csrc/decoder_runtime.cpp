@@ -231,7 +231,7 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
         given += n;
         return ESP_OK;
     };
-    if (matrix_prefill_ && count >= matrix_prefill_min_tokens() && matrix_prefill_supported()) {
+    if (matrix_prefill_ && block_prefill_pays(count, start) && matrix_prefill_supported()) {
         // blocks of rows through the MFMA kernels (one pass over the weights per block)
         for (int off = 0; off < count; off += block_rows_) {
             const int rows = count - off < block_rows_ ? count - off : block_rows_;

@@ -74,7 +74,7 @@ class DecoderRuntime {
     // consumed.  The step graph notices it on the device; the host looks once per 32 replays.
     int continue_greedy_until_stop(int seq, int steps, uint32_t *out_tokens, int *produced);
     void set_use_graph(bool enabled) { use_graph_ = enabled; }
-    // Prompts of matrix_prefill_min_tokens() or more run in blocks through the MFMA kernels, shorter ones two tokens per step (default on;
+    // Prompts for which block_prefill_pays() run in blocks through the MFMA kernels, others two tokens per step (default on;
     // off: one token per step, whatever the prompt's length).
     void set_matrix_prefill(bool enabled) { matrix_prefill_ = enabled; }
     int read_last_hidden(int seq, float *out);
@@ -122,7 +122,8 @@ class DecoderRuntime {
     // `rows` tokens at positions base.. of one sequence as one block; their rows end in hidden_.
     virtual int prefill_block(int seq, const uint32_t *tokens, int rows, int base) = 0;
     virtual bool matrix_prefill_supported() const = 0;
-    virtual int matrix_prefill_min_tokens() const { return kMatrixPrefillMinTokens; }
+    // Whether `count` tokens behind `base` run in blocks rather than in steps (where the layers take blocks at all).
+    virtual bool block_prefill_pays(int count, int base) const { (void)base; return count >= kMatrixPrefillMinTokens; }
     virtual int clear_state() = 0;                       // every cache and state of every sequence, enqueued on the stream
     virtual unsigned tuning_epoch() const { return 0; }
 

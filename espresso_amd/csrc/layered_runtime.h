@@ -93,7 +93,7 @@ class LayeredRuntime : public DecoderRuntime {
     int enqueue_greedy_token(int seq) override;
     int prefill_block(int seq, const uint32_t *tokens, int rows, int base) override;
     bool matrix_prefill_supported() const override { return true; }
-    int matrix_prefill_min_tokens() const override { return min_block_rows_; }
+    bool block_prefill_pays(int count, int) const override { return count >= min_block_rows_; }
     int clear_state() override;
     int enqueue_step(float *final_out);
     int enqueue_step_sequential(float *final_out);

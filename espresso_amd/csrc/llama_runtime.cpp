@@ -529,7 +529,26 @@ bool LlamaRuntime::splits_every_product() const {
 // tokens costs 3 steps per layer, 1B: 2.5).  Distance of the last hidden
 // row from 64 bits, 5 / 13 / 24 / 31 tokens, 1B: blocks 8.3 / 5.8 / 4.6 / 4.0e-5, steps 8.4 / 6.2 / 4.9 / 4.9e-5; four layers of 8B: 2.37 / 2.16 / 2.01 / 1.85e-4 and
 // 2.40 / 2.22 / 2.03 / 1.88e-4 (fp16 caches and contexts).
-int LlamaRuntime::matrix_prefill_min_tokens() const { return split_blocks_supported() ? 4 : short_split_blocks_supported() || short_blocks_exact() ? 5 : kMatrixPrefillMinTokens; }
+bool LlamaRuntime::block_prefill_pays(int count, int base) const {
+    if (count >= kMatrixPrefillMinTokens) return true;
+    if (count < 4) return false;
+    if (split_blocks_supported()) return true;   // whatever is behind them
+    return count >= 5 && (short_split_blocks_supported() || short_blocks_exact()) && short_block_pays(count, base);
+}
+
+// A short block against the steps it replaces, microseconds per layer.  Its products take as long as two steps; its attention, one workgroup per query head and all keys in
+// that workgroup's eight wavefronts, 0.135 (fp16 caches) or 0.36 ns (fp32) a key and dim.  A step takes its launches and its weights' way from memory, and its attention, whose
+// workgroups share the keys, 0.8 ns a key and the keys' bytes at 2.9 TB/s.  So few tokens behind many keys stay steps: behind 8000 / 16000 keys, 5 tokens, steps -> block, four layers
+// of 8B Q4_K with fp32 caches 1010 / 1340 -> 1930 / 3400 us, of 1B Q4_0 467 / 597 -> 525 / 785, where 31 tokens take 5200 / 7000 -> 1960 / 3460 and 2360 / 3000 -> 540 / 800.  Over 5 to 31
+// tokens behind 16 to 16000 keys of fifteen models (six shapes, the four formats, both caches) the choice is 0.02 % off the faster one on average, 5.3 % at worst.
+bool LlamaRuntime::short_block_pays(int count, int base) const {
+    const Layer &L = layers_[0];
+    const bool kv16 = c_.kv_format == FMT_F16;
+    const float passes = (float)(steps_hold_two_rows() ? (count + 1) / 2 : count), keys = (float)(base + count);
+    const float step = 22.0f + (float)(L.wqkv.bytes() + L.wo.bytes() + L.w13.bytes() + L.w2.bytes()) / 4.5e6f;
+    const float step_key = 0.8e-3f + (float)(2 * c_.kv_dim() * (kv16 ? 2 : 4)) / 2.9e6f, block_key = (float)c_.head_dim * (kv16 ? 0.135e-3f : 0.36e-3f);
+    return passes * (step + keys * step_key) >= 2.0f * step + keys * block_key;
+}
 
 // Q4_K models whose long blocks round (three query heads to a key/value head, fp32 caches): from the fifth token on; behind 100 tokens, 4 / 5 / 8 / 31 tokens, 3B 2225 / 3095 /
 // 4272 / 16423 -> 2492 / 2474 / 2467 / 2319 us, four layers of 8B with fp32 caches 567 / 739 / 974 / 3327 -> 696 / 690 / 647 / 629.

@@ -96,7 +96,8 @@ class LlamaRuntime : public DecoderRuntime {
     int enqueue_layers_sixteen(int rows);
     bool matrix_prefill_supported() const override;
     bool steps_hold_two_rows() const override;
-    int matrix_prefill_min_tokens() const override;
+    bool block_prefill_pays(int count, int base) const override;
+    bool short_block_pays(int count, int base) const;
     bool short_blocks_exact() const;
     bool short_split_blocks_supported() const;
     bool splits_every_product() const;
