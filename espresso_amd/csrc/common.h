@@ -186,6 +186,9 @@ struct SplitRowsParams {
 };
 hipError_t launch_split_rows(const SplitRowsParams &p, hipStream_t stream);
 
+// Of the current device (kernels/gemm_split.hip); 0: it does not say.
+int device_compute_units();
+
 // kernels/gemv.hip
 hipError_t launch_gemv(const GemvParams &p, hipStream_t stream);
 bool gemv_splits_activations(const DeviceMatrix &w, int batch);

@@ -406,7 +406,7 @@ hipError_t launch_format(int tm, int nw, bool exact, const BlockArgs &a, hipStre
 
 struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
 
-// The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of 256 workgroups, a step of a round growing with the tile's rows and
+// The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and
 // with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, a kernel of its own).  The
 // constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows, the four formats) and are off by 6 % at the
 // median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst but for fp16.
@@ -416,6 +416,7 @@ Form choose_form(const GemmParams &p, bool exact) {
     const float start = 2.25f, fill = f16 ? 1.84f : 1.34f, step = f16 ? 1.98f : 0.743f, row_tile = f16 ? 0.0f : 0.149f, staged = 0.1f, join = f16 ? 0.47f : 0.383f;
     const float plane_us = f16 ? 0.233f : 0.28f, again_us = 0.2f;   // per MB
     static const int kSplits[] = {1, 2, 3, 4, 6, 8};
+    const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
     Form best;
     float best_us = 0.0f;
     for (int tm = 1; tm <= (exact ? 1 : 4) && tm <= (M + 31) / 32; tm++)
@@ -425,7 +426,7 @@ Form choose_form(const GemmParams &p, bool exact) {
                 const float mb = (float)splits * (float)M * (float)N * 4e-6f;
                 if (splits != want || (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
                 const long wgs = (long)((N + 32 * nw - 1) / (32 * nw)) * ((M + 32 * tm - 1) / (32 * tm)) * splits;
-                const float rounds = (float)((wgs + 255) / 256);
+                const float rounds = (float)((wgs + cus - 1) / cus);
                 float us = start + rounds * (per * unit * (step + tm * (row_tile + staged * kw)) + fill + (kw > 1 ? join * tm : 0.0f)) + plane_us * mb;
                 if (splits > 1) us += again_us * mb + (p.swiglu_out ? 3.0f : 1.0f);
                 if (!best.tm || us < best_us) { best = Form{tm, nw, per * unit, splits}; best_us = us; }

@@ -357,13 +357,14 @@ void block_split_set_form(int form) {
     g_block_split_form.store(known ? form : 0);
 }
 
-// Expected time, as in block_gemm.hip: rounds of 256 workgroups, a step of a round growing with the tile's rows and with the groups that stage their own activations, planes
+// Expected time, as in block_gemm.hip: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and with the groups that stage their own activations, planes
 // written and read once more.  Fitted to 3300 launches (thirteen shapes of 768 to 28672 weight rows and 768 to 14336 columns, 4 to 480 rows): off by 5 % at the median, 13 at the
 // ninetieth percentile.
 BlockSplitForm block_split_form(const GemmSplitParams &p) {
     const bool swiglu = p.swiglu.hi != nullptr;
     const int N = p.w.rows, M = p.rows, units = p.w.cols / 256, forced = g_block_split_form.load();
     static const int kSplits[] = {1, 2, 3, 4, 6, 8};
+    const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
     BlockSplitForm best;
     if (forced < 0 || (swiglu && (N / 2) % 32 != 0)) return best;
     for (const auto &f : kForms)
@@ -375,7 +376,7 @@ BlockSplitForm block_split_form(const GemmSplitParams &p) {
             const float mb = (float)splits * (float)M * (float)N * 4e-6f;
             if (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats)) continue;
             const long wgs = (long)((N + 32 * f.nw - 1) / (32 * f.nw)) * ((M + 32 * f.tm - 1) / (32 * f.tm)) * splits;
-            float us = 1.4f + (float)((wgs + 255) / 256) * (2 * per * (0.44f + f.tm * (0.433f + 0.227f * kw)) + 1.9f) + 0.363f * mb;
+            float us = 1.4f + (float)((wgs + cus - 1) / cus) * (2 * per * (0.44f + f.tm * (0.433f + 0.227f * kw)) + 1.9f) + 0.363f * mb;
             if (splits > 1) us += 0.2f * mb + 1.0f + 0.3f * splits;
             // what a launch has to win by: the kernel of whole tiles is estimated as well, and large products behind a SiLU take longer here than this says
             us = forced > 0 ? 0.0f : us * (swiglu ? 1.25f : 1.12f);

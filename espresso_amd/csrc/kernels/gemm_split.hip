@@ -1060,7 +1060,7 @@ static int regb_shape_setting() {
 //   1B, gate|up 64 / 128 / 256 / 512 rows 66 / 66 / 68 / 80 -> 26 / 31 / 48 / 76, whole layers 152 / 171 / 186 / 232 -> 83 / 99 / 135 / 210
 // (whole layers: the whole form with splits of 256 columns and more, which is already faster than the splits of 1024 it had before:
 // 1B 64 / 512 rows 200 / 265)
-static int device_compute_units() {   // 0: the device does not say
+int device_compute_units() {
     static std::atomic<int> cus[64];
     int device = 0, n = 0;
     if (hipGetDevice(&device) != hipSuccess) return 0;
