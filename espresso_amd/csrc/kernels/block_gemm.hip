@@ -1,4 +1,4 @@
-// y[m][n] = sum_k x[m][k] * W[n][k] for blocks of activation rows, W in Q4_K, Q4_0, Q8_0 or fp16: fp16 operands (every dequantised weight is rounded to fp16
+// y[m][n] = sum_k x[m][k] * W[n][k] for blocks of activation rows, W in Q4_K, Q4_0, Q8_0 or (tall gate|up) fp16: fp16 operands (every dequantised weight is rounded to fp16
 // once), fp32 sums.
 //
 // A workgroup is eight wavefronts, two on every SIMD, so that one unpacks weights while the other multiplies.  NW of them lie side by side along 32 NW weight rows and
@@ -405,6 +405,7 @@ hipError_t launch_format(int tm, int nw, bool exact, const BlockArgs &a, hipStre
 }
 
 struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
+std::atomic<int> g_block_gemm_form{0};
 
 // The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and
 // with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, a kernel of its own).  The
@@ -436,11 +437,10 @@ Form choose_form(const GemmParams &p, bool exact) {
 
 }  // namespace
 
-static std::atomic<int> g_block_gemm_form{0};
 void block_gemm_set_form(int form) {
     const int tm = form / 100, nw = form / 10 % 10, shares = form % 10;
     const bool known = tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
-    g_block_gemm_form.store(known ? form : 0);
+    g_block_gemm_form.store(known || form == -1 ? form : 0);
 }
 
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are
@@ -468,10 +468,17 @@ bool block_gemm_takes(const GemmParams &p) {
     const int fmt = p.w.format;
     if (fmt != FMT_Q4_K && fmt != FMT_Q4_0 && fmt != FMT_Q8_0 && fmt != FMT_F16) return false;
     if (p.w.cols % (fmt == FMT_Q4_K ? 256 : kStep) != 0) return false;
-    if (fmt != FMT_F16 || g_block_gemm_form.load() > 0) return true;
+    const int forced = g_block_gemm_form.load();
+    if (fmt != FMT_F16 || forced > 0) return true;
     // fp16 weights are four times the bytes and nothing to unpack, and planes cost them more than they give: 3072 x 3072, 12 / 128 rows 9.0 / 14.4 us in the tile kernel, 11.2 / 17
-    // here; tall matrices do without planes: 11264 x 2048, 93 / 229 / 512 rows 26 / 39 / 61 -> 21 / 31 / 47
-    return p.rows > 64 && p.w.rows >= 8192 && choose_form(p, false).splits == 1;
+    // here.  Tall gate|up matrices do without planes and win here while the tile kernel has no more than one workgroup of 128 x 128 a compute unit; with more of them it hides its
+    // staging (us, there -> here): 11264 x 2048, 96 / 192 / 256 / 384 / 512 rows 27 / 33 / 34 / 38 / 39 -> 21 / 29 / 32 / 45 / 47; 16384 x 3072, 96 / 256 / 384 rows 38 / 54 / 59 -> 32 / 48 / 67;
+    // 28672 x 4096, 96 / 256 / 384 rows 78 / 93 / 129 -> 64 / 97 / 159.  Over nine heights of 8192 to 32000 rows, 1024 to 8192 columns and 65 to 512 rows of activations, what the rule takes
+    // is 0.97 to 1.6 times as fast.  Longer rows gain nothing (8192 columns: 0.96 to 1.02 at up to 128 rows; 4096 columns beyond 128 rows 0.85 to 1.4), nor do products without the SiLU
+    // (14336 x 2048, 96 / 129 / 256 rows 1.01 / 1.29 / 0.92 times as fast).
+    if (forced < 0 || !p.swiglu_out || p.rows <= 64 || p.w.rows < 8192 || p.w.cols > (p.rows <= 128 ? 4096 : 3072)) return false;
+    const long tiles = (long)((p.w.rows + 127) / 128) * ((p.rows + 127) / 128);
+    return tiles <= (device_compute_units() > 0 ? device_compute_units() : 256) && choose_form(p, false).splits == 1;
 }
 
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {

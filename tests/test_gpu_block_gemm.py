@@ -119,6 +119,27 @@ def test_gate_up_epilogue_matches_planes(ops, fmt):
         assert np.abs(logits[241] - logits[form]).max() <= 2.0 ** -9 * max(1.0, np.abs(logits[241]).max()), form
 
 
+def test_tall_fp16_products_leave_long_prompts_to_the_tile_kernel(ops):
+    """gate|up of 11264 x 512 in fp16: up to 256 rows here, beyond it (more than a tile of 128 x 128 for every compute unit) in the kernel of gemm.hip."""
+    import espresso_amd.llama as ll
+    import espresso_amd.synthetic as syn
+    cfg = ll.MultiModelConfig(n_layer=1, n_head=8, n_kv_head=8, d_model=512, head_dim=64, hidden_dim=5632, vocab=260, max_seq=512)
+    rt, _ = syn.build_runtime(cfg, lib.FORMAT_F16, seed=3, std=0.05)
+    tokens = np.random.default_rng(1).integers(0, 260, 512).astype(np.uint32)
+    try:
+        for count, here in ((64, False), (65, True), (256, True), (257, False), (384, False), (512, False)):
+            logits = {}
+            for form in (0, -1):
+                ops.set_tuning("block_gemm_form", form)
+                rt.reset()
+                logits[form] = rt.append(tokens[:count], want=[0, 31, 32, count - 1])
+            assert np.array_equal(logits[0], logits[-1]) != here, count   # the kernels add in another order
+            assert np.abs(logits[0] - logits[-1]).max() <= 2.0 ** -9 * max(1.0, np.abs(logits[-1]).max()), count
+    finally:
+        ops.set_tuning("block_gemm_form", 0)
+        rt.close()
+
+
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_0"])
 def test_small_products_of_more_rows_keep_their_weights(ops, fmt):
     """33 to 128 rows of 2048 columns whose weights a step keeps, in shares of K, against one launch without shares (rows_gemm = 2: always that kernel)."""
