@@ -6,6 +6,8 @@
 namespace esp {
 
 bool block_gemm_takes(const GemmParams &p);
+// No caller adds shares of K: their sum is a launch of its own.
+inline bool block_gemm_alone(const GemmParams &p) { return !p.deferred_splits && !p.swiglu_out; }
 // Exact here rather than in the kernel of rows_gemm.hip?
 bool block_gemm_keeps(const GemmParams &p);
 // Do products of up to `rows` rows that need not round their weights (GemmParams::unrounded) keep them as they are?

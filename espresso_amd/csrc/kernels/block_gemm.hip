@@ -408,7 +408,8 @@ struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
 std::atomic<int> g_block_gemm_form{0};
 
 // The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and
-// with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, a kernel of its own).  The
+// with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, and where no
+// caller adds them, a launch of its own: 1.6 to 4.3 us; the form that rule chooses is 1 % off the best on average, 11 at worst, 256 x 256).  The
 // constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows, the four formats) and are off by 6 % at the
 // median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst but for fp16.
 Form choose_form(const GemmParams &p, bool exact) {
@@ -429,7 +430,7 @@ Form choose_form(const GemmParams &p, bool exact) {
                 const long wgs = (long)((N + 32 * nw - 1) / (32 * nw)) * ((M + 32 * tm - 1) / (32 * tm)) * splits;
                 const float rounds = (float)((wgs + cus - 1) / cus);
                 float us = start + rounds * (per * unit * (step + tm * (row_tile + staged * kw)) + fill + (kw > 1 ? join * tm : 0.0f)) + plane_us * mb;
-                if (splits > 1) us += again_us * mb + (p.swiglu_out ? 3.0f : 1.0f);
+                if (splits > 1) us += again_us * mb + (p.swiglu_out ? 3.0f : p.deferred_splits ? 1.0f : 1.6f + 0.2f * splits);
                 if (!best.tm || us < best_us) { best = Form{tm, nw, per * unit, splits}; best_us = us; }
             }
     return best;
@@ -447,17 +448,19 @@ void block_gemm_set_form(int form) {
 // rounded).  Against rows_gemm.hip, whose wavefronts walk more of K each, 2560 x 2048, 4 / 31 / 93 rows: Q8_0 8.0 / 9.5 / 9.9 -> 6.2 / 6.4 / 7.8 us, Q4_0 6.8 / 8.2 / 8.4 -> 5.3 / 5.5 /
 // 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Behind a SiLU the shares cost a launch, so there only up to 32 rows.  Matrices of
 // fewer rows gain nothing beyond 32 (768 x 2048, 40 / 128 rows Q8_0 6.1 / 6.3 both ways, Q4_0 5.1 / 5.2 against 5.2 / 5.3) and would still pay for the planes.
+// Where no caller adds the shares, their launch outweighs them as long as the other kernel's workgroups are resident at once (with that launch, 8 rows Q4_0: 2048 x 2048 8.6 us, 6.7
+// there; 3072 x 3072 9.4, 7.4; 5632 x 2048 10.3, 6.9; 8192 x 3072 10.5, 9.2; 11264 x 2048 9.8, 12.6).
 bool block_gemm_keeps(const GemmParams &p) {
     if ((p.w.format != FMT_Q8_0 && p.w.format != FMT_Q4_0) || p.w.cols < 2048 || p.w.cols % kStep != 0 || !p.unrounded) return false;
     const long row_blocks = (p.rows + 31) / 32, groups = (long)((p.w.rows + 31) / 32) * row_blocks;
+    if (block_gemm_alone(p) && groups <= (device_compute_units() > 0 ? device_compute_units() : 256)) return false;
     return row_blocks == 1 || (row_blocks <= 4 && !p.swiglu_out && p.w.rows >= 2048 && p.w.cols <= 3072 && groups * (p.w.cols / 64) <= 8192);
 }
 
-// Few rows keep their weights exact where a format has one scale per block and the steps they stand for do: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows).  Up to
-// eight rows of Q4_0 always have: 2048 x 8192, 4 to 31 rows 7.3 to 7.8 us, where the kernel of gemm.hip for eight rows took 15.5 and rows_gemm.hip 13 to 17.
+// Few rows keep their weights exact where a format has one scale per block and the steps they stand for do: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows; with shares
+// added by the next kernel 2048 x 8192, 4 to 31 rows 7.3 to 7.8 us, in rows_gemm.hip 13 to 17).
 static bool keeps_exact(const GemmParams &p) {
-    if (p.w.format != FMT_Q8_0 && p.w.format != FMT_Q4_0) return false;
-    return p.unrounded ? p.rows <= 32 || block_gemm_keeps(p) : p.w.format == FMT_Q4_0 && p.rows <= 8;
+    return (p.w.format == FMT_Q8_0 || p.w.format == FMT_Q4_0) && p.unrounded && (p.rows <= 32 || block_gemm_keeps(p));
 }
 
 bool block_gemm_exact(const DeviceMatrix &w, int rows) {

@@ -160,3 +160,30 @@ def test_small_products_of_more_rows_keep_their_weights(ops, fmt):
     finally:
         ops.set_tuning("rows_gemm", 1)
         rt.close()
+
+
+@pytest.mark.parametrize("fmt,rows,cols,batch,key,value", [
+    ("q4_0", 256, 256, 3, "rows_gemm", 2), ("q4_0", 768, 768, 8, "rows_gemm", 2), ("q4_0", 2048, 2048, 5, "rows_gemm", 2), ("q4_0", 5632, 2048, 8, "rows_gemm", 2), ("q4_0", 8192, 3072, 3, "rows_gemm", 2),
+    ("q4_0", 11264, 2048, 8, "rows_gemm", 0), ("q4_0", 2048, 5632, 8, "rows_gemm", 0),   # more workgroups than compute units, long rows: here
+    ("q8_0", 768, 768, 16, "block_gemm_form", 121), ("q4_k", 2048, 2048, 16, "block_gemm_form", 122),   # no shares of K whose sum is a launch
+])
+def test_single_products_pay_for_no_launch_that_adds_shares(ops, fmt, rows, cols, batch, key, value):
+    """A matrix handle's product has no next kernel that could add shares of K: where those and their launch cost more than they give, another form is taken.
+    Forms that split K differently add in another order, so equal bits are the same split."""
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    x = np.random.default_rng(cols).normal(0, 1, (batch, cols)).astype(np.float16)
+    default = m.gemv(x)
+    try:
+        ops.set_tuning(key, value)
+        assert np.array_equal(default, m.gemv(x))
+    finally:
+        ops.set_tuning("rows_gemm", 1)
+        ops.set_tuning("block_gemm_form", 0)
+    w = m.dequantize()
+    w = (w if fmt == "q4_0" else w.astype(np.float16)).astype(np.float64)
+    bound = (cols + cols / 16 + 16) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + 1)   # as above
+    if fmt == "q4_k":
+        bound = bound + 4 * 2.0 ** -11 * np.abs(x).max(1).astype(np.float64)[:, None] * np.abs(w).max()
+    assert (np.abs(default - x.astype(np.float64) @ w.T) <= bound).all()
+    m.close()
