@@ -2479,16 +2479,17 @@ hipError_t try_q4k_mfma(const KernelArgs &a, hipStream_t stream, bool *launched)
             if (mode == 1) return launch_q4k_mfma<NB, COLS_ / 64, W_, W_, 1>(a, stream, launched);                 \
             return launch_q4k_mfma<NB, COLS_ / 64, W_, W_, 2>(a, stream, launched);                                \
         }
-        // Output heads have more row blocks than the K-splitting forms have LDS slots for rounds; a wavefront then takes whole rows, as at 4096 columns.  (2048 columns
-        // stay on the persistent dot-product kernel, which reads a 128256-row head at 5.2 TB/s.)  128256 x 3072, arg-max and what follows it: 99 us on the generic kernel (16032 workgroups, as many candidates), 46 here: the 3B step 947 -> 894 us.
-        if (!a.split_x && a.rows > 32768 && (a.cols == 1024 || a.cols == 3072)) {
-            if (a.cols == 1024) {
-                if (mode == 0) return launch_q4k_mfma<NB, 16, 4, 1, 0>(a, stream, launched);
-                if (mode == 1) return launch_q4k_mfma<NB, 16, 4, 1, 1>(a, stream, launched);
-            } else {
-                if (mode == 0) return launch_q4k_mfma<NB, 48, 4, 1, 0>(a, stream, launched);
-                if (mode == 1) return launch_q4k_mfma<NB, 48, 4, 1, 1>(a, stream, launched);
-            }
+        // Tall output heads have more row blocks than the K-splitting forms have LDS slots for rounds (131072 rows of 1024 columns, 32768 of 3072, on 256 compute units): those forms
+        // decline, and a wavefront takes whole rows, as at 4096 columns.  (2048 columns stay on the persistent dot-product kernel, which reads a 128256-row head at 5.2 TB/s.)
+        // Head and arg-max, generic kernel (16032 workgroups, as many candidates) -> here, us: 3072 columns, 32784 / 128256 rows 21 / 72 -> 14 / 34 (the 3B step 947 -> 894);
+        // 1024 columns, 131088 / 151936 rows 44 / 51 -> 15 / 17.  Where the K-splitting forms do launch they are faster: 1024 columns, 32784 / 40960 / 100352 / 128256 rows 5.4 /
+        // 6.1 / 11.8 / 14.6 us, whole rows 7.1 / 7.4 / 13.7 / 15.5.
+        if (!a.split_x && mode != 2 && (a.cols == 1024 || a.cols == 3072)) {
+            const hipError_t e = a.cols == 1024 ? (mode == 0 ? launch_q4k_mfma<NB, 16, 4, 4, 0>(a, stream, launched) : launch_q4k_mfma<NB, 16, 4, 4, 1>(a, stream, launched))
+                                                : (mode == 0 ? launch_q4k_mfma<NB, 48, 12, 12, 0>(a, stream, launched) : launch_q4k_mfma<NB, 48, 12, 12, 1>(a, stream, launched));
+            if (e != hipSuccess || *launched) return e;
+            if (a.cols == 1024) return mode == 0 ? launch_q4k_mfma<NB, 16, 4, 1, 0>(a, stream, launched) : launch_q4k_mfma<NB, 16, 4, 1, 1>(a, stream, launched);
+            return mode == 0 ? launch_q4k_mfma<NB, 48, 4, 1, 0>(a, stream, launched) : launch_q4k_mfma<NB, 48, 4, 1, 1>(a, stream, launched);
         }
         ESP_MFMA_WIDTH(1024, 4)
         ESP_MFMA_WIDTH(2048, 8)
