@@ -160,6 +160,48 @@ int esp_gemv(const ESPMatrix *matrix, const uint16_t *x_f16, int batch, float *y
     return e == hipSuccess ? ESP_OK : fail_hip(e, "gemv");
 }
 
+int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares) {
+    if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: null pointer");
+    if (rows <= 0 || rows > 512) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: rows %d", rows);
+    int rc = ensure_init();
+    if (rc != ESP_OK) return rc;
+    Context &c = context();
+    const DeviceMatrix &m = matrix->m;
+    if (m.format == FMT_F32 || m.cols % 64 != 0) return fail(ESP_ERR_UNSUPPORTED, "layer_product: matrices on the matrix cores");
+    const size_t nx = (size_t)rows * m.cols, ny = (size_t)rows * m.rows;
+    uint16_t *d_x = nullptr;
+    float *d_y = nullptr, *d_ws = nullptr;
+    auto release = [&] {
+        void *ptrs[] = {d_x, d_y, d_ws};
+        for (void *p : ptrs) if (p) (void)hipFree(p);
+    };
+    if ((rc = device_alloc(&d_x, nx)) != ESP_OK || (rc = device_alloc(&d_y, ny)) != ESP_OK || (rc = device_alloc(&d_ws, kGemmWorkspaceFloats)) != ESP_OK) {
+        release();
+        return rc;
+    }
+    int splits = 1;
+    hipError_t e = hipMemcpyAsync(d_x, x_f16, nx * 2, hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess && residual) e = hipMemcpyAsync(d_y, residual, ny * 4, hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess) {
+        GemmParams g;
+        g.w = m; g.x = d_x; g.y = d_y; g.residual = residual ? d_y : nullptr; g.rows = rows; g.unrounded = true; g.workspace = d_ws; g.workspace_floats = kGemmWorkspaceFloats;
+        if (shares) g.deferred_splits = &splits;
+        e = launch_gemm(g, c.stream);
+    }
+    std::vector<float> planes(splits > 1 ? splits * ny : 0);
+    if (e == hipSuccess && splits > 1) e = hipMemcpyAsync(planes.data(), d_ws, planes.size() * 4, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(y, d_y, ny * 4, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    release();
+    if (e != hipSuccess) return fail_hip(e, "layer_product");
+    for (size_t i = 0; i < ny && splits > 1; i++) {
+        float sum = planes[i];
+        for (int s = 1; s < splits; s++) sum += planes[s * ny + i];
+        y[i] = residual ? residual[i] + sum : sum;
+    }
+    return ESP_OK;
+}
+
 int esp_matmul_f32(const ESPMatrix *matrix, const float *x, int rows, float *y, const float *residual) {
     if (!matrix || !x || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "matmul_f32: null pointer");
     if (rows <= 0) return fail(ESP_ERR_INVALID_ARGUMENT, "matmul_f32: rows %d", rows);

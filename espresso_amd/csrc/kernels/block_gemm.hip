@@ -489,7 +489,7 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
     Form f = choose_form(p, exact);
     if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
         f.tm = forced / 100; f.nw = forced / 10 % 10;
-        exact = f.tm == 1 && (exact || (p.w.format == FMT_Q8_0 && p.rows <= 8));   // so that a chosen form reaches every kernel from a single product
+        exact = exact && f.tm == 1;   // forms of more row tiles have no exact kernel
         const int want = forced % 10, kw = 8 / f.nw, unit = p.w.format == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit), per = (units + want * kw - 1) / (want * kw);
         f.per = per * unit; f.splits = (units + per * kw - 1) / (per * kw);
         if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;

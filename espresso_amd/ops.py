@@ -93,6 +93,17 @@ class Matrix:
         _lib.check(_lib.load_library().esp_gemv(self._h, _ptr(x), batch, _ptr(y), _ptr(res) if res is not None else None))
         return y
 
+    def layer_product(self, x_f16: np.ndarray, residual: np.ndarray | None = None, shares: bool = False) -> np.ndarray:
+        """The product as a model's layers ask for it, weights unrounded where a kernel keeps them (esp_layer_product; test aid)."""
+        x = np.ascontiguousarray(x_f16, dtype=np.float16).reshape(-1, self.cols)
+        rows = x.shape[0]
+        y = np.empty((rows, self.rows), dtype=np.float32)
+        res = None
+        if residual is not None:
+            res = np.ascontiguousarray(residual, dtype=np.float32).reshape(rows, self.rows)
+        _lib.check(_lib.load_library().esp_layer_product(self._h, _ptr(x), rows, _ptr(y), _ptr(res) if res is not None else None, int(shares)))
+        return y
+
     def matmul_f32(self, x: np.ndarray, residual: np.ndarray | None = None) -> np.ndarray:
         """fp32 activations [rows][cols] against the matrix with no operand rounded (esp_matmul_f32; Q4_K)."""
         x = np.ascontiguousarray(x, dtype=np.float32).reshape(-1, self.cols)

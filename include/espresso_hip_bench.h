@@ -57,6 +57,10 @@ long long esp_matrix_read_tiled(const ESPMatrix *matrix, void *out, size_t capac
  * (a mismatch fails the call); tuning key split_gemm_shared_k selects how
  * workgroups share an output tile's K range (0 never, 1 where it applies, 2 as 1 with the finishing workgroup never waiting). */
 int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, float *act);
+/* Test aid: the product as the layers of a model ask for it, x [rows][cols] fp16: weights stay unrounded where a kernel for that many rows keeps them, rounded to fp16 once elsewhere.
+ * shares = 1: the launch may leave its sum in shares of K, as in front of a norm or the key/value caches; they and the residual are then added here, in the shares' order.
+ * y, residual (may be NULL) [rows][matrix rows] fp32; host pointers. */
+int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares);
 /* Test aid: causal attention of `rows` (up to 512) consecutive rows of one sequence at positions first, first + 1, ... by one of the kernels a model's
  * layers use.  q [rows][heads][head_dim] fp32; k, v [first + rows][kv_heads][head_dim] fp32, or fp16 bits with kv_f16; ctx [rows][heads][head_dim]
  * as fp32: the fp16 context, or with split_rows the two fp16 planes added back together (hi + lo / 2048).  Host pointers.  `iters` launches;

@@ -44,30 +44,86 @@ def test_products_match_float64(ops, fmt, rows, cols):
     m.close()
 
 
-@pytest.mark.parametrize("fmt,rows,cols", [("q8_0", 256, 128), ("q8_0", 40, 2304), ("q8_0", 290, 1408), ("q4_0", 4, 128), ("q4_0", 300, 1152), ("q4_0", 72, 8320)])
-def test_few_rows_keep_their_weights(ops, fmt, rows, cols):
-    f = lib.FORMAT_NAMES[fmt]
-    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+def check_kept(m, product, batches, rng):
+    """Products that keep every weight: within the rounding of fp32 sums, and far below what weights rounded to fp16 would be off."""
     w = m.dequantize().astype(np.float64)
     rounded = m.dequantize().astype(np.float16).astype(np.float64)
-    rng = np.random.default_rng(cols)
-    for form in (181, 182, 141, 143, 121, 128):
-        ops.set_tuning("block_gemm_form", form)
-        off, off_rounded = [], []
-        for batch in (3, 5, 8):
-            x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
-            x64 = x.astype(np.float64)
-            got = m.gemv(x)
-            # exact products (integers below 2^8 against 11-bit numbers), one rounding per addition and per scale, relative to the sum of the magnitudes
-            bound = (cols + cols / 16 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w).T + 1)
-            assert (np.abs(got - x64 @ w.T) <= bound).all(), (form, batch)
-            spread = np.sqrt((x64 ** 2) @ (w ** 2).T) + 1e-30
-            off.append(((got - x64 @ w.T) / spread).ravel())
-            off_rounded.append(((x64 @ rounded.T - x64 @ w.T) / spread).ravel())
+    off, off_rounded = [], []
+    for batch in batches:
+        x = rng.normal(0, 1, (batch, m.cols)).astype(np.float16)
+        residual = rng.normal(0, 1e-3, (batch, m.rows)).astype(np.float32) if batch % 2 else None
+        x64 = x.astype(np.float64)
+        want = x64 @ w.T + (0 if residual is None else residual)
+        got = product(x, residual)
+        # exact products (integers below 2^8 against 11-bit numbers), one rounding per addition and per scale, relative to the sum of the magnitudes
+        bound = (m.cols + m.cols / 16 + 16) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w).T + 1)
+        assert (np.abs(got - want) <= bound).all(), batch
+        spread = np.sqrt((x64 ** 2) @ (w ** 2).T) + 1e-30
+        off.append(((got - want) / spread).ravel())
+        off_rounded.append(((x64 @ rounded.T - x64 @ w.T) / spread).ravel())
         # fp32 sums cost 2^-24 an addition; fp16-rounded weights are off by 2^-12 / sqrt(3) each
-        rms = lambda parts: np.sqrt(np.mean(np.concatenate(parts) ** 2))  # noqa: E731
-        assert rms(off) <= 2.0 ** -21 < rms(off_rounded) / 8, (form, rms(off), rms(off_rounded))
-    ops.set_tuning("block_gemm_form", 0)
+        rms = lambda v: np.sqrt(np.mean(v ** 2))  # noqa: E731
+        assert batch < 9 or rms(off[-1]) <= 2.0 ** -21 < rms(off_rounded[-1]) / 8, (batch, rms(off[-1]), rms(off_rounded[-1]))
+    off, off_rounded = rms(np.concatenate(off)), rms(np.concatenate(off_rounded))
+    assert off <= 2.0 ** -21 < off_rounded / 8, (off, off_rounded)
+
+
+@pytest.mark.parametrize("fmt,rows,cols", [("q8_0", 256, 128), ("q8_0", 40, 2304), ("q8_0", 290, 1408), ("q4_0", 4, 128), ("q4_0", 300, 1152), ("q4_0", 72, 8320)])
+def test_few_rows_keep_their_weights(ops, fmt, rows, cols):
+    """Up to 32 rows, every exact form."""
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    rng = np.random.default_rng(cols)
+    ops.set_tuning("rows_gemm", 0)
+    try:
+        for form in (181, 182, 141, 143, 121, 128):
+            ops.set_tuning("block_gemm_form", form)
+            check_kept(m, lambda x, r: m.layer_product(x, r, shares=form % 4 != 0), (3, 5, 8, 9, 31, 32), rng)
+    finally:
+        ops.set_tuning("block_gemm_form", 0)
+        ops.set_tuning("rows_gemm", 1)
+    m.close()
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_0"])
+@pytest.mark.parametrize("rows,cols,batches", [(2048, 2048, (9, 31, 33, 64, 65, 97, 128)), (2090, 2048, (33, 64, 65, 96)), (2075, 2304, (32, 33, 61)), (2048, 3072, (9, 33, 64)),
+                                               (768, 2048, (9, 32, 33, 128)), (300, 768, (9, 33, 128)), (2090, 5632, (3, 9, 31, 32))])
+def test_rules_keep_weights_of_small_products(ops, fmt, rows, cols, batches):
+    """What the layers' products take by size: here (one to four row tiles, with and without shares of K, ragged weight rows) or in rows_gemm.hip."""
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    rng = np.random.default_rng(cols)
+    check_kept(m, lambda x, r: m.layer_product(x, r, shares=True), batches, rng)
+    check_kept(m, lambda x, r: m.layer_product(x, r), batches, rng)
+    if cols >= 2048 and rows >= 2048:
+        ops.set_tuning("rows_gemm", 0)
+        try:
+            for form in (181, 143, 121, 124):   # the same products here whatever the rule
+                ops.set_tuning("block_gemm_form", form)
+                check_kept(m, lambda x, r: m.layer_product(x, r, shares=True), batches, rng)
+        finally:
+            ops.set_tuning("block_gemm_form", 0)
+            ops.set_tuning("rows_gemm", 1)
+    m.close()
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_k"])
+def test_forms_do_not_change_how_weights_are_rounded(ops, fmt):
+    """A chosen form is the same product: a handle's five rows of Q8_0 round their weights as they do by size."""
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, 7, 0.02, 300 * 1024), 300, 1024)
+    w = m.dequantize()
+    x = np.random.default_rng(2).normal(0, 1, (9 if fmt == "q4_k" else 5, 1024)).astype(np.float16)
+    x64 = x.astype(np.float64)
+    spread = np.sqrt((x64 ** 2) @ (w.astype(np.float64) ** 2).T)
+    rms = lambda v: np.sqrt(np.mean((v / spread) ** 2))  # noqa: E731
+    try:
+        for form in (0, 181, 143, 121):
+            ops.set_tuning("block_gemm_form", form)
+            got = m.gemv(x)
+            assert rms(got - x64 @ w.astype(np.float16).astype(np.float64).T) <= 2.0 ** -21 < rms(got - x64 @ w.astype(np.float64).T) / 8, form
+    finally:
+        ops.set_tuning("block_gemm_form", 0)
     m.close()
 
 
