@@ -193,6 +193,7 @@ int device_compute_units();
 hipError_t launch_gemv(const GemvParams &p, hipStream_t stream);
 bool gemv_splits_activations(const DeviceMatrix &w, int batch);
 bool gemv_wants_tiled_copy(int format, int cols);
+bool short_blocks_enabled();    // tuning key "short_blocks"
 unsigned gemv_tuning_epoch();   // bumped by every gemv_set_tuning call
 // Slices of the prefix per query head that launch_attention_partials writes and the merging GEMV reads.
 #ifndef ESP_ATTENTION_HEAD_SPLITS

@@ -30,6 +30,7 @@
 #include <cstdlib>
 
 #include <string>
+#include <atomic>
 #include <type_traits>
 
 #include "../common.h"
@@ -2798,6 +2799,8 @@ bool gemv_merges_attention_partials(const DeviceMatrix &w, int batch, int head_d
     return true;
 }
 
+static std::atomic<bool> g_short_blocks{true};
+bool short_blocks_enabled() { return g_short_blocks.load(); }
 static unsigned g_tuning_epoch = 0;
 unsigned gemv_tuning_epoch() { return g_tuning_epoch; }
 
@@ -2814,6 +2817,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "q4k_mfma_rows8_max") { g_q4k_mfma_rows8_max = value; return true; }
     if (k == "q4k_long_row_waves") { g_q4k_long_row_waves = value; return true; }
     if (k == "q4k_wide") { g_q4k_wide_mode = value; return true; }
+    if (k == "short_blocks") { g_short_blocks.store(value != 0); return true; }
     if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
     if (k == "block_split_form") { block_split_set_form(value); return true; }

@@ -531,7 +531,7 @@ bool LlamaRuntime::splits_every_product() const {
 // 2.40 / 2.22 / 2.03 / 1.88e-4 (fp16 caches and contexts).
 bool LlamaRuntime::block_prefill_pays(int count, int base) const {
     if (count >= kMatrixPrefillMinTokens) return true;
-    if (count < 4) return false;
+    if (count < 4 || !short_blocks_enabled()) return false;
     if (split_blocks_supported()) return true;   // whatever is behind them
     return count >= 5 && (short_split_blocks_supported() || short_blocks_exact()) && short_block_pays(count, base);
 }
@@ -554,10 +554,10 @@ bool LlamaRuntime::short_block_pays(int count, int base) const {
 // 4272 / 16423 -> 2492 / 2474 / 2467 / 2319 us, four layers of 8B with fp32 caches 567 / 739 / 974 / 3327 -> 696 / 690 / 647 / 629.
 // Blocks whose products keep every weight and whose attention is 32-bit round nothing that the single-row steps of these formats do not: activations and contexts are fp16 in
 // both.  From the fifth token on they are also faster (behind 100 tokens, 4 / 5 / 16 / 31 tokens, steps -> block, us: 6 layers Q8_0 352 / 470 / 1316 / 2583 -> 337 / 324 / 350 / 366;
-// 1.1B Q8_0 1430 / 2131 / 5436 / 11032 -> 1278 / 1259 / 1260 / 1358; 3B Q4_0 1966 / 2782 / 7341 / 14484 -> 2091 / 2061 / 2100 / 2159).
-// Models narrower than 512 columns keep the two-row steps: none is in use, and the tests of those steps count on them (two layers of 256 columns, 7 tokens: 167 us, 93 as a block).
+// 1.1B Q8_0 1430 / 2131 / 5436 / 11032 -> 1278 / 1259 / 1260 / 1358; 3B Q4_0 1966 / 2782 / 7341 / 14484 -> 2091 / 2061 / 2100 / 2159; two layers of 256 columns,
+// 7 tokens 167 -> 93).
 bool LlamaRuntime::short_blocks_exact() const {
-    if (!short_span_attention_ || c_.d_model < 512) return false;
+    if (!short_span_attention_) return false;
     auto ok = [](const DeviceMatrix &m) {
         GemmParams p;
         p.w = m; p.rows = kMatrixPrefillMinTokens - 1; p.unrounded = true;

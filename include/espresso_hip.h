@@ -234,7 +234,7 @@ int esp_llama_continue_greedy(ESPLlamaRuntime *runtime, int sequence, int steps,
 int esp_llama_set_graph_replay(ESPLlamaRuntime *runtime, int enabled);
 /* Prompts of 32 tokens or more are prefilled in blocks of up to 512 rows with every projection as one
  * dequant-fused MFMA GEMM (fp32 accumulation; fp16 weights after dequantisation, exact ones on the Q4_K block kernels), and so are prompts of
- * four or five tokens and more where a short block rounds nothing that the steps do not (Q4_K models; Q8_0, Q4_0 and fp16 models of 512 columns and more) and is
+ * four or five tokens and more where a short block rounds nothing that the steps do not (Q4_K, Q8_0, Q4_0 and fp16 models) and is
  * the faster of the two (not for a few tokens behind thousands), instead of the
  * reference's token-by-token walk (RealModelInferenceEngine.swift:6365-6375); shorter ones walk two tokens per step.
  * enabled = 0 restores the per-token path for every length, whose arithmetic keeps the dequantised weights in fp32.  Default: enabled. */

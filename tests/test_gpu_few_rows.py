@@ -131,8 +131,13 @@ def test_short_prompts_of_feed_forwards_too_wide_for_pairs(mods, fmt, hidden):
     for t in tokens:
         g.advance(int(t))
     want = g.logits()
-    g.prefill(tokens)
-    assert np.abs(g.logits() - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max())   # as above
+    try:
+        for blocks in (0, 1):   # such steps, then what such prompts take by themselves
+            ops.set_tuning("short_blocks", blocks)
+            g.prefill(tokens)
+            assert np.abs(g.logits() - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max())   # as above
+    finally:
+        ops.set_tuning("short_blocks", 1)
     g.close()
 
 
@@ -169,12 +174,16 @@ def test_without_matrix_prefill_every_token_is_a_step(mods):
     g, _ = syn.build_runtime(cfg, lib.FORMAT_Q8_0, seed=5, std=0.05)
     tokens = np.random.default_rng(1).integers(0, cfg.vocab, 43).astype(np.uint32)
     ll.set_kernel_timing(g, True)
-    for enabled, count, steps in [(False, 43, 43), (False, 7, 7), (True, 7, 4)]:
-        ll.set_matrix_prefill(g, enabled)
-        g.reset()
-        ll.kernel_times(g)
-        g.prefill(tokens[:count])
-        assert ll.kernel_times(g)["qkv"]["launches"] == cfg.n_layer * steps, (enabled, count)
+    try:
+        for enabled, blocks, count, steps in [(False, 1, 43, 43), (False, 1, 7, 7), (True, 0, 7, 4), (True, 1, 7, 0)]:   # (a block's products are not among the counted launches)
+            ops.set_tuning("short_blocks", blocks)
+            ll.set_matrix_prefill(g, enabled)
+            g.reset()
+            ll.kernel_times(g)
+            g.prefill(tokens[:count])
+            assert ll.kernel_times(g)["qkv"]["launches"] == cfg.n_layer * steps, (enabled, blocks, count)
+    finally:
+        ops.set_tuning("short_blocks", 1)
     g.close()
 
 
@@ -208,7 +217,11 @@ def test_q4_0_decode_matches_oracle(mods, d, heads, kv, hidden):
     o = oracle_from_packed(cfg, packed, orc.FMT_Q4_0, 1, True, 48)
     prompt = [1, 8999, 777, 16, 5]
     o.prefill(prompt)
-    g.prefill(np.asarray(prompt, np.uint32))
+    ops.set_tuning("short_blocks", 0)
+    try:
+        g.prefill(np.asarray(prompt, np.uint32))
+    finally:
+        ops.set_tuning("short_blocks", 1)
     for _ in range(5):
         want = o.logits()
         assert np.abs(want - g.logits()).max() <= 2e-2
