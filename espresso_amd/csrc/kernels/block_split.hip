@@ -4,7 +4,7 @@
 // The shape is that of block_gemm.hip: eight wavefronts, NW of them along the weights and 8 / NW sharing K, each with 32 weight rows and all 32 TM activation rows; weights go
 // from memory into the registers that multiply them, read row by row from the packed matrix (no tiled copy is needed), both planes through LDS.  Two wavefronts on every SIMD, and
 // K shared inside a workgroup, are what the narrow forms of gemm_q4k_split_regb_kernel lack: one wavefront per SIMD walks all of K behind a SiLU, which planes cannot split.
-// What bounds it: the weights' way from memory for few rows, the matrix cores and the fold (33 multiply-adds a sum and super-block) for many.  Against those forms, us:
+// What bounds it: the weights' way from memory for few rows, the matrix cores and the fold (two multiply-adds a sum and super-block, and one product per row tile for the minimums) for many.  Against those forms, us:
 //   gate|up 28672 x 4096, 8 / 31 / 60 rows 48 / 48 / 58 -> 29 / 33 / 56;  16384 x 2048, 8 / 31 / 60 / 128 rows 25 / 25 / 26 / 31 -> 13 / 14 / 18 / 28;
 //   6144 x 4096, 31 / 256 / 480 rows and their planes 14.1 / 49.9 / 76.9 -> 12.9 / 40.7 / 67.4;  4096 x 14336, 256 rows 82 -> 76.
 // Kept out: 128 rows a workgroup and 96 for two groups (264 and 92 bytes of scratch a lane), the activations on their way to LDS as uint4 (they stay in scratch: 8 rows of

@@ -38,7 +38,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32;
 
-constexpr int kThreads = 256;
 constexpr int KT = 64;        // k per tile
 constexpr int LDK = KT + 8;   // fp16 per LDS row: 144 bytes, so eight rows cover all banks
 constexpr int NT = 128;       // weight rows per workgroup: two threads per row

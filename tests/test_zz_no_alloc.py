@@ -74,20 +74,25 @@ def make_matrix(ops, fmt, rows, cols, seed):
 def test_two_calls_in_a_row_share_the_scratch_and_match_esp_gemv(env):
     lib, ops, hip, L = env
     rng = np.random.default_rng(1)
-    # first call: Q8_0 768 x 2048 at batch 16 (register-B MFMA kernel, K split four ways: partial sums in the scratch)
+    # first call: Q8_0 768 x 2048 at batch 16, K split four ways (whatever the rule would choose): partial sums in the scratch
     big = make_matrix(ops, orc.FMT_Q8_0, 768, 2048, 2)
     x1 = rng.normal(0, 1, (16, 2048)).astype(np.float16)
     r1 = rng.normal(0, 1, (16, 768)).astype(np.float32)
-    y1 = run_noalloc(env, big, x1, r1)
-    # second call, smaller, over whatever the first left in the scratch
     small = make_matrix(ops, orc.FMT_Q8_0, 256, 1024, 3)
     x2 = rng.normal(0, 1, (5, 1024)).astype(np.float16)
-    y2 = run_noalloc(env, small, x2)
-    # the same kernels, the same split counts, the same order of additions: bit for bit what esp_gemv returns
-    assert np.array_equal(y1.view(np.uint32), big.gemv(x1, r1).view(np.uint32))
-    assert np.array_equal(y2.view(np.uint32), small.gemv(x2).view(np.uint32))
-    # and the first call again after the second
-    assert np.array_equal(run_noalloc(env, big, x1, r1).view(np.uint32), y1.view(np.uint32))
+    try:
+        for form in (184, 0):
+            ops.set_tuning("block_gemm_form", form)
+            y1 = run_noalloc(env, big, x1, r1)
+            # second call, smaller, over whatever the first left in the scratch
+            y2 = run_noalloc(env, small, x2)
+            # the same kernels, the same split counts, the same order of additions: bit for bit what esp_gemv returns
+            assert np.array_equal(y1.view(np.uint32), big.gemv(x1, r1).view(np.uint32))
+            assert np.array_equal(y2.view(np.uint32), small.gemv(x2).view(np.uint32))
+            # and the first call again after the second
+            assert np.array_equal(run_noalloc(env, big, x1, r1).view(np.uint32), y1.view(np.uint32))
+    finally:
+        ops.set_tuning("block_gemm_form", 0)
     # against the oracle's matvec on the dequantised weights (MFMA path: weights rounded to fp16 once)
     deq = big.dequantize()
     want = np.stack([orc.matvec(deq, x1[b].astype(np.float32)) for b in range(16)]) + r1
