@@ -17,20 +17,14 @@
 //   11264 x 2048 Q4_K 60 / 39 / 28 -> 36 / 22 / 14.  62 us are 830 TFLOP/s.
 #include "../common.h"
 #include "block_gemm.h"
+#include "block_tile.h"
 #include "silu.h"
-#include <atomic>
 #include <type_traits>
 
 namespace esp {
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32;
-
-constexpr int kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kStep = 128;     // k per step: four blocks of Q8_0 / Q4_0, half a super-block of Q4_K
+using namespace block_tile;
 
 struct BlockArgs {
     const uint8_t *qs;
@@ -45,10 +39,6 @@ struct BlockArgs {
     int per, splits, n_tiles, m_tiles;   // per: steps of one group of wavefronts
 };
 
-__device__ __forceinline__ h2 as_h2(u32 v) { return __builtin_bit_cast(h2, v); }
-__device__ __forceinline__ u32 as_u32(h2 v) { return __builtin_bit_cast(u32, v); }
-__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
-__device__ __forceinline__ float half_bits_to_float(u32 bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
 __device__ __forceinline__ h2 splat_bits(u32 bits16) { return as_h2(__builtin_amdgcn_perm(bits16, bits16, 0x01000100u)); }
 __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
     return make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
@@ -56,7 +46,6 @@ __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
 }
 constexpr int pairs_of(int fmt) { return fmt == FMT_F16 ? 4 : fmt == FMT_Q8_0 ? 2 : 1; }   // 64-byte stretches of a row in a step
 
-constexpr int kRow = kStep + 8;   // fp16 between the staged activation rows: 272 bytes, sixteen-byte reads of neighbouring rows fall on different banks
 template <int TM, int NW>
 constexpr int block_buffers() { return 2 * (kWaves / NW) * 32 * TM * kRow * 2 <= 160 * 1024 ? 2 : 1; }
 template <int TM, int NW>
@@ -75,10 +64,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     extern __shared__ uint4 smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, col = lane & 31;
     const int wn = wave % NW, wk = wave / NW, gtid = wn * 64 + lane;
-    // workgroups of one die take neighbouring output tiles: the row tiles of one block of weights first
-    const int total = gridDim.x, die = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-    const int unit = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
-    const int m_tile = unit % a.m_tiles, rest = unit / a.m_tiles, n_tile = rest % a.n_tiles, split = rest / a.n_tiles;
+    const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
     const int m0 = m_tile * MT, n0 = (n_tile * NW + wn) * 32, n = n0 + col;
     const int row0 = n0 < a.N ? n0 : a.N - 1;
     auto row_of = [&](int r) { return row0 + r < a.N ? r : a.N - 1 - row0; };   // rows from row0 on, clamped: those beyond are never stored
@@ -107,26 +93,21 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
             *reinterpret_cast<uint4 *>(xt + buf * MT * kRow + r * kRow + part * 8) = FMT == FMT_Q4_0 ? swap_middle(xv[i]) : xv[i];
         }
     };
-    // Weights: lane 16 p + r of a load takes piece p of row r (of row 16 + r in the next), so that four lanes cover 64 bytes of a row; v_permlane16_swap
-    // then leaves pieces 2 h and 2 h + 1 of row lane % 32 in each lane.
+    // Weights (exchange_rows): each lane ends up with pieces 2 h and 2 h + 1 of row lane % 32
     const int piece = EXACT ? 2 * ((lane >> 4) & 1) + h : lane >> 4;   // exact: pieces h and 2 + h
     const uint8_t *wbase = a.qs + (size_t)row0 * a.row_bytes;
     const u32 wlo = (u32)row_of(lane & 15) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + (lane & 15)) * (u32)a.row_bytes + piece * 16;
     const uint16_t *sbase = a.scales + (size_t)row0 * (a.K / 32);
     const u32 so = (u32)row_of(col) * (u32)(a.K / 32) + (FMT == FMT_Q4_0 && !EXACT ? 2 * h : 0), ho = (u32)row_of(col) * (u32)a.row_bytes;
     constexpr int PAIRS = pairs_of(FMT);
-    uint4 raw[2 * PAIRS], q[2];                 // the next step's stretches as they were loaded; the stretch in use, of the lane's own row
+    uint4 raw[PAIRS][2], q[2];                  // the next step's stretches as they were loaded; the stretch in use, of the lane's own row
     auto load_pair = [&](int s, int j) __attribute__((always_inline)) {
         const uint8_t *from = wbase + (FMT == FMT_Q4_K ? (size_t)(at(s) >> 1) * 144 + 16 + (at(s) & 1) * 64 : (size_t)at(s) * (64 * PAIRS)) + 64 * j;
-        raw[2 * j] = *reinterpret_cast<const uint4 *>(from + wlo);
-        raw[2 * j + 1] = *reinterpret_cast<const uint4 *>(from + whi);
+        raw[j][0] = *reinterpret_cast<const uint4 *>(from + wlo);
+        raw[j][1] = *reinterpret_cast<const uint4 *>(from + whi);
     };
     auto use_pair = [&](int j) __attribute__((always_inline)) {
-        auto swap = [](u32 x, u32 y, u32 &u, u32 &v) __attribute__((always_inline)) { const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false); u = p[0]; v = p[1]; };
-        swap(raw[2 * j].x, raw[2 * j + 1].x, q[0].x, q[1].x);
-        swap(raw[2 * j].y, raw[2 * j + 1].y, q[0].y, q[1].y);
-        swap(raw[2 * j].z, raw[2 * j + 1].z, q[0].z, q[1].z);
-        swap(raw[2 * j].w, raw[2 * j + 1].w, q[0].w, q[1].w);
+        exchange_rows(raw[j], q);
         if constexpr (EXACT && FMT == FMT_Q4_0) {   // each half of a wavefront holds a block; it needs bytes 8 h .. of both
 #pragma unroll
             for (int p = 0; p < 2; p++) {
@@ -315,35 +296,17 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
         if constexpr (BUFS == 1) __syncthreads();
     }
 
-    // accumulator r of a lane: activation row 8 (r / 4) + 4 h + r % 4 of its 32, weight row lane % 32
-    auto out_row = [&](int r) { return m0 + 32 * (r >> 4) + 8 * ((r & 15) >> 2) + 4 * h + (r & 3); };
+    auto out_row = [&](int r) { return m0 + tile_row(r, h); };
     constexpr int SHARE = TM * 16 / KW;        // accumulators that a wavefront finishes
     float v[SHARE];
-    int r0 = 0;
-    if constexpr (KW == 1) {
-#pragma unroll
-        for (int r = 0; r < SHARE; r++) v[r] = acc[r >> 4][r & 15];
-    } else {   // the groups' sums meet in LDS (the last barrier is behind everybody's last read of it), in their order
-        float *red = reinterpret_cast<float *>(smem);
-#pragma unroll
-        for (int r = 0; r < TM * 16; r++) red[((size_t)wave * TM * 16 + r) * 64 + lane] = acc[r >> 4][r & 15];
-        __syncthreads();
-        r0 = wk * SHARE;
-#pragma unroll
-        for (int r = 0; r < SHARE; r++) {
-            float sum = red[((size_t)wn * TM * 16 + r0 + r) * 64 + lane];
-#pragma unroll
-            for (int g = 1; g < KW; g++) sum += red[((size_t)(g * NW + wn) * TM * 16 + r0 + r) * 64 + lane];
-            v[r] = sum;
-        }
-    }
-    if (a.swiglu_out) {   // weight rows are (gate, up) pairs, neighbouring lanes: the even lane finishes the even accumulators, the odd lane the odd ones
+    const int r0 = KW == 1 ? 0 : wk * SHARE;
+    share_sums<TM, NW>(acc, reinterpret_cast<float *>(smem), wave, wn, lane, r0, v);
+    if (a.swiglu_out) {
 #pragma unroll
         for (int k = 0; k < SHARE / 2; k++) {
-            const float p0 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k]), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-            const float p1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k + 1]), 0xB1, 0xF, 0xF, false));
             const bool odd = lane & 1;
-            const float g = odd ? p1 : v[2 * k], u = odd ? v[2 * k + 1] : p0;
+            float g, u;
+            gate_and_up(v[2 * k], v[2 * k + 1], odd, g, u);
             const int m = out_row(r0 + 2 * k + (odd ? 1 : 0));
             if (m < a.M && (n | 1) < a.N) {
                 a.swiglu_out[(size_t)m * (a.N / 2) + n / 2] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(silu(g), u));
@@ -369,19 +332,10 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 
 template <int FMT, int TM, int NW, bool EXACT>
 hipError_t launch(const BlockArgs &a, hipStream_t stream) {
-    static std::atomic<uint64_t> raised{0};   // the limit of dynamic LDS is raised once per kernel and device
+    static std::atomic<uint64_t> raised{0};
     constexpr size_t lds = block_lds_bytes<TM, NW>();
-    if (lds > 64 * 1024) {
-        int device = 0;
-        hipError_t err = hipGetDevice(&device);
-        if (err != hipSuccess) return err;
-        const uint64_t bit = 1ull << (device & 63);
-        if (!(raised.load(std::memory_order_acquire) & bit)) {
-            err = hipFuncSetAttribute(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (err != hipSuccess) return err;
-            raised.fetch_or(bit, std::memory_order_release);
-        }
-    }
+    const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT>), lds, raised);
+    if (err != hipSuccess) return err;
     hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW, EXACT>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
     return hipGetLastError();
 }
@@ -424,7 +378,8 @@ Form choose_form(const GemmParams &p, bool exact) {
     for (int tm = 1; tm <= (exact ? 1 : 4) && tm <= (M + 31) / 32; tm++)
         for (int nw = tm < 4 ? 2 : 4; nw <= 8; nw *= 2)
             for (int want : kSplits) {
-                const int kw = 8 / nw, per = (units + want * kw - 1) / (want * kw), splits = (units + per * kw - 1) / (per * kw);
+                const int kw = kWaves / nw;
+                const auto [per, splits] = shares_of(units, nw, want);
                 const float mb = (float)splits * (float)M * (float)N * 4e-6f;
                 if (splits != want || (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
                 const long wgs = (long)((N + 32 * nw - 1) / (32 * nw)) * ((M + 32 * tm - 1) / (32 * tm)) * splits;
@@ -490,8 +445,9 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
     if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
         f.tm = forced / 100; f.nw = forced / 10 % 10;
         exact = exact && f.tm == 1;   // forms of more row tiles have no exact kernel
-        const int want = forced % 10, kw = 8 / f.nw, unit = p.w.format == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit), per = (units + want * kw - 1) / (want * kw);
-        f.per = per * unit; f.splits = (units + per * kw - 1) / (per * kw);
+        const int unit = p.w.format == FMT_Q4_K ? 2 : 1;
+        const Shares shares = shares_of(p.w.cols / (kStep * unit), f.nw, forced % 10);
+        f.per = shares.per * unit; f.splits = shares.splits;
         if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;
     }
     BlockArgs a{p.w.qs, p.w.scales, p.w.qs_row_bytes, p.w.rows, p.w.cols, p.rows, p.x, p.y, p.residual, p.workspace, f.splits == 1 && p.w.rows % 2 == 0 ? p.swiglu_out : nullptr, f.per, f.splits,

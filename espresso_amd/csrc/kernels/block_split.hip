@@ -11,9 +11,9 @@
 // 16384 x 2048 32 us).  With one row tile the activation fragments are read three ahead (one ahead: 42 us for 8 rows of 28672 x 4096 with eight wavefronts along the weights, 62).
 #include "../common.h"
 #include "block_split.h"
+#include "block_tile.h"
 #include "silu.h"
 #include "split_rows.h"
-#include <atomic>
 #include <type_traits>
 
 namespace esp {
@@ -21,15 +21,8 @@ namespace {
 
 using split_rows::kScale;
 using split_rows::kUnscale;
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32;
+using namespace block_tile;
 typedef u32 quad __attribute__((ext_vector_type(4)));
-
-constexpr int kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kStep = 128;        // k per step: half a super-block
-constexpr int kRow = kStep + 8;   // fp16 between the staged activation rows
 
 struct BlockSplitArgs {
     const uint8_t *qs;
@@ -43,10 +36,6 @@ struct BlockSplitArgs {
     int per, splits, n_tiles, m_tiles;   // per: steps of one group of wavefronts, an even number
 };
 
-__device__ __forceinline__ h2 as_h2(u32 v) { return __builtin_bit_cast(h2, v); }
-__device__ __forceinline__ u32 as_u32(h2 v) { return __builtin_bit_cast(u32, v); }
-__device__ __forceinline__ half8 as_half8(const uint4 &v) { return __builtin_bit_cast(half8, v); }
-__device__ __forceinline__ float half_bits_to_float(u32 bits16) { return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16); }
 __device__ __forceinline__ u32 dword_of(const uint4 &v, int k) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; }
 
 constexpr size_t split_tile_bytes(int tm, int nw) { return (size_t)(kWaves / nw) * 2 * 32 * tm * kRow * 2; }   // a step of all groups
@@ -64,10 +53,7 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
     extern __shared__ uint4 smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, col = lane & 31;
     const int wn = wave % NW, wk = wave / NW, gtid = wn * 64 + lane;
-    // workgroups of one die take neighbouring output tiles: the row tiles of one block of weights first
-    const int total = gridDim.x, die = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-    const int unit = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
-    const int m_tile = unit % a.m_tiles, rest = unit / a.m_tiles, n_tile = rest % a.n_tiles, split = rest / a.n_tiles;
+    const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
     const int m0 = m_tile * MT, n0 = (n_tile * NW + wn) * 32, n = n0 + col;
     const int row0 = n0 < a.N ? n0 : a.N - 1;
     auto row_of = [&](int r) { return row0 + r < a.N ? r : a.N - 1 - row0; };   // rows from row0 on, clamped: those beyond are never stored
@@ -99,7 +85,7 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
             *reinterpret_cast<quad *>(xt + (2 * buf + 1) * MT * kRow + r * kRow + part * 8) = lo_x[i];
         }
     };
-    // weights: as in block_gemm.hip, four lanes cover 64 bytes of a row; the two pieces of the pair of sub-blocks h end up in each lane of the row
+    // weights (exchange_rows): the two pieces of the pair of sub-blocks h end up in each lane of the row
     const int piece = lane >> 4;
     const uint8_t *wbase = a.qs + (size_t)row0 * a.row_bytes;
     const u32 wlo = (u32)row_of(lane & 15) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + (lane & 15)) * (u32)a.row_bytes + piece * 16, ho = (u32)row_of(col) * (u32)a.row_bytes;
@@ -108,13 +94,6 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
         const uint8_t *from = wbase + (size_t)(at(s) >> 1) * 144 + 16 + (at(s) & 1) * 64;
         raw[0] = *reinterpret_cast<const uint4 *>(from + wlo);
         raw[1] = *reinterpret_cast<const uint4 *>(from + whi);
-    };
-    auto use_pair = [&]() __attribute__((always_inline)) {
-        auto swap = [](u32 x, u32 y, u32 &u, u32 &v) __attribute__((always_inline)) { const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false); u = p[0]; v = p[1]; };
-        swap(raw[0].x, raw[1].x, q[0].x, q[1].x);
-        swap(raw[0].y, raw[1].y, q[0].y, q[1].y);
-        swap(raw[0].z, raw[1].z, q[0].z, q[1].z);
-        swap(raw[0].w, raw[1].w, q[0].w, q[1].w);
     };
     auto load_hdr = [&](int s) __attribute__((always_inline)) { return *reinterpret_cast<const uint4 *>(wbase + (size_t)(at(s) >> 1) * 144 + ho); };
     // the rows' sums over the sub-blocks of a super-block: (8 x hi, 8 x lo) of sums
@@ -175,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
         };
         auto unpack = [&](int v) __attribute__((always_inline)) {
             if (v == 0) {
-                use_pair();
+                exchange_rows(raw, q);
                 load_pair(s + 1);
             }
             if (!(v & 1)) wq[0] = decode(hdr[H], odd, v >> 1);
@@ -248,29 +227,11 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
         if constexpr (BUFS == 1) __syncthreads();
     }
 
-    // accumulator r of a lane: activation row 8 (r / 4) + 4 h + r % 4 of its 32, weight row lane % 32
-    auto tile_row = [&](int r) { return 32 * (r >> 4) + 8 * ((r & 15) >> 2) + 4 * h + (r & 3); };
     constexpr int SHARE = TM * 16 / KW;        // accumulators that a wavefront finishes
     float v[SHARE];
-    int r0 = 0;
-    if constexpr (KW == 1) {
-#pragma unroll
-        for (int r = 0; r < SHARE; r++) v[r] = tot[r >> 4][r & 15];
-    } else {   // the groups' sums meet in LDS (the last barrier is behind everybody's last read of it), in their order
-        float *red = reinterpret_cast<float *>(smem);
-#pragma unroll
-        for (int r = 0; r < TM * 16; r++) red[((size_t)wave * TM * 16 + r) * 64 + lane] = tot[r >> 4][r & 15];
-        __syncthreads();
-        r0 = wk * SHARE;
-#pragma unroll
-        for (int r = 0; r < SHARE; r++) {
-            float sum = red[((size_t)wn * TM * 16 + r0 + r) * 64 + lane];
-#pragma unroll
-            for (int g = 1; g < KW; g++) sum += red[((size_t)(g * NW + wn) * TM * 16 + r0 + r) * 64 + lane];
-            v[r] = sum;
-        }
-    }
-    if (a.sw_hi) {   // weight rows are (gate, up) pairs, neighbouring lanes: the even lane finishes the even accumulators, the odd lane the odd ones; the units leave through LDS
+    const int r0 = KW == 1 ? 0 : wk * SHARE;
+    share_sums<TM, NW>(tot, reinterpret_cast<float *>(smem), wave, wn, lane, r0, v);
+    if (a.sw_hi) {   // the units leave through LDS
         constexpr int LD = 16 * NW + 8, RP = 2 * NW;   // units between rows, sixteen-byte pieces of a row
         uint16_t *hi = reinterpret_cast<uint16_t *>(smem), *lo = hi + MT * LD;
         if constexpr (KW > 1) __syncthreads();
@@ -278,10 +239,10 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
         const int u = (32 * wn + col) >> 1, slot = u & 3, at_u = (u & ~3) + (slot == 1 ? 2 : slot == 2 ? 1 : slot);   // the planes' order inside fours: 0, 2, 1, 3
 #pragma unroll
         for (int k = 0; k < SHARE / 2; k++) {
-            const float p0 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k]), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-            const float p1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[2 * k + 1]), 0xB1, 0xF, 0xF, false));
-            const float g = odd ? p1 : v[2 * k], up = odd ? v[2 * k + 1] : p0, act = __fmul_rn(silu(g), up);
-            const int o = tile_row(r0 + 2 * k + (odd ? 1 : 0)) * LD + at_u;
+            float g, up;
+            gate_and_up(v[2 * k], v[2 * k + 1], odd, g, up);
+            const float act = __fmul_rn(silu(g), up);
+            const int o = tile_row(r0 + 2 * k + (odd ? 1 : 0), h) * LD + at_u;
             const _Float16 top = (_Float16)act;
             hi[o] = __builtin_bit_cast(uint16_t, top);
             lo[o] = __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(__fsub_rn(act, (float)top), kScale));
@@ -306,7 +267,7 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
         return;
     }
     float *out = a.splits > 1 ? a.partial + (size_t)split * a.M * a.N : a.y;
-    auto out_row = [&](int r) { return m0 + tile_row(r); };
+    auto out_row = [&](int r) { return m0 + tile_row(r, h); };
     if (a.splits == 1 && a.residual) {
         // requested together: y may be the residual's own memory, and a load behind each store is a trip to memory each
 #pragma unroll
@@ -318,18 +279,11 @@ __global__ __launch_bounds__(kThreads) void block_split_kernel(BlockSplitArgs a)
 
 template <int TM, int NW>
 hipError_t launch(const BlockSplitArgs &a, hipStream_t stream) {
-    static std::atomic<uint64_t> raised{0};   // the limit of dynamic LDS is raised once per kernel and device
+    static std::atomic<uint64_t> raised{0};
     constexpr size_t lds = split_lds_bytes(TM, NW);
     static_assert(lds <= 160 * 1024, "LDS of a compute unit");
-    int device = 0;
-    hipError_t err = hipGetDevice(&device);
+    const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(block_split_kernel<TM, NW>), lds, raised);
     if (err != hipSuccess) return err;
-    const uint64_t bit = 1ull << (device & 63);
-    if (!(raised.load(std::memory_order_acquire) & bit)) {
-        err = hipFuncSetAttribute(reinterpret_cast<const void *>(block_split_kernel<TM, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-        raised.fetch_or(bit, std::memory_order_release);
-    }
     hipLaunchKernelGGL((block_split_kernel<TM, NW>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
     return hipGetLastError();
 }
@@ -370,7 +324,8 @@ BlockSplitForm block_split_form(const GemmSplitParams &p) {
     for (const auto &f : kForms)
         for (int want : kSplits) {
             if (f.tm > 1 && f.tm > (M + 31) / 32) continue;
-            const int kw = 8 / f.nw, per = (units + want * kw - 1) / (want * kw), splits = (units + per * kw - 1) / (per * kw);
+            const int kw = kWaves / f.nw;
+            const auto [per, splits] = shares_of(units, f.nw, want);
             if (forced > 0 && (forced != f.tm * 100 + f.nw * 10 + want || (swiglu && splits > 1))) continue;
             if (forced == 0 && (splits != want || (swiglu && splits > 1))) continue;
             const float mb = (float)splits * (float)M * (float)N * 4e-6f;
