@@ -11,10 +11,11 @@
 //   * Activations go through LDS, two buffers and one barrier a step, fragment g + 1 read while g is multiplied (left to the compiler: 3 to 5 % slower).
 //   * Q4_K's n s - dm is one v_fma_mix a weight (a nibble alone in sixteen bits is the fp16 number n 2^-24), rounded once as before; v_cvt_f32_ubyte, an fp32
 //     multiply-add and a conversion take almost twice the instructions.
-// What bounds it: at 512 rows the matrix cores, the unpacking beside them and the power both draw (the same kernel without loads and unpacking: 37 us of the 62 below); at 100 rows
-// and less the weights' way from memory and the steps' latencies.  Against the kernel of 128 x 128 tiles whose weights go through LDS (gemm.hip), us:
-//   16384 x 3072 Q4_0, 512 / 229 / 93 rows 93 / 58 / 39 -> 62 / 32 / 20;  3072 x 8192 Q4_0 53 / 30 / 20 -> 34 / 22 / 14;  11264 x 2048 Q8_0 64 / 39 / 26 -> 38 / 24 / 16;
-//   11264 x 2048 Q4_K 60 / 39 / 28 -> 36 / 22 / 14.  62 us are 830 TFLOP/s.
+// What bounds it: at 512 rows no unit alone (16384 x 3072 Q4_K, 63 us in a prompt's trace: matrix cores 20 us of their own, 10 000 vector instructions a SIMD 17, 52 MB read 10, no LDS
+// bank conflicts; a copy without loads and unpacking took 37); at 100 rows and less the weights' way from memory and the steps' latencies.  Against the kernel of 128 x 128 tiles
+// whose weights go through LDS (gemm.hip), both in turn, us:
+//   16384 x 3072 Q4_0, 512 / 192 / 96 rows 69 / 48 / 33 -> 55 / 30 / 23;  3072 x 8192 Q4_0 45 / 32 / 20 -> 33 / 20 / 14;  11264 x 2048 Q8_0 44 / 36 / 27 -> 38 / 24 / 17;
+//   11264 x 2048 Q4_K 44 / 37 / 29 -> 35 / 20 / 15.
 #include "../common.h"
 #include "block_gemm.h"
 #include "block_tile.h"
