@@ -402,14 +402,21 @@ void block_gemm_set_form(int form) {
 
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are
 // rounded).  Against rows_gemm.hip, whose wavefronts walk more of K each, 2560 x 2048, 4 / 31 / 93 rows: Q8_0 8.0 / 9.5 / 9.9 -> 6.2 / 6.4 / 7.8 us, Q4_0 6.8 / 8.2 / 8.4 -> 5.3 / 5.5 /
-// 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Behind a SiLU the shares cost a launch, so there only up to 32 rows.  Matrices of
-// fewer rows gain nothing beyond 32 (768 x 2048, 40 / 128 rows Q8_0 6.1 / 6.3 both ways, Q4_0 5.1 / 5.2 against 5.2 / 5.3) and would still pay for the planes.
+// 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Of what the launch gains the next kernel takes 1.5 to 2.5 us for the planes, so whole
+// layers decide (q|k|v and wo in shares, a feed-forward of four times the width; us a layer, one launch -> shares): 2048 columns, 12 / 31 / 48 rows Q8_0 65.5 / 74.6 / 75.8 -> 63.3 / 67.6 /
+// 71.6, Q4_0 60 / 66 / 67 -> 58 / 60 / 63;  2560 columns Q8_0 87.2 / 96.9 / 98.6 -> 83.5 / 91.2 / 97.0;  3072 columns Q8_0 96.2 / 102.6 / 105.3 -> 94.5 / 97.1 / 104.6.  Rows that are no
+// multiple of 512 columns spread better over the memory's channels there and gain up to 32 rows only: 2816 columns Q8_0 88.7 / 96.0 / 99.0 -> 89.7 / 92.7 / 100.0, Q4_0 76.8 / 84.4 / 84.8 ->
+// 79.5 / 80.7 / 85.6.
+// Behind a SiLU the shares cost a launch, so there only up to 32 rows.  Matrices of fewer weight rows stay where they are beyond 32: the launch alone would be shorter (512 to 1792 rows,
+// 40 / 128 rows of 2048 columns: Q8_0 9.3 / 9.5 -> 6.0 to 6.3 / 6.1 to 7.6, Q4_0 7.6 to 8 / 7.8 to 8.2 -> 5.0 to 5.4 / 5.2 to 6.7), but most of it goes into the planes, and calls of 48
+// tokens of a six-layer model of 768 columns differ by less than their 3 % noise.
 // Where no caller adds the shares, their launch outweighs them as long as the other kernel's workgroups are resident at once (with that launch, 8 rows Q4_0: 2048 x 2048 8.6 us, 6.7
 // there; 3072 x 3072 9.4, 7.4; 5632 x 2048 10.3, 6.9; 8192 x 3072 10.5, 9.2; 11264 x 2048 9.8, 12.6).
 bool block_gemm_keeps(const GemmParams &p) {
     if ((p.w.format != FMT_Q8_0 && p.w.format != FMT_Q4_0) || p.w.cols < 2048 || p.w.cols % kStep != 0 || !p.unrounded) return false;
     const long row_blocks = (p.rows + 31) / 32, groups = (long)((p.w.rows + 31) / 32) * row_blocks;
     if (block_gemm_alone(p) && groups <= (device_compute_units() > 0 ? device_compute_units() : 256)) return false;
+    if (p.w.cols <= 3072 && p.w.cols % 512 != 0 && (p.rows <= 16 || row_blocks > 1)) return false;
     return row_blocks == 1 || (row_blocks <= 4 && !p.swiglu_out && p.w.rows >= 2048 && p.w.cols <= 3072 && groups * (p.w.cols / 64) <= 8192);
 }
 

@@ -99,7 +99,7 @@ def test_rules_keep_weights_of_small_products(ops, fmt, rows, cols, batches):
     rng = np.random.default_rng(cols)
     check_kept(m, lambda x, r: m.layer_product(x, r, shares=True), batches, rng)
     check_kept(m, lambda x, r: m.layer_product(x, r), batches, rng)
-    if cols >= 2048 and rows >= 2048:
+    if cols >= 2048 and cols % 512 == 0 and rows >= 2048:
         ops.set_tuning("rows_gemm", 0)
         try:
             for form in (181, 143, 121, 124):   # the same products here whatever the rule
@@ -108,6 +108,20 @@ def test_rules_keep_weights_of_small_products(ops, fmt, rows, cols, batches):
         finally:
             ops.set_tuning("block_gemm_form", 0)
             ops.set_tuning("rows_gemm", 1)
+    m.close()
+
+
+@pytest.mark.parametrize("cols,batch,here", [(2304, 12, False), (2304, 31, True), (2304, 48, False), (2816, 48, False), (2048, 48, True), (2560, 12, True)])
+def test_shares_of_k_by_columns(ops, cols, batch, here):
+    """Rows of a multiple of 512 columns are shared where a layer adds the shares; others, which the kernel of one launch reads faster, at 17 to 32 rows only."""
+    m = ops.Matrix(lib.FORMAT_Q8_0, ops.synth_weights(lib.FORMAT_Q8_0, cols, 0.02, 2048 * cols), 2048, cols)
+    x = np.random.default_rng(cols).normal(0, 1, (batch, cols)).astype(np.float16)
+    default = m.layer_product(x, shares=True)
+    try:
+        ops.set_tuning("rows_gemm", 2)   # always that kernel, which adds in another order
+        assert np.array_equal(default, m.layer_product(x, shares=True)) != here
+    finally:
+        ops.set_tuning("rows_gemm", 1)
     m.close()
 
 
