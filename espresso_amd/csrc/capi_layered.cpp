@@ -39,7 +39,7 @@ int esp_layered_trace_layers(ESPLlamaRuntime *runtime, int sequence, const uint3
     LayeredRuntime *rt = nullptr;
     int rc = layered_of(runtime, &rt);
     if (rc != ESP_OK) return rc;
-    if (!out || count < 1 || count > kPrefillBlockRows) return fail(ESP_ERR_INVALID_ARGUMENT, "trace_layers: 1..%d tokens", kPrefillBlockRows);
+    if (!out || count < 1 || count > kMinPrefillBlockRows) return fail(ESP_ERR_INVALID_ARGUMENT, "trace_layers: 1..%d tokens", kMinPrefillBlockRows);   // one block of any runtime
     int status = ESP_OK;
     rt->set_min_block_rows(1);
     rt->set_layer_observer([&](int layer) {

@@ -233,8 +233,10 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
     };
     if (matrix_prefill_ && block_prefill_pays(count, start) && matrix_prefill_supported()) {
         // blocks of rows through the MFMA kernels (one pass over the weights per block)
-        for (int off = 0; off < count; off += block_rows_) {
-            const int rows = count - off < block_rows_ ? count - off : block_rows_;
+        const int blocks = (count + block_rows_ - 1) / block_rows_, even = ((count + blocks - 1) / blocks + 127) / 128 * 128;   // of one size: a short last block costs as much as half a long one
+        const int most = even < block_rows_ ? even : block_rows_;
+        for (int off = 0; off < count; off += most) {
+            const int rows = count - off < most ? count - off : most;
             if ((rc = prefill_block(seq, tokens + off, rows, start + off)) != ESP_OK) return rc;
             if (off + rows == count && (rc = keep_row(rows - 1, seq)) != ESP_OK) return rc;
             while (given < want_count && want[given] < off + rows) {

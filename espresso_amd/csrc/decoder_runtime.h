@@ -15,10 +15,17 @@ namespace esp {
 class LlamaRuntime;
 class LayeredRuntime;
 
-constexpr int kPrefillBlockRows = 512;        // rows per MFMA prefill block
+// Rows of a prompt block: a whole prompt of up to 2048 tokens, so that its products have several rounds of workgroups (one block against blocks of 512, us: 1777 tokens of 3B Q4_K 22510 ->
+// 18770, 1500 of eight layers of 8B 14160 -> 13660, 1100 of 1B Q8_0 6830 -> 4650, 1700 of 30 layers of 576 columns in Q4_0 8910 -> 4040, 1700 of six Ranavik layers of 4096 columns 9920 ->
+// 7970); contexts that hold fewer take what they hold, and no runtime's blocks are shorter than 512.
+constexpr int kMinPrefillBlockRows = 512, kMaxPrefillBlockRows = 2048;
+inline int prefill_block_rows(int max_seq) {
+    const int rows = max_seq > kMaxPrefillBlockRows ? kMaxPrefillBlockRows : (max_seq + 127) / 128 * 128;
+    return rows < kMinPrefillBlockRows ? kMinPrefillBlockRows : rows;
+}
 constexpr int kStepsPerGraph = 8;             // greedy steps in the longer of the two captured step graphs
 constexpr int kMatrixPrefillMinTokens = 32;   // shorter prompts take the steps' kernels, two tokens at a time where a step takes two rows, unless the runtime's short blocks are as exact
-constexpr size_t kGemmWorkspaceFloats = (size_t)8 << 20;
+constexpr size_t kGemmWorkspaceFloatsPerRow = (size_t)16 << 10;   // planes of split-K products, per row of a block
 
 struct DecoderShape {
     int d_model = 0, vocab = 0, max_seq = 0;

@@ -119,7 +119,7 @@ int LayeredRuntime::allocate_cache(size_t index, size_t row_elements) {
     int window = 1;
     for (size_t j = index; j < c_.layers.size(); j++)
         if (has_cache(c_.layers[j].mixer) && (j == index || c_.layers[j].kv_from == (int)index)) window = std::max(window, c_.layers[j].window);
-    L.ring = (int)std::min<long long>(shape_.max_seq, (long long)window - 1 + kPrefillBlockRows);
+    L.ring = (int)std::min<long long>(shape_.max_seq, (long long)window - 1 + prefill_block_rows(shape_.max_seq));
     L.cache_row_bytes = row_elements * precision_bytes(precision_);
     uint8_t *cache = nullptr;
     const int rc = device_alloc(&cache, L.ring * L.cache_row_bytes * shape_.max_sequences);

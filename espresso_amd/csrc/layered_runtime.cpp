@@ -137,7 +137,7 @@ int LayeredRuntime::build(LayeredWeights &weights) {
         L.latent.cache = L.attention.cache = layers_[from].cache;
         L.latent.ring = L.attention.ring = layers_[from].ring;
     }
-    if ((rc = allocate_common(kPrefillBlockRows, width_p_)) != ESP_OK) return rc;
+    if ((rc = allocate_common(prefill_block_rows(shape_.max_seq), width_p_)) != ESP_OK) return rc;
     if ((rc = allocate_scratch()) != ESP_OK) return rc;
     return finish_finalize();
 }
@@ -214,7 +214,7 @@ int LayeredRuntime::allocate_scratch() {
         return rc;
     // columns of an output product's input that no head fills meet zero weights, so they only have to be finite
     ESP_HIP_TRY(hipMemset(act_, 0, R * out_cols_max_ * E));
-    workspace_floats_ = std::max(kGemmWorkspaceFloats, R * width_p_);
+    workspace_floats_ = R * std::max(kGemmWorkspaceFloatsPerRow, (size_t)width_p_);
     if ((rc = device_alloc(&workspace_, workspace_floats_)) != ESP_OK) return rc;
     return allocate_mixer_scratch();
 }

@@ -332,7 +332,16 @@ int LlamaRuntime::finalize() {
         ESP_HIP_TRY(hipMemcpy(rope_sin_, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
     }
     // ---- activations ----
-    const size_t R = kPrefillBlockRows > kMaxStepRows ? kPrefillBlockRows : kMaxStepRows;
+        {
+        const char *pa = getenv("ESPRESSO_HIP_PROMPT_ATTENTION");   // "0": prompt blocks keep the single-query attention kernel
+        const bool block_attention = !(pa && pa[0] == '0');
+        prompt_attention_ = block_attention && attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
+        short_span_attention_ = block_attention && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
+        span_attention_ = block_attention && !prompt_attention_ && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
+    }
+    // the single-query attention kernel leaves its slices of every row of a block in scratch memory: those models keep short blocks
+    const bool rows_attend_alone = !prompt_attention_ && !span_attention_;
+    const size_t R = rows_attend_alone ? kMinPrefillBlockRows : prefill_block_rows(c_.max_seq);
     if ((rc = allocate_common((int)R, d)) != ESP_OK) return rc;
     if ((rc = device_alloc(&qkv_, R * (ad + 2 * kd))) != ESP_OK) return rc;
     if ((rc = device_alloc(&q_, R * ad)) != ESP_OK) return rc;
@@ -350,19 +359,15 @@ int LlamaRuntime::finalize() {
     }
     {
         const size_t per_row = (size_t)c_.n_kv_head * kAttentionMaxSplits * (c_.n_head / c_.n_kv_head) * (c_.head_dim + 2);
-        if ((rc = device_alloc(&attn_scratch_, R * per_row)) != ESP_OK) return rc;
+        if ((rc = device_alloc(&attn_scratch_, (rows_attend_alone ? R : (size_t)kMaxStepRows) * per_row)) != ESP_OK) return rc;
     }
-    if ((rc = device_alloc(&gemm_workspace_, kGemmWorkspaceFloats)) != ESP_OK) return rc;
+    gemm_workspace_floats_ = R * kGemmWorkspaceFloatsPerRow;
+    if ((rc = device_alloc(&gemm_workspace_, gemm_workspace_floats_)) != ESP_OK) return rc;
     if (gemm_split_shared_k_pool(&gemm_shared_k_) != hipSuccess) {   // without the pool the prompt GEMM keeps its plain grid
         (void)hipGetLastError();
         gemm_shared_k_ = GemmSplitSharedK{};
     }
     {
-        const char *pa = getenv("ESPRESSO_HIP_PROMPT_ATTENTION");   // "0": prompt blocks keep the single-query attention kernel
-        const bool block_attention = !(pa && pa[0] == '0');
-        prompt_attention_ = block_attention && attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
-        short_span_attention_ = block_attention && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
-        span_attention_ = block_attention && !prompt_attention_ && span_attention_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
         const char *fh = getenv("ESPRESSO_HIP_FUSED_HEAD_ARGMAX");   // "0": the head stores logits and separate launches pick the token
         fused_head_argmax_ = !(fh && fh[0] == '0');
         const char *sa = getenv("ESPRESSO_HIP_SPLIT_ACTIVATIONS");   // "0": activations rounded to fp16 once
@@ -586,7 +591,7 @@ int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
     for (size_t li = 0; li < layers_.size(); li++) {
         Layer &L = layers_[li];
         GemmSplitParams g;
-        g.rows = rows; g.workspace = gemm_workspace_; g.workspace_floats = kGemmWorkspaceFloats;
+        g.rows = rows; g.workspace = gemm_workspace_; g.workspace_floats = gemm_workspace_floats_;
         int splits = 1;
         g.w = L.wqkv; g.x = xn; g.y = qkv_; g.deferred_splits = &splits;
         ESP_HIP_TRY(launch_gemm_split(g, s));
@@ -626,7 +631,7 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
     const bool kv16 = c_.kv_format == FMT_F16;
     const size_t cache_seq_stride = (size_t)kd * c_.max_seq;
     GemmParams g;
-    g.rows = rows; g.unrounded = true; g.workspace = gemm_workspace_; g.workspace_floats = kGemmWorkspaceFloats;
+    g.rows = rows; g.unrounded = true; g.workspace = gemm_workspace_; g.workspace_floats = gemm_workspace_floats_;
     // The RMSNorm that follows a projection with a residual reads that projection's result; when the GEMM ran split-K the
     // norm kernel adds the partial sums itself (one launch instead of reduce + norm).
     const bool fuse_norm = rmsnorm_reduce_supported(d);
@@ -739,7 +744,7 @@ int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits
             return ESP_OK;
         }
         GemmParams m;
-        m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = kGemmWorkspaceFloats;
+        m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = gemm_workspace_floats_;
         ESP_HIP_TRY(launch_gemm(m, s));
         ESP_HIP_TRY(launch_argmax(logits_, count, c_.vocab, d_out_tokens_, nullptr, argmax_scratch_, s));
         return ESP_OK;

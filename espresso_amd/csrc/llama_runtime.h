@@ -131,6 +131,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool short_span_attention_ = false;   // span_attention_kernel for blocks of few rows
     bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for
     float *gemm_workspace_ = nullptr;
+    size_t gemm_workspace_floats_ = 0;
     GemmSplitSharedK gemm_shared_k_;   // the device's pool for launch_gemm_split's hand-over between workgroups (not owned)
 };
 
