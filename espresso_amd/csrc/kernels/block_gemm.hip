@@ -1,4 +1,4 @@
-// y[m][n] = sum_k x[m][k] * W[n][k] for blocks of activation rows, W in Q4_K, Q4_0, Q8_0 or (tall gate|up) fp16: fp16 operands (every dequantised weight is rounded to fp16
+// y[m][n] = sum_k x[m][k] * W[n][k] for blocks of activation rows, W in Q4_K, Q4_0 or Q8_0: fp16 operands (every dequantised weight is rounded to fp16
 // once), fp32 sums.
 //
 // A workgroup is eight wavefronts, two on every SIMD, so that one unpacks weights while the other multiplies.  NW of them lie side by side along 32 NW weight rows and
@@ -20,6 +20,7 @@
 #include "block_gemm.h"
 #include "block_tile.h"
 #include "silu.h"
+#include "wide_gemm.h"
 #include <type_traits>
 
 namespace esp {
@@ -45,7 +46,7 @@ __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
     return make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
                       __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
 }
-constexpr int pairs_of(int fmt) { return fmt == FMT_F16 ? 4 : fmt == FMT_Q8_0 ? 2 : 1; }   // 64-byte stretches of a row in a step
+constexpr int pairs_of(int fmt) { return fmt == FMT_Q8_0 ? 2 : 1; }   // 64-byte stretches of a row in a step
 
 template <int TM, int NW>
 constexpr int block_buffers() { return 2 * (kWaves / NW) * 32 * TM * kRow * 2 <= 160 * 1024 ? 2 : 1; }
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     // where fragment g (0..7) of a step begins among its 128 k
     auto koff = [&](int g) {
         if constexpr (EXACT) return 32 * (g >> 1) + (FMT == FMT_Q4_0 ? 16 * (g & 1) + 8 * h : 16 * h + 8 * (g & 1));
-        else return FMT == FMT_Q4_0 ? 64 * h + 8 * g : FMT == FMT_Q4_K ? 64 * h + 32 * (g & 1) + 8 * (g >> 1) : FMT == FMT_Q8_0 ? 64 * (g >> 2) + 32 * h + 8 * (g & 3) : 32 * (g >> 1) + 16 * h + 8 * (g & 1);
+        else return FMT == FMT_Q4_0 ? 64 * h + 8 * g : FMT == FMT_Q4_K ? 64 * h + 32 * (g & 1) + 8 * (g >> 1) : 64 * (g >> 2) + 32 * h + 8 * (g & 3);
     };
 
     floatx16 acc[TM];
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = as_u32((as_h2(((j & 1 ? w[j >> 1] >> 8 : w[j >> 1]) & mask) | magic) - off) * sc);
             return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
-        } else if constexpr (FMT == FMT_Q8_0) {
+        } else {
             const u32 pair = g >> 2 ? scales.y : scales.x;
             const h2 sc = splat_bits(h ? pair >> 16 : pair & 0xFFFFu), off = {(_Float16)1152.0f, (_Float16)1152.0f};   // 1024 + 128
             const uint4 &v = q[(g >> 1) & 1];
@@ -212,11 +213,9 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = as_u32((as_h2(__builtin_amdgcn_perm(0x64646464u, w[j >> 1], j & 1 ? 0x04030402u : 0x04010400u)) - off) * sc);
             return as_half8(make_uint4(o[0], o[1], o[2], o[3]));
-        } else {
-            return as_half8(q[g & 1]);
         }
     };
-    constexpr int VALU = FMT == FMT_F16 ? 2 : 16;   // of a fragment, to be spread over its products
+    constexpr int VALU = 16;   // of a fragment, to be spread over its products
     auto step = [&](auto slot_c, int s) __attribute__((always_inline)) {   // slot: s % 4: the buffers by turns, half of a super-block, super-blocks by turns
         constexpr int S = decltype(slot_c)::value & 1, H = decltype(slot_c)::value >> 1;
         constexpr std::integral_constant<int, S> odd{};
@@ -365,13 +364,12 @@ std::atomic<int> g_block_gemm_form{0};
 // The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and
 // with the groups that each stage their own activations, and the bytes of the planes, which the next kernel reads once more (behind a SiLU, and where no
 // caller adds them, a launch of its own: 1.6 to 4.3 us; the form that rule chooses is 1 % off the best on average, 11 at worst, 256 x 256).  The
-// constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows, the four formats) and are off by 6 % at the
-// median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst but for fp16.
+// constants are fitted to 10 000 launches (sixteen shapes of 576 to 32000 weight rows and 768 to 14336 columns, 12 to 512 rows) and are off by 6 % at the
+// median; what the rule chooses takes 1.4 % longer than the best form, 4 % at worst.
 Form choose_form(const GemmParams &p, bool exact) {
     const int fmt = p.w.format, N = p.w.rows, M = p.rows, unit = fmt == FMT_Q4_K ? 2 : 1, units = p.w.cols / (kStep * unit);
-    const bool f16 = fmt == FMT_F16;
-    const float start = 2.25f, fill = f16 ? 1.84f : 1.34f, step = f16 ? 1.98f : 0.743f, row_tile = f16 ? 0.0f : 0.149f, staged = 0.1f, join = f16 ? 0.47f : 0.383f;
-    const float plane_us = f16 ? 0.233f : 0.28f, again_us = 0.2f;   // per MB
+    const float start = 2.25f, fill = 1.34f, step = 0.743f, row_tile = 0.149f, staged = 0.1f, join = 0.383f;
+    const float plane_us = 0.28f, again_us = 0.2f;   // per MB
     static const int kSplits[] = {1, 2, 3, 4, 6, 8};
     const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
     Form best;
@@ -397,7 +395,8 @@ Form choose_form(const GemmParams &p, bool exact) {
 void block_gemm_set_form(int form) {
     const int tm = form / 100, nw = form / 10 % 10, shares = form % 10;
     const bool known = tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
-    g_block_gemm_form.store(known || form == -1 ? form : 0);
+    g_block_gemm_form.store(known ? form : 0);
+    wide_gemm_set_shared(form == -1);
 }
 
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are
@@ -432,19 +431,7 @@ bool block_gemm_exact(const DeviceMatrix &w, int rows) {
 
 bool block_gemm_takes(const GemmParams &p) {
     const int fmt = p.w.format;
-    if (fmt != FMT_Q4_K && fmt != FMT_Q4_0 && fmt != FMT_Q8_0 && fmt != FMT_F16) return false;
-    if (p.w.cols % (fmt == FMT_Q4_K ? 256 : kStep) != 0) return false;
-    const int forced = g_block_gemm_form.load();
-    if (fmt != FMT_F16 || forced > 0) return true;
-    // fp16 weights are four times the bytes and nothing to unpack, and planes cost them more than they give: 3072 x 3072, 12 / 128 rows 9.0 / 14.4 us in the tile kernel, 11.2 / 17
-    // here.  Tall gate|up matrices do without planes and win here while the tile kernel has no more than one workgroup of 128 x 128 a compute unit; with more of them it hides its
-    // staging (us, there -> here): 11264 x 2048, 96 / 192 / 256 / 384 / 512 rows 27 / 33 / 34 / 38 / 39 -> 21 / 29 / 32 / 45 / 47; 16384 x 3072, 96 / 256 / 384 rows 38 / 54 / 59 -> 32 / 48 / 67;
-    // 28672 x 4096, 96 / 256 / 384 rows 78 / 93 / 129 -> 64 / 97 / 159.  Over nine heights of 8192 to 32000 rows, 1024 to 8192 columns and 65 to 512 rows of activations, what the rule takes
-    // is 0.97 to 1.6 times as fast.  Longer rows gain nothing (8192 columns: 0.96 to 1.02 at up to 128 rows; 4096 columns beyond 128 rows 0.85 to 1.4), nor do products without the SiLU
-    // (14336 x 2048, 96 / 129 / 256 rows 1.01 / 1.29 / 0.92 times as fast).
-    if (forced < 0 || !p.swiglu_out || p.rows <= 64 || p.w.rows < 8192 || p.w.cols > (p.rows <= 128 ? 4096 : 3072)) return false;
-    const long tiles = (long)((p.w.rows + 127) / 128) * ((p.rows + 127) / 128);
-    return tiles <= (device_compute_units() > 0 ? device_compute_units() : 256) && choose_form(p, false).splits == 1;
+    return (fmt == FMT_Q4_K || fmt == FMT_Q4_0 || fmt == FMT_Q8_0) && p.w.cols % (fmt == FMT_Q4_K ? 256 : kStep) == 0;
 }
 
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {
@@ -464,8 +451,7 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
     switch (p.w.format) {
     case FMT_Q4_K: return launch_format<FMT_Q4_K>(f.tm, f.nw, false, a, stream);
     case FMT_Q4_0: return launch_format<FMT_Q4_0>(f.tm, f.nw, exact, a, stream);
-    case FMT_Q8_0: return launch_format<FMT_Q8_0>(f.tm, f.nw, exact, a, stream);
-    default: return launch_format<FMT_F16>(f.tm, f.nw, false, a, stream);
+    default: return launch_format<FMT_Q8_0>(f.tm, f.nw, exact, a, stream);
     }
 }
 

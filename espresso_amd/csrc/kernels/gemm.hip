@@ -5,8 +5,8 @@
 // (RealModelInferenceEngine.swift:6674-6697 inside the prefill loop :6365-6375) by one pass over the
 // packed weights per block of rows.
 //
-// launch_gemm chooses: few rows or small matrices with exact weights (rows_gemm.hip), up to eight rows of Q4_K (gemm_rows_kernel below), blocks of rows
-// (block_gemm.hip), and for what is left - columns that are no multiple of 128, most fp16 matrices - gemm_kernel:
+// launch_gemm chooses: few rows or small matrices with exact weights (rows_gemm.hip), fp16 matrices (wide_gemm.hip), up to eight rows of Q4_K (gemm_rows_kernel below), blocks of rows
+// (block_gemm.hip), and for what is left - columns that are no multiple of 128 - gemm_kernel:
 //   * a workgroup of four wavefronts owns 128 weight rows (n) x MT activation rows (m) and walks K in
 //     tiles of 64;
 //   * per K tile every thread fetches the packed bytes of (one weight row, one half of the tile) with
@@ -26,6 +26,7 @@
 #include "../common.h"
 #include "decode_ops.h"
 #include "block_gemm.h"
+#include "wide_gemm.h"
 #include "rows_gemm.h"
 #include <atomic>
 #include <type_traits>
@@ -77,8 +78,6 @@ template <>
 struct Raw<FMT_Q4_0> { uint4 q; u32 d; };        // one block
 template <>
 struct Raw<FMT_Q8_0> { uint4 q0, q1; u32 d; };   // one block
-template <>
-struct Raw<FMT_F16> { uint4 v[4]; };
 
 template <int FMT>
 __device__ __forceinline__ Raw<FMT> fetch_raw(const GemmArgs &a, int row, int tile, int h) {
@@ -88,16 +87,12 @@ __device__ __forceinline__ Raw<FMT> fetch_raw(const GemmArgs &a, int row, int ti
         const int block = tile * 2 + h;
         r.q = *reinterpret_cast<const uint4 *>(base + (size_t)block * 16);
         r.d = a.scales[(size_t)row * (a.K / 32) + block];
-    } else if constexpr (FMT == FMT_Q8_0) {
+    } else {
         const int block = tile * 2 + h;
         const uint4 *q = reinterpret_cast<const uint4 *>(base + (size_t)block * 32);
         r.q0 = q[0];
         r.q1 = q[1];
         r.d = a.scales[(size_t)row * (a.K / 32) + block];
-    } else {
-        const uint4 *q = reinterpret_cast<const uint4 *>(base + ((size_t)tile * KT + h * 32) * 2);
-#pragma unroll
-        for (int i = 0; i < 4; i++) r.v[i] = q[i];
     }
     return r;
 }
@@ -128,7 +123,7 @@ __device__ __forceinline__ uint2 nibbles_to_half(u32 w, bool high, h2 s, h2 dm) 
 }
 
 // Writes the thread's 32 fp16 weights into its LDS row (`wrow` points at k = 0 of the tile).
-// Element order inside each group of four is (0,2,1,3) for Q4_0 and Q8_0, natural for F16.
+// Element order inside each group of four is (0,2,1,3).
 template <int FMT>
 __device__ __forceinline__ void dequant_to_lds(const Raw<FMT> &r, int h, _Float16 *wrow) {
     if constexpr (FMT == FMT_Q4_0) {
@@ -145,7 +140,7 @@ __device__ __forceinline__ void dequant_to_lds(const Raw<FMT> &r, int h, _Float1
         p[1] = make_uint4(lo[2].x, lo[2].y, lo[3].x, lo[3].y);
         p[2] = make_uint4(hi[0].x, hi[0].y, hi[1].x, hi[1].y);
         p[3] = make_uint4(hi[2].x, hi[2].y, hi[3].x, hi[3].y);
-    } else if constexpr (FMT == FMT_Q8_0) {
+    } else {
         const h2 s = splat(half_bits_to_float(r.d)), off = h2{(_Float16)1152.0f, (_Float16)1152.0f};   // 1024 + 128
         uint4 *p = reinterpret_cast<uint4 *>(wrow + 32 * h);
 #pragma unroll
@@ -163,10 +158,6 @@ __device__ __forceinline__ void dequant_to_lds(const Raw<FMT> &r, int h, _Float1
             p[2 * half] = make_uint4(out[0], out[1], out[2], out[3]);
             p[2 * half + 1] = make_uint4(out[4], out[5], out[6], out[7]);
         }
-    } else {
-        uint4 *p = reinterpret_cast<uint4 *>(wrow + 32 * h);
-#pragma unroll
-        for (int i = 0; i < 4; i++) p[i] = r.v[i];
     }
 }
 
@@ -179,7 +170,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
     constexpr int THREADS = 64 * WM * WN, NTILE = 32 * WN * TN;   // two threads per weight row dequantise
     static_assert(2 * NTILE == THREADS, "one (weight row, half tile) per thread");
     constexpr int MT = 32 * WM * TM;
-    constexpr bool kSwap = FMT == FMT_Q4_0 || FMT == FMT_Q8_0;   // formats whose unpacking yields (0,2,1,3) order
     constexpr int XV = MT * KT / 8 / THREADS;   // 128-bit pieces of x per thread per tile
     static_assert(XV >= 1, "tile too small for the copy loop");
     __shared__ _Float16 xt[2][MT * LDK];
@@ -231,7 +221,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(GemmArgs a) {
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int piece = tid + i * THREADS, row = piece >> 3, part = piece & 7;
-            *reinterpret_cast<uint4 *>(xt[buf] + row * LDK + part * 8) = kSwap ? swap_middle(xv[S][i]) : xv[S][i];
+            *reinterpret_cast<uint4 *>(xt[buf] + row * LDK + part * 8) = swap_middle(xv[S][i]);
         }
         const int ahead = tile + DEPTH < t_last ? tile + DEPTH : t_last;
         raw[S] = fetch_raw<FMT>(a, w_row, ahead, wh);
@@ -533,10 +523,10 @@ hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *defe
         if (deferred_splits) { *deferred_splits = used_splits; return hipSuccess; }
         return launch_reduce(a, used_splits, stream);
     };
-    const int n_blocks = (a.N + NT - 1) / NT;
+    [[maybe_unused]] const int n_blocks = (a.N + NT - 1) / NT;
     a.partial = p.workspace;
-    hipError_t e;
-    int splits;
+    [[maybe_unused]] hipError_t e;
+    [[maybe_unused]] int splits;
     if constexpr (FMT == FMT_Q4_K) {
         // one workgroup per 32 weight rows, K split over its wavefronts
         if (a.M <= kRowsMaxRows) {
@@ -560,6 +550,12 @@ hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *defe
             return go(gemm_rows_kernel<4, 4>, 4, rows_lds_bytes<4, 4>(), raised4);
         }
     }
+    if constexpr (FMT == FMT_F16) {
+        const WideGemmForm f = wide_gemm_form(p);
+        if (!f.bm) return hipErrorInvalidValue;
+        *fused = f.splits == 1 && swiglu_out && a.N % 2 == 0;
+        return finish(launch_wide_gemm(p, f, stream), f.splits);
+    } else {
     if (block_gemm_takes(p)) {
         e = launch_block_gemm(p, &splits, stream);
         *fused = splits == 1 && swiglu_out && a.N % 2 == 0;
@@ -579,6 +575,7 @@ hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *defe
     else if (mt == 64) e = launch_tile<FMT, 1, 4, 2, 1, 4>(a, splits, stream);
     else e = launch_tile<FMT, 2, 2, 2, 2, 2>(a, splits, stream);
     return finish(e, splits);
+    }
     }
 }
 

@@ -15,6 +15,7 @@
 //     Q8_0, Q4_K: 32 p + 16 h + 8 i; fp16 and (after the two halves of a wavefront exchanged half of two blocks) Q4_0: 32 p + 16 i + 8 h.
 #include "../common.h"
 #include "block_gemm.h"
+#include "wide_gemm.h"
 #include "rows_gemm.h"
 #include "silu.h"
 #include <cstdlib>
@@ -318,12 +319,16 @@ bool rows_gemm_takes(const GemmParams &p) {
     //   steps one after the other);  32000 x 768, 32 rows: q8_0 15.4 -> 17.9
     // Over 3 to 512 rows of seventeen shapes (576 to 8192 rows, 256 to 3072 columns) and the four formats, what the rule takes is 0.3 to 1.0 times the tile kernel's
     // time; at three rows of the 2048-column Q4_0 and 512 x 256 matrices, five to seven microseconds each way, up to 1.1 times.
-    // fp16 weights of 2048 columns are four loads a step: 2048 x 2048, 16 / 64 / 93 rows 11.0 / 14.2 / 16.2 -> 12.2 / 13.7 / 13.4.
     // Up to 32 rows that no next kernel finishes: deeper launches too, while all workgroups are resident at once (8192 x 3072, 8 / 32 rows, with shares of K and their sum -> here: q4_0
     // 10.5 / 11.9 -> 9.2 / 11.1, q8_0 12.4 / 14.1 -> 11.6 / 13.9, q4_k 16 rows 12.6 -> 9.3).
     const int steps = w.cols / kStep;
     const long groups = (long)((w.rows + 31) / 32) * ((rows + 31) / 32);
-    if (w.format == FMT_F16 && w.cols > 1536 && rows <= 64) return false;
+    if (w.format == FMT_F16) {
+        // rounds of one workgroup per compute unit against the kernel of wide_gemm.hip (us, here / there: 3072 x 576, 64 / 96 rows 5.1 / 6.3, 8.3 / 6.4;  576 x 1536, 16 / 200 / 400 rows
+        // 6.0 / 5.4, 6.7 / 6.6, 6.8 / 7.6;  1152 x 576, 200 / 320 rows 5.3 / 6.1, 8.5 / 6.2;  2048 columns: there at any number of rows)
+        const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
+        return w.cols <= 1536 && 1.7f + (float)((groups + cus - 1) / cus) * (2.6f + 0.19f * (float)steps) < wide_gemm_form(p).us;
+    }
     const bool deep = groups * steps > 8192 && (rows > 32 || !block_gemm_alone(p) || groups > (device_compute_units() > 0 ? device_compute_units() : 256));
     return w.cols <= 3072 && !deep && !block_gemm_keeps(p);
 }
