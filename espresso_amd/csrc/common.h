@@ -186,7 +186,7 @@ struct SplitRowsParams {
 };
 hipError_t launch_split_rows(const SplitRowsParams &p, hipStream_t stream);
 
-// Of the current device (kernels/gemm_split.hip); 0: it does not say.
+// Of the current device (context.cpp); 0: it does not say.
 int device_compute_units();
 
 // kernels/gemv.hip

@@ -1,5 +1,7 @@
 #include "context.h"
 
+#include <atomic>
+
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -63,6 +65,18 @@ int ensure_init() {
     }
     g_context.ready = true;
     return ESP_OK;
+}
+
+int device_compute_units() {
+    static std::atomic<int> cus[64];
+    int device = 0, n = 0;
+    if (hipGetDevice(&device) != hipSuccess) return 0;
+    n = cus[device & 63].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+        cus[device & 63].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 }  // namespace esp

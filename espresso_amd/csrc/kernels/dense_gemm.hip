@@ -1,7 +1,11 @@
 // Blocks of rows against dense matrices on the matrix cores (gfx950): the prompt products of the layered models.
 //
-//   y[m][n] = sum_k a[m][k] b[n][k],   bf16 operands (or fp32 ones: v_mfma_f32_32x32x2_f32), fp32 accumulation
+//   y[m][n] = sum_k a[m][k] b[n][k],   bf16 operands or fp32 ones, fp32 accumulation
 //
+// bf16 operands: the walk of wide_tile.h (tiles of 64 x 128 to 256 x 256, by the cost rule of wide_form.h).  Against tiles of 128 x 128 (64, 32) of
+// four wavefronts, prompts of six layers, us: Ranavik d768, 40 / 600 / 1700 tokens 498 / 765 / 1250 -> 447 / 596 / 982, d4096, 64 / 300 / 1000 tokens 1330 / 2320 / 4480 -> 1190 / 1860 / 3910,
+// Forovik d2048, 60 / 500 / 1100 tokens 649 / 1158 / 1849 -> 591 / 888 / 1543;  steps of 16 sequences of d2048 (prompts and 24 steps) 20470 -> 18940.
+// fp32 operands (v_mfma_f32_32x32x2_f32):
 //   * a workgroup of four wavefronts owns a BM x BN tile of y and walks k in tiles of 128 bytes per row (64 bf16 or 32 fp32
 //     values); LDS holds two tiles of both operands, so one barrier per tile is enough, and two more are on their way in registers;
 //   * rows of LDS are 144 bytes apart: the 128-bit fragment reads of eight rows cover all banks;
@@ -13,8 +17,13 @@
 
 #include <type_traits>
 
+#include <atomic>
+
+#include "../common.h"
 #include "layer_ops.h"
 #include "matrix_ops.h"
+#include "wide_form.h"
+#include "wide_tile.h"
 
 namespace esp {
 namespace {
@@ -59,9 +68,39 @@ __device__ __forceinline__ void store_piece(uintx4 d, float *lds) {
     reinterpret_cast<floatx4 *>(lds)[1] = __builtin_bit_cast(floatx4, __builtin_shufflevector(lo, hi, 2, 6, 3, 7));
 }
 
+// The 32 rows from m0 on of column n (lane % 32 of its 32).
+template <typename E>
+__device__ __forceinline__ void store_tile(const DenseGemmArgs &a, const floatx16 &acc, int m0, int n, int lane, int split, bool after_mix) {
+    const int half = lane >> 5;
+    if (after_mix) {   // even lanes hold gates, their right neighbours the ups: the even lane finishes rows 2 k of both, the odd lane rows 2 k + 1
+        const bool odd = lane & 1;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float even = acc[2 * k], uneven = acc[2 * k + 1];
+            const float p0 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, even), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+            const float p1 = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, uneven), 0xB1, 0xF, 0xF, false));
+            const int m = m0 + matrix::accumulator_row(2 * k + (odd ? 1 : 0), half);
+            if (m < a.m && (n | 1) < a.n)
+                static_cast<E *>(a.act)[(size_t)m * a.ld_act + (n - a.mix_cols) / 2] = Op<E>::from_float(matrix::gated(a.gate_function, odd ? p1 : even, odd ? uneven : p0));
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int m = m0 + matrix::accumulator_row(r, half);
+        const float v = acc[r];
+        if (m >= a.m || n >= a.n) continue;
+        if (a.out == (int)GemmOut::planes) static_cast<float *>(a.y)[((size_t)split * a.m + m) * a.ldy + n] = v;
+        else if (a.out == (int)GemmOut::mix_gated) static_cast<float *>(a.y)[(size_t)m * a.ldy + n] = v;
+        else if (a.out == (int)GemmOut::elems) static_cast<E *>(a.y)[(size_t)m * a.ldy + n] = Op<E>::from_float(v);
+        else if (n < a.n_store) static_cast<float *>(a.y)[(size_t)m * a.ldy + n] = a.cap > 0.0f ? a.cap * tanhf(v / a.cap) : v;
+    }
+}
+
 template <typename TA, typename TB, int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(64 * WM * WN) void dense_gemm_kernel(DenseGemmArgs a) {
-    using E = typename std::conditional<std::is_same<TA, float>::value || std::is_same<TB, float>::value, float, uint16_t>::type;
+    static_assert(std::is_same<TA, float>::value || std::is_same<TB, float>::value, "bf16 operands have a kernel of their own");
+    using E = float;
     constexpr int THREADS = 64 * WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
     constexpr int KT = 128 / sizeof(E), LDK = 144 / sizeof(E), NCH = KT / 8;   // values per tile row, per LDS row; pieces per tile row
     constexpr int XA = BM * NCH / THREADS, XB = BN * NCH / THREADS;
@@ -153,59 +192,103 @@ __global__ __launch_bounds__(64 * WM * WN) void dense_gemm_kernel(DenseGemmArgs 
     }
     if (t0 < t_end) multiply(0);
 
-    const int half = lane >> 5;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
+        for (int j = 0; j < TN; j++) store_tile<E>(a, acc[i][j], m0 + (wm * TM + i) * 32, n0 + (wn * TN + j) * 32 + (lane & 31), lane, blockIdx.y, after_mix);
+}
+
+// bf16 operands
+template <int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(wide::kThreads) void dense_wide_kernel(DenseGemmArgs a) {
+    using T = wide::Tile<WM, WN, TM, TN>;
+    extern __shared__ uint4 smem[];
+    const auto [m_tile, n_tile, split] = wide::place_of(a.m_tiles, a.n_tiles);
+    const int m0 = m_tile * T::BM, n0 = n_tile * T::BN, first = split * a.tiles_per_split, steps = a.tiles - first < a.tiles_per_split ? a.tiles - first : a.tiles_per_split;
+    const bool after_mix = a.out == (int)GemmOut::mix_gated && n0 >= a.mix_cols;   // a tile lies on one side
+    floatx16 acc[TM][TN];
+    wide::Plain<T::BM, T::kDepth> x(static_cast<const uint16_t *>(after_mix ? a.a2 : a.a), (size_t)a.lda, m0, a.m, (size_t)first * wide::kStep, steps);
+    wide::Plain<T::BN, T::kDepth> w(static_cast<const uint16_t *>(a.b), (size_t)a.ldb, n0, a.n, (size_t)first * wide::kStep, steps);
+    wide::walk<true, WM, WN, TM, TN>(x, w, steps, reinterpret_cast<uint16_t *>(smem), acc);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / WN, wn = wave % WN;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + (wm * TM + i) * 32 + matrix::accumulator_row(r, half);
-                const float v = acc[i][j][r];
-                if (after_mix) {   // even lanes hold gates, their right neighbours the ups
-                    const float up = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-                    if (!(lane & 1) && m < a.m && n < a.n)
-                        static_cast<E *>(a.act)[(size_t)m * a.ld_act + (n - a.mix_cols) / 2] = Op<E>::from_float(matrix::gated(a.gate_function, v, up));
-                    continue;
-                }
-                if (m >= a.m || n >= a.n) continue;
-                if (a.out == (int)GemmOut::planes) static_cast<float *>(a.y)[((size_t)blockIdx.y * a.m + m) * a.ldy + n] = v;
-                else if (a.out == (int)GemmOut::mix_gated) static_cast<float *>(a.y)[(size_t)m * a.ldy + n] = v;
-                else if (a.out == (int)GemmOut::elems) static_cast<E *>(a.y)[(size_t)m * a.ldy + n] = Op<E>::from_float(v);
-                else if (n < a.n_store) static_cast<float *>(a.y)[(size_t)m * a.ldy + n] = a.cap > 0.0f ? a.cap * tanhf(v / a.cap) : v;
-            }
-        }
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) store_tile<uint16_t>(a, acc[i][j], m0 + (wm * TM + i) * 32, n0 + (wn * TN + j) * 32 + (lane & 31), lane, split, after_mix);
+}
+
+int ceil_div(int a, int b) { return (a + b - 1) / b; }
+DenseGemmArgs arguments(const DenseGemm &p, int bm, int bn) {
+    DenseGemmArgs a{};
+    a.a = p.a; a.a2 = p.a2; a.b = p.b; a.lda = p.lda; a.ldb = p.ldb; a.m = p.m; a.n = p.n;
+    a.m_tiles = ceil_div(p.m, bm); a.n_tiles = ceil_div(p.n, bn);
+    a.out = (int)p.out; a.y = p.y; a.ldy = p.ldy; a.mix_cols = p.mix_cols; a.act = p.act; a.ld_act = p.ld_act; a.gate_function = (int)p.gate_function; a.n_store = p.n_store; a.cap = p.cap;
+    return a;
+}
+
+std::atomic<int> g_dense_gemm_form{0};
+WideProduct wide_product(int m, int n, int k) {
+    WideProduct w;
+    w.rows = m; w.weight_rows = n; w.steps = k / wide::kStep; w.compute_units = device_compute_units();
+    w.plane_floats = SIZE_MAX;
+    return w;
+}
+template <int WM, int WN, int TM, int TN>
+hipError_t launch_wide(const DenseGemm &p, int splits, int per, hipStream_t s) {
+    using T = wide::Tile<WM, WN, TM, TN>;
+    static std::atomic<uint64_t> raised{0};
+    const void *kernel = reinterpret_cast<const void *>(dense_wide_kernel<WM, WN, TM, TN>);
+    const hipError_t err = wide::raise_lds_limit(kernel, T::kLdsBytes, raised);
+    if (err != hipSuccess) return err;
+    DenseGemmArgs a = arguments(p, T::BM, T::BN);
+    a.tiles = p.k / wide::kStep;
+    a.tiles_per_split = per;
+    hipLaunchKernelGGL((dense_wide_kernel<WM, WN, TM, TN>), dim3(a.m_tiles * a.n_tiles * splits), dim3(wide::kThreads), T::kLdsBytes, s, a);
+    return hipGetLastError();
+}
+hipError_t run_wide(const DenseGemm &p, hipStream_t s) {
+    WideProduct w = wide_product(p.m, p.n, p.k);
+    w.shares = p.splits;
+    const bool gated = p.out == GemmOut::mix_gated;
+    const float gated_cols = gated && p.n > p.mix_cols ? (float)(p.n - p.mix_cols) : 0.0f, elem = p.out == GemmOut::elems ? 2e-6f : 4e-6f;
+    w.stored_mb = (float)p.m * (((float)p.n - gated_cols) * elem + gated_cols * 1e-6f);
+    w.wide_weights = !gated || p.mix_cols % 256 == 0 || p.mix_cols >= p.n;
+    WideForm f;
+    if (const int forced = g_dense_gemm_form.load(); forced > 0) {   // whatever shares it names
+        w.forced = forced / 10 * 10 + p.splits;
+        f = choose_wide_form(w);
+        w.forced = 0;
+    }
+    if (!f.bm) f = choose_wide_form(w);
+    if (f.splits != p.splits) return hipErrorInvalidValue;   // a share without work would leave its plane unwritten
+    switch (f.bm * 1000 + f.bn) {
+    case 256256: return launch_wide<4, 2, 2, 4>(p, f.splits, f.per, s);
+    case 192256: return launch_wide<2, 4, 3, 2>(p, f.splits, f.per, s);
+    case 128256: return launch_wide<2, 4, 2, 2>(p, f.splits, f.per, s);
+    case 256128: return launch_wide<4, 2, 2, 2>(p, f.splits, f.per, s);
+    case 192128: return launch_wide<2, 4, 3, 1>(p, f.splits, f.per, s);
+    case 128128: return launch_wide<2, 4, 2, 1>(p, f.splits, f.per, s);
+    case 64256: return launch_wide<2, 4, 1, 2>(p, f.splits, f.per, s);
+    case 64128: return launch_wide<2, 4, 1, 1>(p, f.splits, f.per, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 struct TileShape { int bm, bn; };
 // Tall tiles unless they leave compute units without one (a launch that may split k fills the chip that way instead).
-TileShape tile_for(int m, int n, bool f32, bool splits) {
-    if (m <= 32 && !f32) return TileShape{32, 128};
+TileShape tile_for(int m, int n, bool splits) {
     if (m <= 64 || (!splits && ((m + 127) / 128) * ((n + 127) / 128) < 200)) return TileShape{64, 128};
     return TileShape{128, 128};
 }
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
-
 template <typename TA, typename TB>
 hipError_t run(const DenseGemm &p, hipStream_t s) {
-    constexpr bool f32 = std::is_same<TA, float>::value || std::is_same<TB, float>::value;
-    constexpr int KT = f32 ? 32 : 64;
-    const TileShape t = tile_for(p.m, p.n, f32, p.out == GemmOut::planes);
-    DenseGemmArgs a{};
-    a.a = p.a; a.a2 = p.a2; a.b = p.b; a.lda = p.lda; a.ldb = p.ldb; a.m = p.m; a.n = p.n;
+    constexpr int KT = 32;
+    const TileShape t = tile_for(p.m, p.n, p.out == GemmOut::planes);
+    DenseGemmArgs a = arguments(p, t.bm, t.bn);
     a.tiles = p.k / KT;
     a.tiles_per_split = ceil_div(a.tiles, p.splits);
     if ((p.splits - 1) * a.tiles_per_split >= a.tiles) return hipErrorInvalidValue;   // a split without work would leave its plane unwritten
-    a.m_tiles = ceil_div(p.m, t.bm); a.n_tiles = ceil_div(p.n, t.bn);
-    a.out = (int)p.out; a.y = p.y; a.ldy = p.ldy; a.mix_cols = p.mix_cols; a.act = p.act; a.ld_act = p.ld_act; a.gate_function = (int)p.gate_function; a.n_store = p.n_store; a.cap = p.cap;
     const dim3 grid(ceil_div(a.n_tiles, kDies) * kDies * a.m_tiles, p.splits);
-    if constexpr (!f32) {
-        if (t.bm == 32) {
-            hipLaunchKernelGGL((dense_gemm_kernel<TA, TB, 1, 4, 1, 1>), grid, dim3(256), 0, s, a);
-            return hipGetLastError();
-        }
-    }
     if (t.bm == 64) hipLaunchKernelGGL((dense_gemm_kernel<TA, TB, 2, 2, 1, 2>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((dense_gemm_kernel<TA, TB, 2, 2, 2, 2>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
@@ -213,9 +296,19 @@ hipError_t run(const DenseGemm &p, hipStream_t s) {
 
 }  // namespace
 
-// Enough workgroups for two per compute unit, at least four tiles of 64 per split, planes within the workspace.
-int gemm_planes_splits(int m, int n, int k, size_t workspace_floats) {
-    const TileShape t = tile_for(m, n, false, true);
+void dense_gemm_set_form(int form) { g_dense_gemm_form.store(wide_form_known(form) ? form : 0); }
+
+// bf16: as many shares of K as the product and the kernel that adds them take the least time with.  fp32: enough workgroups for two per compute unit, at least four tiles of 64 per share.
+// Planes stay within the workspace.
+int gemm_planes_splits(int m, int n, int k, Precision type, size_t workspace_floats) {
+    if (type == Precision::bf16) {
+        WideProduct w = wide_product(m, n, k);
+        w.stored_mb = (float)m * (float)n * 4e-6f;
+        w.plane_floats = workspace_floats;
+        w.after = -0.2f * w.stored_mb;   // that kernel reads one plane in any case
+        return choose_wide_form(w).splits;
+    }
+    const TileShape t = tile_for(m, n, true);
     const int tiles = ceil_div(m, t.bm) * ceil_div(n, t.bn), k_tiles = k / 64;
     int splits = 1;
     for (int s = 2; s <= 16; s++) {
@@ -231,7 +324,7 @@ hipError_t launch_dense_gemm(const DenseGemm &p, hipStream_t s) {
     if (!p.a || !p.b || (!p.y && !gated_only) || p.m < 1 || p.n < 1 || p.k < 64 || p.k % 64 || p.splits < 1 || p.lda < p.k || p.ldb < p.k || p.lda % 8 || p.ldb % 8) return hipErrorInvalidValue;
     if (p.out != GemmOut::planes && p.splits != 1) return hipErrorInvalidValue;
     if (p.out == GemmOut::mix_gated && (p.mix_cols % 128 || p.n % 2 || (p.n > p.mix_cols && (!p.a2 || !p.act)))) return hipErrorInvalidValue;
-    if (p.a_type == Precision::bf16 && p.b_type == Precision::bf16) return run<uint16_t, uint16_t>(p, s);
+    if (p.a_type == Precision::bf16 && p.b_type == Precision::bf16) return run_wide(p, s);
     if (p.a_type == Precision::f32 && p.b_type == Precision::bf16) return run<float, uint16_t>(p, s);
     if (p.a_type == Precision::bf16 && p.b_type == Precision::f32) return run<uint16_t, float>(p, s);
     return hipErrorInvalidValue;

@@ -551,7 +551,7 @@ hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *defe
         }
     }
     if constexpr (FMT == FMT_F16) {
-        const WideGemmForm f = wide_gemm_form(p);
+        const WideForm f = wide_gemm_form(p);
         if (!f.bm) return hipErrorInvalidValue;
         *fused = f.splits == 1 && swiglu_out && a.N % 2 == 0;
         return finish(launch_wide_gemm(p, f, stream), f.splits);

@@ -1060,17 +1060,6 @@ static int regb_shape_setting() {
 //   1B, gate|up 64 / 128 / 256 / 512 rows 66 / 66 / 68 / 80 -> 26 / 31 / 48 / 76, whole layers 152 / 171 / 186 / 232 -> 83 / 99 / 135 / 210
 // (whole layers: the whole form with splits of 256 columns and more, which is already faster than the splits of 1024 it had before:
 // 1B 64 / 512 rows 200 / 265)
-int device_compute_units() {
-    static std::atomic<int> cus[64];
-    int device = 0, n = 0;
-    if (hipGetDevice(&device) != hipSuccess) return 0;
-    n = cus[device & 63].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
-        cus[device & 63].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
 struct RegBForm { int narrow, splits; float us; };
 static int g_regb_narrow = -1;   // -1: the rule; 0: never narrow; 1, 2, 4: always that form (tests, measurements)
 void gemm_split_set_narrow(int form) { g_regb_narrow = form == 0 || form == 1 || form == 2 || form == 4 ? form : -1; }

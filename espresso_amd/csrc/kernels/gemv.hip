@@ -36,6 +36,7 @@
 #include "../common.h"
 #include "block_gemm.h"
 #include "wide_gemm.h"
+#include "layer_ops.h"
 #include "block_split.h"
 #include "rows_gemm.h"
 
@@ -2821,6 +2822,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "short_blocks") { g_short_blocks.store(value != 0); return true; }
     if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
+    if (k == "dense_gemm_form") { dense_gemm_set_form(value); return true; }
     if (k == "wide_gemm_form") { wide_gemm_set_form(value); return true; }
     if (k == "block_split_form") { block_split_set_form(value); return true; }
     if (k == "split_gemm_narrow") { gemm_split_set_narrow(value); return true; }

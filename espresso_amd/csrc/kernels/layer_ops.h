@@ -103,7 +103,8 @@ struct DenseGemm {
     float cap = 0;
     int splits = 1;
 };
-int gemm_planes_splits(int m, int n, int k, size_t workspace_floats);
+int gemm_planes_splits(int m, int n, int k, Precision type, size_t workspace_floats);   // type: of the activations
+void dense_gemm_set_form(int form);   // bf16 products: 0 by size (default), otherwise always that tile: rows * 10000 + weight rows * 10 + 1
 hipError_t launch_dense_gemm(const DenseGemm &p, hipStream_t s);
 
 // ---- embedding, residual stream and norms (layer_ops.hip) -------------------------------------------------

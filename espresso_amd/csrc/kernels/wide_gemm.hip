@@ -35,8 +35,8 @@ __global__ __launch_bounds__(kThreads) void wide_gemm_kernel(WideArgs a) {
     const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
     const int m0 = m_tile * T::BM, n0 = n_tile * T::BN, all = a.K / kStep, first = split * a.per, steps = all - first < a.per ? all - first : a.per;
     floatx16 acc[TM][TN];
-    Plain<T::BM> x(a.x, (size_t)a.K, m0, a.M, (size_t)first * kStep, steps);
-    Plain<T::BN> w(a.w, (size_t)a.K, n0, a.N, (size_t)first * kStep, steps);
+    Plain<T::BM, T::kDepth> x(a.x, (size_t)a.K, m0, a.M, (size_t)first * kStep, steps);
+    Plain<T::BN, T::kDepth> w(a.w, (size_t)a.K, n0, a.N, (size_t)first * kStep, steps);
     walk<false, WM, WN, TM, TN>(x, w, steps, lds, acc);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / WN, wn = wave % WN, h = lane >> 5, col = lane & 31;
     float *out = a.splits > 1 ? a.partial + (size_t)split * a.M * a.N : a.y;
@@ -75,19 +75,12 @@ hipError_t launch(const WideArgs &a, hipStream_t stream) {
     using T = Tile<WM, WN, TM, TN>;
     static std::atomic<uint64_t> raised{0};
     const void *kernel = reinterpret_cast<const void *>(wide_gemm_kernel<WM, WN, TM, TN>);
-    int device = 0;
-    hipError_t err = hipGetDevice(&device);
+    const hipError_t err = raise_lds_limit(kernel, T::kLdsBytes, raised);
     if (err != hipSuccess) return err;
-    const uint64_t bit = 1ull << (device & 63);
-    if (!(raised.load(std::memory_order_acquire) & bit)) {
-        err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::kLdsBytes);
-        if (err != hipSuccess) return err;
-        raised.fetch_or(bit, std::memory_order_release);
-    }
     hipLaunchKernelGGL((wide_gemm_kernel<WM, WN, TM, TN>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), T::kLdsBytes, stream, a);
     return hipGetLastError();
 }
-hipError_t launch_form(const WideGemmForm &f, const WideArgs &a, hipStream_t stream) {
+hipError_t launch_form(const WideForm &f, const WideArgs &a, hipStream_t stream) {
     switch (f.bm * 1000 + f.bn) {
     case 256256: return launch<4, 2, 2, 4>(a, stream);
     case 192256: return launch<2, 4, 3, 2>(a, stream);
@@ -100,54 +93,31 @@ hipError_t launch_form(const WideGemmForm &f, const WideArgs &a, hipStream_t str
     default: return hipErrorInvalidValue;
     }
 }
-// us: a launch's start, a step of 64 k with one workgroup on a compute unit and with two (0: one is resident), filling and emptying a tile
-struct FormCost { int bm, bn; float start, step, step_of_two, fill; };
-constexpr FormCost kForms[] = {{64, 128, 3.17f, 0.339f, 0.657f, 0.0f}, {64, 256, 2.36f, 0.478f, 0.0f, 1.6f}, {128, 128, 3.97f, 0.405f, 0.947f, 0.0f}, {128, 256, 2.80f, 0.655f, 0.0f, 2.57f},
-                               {192, 128, 1.45f, 0.556f, 0.0f, 2.84f}, {192, 256, 1.50f, 0.886f, 0.0f, 5.33f}, {256, 128, 1.44f, 0.669f, 0.0f, 3.91f}, {256, 256, 0.0f, 1.082f, 0.0f, 8.44f}};
 std::atomic<int> g_wide_gemm_form{0};
 std::atomic<bool> g_wide_gemm_shared{false};
 
 }  // namespace
 
 void wide_gemm_set_shared(bool shared) { g_wide_gemm_shared.store(shared); }
-void wide_gemm_set_form(int form) {
-    bool known = false;
-    for (const FormCost &f : kForms) known = known || (form / 10000 == f.bm && form / 10 % 1000 == f.bn && form % 10 >= 1);
-    g_wide_gemm_form.store(known ? form : 0);
+void wide_gemm_set_form(int form) { g_wide_gemm_form.store(wide_form_known(form) ? form : 0); }
+
+// (behind a SiLU, and where no caller adds them, the planes take a launch of their own)
+WideForm wide_gemm_form(const GemmParams &p) {
+    if (p.w.format != FMT_F16 || p.w.cols % kStep != 0) return WideForm{};
+    WideProduct w;
+    w.rows = p.rows; w.weight_rows = p.w.rows; w.steps = p.w.cols / kStep; w.compute_units = device_compute_units();
+    w.stored_mb = (float)p.rows * (float)p.w.rows * (p.swiglu_out ? 1e-6f : 4e-6f);
+    w.plane_floats = p.workspace ? p.workspace_floats : 0;
+    w.after = p.swiglu_out ? 3.0f : p.deferred_splits ? 1.0f : 1.6f;
+    w.after_share = p.swiglu_out || p.deferred_splits ? 0.0f : 0.2f;
+    w.forced = g_wide_gemm_form.load();
+    if (w.forced == 0 && g_wide_gemm_shared.load() && p.swiglu_out && p.workspace && p.w.rows >= 8192 && p.rows > 64 && w.steps > 1 &&
+        (long)((p.w.rows + 127) / 128) * ((p.rows + 127) / 128) <= (w.compute_units > 0 ? w.compute_units : 256))
+        w.shares = 2;
+    return choose_wide_form(w);
 }
 
-// The form by its expected time: rounds of one or two workgroups per compute unit, what they store, and for shares of K the planes that the next kernel reads once more (behind a SiLU, and
-// where no caller adds them, a launch of its own).  Constants fitted to 2500 launches (fourteen shapes of 576 to 28672 weight rows and 576 to 14336 columns, 3 to 2048 rows): off by 4 % at
-// the median, and what the rule chooses takes 0.3 % longer than the best form on average, 10 % at worst.
-WideGemmForm wide_gemm_form(const GemmParams &p) {
-    WideGemmForm best;
-    const int forced = g_wide_gemm_form.load(), all = p.w.cols / kStep, M = p.rows, N = p.w.rows;
-    if (p.w.format != FMT_F16 || p.w.cols % kStep != 0) return best;
-    const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
-    static const int kSplits[] = {1, 2, 3, 4, 6, 8};
-    const bool in_two = forced == 0 && g_wide_gemm_shared.load() && p.swiglu_out && p.workspace && N >= 8192 && M > 64 && all > 1 && (long)((N + 127) / 128) * ((M + 127) / 128) <= cus;
-    for (const FormCost &f : kForms) {
-        if (forced > 0 && (forced / 10000 != f.bm || forced / 10 % 1000 != f.bn)) continue;
-        if (forced == 0 && f.bm > 64 && f.bm - 64 >= M) continue;   // rows that no activation fills
-        const long tiles = (long)((N + f.bn - 1) / f.bn) * ((M + f.bm - 1) / f.bm);
-        for (int want : kSplits) {
-            if ((forced > 0 && forced % 10 != want) || (in_two && want != 2)) continue;
-            const int per = (all + want - 1) / want, splits = (all + per - 1) / per;
-            if ((splits != want && forced == 0) || (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
-            const long wgs = tiles * splits, at_once = f.step_of_two > 0.0f ? 2 * cus : cus, whole = wgs / at_once, rest = wgs % at_once;
-            const float rounds = (float)(whole + (rest > 0));
-            const float steps = (float)per * ((float)whole * (f.step_of_two > 0.0f ? f.step_of_two : f.step) + (rest == 0 ? 0.0f : rest > cus ? f.step_of_two : f.step));
-            const bool gated = p.swiglu_out && splits == 1;
-            const float mb = gated ? (float)M * (float)N * 1e-6f : (float)splits * (float)M * (float)N * 4e-6f;
-            float us = f.start + steps + rounds * f.fill + 0.22f * mb;
-            if (splits > 1) us += 0.2f * mb + (p.swiglu_out ? 3.0f : p.deferred_splits ? 1.0f : 1.6f + 0.2f * (float)splits);
-            if (!best.bm || us < best.us) best = WideGemmForm{f.bm, f.bn, per, splits, us};
-        }
-    }
-    return best;
-}
-
-hipError_t launch_wide_gemm(const GemmParams &p, const WideGemmForm &f, hipStream_t stream) {
+hipError_t launch_wide_gemm(const GemmParams &p, const WideForm &f, hipStream_t stream) {
     const WideArgs a{reinterpret_cast<const uint16_t *>(p.w.qs), p.w.rows, p.w.cols, p.rows, p.x, p.y, p.residual, p.workspace, f.splits == 1 && p.w.rows % 2 == 0 ? p.swiglu_out : nullptr,
                      f.per, f.splits, (p.w.rows + f.bn - 1) / f.bn, (p.rows + f.bm - 1) / f.bm};
     return launch_form(f, a, stream);

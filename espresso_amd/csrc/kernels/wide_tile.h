@@ -1,18 +1,19 @@
-// Products of long blocks of activation rows on the matrix cores, y[m][n] = sum_k x[m][k] w[n][k]: the walk over K that wide_gemm.hip (weights in GGUF formats) and dense_gemm.hip
-// (bf16 weights) share.
+// Products of three and more rows of activations on the matrix cores, y[m][n] = sum_k x[m][k] w[n][k], both operands in sixteen bits: the walk over K that wide_gemm.hip (fp16) and
+// dense_gemm.hip (bf16) share.
 //
 // A workgroup is eight wavefronts, WM x WN of them, each with TM x TN products of 32 x 32; it walks K in steps of 64 through two LDS buffers that hold both operands as sixteen-bit values.
 // What bounds a product of many rows is neither memory nor the matrix cores alone but how long a wavefront waits for its fragments, so
 //   * tiles are as large as the registers allow (256 x 256: six fragments of LDS for eight products; 64 x 64 a wavefront, as in the 128 x 128 tiles of four wavefronts, reads eight for eight);
-//   * a weight is unpacked once for all rows of the tile, by the thread that takes it from memory to LDS;
+//   * small tiles, which few rows take, keep four steps on their way from memory in registers (8 rows of 10368 x 2048, 81 workgroups: 22 us with one step, 16.3);
 //   * fragments of the next sixteen k are read while these are multiplied, also across the step: the barrier stands before the step's last sixteen k, whose fragments are in registers
 //     by then, so one barrier a step suffices and the first fragments behind it are on their way before the products end;
-//   * writes to the other buffer and loads of the step after next are spread over the step (sched_group_barrier: product, read, write, load by turns; left to the compiler 4 to 8 % slower).
+//   * writes to the other buffer and loads of a later step are spread over the step (sched_group_barrier: product, read, write, load by turns; left to the compiler 4 to 8 % slower).
 // Rows of LDS are 144 bytes apart, so that reads of eight rows fall on all banks.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 #include <type_traits>
 
 namespace esp {
@@ -31,6 +32,8 @@ struct Tile {
     static constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, kBuffer = (BM + BN) * kPitch;
     static constexpr size_t kLdsBytes = (size_t)2 * kBuffer * 2;
     static_assert(kLdsBytes <= 160 * 1024, "LDS of a compute unit");
+    // Steps in registers on their way to LDS: small tiles are bound by the weights' way from memory, and what is in flight is all that shortens it
+    static constexpr int kDepth = BM + BN <= 192 ? 4 : BM + BN <= 384 ? 2 : 1;
 };
 
 // The workgroup's place: workgroups of one die take neighbouring output tiles, the row tiles of one block of weights first.
@@ -42,14 +45,26 @@ __device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) {
     return {unit % m_tiles, rest % n_tiles, rest / n_tiles};
 }
 
+// The limit of dynamic LDS, raised once per kernel and device (`raised`: the kernel's own).
+inline hipError_t raise_lds_limit(const void *kernel, size_t lds, std::atomic<uint64_t> &raised) {
+    int device = 0;
+    hipError_t err = hipGetDevice(&device);
+    if (err != hipSuccess) return err;
+    const uint64_t bit = 1ull << (device & 63);
+    if (raised.load(std::memory_order_acquire) & bit) return hipSuccess;
+    err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err == hipSuccess) raised.fetch_or(bit, std::memory_order_release);
+    return err;
+}
+
 // Rows of sixteen-bit values on their way to LDS, 64 k a step: the activations, and weights that need no unpacking.
-template <int ROWS>
+template <int ROWS, int DEPTH>
 struct Plain {
     static constexpr int kPieces = ROWS * 8 / kThreads;
     static_assert(ROWS * 8 % kThreads == 0 && kPieces >= 1, "whole pieces");
     const uint16_t *base;
     uint32_t offset[kPieces];
-    uintx4 raw[kPieces];
+    uintx4 raw[DEPTH][kPieces];
     int last, at_lds;
     // rows row0 .. of a matrix of `count`: those beyond repeat the last one, never stored
     __device__ __forceinline__ Plain(const uint16_t *m, size_t ld, int row0, int count, size_t k0, int steps) : base(m + (size_t)row0 * ld + k0), last(steps - 1) {
@@ -60,19 +75,19 @@ struct Plain {
         }
         at_lds = (threadIdx.x >> 3) * kPitch + (threadIdx.x & 7) * 8;
     }
-    __device__ __forceinline__ void load_piece(int i, int s) { raw[i] = *reinterpret_cast<const uintx4 *>(base + (size_t)(s < last ? s : last) * kStep + offset[i]); }
-    __device__ __forceinline__ void load(int s) {
+    __device__ __forceinline__ void load_piece(int slot, int i, int s) { raw[slot][i] = *reinterpret_cast<const uintx4 *>(base + (size_t)(s < last ? s : last) * kStep + offset[i]); }
+    __device__ __forceinline__ void load(int slot, int s) {
 #pragma unroll
-        for (int i = 0; i < kPieces; i++) load_piece(i, s);
+        for (int i = 0; i < kPieces; i++) load_piece(slot, i, s);
     }
-    // part PART of three of the step in registers to LDS, and what comes after it on its way
-    template <int PART>
+    // part PART of three of the step in slot SLOT to LDS, and step `next` on its way there
+    template <int PART, int SLOT>
     __device__ __forceinline__ void stage(uint16_t *lds, int next) {
 #pragma unroll
         for (int i = 0; i < kPieces; i++)
             if (i * 3 / kPieces == PART) {
-                *reinterpret_cast<uintx4 *>(lds + at_lds + i * (kThreads / 8) * kPitch) = raw[i];
-                load_piece(i, next);
+                *reinterpret_cast<uintx4 *>(lds + at_lds + i * (kThreads / 8) * kPitch) = raw[SLOT][i];
+                load_piece(SLOT, i, next);
             }
     }
 };
@@ -102,29 +117,35 @@ __device__ __forceinline__ void walk(Rows &x, Weights &w, int steps, uint16_t *l
 #pragma unroll
         for (int i = 0; i < TM; i++) xf[slot][i] = *reinterpret_cast<const uintx4 *>(lds + buf * T::kBuffer + fx + i * 32 * kPitch + ks * 16);
     };
-    auto stage = [&](auto part, int buf, int next) __attribute__((always_inline)) {
-        x.template stage<decltype(part)::value>(lds + buf * T::kBuffer, next);
-        w.template stage<decltype(part)::value>(lds + buf * T::kBuffer + T::BM * kPitch, next);
+    constexpr int D = T::kDepth, U = D < 2 ? 2 : D;   // U steps are written out: buffers and slots by turns
+    auto stage = [&](auto part, auto slot, int buf, int next) __attribute__((always_inline)) {
+        x.template stage<decltype(part)::value, decltype(slot)::value>(lds + buf * T::kBuffer, next);
+        w.template stage<decltype(part)::value, decltype(slot)::value>(lds + buf * T::kBuffer + T::BM * kPitch, next);
     };
     typedef std::integral_constant<int, 0> C0;
     typedef std::integral_constant<int, 1> C1;
     typedef std::integral_constant<int, 2> C2;
-    x.load(0);
-    w.load(0);
-    stage(C0{}, 0, 1);
-    stage(C1{}, 0, 1);
-    stage(C2{}, 0, 1);
+    typedef std::integral_constant<int, 3> C3;
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+        x.load(i, i);
+        w.load(i, i);
+    }
+    stage(C0{}, C0{}, 0, D);
+    stage(C1{}, C0{}, 0, D);
+    stage(C2{}, C0{}, 0, D);
     __syncthreads();
     fragments(0, 0, 0);
-    auto step = [&](auto slot, int s) __attribute__((always_inline)) {
-        constexpr int B = decltype(slot)::value;
+    auto step = [&](auto turn, int s) __attribute__((always_inline)) {
+        constexpr int B = decltype(turn)::value & 1;
+        constexpr std::integral_constant<int, (decltype(turn)::value + 1) % D> slot{};   // of the next step
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             if (ks < 3) {
                 fragments((ks + 1) & 1, B, ks + 1);
-                if (ks == 0) stage(C0{}, B ^ 1, s + 2);
-                else if (ks == 1) stage(C1{}, B ^ 1, s + 2);
-                else stage(C2{}, B ^ 1, s + 2);
+                if (ks == 0) stage(C0{}, slot, B ^ 1, s + 1 + D);
+                else if (ks == 1) stage(C1{}, slot, B ^ 1, s + 1 + D);
+                else stage(C2{}, slot, B ^ 1, s + 1 + D);
             } else {
                 __syncthreads();   // everybody has read this buffer, and written the other one
                 fragments(0, B ^ 1, 0);
@@ -144,11 +165,19 @@ __device__ __forceinline__ void walk(Rows &x, Weights &w, int steps, uint16_t *l
         }
     };
     int s = 0;
-    for (; s + 2 <= steps; s += 2) {
+    for (; s + U <= steps; s += U) {
         step(C0{}, s);
         step(C1{}, s + 1);
+        if constexpr (U == 4) {
+            step(C2{}, s + 2);
+            step(C3{}, s + 3);
+        }
     }
     if (s < steps) step(C0{}, s);
+    if constexpr (U == 4) {
+        if (s + 1 < steps) step(C1{}, s + 1);
+        if (s + 2 < steps) step(C2{}, s + 2);
+    }
 }
 
 }  // namespace wide

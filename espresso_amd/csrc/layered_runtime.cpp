@@ -310,7 +310,7 @@ int LayeredRuntime::enqueue_step_sequential(float *final_out) {
 int LayeredRuntime::enqueue_planes(const DenseMatrix &w, int rows, int *splits) {
     DenseGemm o;
     o.a = act_; o.a_type = precision_; o.lda = w.ld; o.b = w.w; o.ldb = w.ld; o.m = rows; o.n = width_p_; o.k = w.ld;
-    o.out = GemmOut::planes; o.y = workspace_; o.ldy = width_p_; o.splits = gemm_planes_splits(rows, width_p_, w.ld, workspace_floats_);
+    o.out = GemmOut::planes; o.y = workspace_; o.ldy = width_p_; o.splits = gemm_planes_splits(rows, width_p_, w.ld, precision_, workspace_floats_);
     const int rc = time_begin(K_OUT);
     if (rc != ESP_OK) return rc;
     ESP_HIP_TRY(launch_dense_gemm(o, context().stream));
