@@ -356,7 +356,7 @@ int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, flo
     // twice: the second launch runs under the next launch number and finds the first one's flags in place
     for (int pass = 0; pass < 2 && e == hipSuccess; pass++) {
         GemmSplitParams g;
-        g.w = m; g.x = v; g.rows = rows; g.swiglu = out; g.shared_k = &pool;
+        g.w = m; g.x = v; g.rows = rows; g.swiglu = out; g.shared_k = &pool; g.wide = false;
         if (pass == 1) e = hipMemsetAsync(out.hi, 0xff, na * 2, c.stream);
         if (e == hipSuccess) e = launch_gemm_split(g, c.stream);
     }

@@ -159,6 +159,7 @@ struct GemmSplitParams {
     // fill whole rounds of the chip runs one workgroup per compute unit with equal shares of K tiles; workgroups that share an output
     // tile hand partial totals over through the pool.  One launch at a time per device.
     const struct GemmSplitSharedK *shared_k = nullptr;
+    bool wide = true;                 // whether wide_split.hip may take the product unasked
 };
 struct GemmSplitSharedK {
     unsigned *flags = nullptr;

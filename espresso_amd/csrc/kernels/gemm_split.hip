@@ -24,6 +24,7 @@
 #include "block_split.h"
 #include "silu.h"
 #include "split_rows.h"
+#include "wide_split.h"
 #include <atomic>
 #include <mutex>
 #include <cmath>
@@ -1126,13 +1127,25 @@ hipError_t launch_gemm_split(const GemmSplitParams &p, hipStream_t stream) {
     if (g_regb_narrow < 0 && !lds_weights && regb_shape_setting() == 4) {
         const BlockSplitForm f = block_split_form(p);
         // (behind a SiLU planes cannot split K, and from some 200 rows on whole tiles and shared K ranges win: 28672 x 4096, 256 / 480 rows 138 / 259 us, 150 / 282 there)
-        if (f.tm && (f.us == 0.0f || !regb || (form.us > 0.0f && f.us < form.us && (!swiglu || p.rows <= 128)))) {
-            if (p.deferred_splits) *p.deferred_splits = 1;
+        const bool block = f.tm && (f.us == 0.0f || !regb || (form.us > 0.0f && f.us < form.us && (!swiglu || p.rows <= 128)));
+        // Whole tiles of 128 x 256 (wide_split.hip) where they are expected to be faster than both; shared K ranges take 2.75 us a tile of K.  Over thirteen shapes and 128 to 2048 rows this takes them for
+        // 50 of 138 products, 1.12 times as fast on average and 0.97 at worst (300 rows of 28672 x 4096).
+        const WideSplitForm wide = wide_split_form(p);
+        const int shared = regb && swiglu ? shared_k_workgroups_for(p, tiles) : 0;
+        const float before = block ? f.us : shared ? 3.0f + 2.75f * (float)((long)((a.N + 255) / 256) * ((a.M + MT - 1) / MT) * tiles / shared) : form.us;
+        int planes = 0;   // 0: neither
+        if (wide.per && (wide.us == 0.0f || (p.wide && before > 0.0f && wide.us < before))) {
+            e = launch_wide_split(p, wide, stream);
+            planes = wide.splits;
+        } else if (block) {
             e = launch_block_split(p, f, stream);
-            if (e != hipSuccess || f.splits == 1) return e;
-            if (p.deferred_splits) { *p.deferred_splits = f.splits; return hipSuccess; }
+            planes = f.splits;
+        }
+        if (planes) {
+            if (p.deferred_splits) *p.deferred_splits = planes;
+            if (e != hipSuccess || planes == 1 || p.deferred_splits) return e;
             const size_t count = (size_t)a.M * a.N;
-            hipLaunchKernelGGL(split_gemm_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, a.partial, f.splits, count, a.residual, a.y);
+            hipLaunchKernelGGL(split_gemm_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, a.partial, planes, count, a.residual, a.y);
             return hipGetLastError();
         }
     }

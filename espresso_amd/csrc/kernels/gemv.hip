@@ -38,6 +38,7 @@
 #include "wide_gemm.h"
 #include "layer_ops.h"
 #include "block_split.h"
+#include "wide_split.h"
 #include "rows_gemm.h"
 
 #include <hip/hip_ext.h>
@@ -2825,6 +2826,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "dense_gemm_form") { dense_gemm_set_form(value); return true; }
     if (k == "wide_gemm_form") { wide_gemm_set_form(value); return true; }
     if (k == "block_split_form") { block_split_set_form(value); return true; }
+    if (k == "wide_split_shares") { wide_split_set_shares(value); return true; }
     if (k == "split_gemm_narrow") { gemm_split_set_narrow(value); return true; }
     if (k == "split_gemm_shared_k") { gemm_split_set_shared_k(value); return true; }
     if (k == "prompt_attention_key_sets") { attention_prompt_set_key_sets(value); return true; }

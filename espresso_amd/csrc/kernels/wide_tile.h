@@ -57,25 +57,33 @@ inline hipError_t raise_lds_limit(const void *kernel, size_t lds, std::atomic<ui
     return err;
 }
 
+// Sixteen (or eight) bytes at a uniform base and a lane's own 32-bit offset, one load without vector arithmetic: the offset is hidden from the optimiser where it is used, or its widening
+// to 64 bits leaves the loop, takes two registers and an addition for each load.
+template <class V>
+__device__ __forceinline__ V load_at(const uint8_t *base, uint32_t offset) {
+    asm volatile("" : "+v"(offset));
+    return *reinterpret_cast<const V *>(base + offset);
+}
+
 // Rows of sixteen-bit values on their way to LDS, 64 k a step: the activations, and weights that need no unpacking.
 template <int ROWS, int DEPTH>
 struct Plain {
     static constexpr int kPieces = ROWS * 8 / kThreads;
     static_assert(ROWS * 8 % kThreads == 0 && kPieces >= 1, "whole pieces");
-    const uint16_t *base;
-    uint32_t offset[kPieces];
+    const uint8_t *base;
+    uint32_t offset[kPieces];   // bytes from base on
     uintx4 raw[DEPTH][kPieces];
     int last, at_lds;
     // rows row0 .. of a matrix of `count`: those beyond repeat the last one, never stored
-    __device__ __forceinline__ Plain(const uint16_t *m, size_t ld, int row0, int count, size_t k0, int steps) : base(m + (size_t)row0 * ld + k0), last(steps - 1) {
+    __device__ __forceinline__ Plain(const uint16_t *m, size_t ld, int row0, int count, size_t k0, int steps) : base(reinterpret_cast<const uint8_t *>(m + (size_t)row0 * ld + k0)), last(steps - 1) {
 #pragma unroll
         for (int i = 0; i < kPieces; i++) {
             const int piece = threadIdx.x + i * kThreads, r = piece >> 3;
-            offset[i] = (uint32_t)(row0 + r < count ? r : count - 1 - row0) * (uint32_t)ld + (piece & 7) * 8;
+            offset[i] = (uint32_t)(row0 + r < count ? r : count - 1 - row0) * (uint32_t)(2 * ld) + (piece & 7) * 16;
         }
         at_lds = (threadIdx.x >> 3) * kPitch + (threadIdx.x & 7) * 8;
     }
-    __device__ __forceinline__ void load_piece(int slot, int i, int s) { raw[slot][i] = *reinterpret_cast<const uintx4 *>(base + (size_t)(s < last ? s : last) * kStep + offset[i]); }
+    __device__ __forceinline__ void load_piece(int slot, int i, int s) { raw[slot][i] = load_at<uintx4>(base + (size_t)(s < last ? s : last) * (2 * kStep), offset[i]); }
     __device__ __forceinline__ void load(int slot, int s) {
 #pragma unroll
         for (int i = 0; i < kPieces; i++) load_piece(slot, i, s);
