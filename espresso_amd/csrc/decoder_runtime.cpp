@@ -207,6 +207,42 @@ int DecoderRuntime::prefill(int seq, const uint32_t *tokens, int count) {
     return append(seq, tokens, count);
 }
 
+int DecoderRuntime::prefill_batch(const uint32_t *const *prompts, const int *counts, int count) {
+    int rc = ESP_OK;
+    bool valid = finalized_ && matrix_prefill_ && count > 1 && count <= shape().max_sequences;   // what is not is refused where its turn comes
+    for (int s = 0; s < count && valid; s++) {
+        valid = prompts[s] && counts[s] > 0 && counts[s] <= shape().max_seq;
+        for (int i = 0; i < counts[s] && valid; i++) valid = prompts[s][i] < (uint32_t)shape().vocab;
+    }
+    std::vector<char> done(count > 0 ? count : 0, 0);
+    for (int kind = 1; kind <= 2 && valid && matrix_prefill_supported(); kind++) {
+        std::vector<PromptSpan> spans;
+        long total = 0;
+        for (int s = 0; s < count; s++)
+            if (counts[s] <= block_rows_ && block_prefill_pays(counts[s], 0) && shared_block_class(counts[s]) == kind) {
+                spans.push_back(PromptSpan{s, prompts[s], counts[s]});
+                total += counts[s];
+            }
+        const long blocks = (total + block_rows_ - 1) / block_rows_, even = blocks > 0 ? (total + blocks - 1) / blocks : 0;   // of about one size
+        for (size_t first = 0, next; first < spans.size(); first = next) {
+            int rows = 0;
+            for (next = first; next < spans.size() && rows < even && rows + spans[next].count <= block_rows_; next++) rows += spans[next].count;
+            if (next - first < 2) continue;   // a block of its own, below
+            if ((rc = prefill_shared_block(&spans[first], (int)(next - first))) != ESP_OK) return rc;
+            for (size_t i = first, row = 0; i < next; i++) {
+                row += spans[i].count;
+                if ((rc = keep_row((int)row - 1, spans[i].sequence)) != ESP_OK) return rc;
+                visible_[spans[i].sequence] = spans[i].count;
+                done[spans[i].sequence] = 1;
+            }
+            ESP_HIP_TRY(hipStreamSynchronize(context().stream));
+        }
+    }
+    for (int s = 0; s < count; s++)
+        if (!done[s] && (rc = prefill(s, prompts[s], counts[s])) != ESP_OK) return rc;
+    return ESP_OK;
+}
+
 int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int *want, int want_count, float *logits) {
     if (!finalized_) return fail(ESP_ERR_INVALID_ARGUMENT, "runtime is not finalized");
     if (count <= 0 || !tokens) return fail(ESP_ERR_INVALID_ARGUMENT, "Prompt tokens must not be empty");
@@ -275,10 +311,12 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
 }
 
 // Token, position and sequence of a block's rows into the device arrays.
-int DecoderRuntime::upload_block_rows(int seq, const uint32_t *tokens, int rows, int base) {
+int DecoderRuntime::upload_block_rows(const PromptSpan *spans, int count, int base) {
     hipStream_t s = context().stream;
-    std::vector<int> h_tok(rows), h_pos(rows), h_seq(rows, seq);
-    for (int i = 0; i < rows; i++) { h_tok[i] = (int)tokens[i]; h_pos[i] = base + i; }
+    std::vector<int> h_tok, h_pos, h_seq;
+    for (int k = 0; k < count; k++)
+        for (int i = 0; i < spans[k].count; i++) { h_tok.push_back((int)spans[k].tokens[i]); h_pos.push_back(base + i); h_seq.push_back(spans[k].sequence); }
+    const size_t rows = h_tok.size();
     ESP_HIP_TRY(hipMemcpyAsync(d_tokens_, h_tok.data(), sizeof(int) * rows, hipMemcpyHostToDevice, s));
     ESP_HIP_TRY(hipMemcpyAsync(d_pos_, h_pos.data(), sizeof(int) * rows, hipMemcpyHostToDevice, s));
     ESP_HIP_TRY(hipMemcpyAsync(d_seq_, h_seq.data(), sizeof(int) * rows, hipMemcpyHostToDevice, s));

@@ -33,6 +33,8 @@ struct DecoderShape {
     int max_sequences = 1;    // independent sequence slots (KV caches, recurrent states)
 };
 
+struct PromptSpan { int sequence; const uint32_t *tokens; int count; };   // a whole prompt of an empty sequence
+
 class DecoderRuntime {
   public:
     virtual ~DecoderRuntime();
@@ -65,6 +67,8 @@ class DecoderRuntime {
     // forward one token at the sequence's visible position and keep its hidden state (:672-680)
     int advance(int seq, uint32_t token);
     int prefill(int seq, const uint32_t *tokens, int count);   // from an empty sequence (:637-645)
+    // Prompts of the sequences 0 .. count - 1, all empty; those that may share a block of rows do, so that the weights are read once for them.
+    int prefill_batch(const uint32_t *const *prompts, const int *counts, int count);
     // The next `count` tokens of a sequence, from the caches and state that its earlier tokens left.  `want` lists (ascending)
     // the places among them whose logits go to `logits` ([want_count][vocab]).
     int append(int seq, const uint32_t *tokens, int count, const int *want = nullptr, int want_count = 0, float *logits = nullptr);
@@ -129,6 +133,10 @@ class DecoderRuntime {
     // `rows` tokens at positions base.. of one sequence as one block; their rows end in hidden_.
     virtual int prefill_block(int seq, const uint32_t *tokens, int rows, int base) = 0;
     virtual bool matrix_prefill_supported() const = 0;
+    // Prompts of one class other than 0 may share a block and come out as in blocks of their own, but for the order of sums.
+    virtual int shared_block_class(int count) const { (void)count; return 0; }
+    // Prompts of a class, their rows behind each other (up to block_rows_), as one block; the rows end in hidden_.
+    virtual int prefill_shared_block(const PromptSpan *spans, int count) { (void)spans; (void)count; return ESP_ERR_UNSUPPORTED; }
     // Whether `count` tokens behind `base` run in blocks rather than in steps (where the layers take blocks at all).
     virtual bool block_prefill_pays(int count, int base) const { (void)base; return count >= kMatrixPrefillMinTokens; }
     virtual int clear_state() = 0;                       // every cache and state of every sequence, enqueued on the stream
@@ -142,7 +150,7 @@ class DecoderRuntime {
     int capture_step_graph(int seq);
     int capture_steps(int seq, int count, hipGraphExec_t *out);
     int replay_steps(int seq, int steps);
-    int upload_block_rows(int seq, const uint32_t *tokens, int rows, int base);
+    int upload_block_rows(const PromptSpan *spans, int count, int base);
     int check_sequence(int seq) const;
 
     bool finalized_ = false;

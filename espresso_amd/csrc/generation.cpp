@@ -143,8 +143,7 @@ int generate_greedy_batch(DecoderRuntime &rt, const uint32_t *const *prompts, co
     out->assign(n_seq, {});
     int eff = 0, rc = batch_budget(rt, nullptr, prompt_counts, n_seq, max_tokens, &eff);
     if (rc != ESP_OK) return rc;
-    for (int s = 0; s < n_seq; s++)
-        if ((rc = rt.prefill(s, prompts[s], prompt_counts[s])) != ESP_OK) return rc;
+    if ((rc = rt.prefill_batch(prompts, prompt_counts, n_seq)) != ESP_OK) return rc;
     auto t0 = Clock::now();
     if (eff > 0) {
         std::vector<uint32_t> current(n_seq);

@@ -52,6 +52,9 @@ struct AttentionArgs {
     // launch_attention_prompt and launch_span_attention only, all three or none: the context as split rows (hi = fp16(v), lo = fp16((v - hi) * 2048),
     // sub-block sums; SplitRowsView) instead of ctx_f16, with the queries and the softmax weights split the same way
     uint16_t *ctx_hi, *ctx_lo, *ctx_sums;
+    // launch_attention_prompt and launch_span_attention only, optional: (first row, rows - 1) of each tile, none of which holds rows of two sequences, instead of every 32 rows of one sequence
+    const int2 *tiles;
+    int tile_count;
 };
 constexpr int kAttentionMaxSplits = 32;
 // Slices of the prefix the grouped-query attention kernel works on in parallel (fixed per runtime).

@@ -510,13 +510,14 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
     static_assert(VP >= 1 && 32 * (HD / 8) % THREADS == 0, "value tile divides over a set of wavefronts");
     static_assert(KP == 1 || KP == 2, "one or two sets");
     __shared__ _Float16 vt_all[KP][2][HD * LDV];
-    const int kvh = blockIdx.x, m0 = blockIdx.y * QT;
+    const int2 tile = a.tiles ? a.tiles[blockIdx.y] : int2{(int)blockIdx.y * QT, rows - 1 - (int)blockIdx.y * QT};
+    const int kvh = blockIdx.x, m0 = tile.x;
     const int phase = KP == 1 ? 0 : (int)threadIdx.x / THREADS;
     const int tid = (int)threadIdx.x - phase * THREADS, lane = tid & 63, wave = tid >> 6, half = lane >> 5, col = lane & 31;
     _Float16 (*vt)[HD * LDV] = vt_all[phase];
     const int head = kvh * (a.n_head / a.n_kv_head) + (int)blockIdx.z * G + wave;   // grid z: sets of G query heads of the KV head
     const int pos0 = a.pos[m0];
-    const int last_row = rows - 1 - m0 < QT - 1 ? rows - 1 - m0 : QT - 1;
+    const int last_row = tile.y < QT - 1 ? tile.y : QT - 1;
     const int t_max = pos0 + last_row;             // last key any row of the tile sees
     const int kd = a.n_kv_head * HD;
     const size_t seq_base = (size_t)a.seq[m0] * a.cache_seq_stride;
@@ -1425,12 +1426,13 @@ bool attention_prompt_supported(int n_head, int n_kv_head, int head_dim) {
 
 template <int HD, int G>
 hipError_t launch_attention_prompt_shape(const AttentionArgs &a, int rows, bool kv_f16, int key_sets, hipStream_t s) {
-    dim3 grid(a.n_kv_head, (rows + 31) / 32);
+    const int tiles = a.tiles ? a.tile_count : (rows + 31) / 32;
+    dim3 grid(a.n_kv_head, tiles);
     // Two sets of wavefronts per workgroup (alternate key tiles) for 128-dim heads: the workgroup keeps its size (the kernel needs more
     // than 256 registers, one wavefront per SIMD), so half of the KV head's query heads go to a second workgroup (grid z).
     constexpr bool kTwoSets = HD == 128;
     constexpr int GS = G >= 2 ? G / 2 : 1;
-    dim3 grid2(a.n_kv_head, (rows + 31) / 32, G / GS);
+    dim3 grid2(a.n_kv_head, tiles, G / GS);
     if (a.ctx_hi) {   // split rows out: fp16 caches only (they hold keys and values exactly)
         if (!kv_f16 || !a.ctx_lo || !a.ctx_sums || (a.n_head * HD) % 256 != 0) return hipErrorInvalidValue;
         if constexpr (kTwoSets) {
@@ -1458,7 +1460,7 @@ static int g_prompt_attention_key_sets = 0;
 void attention_prompt_set_key_sets(int sets) { g_prompt_attention_key_sets = sets == 1 || sets == 2 ? sets : 0; }
 
 hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s) {
-    if (rows <= 0 || !attention_prompt_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
+    if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !attention_prompt_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     const int group = a.n_head / a.n_kv_head;
     const int sets = g_prompt_attention_key_sets ? g_prompt_attention_key_sets : (rows > 64 ? 2 : 1);
     if (a.head_dim == 128) {

@@ -63,8 +63,9 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     __shared__ float state[KP][2][64];
     const int lane = threadIdx.x & 63, phase = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
     const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head;
-    const int m0 = (int)(gridDim.y - 1 - blockIdx.y) * 32;                     // the row tiles with the most keys start first
-    const int last_row = rows - 1 - m0 < 31 ? rows - 1 - m0 : 31;
+    const int y = (int)(gridDim.y - 1 - blockIdx.y);                           // the row tiles with the most keys start first
+    const int2 tile = a.tiles ? a.tiles[y] : int2{32 * y, rows - 1 - 32 * y};
+    const int m0 = tile.x, last_row = tile.y < 31 ? tile.y : 31;
     const int pos0 = a.pos[m0], t_max = pos0 + last_row, kd = a.n_kv_head * HD;
     const size_t base = (size_t)a.seq[m0] * a.cache_seq_stride + (size_t)kvh * HD;
     float scale = 1.0f / sqrtf((float)HD);   // fp16 caches: of the scaled queries
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
 
 template <int HD, bool KV_F16>
 void launch_shape(const AttentionArgs &a, int rows, int sets, hipStream_t s) {
-    const dim3 grid(a.n_head, (rows + 31) / 32);
+    const dim3 grid(a.n_head, a.tiles ? a.tile_count : (rows + 31) / 32);
     if (sets == 1) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 1>), grid, dim3(64), 0, s, a, rows);
     else if (sets == 2) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 2>), grid, dim3(128), 0, s, a, rows);
     else if (sets == 4) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 4>), grid, dim3(256), 0, s, a, rows);
@@ -313,11 +314,11 @@ bool span_attention_supported(int n_head, int n_kv_head, int head_dim) {
 }
 
 hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, bool kv_f16, hipStream_t s) {
-    if (rows <= 0 || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
+    if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
     // 512 rows of 24 heads get four, 241 rows of them eight, 93 rows of 32 heads eight (fp16: 58 us behind 1024, 44 behind 1536, 15.3 of 64 dims behind 700).
-    const int tiles = (keys + 31) / 32, groups = a.n_head * ((rows + 31) / 32);
+    const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32);
     int sets = 1;
     while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
     if (a.head_dim == 128) {

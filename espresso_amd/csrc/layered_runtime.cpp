@@ -394,7 +394,8 @@ int LayeredRuntime::enqueue_block_sequential(int rows, int seq, int base, float 
 }
 
 int LayeredRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int base) {
-    const int rc = upload_block_rows(seq, tokens, rows, base);
+    const PromptSpan span{seq, tokens, rows};
+    const int rc = upload_block_rows(&span, 1, base);
     if (rc != ESP_OK) return rc;
     ESP_HIP_TRY(launch_embed_norm(embedding_, embedding_ld_, d_tokens_, embed_norm_, (float)c_.norm_eps, rows, c_.width, width_p_, hidden_, context().stream));
     return enqueue_block(rows, seq, base, nullptr);

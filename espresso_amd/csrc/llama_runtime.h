@@ -92,6 +92,9 @@ class LlamaRuntime : public DecoderRuntime {
     int clear_state() override;
     unsigned tuning_epoch() const override { return gemv_tuning_epoch(); }
     int enqueue_layers_matrix(int rows, int block_keys = 0);
+    int enqueue_block_attention(AttentionArgs aa, int rows, int block_keys);
+    int shared_block_class(int count) const override;
+    int prefill_shared_block(const PromptSpan *spans, int count) override;
     bool sixteen_rows_supported(int rows) const;
     int enqueue_layers_sixteen(int rows);
     bool matrix_prefill_supported() const override;
@@ -130,6 +133,9 @@ class LlamaRuntime : public DecoderRuntime {
     bool prompt_attention_ = false;   // prompt blocks run attention on the matrix cores
     bool short_span_attention_ = false;   // span_attention_kernel for blocks of few rows
     bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for
+    // the prompts that share the block being enqueued: tiles of those of at least kMatrixPrefillMinTokens tokens, behind them tiles of the shorter ones
+    struct SharedBlock { int long_tiles = 0, short_tiles = 0, longest = 0, longest_short = 0; } shared_;
+    int2 *d_tiles_ = nullptr;
     float *gemm_workspace_ = nullptr;
     size_t gemm_workspace_floats_ = 0;
     GemmSplitSharedK gemm_shared_k_;   // the device's pool for launch_gemm_split's hand-over between workgroups (not owned)

@@ -261,10 +261,8 @@ int generate_two_token_batch(LlamaRuntime &full, LlamaRuntime &draft, const uint
         return fail(ESP_ERR_INVALID_ARGUMENT, "draft vocab %d does not match target vocab %d", draft.config().vocab, full.config().vocab);
     int eff = 0, rc = batch_budget(full, &draft, prompt_counts, n_seq, max_tokens, &eff);
     if (rc != ESP_OK) return rc;
-    for (int s = 0; s < n_seq; s++) {
-        if ((rc = full.prefill(s, prompts[s], prompt_counts[s])) != ESP_OK) return rc;
-        if ((rc = draft.prefill(s, prompts[s], prompt_counts[s])) != ESP_OK) return rc;
-    }
+    if ((rc = full.prefill_batch(prompts, prompt_counts, n_seq)) != ESP_OK) return rc;
+    if ((rc = draft.prefill_batch(prompts, prompt_counts, n_seq)) != ESP_OK) return rc;
     auto t0 = Clock::now();
     std::vector<uint32_t> current(n_seq);
     if (eff > 0) {
