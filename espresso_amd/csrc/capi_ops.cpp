@@ -1,9 +1,8 @@
 // C ABI: library set-up, GGUF block dequantisation, resident matrices and the GEMV entry points.
-#include <cstring>
-#include <vector>
-
 #include <cmath>
 #include <cstring>
+#include <mutex>
+#include <vector>
 
 #include "context.h"
 #include "host/model_support.h"
@@ -37,6 +36,62 @@ static int noalloc_setup(int device) {
 }
 static const DeviceSetup noalloc_scratch(noalloc_setup);
 }  // namespace esp
+
+// ---- staging of single products (esp_gemv) ------------------------------------------------------------------
+// A product of a few rows is 5 us of kernel; three allocations and frees, two pageable copies and their waits made 34 us of it.  One staging area for the process, there while any matrix handle is:
+// pinned memory that takes the call's activations and residual, which a small kernel brings to the device (4 us less than a copy engine's start), and its result, which the product writes there itself.
+// A call that finds it in use by another thread, or that needs more, allocates as before.  4096 x 4096 Q4_K, 2 / 16 / 40 rows 34.8 / 88 / 116 -> 22.7 / 39 / 66 us, of which the caller's Python is 2.
+namespace {
+constexpr size_t kStagedIn = (size_t)1 << 20, kStagedOut = (size_t)4 << 20;   // bytes of activations and of residual or result
+class Staging {
+  public:
+    void join() {   // without memory the calls allocate
+        std::lock_guard<std::mutex> lock(handles_mutex_);
+        if (handles_++ > 0) return;
+        std::lock_guard<std::mutex> call(mutex_);
+        void *host = nullptr;
+        if (hipHostMalloc(&host, kStagedIn + kStagedOut, hipHostMallocDefault) != hipSuccess) host = nullptr;
+        host_ = static_cast<uint8_t *>(host);
+        if (host_ && (hipHostGetDevicePointer(&host, host_, 0) != hipSuccess || device_alloc(&device_, kStagedIn + kStagedOut) != ESP_OK || device_alloc(&planes_, kNoAllocScratchFloats) != ESP_OK)) drop();
+        mapped_ = static_cast<uint8_t *>(host);
+        (void)hipGetLastError();
+        clear_error();
+    }
+    void leave() {
+        std::lock_guard<std::mutex> lock(handles_mutex_);
+        if (--handles_ > 0) return;
+        std::lock_guard<std::mutex> call(mutex_);
+        drop();
+    }
+    std::mutex &mutex() { return mutex_; }
+    bool takes(size_t in, size_t out) const { return host_ && in <= kStagedIn && out <= kStagedOut; }
+    // two regions: activations; the residual, and in its place the result, which comes when the residual is on the device
+    uint8_t *host_in() { return host_; }
+    uint8_t *host_out() { return host_ + kStagedIn; }
+    uint8_t *mapped_in() { return mapped_; }
+    uint8_t *mapped_out() { return mapped_ + kStagedIn; }
+    uint8_t *device_in() { return device_; }
+    uint8_t *device_residual() { return device_ + kStagedIn; }
+    float *planes() { return planes_; }
+
+  private:
+    void drop() {
+        if (host_) (void)hipHostFree(host_);
+        if (device_) (void)hipFree(device_);
+        if (planes_) (void)hipFree(planes_);
+        host_ = device_ = nullptr;
+        planes_ = nullptr;
+    }
+    std::mutex handles_mutex_, mutex_;   // of the count, and of the memory while a call uses it
+    int handles_ = 0;
+    uint8_t *host_ = nullptr, *mapped_ = nullptr, *device_ = nullptr;
+    float *planes_ = nullptr;
+};
+Staging &staging() {
+    static Staging *s = new Staging();   // never destroyed: the device may be gone by then
+    return *s;
+}
+}  // namespace
 
 extern "C" {
 
@@ -73,6 +128,7 @@ ESPMatrix *esp_matrix_create(int format, const void *gguf_blocks, int rows, int 
     if (matrix_upload(format, gguf_blocks, rows, cols, &m) != ESP_OK) return nullptr;
     ESPMatrix *h = new ESPMatrix();
     h->m = m;
+    staging().join();
     return h;
 }
 
@@ -80,6 +136,7 @@ void esp_matrix_free(ESPMatrix *matrix) {
     if (!matrix) return;
     matrix_release(&matrix->m);
     delete matrix;
+    staging().leave();
 }
 
 size_t esp_matrix_bytes(const ESPMatrix *matrix) { return matrix ? matrix->m.bytes() : 0; }
@@ -140,6 +197,21 @@ int esp_gemv(const ESPMatrix *matrix, const uint16_t *x_f16, int batch, float *y
     Context &c = context();
     const DeviceMatrix &m = matrix->m;
     const size_t nx = (size_t)batch * m.cols, ny = (size_t)batch * m.rows;
+    if (Staging &st = staging(); true) {
+        std::unique_lock<std::mutex> use(st.mutex(), std::try_to_lock);
+        if (use.owns_lock() && st.takes(nx * 2, ny * 4)) {
+            std::memcpy(st.host_in(), x_f16, nx * 2);
+            if (residual) std::memcpy(st.host_out(), residual, ny * 4);
+            hipError_t e = launch_bring(st.mapped_in(), st.device_in(), nx * 2, st.mapped_out(), st.device_residual(), residual ? ny * 4 : 0, c.stream);
+            if (e == hipSuccess) e = run_matvec(m, reinterpret_cast<const uint16_t *>(st.device_in()), batch, reinterpret_cast<float *>(st.mapped_out()),
+                                                residual ? reinterpret_cast<const float *>(st.device_residual()) : nullptr, st.planes(), c.stream);
+            const hipError_t done = hipStreamSynchronize(c.stream);   // whatever was launched: the area is the next call's
+            if (e == hipSuccess) e = done;
+            if (e != hipSuccess) return fail_hip(e, "gemv");
+            std::memcpy(y, st.host_out(), ny * 4);
+            return ESP_OK;
+        }
+    }
     uint16_t *d_x = nullptr;
     float *d_y = nullptr, *d_res = nullptr, *d_ws = nullptr;
     if ((rc = device_alloc(&d_x, nx)) != ESP_OK) return rc;

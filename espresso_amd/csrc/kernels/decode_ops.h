@@ -150,6 +150,7 @@ hipError_t launch_two_token_batch_accept(TwoTokenBatchState *state, int n_seq, c
 hipError_t launch_batch_greedy_feed(const int *head_tokens, int n, int *tokens, int *pos, int *log, int *step, int capacity_steps, hipStream_t s);
 hipError_t launch_two_token_accept(TwoTokenState *state, const int *target_head_tokens, int *log, int log_capacity, const float *hidden_rows,
                                    float *last_hidden, int d, int *draft_tokens, int *draft_pos, const EmbedTarget &draft_embed, hipStream_t s);
+hipError_t launch_bring(const void *from0, void *to0, size_t bytes0, const void *from1, void *to1, size_t bytes1, hipStream_t s);   // mapped host memory to the device, two ranges of whole dwords
 hipError_t launch_copy_rows(const float *src, float *dst, int rows, int d, hipStream_t s);
 
 }  // namespace esp

@@ -1166,6 +1166,19 @@ __global__ void copy_rows_kernel(const float *src, float *dst, int d) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < d; i += gridDim.x * blockDim.x) dst[(size_t)m * d + i] = src[(size_t)m * d + i];
 }
 
+// Two ranges of whole dwords from pinned host memory, at sixteen-byte boundaries: everything is requested at once, a trip over the bus costs about 2 us whatever its length.
+__global__ __launch_bounds__(256) void bring_kernel(const uint8_t *from0, uint8_t *to0, uint32_t bytes0, const uint8_t *from1, uint8_t *to1, uint32_t bytes1) {
+    const uint32_t pieces0 = (bytes0 + 15) / 16, i = blockIdx.x * 256 + threadIdx.x;
+    const bool first = i < pieces0;
+    const uint32_t at = (first ? i : i - pieces0) * 16, bytes = first ? bytes0 : bytes1;
+    if (at >= bytes) return;
+    const uint8_t *from = (first ? from0 : from1) + at;
+    uint8_t *to = (first ? to0 : to1) + at;
+    if (at + 16 <= bytes) *reinterpret_cast<uint4 *>(to) = *reinterpret_cast<const uint4 *>(from);
+    else
+        for (uint32_t b = 0; at + b < bytes; b += 4) *reinterpret_cast<uint32_t *>(to + b) = *reinterpret_cast<const uint32_t *>(from + b);
+}
+
 // Rows 0 and 1 of `hidden` = embedding rows of the two tokens (every thread of a 256-thread workgroup calls this).
 __device__ __forceinline__ void embed_two_rows(const EmbedTarget &e, int t0, int t1) {
     if (e.keep_row1) {
@@ -1576,6 +1589,14 @@ hipError_t launch_greedy_feed(const int *next_token, int seq, int *visible, int 
 
 hipError_t launch_set_ints(int *dst0, int v0, int *dst1, int v1, hipStream_t s) {
     hipLaunchKernelGGL(set_ints_kernel, dim3(1), dim3(64), 0, s, dst0, v0, dst1, v1);
+    return hipGetLastError();
+}
+
+hipError_t launch_bring(const void *from0, void *to0, size_t bytes0, const void *from1, void *to1, size_t bytes1, hipStream_t s) {
+    if (bytes0 % 4 != 0 || bytes1 % 4 != 0 || bytes0 + bytes1 == 0 || bytes0 + bytes1 >= (1u << 31)) return hipErrorInvalidValue;
+    const unsigned pieces = (unsigned)((bytes0 + 15) / 16 + (bytes1 + 15) / 16);
+    hipLaunchKernelGGL(bring_kernel, dim3((pieces + 255) / 256), dim3(256), 0, s, static_cast<const uint8_t *>(from0), static_cast<uint8_t *>(to0), (uint32_t)bytes0,
+                       static_cast<const uint8_t *>(from1), static_cast<uint8_t *>(to1), (uint32_t)bytes1);
     return hipGetLastError();
 }
 

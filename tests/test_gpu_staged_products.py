@@ -1,0 +1,62 @@
+"""Single products through the staging area that all matrix handles share: with a residual and without, the largest that fit and the first that do not, several threads at once, handles that come and go."""
+import threading
+
+import numpy as np
+import pytest
+
+import espresso_amd._lib as lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import espresso_amd.ops as o
+    o.init()
+    yield o
+
+
+def matrix(ops, rows, cols, seed):
+    w = np.random.default_rng(seed).normal(0, 0.02, (rows, cols)).astype(np.float16)
+    return ops.Matrix(lib.FORMAT_F16, w.view(np.uint8), rows, cols), w.astype(np.float64)
+
+
+def check(m, w, batch, seed, residual):
+    rng = np.random.default_rng(seed)
+    x = rng.normal(0, 1, (batch, w.shape[1])).astype(np.float16)
+    r = rng.normal(0, 1, (batch, w.shape[0])).astype(np.float32) if residual else None
+    want = x.astype(np.float64) @ w.T + (0 if r is None else r)
+    # exact products, fp32 sums in some order: one rounding per addition, relative to the sum of the magnitudes
+    bound = (w.shape[1] + 16) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(want) + 1)
+    assert (np.abs(m.gemv(x, r) - want) <= bound).all(), (batch, residual)
+
+
+# 1 MiB of activations is 1024 rows of 512 columns, 4 MiB of results 1024 rows of 1024
+@pytest.mark.parametrize("rows,cols,batches", [(24, 8, (1, 2, 5)), (70, 512, (1, 3, 1024, 1025)), (1024, 64, (2, 1024, 1025)), (1023, 72, (7,))])
+def test_every_size_takes_its_way(ops, rows, cols, batches):
+    m, w = matrix(ops, rows, cols, rows)
+    for batch in batches:
+        for residual in (False, True):
+            check(m, w, batch, batch, residual)
+    m.close()
+
+
+def test_threads_and_handles(ops):
+    failures = []
+
+    def work(seed):
+        try:
+            for i in range(12):
+                m, w = matrix(ops, 64 + 16 * seed, 256, seed)
+                for batch in (1, 2, 6, 40):
+                    check(m, w, batch, 100 * seed + i, batch % 2 == 0)
+                m.close()
+        except BaseException as e:   # noqa: BLE001
+            failures.append(e)
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
