@@ -316,11 +316,20 @@ bool span_attention_supported(int n_head, int n_kv_head, int head_dim) {
 hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, bool kv_f16, hipStream_t s) {
     if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
-    // Wavefronts per workgroup: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
-    // 512 rows of 24 heads get four, 241 rows of them eight, 93 rows of 32 heads eight (fp16: 58 us behind 1024, 44 behind 1536, 15.3 of 64 dims behind 700).
+    // Wavefronts per workgroup, fp32 caches: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
+    // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit; two where a few tiles of keys are over before four have met (128 dims: below ten), and for 128 dims
+    // where three workgroups of two fill the chip; eight where a workgroup of 64 dims has the compute unit to itself and keys for all of them.  One wavefront / two / four / eight, us: 1777 rows of 24 heads
+    // of 128 136 / 109 / 112 / 152, 800 of them 63 / 39 / 36 / 53, 160 16.5 / 12.4 / 13.2 / 14.9, 31 rows behind 500 42 / 23 / 19 / 21.5;  512 rows of 32 heads of 64 behind 1024 71 / 53 / 35 / 42, 93 of
+    // them behind 1500 69 / 38 / 24.3 / 22.6, 1200 60 / 46 / 42 / 64.  (One set a SIMD, the rule before, was up to 1.5 times as slow: 1777 rows of 12 heads of 64 54 us, four sets 37.)
     const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32);
     int sets = 1;
-    while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
+    if (!kv_f16) {
+        while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
+    } else if (a.head_dim == 128) {
+        sets = tiles < 2 ? 1 : tiles < 10 || groups > 3 * (device_compute_units() > 0 ? device_compute_units() : 256) ? 2 : 4;
+    } else {
+        sets = tiles < 2 ? 1 : tiles < 3 ? 2 : tiles >= 24 && groups <= (device_compute_units() > 0 ? device_compute_units() : 256) ? 8 : 4;
+    }
     if (a.head_dim == 128) {
         if (kv_f16) launch_shape<128, true>(a, rows, sets, s);
         else launch_shape<128, false>(a, rows, sets, s);
