@@ -106,6 +106,9 @@ struct GemvParams {
     bool split_x = false, split_out = false;
     // one launch for up to sixteen rows of fp16 activations given (gemv_takes_sixteen_rows), every epilogue but the arg-max
     bool sixteen_rows = false;
+    float *workspace = nullptr;       // with sixteen_rows, optional, both or neither: shares of K may be left as planes [shares][batch][rows], and their number in *deferred_splits (1: done)
+    size_t workspace_floats = 0;
+    int *deferred_splits = nullptr;
     // measurement only: device buffer of four wall-clock stamps (100 MHz) per wavefront of the launch, room for stamp_capacity
     // wavefronts (matrix-core Q4_K kernel, fp16 activations given, one or two rows)
     unsigned long long *stamps = nullptr;

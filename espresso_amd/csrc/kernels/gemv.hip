@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "../common.h"
+#include "batch_gemv.h"
 #include "block_gemm.h"
 #include "wide_gemm.h"
 #include "layer_ops.h"
@@ -2379,9 +2380,7 @@ hipError_t try_q40_wide(const KernelArgs &a, int batch, hipStream_t stream, bool
 
 inline bool q40_mfma_width(int cols) { return cols == 2048 || cols == 3072 || cols == 4096 || cols == 8192 || cols == 14336; }
 
-// Up to sixteen rows, every epilogue but the arg-max: bound by the weights' tiled copies.  A batch of sixteen sequences on the 8B model spends
-// 82 us per layer here (gate|up 24.6 us against 12 for the bytes alone) and 135 us as fp16-operand tile products of 64 columns with K
-// splits and their reductions, whose weights are rounded to fp16 on top (logits 4.2e-4 -> 3.6e-4 off the exact ones).
+// Up to sixteen rows, every epilogue but the arg-max: Q4_0, and Q4_K matrices of more columns than batch_gemv.hip takes without shares of K.
 bool wide16_width(int format, int cols) {
     return format == FMT_Q4_K ? cols == 4096 || cols == 14336 || q4k_registry_width(cols) : format == FMT_Q4_0 && q40_mfma_width(cols);
 }
@@ -2396,10 +2395,6 @@ hipError_t launch_wide16(const KernelArgs &a, int format, int batch, hipStream_t
     bool launched = false;
     hipError_t e = hipErrorInvalidValue;
     if (format == FMT_Q4_K) {
-        if (a.cols == 1024) e = launch_wide16_cols<1024, false>(a, batch, stream, &launched);
-        if (a.cols == 2048) e = launch_wide16_cols<2048, false>(a, batch, stream, &launched);
-        if (a.cols == 3072) e = launch_wide16_cols<3072, false>(a, batch, stream, &launched);
-        if (a.cols == 4096) e = launch_wide16_cols<4096, false>(a, batch, stream, &launched);
         if (a.cols == 8192) e = launch_wide16_cols<8192, false>(a, batch, stream, &launched);
         if (a.cols == 14336) e = launch_wide16_cols<14336, false>(a, batch, stream, &launched);
     } else {
@@ -2822,6 +2817,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "q4k_wide") { g_q4k_wide_mode = value; return true; }
     if (k == "short_blocks") { g_short_blocks.store(value != 0); return true; }
     if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
+    if (k == "batch_gemv_form") { batch_gemv_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
     if (k == "dense_gemm_form") { dense_gemm_set_form(value); return true; }
     if (k == "wide_gemm_form") { wide_gemm_set_form(value); return true; }
@@ -2912,6 +2908,8 @@ hipError_t launch_gemv(const GemvParams &p, hipStream_t stream) {
 
     if (p.sixteen_rows) {
         if (!gemv_takes_sixteen_rows(w, p.batch) || !p.x || p.norm_x || p.merge_partials || p.split_x || p.split_out || p.epilogue == EPI_ARGMAX) return hipErrorInvalidValue;
+        if (p.deferred_splits) *p.deferred_splits = 1;
+        if (const BatchGemvForm f = batch_gemv_form(p); f.blocks) return launch_batch_gemv(p, f, stream);
         KernelArgs a{};
         a.tiled = w.tiled; a.qs_row_bytes = w.qs_row_bytes; a.rows = w.rows; a.cols = w.cols; a.x = p.x; a.y = p.y; a.residual = p.residual;
         a.out_f16 = p.out_f16; a.qkv = p.qkv; a.epilogue = p.epilogue;

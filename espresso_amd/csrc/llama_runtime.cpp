@@ -753,10 +753,18 @@ int LlamaRuntime::enqueue_layers_sixteen(int rows) {
     hipStream_t s = context().stream;
     const int d = c_.d_model, kd = c_.kv_dim();
     const bool kv16 = c_.kv_format == FMT_F16;
-    for (Layer &L : layers_) {
+    // the norm behind a projection with a residual, which may have left shares of K as planes
+    auto norm = [&](const float *w, int splits) -> hipError_t {
+        if (splits > 1) return launch_rmsnorm_reduce(gemm_workspace_, splits, (size_t)rows * d, hidden_, hidden_, w, c_.norm_eps, rows, d, xn_, s);
+        return launch_rmsnorm(hidden_, w, c_.norm_eps, rows, d, xn_, nullptr, s);
+    };
+    const bool planes = rmsnorm_reduce_supported(d);
+    ESP_HIP_TRY(norm(layers_.front().rms_att, 1));
+    for (size_t li = 0; li < layers_.size(); li++) {
+        Layer &L = layers_[li];
+        int splits = 1;
         GemvParams g;
         g.batch = rows; g.sixteen_rows = true;
-        ESP_HIP_TRY(launch_rmsnorm(hidden_, L.rms_att, c_.norm_eps, rows, d, xn_, nullptr, s));
         g.w = L.wqkv; g.x = xn_; g.epilogue = EPI_QKV_ROPE;
         g.qkv.n_head = c_.n_head; g.qkv.n_kv_head = c_.n_kv_head; g.qkv.head_dim = c_.head_dim; g.qkv.max_seq = c_.max_seq;
         g.qkv.rope_cos = rope_cos_; g.qkv.rope_sin = rope_sin_; g.qkv.pos = d_pos_; g.qkv.seq = d_seq_;
@@ -769,12 +777,16 @@ int LlamaRuntime::enqueue_layers_sixteen(int rows) {
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_; aa.head_partials = attn_scratch_;
         ESP_HIP_TRY(launch_attention(aa, rows, kv16, s));
         g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL;
+        g.workspace = planes ? gemm_workspace_ : nullptr; g.workspace_floats = gemm_workspace_floats_; g.deferred_splits = planes ? &splits : nullptr;
         ESP_HIP_TRY(launch_gemv(g, s));
-        ESP_HIP_TRY(launch_rmsnorm(hidden_, L.rms_ffn, c_.norm_eps, rows, d, xn_, nullptr, s));
+        ESP_HIP_TRY(norm(L.rms_ffn, splits));
         g.w = L.w13; g.x = xn_; g.y = nullptr; g.residual = nullptr; g.out_f16 = act_; g.epilogue = EPI_SWIGLU_F16;
         ESP_HIP_TRY(launch_gemv(g, s));
         g.w = L.w2; g.x = act_; g.out_f16 = nullptr; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL;
+        splits = 1;
         ESP_HIP_TRY(launch_gemv(g, s));
+        const bool last = li + 1 == layers_.size();   // (behind the last layer only for the sum: the head norms its rows itself)
+        if (!last || splits > 1) ESP_HIP_TRY(norm(last ? final_norm_ : layers_[li + 1].rms_att, splits));
     }
     return ESP_OK;
 }
