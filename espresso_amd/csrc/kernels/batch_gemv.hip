@@ -34,8 +34,17 @@ struct BatchArgs {
 
 struct Tile { uint4 hdr, q0, q1; };
 
+// Where a row's keys and values go, and the RoPE factors of a pair: requested before the sums meet.
+struct Place { int pos, seq; float c, s; };
+__device__ __forceinline__ void rope_factors(const BatchArgs &a, int r0, Place &e) {
+    const QkvEpilogue &q = a.qkv;
+    const int half = q.head_dim / 2, ad = q.n_head * q.head_dim, kd = q.n_kv_head * q.head_dim, j = r0 < ad + kd ? (r0 < ad ? r0 : r0 - ad) / 2 % half : 0;
+    e.c = q.rope_cos[(size_t)e.pos * half + j];
+    e.s = q.rope_sin[(size_t)e.pos * half + j];
+}
+
 // rows r0, r0 + 1 of activation row b
-__device__ __forceinline__ void finish_pair(const BatchArgs &a, int b, int r0, float v0, float v1) {
+__device__ __forceinline__ void finish_pair(const BatchArgs &a, int b, int r0, float v0, float v1, const Place &e) {
     if (r0 + 1 >= a.N) return;
     if (a.epilogue == EPI_SWIGLU_F16) {   // (gate, up): silu_tanh(gate) * up (RealModelInferenceEngine.swift:6825-6827, :6337)
         const float hg = __fmul_rn(0.5f, v0);
@@ -44,8 +53,8 @@ __device__ __forceinline__ void finish_pair(const BatchArgs &a, int b, int r0, f
     }
     // q and k as RoPE pairs (j, j + half), v in natural order (:6745-6772, :6297-6300)
     const QkvEpilogue &q = a.qkv;
-    const int half = q.head_dim / 2, ad = q.n_head * q.head_dim, kd = q.n_kv_head * q.head_dim, pos = q.pos[b];
-    const size_t base = (size_t)q.seq[b] * q.cache_seq_stride + (size_t)pos * kd;
+    const int half = q.head_dim / 2, ad = q.n_head * q.head_dim, kd = q.n_kv_head * q.head_dim;
+    const size_t base = (size_t)e.seq * q.cache_seq_stride + (size_t)e.pos * kd;
     auto keep = [&](void *cache, size_t at, float v) {
         if (q.kv_f16) reinterpret_cast<uint16_t *>(cache)[at] = __builtin_bit_cast(uint16_t, (_Float16)v);
         else reinterpret_cast<float *>(cache)[at] = v;
@@ -57,8 +66,7 @@ __device__ __forceinline__ void finish_pair(const BatchArgs &a, int b, int r0, f
     }
     const bool is_q = r0 < ad;
     const int pr = (is_q ? r0 : r0 - ad) / 2, h = pr / half, j = pr - h * half;
-    const float c = q.rope_cos[(size_t)pos * half + j], s = q.rope_sin[(size_t)pos * half + j];
-    const float o0 = __fsub_rn(__fmul_rn(v0, c), __fmul_rn(v1, s)), o1 = __fadd_rn(__fmul_rn(v0, s), __fmul_rn(v1, c));
+    const float o0 = __fsub_rn(__fmul_rn(v0, e.c), __fmul_rn(v1, e.s)), o1 = __fadd_rn(__fmul_rn(v0, e.s), __fmul_rn(v1, e.c));
     if (is_q) {
         float *dst = q.q_out + (size_t)b * ad + (size_t)h * q.head_dim + j;
         dst[0] = o0;
@@ -100,6 +108,18 @@ __global__ __launch_bounds__(1024) void batch_gemv_kernel(const uint8_t *tiled, 
 #pragma unroll
     for (int i = 0; i < DEPTH; i++) load(ring[i], i);
     __builtin_amdgcn_sched_barrier(0);
+    // a pair's lanes finish activation rows 4 g + 2 k + n % 2
+    const bool odd = n & 1;
+    Place place[2] = {};
+    auto row_of = [&](int k) { return 4 * g + 2 * k + (odd ? 1 : 0); };
+    if (a.epilogue == EPI_QKV_ROPE) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int b = row_of(k) < batch ? row_of(k) : batch - 1;
+            place[k].pos = a.qkv.pos[b];
+            place[k].seq = a.qkv.seq[b];
+        }
+    }
     // to fragments: lane (i = n, g) has chunk g of row i, fours in the order in which nibbles unpack (0, 2, 1, 3); nobody else uses this stretch, and a wavefront's LDS operations keep their order
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -157,6 +177,10 @@ __global__ __launch_bounds__(1024) void batch_gemv_kernel(const uint8_t *tiled, 
         if (i + DEPTH < BLOCKS) load(ring[i % DEPTH], i + DEPTH);
         __builtin_amdgcn_sched_barrier(0);
     }
+    if (a.epilogue == EPI_QKV_ROPE) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) rope_factors(a, (rb0 + wave) * 16 + (n & ~1) < N ? (rb0 + wave) * 16 + (n & ~1) : 0, place[k]);
+    }
     __syncthreads();
     // lane (n, g) holds weight row n of its block for activation rows 4 g .. 4 g + 3
     for (int i = wave; i < BLOCKS; i += waves) {
@@ -169,15 +193,14 @@ __global__ __launch_bounds__(1024) void batch_gemv_kernel(const uint8_t *tiled, 
         if (rb >= row_blocks) return;
         const float out[4] = {t.x, t.y, t.z, t.w};
         if (a.epilogue == EPI_SWIGLU_F16 || a.epilogue == EPI_QKV_ROPE) {
-            // rows n and n + 1 (n even) are a pair: the even lane finishes activation rows 4 g and 4 g + 2, the odd lane the others
+            // rows n and n + 1 (n even) are a pair
             float other[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) other[r] = dpp_term<0xB1, 0xF>(out[r]);   // the neighbouring lane's row
-            const bool odd = n & 1;
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                const int b = 4 * g + 2 * k + (odd ? 1 : 0);
-                if (b < batch) finish_pair(a, b, row & ~1, odd ? other[2 * k + 1] : out[2 * k], odd ? out[2 * k + 1] : other[2 * k]);
+                if (i != wave && a.epilogue == EPI_QKV_ROPE) rope_factors(a, (row & ~1) < N ? row & ~1 : 0, place[k]);
+                if (row_of(k) < batch) finish_pair(a, row_of(k), row & ~1, odd ? other[2 * k + 1] : out[2 * k], odd ? out[2 * k + 1] : other[2 * k], place[k]);
             }
             continue;
         }

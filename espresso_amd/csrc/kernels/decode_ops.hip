@@ -14,10 +14,27 @@ namespace {
 
 constexpr int kBlock = 256;
 
+// DPP row operations and exchanges of half and quarter wavefronts: no trip through LDS, which a shuffle is (some 100 cycles a step).
+template <int CTRL>
+__device__ __forceinline__ float dpp_get(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
+}
+// x of lane ^ OFF (8, 16 or 32) plus the lane's own
+template <int OFF>
+__device__ __forceinline__ float add_across(float x) {
+    static_assert(OFF == 8 || OFF == 16 || OFF == 32, "rows of sixteen lanes and their halves");
+    if constexpr (OFF == 8) return x + dpp_get<0x128>(x);   // row_ror:8
+    const uint32_t b = __builtin_bit_cast(uint32_t, x);
+    const auto p = OFF == 16 ? __builtin_amdgcn_permlane16_swap(b, b, false, false) : __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return __builtin_bit_cast(float, (uint32_t)p[0]) + __builtin_bit_cast(float, (uint32_t)p[1]);
+}
 __device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v += dpp_get<0xB1>(v);     // quad_perm [1,0,3,2]
+    v += dpp_get<0x4E>(v);     // quad_perm [2,3,0,1]
+    v += dpp_get<0x141>(v);    // row_half_mirror
+    v = add_across<8>(v);
+    v = add_across<16>(v);
+    return add_across<32>(v);
 }
 __device__ __forceinline__ float wave_max_f(float v) {
 #pragma unroll
@@ -46,12 +63,7 @@ __device__ __forceinline__ float block_max(float v, float *scratch) {
     return t;
 }
 
-// DPP row operations (no LDS traffic).  group_sum<N>: sum over aligned groups of N lanes (N = 8 or 16),
-// result in every lane of the group.
-template <int CTRL>
-__device__ __forceinline__ float dpp_get(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
-}
+// group_sum<N>: sum over aligned groups of N lanes (N = 8 or 16), result in every lane of the group.
 template <int N>
 __device__ __forceinline__ float group_sum(float v) {
     v += dpp_get<0xB1>(v);                 // quad_perm [1,0,3,2]
@@ -86,13 +98,15 @@ __global__ void embed_kernel(const void *table, int table_is_f16, const int *tok
 // its chain of trips to memory: every load of the row (and of its partial sums, eight at a time) is requested before the first use.
 // Threads beyond the row load its last element again and drop it: a guarded load becomes a branch that waits for its own trip
 // (93 rows of 2048: 4.7 -> 3.9 us, with 4 partial sums 8.7 -> 5.6 us; 16 rows of 4096 5.5 -> 5.4).
-template <int VEC>
+// Few rows take 1024 threads: the chip is idle anyway, and a thread's part of the row's squares is a quarter as long (16 rows of 4096 5.0 -> 4.6 us, behind four planes 6.3 -> 4.9).
+constexpr int kFewRows = 64, kManyThreads = 1024;
+template <int VEC, int THREADS>
 struct RowLoads {
     float4 v[VEC], g[VEC];
     __device__ __forceinline__ void request(const float4 *x4, const float4 *w4, int n4) {
 #pragma unroll
         for (int k = 0; k < VEC; k++) {
-            const int i = threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1;
+            const int i = threadIdx.x + k * THREADS < n4 ? threadIdx.x + k * THREADS : n4 - 1;
             v[k] = x4[i];
             g[k] = w4[i];
         }
@@ -101,13 +115,13 @@ struct RowLoads {
         float s = 0.0f;
 #pragma unroll
         for (int k = 0; k < VEC; k++) {
-            if (threadIdx.x + k * kBlock >= n4) v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (threadIdx.x + k * THREADS >= n4) v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
             s += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
         }
         const float inv = 1.0f / sqrtf(block_sum(s, scratch) / (float)d + eps);
 #pragma unroll
         for (int k = 0; k < VEC; k++) {
-            const int i = threadIdx.x + k * kBlock;
+            const int i = threadIdx.x + k * THREADS;
             if (i < n4) {
                 uint2 o;
                 o.x = to_half_bits(__fmul_rn(__fmul_rn(v[k].x, inv), g[k].x)) | ((uint32_t)to_half_bits(__fmul_rn(__fmul_rn(v[k].y, inv), g[k].y)) << 16);
@@ -120,14 +134,14 @@ struct RowLoads {
 
 // out[m][i] = fp16( (x[m][i] * inv) * w[i] ),  inv = 1/sqrt(sum x^2 / d + eps)      (:6724-6743)
 // One workgroup per row.  Also clears the row's argmax cell when one is given.  VEC 0: rows wider than 8192 or not whole float4.
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void rmsnorm_kernel(const float *x, const float *w, float eps, int d,
+template <int VEC, int THREADS = kBlock>
+__global__ __launch_bounds__(THREADS) void rmsnorm_kernel(const float *x, const float *w, float eps, int d,
                                                          uint16_t *out_f16, unsigned long long *argmax_cells) {
     __shared__ float scratch[16];
     const int m = blockIdx.x;
     const float *xr = x + (size_t)m * d;
     if constexpr (VEC > 0) {
-        RowLoads<VEC> row;
+        RowLoads<VEC, THREADS> row;
         row.request(reinterpret_cast<const float4 *>(xr), reinterpret_cast<const float4 *>(w), d / 4);
         row.normalize(d / 4, d, eps, scratch, reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d));
     } else {
@@ -209,26 +223,26 @@ __global__ void qkv_post_kernel(QkvPostArgs a) {
 // rmsnorm_kernel for a row whose values are still split-K partial sums of a GEMM: x = (residual +) partial[0] + partial[1]
 // + ... in split order (the sum gemm_reduce_kernel forms), written to y, then normalised as above.  One workgroup per row,
 // d a multiple of four and at most 8192.
-template <int VEC>
-__global__ __launch_bounds__(kBlock) void rmsnorm_reduce_kernel(const float *partial, int splits, size_t plane, const float *residual, float *y,
+template <int VEC, int THREADS = kBlock>
+__global__ __launch_bounds__(THREADS) void rmsnorm_reduce_kernel(const float *partial, int splits, size_t plane, const float *residual, float *y,
                                                                 const float *w, float eps, int d, uint16_t *out_f16) {
     __shared__ float scratch[16];
     const int m = blockIdx.x, n4 = d / 4;
     constexpr int AT_ONCE = VEC >= 8 ? 2 : 8 / VEC;   // planes requested together
     const size_t row4 = (size_t)m * n4, plane4 = plane / 4;
-    RowLoads<VEC> row;
+    RowLoads<VEC, THREADS> row;
     row.request(reinterpret_cast<const float4 *>(partial) + row4, reinterpret_cast<const float4 *>(w), n4);
     float4 r[VEC];
     const float4 *r4 = reinterpret_cast<const float4 *>(residual ? residual : partial) + row4;
 #pragma unroll
-    for (int k = 0; k < VEC; k++) r[k] = r4[threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1];
+    for (int k = 0; k < VEC; k++) r[k] = r4[threadIdx.x + k * THREADS < n4 ? threadIdx.x + k * THREADS : n4 - 1];
     for (int sp = 1; sp < splits; sp += AT_ONCE) {
         float4 t[AT_ONCE][VEC];
 #pragma unroll
         for (int q = 0; q < AT_ONCE; q++) {
             const float4 *p4 = reinterpret_cast<const float4 *>(partial) + (sp + q < splits ? sp + q : splits - 1) * plane4 + row4;
 #pragma unroll
-            for (int k = 0; k < VEC; k++) t[q][k] = p4[threadIdx.x + k * kBlock < n4 ? threadIdx.x + k * kBlock : n4 - 1];
+            for (int k = 0; k < VEC; k++) t[q][k] = p4[threadIdx.x + k * THREADS < n4 ? threadIdx.x + k * THREADS : n4 - 1];
         }
 #pragma unroll
         for (int q = 0; q < AT_ONCE; q++) {
@@ -240,7 +254,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_reduce_kernel(const float *par
 #pragma unroll
     for (int k = 0; k < VEC; k++) {
         if (residual) { row.v[k].x = r[k].x + row.v[k].x; row.v[k].y = r[k].y + row.v[k].y; row.v[k].z = r[k].z + row.v[k].z; row.v[k].w = r[k].w + row.v[k].w; }
-        const int i = threadIdx.x + k * kBlock;
+        const int i = threadIdx.x + k * THREADS;
         if (i < n4) reinterpret_cast<float4 *>(y)[row4 + i] = row.v[k];
     }
     row.normalize(n4, d, eps, scratch, reinterpret_cast<uint2 *>(out_f16 + (size_t)m * d));
@@ -510,6 +524,7 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
     static_assert(VP >= 1 && 32 * (HD / 8) % THREADS == 0, "value tile divides over a set of wavefronts");
     static_assert(KP == 1 || KP == 2, "one or two sets");
     __shared__ _Float16 vt_all[KP][2][HD * LDV];
+    asm volatile("" ::"s"(a.tiles), "s"(a.pos), "s"(a.seq), "s"(a.q), "s"(a.k_cache), "s"(a.v_cache));   // fetched together, ahead of the branch
     const int2 tile = a.tiles ? a.tiles[blockIdx.y] : int2{(int)blockIdx.y * QT, rows - 1 - (int)blockIdx.y * QT};
     const int kvh = blockIdx.x, m0 = tile.x;
     const int phase = KP == 1 ? 0 : (int)threadIdx.x / THREADS;
@@ -762,7 +777,8 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
 // that consumes the context merges the splits while it stages its input, so no merge launch follows.
 // Workgroups x, x + kvHeads, ... serve the query heads of KV head x: with eight KV heads the group shares
 // one L2, which then reads K and V from memory once.
-template <int HD, bool KV_F16, int WAVES, int U>
+// SPLITS 1: the workgroup has the whole prefix, and head_partials is the context as fp16 rows.
+template <int HD, bool KV_F16, int WAVES, int U, int SPLITS = kAttentionHeadSplits>
 __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const float *q_rows, const void *k_cache, const void *v_cache, const int *pos,
                                                                        const int *seq, float *head_partials, unsigned cache_seq_stride, unsigned heads) {
     // Fourteen 32-bit words of scalar arguments (heads = query heads | key/value heads << 16): all of them are
@@ -777,7 +793,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
     const int group = a.n_head / a.n_kv_head;
     const int kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head, m = blockIdx.y;
     const int split = blockIdx.z;
-    constexpr int splits = kAttentionHeadSplits;
+    constexpr int splits = SPLITS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // both row descriptors are fetched in one round trip, before anything branches on the first
     const int row_pos = a.pos[m], row_seq = a.seq[m];
@@ -858,12 +874,13 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
     }
     // ---- the wavefront's token slots share one m: their sums and accumulators add up across the lanes that differ in the slot
     // index only, and the wavefront publishes one state ----
+    auto across = [](float v) {
+        if constexpr (LPT == 8) v = add_across<8>(v);
+        return add_across<32>(add_across<16>(v));
+    };
+    l = across(l);
 #pragma unroll
-    for (int off = LPT; off < 64; off <<= 1) {
-        l += __shfl_xor(l, off);
-#pragma unroll
-        for (int i = 0; i < 8; i++) acc[i] += __shfl_xor(acc[i], off);
-    }
+    for (int i = 0; i < 8; i++) acc[i] = across(acc[i]);
     if (slot == 0) {
 #pragma unroll
         for (int i = 0; i < 8; i++) wacc[wave][seg + i] = acc[i];
@@ -882,6 +899,10 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
             const float f = wm[w] == -INFINITY ? 0.0f : expf(wm[w] - M);
             L = __builtin_fmaf(wl[w], f, L);
             A = __builtin_fmaf(wacc[w][dch], f, A);
+        }
+        if constexpr (SPLITS == 1) {
+            reinterpret_cast<uint16_t *>(a.head_partials)[((size_t)m * a.n_head + head) * HD + dch] = to_half_bits(L > 0.0f ? A / L : 0.0f);
+            continue;
         }
         ps[dch] = A;
         if (dch == 0) { ps[HD] = M; ps[HD + 1] = L; }
@@ -1370,6 +1391,11 @@ hipError_t launch_embed(const void *table, bool table_is_f16, const int *tokens,
 
 hipError_t launch_rmsnorm(const float *x, const float *w, float eps, int rows, int d, uint16_t *out_f16,
                           unsigned long long *argmax_cells, hipStream_t s) {
+    if (rows <= kFewRows && d % 4 == 0 && d > 4 * kBlock && d <= 8 * kManyThreads) {
+        auto few = d <= 4 * kManyThreads ? rmsnorm_kernel<1, kManyThreads> : rmsnorm_kernel<2, kManyThreads>;
+        hipLaunchKernelGGL(few, dim3(rows), dim3(kManyThreads), 0, s, x, w, eps, d, out_f16, argmax_cells);
+        return hipGetLastError();
+    }
     const int vec = d % 4 ? 9 : (d / 4 + kBlock - 1) / kBlock;
     auto kernel = vec <= 1 ? rmsnorm_kernel<1> : vec <= 2 ? rmsnorm_kernel<2> : vec <= 4 ? rmsnorm_kernel<4> : vec <= 8 ? rmsnorm_kernel<8> : rmsnorm_kernel<0>;
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, s, x, w, eps, d, out_f16, argmax_cells);
@@ -1414,6 +1440,18 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
         }
     }
     // short contexts and other head groups: the kernel of the single-row step and a merge launch
+    if (by_head && a.max_seq <= 512) {   // the whole prefix in one workgroup: no merge (sixteen sequences of 8B, prefix 60-84 of 512, 6.5 + 4.8 -> 5.5 us)
+        const unsigned heads = (unsigned)a.n_head | ((unsigned)a.n_kv_head << 16);
+        auto launch = [&](auto kernel, int waves) {
+            hipLaunchKernelGGL(kernel, dim3(a.n_head, rows), dim3(waves * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, reinterpret_cast<float *>(a.ctx_f16), (unsigned)a.cache_seq_stride, heads);
+        };
+        if (a.head_dim == 128) {
+            if (kv_f16) launch(attention_partial_kernel<128, true, 8, 4, 1>, 8);
+            else launch(attention_partial_kernel<128, false, 8, 4, 1>, 8);
+        } else if (kv_f16) launch(attention_partial_kernel<64, true, 8, 2, 1>, 8);
+        else launch(attention_partial_kernel<64, false, 8, 2, 1>, 8);
+        return hipGetLastError();
+    }
     if (by_head) {
         const hipError_t e = launch_attention_partials(a, rows, kv_f16, s);
         if (e != hipSuccess) return e;
@@ -1524,6 +1562,11 @@ bool rmsnorm_reduce_supported(int d) { return d % 4 == 0 && d <= 8 * 4 * kBlock;
 hipError_t launch_rmsnorm_reduce(const float *partial, int splits, size_t plane, const float *residual, float *y, const float *w, float eps,
                                  int rows, int d, uint16_t *out_f16, hipStream_t s) {
     if (!rmsnorm_reduce_supported(d) || splits < 1 || plane % 4 != 0) return hipErrorInvalidValue;
+    if (rows <= kFewRows && d > 4 * kBlock) {
+        auto few = d <= 4 * kManyThreads ? rmsnorm_reduce_kernel<1, kManyThreads> : rmsnorm_reduce_kernel<2, kManyThreads>;
+        hipLaunchKernelGGL(few, dim3(rows), dim3(kManyThreads), 0, s, partial, splits, plane, residual, y, w, eps, d, out_f16);
+        return hipGetLastError();
+    }
     const int vec = (d / 4 + kBlock - 1) / kBlock;
     auto kernel = vec <= 1 ? rmsnorm_reduce_kernel<1> : vec <= 2 ? rmsnorm_reduce_kernel<2> : vec <= 4 ? rmsnorm_reduce_kernel<4> : rmsnorm_reduce_kernel<8>;
     hipLaunchKernelGGL(kernel, dim3(rows), dim3(kBlock), 0, s, partial, splits, plane, residual, y, w, eps, d, out_f16);

@@ -64,6 +64,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     const int lane = threadIdx.x & 63, phase = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
     const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head;
     const int y = (int)(gridDim.y - 1 - blockIdx.y);                           // the row tiles with the most keys start first
+    asm volatile("" ::"s"(a.tiles), "s"(a.pos), "s"(a.seq), "s"(a.q), "s"(a.k_cache), "s"(a.v_cache));   // fetched together, ahead of the branch
     const int2 tile = a.tiles ? a.tiles[y] : int2{32 * y, rows - 1 - 32 * y};
     const int m0 = tile.x, last_row = tile.y < 31 ? tile.y : 31;
     const int pos0 = a.pos[m0], t_max = pos0 + last_row, kd = a.n_kv_head * HD;
