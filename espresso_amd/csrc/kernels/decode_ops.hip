@@ -8,6 +8,7 @@
 #include "../common.h"
 #include "attention_rows.h"
 #include "decode_ops.h"
+#include <type_traits>
 
 namespace esp {
 namespace {
@@ -971,24 +972,38 @@ constexpr int kArgmaxBlocks = 128;
 
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
 
+// The best candidate of a workgroup of up to sixteen wavefronts, in every thread; bv and bi: one of each per wavefront.  Inside a wavefront through DPP, as add_across (a tree through LDS took a barrier
+// for each halving, 0.4 us).
 __device__ __forceinline__ void argmax_block_reduce(float &best, int &best_i, float *bv, int *bi) {
-    bv[threadIdx.x] = best;
-    bi[threadIdx.x] = best_i;
+    auto take = [&](float v, int i) { if (better(v, i, best, best_i)) { best = v; best_i = i; } };
+    auto dpp = [&](auto ctrl) {
+        constexpr int CTRL = decltype(ctrl)::value;
+        const float v = dpp_get<CTRL>(best);
+        take(v, __builtin_amdgcn_update_dpp(0, best_i, CTRL, 0xF, 0xF, false));
+    };
+    dpp(std::integral_constant<int, 0xB1>{});
+    dpp(std::integral_constant<int, 0x4E>{});
+    dpp(std::integral_constant<int, 0x141>{});
+    dpp(std::integral_constant<int, 0x128>{});
+    auto swapped = [&](const auto &v, const auto &i) {
+        best = __builtin_bit_cast(float, (uint32_t)v[0]); best_i = (int)i[0];
+        take(__builtin_bit_cast(float, (uint32_t)v[1]), (int)i[1]);
+    };
+    const uint32_t v16 = __builtin_bit_cast(uint32_t, best), i16 = (uint32_t)best_i;
+    swapped(__builtin_amdgcn_permlane16_swap(v16, v16, false, false), __builtin_amdgcn_permlane16_swap(i16, i16, false, false));
+    const uint32_t v32 = __builtin_bit_cast(uint32_t, best), i32 = (uint32_t)best_i;
+    swapped(__builtin_amdgcn_permlane32_swap(v32, v32, false, false), __builtin_amdgcn_permlane32_swap(i32, i32, false, false));
+    const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) { bv[wave] = best; bi[wave] = best_i; }
     __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s && better(bv[threadIdx.x + s], bi[threadIdx.x + s], bv[threadIdx.x], bi[threadIdx.x])) {
-            bv[threadIdx.x] = bv[threadIdx.x + s];
-            bi[threadIdx.x] = bi[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
     best = bv[0];
     best_i = bi[0];
+    for (int w = 1; w < waves; w++) take(bv[w], bi[w]);
 }
 
 __global__ __launch_bounds__(kBlock) void argmax_partial_kernel(const float *logits, int vocab, float *part_value, int *part_index) {
-    __shared__ float bv[kBlock];
-    __shared__ int bi[kBlock];
+    __shared__ float bv[16];
+    __shared__ int bi[16];
     const int m = blockIdx.y, blk = blockIdx.x, nblk = gridDim.x;
     const float *row = logits + (size_t)m * vocab;
     const int per = (vocab + nblk - 1) / nblk;
@@ -1008,8 +1023,8 @@ __global__ __launch_bounds__(kBlock) void argmax_partial_kernel(const float *log
 
 __global__ __launch_bounds__(kBlock) void argmax_final_kernel(const float *part_value, const int *part_index, int nblk,
                                                               int *out_token, float *out_value) {
-    __shared__ float bv[kBlock];
-    __shared__ int bi[kBlock];
+    __shared__ float bv[16];
+    __shared__ int bi[16];
     const int m = blockIdx.x;
     float best = -INFINITY;
     int best_i = 0x7FFFFFFF;
@@ -1116,8 +1131,8 @@ struct GreedyTailArgs {
     int eos;
 };
 __global__ __launch_bounds__(kBlock) void greedy_tail_kernel(GreedyTailArgs a) {
-    __shared__ float bv[kBlock];
-    __shared__ int bi[kBlock];
+    __shared__ float bv[16];
+    __shared__ int bi[16];
     // The loop state the bookkeeping below branches on is requested first, all of it at once: read where it is needed, its five
     // words would be a chain of trips to memory behind the reduction (every replay finds them written by the replay before).
     // (Through pointers the compiler must keep in vector registers: vector loads share a counter with the candidates' loads below and

@@ -1,0 +1,35 @@
+"""Single steps of the layered models at widths around the ring of steps in flight (512 columns each, four or two), vocabularies of more than one round of the head's workgroups, and chains of captured
+greedy steps, against the plain statement."""
+import numpy as np
+import pytest
+
+import espresso_amd.layered as layered
+import layered_util as lu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width,ff,vocab", [(512, 300, 97), (1024, 1500, 9000), (1030, 2100, 333), (2048, 1030, 97), (2050, 4100, 97)])
+@pytest.mark.parametrize("parallel", [True, False])
+def test_steps_at_the_rings_edges(tmp_path, width, ff, vocab, parallel):
+    if parallel:
+        cfg = lu.config([lu.retention(heads=3, dim=48, vdim=72, ff=ff), lu.latent(heads=5, dim=40, ff=ff)], width=width, vocab=vocab)
+    else:
+        cfg = lu.sequential([lu.mamba2(heads=6, vdim=40, state=40, ff=ff), lu.attention(heads=8, dim=32, vdim=40, dims=16, ff=ff)], width=width, vocab=vocab)
+    m = lu.Model(tmp_path, cfg, seed=3, gain=1.5)
+    t = lu.tokens(m.cfg, 6, 3)
+    want = m.logits(t)
+    rt = m.runtime("bf16", max_seq=32)
+    got = lu.feed(rt, t, [1] * 6)
+    assert lu.error(got, want) < lu.limit("bf16")
+    # captured steps: the same tokens as one step at a time
+    rt.reset()
+    rt.prefill(t)
+    chain = [int(x) for x in rt.generate(t, 9)[0]]
+    rt.reset()
+    rt.prefill(t)
+    alone = []
+    for _ in range(9):
+        alone.append(int(np.argmax(rt.logits())))
+        rt.advance(alone[-1])
+    assert chain == alone
