@@ -1040,16 +1040,21 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kMfmaRounds = 8;   // rounds whose partial sums have an LDS slot of their own (KS > 1)
 
-// Sum over the workgroup's WAVES wavefronts, added in wavefront order; `red` holds WAVES floats.
-template <int WAVES>
-__device__ __forceinline__ float workgroup_sum_waves(float v, float *red) {
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float t = red[0];
+// Sums over the workgroup's WAVES wavefronts, added in wavefront order, one barrier for all rows; `red` holds ROWS x WAVES floats.
+template <int WAVES, int ROWS>
+__device__ __forceinline__ void workgroup_sums_waves(float (&v)[ROWS], float *red) {
 #pragma unroll
-    for (int w = 1; w < WAVES; w++) t += red[w];
-    return t;
+    for (int b = 0; b < ROWS; b++) {
+        v[b] = wave_sum(v[b]);
+        if ((threadIdx.x & 63) == 0) red[b * WAVES + (threadIdx.x >> 6)] = v[b];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < ROWS; b++) {
+        v[b] = red[b * WAVES];
+#pragma unroll
+        for (int w = 1; w < WAVES; w++) v[b] += red[b * WAVES + w];
+    }
 }
 
 // Activations of a row (fp16 as given, RMSNorm fused, or attention states merged) into LDS for the matrix-core kernel:
@@ -1061,6 +1066,9 @@ struct MfmaStage {
     static constexpr int GROUPS = IPR * 8, K = (GROUPS + THREADS - 1) / THREADS, cols = IPR * 64, WAVES = THREADS / 64;
     static constexpr int NBX = SPLIT ? 2 * NB : NB;
     static constexpr bool FULL = GROUPS % THREADS == 0;
+    // Partial states of several rows where the threads that a single row leaves idle suffice for the others: all rows on their way at once, one trip to memory instead of one a row
+    // (two rows of 768 x 768 in fp16 with the residual's early request: 6.2 -> 4.5 us in a trace).  Wider rows stay one after the other: twice the registers would cost wavefronts.
+    static constexpr bool ROWS_AT_ONCE = MODE == 2 && NB > 1 && NB * GROUPS <= K * THREADS;
     static_assert(!(Q40 && SPLIT), "split activations: Q4_K only");
     float4 v0[MODE == 1 ? NB : 1][K], v1[MODE == 1 ? NB : 1][K], g0[K], g1[K];
     uint4 v[MODE == 0 ? NBX : 1][K];
@@ -1069,6 +1077,8 @@ struct MfmaStage {
 
     __device__ __forceinline__ int group(int k) const { return FULL || (int)threadIdx.x + k * THREADS < GROUPS ? (int)threadIdx.x + k * THREADS : 0; }
     __device__ __forceinline__ bool mine(int k) const { return FULL || (int)threadIdx.x + k * THREADS < GROUPS; }
+
+    __device__ __forceinline__ int row_item(int k) const { return (int)threadIdx.x + k * THREADS < NB * GROUPS ? (int)threadIdx.x + k * THREADS : 0; }   // ROWS_AT_ONCE
 
     __device__ __forceinline__ void load_merge_row(const KernelArgs &a, int b) {
 #pragma unroll
@@ -1092,7 +1102,12 @@ struct MfmaStage {
                 }
             }
         } else if constexpr (MODE == 2) {
-            load_merge_row(a, 0);
+            if constexpr (ROWS_AT_ONCE) {
+#pragma unroll
+                for (int k = 0; k < K; k++) merge_group_load(a, row_item(k) / GROUPS, row_item(k) % GROUPS, cols, ml[k], a0[k], a1[k]);
+            } else {
+                load_merge_row(a, 0);
+            }
         } else {
 #pragma unroll
             for (int b = 0; b < NBX; b++)
@@ -1102,12 +1117,17 @@ struct MfmaStage {
     }
     __device__ __forceinline__ void finish(const KernelArgs &a, uint4 *xs4, float *xsum, float *red) {
         if constexpr (MODE == 1) {
+            float s[NB];
 #pragma unroll
             for (int b = 0; b < NB; b++) {
-                float s = 0.0f;
+                s[b] = 0.0f;
 #pragma unroll
-                for (int k = 0; k < K; k++) s += sum_squares(v0[b][k], v1[b][k]);
-                const float inv = 1.0f / sqrtf(workgroup_sum_waves<WAVES>(s, red + b * WAVES) / (float)cols + a.norm_eps);
+                for (int k = 0; k < K; k++) s[b] += sum_squares(v0[b][k], v1[b][k]);
+            }
+            workgroup_sums_waves<WAVES>(s, red);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const float inv = 1.0f / sqrtf(s[b] / (float)cols + a.norm_eps);
 #pragma unroll
                 for (int k = 0; k < K; k++) {
                     if (!mine(k)) continue;
@@ -1118,6 +1138,19 @@ struct MfmaStage {
                     } else {
                         q4k_store_group_natural<Q40>(normalized_group(v0[b][k], v1[b][k], g0[k], g1[k], inv), b, group(k), cols, xs4, xsum);
                     }
+                }
+            }
+        } else if constexpr (ROWS_AT_ONCE) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const int b = row_item(k) / GROUPS, g = row_item(k) % GROUPS;
+                if ((int)threadIdx.x + k * THREADS >= NB * GROUPS) continue;
+                if constexpr (SPLIT) {
+                    float c[8];
+                    merge_group_values(ml[k], a0[k], a1[k], c);
+                    q4k_store_split_natural(split_group(c), b, g, cols, xs4, xsum);
+                } else {
+                    q4k_store_group_natural<Q40>(merge_group(ml[k], a0[k], a1[k]), b, g, cols, xs4, xsum);
                 }
             }
         } else if constexpr (MODE == 2) {
@@ -2012,6 +2045,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_mfma_kernel(const uint8_t
         return it;
     };
 
+    // The epilogue's operands early, as in gemv_kernel: these matrices are one round of short steps a workgroup, nothing else hides their trips to memory (two rows of 768 x 2048 in fp16, residual:
+    // 4.3 -> 3.6 us; 2304 x 768, position and RoPE factors: 4.8 -> 4.6).  The Q4_K kernel of 4096 columns measured no gain: its weights' own way is longer.
+    EarlyEpilogue<NB> early;
+    if constexpr (KS > 1) early_positions<NB>(a, early);
     MfmaStage<NB, IPR, THREADS, MODE> stage;
     stage.issue(a);
     constexpr int AHEAD = DEPTH == 2 ? 1 : DEPTH;
@@ -2021,6 +2058,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_mfma_kernel(const uint8_t
     if (tid < 8) zero4[tid] = make_uint4(0, 0, 0, 0);
     stage.finish(a, xs4, xsum, misc);
     __syncthreads();
+    auto pair_of = [&](int rb) { return (rb < row_blocks ? rb : row_blocks - 1) * 8 + ((lane & 15) >> 1); };
+    if constexpr (KS > 1) {
+        if (__builtin_amdgcn_readfirstlane(ks) == 0) early_operands<NB>(a, pair_of(block_of(0)), early);
+    }
 
     // A operand: slot i = lane % 16 carries activation row i % 4 in lane group i / 4 only; group index of (tile step, j, fragment m)
     // = 32 step + 16 j + 4 g + m
@@ -2077,7 +2118,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_mfma_kernel(const uint8_t
         float other[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) other[b] = dpp_term<0xB1, 0xF>(sum[b]);
-        if (lane < 16 && (lane & 1) == 0 && rb < row_blocks) pair_epilogue<NB>(a, rb * 8 + (lane >> 1), sum, other);
+        if (lane < 16 && (lane & 1) == 0 && rb < row_blocks) pair_epilogue<NB, (KS > 1)>(a, rb * 8 + (lane >> 1), sum, other, &early);
     };
 
     for (int round = 0; round < iters; round++) {
@@ -2114,6 +2155,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_mfma_kernel(const uint8_t
         __syncthreads();
         if (ks == 0) {   // the team's shares in wavefront order, then the epilogue
             for (int round = 0; round < iters; round++) {
+                if (round > 0) early_operands<NB>(a, pair_of(block_of(round)), early);
                 float sum[NB];
 #pragma unroll
                 for (int b = 0; b < NB; b++) {

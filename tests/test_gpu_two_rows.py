@@ -1,0 +1,41 @@
+"""Passes of the exact two-token loop on the device where their kernels branch: widths whose two rows of attention states are merged at once (768 and 2048 columns; 4096 row after row), heads that leave
+candidates of one or many workgroups and heads that leave tokens, drafts that are right (the model itself) and wrong (another model)."""
+import numpy as np
+import pytest
+
+import model_util as mu
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ll():
+    import espresso_amd.llama as ll
+    import espresso_amd.ops as ops
+    ops.init()
+    return ll
+
+
+def model(ll, fmt, width, head_dim, vocab, seed):
+    kw = dict(n_layer=2, n_head=width // head_dim, n_kv_head=max(1, width // head_dim // 2), d_model=width, head_dim=head_dim, hidden_dim=768, vocab=vocab, max_seq=96)
+    packed, _ = mu.pack_weights(mu.random_weights(orc.LlamaConfig(**kw), seed, std=0.05), fmt)
+    g = ll.LlamaRuntime(ll.MultiModelConfig(**kw))
+    ll.load_packed_weights(g, packed, fmt)
+    return g
+
+
+@pytest.mark.parametrize("fused_argmax", [True, False])
+@pytest.mark.parametrize("fmt,width,head_dim,vocab", [(orc.FMT_F16, 768, 64, 9000), (orc.FMT_Q8_0, 768, 128, 130), (orc.FMT_F16, 2048, 64, 500), (orc.FMT_Q8_0, 2048, 128, 20000),
+                                                      (orc.FMT_Q8_0, 4096, 128, 300), (orc.FMT_Q4_K, 4096, 128, 300), (orc.FMT_Q4_0, 2048, 64, 500), (orc.FMT_F32, 256, 64, 77)])
+def test_two_token_stream_is_the_greedy_stream(ll, monkeypatch, fmt, width, head_dim, vocab, fused_argmax):
+    monkeypatch.setenv("ESPRESSO_HIP_FUSED_HEAD_ARGMAX", "1" if fused_argmax else "0")   # read when a model is finished
+    g = model(ll, fmt, width, head_dim, vocab, 5)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).tolist()
+    want = g.generate(prompt, 41)[0]
+    for draft in (model(ll, fmt, width, head_dim, vocab, 5), model(ll, orc.FMT_F16, 768, 64, vocab, 8), model(ll, orc.FMT_F32, 64, 16, vocab, 9)):
+        for _ in range(2):   # the second call replays the passes that the first has captured
+            got = ll.generate_two_token(g, draft, prompt, 41)[0]
+            assert got == want
+        draft.close()
+    g.close()
