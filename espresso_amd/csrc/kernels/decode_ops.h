@@ -129,7 +129,14 @@ struct EmbedTarget {
     float *hidden = nullptr;       // [2][d]
     float *keep_row1 = nullptr;    // when set: row 1 of `hidden` (the model's last output) is copied here before the rows are overwritten
 };
-hipError_t launch_two_token_verify_rows(TwoTokenState *state, const int *draft_head_tokens, int *target_tokens, int *target_pos, const EmbedTarget &embed,
+// The tokens of two rows of a head: in `tokens`, or still to be taken from the candidates of its `blocks` workgroups (EPI_ARGMAX) and stored there.
+struct HeadTokens {
+    int *tokens = nullptr;
+    const float *part_value = nullptr;
+    const int *part_index = nullptr;
+    int blocks = 0;
+};
+hipError_t launch_two_token_verify_rows(TwoTokenState *state, const HeadTokens &draft_head, int *target_tokens, int *target_pos, const EmbedTarget &embed,
                                         hipStream_t s);
 // After the target's two rows went through its head: emits one or two tokens into log, keeps the matching hidden row of the
 // target (d floats from hidden_rows into last_hidden), advances the state and writes the draft's two rows of the next pass.
@@ -148,7 +155,7 @@ hipError_t launch_two_token_batch_accept(TwoTokenBatchState *state, int n_seq, c
                                          float *last_hidden, int d, int *draft_tokens, int *draft_pos, hipStream_t s);
 // Greedy step of n sequences: the head's tokens become the next rows at the next positions and go to log[step][n].
 hipError_t launch_batch_greedy_feed(const int *head_tokens, int n, int *tokens, int *pos, int *log, int *step, int capacity_steps, hipStream_t s);
-hipError_t launch_two_token_accept(TwoTokenState *state, const int *target_head_tokens, int *log, int log_capacity, const float *hidden_rows,
+hipError_t launch_two_token_accept(TwoTokenState *state, const HeadTokens &target_head, int *log, int log_capacity, const float *hidden_rows,
                                    float *last_hidden, int d, int *draft_tokens, int *draft_pos, const EmbedTarget &draft_embed, hipStream_t s);
 hipError_t launch_bring(const void *from0, void *to0, size_t bytes0, const void *from1, void *to1, size_t bytes1, hipStream_t s);   // mapped host memory to the device, two ranges of whole dwords
 hipError_t launch_copy_rows(const float *src, float *dst, int rows, int d, hipStream_t s);

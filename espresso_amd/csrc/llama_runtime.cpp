@@ -791,19 +791,33 @@ int LlamaRuntime::enqueue_layers_sixteen(int rows) {
     return ESP_OK;
 }
 
+// The head of one or two rows with its arg-max inside: final RMSNorm in the staging, one candidate per row and workgroup, no logits are written (:8219-8275).
+int LlamaRuntime::run_head_candidates(const float *hidden_rows, int count, int *blocks) {
+    hipStream_t s = context().stream;
+    GemvParams g;
+    g.w = lm_head_; g.norm_x = hidden_rows; g.norm_w = final_norm_; g.norm_eps = c_.norm_eps; g.batch = count; g.epilogue = EPI_ARGMAX;
+    g.argmax_value = argmax_scratch_.part_value; g.argmax_index = argmax_scratch_.part_index; g.argmax_capacity = head_partial_capacity_;
+    g.argmax_blocks = blocks;
+    int rc;
+    if ((rc = time_begin(K_HEAD)) != ESP_OK) return rc;
+    ESP_HIP_TRY(launch_gemv(g, s));
+    return time_end();
+}
+
+int LlamaRuntime::enqueue_device_head_candidates(HeadTokens *head) {
+    *head = HeadTokens{};
+    head->tokens = d_out_tokens_;
+    if (!head_fuses_argmax()) return run_head(hidden_, 2);
+    head->part_value = argmax_scratch_.part_value;
+    head->part_index = argmax_scratch_.part_index;
+    return run_head_candidates(hidden_, 2, &head->blocks);
+}
+
 int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits) {
     hipStream_t s = context().stream;
     if (count <= 2 && !want_logits && head_fuses_argmax()) {
-        // final RMSNorm in the staging, first-max arg-max in the epilogue: no logits are written (:8219-8275)
-        GemvParams g;
-        int blocks = 0;
-        g.w = lm_head_; g.norm_x = hidden_rows; g.norm_w = final_norm_; g.norm_eps = c_.norm_eps; g.batch = count; g.epilogue = EPI_ARGMAX;
-        g.argmax_value = argmax_scratch_.part_value; g.argmax_index = argmax_scratch_.part_index; g.argmax_capacity = head_partial_capacity_;
-        g.argmax_blocks = &blocks;
-        int rc;
-        if ((rc = time_begin(K_HEAD)) != ESP_OK) return rc;
-        ESP_HIP_TRY(launch_gemv(g, s));
-        if ((rc = time_end()) != ESP_OK) return rc;
+        int blocks = 0, rc;
+        if ((rc = run_head_candidates(hidden_rows, count, &blocks)) != ESP_OK) return rc;
         ESP_HIP_TRY(launch_argmax_final(argmax_scratch_, blocks, count, d_out_tokens_, s));
         return ESP_OK;
     }

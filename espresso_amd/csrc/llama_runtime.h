@@ -63,6 +63,7 @@ class LlamaRuntime : public DecoderRuntime {
     size_t weight_bytes_per_token() const override { return weight_bytes_; }
     size_t resident_weight_bytes() const override { return resident_weight_bytes_; }
 
+    int enqueue_device_head_candidates(HeadTokens *head);   // rows 0 and 1, for a kernel that takes the candidates itself
     EmbedTarget device_embed_target() { EmbedTarget e; e.table = embedding_; e.table_is_f16 = embedding_f16_ ? 1 : 0; e.d = c_.d_model; e.hidden = hidden_; return e; }
     DeviceLoopSession &loop_session() { return loop_session_; }
     void release_loop_session();   // destroys the session's graphs and frees its buffers
@@ -85,6 +86,7 @@ class LlamaRuntime : public DecoderRuntime {
     int upload_vector(const HostTensor &t, size_t count, float **out, const char *what);
     // without want_logits one or two rows take the head whose epilogue is the arg-max and store none
     int run_head(const float *hidden_rows, int count, bool want_logits = false) override;
+    int run_head_candidates(const float *hidden_rows, int count, int *blocks);   // head_fuses_argmax() only
     bool head_fuses_argmax() const { return fused_head_argmax_ && gemv_supports_argmax(lm_head_); }
     int enqueue_trunk(int rows, bool embedded = false, float *final_out = nullptr) override;
     int enqueue_greedy_token(int seq) override;

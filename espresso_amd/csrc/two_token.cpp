@@ -20,15 +20,16 @@ int enqueue_two_token_pass(LlamaRuntime &full, LlamaRuntime &draft, TwoTokenStat
     hipStream_t s = context().stream;
     int rc;
     if ((rc = draft.enqueue_device_rows(2, draft_rows_embedded)) != ESP_OK) return rc;
-    if ((rc = draft.enqueue_device_head(2)) != ESP_OK) return rc;
-    // the two small kernels between the models also fetch the embedding rows of the model that runs next: two launches fewer per pass
-    ESP_HIP_TRY(launch_two_token_verify_rows(state, draft.device_head_tokens(), full.device_row_tokens(), full.device_row_positions(),
+    HeadTokens proposed, verified;
+    if ((rc = draft.enqueue_device_head_candidates(&proposed)) != ESP_OK) return rc;
+    // the two small kernels between the models also take the best of the heads' candidates and fetch the embedding rows of the model that runs next: four launches fewer per pass
+    ESP_HIP_TRY(launch_two_token_verify_rows(state, proposed, full.device_row_tokens(), full.device_row_positions(),
                                              full.device_embed_target(), s));
     if ((rc = full.enqueue_device_rows(2, true)) != ESP_OK) return rc;
-    if ((rc = full.enqueue_device_head(2)) != ESP_OK) return rc;
+    if ((rc = full.enqueue_device_head_candidates(&verified)) != ESP_OK) return rc;
     EmbedTarget draft_rows = draft.device_embed_target();
     draft_rows.keep_row1 = draft.device_last_hidden(0);   // the draft's last output row, before the embeddings replace it
-    ESP_HIP_TRY(launch_two_token_accept(state, full.device_head_tokens(), log, log_capacity, full.device_hidden_rows(), full.device_last_hidden(0),
+    ESP_HIP_TRY(launch_two_token_accept(state, verified, log, log_capacity, full.device_hidden_rows(), full.device_last_hidden(0),
                                         full.config().d_model, draft.device_row_tokens(), draft.device_row_positions(), draft_rows, s));
     return ESP_OK;
 }
