@@ -33,3 +33,14 @@ def test_steps_at_the_rings_edges(tmp_path, width, ff, vocab, parallel):
         alone.append(int(np.argmax(rt.logits())))
         rt.advance(alone[-1])
     assert chain == alone
+
+
+# Slices of latent attention merged in one request (32 and fewer of a rank of up to 512) and in several
+@pytest.mark.parametrize("rank,keys", [(64, 1), (64, 33), (512, 65), (576, 40), (960, 1100), (128, 2100)])
+def test_slices_of_latents_merged(tmp_path, rank, keys):
+    m = lu.Model(tmp_path, lu.config([lu.latent(heads=3, dim=40, kv_rank=rank, window=4096, ff=64)], width=96, vocab=61), seed=5, gain=1.5)
+    t = lu.tokens(m.cfg, keys + 2, 7)
+    want = m.logits(t)
+    rt = m.runtime("bf16", max_seq=4096)
+    got = lu.feed(rt, t, [200] * (keys // 200) + ([keys % 200] if keys % 200 else []) + [1])
+    assert lu.error(got[-2:], want[-2:]) < lu.limit("bf16")
