@@ -44,3 +44,14 @@ def test_slices_of_latents_merged(tmp_path, rank, keys):
     rt = m.runtime("bf16", max_seq=4096)
     got = lu.feed(rt, t, [200] * (keys // 200) + ([keys % 200] if keys % 200 else []) + [1])
     assert lu.error(got[-2:], want[-2:]) < lu.limit("bf16")
+
+
+# Groups of query heads whose sums meet together, fewer than a full set of them too, long heads beside eight queries; slices in one request and in several
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,keys", [(4, 4, 16, 24, 1), (6, 3, 32, 40, 33), (3, 1, 64, 128, 300), (10, 2, 40, 72, 70), (7, 1, 136, 16, 290), (8, 1, 480, 320, 40), (16, 2, 1024, 1024, 36)])
+def test_heads_of_a_group_together(tmp_path, heads, kv_heads, dim, vdim, keys):
+    m = lu.Model(tmp_path, lu.sequential([lu.attention(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, dims=16, window=512, ff=64)], width=96, vocab=61), seed=5, gain=1.5)
+    t = lu.tokens(m.cfg, keys + 2, 7)
+    want = m.logits(t)
+    rt = m.runtime("bf16", max_seq=512)
+    got = lu.feed(rt, t, [200] * (keys // 200) + ([keys % 200] if keys % 200 else []) + [1])
+    assert lu.error(got[-2:], want[-2:]) < lu.limit("bf16")
