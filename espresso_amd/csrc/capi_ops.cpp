@@ -234,7 +234,7 @@ int esp_gemv(const ESPMatrix *matrix, const uint16_t *x_f16, int batch, float *y
 
 int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares) {
     if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: null pointer");
-    if (rows <= 0 || rows > 512) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: rows %d", rows);
+    if (rows <= 0 || rows > 2048) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: rows %d", rows);
     int rc = ensure_init();
     if (rc != ESP_OK) return rc;
     Context &c = context();

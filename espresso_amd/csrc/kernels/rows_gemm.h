@@ -5,6 +5,7 @@
 
 namespace esp {
 
+constexpr int kExactRows = 512;   // products that need not round packed weights (GemmParams::unrounded) are exact or not by their rows up to here, and as here beyond
 bool rows_gemm_takes(const GemmParams &p);
 // p.rows rows; y (+ residual), or swiglu_out for a matrix of (gate, up) row pairs.  The workspace is not used.
 hipError_t launch_rows_gemm(const GemmParams &p, hipStream_t stream);

@@ -305,8 +305,8 @@ void rows_gemm_set_mode(int mode) { g_rows_gemm_mode = mode < 0 ? 1 : mode; }
 
 bool rows_gemm_takes(const GemmParams &p) {
     const DeviceMatrix &w = p.w;
-    const int mode = rows_gemm_mode(), rows = p.rows;
-    if (mode == 0 || (mode == 1 && !p.unrounded) || (p.swiglu_out && (w.rows % 2 != 0 || p.residual)) || rows < 1 || w.cols % kStep != 0 || w.qs_row_bytes % 16 != 0) return false;
+    const int mode = rows_gemm_mode();
+    if (mode == 0 || (mode == 1 && !p.unrounded) || (p.swiglu_out && (w.rows % 2 != 0 || p.residual)) || p.rows < 1 || w.cols % kStep != 0 || w.qs_row_bytes % 16 != 0) return false;
     if (w.format == FMT_Q4_K) { if (w.cols % 256 != 0) return false; }
     else if (w.format != FMT_Q4_0 && w.format != FMT_Q8_0 && w.format != FMT_F16) return false;
     if (mode == 2) return true;
@@ -321,7 +321,9 @@ bool rows_gemm_takes(const GemmParams &p) {
     // time; at three rows of the 2048-column Q4_0 and 512 x 256 matrices, five to seven microseconds each way, up to 1.1 times.
     // Up to 32 rows that no next kernel finishes: deeper launches too, while all workgroups are resident at once (8192 x 3072, 8 / 32 rows, with shares of K and their sum -> here: q4_0
     // 10.5 / 11.9 -> 9.2 / 11.1, q8_0 12.4 / 14.1 -> 11.6 / 13.9, q4_k 16 rows 12.6 -> 9.3).
-    const int steps = w.cols / kStep;
+    // Beyond kExactRows the rule is what it is there: a prompt's rows keep the weights that they keep in a block of that length, however long theirs is (30 layers of 576 columns, 1000 / 1777
+    // tokens, rounded -> kept: Q8_0 2660 / 4040 -> 2750 / 4380 us, Q4_0 2220 / 3010 -> 2320 / 3290).
+    const int steps = w.cols / kStep, rows = w.format != FMT_F16 && p.rows > kExactRows ? kExactRows : p.rows;
     const long groups = (long)((w.rows + 31) / 32) * ((rows + 31) / 32);
     if (w.format == FMT_F16) {
         // rounds of one workgroup per compute unit against the kernel of wide_gemm.hip (us, here / there: 3072 x 576, 64 / 96 rows 5.1 / 6.3, 8.3 / 6.4;  576 x 1536, 16 / 200 / 400 rows

@@ -2,11 +2,13 @@
 import numpy as np
 import pytest
 
+import espresso_amd._lib as lib
 import espresso_amd.layered as layered
 import espresso_amd.llama as ll
 import layered_util as lu
 import model_util as mu
 from oracle import oracle as orc
+from test_gpu_block_gemm import check_kept
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +59,19 @@ def test_layered_blocks_past_the_ring(tmp_path, precision, config):
     rt = m.runtime(precision, max_seq=2500)
     for s, portions in enumerate(([2400, 1], [2100, 3, 300, 1], [513, 1700, 2])):
         assert lu.error(lu.feed(rt, t, portions, s), want) < lu.limit(precision), portions
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_0", "q4_k"])
+@pytest.mark.parametrize("rows,cols", [(576, 1536), (960, 576), (576, 576), (768, 768), (2048, 512)])   # smallest-model shapes, the most that is kept (2^20 weights)
+def test_small_products_keep_their_weights_in_long_blocks(fmt, rows, cols):
+    """What a block of 512 rows keeps exact, a longer one does: one row more, between, and the longest block."""
+    import espresso_amd.ops as ops
+    f = lib.FORMAT_NAMES[fmt]
+    cols = (cols + 255) // 256 * 256 if fmt == "q4_k" else cols
+    rows = min(rows, 2 ** 20 // cols // 32 * 32)
+    ops.init()
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    rng = np.random.default_rng(cols)
+    for shares in (False, True):
+        check_kept(m, lambda x, r: m.layer_product(x, r, shares=shares), (512, 513, 1055, 2048), rng)
+    m.close()
