@@ -219,6 +219,7 @@ bool gemv_supports_argmax(const DeviceMatrix &w);
 bool gemv_merges_attention_partials(const DeviceMatrix &w, int batch, int head_dim);
 // kernels/gemm.hip
 hipError_t launch_gemm(const GemmParams &p, hipStream_t stream);
+bool gemm_keeps_weights(const GemmParams &p);   // does launch_gemm multiply with the weights as they are, none rounded to fp16?
 // kernels/dequant.hip — GGUF-layout blocks -> fp32, bit-exact to the block definitions
 hipError_t launch_dequant(int format, const uint8_t *blocks, size_t elems, float *out, hipStream_t stream);
 // GGUF-layout blocks -> DeviceMatrix planes (device to device)

@@ -269,11 +269,12 @@ int DecoderRuntime::append(int seq, const uint32_t *tokens, int count, const int
     };
     if (matrix_prefill_ && block_prefill_pays(count, start) && matrix_prefill_supported()) {
         // blocks of rows through the MFMA kernels (one pass over the weights per block)
-        const int blocks = (count + block_rows_ - 1) / block_rows_, even = ((count + blocks - 1) / blocks + 127) / 128 * 128;   // of one size: a short last block costs as much as half a long one
+        const LastRows last = last_rows(count);
+        const int body = count - last.own_block, blocks = (body + block_rows_ - 1) / block_rows_, even = ((body + blocks - 1) / blocks + 127) / 128 * 128;   // of one size: a short last block costs as much as half a long one
         const int most = even < block_rows_ ? even : block_rows_;
-        for (int off = 0; off < count; off += most) {
-            const int rows = count - off < most ? count - off : most;
-            if ((rc = prefill_block(seq, tokens + off, rows, start + off)) != ESP_OK) return rc;
+        for (int off = 0, rows; off < count; off += rows) {
+            rows = off == body ? count - body : body - off < most ? body - off : most;
+            if ((rc = prefill_block(seq, tokens + off, rows, start + off, off + rows == body ? last.in_block : 0)) != ESP_OK) return rc;
             if (off + rows == count && (rc = keep_row(rows - 1, seq)) != ESP_OK) return rc;
             while (given < want_count && want[given] < off + rows) {
                 int n = 0;

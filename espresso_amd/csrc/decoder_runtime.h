@@ -33,6 +33,7 @@ struct DecoderShape {
     int max_sequences = 1;    // independent sequence slots (KV caches, recurrent states)
 };
 
+struct LastRows { int own_block = 0, in_block = 0; };
 struct PromptSpan { int sequence; const uint32_t *tokens; int count; };   // a whole prompt of an empty sequence
 
 class DecoderRuntime {
@@ -130,13 +131,16 @@ class DecoderRuntime {
     // One greedy choice under capture: head over the sequence's kept state, the token into row 0 and the log, and what
     // enqueue_trunk(1, true) needs of its embedding.
     virtual int enqueue_greedy_token(int seq) = 0;
-    // `rows` tokens at positions base.. of one sequence as one block; their rows end in hidden_.
-    virtual int prefill_block(int seq, const uint32_t *tokens, int rows, int base) = 0;
+    // `rows` tokens at positions base.. of one sequence as one block, the last of them by last_rows; their rows end in hidden_.
+    virtual int prefill_block(int seq, const uint32_t *tokens, int rows, int base, int last) = 0;
     virtual bool matrix_prefill_supported() const = 0;
     // Prompts of one class other than 0 may share a block and come out as in blocks of their own, but for the order of sums.
     virtual int shared_block_class(int count) const { (void)count; return 0; }
     // Prompts of a class, their rows behind each other (up to block_rows_), as one block; the rows end in hidden_.
     virtual int prefill_shared_block(const PromptSpan *spans, int count) { (void)spans; (void)count; return ESP_ERR_UNSUPPORTED; }
+    // The last rows of `count` that a block of so few would compute more exactly than a long one: they go in such a block, or at the end of a long one whose kernels are others for them.  Fewer than
+    // kMinPrefillBlockRows, and fewer than `count`.
+    virtual LastRows last_rows(int count) const { (void)count; return {}; }
     // Whether `count` tokens behind `base` run in blocks rather than in steps (where the layers take blocks at all).
     virtual bool block_prefill_pays(int count, int base) const { (void)base; return count >= kMatrixPrefillMinTokens; }
     virtual int clear_state() = 0;                       // every cache and state of every sequence, enqueued on the stream

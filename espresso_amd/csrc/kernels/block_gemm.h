@@ -10,6 +10,7 @@ bool block_gemm_takes(const GemmParams &p);
 inline bool block_gemm_alone(const GemmParams &p) { return !p.deferred_splits && !p.swiglu_out; }
 // Exact here rather than in the kernel of rows_gemm.hip?
 bool block_gemm_keeps(const GemmParams &p);
+bool block_gemm_exact(const GemmParams &p);   // of a product that runs here
 // Do products of up to `rows` rows that need not round their weights (GemmParams::unrounded) keep them as they are?
 bool block_gemm_exact(const DeviceMatrix &w, int rows);
 // Complete in p.y (+ residual) or p.swiglu_out where *splits is 1; otherwise *splits planes of sums in p.workspace, residual and SiLU left to whoever adds them.

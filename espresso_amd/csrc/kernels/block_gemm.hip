@@ -421,7 +421,7 @@ bool block_gemm_keeps(const GemmParams &p) {
 
 // Few rows keep their weights exact where a format has one scale per block and the steps they stand for do: the same time for Q8_0, 0 to 12 % more for Q4_0 (12 rows; with shares
 // added by the next kernel 2048 x 8192, 4 to 31 rows 7.3 to 7.8 us, in rows_gemm.hip 13 to 17).
-static bool keeps_exact(const GemmParams &p) {
+bool block_gemm_exact(const GemmParams &p) {
     return (p.w.format == FMT_Q8_0 || p.w.format == FMT_Q4_0) && p.unrounded && (p.rows <= 32 || block_gemm_keeps(p));
 }
 
@@ -435,7 +435,7 @@ bool block_gemm_takes(const GemmParams &p) {
 }
 
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {
-    bool exact = keeps_exact(p);
+    bool exact = block_gemm_exact(p);
     Form f = choose_form(p, exact);
     if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
         f.tm = forced / 100; f.nw = forced / 10 % 10;

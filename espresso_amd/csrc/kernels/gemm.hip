@@ -581,6 +581,10 @@ hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *defe
 
 }  // namespace
 
+bool gemm_keeps_weights(const GemmParams &p) {
+    return p.w.format == FMT_F16 || rows_gemm_takes(p) || (p.w.format == FMT_Q4_K ? p.rows <= kRowsMaxRows : block_gemm_takes(p) && block_gemm_exact(p));
+}
+
 hipError_t launch_gemm(const GemmParams &params, hipStream_t stream) {
     GemmParams p = params;
     const DeviceMatrix &w = p.w;

@@ -393,7 +393,7 @@ int LayeredRuntime::enqueue_block_sequential(int rows, int seq, int base, float 
     return ESP_OK;
 }
 
-int LayeredRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int base) {
+int LayeredRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int base, int) {
     const PromptSpan span{seq, tokens, rows};
     const int rc = upload_block_rows(&span, 1, base);
     if (rc != ESP_OK) return rc;

@@ -91,7 +91,7 @@ class LayeredRuntime : public DecoderRuntime {
     int enqueue_trunk(int rows, bool embedded = false, float *final_out = nullptr) override;
     int run_head(const float *hidden_rows, int count, bool want_logits = false) override;
     int enqueue_greedy_token(int seq) override;
-    int prefill_block(int seq, const uint32_t *tokens, int rows, int base) override;
+    int prefill_block(int seq, const uint32_t *tokens, int rows, int base, int last) override;
     bool matrix_prefill_supported() const override { return true; }
     bool block_prefill_pays(int count, int) const override { return count >= min_block_rows_; }
     int clear_state() override;

@@ -510,25 +510,51 @@ bool LlamaRuntime::steps_hold_two_rows() const {
 // `rows` prompt tokens at positions base.. of one sequence: the layer loop of forwardToken (:6221-6347) over
 // a block of rows, every projection as one dequant-fused MFMA GEMM.  Rows of the block see each other's
 // keys and values causally because the whole block's K/V is written before its attention runs.
-int LlamaRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int base) {
+int LlamaRuntime::prefill_block(int seq, const uint32_t *tokens, int rows, int base, int last) {
     const PromptSpan span{seq, tokens, rows};
     const int rc = upload_block_rows(&span, 1, base);
     if (rc != ESP_OK) return rc;
     ESP_HIP_TRY(launch_embed(embedding_, embedding_f16_, d_tokens_, rows, c_.d_model, hidden_, context().stream));
-    return enqueue_layers_matrix(rows, base + rows);
+    return enqueue_layers_matrix(rows, base + rows, last < rows ? last : 0);
+}
+
+// The rows beyond the last multiple of kMinPrefillBlockRows: a block of them alone is more exact where it takes 32-bit attention (fewer than 32 rows) or keeps weights that a long one rounds.  They are
+// the rows whose logits the caller reads, so they stay as exact whatever is in front of them.
+LastRows LlamaRuntime::last_rows(int count) const {
+    const int rows = count % kMinPrefillBlockRows;
+    if (count < kMinPrefillBlockRows || rows == 0) return {};
+    const bool few = rows < kMatrixPrefillMinTokens;
+    if (few && short_split_blocks_supported() && !split_blocks_supported()) return {rows, 0};   // activations are pairs there, which a long block has no place for
+    if (few && finer_short_attention()) return {0, rows};
+    if (split_blocks_supported()) return {};
+    for (const Layer &L : layers_)
+        for (const DeviceMatrix *m : {&L.wqkv, &L.wo, &L.w13, &L.w2})
+            if (rounds_but_for_last(*m, rows, m == &L.w13)) return {0, rows};
+    return {};
+}
+bool LlamaRuntime::rounds_but_for_last(const DeviceMatrix &m, int last, bool gate_up) const {
+    return keeps_weights(m, last, gate_up) && !keeps_weights(m, kMinPrefillBlockRows, gate_up);
+}
+
+// Does a block of `rows` rows multiply with a layer's matrix as it is, no weight rounded to fp16?  (enqueue_layers_matrix asks launch_gemm)
+bool LlamaRuntime::keeps_weights(const DeviceMatrix &m, int rows, bool gate_up) const {
+    GemmParams p;
+    int splits = 1;
+    p.w = m; p.rows = rows; p.unrounded = true;
+    if (gate_up) p.swiglu_out = act_;
+    else p.deferred_splits = &splits;
+    return gemm_keeps_weights(p);
 }
 
 // Products whose arithmetic does not hang on the block's rows: split rows (class 1); fp16 matrices, and packed ones that round their weights at the prompt's own rows already (class 2).  Attention
 // is by prompt, with the kernel that the prompt's own length asks for.
 int LlamaRuntime::shared_block_class(int count) const {
     const bool few = count < kMatrixPrefillMinTokens;
+    if (const LastRows last = last_rows(count); last.own_block || last.in_block) return 0;
     if (few ? short_split_blocks_supported() : split_blocks_supported()) return 1;
     for (const Layer &L : layers_)
-        for (const DeviceMatrix *m : {&L.wqkv, &L.wo, &L.w13, &L.w2}) {
-            GemmParams p;
-            p.w = *m; p.rows = count; p.unrounded = true;
-            if (m->format != FMT_F16 && (m->format == FMT_F32 || count <= 128 || rows_gemm_takes(p) || block_gemm_keeps(p))) return 0;
-        }
+        for (const DeviceMatrix *m : {&L.wqkv, &L.wo, &L.w13, &L.w2})
+            if (m->format != FMT_F16 && (m->format == FMT_F32 || count <= 128 || keeps_weights(*m, count, m == &L.w13))) return 0;
     return few && !short_span_attention_ ? 0 : 2;
 }
 
@@ -560,9 +586,19 @@ int LlamaRuntime::prefill_shared_block(const PromptSpan *spans, int count) {
 
 // Attention of a block: one prompt's rows (block_keys: the keys that the last of them sees), prompts that share it, or (neither) rows that attend alone.  Fewer than 32 rows of a prompt take 32-bit
 // attention, as the steps they stand for.
-int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_keys) {
+int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_keys, int last) {
     hipStream_t s = context().stream;
     const bool kv16 = c_.kv_format == FMT_F16;
+    if (last > 0 && last < kMatrixPrefillMinTokens && finer_short_attention()) {
+        const int ahead = rows - last;
+        const size_t at = (size_t)ahead * c_.attention_dim();
+        ESP_HIP_TRY(launch_attention_prompt(aa, ahead, kv16, s));
+        aa.q += at; aa.pos += ahead; aa.seq += ahead;
+        if (aa.ctx_f16) aa.ctx_f16 += at;
+        if (aa.ctx_hi) { aa.ctx_hi += at; aa.ctx_lo += at; aa.ctx_sums += at / 16; }
+        ESP_HIP_TRY(launch_span_attention(aa, last, block_keys, kv16, s));
+        return ESP_OK;
+    }
     if (shared_.long_tiles + shared_.short_tiles > 0 && (prompt_attention_ || span_attention_)) {
         aa.tiles = d_tiles_; aa.tile_count = shared_.long_tiles;
         if (shared_.long_tiles && prompt_attention_) ESP_HIP_TRY(launch_attention_prompt(aa, shared_.longest, kv16, s));
@@ -639,7 +675,7 @@ bool LlamaRuntime::short_blocks_exact() const {
     return true;
 }
 
-int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
+int LlamaRuntime::enqueue_layers_split(int rows, int block_keys, int last) {
     hipStream_t s = context().stream;
     const bool kv16 = c_.kv_format == FMT_F16;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
@@ -672,7 +708,7 @@ int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_hi = ctx.hi; aa.ctx_lo = ctx.lo; aa.ctx_sums = ctx.sums;
-        { int rc = enqueue_block_attention(aa, rows, block_keys); if (rc != ESP_OK) return rc; }
+        { int rc = enqueue_block_attention(aa, rows, block_keys, last); if (rc != ESP_OK) return rc; }
         g.w = L.wo; g.x = ctx; g.y = hidden_; g.residual = hidden_; splits = 1;
         ESP_HIP_TRY(launch_gemm_split(g, s));
         ESP_HIP_TRY(norm(L.rms_ffn, splits));
@@ -688,22 +724,40 @@ int LlamaRuntime::enqueue_layers_split(int rows, int block_keys) {
     return ESP_OK;
 }
 
-// block_keys: the keys that the last row of a prompt block sees; 0 for rows that are not one sequence at consecutive positions.
-int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
-    if (block_keys && (rows < kMatrixPrefillMinTokens ? short_split_blocks_supported() : split_blocks_supported())) return enqueue_layers_split(rows, block_keys);
+// block_keys: the keys that the last row of a prompt block sees; 0 for rows that are not one sequence at consecutive positions.  last: rows at the end that are as in a block of their own (last_rows).
+int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys, int last) {
+    if (block_keys && (rows < kMatrixPrefillMinTokens ? short_split_blocks_supported() : split_blocks_supported())) return enqueue_layers_split(rows, block_keys, last);
     hipStream_t s = context().stream;
     const int d = c_.d_model, ad = c_.attention_dim(), kd = c_.kv_dim();
     const bool kv16 = c_.kv_format == FMT_F16;
     const size_t cache_seq_stride = (size_t)kd * c_.max_seq;
     GemmParams g;
     g.rows = rows; g.unrounded = true; g.workspace = gemm_workspace_; g.workspace_floats = gemm_workspace_floats_;
+    // A product, in two launches where its last rows keep the weights and the others do not (each complete: no shares of K are left).  Prompts of 22 layers of
+    // 1.1B Q8_0 and 30 of 576 columns in it, rounded like the others / in two launches / in a block of their own, us: 600 tokens 2990 / 3300 / 4250 and 2040 / 2260 / 3360, 520 2820 / 3550 / 3990 and
+    // 1970 / 2070 / 3210.
+    auto product = [&](bool gate_up) -> hipError_t {
+        if (last == 0 || !rounds_but_for_last(g.w, last, gate_up)) return launch_gemm(g, s);
+        GemmParams part = g;
+        part.rows = rows - last;
+        part.deferred_splits = nullptr;
+        const hipError_t e = launch_gemm(part, s);
+        if (e != hipSuccess) return e;
+        const size_t at = (size_t)part.rows * g.w.rows;
+        part.x += (size_t)part.rows * g.w.cols;
+        part.y += at;
+        if (part.residual) part.residual += at;
+        if (part.swiglu_out) part.swiglu_out += at / 2;
+        part.rows = last;
+        return launch_gemm(part, s);
+    };
     // The RMSNorm that follows a projection with a residual reads that projection's result; when the GEMM ran split-K the
     // norm kernel adds the partial sums itself (one launch instead of reduce + norm).
     const bool fuse_norm = rmsnorm_reduce_supported(d);
     auto project_and_norm = [&](const float *norm_w) -> int {   // g is set up for a GEMM into hidden_ with hidden_ as residual
         int splits = 1;
         g.deferred_splits = norm_w && fuse_norm ? &splits : nullptr;
-        ESP_HIP_TRY(launch_gemm(g, s));
+        ESP_HIP_TRY(product(false));
         g.deferred_splits = nullptr;
         if (!norm_w) return ESP_OK;
         if (splits > 1) ESP_HIP_TRY(launch_rmsnorm_reduce(gemm_workspace_, splits, (size_t)rows * d, hidden_, hidden_, norm_w, c_.norm_eps, rows, d, xn_, s));
@@ -715,7 +769,7 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
         Layer &L = layers_[li];
         int qkv_splits = 1;   // split-K partial sums of q|k|v are added by the kernel that applies norm / RoPE and writes the caches
         g.w = L.wqkv; g.x = xn_; g.y = qkv_; g.residual = nullptr; g.deferred_splits = &qkv_splits;
-        ESP_HIP_TRY(launch_gemm(g, s));
+        ESP_HIP_TRY(product(false));
         g.deferred_splits = nullptr;
         QkvPostArgs qa{};
         qa.qkv = qkv_splits > 1 ? gemm_workspace_ : qkv_; qa.splits = qkv_splits; qa.plane = (size_t)rows * (ad + 2 * kd);
@@ -728,11 +782,11 @@ int LlamaRuntime::enqueue_layers_matrix(int rows, int block_keys) {
         aa.q = q_; aa.k_cache = L.k_cache; aa.v_cache = L.v_cache; aa.cache_seq_stride = cache_seq_stride;
         aa.n_head = c_.n_head; aa.n_kv_head = c_.n_kv_head; aa.head_dim = c_.head_dim; aa.max_seq = c_.max_seq;
         aa.pos = d_pos_; aa.seq = d_seq_; aa.ctx_f16 = ctx_; aa.split_scratch = attn_scratch_; aa.head_partials = attn_scratch_;
-        { int rc = enqueue_block_attention(aa, rows, block_keys); if (rc != ESP_OK) return rc; }
+        { int rc = enqueue_block_attention(aa, rows, block_keys, last); if (rc != ESP_OK) return rc; }
         g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_;
         { int rc = project_and_norm(L.rms_ffn); if (rc != ESP_OK) return rc; }
         g.w = L.w13; g.x = xn_; g.y = gu_; g.residual = nullptr; g.swiglu_out = act_;   // SwiGLU in the GEMM's epilogue where it can be
-        ESP_HIP_TRY(launch_gemm(g, s));
+        ESP_HIP_TRY(product(true));
         g.swiglu_out = nullptr;
         g.w = L.w2; g.x = act_; g.y = hidden_; g.residual = hidden_;
         { int rc = project_and_norm(li + 1 < layers_.size() ? layers_[li + 1].rms_att : nullptr); if (rc != ESP_OK) return rc; }

@@ -90,11 +90,15 @@ class LlamaRuntime : public DecoderRuntime {
     bool head_fuses_argmax() const { return fused_head_argmax_ && gemv_supports_argmax(lm_head_); }
     int enqueue_trunk(int rows, bool embedded = false, float *final_out = nullptr) override;
     int enqueue_greedy_token(int seq) override;
-    int prefill_block(int seq, const uint32_t *tokens, int rows, int base) override;
+    int prefill_block(int seq, const uint32_t *tokens, int rows, int base, int last) override;
     int clear_state() override;
     unsigned tuning_epoch() const override { return gemv_tuning_epoch(); }
-    int enqueue_layers_matrix(int rows, int block_keys = 0);
-    int enqueue_block_attention(AttentionArgs aa, int rows, int block_keys);
+    int enqueue_layers_matrix(int rows, int block_keys = 0, int last = 0);
+    int enqueue_block_attention(AttentionArgs aa, int rows, int block_keys, int last);
+    LastRows last_rows(int count) const override;
+    bool rounds_but_for_last(const DeviceMatrix &m, int last, bool gate_up) const;
+    bool finer_short_attention() const { return prompt_attention_ && short_span_attention_; }   // fewer than 32 rows: 32-bit, longer blocks: queries and softmax weights in fp16, or pairs of it
+    bool keeps_weights(const DeviceMatrix &m, int rows, bool gate_up) const;
     int shared_block_class(int count) const override;
     int prefill_shared_block(const PromptSpan *spans, int count) override;
     bool sixteen_rows_supported(int rows) const;
@@ -125,7 +129,7 @@ class LlamaRuntime : public DecoderRuntime {
     // prompt blocks with split activations: the lo planes and sub-block sums beside xn_, ctx_ and act_ (SplitRowsView)
     uint16_t *xn_lo_ = nullptr, *ctx_lo_ = nullptr, *act_lo_ = nullptr, *xn_sums_ = nullptr, *ctx_sums_ = nullptr, *act_sums_ = nullptr;
     bool split_blocks_supported() const;
-    int enqueue_layers_split(int rows, int block_keys);
+    int enqueue_layers_split(int rows, int block_keys, int last = 0);
     size_t weight_bytes_ = 0, resident_weight_bytes_ = 0;
     DeviceLoopSession loop_session_;
     bool fused_head_argmax_ = true;      // ESPRESSO_HIP_FUSED_HEAD_ARGMAX=0: head GEMV stores logits, separate arg-max launches

@@ -8,13 +8,13 @@ import espresso_amd.llama as ll
 import layered_util as lu
 import model_util as mu
 from oracle import oracle as orc
-from test_gpu_block_gemm import check_kept
+from test_gpu_block_gemm import check_kept, rms_off
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("fmt,heads,kv_heads,kv_fp16,count", [
-    (orc.FMT_Q8_0, 4, 2, True, 2049),    # two blocks of 1152 and 897 rows, both attention kernels of long blocks
+    (orc.FMT_Q8_0, 4, 2, True, 2049),    # a block of 2048 rows and one row in a block of its own
     (orc.FMT_Q8_0, 3, 1, False, 1999), (orc.FMT_Q4_0, 3, 1, True, 2304), (orc.FMT_F16, 4, 4, True, 1025),
     (orc.FMT_Q4_K, 4, 1, True, 2111),    # exact products, queries and softmax weights as pairs
     (orc.FMT_Q4_K, 4, 2, False, 1537),
@@ -75,3 +75,56 @@ def test_small_products_keep_their_weights_in_long_blocks(fmt, rows, cols):
     for shares in (False, True):
         check_kept(m, lambda x, r: m.layer_product(x, r, shares=shares), (512, 513, 1055, 2048), rng)
     m.close()
+
+
+# shape, format, caches; prompts and the rows beyond 512 k that are more exact in a block of their own: weights kept at 40 and at 200 rows but not at 512 (gate|up of 4608 x 768, down of
+# 768 x 2304), 32-bit attention of fewer than 32 rows (three query heads to a key/value head have it in every block)
+WIDE = dict(n_head=12, n_kv_head=4, d_model=768, head_dim=64, hidden_dim=2304)
+PAIRS = dict(WIDE, n_kv_head=6)
+CASES = [
+    (PAIRS, lib.FORMAT_Q8_0, lib.FORMAT_F16, 552, 40), (WIDE, lib.FORMAT_Q8_0, lib.FORMAT_F32, 552, 40), (WIDE, lib.FORMAT_Q4_0, lib.FORMAT_F16, 2760, 200), (WIDE, lib.FORMAT_Q4_K, lib.FORMAT_F16, 1064, 40),
+    (PAIRS, lib.FORMAT_Q8_0, lib.FORMAT_F16, 1034, 10), (PAIRS, lib.FORMAT_Q4_0, lib.FORMAT_F32, 513, 1),
+    (WIDE, lib.FORMAT_Q4_K, lib.FORMAT_F16, 1031, 7),   # activations as pairs: a block of its own
+    (PAIRS, lib.FORMAT_F16, lib.FORMAT_F16, 1031, 7), (dict(n_head=8, n_kv_head=2, d_model=512, head_dim=64, hidden_dim=768), lib.FORMAT_Q4_K, lib.FORMAT_F16, 543, 31),   # attention alone
+]
+
+
+@pytest.mark.parametrize("shape,fmt,kv,count,last", CASES)
+def test_last_rows_are_as_exact_as_in_a_block_of_their_own(shape, fmt, kv, count, last):
+    import espresso_amd.ops as ops
+    import espresso_amd.synthetic as syn
+    ops.init()
+    cfg = ll.MultiModelConfig(n_layer=2, vocab=260, max_seq=2816, **shape)
+    rt, _ = syn.build_runtime(cfg, fmt, seed=3, std=0.05, kv_format=kv, max_sequences=2)
+    prompt = np.random.default_rng(count).integers(0, 260, count).astype(np.uint32)
+    rt.prefill(prompt[:count - last])
+    want = rt.append(prompt[count - last:], want=range(last))
+    rt.reset()
+    got = rt.append(prompt, want=range(count - last, count))
+    hidden = rt.last_hidden()
+    # the same roundings, sums in another order: a last bit of an fp16 activation falls either way, up to 5.3e-4 of the logits' size; in a long block like its other rows they are 1.0 to 1.7e-3 off
+    # (products and attention of pairs of fp16: 0, and 2.3e-5)
+    assert rms_off(got, want) <= (2.0 ** -18 if shape["d_model"] == 512 else 3 * 2.0 ** -12)
+    rt.reset()
+    ll.generate_batch(rt, [prompt, prompt[:count - 3]], 1)
+    assert np.array_equal(rt.last_hidden(), hidden)
+    rt.close()
+
+
+@pytest.mark.parametrize("fmt,kv,count", [(lib.FORMAT_F16, lib.FORMAT_F16, 600), (lib.FORMAT_Q8_0, lib.FORMAT_F16, 1008), (lib.FORMAT_Q4_K, lib.FORMAT_F32, 1012)])
+def test_rows_that_gain_nothing_stay_in_the_long_block(fmt, kv, count):
+    """A last stretch whose block would round the same way adds no pass over the weights: one launch of each product, whatever follows the last 512 rows."""
+    import espresso_amd.ops as ops
+    import espresso_amd.synthetic as syn
+    ops.init()
+    cfg = ll.MultiModelConfig(n_layer=1, vocab=260, max_seq=1024, n_head=16, n_kv_head=16, d_model=2048, head_dim=128, hidden_dim=5632)
+    rt, _ = syn.build_runtime(cfg, fmt, seed=3, std=0.03, kv_format=kv)
+    prompt = np.random.default_rng(count).integers(0, 260, count).astype(np.uint32)
+    rt.prefill(prompt[:512])
+    rt.append(prompt[512:])
+    apart = rt.last_hidden()
+    rt.reset()
+    rt.prefill(prompt)
+    # another order of sums somewhere
+    assert not np.array_equal(rt.last_hidden(), apart) and np.abs(rt.last_hidden() - apart).max() <= 4e-3 * max(1.0, np.abs(apart).max())
+    rt.close()
