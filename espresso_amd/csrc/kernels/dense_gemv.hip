@@ -393,8 +393,11 @@ int resident_workgroups() {
 template <int KIND, int RPW, int AHEAD>
 hipError_t run(DenseGemvArgs a, int grid, hipStream_t s) {
     a.k_pad = (a.ld + kStep * AHEAD - 1) / (kStep * AHEAD) * (kStep * AHEAD);
-    const size_t lds = (size_t)(a.k_pad + a.heads + a.part_count * a.part_pieces) * 4;
-    if (lds > 150 * 1024 || grid < 1) return hipErrorInvalidValue;
+    // rows of up to 150 KB in whole steps, whose whole turns add at most 6 KB: 156 of the compute unit's 160
+    const int columns = (a.ld + kStep - 1) / kStep * kStep, beside = a.heads + a.part_count * a.part_pieces;
+    static_assert(AHEAD <= 4, "three steps of padding at most");
+    if ((size_t)(columns + beside) * 4 > 150 * 1024 || grid < 1) return hipErrorInvalidValue;
+    const size_t lds = (size_t)(a.k_pad + beside) * 4;
     static size_t allowed = 0;
     if (lds > 48 * 1024 && lds > allowed) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_gemv_kernel<KIND, RPW, AHEAD>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

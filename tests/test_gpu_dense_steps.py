@@ -35,6 +35,21 @@ def test_steps_at_the_rings_edges(tmp_path, width, ff, vocab, parallel):
     assert chain == alone
 
 
+# Rows of 36865 to 38400 columns: whole steps of 512 within 150 KB, whole turns of four beyond it
+@pytest.mark.parametrize("ff", [36700, 37300, 37500])
+@pytest.mark.parametrize("parallel", [True, False])
+def test_the_longest_rows(tmp_path, ff, parallel):
+    if parallel:
+        cfg = lu.config([lu.retention(heads=3, dim=48, vdim=72, ff=ff), lu.latent(heads=5, dim=40, ff=ff)], width=64, vocab=97)
+    else:
+        cfg = lu.sequential([lu.mamba2(heads=6, vdim=40, state=40, ff=ff), lu.attention(heads=8, dim=32, vdim=40, dims=16, ff=ff)], width=64, vocab=97)
+    m = lu.Model(tmp_path, cfg, seed=3, gain=1.5)
+    t = lu.tokens(m.cfg, 5, 3)
+    want = m.logits(t)
+    rt = m.runtime("bf16", max_seq=32)
+    assert lu.error(lu.feed(rt, t, [1] * 5), want) < lu.limit("bf16")
+
+
 # Slices of latent attention merged in one request (32 and fewer of a rank of up to 512) and in several
 @pytest.mark.parametrize("rank,keys", [(64, 1), (64, 33), (512, 65), (576, 40), (960, 1100), (128, 2100)])
 def test_slices_of_latents_merged(tmp_path, rank, keys):
