@@ -228,14 +228,17 @@ int DecoderRuntime::prefill_batch(const uint32_t *const *prompts, const int *cou
             int rows = 0;
             for (next = first; next < spans.size() && rows < even && rows + spans[next].count <= block_rows_; next++) rows += spans[next].count;
             if (next - first < 2) continue;   // a block of its own, below
+            for (size_t i = first; i < next; i++) visible_[spans[i].sequence] = 0;   // until the block is done: what fails leaves no tokens over caches that it has begun to write
             if ((rc = prefill_shared_block(&spans[first], (int)(next - first))) != ESP_OK) return rc;
             for (size_t i = first, row = 0; i < next; i++) {
                 row += spans[i].count;
                 if ((rc = keep_row((int)row - 1, spans[i].sequence)) != ESP_OK) return rc;
+            }
+            ESP_HIP_TRY(hipStreamSynchronize(context().stream));
+            for (size_t i = first; i < next; i++) {
                 visible_[spans[i].sequence] = spans[i].count;
                 done[spans[i].sequence] = 1;
             }
-            ESP_HIP_TRY(hipStreamSynchronize(context().stream));
         }
     }
     for (int s = 0; s < count; s++)
