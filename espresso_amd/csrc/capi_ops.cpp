@@ -49,13 +49,14 @@ class Staging {
         std::lock_guard<std::mutex> lock(handles_mutex_);
         if (handles_++ > 0) return;
         std::lock_guard<std::mutex> call(mutex_);
-        void *host = nullptr;
-        if (hipHostMalloc(&host, kStagedIn + kStagedOut, hipHostMallocDefault) != hipSuccess) host = nullptr;
-        host_ = static_cast<uint8_t *>(host);
-        if (host_ && (hipHostGetDevicePointer(&host, host_, 0) != hipSuccess || device_alloc(&device_, kStagedIn + kStagedOut) != ESP_OK || device_alloc(&planes_, kNoAllocScratchFloats) != ESP_OK)) drop();
-        mapped_ = static_cast<uint8_t *>(host);
+        // (not by device_alloc: what fails here fails no call, and the thread's last error stays what it is)
+        void *host = nullptr, *mapped = nullptr, *device = nullptr, *planes = nullptr;
+        const bool got = hipHostMalloc(&host, kStagedIn + kStagedOut, hipHostMallocDefault) == hipSuccess && hipHostGetDevicePointer(&mapped, host, 0) == hipSuccess &&
+                         hipMalloc(&device, kStagedIn + kStagedOut) == hipSuccess && hipMalloc(&planes, kNoAllocScratchFloats * sizeof(float)) == hipSuccess;
+        host_ = static_cast<uint8_t *>(host); mapped_ = static_cast<uint8_t *>(mapped); device_ = static_cast<uint8_t *>(device); planes_ = static_cast<float *>(planes);
+        if (got) return;
         (void)hipGetLastError();
-        clear_error();
+        drop();
     }
     void leave() {
         std::lock_guard<std::mutex> lock(handles_mutex_);

@@ -60,3 +60,18 @@ def test_threads_and_handles(ops):
     for t in threads:
         t.join()
     assert not failures, failures
+
+
+def test_a_handle_leaves_the_last_error(ops):
+    """A matrix that is made, the first of its process or not, is no failure: the most recent one stays what it was."""
+    m, _ = matrix(ops, 32, 64, 1)
+    with pytest.raises(lib.EspressoError, match="layer_product: rows 0"):
+        m.layer_product(np.zeros((0, 64), np.float16))
+    m.close()
+    said = lib.last_error()
+    other, w = matrix(ops, 32, 64, 2)
+    assert lib.last_error() == said and "layer_product" in said
+    check(other, w, 2, 3, True)
+    assert lib.last_error() == said
+    other.close()
+    assert lib.last_error() == said
