@@ -38,34 +38,33 @@ static const DeviceSetup noalloc_scratch(noalloc_setup);
 }  // namespace esp
 
 // ---- staging of single products (esp_gemv) ------------------------------------------------------------------
-// A product of a few rows is 5 us of kernel; three allocations and frees, two pageable copies and their waits made 34 us of it.  One staging area for the process, there while any matrix handle is:
+// A product of a few rows is 5 us of kernel; three allocations and frees, two pageable copies and their waits made 34 us of it.  One staging area for the process, there from the second product on
+// while any matrix handle is (a program that makes a handle for one product does without: made with the handle, 2048 x 2048 Q8_0 made, multiplied once and freed 870 us, 293 without; 768 x 768 168 and 89):
 // pinned memory that takes the call's activations and residual, which a small kernel brings to the device (4 us less than a copy engine's start), and its result, which the product writes there itself.
-// A call that finds it in use by another thread, or that needs more, allocates as before.  4096 x 4096 Q4_K, 2 / 16 / 40 rows 34.8 / 88 / 116 -> 22.7 / 39 / 66 us, of which the caller's Python is 2.
+// A call that finds it in use by another thread, or that needs more, allocates as before.  4096 x 4096 Q4_K, 2 / 16 / 40 / 128 rows 34.8 / 88 / 116 / 256 -> 22.7 / 39 / 66 / 185 us, of which the
+// caller's Python is 2; 768 x 768 Q8_0, 512 rows 178 -> 133, with a residual 265 -> 205: as far as the area goes, results cross the bus faster than through a copy.
 namespace {
 constexpr size_t kStagedIn = (size_t)1 << 20, kStagedOut = (size_t)4 << 20;   // bytes of activations and of residual or result
 class Staging {
   public:
-    void join() {   // without memory the calls allocate
+    void join() {
         std::lock_guard<std::mutex> lock(handles_mutex_);
-        if (handles_++ > 0) return;
-        std::lock_guard<std::mutex> call(mutex_);
-        // (not by device_alloc: what fails here fails no call, and the thread's last error stays what it is)
-        void *host = nullptr, *mapped = nullptr, *device = nullptr, *planes = nullptr;
-        const bool got = hipHostMalloc(&host, kStagedIn + kStagedOut, hipHostMallocDefault) == hipSuccess && hipHostGetDevicePointer(&mapped, host, 0) == hipSuccess &&
-                         hipMalloc(&device, kStagedIn + kStagedOut) == hipSuccess && hipMalloc(&planes, kNoAllocScratchFloats * sizeof(float)) == hipSuccess;
-        host_ = static_cast<uint8_t *>(host); mapped_ = static_cast<uint8_t *>(mapped); device_ = static_cast<uint8_t *>(device); planes_ = static_cast<float *>(planes);
-        if (got) return;
-        (void)hipGetLastError();
-        drop();
+        handles_++;
     }
     void leave() {
         std::lock_guard<std::mutex> lock(handles_mutex_);
         if (--handles_ > 0) return;
         std::lock_guard<std::mutex> call(mutex_);
         drop();
+        products_ = 0;
     }
     std::mutex &mutex() { return mutex_; }
-    bool takes(size_t in, size_t out) const { return host_ && in <= kStagedIn && out <= kStagedOut; }
+    // whether a call (of the holder of the mutex) is staged; without memory none is until the last handle has gone
+    bool takes(size_t in, size_t out) {
+        if (in > kStagedIn || out > kStagedOut) return false;
+        if (products_ < 2 && ++products_ == 2) allocate();
+        return host_ != nullptr;
+    }
     // two regions: activations; the residual, and in its place the result, which comes when the residual is on the device
     uint8_t *host_in() { return host_; }
     uint8_t *host_out() { return host_ + kStagedIn; }
@@ -76,6 +75,15 @@ class Staging {
     float *planes() { return planes_; }
 
   private:
+    void allocate() {   // not by device_alloc: what fails here fails no call, and the thread's last error stays what it is
+        void *host = nullptr, *mapped = nullptr, *device = nullptr, *planes = nullptr;
+        const bool got = hipHostMalloc(&host, kStagedIn + kStagedOut, hipHostMallocDefault) == hipSuccess && hipHostGetDevicePointer(&mapped, host, 0) == hipSuccess &&
+                         hipMalloc(&device, kStagedIn + kStagedOut) == hipSuccess && hipMalloc(&planes, kNoAllocScratchFloats * sizeof(float)) == hipSuccess;
+        host_ = static_cast<uint8_t *>(host); mapped_ = static_cast<uint8_t *>(mapped); device_ = static_cast<uint8_t *>(device); planes_ = static_cast<float *>(planes);
+        if (got) return;
+        (void)hipGetLastError();
+        drop();
+    }
     void drop() {
         if (host_) (void)hipHostFree(host_);
         if (device_) (void)hipFree(device_);
@@ -84,7 +92,7 @@ class Staging {
         planes_ = nullptr;
     }
     std::mutex handles_mutex_, mutex_;   // of the count, and of the memory while a call uses it
-    int handles_ = 0;
+    int handles_ = 0, products_ = 0;     // products_: that could be staged, up to two
     uint8_t *host_ = nullptr, *mapped_ = nullptr, *device_ = nullptr;
     float *planes_ = nullptr;
 };
