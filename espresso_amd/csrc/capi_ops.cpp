@@ -331,7 +331,7 @@ int esp_block_attention(int kernel, const float *q, const void *k, const void *v
     a.n_head = heads; a.n_kv_head = kv_heads; a.head_dim = head_dim; a.max_seq = first + rows;
     const size_t nq = (size_t)rows * heads * head_dim, nk = (size_t)a.max_seq * kv_heads * head_dim;
     a.cache_seq_stride = nk;
-    const bool takes = kernel == ESP_ATTENTION_SINGLE_ROW ? heads % kv_heads == 0 && (head_dim == 64 || head_dim == 128) && !split_rows
+    const bool takes = kernel == ESP_ATTENTION_SINGLE_ROW || (kernel == ESP_ATTENTION_STEP && rows <= kMaxStepRows) ? heads % kv_heads == 0 && (head_dim == 64 || head_dim == 128) && !split_rows
                        : kernel == ESP_ATTENTION_PROMPT ? attention_prompt_supported(heads, kv_heads, head_dim) && (!split_rows || (kv_f16 && heads * head_dim % 256 == 0))
                        : kernel == ESP_ATTENTION_SPAN ? span_attention_supported(heads, kv_heads, head_dim) && (!split_rows || heads * head_dim % 256 == 0) : false;
     if (!takes) return fail(ESP_ERR_UNSUPPORTED, "block_attention: kernel %d does not take this shape", kernel);
@@ -352,7 +352,7 @@ int esp_block_attention(int kernel, const float *q, const void *k, const void *v
     const size_t each = kv_f16 ? 2 : 4, partials = (size_t)rows * heads * kAttentionMaxSplits * (head_dim + 4);
     if ((rc = device_alloc(&d_q, nq)) != ESP_OK || (rc = device_alloc(&d_k, nk * each)) != ESP_OK || (rc = device_alloc(&d_v, nk * each)) != ESP_OK ||
         (rc = device_alloc(&d_at, (size_t)2 * rows)) != ESP_OK || (rc = device_alloc(&d_hi, nq)) != ESP_OK || (rc = device_alloc(&d_lo, nq)) != ESP_OK ||
-        (rc = device_alloc(&d_sums, nq / 16 + 16)) != ESP_OK || (kernel == ESP_ATTENTION_SINGLE_ROW && (rc = device_alloc(&d_scratch, partials)) != ESP_OK)) {
+        (rc = device_alloc(&d_sums, nq / 16 + 16)) != ESP_OK || ((kernel == ESP_ATTENTION_SINGLE_ROW || kernel == ESP_ATTENTION_STEP) && (rc = device_alloc(&d_scratch, partials)) != ESP_OK)) {
         release();
         return rc;
     }
@@ -363,6 +363,7 @@ int esp_block_attention(int kernel, const float *q, const void *k, const void *v
     if (e == hipSuccess) e = hipMemcpy(d_v, v, nk * each, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_at, at.data(), at.size() * sizeof(int), hipMemcpyHostToDevice);
     a.q = d_q; a.k_cache = d_k; a.v_cache = d_v; a.pos = d_at; a.seq = d_at + rows; a.split_scratch = d_scratch;
+    if (kernel == ESP_ATTENTION_STEP) a.head_partials = d_scratch;
     if (split_rows) { a.ctx_hi = d_hi; a.ctx_lo = d_lo; a.ctx_sums = d_sums; }
     else a.ctx_f16 = d_hi;
     auto launch = [&] {

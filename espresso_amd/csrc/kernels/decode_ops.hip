@@ -1493,11 +1493,9 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
     const int group = a.n_head / a.n_kv_head;
     const bool by_head = a.head_partials && (a.head_dim == 128 || a.head_dim == 64) && a.n_head % a.n_kv_head == 0 && rows <= kMaxStepRows &&
                          a.cache_seq_stride <= 0xFFFFFFFFull && a.n_head <= 0xFFFF;
-    // Contexts of up to 512 tokens: the kernel of the single-row step, whose four slices of a head cover them in two passes (sixteen
-    // sequences of the 8B model, attention + merge of a layer: prefix 60-84 of 512 8.4 + 6.6 -> 6.4 + 4.8 us, 384 of 512 14.4 + 6.6 -> 12.7 + 4.9;
-    // 768 of 1024 19.5 + 6.7 against 21.4 + 4.9, 3072 of 4096 55.7 + 6.6 against 65.9 + 4.9: those keep the kernel that reads a key once per group).  Whole layers of
-    // three to sixteen sequences, contexts of 128, 256 and 512, fp16 and fp32 caches: 12 over 12 heads of 64 2 to 3 us less of 36 to 50, 32 over 8 of 64 0.5 to 4 of 43 to 58, 16 over 16 and
-    // over 8 of 128 1.5 to 4 of 43 to 70, 32 over 8 of 128 3 to 7 of 93 to 124.  The line lies at the context's size, not at the prefix's: a captured step replays the kernel.
+    // Contexts of up to 512 tokens: the kernel of the single-row step, which with one slice or four of a head and two passes over them was 0.5 to 7 us a layer faster than the kernel that reads a key
+    // once per group (whole layers of three to sixteen sequences, contexts of 128, 256 and 512, both caches, heads of 64 and 128; attention alone, sixteen sequences of 8B: prefix 384 of 512
+    // 14.4 + 6.6 -> 12.7 + 4.9, but 768 of 1024 19.5 + 6.7 against 21.4 + 4.9).  The line lies at the context's size, not at the prefix's: a captured step replays the kernel.
     if (a.n_head % a.n_kv_head == 0 && !(by_head && a.max_seq <= 512)) {
         if (a.head_dim == 128) {
             if (group == 1) return launch_attention_gqa<128, 1>(a, rows, kv_f16, s);
@@ -1510,7 +1508,12 @@ hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipSt
         }
     }
     // short contexts and other head groups: the kernel of the single-row step and a merge launch
-    if (by_head && a.max_seq <= 512) {   // the whole prefix in one workgroup: no merge (sixteen sequences of 8B, prefix 60-84 of 512, 6.5 + 4.8 -> 5.5 us)
+    // The whole prefix in one workgroup of eight wavefronts, no merge (sixteen sequences of 8B, prefix 60-84 of 512, 6.5 + 4.8 -> 5.5 us).  Keys of 128 dims in 32 bits are four passes of 512 bytes each
+    // for every 128 of them: there only where the workgroups nearly fill the chip, or the context is short.  Steps of one to eight sequences, contexts of 512, prefixes of 40 / 150 / 300 / 470, one
+    // workgroup against four slices and a merge: 128 dims, fp32 caches, 32 heads x 1 -2.4 / +2.4 / +4.0 / +7.2 %, x 4 -3.0 / 0 / -0.5 / +1.9, x 8 -4.9 / -2.7 / -4.4 / -3.0, 16 heads x 2
+    // -4.7 / +1.9 / +4.7 / +10.7, x 8 -3.3 / +0.8 / +0.4 / +2.9 (contexts of 256: -2 to -5 / -3 to +2 %); fp16 caches -2.7 to -6.5 / -3.7 to +0.3 / -5.1 to +0.4 / -4.2 to +2.3; 64 dims, both caches,
+    // -3.7 to -9.0 / -2.4 to -6.5 / -2.1 to -7.3 / -5.7 to +2.2.
+    if (by_head && a.max_seq <= 512 && (a.head_dim == 64 || kv_f16 || a.max_seq <= 256 || rows * a.n_head >= 192)) {
         const unsigned heads = (unsigned)a.n_head | ((unsigned)a.n_kv_head << 16);
         auto launch = [&](auto kernel, int waves) {
             hipLaunchKernelGGL(kernel, dim3(a.n_head, rows), dim3(waves * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, reinterpret_cast<float *>(a.ctx_f16), (unsigned)a.cache_seq_stride, heads);

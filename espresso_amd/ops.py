@@ -212,7 +212,7 @@ def hbm_read_probe_pairs(bytes_per_launch: int, pair_bytes: int = 2304, workgrou
     return {"mean_us": us.value, "gbps": gbps.value}
 
 
-ATTENTION_KERNELS = ("single_row", "prompt", "span")
+ATTENTION_KERNELS = ("single_row", "prompt", "span", "step")
 
 
 def block_attention(kernel: str, q: np.ndarray, k: np.ndarray, v: np.ndarray, split_rows: bool = False, iters: int = 1) -> tuple[np.ndarray, float]:

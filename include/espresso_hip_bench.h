@@ -70,6 +70,7 @@ int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, 
 #define ESP_ATTENTION_SINGLE_ROW 0   /* every row by itself */
 #define ESP_ATTENTION_PROMPT 1       /* prompt blocks, one, two or four query heads per key/value head */
 #define ESP_ATTENTION_SPAN 2         /* blocks of any head group */
+#define ESP_ATTENTION_STEP 3         /* up to 32 rows as a step of several sequences has them, the context as long as it is */
 int esp_block_attention(int kernel, const float *q, const void *k, const void *v, int kv_f16, int rows, int first, int heads, int kv_heads, int head_dim,
                         int split_rows, float *ctx, int iters, double *mean_us);
 int esp_hbm_read_probe(size_t bytes, int iters, double *gb_per_s);

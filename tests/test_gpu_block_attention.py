@@ -148,3 +148,21 @@ def test_fp32_values_beyond_fp16_that_add_up(ops, kernel):
     got, _ = ops.block_attention(kernel, q, k, v)
     assert np.abs(want).max() < 65504 and np.isfinite(got).all()
     assert np.abs(got - want).max() <= 2.0 ** -11 * np.abs(want).max()
+
+
+# One workgroup a head (64 dims, fp16 caches, contexts of up to 256, 192 rows x heads and more), four slices and a merge, and the kernel of longer contexts; keys that end at, before and behind a pass of
+# eight wavefronts (128 or 256 keys) and several passes
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("rows,first,heads,kv_heads,size", [
+    (1, 0, 4, 4, 128), (3, 124, 8, 2, 128), (3, 125, 8, 8, 128), (2, 127, 6, 2, 64), (4, 253, 6, 2, 128), (5, 254, 4, 1, 128), (16, 300, 12, 4, 128), (3, 480, 32, 8, 128), (16, 496, 16, 16, 64), (8, 381, 9, 3, 64),
+    (32, 200, 8, 2, 128), (6, 500, 32, 8, 128), (7, 600, 8, 2, 64)])
+def test_steps_are_as_exact_as_fp32(ops, rows, first, heads, kv_heads, size, dtype):
+    for sharp in (1.0, 60.0):
+        q, k, v = inputs(rows, first, heads, kv_heads, size, dtype, rows + first, sharp)
+        want = exact(q, k, v)
+        got, _ = ops.block_attention("step", q, k, v)
+        one, _ = ops.block_attention("single_row", q, k, v)
+        off = lambda c: np.sqrt(np.mean((c - want) ** 2))  # noqa: E731
+        # fp32 arithmetic as above, the context rounded to fp16 once (2^-11 at most); the kernel of longer contexts rounds likewise
+        assert off(got) <= 2.0 ** -24 * (np.sqrt(size) * sharp + 8) + 2.0 ** -11 * np.sqrt(np.mean(want ** 2)), sharp
+        assert off(got) <= 1.02 * off(one) + 2.0 ** -24 * np.sqrt(size) * sharp, sharp
