@@ -114,6 +114,9 @@ WideForm wide_gemm_form(const GemmParams &p) {
     if (w.forced == 0 && g_wide_gemm_shared.load() && p.swiglu_out && p.workspace && p.w.rows >= 8192 && p.rows > 64 && w.steps > 1 &&
         (long)((p.w.rows + 127) / 128) * ((p.rows + 127) / 128) <= (w.compute_units > 0 ? w.compute_units : 256))
         w.shares = 2;
+    const WideForm f = choose_wide_form(w);
+    if (f.bm || w.forced == 0) return f;
+    w.forced = 0;   // shares whose planes have no room: by size
     return choose_wide_form(w);
 }
 

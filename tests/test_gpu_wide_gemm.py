@@ -58,3 +58,16 @@ def test_what_is_not_finite_stays_in_its_row(ops, planted):
         assert np.array_equal(got[:-1], clean[:-1]) and not np.isfinite(got[-1]).any(), form
     ops.set_tuning("wide_gemm_form", 0)
     m.close()
+
+
+def test_a_form_without_room_for_its_planes_is_by_size(ops):
+    """Eight shares of 512 x 1100 sums are more than a product's workspace."""
+    rng = np.random.default_rng(3)
+    m, _ = matrix(ops, rng, 1100, 1024)
+    x = rng.normal(0, 1, (512, 1024)).astype(np.float16)
+    by_size = m.layer_product(x)
+    for form in (641288, 2562568):
+        ops.set_tuning("wide_gemm_form", form)
+        assert np.array_equal(m.layer_product(x), by_size), form
+    ops.set_tuning("wide_gemm_form", 0)
+    m.close()
