@@ -241,6 +241,37 @@ int esp_gemv(const ESPMatrix *matrix, const uint16_t *x_f16, int batch, float *y
     return e == hipSuccess ? ESP_OK : fail_hip(e, "gemv");
 }
 
+int esp_layer_gate_up(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, uint16_t *act_f16) {
+    if (!matrix || !x_f16 || !act_f16) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_gate_up: null pointer");
+    const DeviceMatrix &m = matrix->m;
+    if (rows <= 0 || rows > 2048 || m.rows % 2 != 0) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_gate_up: rows %d of %d", rows, m.rows);
+    int rc = ensure_init();
+    if (rc != ESP_OK) return rc;
+    if (m.format == FMT_F32 || m.cols % 64 != 0) return fail(ESP_ERR_UNSUPPORTED, "layer_gate_up: matrices on the matrix cores");
+    Context &c = context();
+    const size_t nx = (size_t)rows * m.cols, na = (size_t)rows * (m.rows / 2);
+    uint16_t *d_x = nullptr, *d_act = nullptr;
+    float *d_y = nullptr, *d_ws = nullptr;
+    auto release = [&] {
+        void *ptrs[] = {d_x, d_act, d_y, d_ws};
+        for (void *p : ptrs) if (p) (void)hipFree(p);
+    };
+    if ((rc = device_alloc(&d_x, nx)) != ESP_OK || (rc = device_alloc(&d_act, na)) != ESP_OK || (rc = device_alloc(&d_y, 2 * na)) != ESP_OK || (rc = device_alloc(&d_ws, kGemmWorkspaceFloats)) != ESP_OK) {
+        release();
+        return rc;
+    }
+    hipError_t e = hipMemcpyAsync(d_x, x_f16, nx * 2, hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess) {
+        GemmParams g;
+        g.w = m; g.x = d_x; g.y = d_y; g.swiglu_out = d_act; g.rows = rows; g.unrounded = true; g.workspace = d_ws; g.workspace_floats = kGemmWorkspaceFloats;
+        e = launch_gemm(g, c.stream);
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(act_f16, d_act, na * 2, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    release();
+    return e == hipSuccess ? ESP_OK : fail_hip(e, "layer_gate_up");
+}
+
 int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares) {
     if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: null pointer");
     if (rows <= 0 || rows > 2048) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: rows %d", rows);

@@ -20,7 +20,6 @@
 #include "block_gemm.h"
 #include "block_tile.h"
 #include "silu.h"
-#include "wide_gemm.h"
 #include <type_traits>
 
 namespace esp {
@@ -396,7 +395,6 @@ void block_gemm_set_form(int form) {
     const int tm = form / 100, nw = form / 10 % 10, shares = form % 10;
     const bool known = tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
     g_block_gemm_form.store(known ? form : 0);
-    wide_gemm_set_shared(form == -1);
 }
 
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are

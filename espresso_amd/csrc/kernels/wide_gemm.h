@@ -11,6 +11,4 @@ WideForm wide_gemm_form(const GemmParams &p);   // no tile: not an fp16 matrix
 hipError_t launch_wide_gemm(const GemmParams &p, const WideForm &form, hipStream_t stream);
 void wide_gemm_set_form(int form);   // 0 by size (default), otherwise always, where its planes have room: rows of a tile * 10000 + weight rows * 10 + shares of K
 
-void wide_gemm_set_shared(bool shared);   // gate|up of 8192 and more rows, beyond 64 rows of activations and up to one 128 x 128 tile per compute unit: in two shares of K (measurements, tests)
-
 }  // namespace esp

@@ -94,11 +94,9 @@ hipError_t launch_form(const WideForm &f, const WideArgs &a, hipStream_t stream)
     }
 }
 std::atomic<int> g_wide_gemm_form{0};
-std::atomic<bool> g_wide_gemm_shared{false};
 
 }  // namespace
 
-void wide_gemm_set_shared(bool shared) { g_wide_gemm_shared.store(shared); }
 void wide_gemm_set_form(int form) { g_wide_gemm_form.store(wide_form_known(form) ? form : 0); }
 
 // (behind a SiLU, and where no caller adds them, the planes take a launch of their own)
@@ -111,9 +109,6 @@ WideForm wide_gemm_form(const GemmParams &p) {
     w.after = p.swiglu_out ? 3.0f : p.deferred_splits ? 1.0f : 1.6f;
     w.after_share = p.swiglu_out || p.deferred_splits ? 0.0f : 0.2f;
     w.forced = g_wide_gemm_form.load();
-    if (w.forced == 0 && g_wide_gemm_shared.load() && p.swiglu_out && p.workspace && p.w.rows >= 8192 && p.rows > 64 && w.steps > 1 &&
-        (long)((p.w.rows + 127) / 128) * ((p.rows + 127) / 128) <= (w.compute_units > 0 ? w.compute_units : 256))
-        w.shares = 2;
     const WideForm f = choose_wide_form(w);
     if (f.bm || w.forced == 0) return f;
     w.forced = 0;   // shares whose planes have no room: by size

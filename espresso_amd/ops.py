@@ -104,6 +104,13 @@ class Matrix:
         _lib.check(_lib.load_library().esp_layer_product(self._h, _ptr(x), rows, _ptr(y), _ptr(res) if res is not None else None, int(shares)))
         return y
 
+    def layer_gate_up(self, x_f16: np.ndarray) -> np.ndarray:
+        """SiLU(gate) * up of interleaved gate / up rows as a model's layers ask for it, fp16 (esp_layer_gate_up; test aid)."""
+        x = np.ascontiguousarray(x_f16, dtype=np.float16).reshape(-1, self.cols)
+        act = np.empty((x.shape[0], self.rows // 2), dtype=np.float16)
+        _lib.check(_lib.load_library().esp_layer_gate_up(self._h, _ptr(x), x.shape[0], _ptr(act)))
+        return act
+
     def matmul_f32(self, x: np.ndarray, residual: np.ndarray | None = None) -> np.ndarray:
         """fp32 activations [rows][cols] against the matrix with no operand rounded (esp_matmul_f32; Q4_K)."""
         x = np.ascontiguousarray(x, dtype=np.float32).reshape(-1, self.cols)

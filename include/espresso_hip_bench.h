@@ -39,8 +39,8 @@ int esp_gemv_stamps(const ESPMatrix *matrix, int batch, int launches, uint64_t *
  * "q4k_mfma_ragged": 0 = every workgroup runs the same number of rounds.
  * "q4k_long_row_waves" (ESPRESSO_HIP_Q4K_LONG_ROW_WAVES): one activation row at 14336 columns: 0 (default) = the matrix-core
  * kernel, 8 or 4 = the dot-product kernel with that many wavefronts per workgroup (one or three workgroups per compute unit).
- * "block_gemm_form": blocks of rows with fp16 operands, rows of a tile / 32 * 100 + wavefronts along the weights * 10 + shares of K
- * (141, 282, ...), 0 (default) = by size, -1 = by size and tall fp16 gate|up products of 65 rows and more in two shares of K.  "wide_gemm_form": products with fp16 matrices, rows of a tile * 10000 + weight rows * 10 + shares of K (641284, 2562561, ...), 0 (default) = by size, as is a form whose planes have no room.
+ * "block_gemm_form": blocks of rows with packed weights, rows of a tile / 32 * 100 + wavefronts along the weights * 10 + shares of K
+ * (141, 282, ...), 0 (default) = by size.  "wide_gemm_form": products with fp16 matrices, rows of a tile * 10000 + weight rows * 10 + shares of K (641284, 2562561, ...), 0 (default) = by size, as is a form whose planes have no room.
  * "dense_gemm_form": bf16 products of the layered models, the same numbers; shares of K stay by size.
  * "block_split_form": the same for exact Q4_K products of split rows, -1 = never this kernel.  "batch_gemv_form": steps of three to sixteen rows with Q4_K matrices, row blocks of a workgroup * 10 + shares of K, 0 (default) = by size.  "wide_split_shares": exact Q4_K products of split rows in whole tiles, shares of K (1, 2, 3, 4, 6, 8), 0 (default) = by size, -1 = never.
  * "short_blocks": 0 = prompts of fewer than 32 tokens walk the steps, 1 (default) = a block where it is as exact and faster.
@@ -64,6 +64,9 @@ int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, flo
  * shares = 1: the launch may leave its sum in shares of K, as in front of a norm or the key/value caches; they and the residual are then added here, in the shares' order.
  * y, residual (may be NULL) [rows][matrix rows] fp32; host pointers. */
 int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares);
+/* Test aid: SiLU(gate) * up as the layers ask for it, of a matrix of interleaved gate / up rows (2i = gate_i, 2i + 1 = up_i), in the product's epilogue or by the launch that adds shares of K.
+ * act_f16 [rows][matrix rows / 2] fp16; host pointers. */
+int esp_layer_gate_up(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, uint16_t *act_f16);
 /* Test aid: causal attention of `rows` (up to 512) consecutive rows of one sequence at positions first, first + 1, ... by one of the kernels a model's
  * layers use.  q [rows][heads][head_dim] fp32; k, v [first + rows][kv_heads][head_dim] fp32, or fp16 bits with kv_f16; ctx [rows][heads][head_dim]
  * as fp32: the fp16 context, or with split_rows the two fp16 planes added back together (hi + lo / 2048).  Host pointers.  `iters` launches;

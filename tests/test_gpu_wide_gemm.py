@@ -42,6 +42,31 @@ def test_products_match_float64(ops, rows, cols, batches):
     m.close()
 
 
+# weight rows that end inside a tile, between two wavefronts and at a tile's end; fewer rows of activations than a tile, ragged ones, whole tiles
+@pytest.mark.parametrize("rows,cols,batches", [(134, 192, (3, 65, 193)), (522, 448, (64, 130, 257)), (256, 64, (9, 300))])
+def test_gate_up_matches_float64(ops, rows, cols, batches):
+    """SiLU(gate) * up in the product's epilogue (one share of K) and by the launch that adds planes (more), every tile."""
+    rng = np.random.default_rng(rows)
+    w = rng.normal(0, 2.0 / np.sqrt(cols), (rows, cols)).astype(np.float16)   # gates of both signs, up to six or so
+    m = ops.Matrix(lib.FORMAT_NAMES["f16"], w.view(np.uint8), rows, cols)
+    w = w.astype(np.float64)
+    for batch in batches:
+        x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
+        y = x.astype(np.float64) @ w.T
+        gate, up = y[:, 0::2], y[:, 1::2]
+        silu = gate / (1 + np.exp(-gate))
+        want = silu * up
+        # products as above; SiLU's slope is at most 1.1; its fp32 forms are off by 2^-22 of the gate, and the result is rounded to fp16 once
+        off = (cols + 16) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + 1)
+        bound = (1.1 * off[:, 0::2] + 2.0 ** -22 * np.abs(gate)) * (np.abs(up) + off[:, 1::2]) + np.abs(silu) * off[:, 1::2] + 2.0 ** -11 * np.abs(want) + 2.0 ** -25
+        for form in [0] + [10000 * bm + 10 * bn + shares for bm, bn in TILES for shares in (1, 2, 3)]:
+            ops.set_tuning("wide_gemm_form", form)
+            got = m.layer_gate_up(x).astype(np.float64)
+            assert (np.abs(got - want) <= bound).all(), (form, batch)
+    ops.set_tuning("wide_gemm_form", 0)
+    m.close()
+
+
 @pytest.mark.parametrize("planted", [np.inf, -np.inf, np.nan])
 def test_what_is_not_finite_stays_in_its_row(ops, planted):
     """Rows past the end of a tile repeat the last one, steps past the end of a share its last: neither may reach another row's sum."""
