@@ -512,71 +512,62 @@ int choose_splits(int blocks, int units, int min_units, int target, const GemmAr
     return splits;
 }
 
-// `swiglu_out` (may be null) is handed to the tile kernel when it runs without split-K; *fused tells the caller.
+// Up to eight rows of Q4_K: one workgroup per 32 weight rows, K split over its wavefronts.  The kernels' LDS (above 64 KB) is dynamic: the limit is raised once per kernel and device.
+hipError_t launch_few_rows(const GemmArgs &a, hipStream_t stream) {
+    const int groups = (a.N + 31) / 32;
+    auto go = [&](auto kernel, int waves, size_t lds, std::atomic<uint64_t> &raised) {
+        int device = 0;
+        hipError_t err = hipGetDevice(&device);
+        if (err != hipSuccess) return err;
+        const uint64_t bit = 1ull << (device & 63);
+        if (!(raised.load(std::memory_order_acquire) & bit)) {
+            err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (err != hipSuccess) return err;
+            raised.fetch_or(bit, std::memory_order_release);
+        }
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(waves * 64), lds, stream, a);
+        return hipGetLastError();
+    };
+    static std::atomic<uint64_t> raised8{0}, raised4{0};
+    if (groups <= 256) return go(gemm_rows_kernel<8, 8>, 8, rows_lds_bytes<8, 8>(), raised8);
+    return go(gemm_rows_kernel<4, 4>, 4, rows_lds_bytes<4, 4>(), raised4);
+}
+
+// gemm_kernel by size.  (Eight wavefronts on a 128 x 256 tile measure 2-5 % faster at 4096 and more weight rows and 10 % slower at 1024; a 256 x 256 tile is 25 % slower: not instantiated.)
+template <int FMT>
+hipError_t launch_tiles(const GemmParams &p, GemmArgs a, int *used_splits, hipStream_t stream) {
+    const int tiles = a.K / KT, mt = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
+    int splits = choose_splits((a.N + NT - 1) / NT * ((a.M + mt - 1) / mt), tiles, 8, 1024, a, p.workspace_floats);
+    a.tiles_per_split = ((tiles + splits - 1) / splits + 3) & ~3;   // every split starts on a multiple of four tiles
+    *used_splits = splits = (tiles + a.tiles_per_split - 1) / a.tiles_per_split;
+    if (splits == 1 && a.N % 2 == 0) a.swiglu_out = p.swiglu_out;
+    if (mt == 32) return launch_tile<FMT, 1, 4, 1, 1, 4>(a, splits, stream);
+    if (mt == 64) return launch_tile<FMT, 1, 4, 2, 1, 4>(a, splits, stream);
+    return launch_tile<FMT, 2, 2, 2, 2, 2>(a, splits, stream);
+}
+
+// p.swiglu_out (may be null) is written by a kernel that runs without shares of K; *fused tells the caller.  Partial sums are added by gemm_reduce_kernel, or left to the caller's next kernel
+// when it asked for that.
 template <int FMT>
 hipError_t launch_format(const GemmParams &p, GemmArgs a, bool *fused, int *deferred_splits, hipStream_t stream) {
-    uint16_t *const swiglu_out = p.swiglu_out;
-    *fused = false;
-    // split-K partial sums are added by gemm_reduce_kernel, or left to the caller's next kernel when it asked for that
-    auto finish = [&](hipError_t err, int used_splits) {
-        if (err != hipSuccess || used_splits == 1) return err;
-        if (deferred_splits) { *deferred_splits = used_splits; return hipSuccess; }
-        return launch_reduce(a, used_splits, stream);
-    };
-    [[maybe_unused]] const int n_blocks = (a.N + NT - 1) / NT;
+    if (FMT == FMT_Q4_K && a.M <= kRowsMaxRows) return launch_few_rows(a, stream);
     a.partial = p.workspace;
-    [[maybe_unused]] hipError_t e;
-    [[maybe_unused]] int splits;
-    if constexpr (FMT == FMT_Q4_K) {
-        // one workgroup per 32 weight rows, K split over its wavefronts
-        if (a.M <= kRowsMaxRows) {
-            const int groups = (a.N + 31) / 32;
-            // the kernels' LDS (above 64 KB) is dynamic: the limit is raised once per kernel and device
-            auto go = [&](auto kernel, int waves, size_t lds, std::atomic<uint64_t> &raised) {
-                int device = 0;
-                hipError_t err = hipGetDevice(&device);
-                if (err != hipSuccess) return err;
-                const uint64_t bit = 1ull << (device & 63);
-                if (!(raised.load(std::memory_order_acquire) & bit)) {
-                    err = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                    if (err != hipSuccess) return err;
-                    raised.fetch_or(bit, std::memory_order_release);
-                }
-                hipLaunchKernelGGL(kernel, dim3(groups), dim3(waves * 64), lds, stream, a);
-                return hipGetLastError();
-            };
-            static std::atomic<uint64_t> raised8{0}, raised4{0};
-            if (groups <= 256) return go(gemm_rows_kernel<8, 8>, 8, rows_lds_bytes<8, 8>(), raised8);
-            return go(gemm_rows_kernel<4, 4>, 4, rows_lds_bytes<4, 4>(), raised4);
-        }
-    }
+    int splits = 1;
+    hipError_t e;
     if constexpr (FMT == FMT_F16) {
         const WideForm f = wide_gemm_form(p);
         if (!f.bm) return hipErrorInvalidValue;
-        *fused = f.splits == 1 && swiglu_out && a.N % 2 == 0;
-        return finish(launch_wide_gemm(p, f, stream), f.splits);
+        splits = f.splits;
+        e = launch_wide_gemm(p, f, stream);
     } else {
-    if (block_gemm_takes(p)) {
-        e = launch_block_gemm(p, &splits, stream);
-        *fused = splits == 1 && swiglu_out && a.N % 2 == 0;
-        return finish(e, splits);
+        if (block_gemm_takes(p)) e = launch_block_gemm(p, &splits, stream);
+        else if constexpr (FMT == FMT_Q4_K) return hipErrorInvalidValue;   // whole super-blocks: block_gemm.hip takes them all
+        else e = launch_tiles<FMT>(p, a, &splits, stream);
     }
-    if constexpr (FMT == FMT_Q4_K) return hipErrorInvalidValue;   // whole super-blocks: the kernel above takes them all
-    else {
-    const int tiles = a.K / KT;
-    const int mt = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
-    // (eight wavefronts on a 128 x 256 tile measure 2-5 % faster at 4096 and more weight rows and 10 % slower at 1024;
-    //  a 256 x 256 tile is 25 % slower: not instantiated)
-    splits = choose_splits(n_blocks * ((a.M + mt - 1) / mt), tiles, 8, 1024, a, p.workspace_floats);
-    a.tiles_per_split = ((tiles + splits - 1) / splits + 3) & ~3;   // every split starts on a multiple of four tiles
-    splits = (tiles + a.tiles_per_split - 1) / a.tiles_per_split;
-    if (splits == 1 && swiglu_out && a.N % 2 == 0) { a.swiglu_out = swiglu_out; *fused = true; }
-    if (mt == 32) e = launch_tile<FMT, 1, 4, 1, 1, 4>(a, splits, stream);
-    else if (mt == 64) e = launch_tile<FMT, 1, 4, 2, 1, 4>(a, splits, stream);
-    else e = launch_tile<FMT, 2, 2, 2, 2, 2>(a, splits, stream);
-    return finish(e, splits);
-    }
-    }
+    *fused = splits == 1 && p.swiglu_out && a.N % 2 == 0;
+    if (e != hipSuccess || splits == 1) return e;
+    if (deferred_splits) { *deferred_splits = splits; return hipSuccess; }
+    return launch_reduce(a, splits, stream);
 }
 
 }  // namespace

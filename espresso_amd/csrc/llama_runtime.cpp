@@ -334,7 +334,7 @@ int LlamaRuntime::finalize() {
         ESP_HIP_TRY(hipMemcpy(rope_sin_, sn.data(), sn.size() * 4, hipMemcpyHostToDevice));
     }
     // ---- activations ----
-        {
+    {
         const char *pa = getenv("ESPRESSO_HIP_PROMPT_ATTENTION");   // "0": prompt blocks keep the single-query attention kernel
         const bool block_attention = !(pa && pa[0] == '0');
         prompt_attention_ = block_attention && attention_prompt_supported(c_.n_head, c_.n_kv_head, c_.head_dim);
