@@ -166,6 +166,8 @@ def _declare_llama(L: C.CDLL) -> None:
     L.esp_matrix_resident_bytes.argtypes = [vp]
     L.esp_llama_resident_weight_bytes.restype = C.c_size_t
     L.esp_llama_resident_weight_bytes.argtypes = [vp]
+    L.esp_step_product.restype = i32
+    L.esp_step_product.argtypes = [vp, vp, i32, vp, vp, i32]
     L.esp_layer_gate_up.restype = i32
     L.esp_layer_gate_up.argtypes = [vp, vp, i32, vp]
     L.esp_layer_product.restype = i32

@@ -198,6 +198,45 @@ hipError_t run_matvec(const DeviceMatrix &m, const uint16_t *d_x, int batch, flo
 }
 }  // namespace
 
+}  // extern "C"
+
+// A product of host rows through `launch`(activations, y that holds the residual, workspace, shares of K left there): the shares and the residual are added here, in the shares' order.
+template <class Launch>
+static int product_for_test(const DeviceMatrix &m, const uint16_t *x_f16, int rows, float *y, const float *residual, const char *name, Launch launch) {
+    int rc = ensure_init();
+    if (rc != ESP_OK) return rc;
+    Context &c = context();
+    const size_t nx = (size_t)rows * m.cols, ny = (size_t)rows * m.rows;
+    uint16_t *d_x = nullptr;
+    float *d_y = nullptr, *d_ws = nullptr;
+    auto release = [&] {
+        void *ptrs[] = {d_x, d_y, d_ws};
+        for (void *p : ptrs) if (p) (void)hipFree(p);
+    };
+    if ((rc = device_alloc(&d_x, nx)) != ESP_OK || (rc = device_alloc(&d_y, ny)) != ESP_OK || (rc = device_alloc(&d_ws, kGemmWorkspaceFloats)) != ESP_OK) {
+        release();
+        return rc;
+    }
+    int splits = 1;
+    hipError_t e = hipMemcpyAsync(d_x, x_f16, nx * 2, hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess && residual) e = hipMemcpyAsync(d_y, residual, ny * 4, hipMemcpyHostToDevice, c.stream);
+    if (e == hipSuccess) e = launch(d_x, d_y, d_ws, &splits, c.stream);
+    std::vector<float> planes(splits > 1 ? splits * ny : 0);
+    if (e == hipSuccess && splits > 1) e = hipMemcpyAsync(planes.data(), d_ws, planes.size() * 4, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(y, d_y, ny * 4, hipMemcpyDeviceToHost, c.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    release();
+    if (e != hipSuccess) return fail_hip(e, name);
+    for (size_t i = 0; i < ny && splits > 1; i++) {
+        float sum = planes[i];
+        for (int s = 1; s < splits; s++) sum += planes[s * ny + i];
+        y[i] = residual ? residual[i] + sum : sum;
+    }
+    return ESP_OK;
+}
+
+extern "C" {
+
 int esp_gemv(const ESPMatrix *matrix, const uint16_t *x_f16, int batch, float *y, const float *residual) {
     if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "gemv: null pointer");
     if (batch <= 0) return fail(ESP_ERR_INVALID_ARGUMENT, "gemv: batch %d", batch);
@@ -275,43 +314,27 @@ int esp_layer_gate_up(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, 
 int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares) {
     if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: null pointer");
     if (rows <= 0 || rows > 2048) return fail(ESP_ERR_INVALID_ARGUMENT, "layer_product: rows %d", rows);
-    int rc = ensure_init();
-    if (rc != ESP_OK) return rc;
-    Context &c = context();
     const DeviceMatrix &m = matrix->m;
     if (m.format == FMT_F32 || m.cols % 64 != 0) return fail(ESP_ERR_UNSUPPORTED, "layer_product: matrices on the matrix cores");
-    const size_t nx = (size_t)rows * m.cols, ny = (size_t)rows * m.rows;
-    uint16_t *d_x = nullptr;
-    float *d_y = nullptr, *d_ws = nullptr;
-    auto release = [&] {
-        void *ptrs[] = {d_x, d_y, d_ws};
-        for (void *p : ptrs) if (p) (void)hipFree(p);
-    };
-    if ((rc = device_alloc(&d_x, nx)) != ESP_OK || (rc = device_alloc(&d_y, ny)) != ESP_OK || (rc = device_alloc(&d_ws, kGemmWorkspaceFloats)) != ESP_OK) {
-        release();
-        return rc;
-    }
-    int splits = 1;
-    hipError_t e = hipMemcpyAsync(d_x, x_f16, nx * 2, hipMemcpyHostToDevice, c.stream);
-    if (e == hipSuccess && residual) e = hipMemcpyAsync(d_y, residual, ny * 4, hipMemcpyHostToDevice, c.stream);
-    if (e == hipSuccess) {
+    return product_for_test(m, x_f16, rows, y, residual, "layer_product", [&](const uint16_t *d_x, float *d_y, float *workspace, int *splits, hipStream_t s) {
         GemmParams g;
-        g.w = m; g.x = d_x; g.y = d_y; g.residual = residual ? d_y : nullptr; g.rows = rows; g.unrounded = true; g.workspace = d_ws; g.workspace_floats = kGemmWorkspaceFloats;
-        if (shares) g.deferred_splits = &splits;
-        e = launch_gemm(g, c.stream);
-    }
-    std::vector<float> planes(splits > 1 ? splits * ny : 0);
-    if (e == hipSuccess && splits > 1) e = hipMemcpyAsync(planes.data(), d_ws, planes.size() * 4, hipMemcpyDeviceToHost, c.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(y, d_y, ny * 4, hipMemcpyDeviceToHost, c.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-    release();
-    if (e != hipSuccess) return fail_hip(e, "layer_product");
-    for (size_t i = 0; i < ny && splits > 1; i++) {
-        float sum = planes[i];
-        for (int s = 1; s < splits; s++) sum += planes[s * ny + i];
-        y[i] = residual ? residual[i] + sum : sum;
-    }
-    return ESP_OK;
+        g.w = m; g.x = d_x; g.y = d_y; g.residual = residual ? d_y : nullptr; g.rows = rows; g.unrounded = true; g.workspace = workspace; g.workspace_floats = kGemmWorkspaceFloats;
+        if (shares) g.deferred_splits = splits;
+        return launch_gemm(g, s);
+    });
+}
+
+int esp_step_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares) {
+    if (!matrix || !x_f16 || !y) return fail(ESP_ERR_INVALID_ARGUMENT, "step_product: null pointer");
+    if (rows <= 0) return fail(ESP_ERR_INVALID_ARGUMENT, "step_product: rows %d", rows);
+    const DeviceMatrix &m = matrix->m;
+    if (!gemv_takes_sixteen_rows(m, rows)) return fail(ESP_ERR_UNSUPPORTED, "step_product: %d rows of %d columns", rows, m.cols);
+    return product_for_test(m, x_f16, rows, y, residual, "step_product", [&](const uint16_t *d_x, float *d_y, float *workspace, int *splits, hipStream_t s) {
+        GemvParams g;
+        g.w = m; g.x = d_x; g.y = d_y; g.residual = residual ? d_y : nullptr; g.batch = rows; g.sixteen_rows = true; g.epilogue = residual ? EPI_ADD_RESIDUAL : EPI_STORE_F32;
+        if (shares) { g.workspace = workspace; g.workspace_floats = kGemmWorkspaceFloats; g.deferred_splits = splits; }
+        return launch_gemv(g, s);
+    });
 }
 
 int esp_matmul_f32(const ESPMatrix *matrix, const float *x, int rows, float *y, const float *residual) {

@@ -104,6 +104,14 @@ class Matrix:
         _lib.check(_lib.load_library().esp_layer_product(self._h, _ptr(x), rows, _ptr(y), _ptr(res) if res is not None else None, int(shares)))
         return y
 
+    def step_product(self, x_f16: np.ndarray, residual: np.ndarray | None = None, shares: bool = False) -> np.ndarray:
+        """The product as a step of up to sixteen sequences asks for it (esp_step_product; test aid)."""
+        x = np.ascontiguousarray(x_f16, dtype=np.float16).reshape(-1, self.cols)
+        y = np.empty((x.shape[0], self.rows), dtype=np.float32)
+        res = None if residual is None else np.ascontiguousarray(residual, dtype=np.float32).reshape(y.shape)
+        _lib.check(_lib.load_library().esp_step_product(self._h, _ptr(x), x.shape[0], _ptr(y), _ptr(res) if res is not None else None, int(shares)))
+        return y
+
     def layer_gate_up(self, x_f16: np.ndarray) -> np.ndarray:
         """SiLU(gate) * up of interleaved gate / up rows as a model's layers ask for it, fp16 (esp_layer_gate_up; test aid)."""
         x = np.ascontiguousarray(x_f16, dtype=np.float16).reshape(-1, self.cols)

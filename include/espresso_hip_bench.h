@@ -64,6 +64,8 @@ int esp_matmul_f32_swiglu(const ESPMatrix *matrix, const float *x, int rows, flo
  * shares = 1: the launch may leave its sum in shares of K, as in front of a norm or the key/value caches; they and the residual are then added here, in the shares' order.
  * y, residual (may be NULL) [rows][matrix rows] fp32; host pointers. */
 int esp_layer_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares);
+/* Test aid: the product as a step of up to sixteen sequences asks for it (matrices that such steps take in one launch; ESP_ERR_UNSUPPORTED for others); arguments as esp_layer_product. */
+int esp_step_product(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, float *y, const float *residual, int shares);
 /* Test aid: SiLU(gate) * up as the layers ask for it, of a matrix of interleaved gate / up rows (2i = gate_i, 2i + 1 = up_i), in the product's epilogue or by the launch that adds shares of K.
  * act_f16 [rows][matrix rows / 2] fp16; host pointers. */
 int esp_layer_gate_up(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, uint16_t *act_f16);

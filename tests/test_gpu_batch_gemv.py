@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import espresso_amd._lib as lib
+from test_gpu_block_gemm import check_kept, rms_off
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +43,52 @@ def test_batches_are_their_sequences(shape, kv):
         o.set_tuning("batch_gemv_form", 0)
         rt.close()
         one.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(515, 1024), (40, 2048), (272, 3072), (129, 4096), (96, 8192), (48, 14336)])
+def test_step_products_keep_their_weights(rows, cols):
+    """The product by itself against 64 bits, every number of row blocks and shares of K: no weight is rounded (fp16 ones would be 2e-4 off), rows that fill no block and no workgroup."""
+    import espresso_amd.ops as o
+    o.init()
+    m = o.Matrix(lib.FORMAT_Q4_K, o.synth_weights(lib.FORMAT_Q4_K, rows + cols, 0.02, rows * cols), rows, cols)
+    rng = np.random.default_rng(cols)
+    try:
+        for form in [0] + [10 * blocks + shares for blocks in range(1, 9) for shares in (1, 2, 4, 7)]:
+            o.set_tuning("batch_gemv_form", form)
+            check_kept(m, lambda x, r: m.step_product(x, r, shares=True), (3, 16) if form else (1, 3, 9, 15, 16), rng)
+            if form in (0, 31):
+                check_kept(m, lambda x, r: m.step_product(x, r), (3, 16), rng)
+    finally:
+        o.set_tuning("batch_gemv_form", 0)
+    m.close()
+
+
+@pytest.mark.parametrize("width", [1088, 4096, 4160, 8192])
+def test_norms_of_few_rows(width):
+    """Norms of up to 64 rows in 1024 threads, one and two fours of columns each, and of one row more: prompts, and steps of a batch, against the tokens one at a time, whose norms are in the products."""
+    import espresso_amd.llama as ll
+    import espresso_amd.ops as o
+    import espresso_amd.synthetic as syn
+    o.init()
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=4, n_kv_head=4, d_model=width, head_dim=64, hidden_dim=256, vocab=260, max_seq=128)
+    rt, _ = syn.build_runtime(cfg, lib.FORMAT_F16, seed=3, std=width ** -0.5, max_sequences=3)   # products as large as their inputs: scores of a few units, which carry no rounding further
+    tokens = np.random.default_rng(width).integers(0, 260, 65).astype(np.uint32)
+    steps = []
+    for t in tokens:
+        rt.advance(int(t))
+        steps.append(rt.logits())
+    for count in (64, 65):
+        rt.reset()
+        got = rt.append(tokens[:count], want=range(count))
+        # activations and contexts are fp16 in both, queries and softmax weights in blocks: 2^-12 of each at the root mean square, some ten of them in two layers, where a last bit may fall either way
+        assert rms_off(got, np.stack(steps[:count])) <= 2.0 ** -9, count
+    out, _ = ll.generate_batch(rt, [tokens[:40], tokens[:41], tokens[:42]], 4)
+    for s in range(3):
+        n = 40 + s + len(out[s])
+        rt.set_visible(n - 1, sequence=s)
+        b = rt.append(np.array(out[s][-1:], np.uint32), want=[0], sequence=s)[0]
+        rt.set_visible(0)
+        for t in list(tokens[:40 + s]) + out[s]:
+            rt.advance(int(t))
+        assert rms_off(b, rt.logits()) <= 2.0 ** -9, s
+    rt.close()
