@@ -38,12 +38,16 @@ static const DeviceSetup noalloc_scratch(noalloc_setup);
 }  // namespace esp
 
 // ---- staging of single products (esp_gemv) ------------------------------------------------------------------
-// A product of a few rows is 5 us of kernel; three allocations and frees, two pageable copies and their waits made 34 us of it.  One staging area for the process, there from the second product on
-// while any matrix handle is (a program that makes a handle for one product does without: made with the handle, 2048 x 2048 Q8_0 made, multiplied once and freed 870 us, 293 without; 768 x 768 168 and 89):
+// A product of a few rows is 5 us of kernel; three allocations and frees, two pageable copies and their waits made 34 us of it.  One staging area for the process, there from the 128th product on
+// while any matrix handle is:
 // pinned memory that takes the call's activations and residual, which a small kernel brings to the device (4 us less than a copy engine's start), and its result, which the product writes there itself.
 // A call that finds it in use by another thread, or that needs more, allocates as before.  4096 x 4096 Q4_K, 2 / 16 / 40 / 128 rows 34.8 / 88 / 116 / 256 -> 22.7 / 39 / 66 / 185 us, of which the
-// caller's Python is 2; 768 x 768 Q8_0, 512 rows 178 -> 133, with a residual 265 -> 205: as far as the area goes, results cross the bus faster than through a copy.
+// caller's Python is 2; 768 x 768 Q8_0, 512 rows 178 -> 133, with a residual 265 -> 205: as far as the area goes, results cross the bus faster than through a copy (86 products of f16, q8_0 and q4_k,
+// 768 x 768 to 32000 x 2048 and 1 to 512 rows: 0.35 to 0.77 times the time).
+// Why the 128th: the area's memory, made and given back, costs the program 0.1 to 0.9 ms (allocations of other sizes leave the runtime's cache with it: the next 2048 x 2048 matrix takes 531 us instead of
+// 223), and a product of one or two rows gains 11 us.  2048 x 2048 Q8_0 made, multiplied 2 / 10 / 60 times and freed, us: 320 / 566 / 2094 without the area, 890 / 1051 / 2082 with it from the second product.
 namespace {
+constexpr int kProductsBefore = 128;
 constexpr size_t kStagedIn = (size_t)1 << 20, kStagedOut = (size_t)4 << 20;   // bytes of activations and of residual or result
 class Staging {
   public:
@@ -62,7 +66,7 @@ class Staging {
     // whether a call (of the holder of the mutex) is staged; without memory none is until the last handle has gone
     bool takes(size_t in, size_t out) {
         if (in > kStagedIn || out > kStagedOut) return false;
-        if (products_ < 2 && ++products_ == 2) allocate();
+        if (products_ < kProductsBefore && ++products_ == kProductsBefore) allocate();
         return host_ != nullptr;
     }
     // two regions: activations; the residual, and in its place the result, which comes when the residual is on the device
@@ -92,7 +96,7 @@ class Staging {
         planes_ = nullptr;
     }
     std::mutex handles_mutex_, mutex_;   // of the count, and of the memory while a call uses it
-    int handles_ = 0, products_ = 0;     // products_: that could be staged, up to two
+    int handles_ = 0, products_ = 0;     // products_: that could be staged, up to kProductsBefore
     uint8_t *host_ = nullptr, *mapped_ = nullptr, *device_ = nullptr;
     float *planes_ = nullptr;
 };

@@ -34,9 +34,22 @@ def check(m, w, batch, seed, residual):
     assert (np.abs(m.gemv(x, r) - want) <= bound).all(), (batch, residual)
 
 
+PRODUCTS_BEFORE = 128   # that a program makes before the area is worth its memory
+
+
+@pytest.fixture()
+def area(ops):
+    """The area is there for as long as this matrix is."""
+    m, _ = matrix(ops, 16, 8, 0)
+    for _ in range(PRODUCTS_BEFORE):
+        m.gemv(np.zeros((1, 8), np.float16))
+    yield m
+    m.close()
+
+
 # 1 MiB of activations is 1024 rows of 512 columns, 4 MiB of results 1024 rows of 1024
 @pytest.mark.parametrize("rows,cols,batches", [(24, 8, (1, 2, 5)), (70, 512, (1, 3, 1024, 1025)), (1024, 64, (2, 1024, 1025)), (1023, 72, (7,))])
-def test_every_size_takes_its_way(ops, rows, cols, batches):
+def test_every_size_takes_its_way(ops, area, rows, cols, batches):
     m, w = matrix(ops, rows, cols, rows)
     for batch in batches:
         for residual in (False, True):
@@ -44,7 +57,10 @@ def test_every_size_takes_its_way(ops, rows, cols, batches):
     m.close()
 
 
-def test_threads_and_handles(ops):
+@pytest.mark.parametrize("held", [False, True])
+def test_threads_and_handles(ops, held, request):
+    if held:
+        request.getfixturevalue("area")
     failures = []
 
     def work(seed):
@@ -66,7 +82,7 @@ def test_threads_and_handles(ops):
 
 
 def test_a_handle_leaves_the_last_error(ops):
-    """A matrix that is made, the first of its process or not, is no failure: the most recent one stays what it was."""
+    """A matrix that is made and multiplied, whether or not the area comes with it, is no failure: the most recent one stays what it was."""
     m, _ = matrix(ops, 32, 64, 1)
     with pytest.raises(lib.EspressoError, match="layer_product: rows 0"):
         m.layer_product(np.zeros((0, 64), np.float16))
@@ -74,14 +90,15 @@ def test_a_handle_leaves_the_last_error(ops):
     said = lib.last_error()
     other, w = matrix(ops, 32, 64, 2)
     assert lib.last_error() == said and "layer_product" in said
-    check(other, w, 2, 3, True)
+    for _ in range(PRODUCTS_BEFORE):
+        check(other, w, 2, 3, True)
     assert lib.last_error() == said
     other.close()
     assert lib.last_error() == said
 
 
-def test_the_area_comes_with_the_second_product_and_goes_with_the_last_handle(ops):
-    """A handle made for one product costs what it did without the area (21 MiB of device memory, 5 of pinned)."""
+def test_the_area_comes_when_products_have_paid_for_it_and_goes_with_the_last_handle(ops):
+    """Handles made for a few products cost what they did without the area (21 MiB of device memory, 5 of pinned)."""
     gc.collect()   # handles of other tests
     with open("/proc/self/maps") as f:
         hip = ctypes.CDLL(re.search(r"/\S*libamdhip64\.so\S*", f.read()).group(0))
@@ -95,19 +112,21 @@ def test_the_area_comes_with_the_second_product_and_goes_with_the_last_handle(op
         return held(since) / 2 ** 20
 
     m, w = matrix(ops, 32, 64, 1)
-    check(m, w, 2, 3, True)   # whatever the first products of a process allocate for good
-    check(m, w, 2, 3, True)
+    for _ in range(PRODUCTS_BEFORE + 1):
+        check(m, w, 2, 3, True)   # whatever the first products of a process allocate for good
     m.close()
     start = -held(0)
     for _ in range(3):
         m, w = matrix(ops, 32, 64, 1)
-        check(m, w, 2, 3, True)
+        for _ in range(PRODUCTS_BEFORE - 1):
+            check(m, w, 2, 3, True)
         assert mebibytes(start) < 16
         m.close()
     a, w = matrix(ops, 32, 64, 1)
     b, _ = matrix(ops, 32, 64, 2)
-    for batch in (2, 5, 2):
-        check(a, w, batch, 3, True)
+    for i in range(PRODUCTS_BEFORE):
+        assert mebibytes(start) < 16
+        check(a, w, (2, 5, 2)[i % 3], 3, True)
     assert mebibytes(start) >= 16
     a.close()
     assert mebibytes(start) >= 16
