@@ -7,7 +7,8 @@
 //     of their own, so that a lane's two 128-bit reads are free of bank conflicts) and then walks units of weight rows: two rows per
 //     wavefront (four leave the last round of workgroups half empty), one at the output side, which has too few rows to give every compute unit work;
 //   * four steps of every row are in flight from the launch's first instructions on: requested behind the activations, whose loads are waited for without them, and across units;
-//     rows are padded to whole turns of four, with a remainder every turn waits for all that is in flight.  Before, weights were first asked for when the activations were staged; us, weights that
+//     rows are padded to whole turns of four, with a remainder every turn waits for all that is in flight.  (Where the padding is longest it costs less than the ring gains: steps of six layers of 2560 / 5120 columns,
+//     3 and 2 of 8 and 12 steps of padding in the input products, 349 -> 303 and 884 -> 828 us, Forovik's 271 -> 254 and 655 -> 601.)  Before, weights were first asked for when the activations were staged; us, weights that
 //     no cache holds: input 24576 x 2048 22.1 -> 19.3, 16384 x 2048 16.3 -> 13.6, 10368 x 2048 10.1 -> 9.6, 45056 x 4096 70 -> 62 (5.9 TB/s);  output 2048 x 10240 with retention's heads 12.7 ->
 //     9.9, 2048 x 4096 by parts 8.2 -> 6.6, 2048 x 2048 4.4 -> 4.05, 4096 x 18432 32 -> 28;  head 32000 x 2048 26.9 -> 23.9.  What is left is the launch, the activations' trip and their staging (3 us);
 //   * what surrounds the product lives in the staging and the epilogue: RMS norm (its scale factors out of the dot product), the
