@@ -15,9 +15,9 @@ namespace esp {
 class LlamaRuntime;
 class LayeredRuntime;
 
-// Rows of a prompt block: a whole prompt of up to 2048 tokens, so that its products have several rounds of workgroups (one block against blocks of 512, us: 1777 tokens of 3B Q4_K 22510 ->
-// 18770, 1500 of eight layers of 8B 14160 -> 13660, 1100 of 1B Q8_0 6830 -> 4650, 1700 of 30 layers of 576 columns in Q4_0 8910 -> 4040, 1700 of six Ranavik layers of 4096 columns 9920 ->
-// 7970); contexts that hold fewer take what they hold, and no runtime's blocks are shorter than 512.
+// Rows of a prompt block: a whole prompt of up to 2048 tokens, so that its products have several rounds of workgroups (blocks of 512 -> one block, us: 1777 tokens of 3B Q4_K 20960 ->
+// 16200, 1500 of eight layers of 8B 12580 -> 12150, 1100 of 1B Q8_0 6510 -> 4440, 1777 of 1.1B Q8_0 10930 -> 7160, 1700 of 30 layers of 576 columns in Q4_0 7250 -> 3570, 1700 of six Ranavik layers of
+// 4096 columns 8150 -> 6230; as exact as blocks of 512: LlamaRuntime::last_rows, kExactRows); contexts that hold fewer take what they hold, and no runtime's blocks are shorter than 512.
 constexpr int kMinPrefillBlockRows = 512, kMaxPrefillBlockRows = 2048;
 inline int prefill_block_rows(int max_seq) {
     const int rows = max_seq > kMaxPrefillBlockRows ? kMaxPrefillBlockRows : (max_seq + 127) / 128 * 128;
