@@ -425,7 +425,7 @@ int esp_block_attention(int kernel, const float *q, const void *k, const void *v
     if (split_rows) { a.ctx_hi = d_hi; a.ctx_lo = d_lo; a.ctx_sums = d_sums; }
     else a.ctx_f16 = d_hi;
     auto launch = [&] {
-        if (kernel == ESP_ATTENTION_PROMPT) return launch_attention_prompt(a, rows, kv_f16 != 0, c.stream);
+        if (kernel == ESP_ATTENTION_PROMPT) return launch_prompt_attention(a, rows, a.max_seq, kv_f16 != 0, c.stream);
         if (kernel == ESP_ATTENTION_SPAN) return launch_span_attention(a, rows, a.max_seq, kv_f16 != 0, c.stream);
         return launch_attention(a, rows, kv_f16 != 0, c.stream);
     };

@@ -49,8 +49,8 @@ struct AttentionArgs {
     float *split_scratch;
     // partial results of attention_partial_kernel: [rows][heads][attention_head_splits][head_dim + 4] floats
     float *head_partials;
-    // launch_attention_prompt and launch_span_attention only, all three or none: the context as split rows (hi = fp16(v), lo = fp16((v - hi) * 2048),
-    // sub-block sums; SplitRowsView) instead of ctx_f16, with the queries and the softmax weights split the same way
+    // launch_span_attention only, all three or none: the context as split rows (hi = fp16(v), lo = fp16((v - hi) * 2048),
+    // sub-block sums; SplitRowsView) instead of ctx_f16
     uint16_t *ctx_hi, *ctx_lo, *ctx_sums;
     // launch_attention_prompt and launch_span_attention only, optional: (first row, rows - 1) of each tile, none of which holds rows of two sequences, instead of every 32 rows of one sequence
     const int2 *tiles;
@@ -71,9 +71,9 @@ hipError_t launch_rmsnorm_reduce(const float *partial, int splits, size_t plane,
 hipError_t launch_qkv_post(const QkvPostArgs &a, int rows, bool kv_f16, hipStream_t s);
 hipError_t launch_attention(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s);
 // Causal attention of `rows` rows that are ONE sequence at consecutive positions (a prompt block), on the matrix cores.
-// Head dim 64 or 128, 1, 2 or 4 query heads per KV head (attention_prompt_supported); Q, K, V, P as fp16, fp32 sums.
+// Head dim 64 or 128, 1, 2 or 4 query heads per KV head (attention_prompt_supported), 32-bit caches; Q, K, V, P as fp16, fp32 sums.
 bool attention_prompt_supported(int n_head, int n_kv_head, int head_dim);
-hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s);
+hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, hipStream_t s);
 // Attention that stops at per-split partial states (head_dim 64 or 128, up to kMaxStepRows rows); the GEMV that reads
 // the context merges them (GemvParams::merge_partials).  attention_head_splits: slices per query head.
 int attention_head_splits(int max_seq);

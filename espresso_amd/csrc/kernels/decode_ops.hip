@@ -498,8 +498,8 @@ __global__ __launch_bounds__(HD) void attention_merge_kernel(AttentionArgs a, in
 // sequence at consecutive positions (pos[m0 + i] = pos[m0] + i), which is what a prompt block is.  Replaces the per-row
 // loop of the reference's attention (:6774-6823) over a block: the single-query kernels above read a row's whole prefix
 // once per row, this one reads a key tile once per 32 rows.
-// grid (KV heads, tiles of 32 rows, sets of G query heads); wavefront g of a workgroup serves query head kvh * group + G z + g,
-// so G heads that share a KV head share the value tiles.  Per tile of 32 keys:
+// 32-bit caches alone: fp16 ones have span_attention.hip, as exact as 32 bits and no slower.
+// grid (KV heads, tiles of 32 rows); wavefront g of a workgroup serves query head kvh * G + g, so the G heads that share a KV head share the value tiles.  Per tile of 32 keys:
 //   * S^T = K Q^T: keys are the A rows (a lane loads eight consecutive dims of its key straight from the cache, two
 //     tiles ahead), queries the B columns (fragments kept in registers); a lane's 16 accumulators are
 //     16 keys of ONE query, so the row maximum and sum of the online softmax are in-lane plus one exchange with lane ^ 32;
@@ -507,31 +507,23 @@ __global__ __launch_bounds__(HD) void attention_merge_kernel(AttentionArgs a, in
 //     the A operand is the value tile transposed in LDS (written once per workgroup, double-buffered: one barrier per tile),
 //     read so that k slot (lane / 32, i) is key 16 j + 8 (i / 4) + 4 (lane / 32) + i % 4, the key of accumulator 8 j + i.
 // Q, K, V and the probabilities enter the matrix cores as fp16, sums are fp32.
-// SPLIT: queries and probabilities go in as hi / lo pairs (v = hi + lo / 2048: two MFMAs each against the same keys / values, which
-// the fp16 cache holds exactly), and the context comes out as split rows for the GEMM that consumes it.
 typedef _Float16 attn_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 attn_half4 __attribute__((ext_vector_type(4)));
 typedef float attn_floatx16 __attribute__((ext_vector_type(16)));
 
-// KP = 2: the workgroup has two sets of G wavefronts; set p takes the key tiles p, p + 2, ... with value tiles of its own, and the two
-// (maximum, sum, context) states of a head are merged through LDS at the end.  A workgroup's time is the length of its chain of key
-// tiles (a tile of arithmetic is shorter than the trip to memory behind it), and the last row tile of a 512-row block has sixteen.
 // Heads of 64 dims ask for two wavefronts per SIMD: without it the compiler spreads over accumulator registers past what two share (512 rows of 32
 // heads behind 512, split rows: 49 us, 44 with it).
-template <int HD, int G, bool KV_F16, bool SPLIT, int KP>
-__global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_prompt_kernel(AttentionArgs a, int rows) {
-    constexpr int THREADS = G * 64, QT = 32, KS = HD / 16, MTILES = HD / 32, LDV = 32 + 8;   // THREADS: of one set; LDV: fp16 per row of V^T
+template <int HD, int G>
+__global__ __launch_bounds__(G * 64, HD == 64 ? 2 : 1) void attention_prompt_kernel(AttentionArgs a, int rows) {
+    constexpr int THREADS = G * 64, QT = 32, KS = HD / 16, MTILES = HD / 32, LDV = 32 + 8;   // LDV: fp16 per row of V^T
     constexpr int VP = 32 * (HD / 8) / THREADS;                                            // 8-dim pieces of V per thread
-    static_assert(VP >= 1 && 32 * (HD / 8) % THREADS == 0, "value tile divides over a set of wavefronts");
-    static_assert(KP == 1 || KP == 2, "one or two sets");
-    __shared__ _Float16 vt_all[KP][2][HD * LDV];
+    static_assert(VP >= 1 && 32 * (HD / 8) % THREADS == 0, "value tile divides over the wavefronts");
+    __shared__ _Float16 vt[2][HD * LDV];
     asm volatile("" ::"s"(a.tiles), "s"(a.pos), "s"(a.seq), "s"(a.q), "s"(a.k_cache), "s"(a.v_cache));   // fetched together, ahead of the branch
     const int2 tile = a.tiles ? a.tiles[blockIdx.y] : int2{(int)blockIdx.y * QT, rows - 1 - (int)blockIdx.y * QT};
     const int kvh = blockIdx.x, m0 = tile.x;
-    const int phase = KP == 1 ? 0 : (int)threadIdx.x / THREADS;
-    const int tid = (int)threadIdx.x - phase * THREADS, lane = tid & 63, wave = tid >> 6, half = lane >> 5, col = lane & 31;
-    _Float16 (*vt)[HD * LDV] = vt_all[phase];
-    const int head = kvh * (a.n_head / a.n_kv_head) + (int)blockIdx.z * G + wave;   // grid z: sets of G query heads of the KV head
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, col = lane & 31;
+    const int head = kvh * G + wave;
     const int pos0 = a.pos[m0];
     const int last_row = tile.y < QT - 1 ? tile.y : QT - 1;
     const int t_max = pos0 + last_row;             // last key any row of the tile sees
@@ -543,18 +535,13 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
         return attn_half8{(_Float16)x0.x, (_Float16)x0.y, (_Float16)x0.z, (_Float16)x0.w, (_Float16)x1.x, (_Float16)x1.y, (_Float16)x1.z, (_Float16)x1.w};
     };
     // query fragments: column = query `col` (rows beyond the block repeat its last row, never stored), dims 16 ks + 8 half ..
-    attn_half8 qf[KS], ql[SPLIT ? KS : 1];
+    attn_half8 qf[KS];
     {
         const float *qp = a.q + (size_t)(m0 + (col <= last_row ? col : last_row)) * a.n_head * HD + (size_t)head * HD + 8 * half;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const float4 x0 = *reinterpret_cast<const float4 *>(qp + 16 * ks), x1 = *reinterpret_cast<const float4 *>(qp + 16 * ks + 4);
             qf[ks] = to_half8(x0, x1);
-            if constexpr (SPLIT) {
-                const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-                for (int e = 0; e < 8; e++) ql[ks][e] = (_Float16)__fmul_rn(__fsub_rn(v[e], (float)qf[ks][e]), 2048.0f);
-            }
         }
     }
     // keys beyond t_max are clamped to it: in bounds, and masked below
@@ -563,11 +550,8 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
         const size_t off = seq_base + (size_t)t * kd + (size_t)kvh * HD + 8 * half;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            if (KV_F16) kf[ks] = *reinterpret_cast<const attn_half8 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + off + 16 * ks);
-            else {
-                const float *kp = reinterpret_cast<const float *>(a.k_cache) + off + 16 * ks;
-                kf[ks] = to_half8(*reinterpret_cast<const float4 *>(kp), *reinterpret_cast<const float4 *>(kp + 4));
-            }
+            const float *kp = reinterpret_cast<const float *>(a.k_cache) + off + 16 * ks;
+            kf[ks] = to_half8(*reinterpret_cast<const float4 *>(kp), *reinterpret_cast<const float4 *>(kp + 4));
         }
     };
     // value tile: piece = (key, group of eight dims); consecutive lanes take consecutive keys so that the transposed
@@ -578,11 +562,8 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
             const int piece = tid + i * THREADS, key = piece & 31, dg = piece >> 5;
             const int t = t0 + key < t_max ? t0 + key : t_max;
             const size_t off = seq_base + (size_t)t * kd + (size_t)kvh * HD + 8 * dg;
-            if (KV_F16) vreg[i] = *reinterpret_cast<const attn_half8 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + off);
-            else {
-                const float *vp = reinterpret_cast<const float *>(a.v_cache) + off;
-                vreg[i] = to_half8(*reinterpret_cast<const float4 *>(vp), *reinterpret_cast<const float4 *>(vp + 4));
-            }
+            const float *vp = reinterpret_cast<const float *>(a.v_cache) + off;
+            vreg[i] = to_half8(*reinterpret_cast<const float4 *>(vp), *reinterpret_cast<const float4 *>(vp + 4));
         }
     };
     auto store_v = [&](int buf, const attn_half8 (&vreg)[VP]) {
@@ -594,46 +575,31 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
         }
     };
 
-    attn_floatx16 o[MTILES], ol[SPLIT ? MTILES : 1];
+    attn_floatx16 o[MTILES];
 #pragma unroll
     for (int mt = 0; mt < MTILES; mt++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[mt][r] = 0.0f;
-#pragma unroll
-    for (int mt = 0; mt < (SPLIT ? MTILES : 1); mt++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) ol[mt][r] = 0.0f;
     float mx = -INFINITY, l = 0.0f;
     const int qpos = pos0 + col;
 
     // Keys and values are fetched two tiles ahead: one tile of arithmetic is shorter than a trip to memory.
-    constexpr int STEP = 32 * KP;   // keys between a set's tiles
     attn_half8 kf[KS], k1[KS], k2[KS], v1[VP], v2[VP];
-    load_k(32 * phase, kf);
-    load_v(32 * phase, v1);
+    load_k(0, kf);
+    load_v(0, v1);
     store_v(0, v1);
-    load_k(32 * phase + STEP, k1);      // tiles beyond t_max are clamped to it, in bounds and masked
-    load_v(32 * phase + STEP, v1);
+    load_k(32, k1);      // tiles beyond t_max are clamped to it, in bounds and masked
+    load_v(32, v1);
     __syncthreads();
-    for (int base = 0, buf = 0; base <= t_max; base += STEP, buf ^= 1) {   // the same number of rounds for both sets
-        const int t0 = base + 32 * phase;
-        const bool more = base + STEP <= t_max;
-        load_k(t0 + 2 * STEP, k2);
-        load_v(t0 + 2 * STEP, v2);
+    for (int t0 = 0, buf = 0; t0 <= t_max; t0 += 32, buf ^= 1) {
+        const bool more = t0 + 32 <= t_max;
+        load_k(t0 + 64, k2);
+        load_v(t0 + 64, v2);
         attn_floatx16 sc;
 #pragma unroll
         for (int r = 0; r < 16; r++) sc[r] = 0.0f;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qf[ks], sc, 0, 0, 0);
-        if constexpr (SPLIT) {
-            attn_floatx16 sl;
-#pragma unroll
-            for (int r = 0; r < 16; r++) sl[r] = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], ql[ks], sl, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; r++) sc[r] = __builtin_fmaf(sl[r], 1.0f / 2048.0f, sc[r]);
-        }
         // accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`
         float tile_max = -INFINITY;
 #pragma unroll
@@ -643,44 +609,30 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
             tile_max = fmaxf(tile_max, sc[r]);
         }
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-        // finite from the first tile on in set 0 (key 0 is visible to every query); set 1 may see only masked keys for a while:
-        // its state then stays (-inf, 0, 0) (exponents taken against 0 instead of -inf)
-        const float m_new = fmaxf(mx, tile_max);
-        const float m_ref = (KP > 1 && m_new == -INFINITY) ? 0.0f : m_new;
-        const float alpha = __expf(mx - m_ref);      // exp(-inf) = 0 on the first tile
+        const float m_new = fmaxf(mx, tile_max);     // finite from the first tile on: key 0 is visible to every query
+        const float alpha = __expf(mx - m_new);      // exp(-inf) = 0 on the first tile
         float psum = 0.0f;
-        _Float16 ph[16], pl[SPLIT ? 16 : 1];
+        _Float16 ph[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const float pr = __expf(sc[r] - m_ref);  // masked keys: exp(-inf) = 0
+            const float pr = __expf(sc[r] - m_new);  // masked keys: exp(-inf) = 0
             psum += pr;
             ph[r] = (_Float16)pr;
-            if constexpr (SPLIT) pl[r] = (_Float16)__fmul_rn(__fsub_rn(pr, (float)ph[r]), 2048.0f);
         }
         l = __builtin_fmaf(l, alpha, psum);
         mx = m_new;
         const attn_half8 pf[2] = {attn_half8{ph[0], ph[1], ph[2], ph[3], ph[4], ph[5], ph[6], ph[7]},
                                   attn_half8{ph[8], ph[9], ph[10], ph[11], ph[12], ph[13], ph[14], ph[15]}};
-        attn_half8 pfl[2];
-        if constexpr (SPLIT) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) { pfl[0][e] = pl[e]; pfl[1][e] = pl[8 + e]; }
-        }
 #pragma unroll
         for (int mt = 0; mt < MTILES; mt++) {
 #pragma unroll
             for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
-            if constexpr (SPLIT) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) ol[mt][r] *= alpha;
-            }
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const _Float16 *vrow = vt[buf] + (32 * mt + col) * LDV + 16 * j + 4 * half;
                 const attn_half4 lo = *reinterpret_cast<const attn_half4 *>(vrow), hi = *reinterpret_cast<const attn_half4 *>(vrow + 8);
                 const attn_half8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                 o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[j], o[mt], 0, 0, 0);
-                if constexpr (SPLIT) ol[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pfl[j], ol[mt], 0, 0, 0);
             }
         }
         if (more) store_v(buf ^ 1, v1);
@@ -690,70 +642,15 @@ __global__ __launch_bounds__(G * KP * 64, HD == 64 ? 2 : 1) void attention_promp
         for (int i = 0; i < VP; i++) v1[i] = v2[i];
         __syncthreads();
     }
-    if constexpr (KP == 2) {
-        // set 1 hands (maximum, sum, context) to set 0 through the value tiles' LDS, 32 dims at a time: [wave][value][lane]
-        float *mb = reinterpret_cast<float *>(&vt_all[0][0][0]);
-        constexpr int kPerWave = (SPLIT ? 32 : 16) * 64, kStateBase = G * kPerWave;
-        static_assert((size_t)(kStateBase + G * 2 * 64) * 4 <= sizeof(vt_all), "the merge fits the value tiles");
-        float f0 = 1.0f, f1 = 0.0f;
-        if (phase == 1) { mb[kStateBase + (wave * 2) * 64 + lane] = mx; mb[kStateBase + (wave * 2 + 1) * 64 + lane] = l; }
-#pragma unroll
-        for (int mt = 0; mt < MTILES; mt++) {
-            if (phase == 1) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    mb[wave * kPerWave + r * 64 + lane] = o[mt][r];
-                    if constexpr (SPLIT) mb[wave * kPerWave + (16 + r) * 64 + lane] = ol[mt][r];
-                }
-            }
-            __syncthreads();
-            if (phase == 0) {
-                if (mt == 0) {
-                    const float m1 = mb[kStateBase + (wave * 2) * 64 + lane], l1 = mb[kStateBase + (wave * 2 + 1) * 64 + lane];
-                    const float m_all = fmaxf(mx, m1);   // finite: set 0 saw key 0
-                    f0 = __expf(mx - m_all); f1 = __expf(m1 - m_all);
-                    l = __builtin_fmaf(l, f0, __fmul_rn(l1, f1));
-                }
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    o[mt][r] = __builtin_fmaf(o[mt][r], f0, __fmul_rn(mb[wave * kPerWave + r * 64 + lane], f1));
-                    if constexpr (SPLIT) ol[mt][r] = __builtin_fmaf(ol[mt][r], f0, __fmul_rn(mb[wave * kPerWave + (16 + r) * 64 + lane], f1));
-                }
-            }
-            __syncthreads();
-        }
-        if (phase == 1) return;
-    }
     l += __shfl_xor(l, 32);
     // A masked key takes part with weight 0, and fp16 ends at 65504: where something was not finite, the rows once more from the keys they see alone
     float check = 0.0f;
 #pragma unroll
     for (int mt = 0; mt < MTILES; mt++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) check = __builtin_fmaf(SPLIT ? o[mt][r] + ol[mt][r] : o[mt][r], 0.0f, check);
+        for (int r = 0; r < 16; r++) check = __builtin_fmaf(o[mt][r], 0.0f, check);
     if (__any(!(check == 0.0f && l < INFINITY))) {
-        for (int i = 0; i <= last_row; i++) plain_attention_row<HD, KV_F16>(a, m0 + i, head);
-        return;
-    }
-    if constexpr (SPLIT) {
-        // context = (o + ol / 2048) / l as split rows; dims 32 mt .. 32 mt + 31 of a head are one sub-block of the row, half of it in
-        // this lane and half in lane ^ 32
-        const float inv = 1.0f / l;
-        const size_t row = (size_t)(m0 + (col <= last_row ? col : last_row));
-        const int ad = a.n_head * HD;
-#pragma unroll
-        for (int mt = 0; mt < MTILES; mt++) {
-            float s = 0.0f;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = __fmul_rn(__builtin_fmaf(ol[mt][4 * q4 + e], 1.0f / 2048.0f, o[mt][4 * q4 + e]), inv);
-                if (col <= last_row) s += store_context4(a, row * ad + (size_t)head * HD + 32 * mt + 8 * q4 + 4 * half, v);
-            }
-            s += __shfl_xor(s, 32);
-            if (half == 0 && col <= last_row) store_context_sum(a, row, ad, head * (HD / 32) + mt, s);
-        }
+        for (int i = 0; i <= last_row; i++) plain_attention_row<HD, false>(a, m0 + i, head);
         return;
     }
     if (col <= last_row) {
@@ -1549,52 +1446,22 @@ bool attention_prompt_supported(int n_head, int n_kv_head, int head_dim) {
 }
 
 template <int HD, int G>
-hipError_t launch_attention_prompt_shape(const AttentionArgs &a, int rows, bool kv_f16, int key_sets, hipStream_t s) {
-    const int tiles = a.tiles ? a.tile_count : (rows + 31) / 32;
-    dim3 grid(a.n_kv_head, tiles);
-    // Two sets of wavefronts per workgroup (alternate key tiles) for 128-dim heads: the workgroup keeps its size (the kernel needs more
-    // than 256 registers, one wavefront per SIMD), so half of the KV head's query heads go to a second workgroup (grid z).
-    constexpr bool kTwoSets = HD == 128;
-    constexpr int GS = G >= 2 ? G / 2 : 1;
-    dim3 grid2(a.n_kv_head, tiles, G / GS);
-    if (a.ctx_hi) {   // split rows out: fp16 caches only (they hold keys and values exactly)
-        if (!kv_f16 || !a.ctx_lo || !a.ctx_sums || (a.n_head * HD) % 256 != 0) return hipErrorInvalidValue;
-        if constexpr (kTwoSets) {
-            if (key_sets == 2) {
-                hipLaunchKernelGGL((attention_prompt_kernel<HD, GS, true, true, 2>), grid2, dim3(GS * 128), 0, s, a, rows);
-                return hipGetLastError();
-            }
-        }
-        hipLaunchKernelGGL((attention_prompt_kernel<HD, G, true, true, 1>), grid, dim3(G * 64), 0, s, a, rows);
-        return hipGetLastError();
-    }
-    if constexpr (kTwoSets) {
-        if (key_sets == 2 && kv_f16) {
-            hipLaunchKernelGGL((attention_prompt_kernel<HD, GS, true, false, 2>), grid2, dim3(GS * 128), 0, s, a, rows);
-            return hipGetLastError();
-        }
-    }
-    if (kv_f16) hipLaunchKernelGGL((attention_prompt_kernel<HD, G, true, false, 1>), grid, dim3(G * 64), 0, s, a, rows);
-    else hipLaunchKernelGGL((attention_prompt_kernel<HD, G, false, false, 1>), grid, dim3(G * 64), 0, s, a, rows);
+hipError_t launch_attention_prompt_shape(const AttentionArgs &a, int rows, hipStream_t s) {
+    hipLaunchKernelGGL((attention_prompt_kernel<HD, G>), dim3(a.n_kv_head, a.tiles ? a.tile_count : (rows + 31) / 32), dim3(G * 64), 0, s, a, rows);
     return hipGetLastError();
 }
 
-// 0 (default): two sets of wavefronts for blocks of more than 64 rows; 1 / 2: always that many (tests, measurements)
-static int g_prompt_attention_key_sets = 0;
-void attention_prompt_set_key_sets(int sets) { g_prompt_attention_key_sets = sets == 1 || sets == 2 ? sets : 0; }
-
-hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s) {
-    if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !attention_prompt_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
+hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, hipStream_t s) {
+    if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !attention_prompt_supported(a.n_head, a.n_kv_head, a.head_dim) || a.ctx_hi) return hipErrorInvalidValue;
     const int group = a.n_head / a.n_kv_head;
-    const int sets = g_prompt_attention_key_sets ? g_prompt_attention_key_sets : (rows > 64 ? 2 : 1);
     if (a.head_dim == 128) {
-        if (group == 1) return launch_attention_prompt_shape<128, 1>(a, rows, kv_f16, sets, s);
-        if (group == 2) return launch_attention_prompt_shape<128, 2>(a, rows, kv_f16, sets, s);
-        return launch_attention_prompt_shape<128, 4>(a, rows, kv_f16, sets, s);
+        if (group == 1) return launch_attention_prompt_shape<128, 1>(a, rows, s);
+        if (group == 2) return launch_attention_prompt_shape<128, 2>(a, rows, s);
+        return launch_attention_prompt_shape<128, 4>(a, rows, s);
     }
-    if (group == 1) return launch_attention_prompt_shape<64, 1>(a, rows, kv_f16, sets, s);
-    if (group == 2) return launch_attention_prompt_shape<64, 2>(a, rows, kv_f16, sets, s);
-    return launch_attention_prompt_shape<64, 4>(a, rows, kv_f16, sets, s);
+    if (group == 1) return launch_attention_prompt_shape<64, 1>(a, rows, s);
+    if (group == 2) return launch_attention_prompt_shape<64, 2>(a, rows, s);
+    return launch_attention_prompt_shape<64, 4>(a, rows, s);
 }
 
 int attention_head_splits(int) { return kAttentionHeadSplits; }

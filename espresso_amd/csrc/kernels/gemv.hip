@@ -41,6 +41,7 @@
 #include "block_split.h"
 #include "wide_split.h"
 #include "rows_gemm.h"
+#include "span_attention.h"
 
 #include <hip/hip_ext.h>
 #include "gemv_device.h"

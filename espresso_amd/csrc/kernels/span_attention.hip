@@ -1,10 +1,9 @@
-// Causal attention of a prompt block on the matrix cores with 32-bit arithmetic, for any number of query heads per key/value head: the
-// block form of models whose heads attention_prompt_kernel (decode_ops.hip) is not written for (three or eight query heads per key/value
-// head, say), and of short blocks that must be as exact as the single-row steps.
+// Causal attention of a prompt block on the matrix cores with 32-bit arithmetic, for any number of query heads per key/value head: every block of models with fp16 caches, and with 32-bit caches the
+// blocks of head groups that attention_prompt_kernel (decode_ops.hip) is not written for and short blocks that must be as exact as the single-row steps.
 //
 // grid (query heads, tiles of 32 rows); a workgroup is KP wavefronts that share the 32 queries (in LDS) and deal the tiles of 32 keys
 // among themselves (wavefront p takes tiles p, p + KP, ...).  A wavefront runs by itself from its first tile to its last, without a barrier; the
-// KP states (maximum, sum, context) are merged pairwise through LDS at the end.  KP fills the chip where heads x row tiles do not
+// KP states (maximum, sum, context) meet in LDS at the end, where each wavefront finishes a share of the dims.  KP fills the chip where heads x row tiles do not
 // (launch_span_attention).
 //   * S^T = K Q^T and O^T += V^T P on 32 x 32 tiles: keys are the A rows, queries the B columns, so a lane's 16 accumulators are 16 keys of
 //     one query, and its softmax weights are the B operand of the second product as they are.
@@ -12,29 +11,75 @@
 //     is free as long as both operands agree); values come straight from memory, 32 dims of one key per half wavefront.  Bound by those
 //     products: 8192 cycles per tile of 128 dims.
 //   * fp16 caches hold keys and values exactly, so only the fp32 operands are split, each into three fp16 parts that add up to its 24 bits: a query scaled
-//     by a power of two that takes its largest value to 2^14..2^15, a softmax weight times 2^15 (parts end at 2^-25, so what they leave is below
-//     2^-39 of the largest).  Three v_mfma_f32_32x32x16_f16 into one fp32 sum take 96 cycles where the fp32 form takes 512.
+//     by a power of two that takes its largest value to 2^14..2^15, a softmax weight times 2^15 (parts end at 2^-24, so what they leave is below
+//     2^-38 of the largest).  Three v_mfma_f32_32x32x16_f16 into one fp32 sum take 96 cycles where the fp32 form takes 512.  Values go through LDS as rows, whose transposed reads
+//     (ds_read_b64_tr_b16) are the A operand.
 // A row whose result is not finite is done again from the keys it sees alone (plain_attention_row).
-// 512 rows of 24 heads of 128 (8 key/value heads) behind 1024: 58 us with fp16 caches, 137 with fp32 ones; row by row 780 (fp16).  Pairs of fp16 parts
-// (22 bits) in the place of the three took 53 and 98, but were less exact than the row by row kernel.
+// What bounds it (fp16 caches, 128 dims, a tile): 48 products, 0.78 us of a SIMD at the 2 GHz that the chip holds with all of them at work, beside 200 vector instructions: 1.5 us with two wavefronts a
+// SIMD; and a workgroup's way in and out, 9 us of 30 at 1777 rows.  Transposed two-byte writes of values, exponentials with a correction term, parts by rounding conversions, every wavefront reading every
+// query for its exponent and states handed on pairwise took: 1777 rows of 24 heads (8 key/value heads) 100 -> 79 us, 512 rows 21.6 -> 15.6, 93 rows of 32 heads of 64 behind 700 15.0 -> 10.4.  Against
+// attention_prompt_kernel with fp16 operands (and with pairs of them, inside a model), 32 heads, 8 key/value heads: 128 dims, 64 / 512 / 1500 rows 10.2 / 20.4 (38) / 93 (182) -> 8.3 / 17.3 / 75, 512 behind
+// 3000 85 -> 91; 64 dims, 128 / 1100 rows 7.8 / 35.5 -> 6.5 / 27.2: that kernel has 32-bit caches alone.  512 rows of 24 heads of 128 behind 1024 from fp32 caches: 137 us.
 // Query heads of a key/value head are x, x + kv_heads, ...: with eight key/value heads they share one L2.
 #include "../common.h"
 #include "attention_rows.h"
 #include "span_attention.h"
+#include <atomic>
+#include <type_traits>
 
 namespace esp {
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+typedef short short4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// v = p[0] + p[1] + p[2] in element e, for |v| up to 2^15
-__device__ __forceinline__ void split3(float v, half8 (&p)[3], int e) {
-    p[0][e] = (_Float16)v;
-    const float rest = __fsub_rn(v, (float)p[0][e]);
-    p[1][e] = (_Float16)rest;
-    p[2][e] = (_Float16)__fsub_rn(rest, (float)p[1][e]);
+// Two numbers of up to 2^15 as fp16 parts that add up to their 24 bits (each part cut off towards 0): elements e, e + 1 of p.
+__device__ __forceinline__ void split3(float v0, float v1, half8 (&p)[3], int e) {
+    float minus = -1.0f;
+    asm("" : "+v"(minus));   // v - part as one v_fma_mix: a conversion and a subtraction otherwise
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const half2 part = __builtin_bit_cast(half2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+        p[i][e] = part[0];
+        p[i][e + 1] = part[1];
+        if (i == 2) break;
+        v0 = __builtin_fmaf((float)part[0], minus, v0);
+        v1 = __builtin_fmaf((float)part[1], minus, v1);
+    }
+}
+
+__device__ __forceinline__ half4 read_transposed(const _Float16 *p) {
+    return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4 *)p));
+}
+
+// the larger of what the two halves of a wavefront hold
+__device__ __forceinline__ float max_of_halves(float v) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+    const uint32_t lower = p[0], upper = p[1];
+    return fmaxf(__builtin_bit_cast(float, lower), __builtin_bit_cast(float, upper));
+}
+
+// the largest of 16 or 32 neighbouring lanes
+template <int LANES>
+__device__ __forceinline__ float row_max(float v) {
+    static_assert(LANES == 16 || LANES == 32, "rows of the wavefront");
+    auto from = [](float x, auto control) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(control)::value, 0xF, 0xF, false)); };
+    v = fmaxf(v, from(v, std::integral_constant<int, 0xB1>{}));    // quad_perm [1,0,3,2]
+    v = fmaxf(v, from(v, std::integral_constant<int, 0x4E>{}));    // quad_perm [2,3,0,1]
+    v = fmaxf(v, from(v, std::integral_constant<int, 0x141>{}));   // row_half_mirror
+    v = fmaxf(v, from(v, std::integral_constant<int, 0x128>{}));   // row_ror:8
+    if constexpr (LANES == 32) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+        const auto p = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+        const uint32_t even = p[0], odd = p[1];
+        v = fmaxf(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
+    }
+    return v;
 }
 
 // e^x for x <= 0: the hardware's 2^t at the rounded t = x log2(e), times 1 + what the rounding left of it.  Within 2^-22 of e^x for results above 2^-126 (smaller ones are
@@ -52,87 +97,98 @@ constexpr int span_waves_per_simd(int hd, bool kv_f16, int kp) { return hd == 64
 
 template <int HD, bool KV_F16, int KP>
 __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void span_attention_kernel(AttentionArgs a, int rows) {
-    constexpr int KS = HD / 16, MT = HD / 32, LDV = 32 + 8, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane
+    constexpr int KS = HD / 16, MT = HD / 32, LDV = HD + 16, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane; LDV: four keys' dims fall on all banks
     constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
     constexpr int kQueryBytes = KV_F16 ? 3 * 32 * LDQ * 2 : 32 * LDQ * 4;
-    constexpr int kWave = KV_F16 ? HD * LDV * 2 : 0;                        // a value tile per wavefront
-    constexpr int kMergeBytes = KP > 1 ? (KP / 2) * MT * 16 * 64 * 4 : 16;
-    __shared__ __attribute__((aligned(16))) unsigned char query_mem[kQueryBytes];
-    __shared__ __attribute__((aligned(16))) unsigned char smem[KP * kWave > kMergeBytes ? KP * kWave : kMergeBytes];
+    constexpr int kWave = KV_F16 ? 32 * LDV * 2 : 0;                        // a value tile per wavefront
+    constexpr int OWN = MT * 16 / KP, kMergeBytes = KP > 1 ? KP * (KP - 1) * OWN * 64 * 4 : 16;   // accumulators that a wavefront finishes
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kQueryBytes + KP * kWave > kMergeBytes ? kQueryBytes + KP * kWave : kMergeBytes];
+    unsigned char *const query_mem = smem;
     __shared__ int not_finite;
-    __shared__ float state[KP][2][64];
-    const int lane = threadIdx.x & 63, phase = threadIdx.x >> 6, half = lane >> 5, col = lane & 31;
+    __shared__ float state[KP][2][64], row_scale[32];
+    const int lane = threadIdx.x & 63, phase = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
     const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head;
     const int y = (int)(gridDim.y - 1 - blockIdx.y);                           // the row tiles with the most keys start first
     asm volatile("" ::"s"(a.tiles), "s"(a.pos), "s"(a.seq), "s"(a.q), "s"(a.k_cache), "s"(a.v_cache));   // fetched together, ahead of the branch
     const int2 tile = a.tiles ? a.tiles[y] : int2{32 * y, rows - 1 - 32 * y};
     const int m0 = tile.x, last_row = tile.y < 31 ? tile.y : 31;
-    const int pos0 = a.pos[m0], t_max = pos0 + last_row, kd = a.n_kv_head * HD;
-    const size_t base = (size_t)a.seq[m0] * a.cache_seq_stride + (size_t)kvh * HD;
-    float scale = 1.0f / sqrtf((float)HD);   // fp16 caches: of the scaled queries
+    const int pos0 = __builtin_amdgcn_readfirstlane(a.pos[m0]), t_max = pos0 + last_row, kd = a.n_kv_head * HD;
+    const size_t base = (size_t)__builtin_amdgcn_readfirstlane(a.seq[m0]) * a.cache_seq_stride + (size_t)kvh * HD;
     const int qpos = pos0 + col;
 
-    // Keys beyond t_max are clamped to it: in bounds, and masked.  A lane's keys: row `col` of the tile, dims 16 ks + 8 half .. (fp16), 8 j + 4 half .. (fp32)
-    constexpr int NK = KV_F16 ? KS : HD / 8;
-    float4 kr[NK];
-    auto load_keys = [&](int t0) {
+    // Keys beyond t_max are clamped to it: in bounds, and masked.
+    // fp32 keys: row `col` of the tile, dims 8 j + 4 half ..
+    float4 kr32[KV_F16 ? 1 : HD / 8];
+    auto load_keys32 = [&](int t0) {
         const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
 #pragma unroll
-        for (int j = 0; j < NK; j++)
-            kr[j] = KV_F16 ? *reinterpret_cast<const float4 *>(reinterpret_cast<const uint16_t *>(a.k_cache) + kt + 16 * j + 8 * half)
-                           : *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 8 * j + 4 * half);
+        for (int j = 0; j < HD / 8; j++) kr32[j] = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(a.k_cache) + kt + 8 * j + 4 * half);
     };
-    // an fp16 value tile on its way to LDS: key = lane % 32, dims 8 (lane / 32 + 2 i) ..: the transposed two-byte writes spread over the banks
-    uint4 vr[KV_F16 ? VP : 1];
-    auto load_values = [&](int t0) {
-        const size_t kt = base + (size_t)(t0 + col < t_max ? t0 + col : t_max) * kd;
+    // fp16 keys: row `col`, dims 16 ks + 8 half ..; values on their way to LDS, whole rows by neighbouring lanes.  The tile's first row is uniform, so a lane adds 32-bit offsets alone.
+    constexpr int VL = HD / 8, VR = 64 / VL;   // lanes of a row, rows of a load
+    uintx4 kr[KV_F16 ? KS : 1], vr[KV_F16 ? VP : 1];
+    const uint32_t row_bytes = (uint32_t)kd * 2, k_row = (uint32_t)col * row_bytes, v_row = (uint32_t)(lane / VL) * row_bytes;
+    auto first_row = [&](const void *cache, int t0) { return reinterpret_cast<const uint8_t *>(cache) + (base + (size_t)(t0 < t_max ? t0 : t_max) * kd) * 2; };
+    auto last_offset = [&](int t0) { return (uint32_t)(t0 < t_max ? t_max - t0 : 0) * row_bytes; };   // t_max's, from the tile's first row on (far tiles: beyond every lane's own)
+    auto load_keys = [&](int t0) __attribute__((always_inline)) {
+        const uint8_t *from = first_row(a.k_cache, t0);
+        const uint32_t most = last_offset(t0), at = (k_row < most ? k_row : most) + 16 * half;
 #pragma unroll
-        for (int i = 0; i < (KV_F16 ? VP : 0); i++) vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(a.v_cache) + kt + 8 * (half + 2 * i));
+        for (int ks = 0; ks < KS; ks++) kr[ks] = *reinterpret_cast<const uintx4 *>(from + at + 32 * ks);
     };
-    // The first tile's keys: ahead of the queries from fp32 caches (512 rows behind 1024: 152 -> 137 us), behind them from fp16 ones, whose queries take longer to lay out
-    // and then come first (93 rows of 64 dims behind 700: 15.3 us against 16.3).
-    if (!KV_F16 && 32 * phase <= t_max) load_keys(32 * phase);
+    auto load_values = [&](int t0) __attribute__((always_inline)) {
+        const uint8_t *from = first_row(a.v_cache, t0);
+        const uint32_t most = last_offset(t0);
+#pragma unroll
+        for (int i = 0; i < VP; i++) {
+            const uint32_t row = v_row + i * VR * row_bytes;
+            vr[i] = *reinterpret_cast<const uintx4 *>(from + ((row < most ? row : most) + 16 * (lane % VL)));
+        }
+    };
+    // The first tile of fp32 keys ahead of the queries (512 rows behind 1024: 152 -> 137 us).
+    if (!KV_F16 && 32 * phase <= t_max) load_keys32(32 * phase);
 
-    // query `col` (rows beyond the block repeat its last row, never stored)
-    const float *query = a.q + (size_t)(m0 + (col <= last_row ? col : last_row)) * a.n_head * HD + (size_t)head * HD;
+    // the queries (rows beyond the block repeat its last row, never stored)
+    const size_t q_pitch = (size_t)a.n_head * HD;
+    const float *queries = a.q + (size_t)m0 * q_pitch + (size_t)head * HD;
     _Float16 *q16 = reinterpret_cast<_Float16 *>(query_mem);                   // [3][32][LDQ]
     float *q32 = reinterpret_cast<float *>(query_mem);                         // [32][LDQ]
-    {
-        float4 x[KS][2];   // dims 16 ks + 8 half ..
-        int q_exp = 0;
+    if constexpr (KV_F16) {   // whole rows by neighbouring lanes, 32 / KP of them a wavefront
+        constexpr int QL = HD / 4, QR = 64 / QL, PASSES = 32 / KP / QR;   // lanes of a row, rows of a load
+        float4 x[PASSES];
+#pragma unroll
+        for (int i = 0; i < PASSES; i++) {
+            const int r = phase * (32 / KP) + i * QR + lane / QL;
+            x[i] = *reinterpret_cast<const float4 *>(queries + (size_t)(r <= last_row ? r : last_row) * q_pitch + 4 * (lane % QL));
+        }
+        if (32 * phase <= t_max) { load_keys(32 * phase); load_values(32 * phase); }
+#pragma unroll
+        for (int i = 0; i < PASSES; i++) {
+            const int r = phase * (32 / KP) + i * QR + lane / QL;
+            const float most = row_max<QL>(fmaxf(fmaxf(fabsf(x[i].x), fabsf(x[i].y)), fmaxf(fabsf(x[i].z), fabsf(x[i].w))));
+            // where the power of two would not be a float (scores are 0 or beyond every type there), some other will do
+            int q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
+            q_exp = q_exp < -100 ? -100 : q_exp > 100 ? 100 : q_exp;
+            half8 p[3];
+            split3(__builtin_amdgcn_ldexpf(x[i].x, q_exp), __builtin_amdgcn_ldexpf(x[i].y, q_exp), p, 0);
+            split3(__builtin_amdgcn_ldexpf(x[i].z, q_exp), __builtin_amdgcn_ldexpf(x[i].w, q_exp), p, 2);
+#pragma unroll
+            for (int k = 0; k < 3; k++) *reinterpret_cast<half4 *>(q16 + (k * 32 + r) * LDQ + 4 * (lane % QL)) = half4{p[k][0], p[k][1], p[k][2], p[k][3]};
+            if (lane % QL == 0) row_scale[r] = __builtin_amdgcn_ldexpf(__fmul_rn(1.0f / sqrtf((float)HD), 1.44269504f), -q_exp);
+        }
+    } else {
+        const float *query = queries + (size_t)(col <= last_row ? col : last_row) * q_pitch;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++)
+            if (ks % KP == phase)
 #pragma unroll
-            for (int w = 0; w < 2; w++) x[ks][w] = *reinterpret_cast<const float4 *>(query + 16 * ks + 8 * half + 4 * w);
-        if constexpr (KV_F16) {
-            float most = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-                for (int w = 0; w < 2; w++) most = fmaxf(fmaxf(most, fmaxf(fabsf(x[ks][w].x), fabsf(x[ks][w].y))), fmaxf(fabsf(x[ks][w].z), fabsf(x[ks][w].w)));
-            most = fmaxf(most, __shfl_xor(most, 32));
-            // where the power of two would not be a float (scores are 0 or beyond every type there), some other will do
-            q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
-            q_exp = q_exp < -100 ? -100 : q_exp > 100 ? 100 : q_exp;
-            scale = __builtin_amdgcn_ldexpf(scale, -q_exp);
-        }
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            if (ks % KP != phase) continue;   // the wavefronts share the work; each has read the row for its exponent
-            if constexpr (KV_F16) {
-                const float v[8] = {x[ks][0].x, x[ks][0].y, x[ks][0].z, x[ks][0].w, x[ks][1].x, x[ks][1].y, x[ks][1].z, x[ks][1].w};
-                half8 p[3];
-#pragma unroll
-                for (int e = 0; e < 8; e++) split3(__builtin_amdgcn_ldexpf(v[e], q_exp), p, e);
-#pragma unroll
-                for (int i = 0; i < 3; i++) *reinterpret_cast<half8 *>(q16 + (i * 32 + col) * LDQ + 16 * ks + 8 * half) = p[i];
-            } else {
-#pragma unroll
-                for (int w = 0; w < 2; w++) *reinterpret_cast<float4 *>(q32 + col * LDQ + 16 * ks + 8 * half + 4 * w) = x[ks][w];
-            }
-        }
+                for (int w = 0; w < 2; w++) *reinterpret_cast<float4 *>(q32 + col * LDQ + 16 * ks + 8 * half + 4 * w) = *reinterpret_cast<const float4 *>(query + 16 * ks + 8 * half + 4 * w);
     }
+    if (threadIdx.x == 0) not_finite = 0;
     __syncthreads();
+    // fp16 caches: of the scaled query, in powers of two
+    const float scale = KV_F16 ? row_scale[col] : 1.0f / sqrtf((float)HD);
+    auto weight_of = [&](float above) { return KV_F16 ? __builtin_amdgcn_exp2f(__fmul_rn(above, scale)) : exp_weight(above); };
 
     // fp32 values of dims 32 mt .. for the product's 16 steps: step r takes key 8 (r / 4) + 4 half + r % 4, the key of accumulator r
     auto load_value_dims = [&](int t0, int mt, float (&v)[16]) {
@@ -149,90 +205,125 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
 #pragma unroll
         for (int r = 0; r < 16; r++) o[mt][r] = 0.0f;
     float mx = -INFINITY, l = 0.0f;
-    _Float16 *vt = reinterpret_cast<_Float16 *>(smem + phase * kWave);
+    _Float16 *vt = reinterpret_cast<_Float16 *>(smem + kQueryBytes + phase * kWave);
 
-    if (KV_F16 && 32 * phase <= t_max) { load_keys(32 * phase); load_values(32 * phase); }
-    for (int t0 = 32 * phase; t0 <= t_max; t0 += 32 * KP) {
-        float vd[KV_F16 ? 1 : 2][16];
-        if constexpr (!KV_F16) load_value_dims(t0, 0, vd[0]);
-        floatx16 s0;
+    if constexpr (KV_F16) {
+        for (int t0 = 32 * phase; t0 <= t_max; t0 += 32 * KP) {
+            floatx16 s;
 #pragma unroll
-        for (int r = 0; r < 16; r++) s0[r] = 0.0f;
-        if constexpr (KV_F16) {
+            for (int r = 0; r < 16; r++) s[r] = 0.0f;
+            half8 qf[2][3];   // query parts of this step and the next: an LDS read takes as long as two steps' products
+            auto read_query = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+                for (int p = 0; p < 3; p++) qf[ks & 1][p] = *reinterpret_cast<const half8 *>(q16 + (p * 32 + col) * LDQ + 16 * ks + 8 * half);
+            };
+            read_query(0);
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
-                const half8 k = __builtin_bit_cast(half8, kr[ks]);
-                const _Float16 *qp = q16 + col * LDQ + 16 * ks + 8 * half;
+                if (ks + 1 < KS) read_query(ks + 1);
 #pragma unroll
-                for (int p = 2; p >= 0; p--) s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k, *reinterpret_cast<const half8 *>(qp + p * 32 * LDQ), s0, 0, 0, 0);
-                if (KP == 8 && ks % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // two wavefronts per SIMD: query parts of two steps at a time
+                for (int p = 2; p >= 0; p--) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kr[ks]), qf[ks & 1][p], s, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            // values of this tile into LDS, transposed; nobody else reads this stretch, and a wavefront's LDS operations keep their order
+            // values of this tile into LDS; nobody else reads this stretch, and a wavefront's LDS operations keep their order
 #pragma unroll
-            for (int i = 0; i < VP; i++) {
-                const half8 v = __builtin_bit_cast(half8, vr[i]);
-#pragma unroll
-                for (int e = 0; e < 8; e++) vt[(8 * (half + 2 * i) + e) * LDV + col] = v[e];
-            }
+            for (int i = 0; i < VP; i++) *reinterpret_cast<uintx4 *>(vt + (i * VR + lane / VL) * LDV + 8 * (lane % VL)) = vr[i];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             load_keys(t0 + 32 * KP);   // clamped beyond the last tile
             load_values(t0 + 32 * KP);
-        } else {
+            // Accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`.  Scores stay as they are summed: a weight is 2^((s - m) c) with c = scale log2(e), a subtraction, a product and
+            // the hardware's 2^t.
+            if (t0 + 31 > pos0) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[r] = t0 + 8 * (r >> 2) + 4 * half + (r & 3) <= qpos ? s[r] : -INFINITY;
+            }
+            float tile_max = s[0];
+#pragma unroll
+            for (int r = 1; r < 16; r++) tile_max = fmaxf(tile_max, s[r]);
+            // a wavefront may see only masked keys of a query for a while: its state stays (-inf, 0, 0), exponents taken against 0
+            const float m_new = fmaxf(mx, max_of_halves(tile_max)), m_ref = m_new == -INFINITY ? 0.0f : m_new;
+            const float alpha = weight_of(mx - m_ref);       // 2^-inf = 0 on the first tile
+            mx = m_new;
+            // A operand of the second product, k slot (lane / 32, i): key 16 j + 8 (i / 4) + 4 (lane / 32) + i % 4 of dim 32 mt + col, the key of accumulator 8 j + i
+            // (ds_read_tr: of sixteen lanes, lane 4 k + c names four dims of key k; lane i receives dim i of all four keys)
+            auto read_value = [&](int j, int mt) __attribute__((always_inline)) {
+                const _Float16 *vrow = vt + (16 * j + 4 * half + ((lane & 15) >> 2)) * LDV + 32 * mt + (lane & 16) + 4 * (lane & 3);
+                const half4 lo = read_transposed(vrow), hi = read_transposed(vrow + 8 * LDV);
+                return half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            };
+            half8 v[2][MT], p[2][3];
+            float psum = 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) v[0][mt] = read_value(0, mt);
+            auto weights = [&](int j) __attribute__((always_inline)) {
+                float w[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    w[i] = weight_of(s[8 * j + i] - m_ref);   // masked keys: 2^-inf = 0
+                    psum += w[i];
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) split3(__fmul_rn(w[i], 32768.0f), __fmul_rn(w[i + 1], 32768.0f), p[j], i);
+            };
+            weights(0);
+            if (__any(alpha != 1.0f)) {   // the maximum has moved
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) v[1][mt] = read_value(1, mt);
+            weights(1);
+            l = __builtin_fmaf(l, alpha, psum);
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int i = 2; i >= 0; i--)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[j][mt], p[j][i], o[mt], 0, 0, 0);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    } else {
+        for (int t0 = 32 * phase; t0 <= t_max; t0 += 32 * KP) {
+            float vd[2][16];
+            load_value_dims(t0, 0, vd[0]);
+            floatx16 s0;
+#pragma unroll
+            for (int r = 0; r < 16; r++) s0[r] = 0.0f;
 #pragma unroll
             for (int j = 0; j < HD / 8; j++) {
                 const float4 q = *reinterpret_cast<const float4 *>(q32 + col * LDQ + 8 * j + 4 * half);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].x, q.x, s0, 0, 0, 0);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].y, q.y, s0, 0, 0, 0);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].z, q.z, s0, 0, 0, 0);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j].w, q.w, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr32[j].x, q.x, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr32[j].y, q.y, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr32[j].z, q.z, s0, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(kr32[j].w, q.w, s0, 0, 0, 0);
             }
-            load_keys(t0 + 32 * KP);
-        }
-        // accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`
-        float tile_max = -INFINITY;
+            load_keys32(t0 + 32 * KP);
+            // accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`
+            float tile_max = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            s0[r] = t0 + 8 * (r >> 2) + 4 * half + (r & 3) <= qpos ? __fmul_rn(s0[r], scale) : -INFINITY;
-            tile_max = fmaxf(tile_max, s0[r]);
-        }
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-        // a wavefront may see only masked keys of a query for a while: its state stays (-inf, 0, 0), exponents taken against 0
-        const float m_new = fmaxf(mx, tile_max), m_ref = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = exp_weight(mx - m_ref);      // exp(-inf) = 0 on the first tile
-        float psum = 0.0f, pr[16];
+            for (int r = 0; r < 16; r++) {
+                s0[r] = t0 + 8 * (r >> 2) + 4 * half + (r & 3) <= qpos ? __fmul_rn(s0[r], scale) : -INFINITY;
+                tile_max = fmaxf(tile_max, s0[r]);
+            }
+            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+            const float m_new = fmaxf(mx, tile_max), m_ref = m_new == -INFINITY ? 0.0f : m_new;
+            const float alpha = weight_of(mx - m_ref);      // exp(-inf) = 0 on the first tile
+            float psum = 0.0f, pr[16];
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            pr[r] = exp_weight(s0[r] - m_ref);           // masked keys: exp(-inf) = 0
-            psum += pr[r];
-        }
-        l = __builtin_fmaf(l, alpha, psum);
-        mx = m_new;
-        if (!KV_F16 || __any(alpha != 1.0f)) {   // the maximum has moved (beside fp32 products it makes no difference)
+            for (int r = 0; r < 16; r++) {
+                pr[r] = weight_of(s0[r] - m_ref);            // masked keys: exp(-inf) = 0
+                psum += pr[r];
+            }
+            l = __builtin_fmaf(l, alpha, psum);
+            mx = m_new;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
+            for (int mt = 0; mt < MT; mt++)   // whether the maximum has moved or not: beside fp32 products it makes no difference
 #pragma unroll
                 for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
-        }
-        if constexpr (KV_F16) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                half8 p[3];
-#pragma unroll
-                for (int i = 0; i < 8; i++) split3(__fmul_rn(pr[8 * j + i], 32768.0f), p, i);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    // k slot (lane / 32, i) is key 16 j + 8 (i / 4) + 4 (lane / 32) + i % 4, the key of accumulator 8 j + i
-                    const _Float16 *vrow = vt + (32 * mt + col) * LDV + 16 * j + 4 * half;
-                    const half4 lo = *reinterpret_cast<const half4 *>(vrow), hi = *reinterpret_cast<const half4 *>(vrow + 8);
-                    const half8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-                    for (int i = 2; i >= 0; i--) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[i], o[mt], 0, 0, 0);
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        } else {
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 if (mt + 1 < MT) load_value_dims(t0, mt + 1, vd[(mt + 1) & 1]);
@@ -241,74 +332,110 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             }
         }
     }
+    // The wavefronts' states meet: each leaves the others' accumulators in LDS and finishes OWN of its own, with factors that take every state to the largest maximum, sums in pairs.
     l += __shfl_xor(l, 32);
-    // the upper half of the wavefronts hands its states to the lower half, until wavefront 0 holds the sum of all
-    float *merge = reinterpret_cast<float *>(smem);
+    float mine[OWN];
+    if constexpr (KP > 1) {
+        state[phase][0][lane] = mx;
+        state[phase][1][lane] = l;
+        __syncthreads();   // and everybody is done with queries and values
+        float m_all = mx;
 #pragma unroll
-    for (int s = KP / 2; s >= 1; s >>= 1) {
+        for (int w = 0; w < KP; w++) m_all = fmaxf(m_all, state[w][0][lane]);
+        const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
+        float f[KP], part[KP];
+#pragma unroll
+        for (int w = 0; w < KP; w++) { f[w] = weight_of(state[w][0][lane] - m_ref); part[w] = state[w][1][lane]; }
+        auto total = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int w = 0; w < KP; w += 2) part[w] = __builtin_fmaf(part[w + 1], f[w + 1], __fmul_rn(part[w], f[w]));
+#pragma unroll
+            for (int d = 2; d < KP; d *= 2)
+#pragma unroll
+                for (int w = 0; w < KP; w += 2 * d) part[w] += part[w + d];
+            return part[0];
+        };
+        l = total();
+        float *merge = reinterpret_cast<float *>(smem);   // [from][to, but for itself][OWN][64]
+#pragma unroll
+        for (int w = 0; w < KP; w++)
+#pragma unroll
+            for (int r = 0; r < OWN; r++) {
+                const float v = o[(w * OWN + r) >> 4][(w * OWN + r) & 15];
+                if (w == phase) mine[r] = v;
+                else merge[((phase * (KP - 1) + w - (w > phase)) * OWN + r) * 64 + lane] = v;
+            }
         __syncthreads();
-        if (phase >= s && phase < 2 * s) {
-            state[phase][0][lane] = mx;
-            state[phase][1][lane] = l;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
+        for (int r = 0; r < OWN; r++) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) merge[(((phase - s) * MT + mt) * 16 + r) * 64 + lane] = o[mt][r];
+            for (int w = 0; w < KP; w++) part[w] = w == phase ? mine[r] : merge[((w * (KP - 1) + phase - (phase > w)) * OWN + r) * 64 + lane];
+            mine[r] = total();
         }
-        __syncthreads();
-        if (phase < s) {
-            const float m1 = state[phase + s][0][lane], l1 = state[phase + s][1][lane];
-            const float m_all = fmaxf(mx, m1), m_ref = m_all == -INFINITY ? 0.0f : m_all;
-            const float f0 = exp_weight(mx - m_ref), f1 = exp_weight(m1 - m_ref);
-            l = __builtin_fmaf(l, f0, __fmul_rn(l1, f1));
-            mx = m_all;
+    } else {
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) o[mt][r] = __builtin_fmaf(o[mt][r], f0, __fmul_rn(merge[((phase * MT + mt) * 16 + r) * 64 + lane], f1));
-        }
+        for (int r = 0; r < OWN; r++) mine[r] = o[r >> 4][r & 15];
     }
-    if (phase == 0) {
-        float check = 0.0f;
+    float check = 0.0f;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+    for (int r = 0; r < OWN; r++) check = __builtin_fmaf(mine[r], 0.0f, check);
+    if (__any(!(check == 0.0f && l < INFINITY)) && lane == 0) not_finite = 1;   // NaN wherever an infinity or a NaN went in
+    __syncthreads();
+    if (!not_finite) {
+        const float inv = 1.0f / (KV_F16 ? __fmul_rn(l, 32768.0f) : l);   // key 0 is visible to every query: l > 0
+        const size_t row = (size_t)(m0 + (col <= last_row ? col : last_row));
+        float sums[OWN < 16 ? 1 : OWN / 16];   // of 32 dims each, or of this wavefront's share of them
 #pragma unroll
-            for (int r = 0; r < 16; r++) check = __builtin_fmaf(o[mt][r], 0.0f, check);
-        const bool odd = __any(!(check == 0.0f && l < INFINITY));   // NaN wherever an infinity or a NaN went in
-        if (lane == 0) not_finite = odd;
-        if (!odd) {
-            const float inv = 1.0f / (KV_F16 ? __fmul_rn(l, 32768.0f) : l);   // key 0 is visible to every query: l > 0
-            const size_t row = (size_t)(m0 + (col <= last_row ? col : last_row));
+        for (int r = 0; r < OWN; r += 4) {
+            const int at = phase * OWN + r;   // accumulator: dims 32 (at / 16) + 8 (at / 4 % 4) + 4 half ..
+            const float v[4] = {__fmul_rn(mine[r], inv), __fmul_rn(mine[r + 1], inv), __fmul_rn(mine[r + 2], inv), __fmul_rn(mine[r + 3], inv)};
+            float s = 0.0f;
+            if (col <= last_row) s = store_context4(a, row * q_pitch + (size_t)head * HD + 32 * (at >> 4) + 8 * ((at >> 2) & 3) + 4 * half, v);
+            sums[r >> 4] = r % 16 == 0 ? s : sums[r >> 4] + s;
+        }
+        if (a.ctx_hi) {
+            constexpr int PARTS = OWN < 16 ? 16 / OWN : 1;   // wavefronts that share 32 dims
+            float *parts = reinterpret_cast<float *>(smem);  // [PARTS][32 queries] of every 32 dims; the merge is behind everybody
+            if constexpr (PARTS > 1) {
+                const float s = sums[0] + __shfl_xor(sums[0], 32);
+                if (half == 0) parts[phase * 32 + col] = s;
+                __syncthreads();
+            }
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
+            for (int i = 0; i < (OWN < 16 ? 1 : OWN / 16); i++) {
                 float s = 0.0f;
+                if constexpr (PARTS > 1) {
 #pragma unroll
-                for (int q4 = 0; q4 < 4; q4++) {
-                    const float v[4] = {__fmul_rn(o[mt][4 * q4], inv), __fmul_rn(o[mt][4 * q4 + 1], inv), __fmul_rn(o[mt][4 * q4 + 2], inv), __fmul_rn(o[mt][4 * q4 + 3], inv)};
-                    if (col <= last_row) s += store_context4(a, row * a.n_head * HD + (size_t)head * HD + 32 * mt + 8 * q4 + 4 * half, v);
-                }
-                if (a.ctx_hi) {
-                    s += __shfl_xor(s, 32);
-                    if (half == 0 && col <= last_row) store_context_sum(a, row, a.n_head * HD, head * (HD / 32) + mt, s);
-                }
+                    for (int w = 0; w < PARTS; w++) s += parts[(phase / PARTS * PARTS + w) * 32 + col];
+                } else s = sums[i] + __shfl_xor(sums[i], 32);
+                if (phase % PARTS == 0 && half == 0 && col <= last_row) store_context_sum(a, row, a.n_head * HD, head * (HD / 32) + (phase * OWN >> 4) + i, s);
             }
         }
+        return;
     }
-    __syncthreads();
-    if (not_finite)
-        for (int i = phase; i <= last_row; i += KP) plain_attention_row<HD, KV_F16>(a, m0 + i, head);
+    for (int i = phase; i <= last_row; i += KP) plain_attention_row<HD, KV_F16>(a, m0 + i, head);
 }
 
 template <int HD, bool KV_F16>
 void launch_shape(const AttentionArgs &a, int rows, int sets, hipStream_t s) {
     const dim3 grid(a.n_head, a.tiles ? a.tile_count : (rows + 31) / 32);
-    if (sets == 1) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 1>), grid, dim3(64), 0, s, a, rows);
-    else if (sets == 2) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 2>), grid, dim3(128), 0, s, a, rows);
-    else if (sets == 4) hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 4>), grid, dim3(256), 0, s, a, rows);
-    else hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 8>), grid, dim3(512), 0, s, a, rows);
+    auto go = [&](auto waves) {
+        constexpr int KP = decltype(waves)::value;
+        hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, KP>), grid, dim3(64 * KP), 0, s, a, rows);
+    };
+    if constexpr (!KV_F16) {
+        if (sets == 1) return go(std::integral_constant<int, 1>{});
+        if (sets == 2) return go(std::integral_constant<int, 2>{});
+    }
+    if (sets == 4) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 8>{});
 }
 
+std::atomic<int> g_key_sets{0};
+
 }  // namespace
+
+void attention_prompt_set_key_sets(int sets) { g_key_sets.store(sets == 1 || sets == 2 ? sets : 0); }
 
 bool span_attention_supported(int n_head, int n_kv_head, int head_dim) {
     return n_kv_head > 0 && n_head % n_kv_head == 0 && (head_dim == 64 || head_dim == 128);
@@ -318,18 +445,16 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup, fp32 caches: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
-    // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit; two where a few tiles of keys are over before four have met (128 dims: below ten), and for 128 dims
-    // where three workgroups of two fill the chip; eight where a workgroup of 64 dims has the compute unit to itself and keys for all of them.  One wavefront / two / four / eight, us: 1777 rows of 24 heads
-    // of 128 136 / 109 / 112 / 152, 800 of them 63 / 39 / 36 / 53, 160 16.5 / 12.4 / 13.2 / 14.9, 31 rows behind 500 42 / 23 / 19 / 21.5;  512 rows of 32 heads of 64 behind 1024 71 / 53 / 35 / 42, 93 of
-    // them behind 1500 69 / 38 / 24.3 / 22.6, 1200 60 / 46 / 42 / 64.  (One set a SIMD, the rule before, was up to 1.5 times as slow: 1777 rows of 12 heads of 64 54 us, four sets 37.)
-    const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32);
+    // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit, or eight where a workgroup has the compute unit to itself and keys for all of them.  Two wavefronts / four /
+    // eight, us: 1777 rows of 24 heads of 128 79 / 80 / 104, 512 rows 18.8 / 15.6 / 21.2, 64 rows 8.5 / 8.4 / 9.1, 93 rows behind 1000 31 / 21.9 / 20.5, 31 rows behind 4000 (32 heads) 87 / 51 / 49.5;
+    // heads of 64: 1100 rows of 32 heads 28.2 / 27.2 / 41, 128 rows 6.5 / 6.3 / 6.7, 93 rows behind 700 15.2 / 11.1 / 10.4, behind 1500 25 / 16.7 / 14.9, 512 rows behind 1024 33 / 23.8 / 28.
+    const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32), cus = device_compute_units() > 0 ? device_compute_units() : 256;
     int sets = 1;
     if (!kv_f16) {
         while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
-    } else if (a.head_dim == 128) {
-        sets = tiles < 2 ? 1 : tiles < 10 || groups > 3 * (device_compute_units() > 0 ? device_compute_units() : 256) ? 2 : 4;
     } else {
-        sets = tiles < 2 ? 1 : tiles < 3 ? 2 : tiles >= 24 && groups <= (device_compute_units() > 0 ? device_compute_units() : 256) ? 8 : 4;
+        const int forced = g_key_sets.load();
+        sets = forced ? 4 * forced : tiles >= 24 && groups <= cus ? 8 : 4;
     }
     if (a.head_dim == 128) {
         if (kv_f16) launch_shape<128, true>(a, rows, sets, s);

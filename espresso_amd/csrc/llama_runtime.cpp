@@ -584,15 +584,15 @@ int LlamaRuntime::prefill_shared_block(const PromptSpan *spans, int count) {
     return rc;
 }
 
-// Attention of a block: one prompt's rows (block_keys: the keys that the last of them sees), prompts that share it, or (neither) rows that attend alone.  Fewer than 32 rows of a prompt take 32-bit
-// attention, as the steps they stand for.
+// Attention of a block: one prompt's rows (block_keys: the keys that the last of them sees), prompts that share it, or (neither) rows that attend alone.  Fewer than 32 rows of a prompt, and all rows of
+// models with fp16 caches, take 32-bit attention, as the steps they stand for.
 int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_keys, int last) {
     hipStream_t s = context().stream;
     const bool kv16 = c_.kv_format == FMT_F16;
-    if (last > 0 && last < kMatrixPrefillMinTokens && finer_short_attention()) {
+    if (last > 0 && last < kMatrixPrefillMinTokens && finer_short_attention() && !kv16) {   // (fp16 caches: 32-bit attention for every row)
         const int ahead = rows - last;
         const size_t at = (size_t)ahead * c_.attention_dim();
-        ESP_HIP_TRY(launch_attention_prompt(aa, ahead, kv16, s));
+        ESP_HIP_TRY(launch_prompt_attention(aa, ahead, block_keys - last, kv16, s));
         aa.q += at; aa.pos += ahead; aa.seq += ahead;
         if (aa.ctx_f16) aa.ctx_f16 += at;
         if (aa.ctx_hi) { aa.ctx_hi += at; aa.ctx_lo += at; aa.ctx_sums += at / 16; }
@@ -601,14 +601,14 @@ int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_
     }
     if (shared_.long_tiles + shared_.short_tiles > 0 && (prompt_attention_ || span_attention_)) {
         aa.tiles = d_tiles_; aa.tile_count = shared_.long_tiles;
-        if (shared_.long_tiles && prompt_attention_) ESP_HIP_TRY(launch_attention_prompt(aa, shared_.longest, kv16, s));
+        if (shared_.long_tiles && prompt_attention_) ESP_HIP_TRY(launch_prompt_attention(aa, shared_.longest, shared_.longest, kv16, s));
         else if (shared_.long_tiles) ESP_HIP_TRY(launch_span_attention(aa, shared_.longest, shared_.longest, kv16, s));
         aa.tiles = d_tiles_ + shared_.long_tiles; aa.tile_count = shared_.short_tiles;
         if (shared_.short_tiles) ESP_HIP_TRY(launch_span_attention(aa, shared_.longest_short, shared_.longest_short, kv16, s));
         return ESP_OK;
     }
     const bool few = rows < kMatrixPrefillMinTokens && short_span_attention_;
-    if (block_keys && prompt_attention_ && !few) ESP_HIP_TRY(launch_attention_prompt(aa, rows, kv16, s));
+    if (block_keys && prompt_attention_ && !few) ESP_HIP_TRY(launch_prompt_attention(aa, rows, block_keys, kv16, s));
     else if (block_keys && (span_attention_ || few)) ESP_HIP_TRY(launch_span_attention(aa, rows, block_keys, kv16, s));
     else ESP_HIP_TRY(launch_attention(aa, rows, kv16, s));
     return ESP_OK;

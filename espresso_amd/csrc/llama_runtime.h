@@ -97,7 +97,7 @@ class LlamaRuntime : public DecoderRuntime {
     int enqueue_block_attention(AttentionArgs aa, int rows, int block_keys, int last);
     LastRows last_rows(int count) const override;
     bool rounds_but_for_last(const DeviceMatrix &m, int last, bool gate_up) const;
-    bool finer_short_attention() const { return prompt_attention_ && short_span_attention_; }   // fewer than 32 rows: 32-bit, longer blocks: queries and softmax weights in fp16, or pairs of it
+    bool finer_short_attention() const { return prompt_attention_ && short_span_attention_; }   // fewer than 32 rows: 32-bit, longer blocks of models with 32-bit caches: queries and softmax weights in fp16
     bool keeps_weights(const DeviceMatrix &m, int rows, bool gate_up) const;
     int shared_block_class(int count) const override;
     int prefill_shared_block(const PromptSpan *spans, int count) override;
@@ -138,7 +138,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool split_activations_ = true;
     bool prompt_attention_ = false;   // prompt blocks run attention on the matrix cores
     bool short_span_attention_ = false;   // span_attention_kernel for blocks of few rows
-    bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for
+    bool span_attention_ = false;     // the same for head groups that attention_prompt_kernel is not written for, whatever the caches
     // the prompts that share the block being enqueued: tiles of those of at least kMatrixPrefillMinTokens tokens, behind them tiles of the shorter ones
     struct SharedBlock { int long_tiles = 0, short_tiles = 0, longest = 0, longest_short = 0; } shared_;
     int2 *d_tiles_ = nullptr;

@@ -56,6 +56,20 @@ def test_span_attention_is_as_exact_as_fp32(ops, rows, first, heads, kv_heads, s
             assert off(got) <= 1.02 * off(one) + 1e-9, sharp
 
 
+# four and eight wavefronts (1, 2) where some have no tile of keys, one, or one more than the others; the shares of dims that they finish, and their sums of 32
+@pytest.mark.parametrize("sets", [1, 2])
+@pytest.mark.parametrize("rows,first,heads,kv_heads,size", [(1, 0, 4, 4, 64), (1, 31, 2, 1, 128), (32, 1, 12, 4, 64), (33, 95, 2, 2, 128), (64, 193, 6, 2, 128), (31, 224, 4, 1, 64), (2, 255, 8, 2, 128)])
+def test_span_attention_by_any_number_of_wavefronts(ops, rows, first, heads, kv_heads, size, sets):
+    ops.set_tuning("prompt_attention_key_sets", sets)
+    q, k, v = inputs(rows, first, heads, kv_heads, size, np.float16, rows + first, 4.0)
+    want = exact(q, k, v)
+    for planes in (True, False):
+        got, _ = ops.block_attention("span", q, k, v, split_rows=planes)
+        # as above: 2^-24 of scores and sums, planes end at 2^-22 and fp16 at 2^-11 of the result
+        assert np.sqrt(np.mean((got - want) ** 2)) <= 2.0 ** -24 * (np.sqrt(size) * 4.0 + 8) + 2.0 ** (-22 if planes else -11) * np.sqrt(np.mean(want ** 2)), planes
+    ops.set_tuning("prompt_attention_key_sets", 0)
+
+
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("scale", [2.0 ** -40, 2.0 ** -12, 2.0 ** 14, 2.0 ** 60])
 def test_span_attention_takes_queries_of_any_size(ops, scale, dtype):
