@@ -89,6 +89,11 @@ struct GemvParams {
     // fp16; `x` and `norm_x` are ignored.  [batch][cols / head_dim][kAttentionHeadSplits][head_dim + 4] floats.
     const float *merge_partials = nullptr;
     int merge_head_dim = 0;
+    // fused RMSNorm of rows that are still sums of planes (gemv_adds_planes; batch <= 2): norm_x = null, norm_planes [batch][norm_plane_count][cols], the sums (the first plane added to the sum of the
+    // others) go to norm_sum [batch][cols] as well
+    const float *norm_planes = nullptr;
+    int norm_plane_count = 0;
+    float *norm_sum = nullptr;
     float *y = nullptr;           // fp32 out [batch][rows]
     const float *residual = nullptr;
     uint16_t *out_f16 = nullptr;  // EPI_SWIGLU_F16: [batch][rows/2]
@@ -216,6 +221,9 @@ bool gemv_holds_two_rows(const DeviceMatrix &w);
 bool gemv_supports_argmax(const DeviceMatrix &w);
 // True when launch_gemv can take its input as attention partial states (batch <= 2, head size 64 or 128).
 bool gemv_merges_attention_partials(const DeviceMatrix &w, int batch, int head_dim);
+// True when launch_gemv can take one or two rows as sums of planes (GemvParams::norm_planes).
+constexpr int kMaxNormPlanes = 12;
+bool gemv_adds_planes(const DeviceMatrix &w);
 // kernels/gemm.hip
 hipError_t launch_gemm(const GemmParams &p, hipStream_t stream);
 bool gemm_keeps_weights(const GemmParams &p);   // does launch_gemm multiply with the weights as they are, none rounded to fp16?

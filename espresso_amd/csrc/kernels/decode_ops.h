@@ -78,6 +78,9 @@ hipError_t launch_attention_prompt(const AttentionArgs &a, int rows, hipStream_t
 // the context merges them (GemvParams::merge_partials).  attention_head_splits: slices per query head.
 int attention_head_splits(int max_seq);
 hipError_t launch_attention_partials(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s);
+// Attention of one row or two and its product with wo: planes [rows][n_head][wo.rows] that add up to residual + wo context, for a GEMV that takes them (GemvParams::norm_planes, gemv_adds_planes).
+bool attention_project_supported(const DeviceMatrix &wo, int n_head, int n_kv_head, int head_dim, int max_seq);
+hipError_t launch_attention_project(const AttentionArgs &a, const DeviceMatrix &wo, int rows, const float *residual, float *planes, bool kv_f16, hipStream_t s);
 hipError_t launch_swiglu(const float *gu, int splits, size_t plane, int rows, int hidden, uint16_t *act_f16, hipStream_t s);
 // Scratch of the two-launch argmax: kMaxStepRows x 128 partial (value, index) pairs.
 struct ArgmaxScratch {

@@ -666,37 +666,13 @@ __global__ __launch_bounds__(G * 64, HD == 64 ? 2 : 1) void attention_prompt_ker
     }
 }
 
-// Single-query attention whose merge is left to the consumer: grid (query heads, rows, kAttentionHeadSplits),
-// WAVES wavefronts per workgroup, one query head each.  Chunks, lane mapping and the (m, l, acc) arithmetic are
-// those of attention_flash_kernel; a wavefront keeps U chunks of loads in flight, so kAttentionHeadSplits *
-// WAVES * U chunks of the prefix cost one memory round trip and longer prefixes loop.  The arithmetic per
-// chunk is what a wavefront spends its time on, hence many wavefronts with few chunks each.  Every workgroup writes its
-// state to `head_partials` as [row][head][split][HD values, m, l, 2 pad] (16-byte aligned rows); the GEMV
-// that consumes the context merges the splits while it stages its input, so no merge launch follows.
-// Workgroups x, x + kvHeads, ... serve the query heads of KV head x: with eight KV heads the group shares
-// one L2, which then reads K and V from memory once.
-// SPLITS 1: the workgroup has the whole prefix, and head_partials is the context as fp16 rows.
-template <int HD, bool KV_F16, int WAVES, int U, int SPLITS = kAttentionHeadSplits>
-__global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const float *q_rows, const void *k_cache, const void *v_cache, const int *pos,
-                                                                       const int *seq, float *head_partials, unsigned cache_seq_stride, unsigned heads) {
-    // Fourteen 32-bit words of scalar arguments (heads = query heads | key/value heads << 16): all of them are
-    // preloaded into registers with the wavefront's launch, so the first loads do not wait for an argument fetch
-    // from memory, which the fields of a structure passed by value would need.
-    AttentionArgs a = {};
-    a.q = q_rows; a.k_cache = k_cache; a.v_cache = v_cache; a.pos = pos; a.seq = seq; a.head_partials = head_partials;
-    a.cache_seq_stride = cache_seq_stride; a.n_head = (int)(heads & 0xFFFFu); a.n_kv_head = (int)(heads >> 16);
-    constexpr int LPT = HD / 8, SLOTS = 64 / LPT, KW = KV_F16 ? 1 : 2, STRIDE = HD + 4;
-    __shared__ float wm[WAVES], wl[WAVES];
-    __shared__ float wacc[WAVES][HD];
-    const int group = a.n_head / a.n_kv_head;
-    const int kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head, m = blockIdx.y;
-    const int split = blockIdx.z;
-    constexpr int splits = SPLITS;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // both row descriptors are fetched in one round trip, before anything branches on the first
-    const int row_pos = a.pos[m], row_seq = a.seq[m];
-    asm volatile("" ::"s"(row_pos), "s"(row_seq));
-    const int visible = row_pos + 1;
+// One query head's slice of a row's prefix by WAVES wavefronts: chunks of SLOTS tokens, U of them in flight a wavefront; every wavefront leaves one (maximum, sum, accumulators) in LDS, and all have
+// when it returns.
+template <int HD, bool KV_F16, int WAVES, int U>
+__device__ __forceinline__ void attend_slice(const AttentionArgs &a, int m, int head, int kvh, int row_seq, int visible, int slice, int slices, float (&wm)[WAVES], float (&wl)[WAVES],
+                                             float (&wacc)[WAVES][HD]) {
+    constexpr int LPT = HD / 8, SLOTS = 64 / LPT, KW = KV_F16 ? 1 : 2;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int kd = a.n_kv_head * HD;
     const size_t seq_base = (size_t)row_seq * a.cache_seq_stride;
     const float scale = 1.0f / sqrtf((float)HD);
@@ -724,8 +700,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
         }
     };
 
-    const int stride = splits * WAVES * SLOTS;
-    for (int t0 = (split * WAVES + wave) * SLOTS; t0 < visible; t0 += stride * U) {
+    const int stride = slices * WAVES * SLOTS;
+    for (int t0 = (slice * WAVES + wave) * SLOTS; t0 < visible; t0 += stride * U) {
         uint4 kr[U][KW], vr[U][KW];
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -785,6 +761,40 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
     }
     if (lane == 0) { wl[wave] = l; wm[wave] = mx; }
     __syncthreads();
+}
+
+// Single-query attention whose merge is left to the consumer: grid (query heads, rows, kAttentionHeadSplits),
+// WAVES wavefronts per workgroup, one query head each.  Chunks, lane mapping and the (m, l, acc) arithmetic are
+// those of attention_flash_kernel; a wavefront keeps U chunks of loads in flight, so kAttentionHeadSplits *
+// WAVES * U chunks of the prefix cost one memory round trip and longer prefixes loop.  The arithmetic per
+// chunk is what a wavefront spends its time on, hence many wavefronts with few chunks each.  Every workgroup writes its
+// state to `head_partials` as [row][head][split][HD values, m, l, 2 pad] (16-byte aligned rows); the GEMV
+// that consumes the context merges the splits while it stages its input, so no merge launch follows.
+// Workgroups x, x + kvHeads, ... serve the query heads of KV head x: with eight KV heads the group shares
+// one L2, which then reads K and V from memory once.
+// SPLITS 1: the workgroup has the whole prefix, and head_partials is the context as fp16 rows.
+template <int HD, bool KV_F16, int WAVES, int U, int SPLITS = kAttentionHeadSplits>
+__global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const float *q_rows, const void *k_cache, const void *v_cache, const int *pos,
+                                                                       const int *seq, float *head_partials, unsigned cache_seq_stride, unsigned heads) {
+    // Fourteen 32-bit words of scalar arguments (heads = query heads | key/value heads << 16): all of them are
+    // preloaded into registers with the wavefront's launch, so the first loads do not wait for an argument fetch
+    // from memory, which the fields of a structure passed by value would need.
+    AttentionArgs a = {};
+    a.q = q_rows; a.k_cache = k_cache; a.v_cache = v_cache; a.pos = pos; a.seq = seq; a.head_partials = head_partials;
+    a.cache_seq_stride = cache_seq_stride; a.n_head = (int)(heads & 0xFFFFu); a.n_kv_head = (int)(heads >> 16);
+    constexpr int STRIDE = HD + 4;
+    __shared__ float wm[WAVES], wl[WAVES];
+    __shared__ float wacc[WAVES][HD];
+    const int group = a.n_head / a.n_kv_head;
+    const int kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head, m = blockIdx.y;
+    const int split = blockIdx.z;
+    constexpr int splits = SPLITS;
+    const int tid = threadIdx.x;
+    // both row descriptors are fetched in one round trip, before anything branches on the first
+    const int row_pos = a.pos[m], row_seq = a.seq[m];
+    asm volatile("" ::"s"(row_pos), "s"(row_seq));
+    const int visible = row_pos + 1;
+    attend_slice<HD, KV_F16, WAVES, U>(a, m, head, kvh, row_seq, visible, split, splits, wm, wl, wacc);
     // ---- merge over wavefronts in wavefront order: thread = channel ----
     float *ps = a.head_partials + (((size_t)m * a.n_head + head) * splits + split) * STRIDE;
     for (int dch = tid; dch < HD; dch += WAVES * 64) {
@@ -804,6 +814,85 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
         }
         ps[dch] = A;
         if (dch == 0) { ps[HD] = M; ps[HD + 1] = L; }
+    }
+}
+
+constexpr int kProjectRows = 64;
+struct AttentionProject {
+    size_t cache_seq_stride;
+    const uint16_t *scales;
+    const float *residual;
+    float *planes;
+    int rows;
+};
+// Attention and output projection of one row or two in one launch: grid (query heads, blocks of 64 rows of wo, rows).  A workgroup attends for its head over the whole prefix, as every other
+// workgroup of the head does, and multiplies the context with its rows' 64 columns of that head; the heads' products are planes [row][heads][wo.rows] that the next norm adds
+// (GemvParams::norm_planes), the first with the residual in it.  Nothing of the context is rounded.  Bound by the launch, like everything beside it, and by its chain of memory trips: position ->
+// keys and values -> store; weights and residual are requested first.  In place of partial states and a GEMV that merges them, a step of 768 wide, 6 layers, Q8_0 went from 117 to 105 us, of 576
+// wide, 30 layers, fp16 from 580 to 528, and a speculative pass of the former (two rows) from 6.5 to 6.3 ms a generation of 64 tokens.
+template <bool KV_F16, int FMT, int WAVES, int U>
+__global__ __launch_bounds__(WAVES * 64) void attention_project_kernel(const float *q_rows, const void *k_cache, const void *v_cache, const int *pos, const int *seq, const uint8_t *qs, unsigned heads,
+                                                                       unsigned row_bytes, AttentionProject p) {
+    constexpr int HD = 64, THREADS = WAVES * 64, LPR = FMT == FMT_F16 ? 8 : FMT == FMT_Q8_0 ? 4 : 2, PASS = THREADS / LPR, PASSES = (kProjectRows + PASS - 1) / PASS;   // LPR: lanes of a row's 64 columns
+    AttentionArgs a = {};
+    a.q = q_rows; a.k_cache = k_cache; a.v_cache = v_cache; a.n_head = (int)(heads & 0xFFFFu); a.n_kv_head = (int)(heads >> 16); a.cache_seq_stride = p.cache_seq_stride;
+    __shared__ float wm[WAVES], wl[WAVES], wacc[WAVES][HD], ctx[HD];
+    const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head, tid = threadIdx.x, part = tid % LPR;
+    const int m = blockIdx.z, row_pos = pos[m], row_seq = seq[m];
+    asm volatile("" ::"s"(row_pos), "s"(row_seq));
+    uint4 w[PASSES];
+    uint16_t d[PASSES];
+    float before[PASSES];
+    auto row_of = [&](int i) { const int r = (int)blockIdx.y * kProjectRows + i * PASS + tid / LPR; return r < p.rows ? r : p.rows - 1; };
+#pragma unroll
+    for (int i = 0; i < PASSES; i++) {
+        const int r = row_of(i);
+        w[i] = *reinterpret_cast<const uint4 *>(qs + (size_t)r * row_bytes + (size_t)head * (16 * LPR) + part * 16);
+        d[i] = FMT == FMT_F16 ? (uint16_t)0 : p.scales[(size_t)r * (a.n_head * 2) + head * 2 + (FMT == FMT_Q8_0 ? part >> 1 : part)];
+        before[i] = p.residual[m * p.rows + r];
+    }
+    asm volatile("" ::: "memory");   // requested here, ahead of keys and values
+    __builtin_amdgcn_sched_barrier(0);
+    attend_slice<HD, KV_F16, WAVES, U>(a, m, head, kvh, row_seq, row_pos + 1, 0, 1, wm, wl, wacc);
+    if (tid < HD) {   // over wavefronts in their order
+        float M = wm[0];
+#pragma unroll
+        for (int v = 1; v < WAVES; v++) M = fmaxf(M, wm[v]);
+        float L = 0.0f, A = 0.0f;
+#pragma unroll
+        for (int v = 0; v < WAVES; v++) {
+            const float f = wm[v] == -INFINITY ? 0.0f : expf(wm[v] - M);
+            L = __builtin_fmaf(wl[v], f, L);
+            A = __builtin_fmaf(wacc[v][tid], f, A);
+        }
+        ctx[tid] = L > 0.0f ? A / L : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PASSES; i++) {
+        const uint32_t dw[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+        float sum = 0.0f;
+        if constexpr (FMT == FMT_F16) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) sum = __builtin_fmaf(from_half_bits((uint16_t)(k & 1 ? dw[k >> 1] >> 16 : dw[k >> 1] & 0xFFFFu)), ctx[8 * part + k], sum);
+        } else if constexpr (FMT == FMT_Q8_0) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) sum = __builtin_fmaf((float)(int8_t)(dw[k >> 2] >> (8 * (k & 3))), ctx[16 * part + k], sum);
+            sum = __fmul_rn(from_half_bits(d[i]), sum);
+        } else {   // Q4_0: the low nibbles are the block's first half
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const uint32_t byte = dw[k >> 2] >> (8 * (k & 3));
+                sum = __builtin_fmaf((float)((int)(byte & 15u) - 8), ctx[32 * part + k], sum);
+                sum = __builtin_fmaf((float)((int)((byte >> 4) & 15u) - 8), ctx[32 * part + 16 + k], sum);
+            }
+            sum = __fmul_rn(from_half_bits(d[i]), sum);
+        }
+        sum += dpp_get<0xB1>(sum);                          // quad_perm [1,0,3,2]
+        if constexpr (LPR >= 4) sum += dpp_get<0x4E>(sum);  // quad_perm [2,3,0,1]
+        if constexpr (LPR == 8) sum += dpp_get<0x141>(sum); // row_half_mirror
+        const int r = (int)blockIdx.y * kProjectRows + i * PASS + tid / LPR;
+        if (part == 0 && i * PASS + tid / LPR < kProjectRows && r < p.rows) p.planes[(size_t)(m * a.n_head + head) * p.rows + r] = head == 0 ? before[i] + sum : sum;
     }
 }
 
@@ -1470,6 +1559,32 @@ template <int HD, int WAVES, int U>
 void launch_attention_partial_shape(const AttentionArgs &a, dim3 grid, bool kv_f16, unsigned heads, hipStream_t s) {
     if (kv_f16) hipLaunchKernelGGL((attention_partial_kernel<HD, true, WAVES, U>), grid, dim3(WAVES * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, a.head_partials, (unsigned)a.cache_seq_stride, heads);
     else hipLaunchKernelGGL((attention_partial_kernel<HD, false, WAVES, U>), grid, dim3(WAVES * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, a.head_partials, (unsigned)a.cache_seq_stride, heads);
+}
+
+// Small models and short contexts.  Every block of rows repeats the head's attention, so its cost grows with wo.rows and the context: 12 heads of 768 rows and up to 512 positions were faster at every position
+// (below), 16 heads of 1024 rows faster from position 16 of 512 (12 layers of Q8_0, 48 tokens: 11.8 ms -> 11.4) and slower from 440 (12.5 -> 12.9, fp16 15.0 -> 15.9).
+bool attention_project_supported(const DeviceMatrix &wo, int n_head, int n_kv_head, int head_dim, int max_seq) {
+    return head_dim == 64 && n_kv_head > 0 && n_head % n_kv_head == 0 && n_head <= kMaxNormPlanes && wo.cols == n_head * 64 && wo.rows <= 768 && wo.rows % 8 == 0 && max_seq <= 512 &&
+           wo.qs && wo.qs_row_bytes % 16 == 0 && wo.qs_row_bytes <= 0xFFFFFFFFull && (wo.format == FMT_F16 || ((wo.format == FMT_Q8_0 || wo.format == FMT_Q4_0) && wo.scales));
+}
+
+template <bool KV_F16, int FMT>
+void launch_attention_project_format(const AttentionArgs &a, const DeviceMatrix &wo, const AttentionProject &p, int rows, hipStream_t s) {
+    const dim3 grid(a.n_head, (wo.rows + kProjectRows - 1) / kProjectRows, rows);
+    const unsigned heads = (unsigned)a.n_head | ((unsigned)a.n_kv_head << 16);
+    // Four wavefronts start and merge sooner, eight walk a longer prefix in fewer passes.  48 tokens, four / eight: 768 wide, 6 layers, Q8_0 from position 16 of 256 5.22 / 5.35 ms, from 200 of 256
+    // 5.61 / 5.61; 576 wide, 30 layers, fp16 and 32-bit caches from 16 of 512 24.1 / 24.6, from 440 of 512 30.1 / 27.8 (sixteen: 28.9).
+    if (a.max_seq <= 256) hipLaunchKernelGGL((attention_project_kernel<KV_F16, FMT, 4, 2>), grid, dim3(256), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, wo.qs, heads, (unsigned)wo.qs_row_bytes, p);
+    else hipLaunchKernelGGL((attention_project_kernel<KV_F16, FMT, 8, 2>), grid, dim3(512), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, wo.qs, heads, (unsigned)wo.qs_row_bytes, p);
+}
+
+hipError_t launch_attention_project(const AttentionArgs &a, const DeviceMatrix &wo, int rows, const float *residual, float *planes, bool kv_f16, hipStream_t s) {
+    if (rows < 1 || rows > 2 || !attention_project_supported(wo, a.n_head, a.n_kv_head, a.head_dim, a.max_seq) || !residual || !planes) return hipErrorInvalidValue;
+    const AttentionProject p{a.cache_seq_stride, wo.scales, residual, planes, wo.rows};
+    if (wo.format == FMT_F16) { if (kv_f16) launch_attention_project_format<true, FMT_F16>(a, wo, p, rows, s); else launch_attention_project_format<false, FMT_F16>(a, wo, p, rows, s); }
+    else if (wo.format == FMT_Q8_0) { if (kv_f16) launch_attention_project_format<true, FMT_Q8_0>(a, wo, p, rows, s); else launch_attention_project_format<false, FMT_Q8_0>(a, wo, p, rows, s); }
+    else { if (kv_f16) launch_attention_project_format<true, FMT_Q4_0>(a, wo, p, rows, s); else launch_attention_project_format<false, FMT_Q4_0>(a, wo, p, rows, s); }
+    return hipGetLastError();
 }
 
 hipError_t launch_attention_partials(const AttentionArgs &a, int rows, bool kv_f16, hipStream_t s) {

@@ -110,6 +110,10 @@ struct KernelArgs {
     // while staging (x and norm_x unused): [batch][cols / head_dim heads][kMergeSplits][head_dim values, m, l, 2 pad]
     const float *merge_partials;
     int merge_head_dim;
+    // when norm_planes is set a row is the sum of its norm_plane_count planes [batch][planes][cols], normed while staging (x, norm_x and merge_partials unused), and the sum is written to norm_sum
+    const float *norm_planes;
+    int norm_plane_count;
+    float *norm_sum;
     // EPI_ARGMAX: one (value, index) pair per workgroup and batch row, [batch][gridDim.x]
     float *part_value;
     int *part_index;
@@ -352,7 +356,7 @@ __device__ __forceinline__ void pair_epilogue(const KernelArgs &a, int pair, con
 // The scalar arguments that the first loads of a GEMV kernel need.  Leading scalar arguments are preloaded
 // into registers with the wavefront's launch; the fields of a structure passed by value are fetched from
 // memory first, which costs the start of every kernel a memory round trip.
-// mode: 0 = fp16 activations, 1 = RMSNorm fused into the staging, 2 = attention partial states (head size in bits 8..).
+// mode: 0 = fp16 activations, 1 = RMSNorm fused into the staging, 2 = attention partial states (head size in bits 8..), 3 = the norm of a sum of planes (their number in bits 8..).
 __device__ __forceinline__ KernelArgs with_leading_args(const KernelArgs &rest, const uint8_t *qs, const uint16_t *scales, const void *activations,
                                                         const float *norm_w, int rows, int cols, int row_bytes, int mode, float norm_eps) {
     KernelArgs a = rest;
@@ -367,12 +371,15 @@ __device__ __forceinline__ KernelArgs with_leading_args(const KernelArgs &rest, 
     a.norm_x = (mode & 0xFF) == 1 ? static_cast<const float *>(activations) : nullptr;
     a.merge_partials = (mode & 0xFF) == 2 ? static_cast<const float *>(activations) : nullptr;
     a.merge_head_dim = mode >> 8;
+    a.norm_planes = (mode & 0xFF) == 3 ? static_cast<const float *>(activations) : nullptr;
+    a.norm_plane_count = mode >> 8;
     return a;
 }
 inline const void *leading_activations(const KernelArgs &a) {
+    if (a.norm_planes) return a.norm_planes;
     return a.merge_partials ? static_cast<const void *>(a.merge_partials) : a.norm_x ? static_cast<const void *>(a.norm_x) : static_cast<const void *>(a.x);
 }
-inline int leading_mode(const KernelArgs &a) { return a.merge_partials ? (2 | (a.merge_head_dim << 8)) : a.norm_x ? 1 : 0; }
+inline int leading_mode(const KernelArgs &a) { return a.norm_planes ? (3 | (a.norm_plane_count << 8)) : a.merge_partials ? (2 | (a.merge_head_dim << 8)) : a.norm_x ? 1 : 0; }
 
 // Dot products, any column count.  Bound by its chain of memory round trips, not by bytes (576 x 576 fp16: 0.7 MB in 5 us), so everything whose
 // address is known is requested at once: the first DEPTH (x 64) items of the wavefront's R rows, the values and norm weights of up to
@@ -400,7 +407,19 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
     const int per_row = cols / (kFours ? 4 : 8), last_group = per_row > 1 ? per_row - 1 : 0;
     float4 nv0[MODE == 1 ? B : 1][KS], nv1[MODE == 1 ? B : 1][KS], ng0[KS], ng1[KS];
     Group xv0[MODE == 0 ? B : 1][KS];
-    if constexpr (MODE != 2) {
+    // planes: four columns a thread, all of them requested at once (those beyond the last repeat it, from the cache), so that they come back in one memory trip, like the finished row of mode 1.  What
+    // they cost beside that (4096 x 768 Q8_0, 12 planes: 5.0 -> 5.5 us) is less than the launch of a product that adds the heads itself.
+    float4 pv[MODE == 3 ? B : 1][MODE == 3 ? kMaxNormPlanes : 1], pg;
+    const int fours = cols / 4, four = tid < fours ? tid : fours - 1;
+    if constexpr (MODE == 3) {
+        const float4 *p4 = reinterpret_cast<const float4 *>(a.norm_planes);
+#pragma unroll
+        for (int b = 0; b < B; b++)
+#pragma unroll
+            for (int k = 0; k < kMaxNormPlanes; k++) pv[b][k] = p4[(b * a.norm_plane_count + (k < a.norm_plane_count ? k : a.norm_plane_count - 1)) * fours + four];
+        pg = reinterpret_cast<const float4 *>(a.norm_w)[four];
+    }
+    if constexpr (MODE < 2) {
 #pragma unroll
         for (int k = 0; k < KS; k++) {
             const int g = tid + k * kThreads < per_row ? tid + k * kThreads : last_group;
@@ -477,7 +496,21 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
                 for (int g = tid + KS * kThreads; g < per_row; g += kThreads) s += sum_squares(x4[2 * g], x4[2 * g + 1]);
                 inv = 1.0f / sqrtf(workgroup_sum(s, norm_red + b * kWaves) / (float)cols + a.norm_eps);
             }
-            if constexpr (MODE != 2) {
+            if constexpr (MODE == 3) {   // the first plane, which holds the residual, last
+                float4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 1; k < kMaxNormPlanes; k++)
+                    if (k < a.norm_plane_count) { v.x += pv[b][k].x; v.y += pv[b][k].y; v.z += pv[b][k].z; v.w += pv[b][k].w; }
+                v.x += pv[b][0].x; v.y += pv[b][0].y; v.z += pv[b][0].z; v.w += pv[b][0].w;
+                const float s = tid < fours ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.0f;
+                inv = 1.0f / sqrtf(workgroup_sum(s, norm_red + b * kWaves) / (float)cols + a.norm_eps);
+                if (tid < fours) {
+                    if (blockIdx.x == 0) reinterpret_cast<float4 *>(a.norm_sum)[b * fours + tid] = v;
+                    const u32 lo = pack_half2(__fmul_rn(__fmul_rn(v.x, inv), pg.x), __fmul_rn(__fmul_rn(v.y, inv), pg.y)), hi = pack_half2(__fmul_rn(__fmul_rn(v.z, inv), pg.z), __fmul_rn(__fmul_rn(v.w, inv), pg.w));
+                    reinterpret_cast<uint2 *>(xs)[b * fours + tid] = T::kPermuteX ? make_uint2(__builtin_amdgcn_perm(hi, lo, 0x05040100u), __builtin_amdgcn_perm(hi, lo, 0x07060302u)) : make_uint2(lo, hi);
+                }
+            }
+            if constexpr (MODE < 2) {
 #pragma unroll
                 for (int k = 0; k < KS; k++)
                     if (tid + k * kThreads < per_row) {
@@ -496,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void gemv_kernel(const uint8_t *qs, const
                     for (int k = 0; k < 4; k++)
                         if (g0 + k * kThreads < per_row) put(b, g0 + k * kThreads, t[k]);
                 }
-            } else {
+            } else if constexpr (MODE != 3) {
                 if constexpr (MODE == 2) {
                     if (tid < per_row) put(b, tid, merge_group(mml[b], mm0[b], mm1[b]));
                 }
@@ -2615,6 +2648,10 @@ hipError_t launch_one(const KernelArgs &a, hipStream_t stream) {
 template <int FMT, int B, int R>
 hipError_t launch_mode(const KernelArgs &a, hipStream_t stream) {
     const int mode = leading_mode(a) & 0xFF;
+    if (mode == 3) {
+        if constexpr (R == 2 && FMT != FMT_F32) return a.cols / Traits<FMT>::kItemElems <= 64 ? launch_one<FMT, B, R, 3, 1>(a, stream) : launch_one<FMT, B, R, 3, 2>(a, stream);
+        return hipErrorInvalidValue;
+    }
     if constexpr (R == 2) {
         if (a.cols / Traits<FMT>::kItemElems <= 64)
             return mode == 1 ? launch_one<FMT, B, R, 1, 1>(a, stream) : mode == 2 ? launch_one<FMT, B, R, 2, 1>(a, stream) : launch_one<FMT, B, R, 0, 1>(a, stream);
@@ -2801,7 +2838,7 @@ hipError_t try_q80_mfma(const KernelArgs &a, hipStream_t stream, bool *launched)
 // fp16 weights (768 and 2048 columns): the same rule
 template <int B>
 hipError_t launch_f16(const KernelArgs &a, hipStream_t stream) {
-    if (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192))) {
+    if (!a.norm_planes && (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192)))) {
         bool launched = false;
         const hipError_t e = try_q80_mfma<B, true>(a, stream, &launched);
         if (e != hipSuccess || launched) return e;
@@ -2814,7 +2851,7 @@ hipError_t launch_q80(const KernelArgs &a, hipStream_t stream) {
     // measured (us, dot-product / matrix cores): one row 2304 x 768 2.74 / 2.96, 4096 x 768 3.08 / 3.22, 768 x 2048 3.01 / 3.00, 4096 x 4096
     // 6.36 / 5.52, 32000 x 768 9.26 / 6.76, 32000 x 4096 31.5 / 26.9; two rows 3.36 / 3.17, 3.77 / 3.31, 3.47 / 3.36, 7.23 / 5.69, 12.1 / 6.8, 32.8 / 27.6:
     // two rows always, one row where the matrix is tall or wide ("q80_mfma" = 1: wherever an instantiation exists)
-    if (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192 || a.cols >= 4096))) {
+    if (!a.norm_planes && (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192 || a.cols >= 4096)))) {
         bool launched = false;
         const hipError_t e = try_q80_mfma<B>(a, stream, &launched);
         if (e != hipSuccess || launched) return e;
@@ -2824,7 +2861,7 @@ hipError_t launch_q80(const KernelArgs &a, hipStream_t stream) {
 
 template <int B>
 hipError_t launch_q40(const KernelArgs &a, hipStream_t stream) {
-    if (q40_mfma_mode() == 1 || (q40_mfma_mode() < 0 && (B >= 2 || a.rows >= 2048))) {
+    if (!a.norm_planes && (q40_mfma_mode() == 1 || (q40_mfma_mode() < 0 && (B >= 2 || a.rows >= 2048)))) {
         bool launched = false;
         const hipError_t e = try_q40_mfma<B>(a, stream, &launched);
         if (e != hipSuccess || launched) return e;
@@ -2832,6 +2869,12 @@ hipError_t launch_q40(const KernelArgs &a, hipStream_t stream) {
     return launch_fmt<FMT_Q4_0>(a, B, stream);
 }
 }  // namespace
+
+// The dot-product kernel's matrices, at the sizes where it takes one row of fp16 and Q8_0 anyway.  One row of 2048 or more Q4_0 rows is the matrix-core kernel's, so there this kernel has to cost less than the
+// launch that planes save: 4096 x 768 measured (a step of 768 wide, 6 layers: 122.5 us -> 113.8 at position 40), taller ones not.
+bool gemv_adds_planes(const DeviceMatrix &w) {
+    return ((w.rows <= 8192 && (w.format == FMT_F16 || w.format == FMT_Q8_0)) || (w.rows <= 4096 && w.format == FMT_Q4_0)) && w.cols <= 4 * kThreads && w.cols % 8 == 0;
+}
 
 bool gemv_merges_attention_partials(const DeviceMatrix &w, int batch, int head_dim) {
     if (batch < 1 || batch > 2 || (head_dim != 64 && head_dim != 128) || w.cols % head_dim != 0) return false;
@@ -2930,7 +2973,10 @@ bool gemv_supports_argmax(const DeviceMatrix &w) {
 
 hipError_t launch_gemv(const GemvParams &p, hipStream_t stream) {
     const DeviceMatrix &w = p.w;
-    if (!w.qs || (!p.x && !p.norm_x && !p.merge_partials) || (p.norm_x && !p.norm_w) || w.rows <= 0 || w.cols <= 0 || p.batch <= 0) return hipErrorInvalidValue;
+    if (p.norm_planes && (p.norm_plane_count < 1 || p.norm_plane_count > kMaxNormPlanes || !p.norm_w || !p.norm_sum || p.batch > 2 || p.x || p.norm_x || p.merge_partials || p.split_x || p.sixteen_rows ||
+                          p.epilogue == EPI_ARGMAX || !gemv_adds_planes(w)))
+        return hipErrorInvalidValue;
+    if (!w.qs || (!p.x && !p.norm_x && !p.merge_partials && !p.norm_planes) || (p.norm_x && !p.norm_w) || w.rows <= 0 || w.cols <= 0 || p.batch <= 0) return hipErrorInvalidValue;
     if (p.merge_partials && !gemv_merges_attention_partials(w, p.batch, p.merge_head_dim)) return hipErrorInvalidValue;
     if ((p.epilogue == EPI_STORE_F32 || p.epilogue == EPI_ADD_RESIDUAL) && !p.y) return hipErrorInvalidValue;
     if (p.epilogue == EPI_ADD_RESIDUAL && !p.residual) return hipErrorInvalidValue;
@@ -2998,6 +3044,9 @@ hipError_t launch_gemv(const GemvParams &p, hipStream_t stream) {
         a.norm_x = p.norm_x ? p.norm_x + (size_t)b0 * w.cols : nullptr;
         a.norm_w = p.norm_w;
         a.norm_eps = p.norm_eps;
+        a.norm_planes = p.norm_planes;   // batch <= 2 here: one launch
+        a.norm_plane_count = p.norm_plane_count;
+        a.norm_sum = p.norm_sum;
         hipError_t e;
         switch (w.format) {
         case FMT_Q4_K:

@@ -82,6 +82,12 @@ bool LlamaRuntime::wo_merges_attention(const Layer &L, int rows) const {
            L.wo.cols == c_.attention_dim() && gemv_merges_attention_partials(L.wo, rows, c_.head_dim);
 }
 
+// Small models, one row or two: five launches a layer are four.  Both counts, so that a row is the same alone and beside another.
+bool LlamaRuntime::projects_attention(const Layer &L, int rows) const {
+    return merged_attention_ && rows <= 2 && attention_project_supported(L.wo, c_.n_head, c_.n_kv_head, c_.head_dim, c_.max_seq) && gemv_adds_planes(L.w13) && L.w13.cols == L.wo.rows &&
+           (size_t)rows * (c_.n_head + 1) * c_.d_model <= gemm_workspace_floats_;
+}
+
 int LlamaRuntime::time_kernel_class(int kernel_class, int iters, double *mean_us, double *kernel_only_us) {
     if (!finalized_ || iters < 1 || !mean_us) return fail(ESP_ERR_INVALID_ARGUMENT, "time_kernel_class: bad argument");
     if (kernel_class < K_QKV || kernel_class > K_HEAD) return fail(ESP_ERR_INVALID_ARGUMENT, "time_kernel_class: class %d", kernel_class);
@@ -439,22 +445,29 @@ int LlamaRuntime::enqueue_trunk(int M, bool embedded, float *final_out) {
         aa.split_scratch = attn_scratch_;
         aa.head_partials = attn_scratch_;
         // one attention launch instead of two where the wo GEMV can merge the partial states in its staging
-        const bool merge_in_wo = wo_merges_attention(L, M);
+        const bool project = projects_attention(L, M);   // one launch for attention and wo, whose planes the gate|up GEMV adds
+        float *const planes = gemm_workspace_, *const joined = gemm_workspace_ + (size_t)M * c_.n_head * d;
+        const bool merge_in_wo = !project && wo_merges_attention(L, M);
         if ((rc = time_begin(K_ATTENTION)) != ESP_OK) return rc;
-        if (merge_in_wo) ESP_HIP_TRY(launch_attention_partials(aa, M, kv16, s));
+        if (project) ESP_HIP_TRY(launch_attention_project(aa, L.wo, M, hidden_, planes, kv16, s));
+        else if (merge_in_wo) ESP_HIP_TRY(launch_attention_partials(aa, M, kv16, s));
         else ESP_HIP_TRY(launch_attention(aa, M, kv16, s));
         if ((rc = time_end()) != ESP_OK) return rc;
         g = GemvParams{};
         g.batch = M;
         g.w = L.wo; g.x = ctx_; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL;
-        if (merge_in_wo) {
-            g.x = nullptr; g.merge_partials = attn_scratch_; g.merge_head_dim = c_.head_dim;
-            g.split_x = split_activations_ && gemv_splits_activations(L.wo, M);   // the merge leaves fp32 values to split
+        if (!project) {
+            if (merge_in_wo) {
+                g.x = nullptr; g.merge_partials = attn_scratch_; g.merge_head_dim = c_.head_dim;
+                g.split_x = split_activations_ && gemv_splits_activations(L.wo, M);   // the merge leaves fp32 values to split
+            }
+            if ((rc = time_begin(K_WO)) != ESP_OK) return rc;
+            ESP_HIP_TRY(launch_gemv(g, s));
+            if ((rc = time_end()) != ESP_OK) return rc;
         }
-        if ((rc = time_begin(K_WO)) != ESP_OK) return rc;
-        ESP_HIP_TRY(launch_gemv(g, s));
-        if ((rc = time_end()) != ESP_OK) return rc;
-        g.w = L.w13; g.x = nullptr; g.merge_partials = nullptr; g.norm_x = hidden_; g.norm_w = L.rms_ffn; g.norm_eps = c_.norm_eps;
+        g.w = L.w13; g.x = nullptr; g.merge_partials = nullptr; g.norm_w = L.rms_ffn; g.norm_eps = c_.norm_eps;
+        if (project) { g.norm_planes = planes; g.norm_plane_count = c_.n_head; g.norm_sum = joined; }
+        else g.norm_x = hidden_;
         g.y = nullptr; g.residual = nullptr; g.out_f16 = act_; g.epilogue = EPI_SWIGLU_F16;
         const bool split_down = split_activations_ && gemv_splits_activations(L.w2, M);   // act_ then holds hi / lo row pairs
         g.split_x = split_activations_ && gemv_splits_activations(L.w13, M);
@@ -462,9 +475,9 @@ int LlamaRuntime::enqueue_trunk(int M, bool embedded, float *final_out) {
         if ((rc = time_begin(K_GATE_UP)) != ESP_OK) return rc;
         ESP_HIP_TRY(launch_gemv(g, s));
         if ((rc = time_end()) != ESP_OK) return rc;
-        g.w = L.w2; g.x = act_; g.norm_x = nullptr; g.norm_w = nullptr; g.split_x = split_down; g.split_out = false;
+        g.w = L.w2; g.x = act_; g.norm_x = nullptr; g.norm_planes = nullptr; g.norm_w = nullptr; g.split_x = split_down; g.split_out = false;
         g.y = final_out && &L == &layers_.back() ? final_out : hidden_;   // the last layer's output may go straight to its keeper
-        g.residual = hidden_; g.out_f16 = nullptr; g.epilogue = EPI_ADD_RESIDUAL;
+        g.residual = project ? joined : hidden_; g.out_f16 = nullptr; g.epilogue = EPI_ADD_RESIDUAL;
         if ((rc = time_begin(K_DOWN)) != ESP_OK) return rc;
         ESP_HIP_TRY(launch_gemv(g, s));
         if ((rc = time_end()) != ESP_OK) return rc;

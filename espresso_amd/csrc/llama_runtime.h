@@ -111,6 +111,7 @@ class LlamaRuntime : public DecoderRuntime {
     bool short_split_blocks_supported() const;
     bool splits_every_product() const;
     bool wo_merges_attention(const Layer &L, int rows) const;
+    bool projects_attention(const Layer &L, int rows) const;
     HostTensor *host_slot(int layer, int slot);
 
     LlamaConfig c_;

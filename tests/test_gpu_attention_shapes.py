@@ -47,3 +47,32 @@ def test_attention_shape_for_the_context_size_matches_oracle(mods, head_dim, max
         o.advance(t)
         g.advance(t)
     g.close()
+
+
+# One row of a small model: attention and wo are one launch, its workgroups 64 rows of wo each, and the gate|up GEMV adds the heads' planes.  Passes of a workgroup are 64 positions up to a context of 256 and
+# 128 up to 512; rows beside a multiple of 64, one head and the most; the last two are one head, one context too many.
+@pytest.mark.parametrize("n_head,n_kv,d_model,fmt,kv_fp16,max_seq,prompt_len", [
+    (1, 1, 64, orc.FMT_F16, False, 256, 1), (3, 1, 200, orc.FMT_F16, True, 256, 62), (12, 12, 768, orc.FMT_Q4_0, False, 256, 252),
+    (9, 3, 576, orc.FMT_Q8_0, False, 512, 126), (4, 2, 256, orc.FMT_Q4_0, True, 512, 254), (12, 4, 768, orc.FMT_Q8_0, True, 512, 508),
+    (12, 12, 768, orc.FMT_F16, False, 512, 62), (13, 1, 256, orc.FMT_F16, False, 512, 20), (2, 2, 128, orc.FMT_Q8_0, True, 513, 20),
+])
+def test_attention_and_projection_in_one_launch_match_oracle(mods, n_head, n_kv, d_model, fmt, kv_fp16, max_seq, prompt_len):
+    ll, ops, syn = mods
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=n_head, n_kv_head=n_kv, d_model=d_model, head_dim=64, hidden_dim=256, vocab=512, max_seq=max_seq, norm_eps=1e-5, rope_theta=10000.0,
+                              name="attention-projection")
+    g, packed = syn.build_runtime(cfg, fmt, seed=n_head + max_seq, std=0.05, keep_packed=True, kv_format=orc.FMT_F16 if kv_fp16 else orc.FMT_F32)
+    o = oracle_from_packed(cfg, packed, fmt, 2, kv_fp16, max_seq)
+    prompt = [int(t) for t in np.random.default_rng(prompt_len).integers(0, cfg.vocab, prompt_len)]
+    o.prefill(prompt)
+    g.prefill(np.asarray(prompt, np.uint32))
+    for step in range(3):
+        t = o.select_greedy()
+        o.advance(t)
+        g.advance(t)
+        ho, hg = o.last_hidden(), g.last_hidden()
+        assert np.abs(ho - hg).max() <= 2e-3 * max(1.0, np.abs(ho).max()), (step, np.abs(ho - hg).max())
+        assert np.abs(o.logits() - g.logits()).max() <= 2e-2
+    ll.set_kernel_timing(g, True)
+    g.advance(0)
+    assert (ll.kernel_times(g)["wo"]["launches"] == 0) == (n_head <= 12 and max_seq <= 512)
+    g.close()
