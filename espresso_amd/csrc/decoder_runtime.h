@@ -75,6 +75,8 @@ class DecoderRuntime {
     int append(int seq, const uint32_t *tokens, int count, const int *want = nullptr, int want_count = 0, float *logits = nullptr);
     // Final norm + LM head + first-max argmax of kept hidden states (:663-670, :825-849).
     int select_greedy(int seq, uint32_t *token);
+    // The same for the sequences 0 .. count - 1, with the head read once for all of them where that is as exact.
+    int select_greedy_rows(int count, uint32_t *tokens);
     // Head over rows of the most recent forward_rows(); tokens[i] for row i.
     int head_rows(int count, uint32_t *tokens);
     // Keep row `row` of the most recent forward_rows() as sequence `seq`'s last hidden state.
@@ -128,6 +130,9 @@ class DecoderRuntime {
     virtual int enqueue_trunk(int rows, bool embedded = false, float *final_out = nullptr) = 0;
     // want_logits: the full-vocabulary logits are needed in logits_ (otherwise the head may store none)
     virtual int run_head(const float *hidden_rows, int count, bool want_logits = false) = 0;
+    int select_rows(const float *hidden_rows, int count, uint32_t *tokens);   // run_head and its tokens
+    // Does run_head round the rows of a batch no more than a single one?
+    virtual bool head_is_as_exact_for_rows() const { return false; }
     // One greedy choice under capture: head over the sequence's kept state, the token into row 0 and the log, and what
     // enqueue_trunk(1, true) needs of its embedding.
     virtual int enqueue_greedy_token(int seq) = 0;

@@ -147,10 +147,8 @@ int generate_greedy_batch(DecoderRuntime &rt, const uint32_t *const *prompts, co
     auto t0 = Clock::now();
     if (eff > 0) {
         std::vector<uint32_t> current(n_seq);
-        for (int s = 0; s < n_seq; s++) {
-            if ((rc = rt.select_greedy(s, &current[s])) != ESP_OK) return rc;
-            (*out)[s].push_back(current[s]);
-        }
+        if ((rc = rt.select_greedy_rows(n_seq, current.data())) != ESP_OK) return rc;
+        for (int s = 0; s < n_seq; s++) (*out)[s].push_back(current[s]);
         int first_host_step = 1;
         if (rt.graph_replay_enabled() && eff > 2) {
             // every step but none of the decisions needs the host: rows feed themselves on the device, one graph per step

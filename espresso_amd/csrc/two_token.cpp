@@ -267,10 +267,8 @@ int generate_two_token_batch(LlamaRuntime &full, LlamaRuntime &draft, const uint
     auto t0 = Clock::now();
     std::vector<uint32_t> current(n_seq);
     if (eff > 0) {
-        for (int s = 0; s < n_seq; s++) {
-            if ((rc = full.select_greedy(s, &current[s])) != ESP_OK) return rc;
-            (*out)[s].push_back(current[s]);
-        }
+        if ((rc = full.select_greedy_rows(n_seq, current.data())) != ESP_OK) return rc;
+        for (int s = 0; s < n_seq; s++) (*out)[s].push_back(current[s]);
     }
     if (full.graph_replay_enabled() && draft.graph_replay_enabled() && &full != &draft && eff > 2 && n_seq <= kMaxLoopSequences) {
         // the passes run on the device: per-sequence variables in TwoTokenBatchState, rows 2 s and 2 s + 1 of both models belong to

@@ -176,3 +176,18 @@ def test_device_loop_session_is_reused_and_rebuilt(llama):
         assert tokens == seen[0]
     for rt in (target, draft_a, draft_b):
         rt.close()
+
+
+@pytest.mark.parametrize("fmt", [orc.FMT_Q8_0, orc.FMT_F16])
+@pytest.mark.parametrize("n_seq", [1, 2, 3, 16])
+def test_first_tokens_of_a_batch_are_those_of_its_sequences(llama, fmt, n_seq):
+    """The head over the kept rows of all sequences at once against one sequence at a time (margins of 1e-3 and more)."""
+    rt = build_batch(llama, weights(fmt, 31, 2), fmt, 2, 64, n_seq)
+    rng = np.random.default_rng(n_seq)
+    prompts = [rng.integers(0, BASE["vocab"], 3 + s % 5).astype(np.uint32) for s in range(n_seq)]
+    got = llama.generate_batch(rt, prompts, 1)[0]
+    for s in range(n_seq):
+        top = np.sort(rt.logits(s))[-2:]
+        if top[1] - top[0] > 1e-3:
+            assert got[s] == [rt.select_greedy(s)]
+    rt.close()
