@@ -4,7 +4,7 @@
 //   mixed row   [q: heads | k: kv_heads | v: kv_heads], heads padded; a layer that reads another one's cache has q alone
 //   cached row  [k: kv_heads x dim_p | v: kv_heads x vdim_p], one per token, at position % ring, keys normed and rotated
 //
-// A decode step is two launches.  partial: a workgroup takes a slice of the window for the query heads of one key head; it norms and
+// A decode step of one row or a few with a short window is one launch (attention_window_kernel).  Otherwise it is two.  partial: a workgroup takes a slice of the window for the query heads of one key head; it norms and
 // rotates their queries itself (the norm's sum runs over the whole projection, which every workgroup reads), and the workgroup whose
 // slice holds the row's own token puts its key and value into the cache first.  Eight lanes share a key, so a key is read once for all
 // query heads of the group.  merge: the slices' (maximum, sum, weighted values) joined.
@@ -273,6 +273,153 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttentionShape l, 
     }
 }
 
+// One element of a head before its norm is known: what normed_rotated reads.
+struct Element {
+    float u, v, wu, wv, c, s;
+    __device__ __forceinline__ void load(const float *x, const float *w, int d, int dims, const float *cos, const float *sin) {
+        const int half = dims / 2, i = d < dims && d >= half ? d - half : d, j = d < dims ? i + half : d;
+        u = x[i]; v = x[j]; wu = w[i]; wv = w[j];
+        c = d < dims ? cos[i] : 1.0f;
+        s = d < dims ? sin[i] : 0.0f;
+    }
+    __device__ __forceinline__ float value(float inv, int d, int dims) const {
+        if (d >= dims) return u * inv * wu;
+        const float x = u * inv * wu, y = v * inv * wv;
+        return d < dims / 2 ? x * c - y * s : y * c + x * s;
+    }
+};
+
+constexpr int kWindowHead = 128, kWindowSlice = 32, kWindowKeys = 128;   // longest key; values of a workgroup, keys of a pass
+// A short window in one launch: grid (heads x slices of 32 values, rows).  Bound by its chain of memory trips, position -> keys and values -> store, so sixteen wavefronts ask for all of the window's keys (eight lanes a
+// key) and their slice of its values (four lanes a key) at once, together with what the norms and the rotation read; a workgroup needs every score of its head, which is why keys are read once per slice, from the cache
+// after the first.  No state passes between workgroups, and no sum is rescaled: maximum, weights and sum are taken over the whole window.  Window of 256, heads of 128: 7 us instead of 8.7 + 4.7 for slices and their merge.
+template <typename T, int PASSES>
+__global__ __launch_bounds__(1024) void attention_window_kernel(AttentionShape l, AttentionStep p) {
+    constexpr int VP = PASSES / 2;   // passes over the values: 256 keys each
+    static_assert(PASSES % 2 == 0, "whole passes over the values");
+    __shared__ float q[kWindowHead], own_key[kWindowHead], own_value[kWindowSlice], scores[256 * VP], red[2][16], meet[64][kWindowSlice];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slices = l.vdim_p / kWindowSlice, h = blockIdx.x / slices, slice = blockIdx.x % slices, m = blockIdx.y;
+    const int share = l.heads / l.kv_heads, kv = h / share, width = cached_row(l), count_q = l.heads * l.dim_p, count_k = l.k_at >= 0 ? l.kv_heads * l.dim_p : 0;
+    const float *row = p.mixed + (size_t)m * l.ld_mix, *row_k = row + (l.k_at >= 0 ? l.k_at : 0);
+    // whatever the position: the norms' first values
+    const float4 first_q = *reinterpret_cast<const float4 *>(row + (tid * 4 < count_q ? tid * 4 : 0)), first_k = *reinterpret_cast<const float4 *>(row_k + (tid * 4 < count_k ? tid * 4 : 0));
+    const int pos = p.pos[m], seq = p.seq[m];
+    const int lo = first_seen(pos, l.window), keys = pos - lo + 1;
+    const float *cos = l.cos + (size_t)pos * (l.rot_dims / 2), *sin = l.sin + (size_t)pos * (l.rot_dims / 2);
+    T *cache = static_cast<T *>(l.cache) + (size_t)seq * l.ring * width;
+    auto row_of = [&](int i) { return (size_t)((i < keys ? lo + i : pos) % l.ring) * width; };   // keys past the query repeat it and weigh nothing
+    const int e = tid & 7, key_in = tid >> 3, piece = tid & 3, value_in = tid >> 2;
+    Piece<T> key_piece[PASSES][2], value_piece[VP];
+#pragma unroll
+    for (int k = 0; k < PASSES; k++) {
+        const T *from = cache + kv * l.dim_p + row_of(k * kWindowKeys + key_in);
+#pragma unroll
+        for (int i = 0; i < 2; i++) key_piece[k][i].load(from + (e * 8 + i * 64 < l.dim_p ? e * 8 + i * 64 : 0));
+    }
+#pragma unroll
+    for (int k = 0; k < VP; k++) value_piece[k].load(cache + l.kv_heads * l.dim_p + kv * l.vdim_p + slice * kWindowSlice + piece * 8 + row_of(k * 256 + value_in));
+    const int d = tid & 127;
+    const bool makes_q = tid < l.dim_p, makes_k = tid >= 128 && tid < 128 + l.dim_p && count_k > 0, makes_v = tid >= 256 && tid < 256 + kWindowSlice && count_k > 0;
+    const bool keeps = count_k > 0 && h % share == 0 && slice == 0;   // one workgroup of a key head puts the row's own key and value into the cache
+    const float *row_v = row_k + count_k + kv * l.vdim_p;
+    Element x = {};
+    float v = 0.0f;
+    if (makes_q) x.load(row + h * l.dim_p, l.q_norm + h * l.dim_p, d, l.rot_dims, cos, sin);
+    if (makes_k) x.load(row_k + kv * l.dim_p, l.k_norm + kv * l.dim_p, d, l.rot_dims, cos, sin);
+    if (makes_v) v = row_v[slice * kWindowSlice + tid - 256];
+    __builtin_amdgcn_sched_barrier(0);   // all of it is requested before anything is waited for
+    auto dot4 = [](const float4 &f) { return f.x * f.x + f.y * f.y + f.z * f.z + f.w * f.w; };
+    float sq = tid * 4 < count_q ? dot4(first_q) : 0.0f, sk = tid * 4 < count_k ? dot4(first_k) : 0.0f;
+    for (int i = 4096 + tid * 4; i < count_q; i += 4096) sq += dot4(*reinterpret_cast<const float4 *>(row + i));
+    for (int i = 4096 + tid * 4; i < count_k; i += 4096) sk += dot4(*reinterpret_cast<const float4 *>(row_k + i));
+    sq = detail::wave_sum(sq);
+    sk = detail::wave_sum(sk);
+    if (lane == 0) { red[0][wave] = sq; red[1][wave] = sk; }
+    __syncthreads();
+    sq = 0.0f;
+    sk = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) { sq += red[0][i]; sk += red[1][i]; }
+    if (makes_q) q[d] = l.scale * x.value(1.0f / sqrtf(sq / ((float)l.heads * (float)l.dim) + l.eps), d, l.rot_dims);
+    T *own = cache + (size_t)(pos % l.ring) * width;
+    if (makes_k) {
+        const T k = Op<T>::from_float(x.value(1.0f / sqrtf(sk / ((float)l.kv_heads * (float)l.dim) + l.eps), d, l.rot_dims));
+        if (keeps) own[kv * l.dim_p + d] = k;
+        own_key[d] = Op<T>::to_float(k);
+    }
+    if (makes_v) own_value[tid - 256] = Op<T>::to_float(Op<T>::from_float(v));
+    if (keeps)
+        for (int i = tid - 512; i < l.vdim_p; i += 512)
+            if (i >= 0) own[l.kv_heads * l.dim_p + kv * l.vdim_p + i] = Op<T>::from_float(row_v[i]);
+    __syncthreads();
+    auto own_or = [&](const Piece<T> &from, bool own_row, const float *own_at, float (&f)[8]) __attribute__((always_inline)) {
+        from.unpack(f);
+        if (own_row) load8(own_at, f);
+    };
+#pragma unroll
+    for (int k = 0; k < PASSES; k++) {
+        const int i = k * kWindowKeys + key_in;
+        float s = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int at = e * 8 + c * 64;
+            if (at < l.dim_p) {
+                float f[8], y[8];
+                own_or(key_piece[k][c], count_k > 0 && i >= keys - 1, own_key + at, f);
+                load8(q + at, y);
+#pragma unroll
+                for (int j = 0; j < 8; j++) s = __builtin_fmaf(f[j], y[j], s);
+            }
+        }
+        s += detail::dpp_term<0xB1, 0xF>(s);
+        s += detail::dpp_term<0x4E, 0xF>(s);
+        s += detail::dpp_term<0x141, 0xF>(s);
+        if (e == 0) scores[i] = i < keys ? s : -INFINITY;
+    }
+    __syncthreads();
+    // every wavefront has the maximum and the sum by itself
+    float top = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4 * VP; k++) top = fmaxf(top, scores[k * 64 + lane]);
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) top = fmaxf(top, __shfl_xor(top, k));
+#pragma unroll
+    for (int k = 0; k < 4 * VP; k++) sum += matrix::weight_exp<T>(scores[k * 64 + lane] - top);
+    sum = detail::wave_sum(sum);
+    float acc[8] = {};
+#pragma unroll
+    for (int k = 0; k < VP; k++) {
+        const int i = k * 256 + value_in;
+        const float w = matrix::weight_exp<T>(scores[i] - top);
+        float f[8];
+        own_or(value_piece[k], count_k > 0 && i >= keys - 1, own_value + piece * 8, f);
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[j] = __builtin_fmaf(w, f[j], acc[j]);
+    }
+    // lanes of a row of sixteen with the same values, then the 64 rows in LDS
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        acc[j] += detail::dpp_term<0x128, 0xF>(acc[j]);   // row_ror 8
+        acc[j] += detail::dpp_term<0x124, 0xF>(acc[j]);   // row_ror 4
+    }
+    if ((lane & 15) < 4) {
+        float4 *to = reinterpret_cast<float4 *>(&meet[tid >> 4][piece * 8]);
+        to[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        to[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    }
+    __syncthreads();
+    if (wave) return;
+    float o = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) o += meet[(lane >> 5) * 32 + i][lane & 31];
+    o += __shfl_xor(o, 32);
+    if (lane >= kWindowSlice) return;
+    o /= sum;
+    const int at = h * l.vdim_p + slice * kWindowSlice + lane;
+    if (p.mix) p.mix[(size_t)m * l.heads * l.vdim_p + at] = o;
+    else static_cast<T *>(p.act)[(size_t)m * p.ld_act + at] = Op<T>::from_float(o);
+}
+
 // ---- prompt blocks ---------------------------------------------------------------------------------------
 // One workgroup per row: queries normed and rotated to [heads][rows_p][dim_p] (rows past the block are zero), keys and values to the ring.
 template <typename T>
@@ -356,6 +503,14 @@ hipError_t run_partial(const AttentionShape &l, const AttentionStep &p, hipStrea
 template <typename T>
 hipError_t run_step(const AttentionShape &l, const AttentionStep &p, hipStream_t s) {
     hipError_t e;
+    const int span = l.window < l.max_seq ? l.window : l.max_seq;
+    // Windows that a workgroup's registers hold, and as many workgroups as there are compute units: every one of them reads all keys of its head.  Layers of 16 heads of 128, four key heads (64 workgroups a row), us a
+    // layer and step, two launches / one: window 256, one row 13.4 / 7, 512 bf16 13.4 / 9 (1024, two spans of registers: 13.4 / 15; 512 fp32: the same); a generation of 4 rows 11.4 / 11.2 ms, of 16 rows 20.2 / 20.5.
+    if (const dim3 grid(l.heads * (l.vdim_p / kWindowSlice), p.rows); l.dim_p <= kWindowHead && (long)grid.x * grid.y <= 256 && span <= (sizeof(T) == 2 ? 512 : 256)) {
+        if (span <= 256) hipLaunchKernelGGL((attention_window_kernel<T, 2>), grid, dim3(1024), 0, s, l, p);
+        else if constexpr (sizeof(T) == 2) hipLaunchKernelGGL((attention_window_kernel<T, 4>), grid, dim3(1024), 0, s, l, p);
+        return hipGetLastError();
+    }
     switch (heads_together(l)) {
         case 1: e = run_partial<T, 1>(l, p, s); break;
         case 2: e = run_partial<T, 2>(l, p, s); break;

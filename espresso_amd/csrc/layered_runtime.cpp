@@ -235,7 +235,7 @@ int LayeredRuntime::enqueue_trunk(int rows, bool, float *final_out) {
     return rows == 1 ? enqueue_step(final_out) : enqueue_block(rows, -1, 0, final_out);
 }
 
-// One row: three launches per recurrent layer, four or five per attention layer, two more for a feed-forward of its own.
+// One row: three launches per recurrent layer, three to five per attention layer, two more for a feed-forward of its own.
 int LayeredRuntime::enqueue_step(float *final_out) {
     if (c_.block == BlockKind::sequential_post_norms) return enqueue_step_sequential(final_out);
     hipStream_t s = context().stream;

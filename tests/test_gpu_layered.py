@@ -345,6 +345,30 @@ def test_a_marked_key_just_inside_and_just_outside_the_window(tmp_path, window, 
             assert lu.error(lu.feed(rt, t, portions, s), want) < lu.limit(precision), (precision, portions)
 
 
+# A step's attention is one launch for windows of up to 512 (fp32 256) and heads of up to 128, in as many workgroups as compute units (heads x slices of 32 values x rows <= 256), otherwise two.
+@pytest.mark.parametrize("window,heads,kv_heads,dim,vdim", [(1, 2, 1, 128, 32), (129, 5, 1, 96, 40), (255, 4, 2, 128, 128), (256, 3, 3, 128, 160), (257, 4, 4, 40, 24), (511, 2, 1, 128, 64), (512, 8, 2, 64, 33),
+                                                            (513, 2, 2, 128, 32), (256, 2, 1, 129, 32)])
+def test_windows_in_one_launch_and_in_two(tmp_path, window, heads, kv_heads, dim, vdim):
+    form = dict(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, dims=dim // 2 // 2 * 2, ff=0)
+    m = lu.Model(tmp_path, lu.sequential([lu.attention(window=window, **form), lu.attention(window=window, kv_from=0, **form)]), seed=window, gain=1.5)
+    t = lu.tokens(m.cfg, window + 40, 4)
+    want = m.logits(t)
+    for precision in ("f32", "bf16"):
+        rt = m.runtime(precision, max_seq=window + 60)
+        for s, first in enumerate((window - 10 if window > 10 else 1, window + 20)):
+            assert lu.error(lu.feed(rt, t, [first, 1], s), want) < lu.limit(precision), (precision, first)
+
+
+@pytest.mark.parametrize("n_seq", [2, 4, 5])
+def test_windows_of_several_rows(tmp_path, n_seq):
+    m = lu.Model(tmp_path, lu.sequential([lu.attention(window=70, heads=16, kv_heads=4, dim=32, vdim=128)]), seed=6, gain=1.5)   # 64 workgroups a row
+    rt = m.runtime("f32", max_seq=160, sequences=n_seq)
+    prompts = [lu.tokens(m.cfg, n, 90 + n) for n in (3, 75, 17, 64, 1)[:n_seq]]
+    got, _ = ll.generate_batch(rt, prompts, 12)
+    for p, g in zip(prompts, got):
+        assert g == m.greedy(p, 12)
+
+
 @pytest.mark.parametrize("name,a_log,dt_bias,dt_gain", [("nothing is forgotten", -30.0, -1.0, 1.0), ("everything is forgotten", 5.0, 2.0, 1.0), ("now and then everything is forgotten", 3.5, -6.0, 9.0),
                                                         ("large steps", -8.0, 30.0, 1.0), ("steps of almost nothing", 0.0, -14.0, 0.1)])
 def test_states_from_kept_to_forgotten(tmp_path, name, a_log, dt_bias, dt_gain):
