@@ -827,7 +827,7 @@ struct AttentionProject {
 };
 // Attention and output projection of one row or two in one launch: grid (query heads, blocks of 64 rows of wo, rows).  A workgroup attends for its head over the whole prefix, as every other
 // workgroup of the head does, and multiplies the context with its rows' 64 columns of that head; the heads' products are planes [row][heads][wo.rows] that the next norm adds
-// (GemvParams::norm_planes), the first with the residual in it.  Nothing of the context is rounded.  Bound by the launch, like everything beside it, and by its chain of memory trips: position ->
+// (GemvParams::norm_planes), the first with the residual in it.  The context is rounded to fp16 as in a block of rows, whose logits a step's are held to.  Bound by the launch, like everything beside it, and by its chain of memory trips: position ->
 // keys and values -> store; weights and residual are requested first.  In place of partial states and a GEMV that merges them, a step of 768 wide, 6 layers, Q8_0 went from 117 to 105 us, of 576
 // wide, 30 layers, fp16 from 580 to 528, and a speculative pass of the former (two rows) from 6.5 to 6.3 ms a generation of 64 tokens.
 template <bool KV_F16, int FMT, int WAVES, int U>
@@ -865,7 +865,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_project_kernel(const flo
             L = __builtin_fmaf(wl[v], f, L);
             A = __builtin_fmaf(wacc[v][tid], f, A);
         }
-        ctx[tid] = L > 0.0f ? A / L : 0.0f;
+        ctx[tid] = from_half_bits(to_half_bits(L > 0.0f ? A / L : 0.0f));
     }
     __syncthreads();
 #pragma unroll
