@@ -453,7 +453,7 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     if (!kv_f16) {
         while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
     } else {
-        const int forced = g_key_sets.load();
+        const int forced = rows < 32 ? 0 : g_key_sets.load();   // (short blocks are by size whatever the key says)
         sets = forced ? 4 * forced : tiles >= 24 && groups <= cus ? 8 : 4;
     }
     if (a.head_dim == 128) {
