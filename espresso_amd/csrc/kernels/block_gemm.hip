@@ -5,7 +5,10 @@
 // 8 / NW groups share K; each wavefront owns 32 weight rows and all 32 TM activation rows of the workgroup's tile.
 //   * The weights never enter LDS: a lane unpacks eight k of its own row into the B operand of v_mfma_f32_32x32x16_f16, which then serves TM products.
 //   * Four lanes cover 64 bytes of a row (sixteen rows a load), and v_permlane16_swap brings each lane the two pieces of its own row: a quarter to a half of the cache
-//     accesses of lanes that read their own rows.
+//     accesses of lanes that read their own rows.  Those lanes are sixteen apart, so the cache still looks every sixteen bytes up by themselves; Q8_0, which has two such loads for each of the others',
+//     takes neighbouring lanes and turns the rows in LDS, one fragment ahead of their use.  us, exchanged -> turned: 2048 x 5632, 33 / 93 / 512 rows 11.7 / 13.6 / 27.8 -> 10.8 / 12.4 / 26.2;
+//     2560 x 2048 exact, 33 / 64 / 93 rows 9.5 / 10.3 / 10.2 -> 8.8 / 9.3 / 8.4;  11264 x 2048, 64 / 320 / 512 rows 16.8 / 33.8 / 42.1 -> 15.1 / 30.3 / 40.4, 1777 rows the same.  The others
+//     lose 2 to 10 % by the longer way (3072 x 2048 Q4_0, 64 rows 7.7 -> 9.6; 3072 x 8192 Q4_K, 33 rows 13.3 -> 15.4).
 //   * Loads are spread over the step, one step of 128 k ahead: more in flight only blocks the wavefronts that issue them (two steps ahead, requested in one go:
 //     11264 x 2048 Q8_0, 512 rows 38.8 us, 16 rows 11.9 against 37.8 and 11.6; 3072 x 8192 Q4_0, 512 rows 35.9 against 33.9).
 //   * Activations go through LDS, two buffers and one barrier a step, fragment g + 1 read while g is multiplied (left to the compiler: 3 to 5 % slower).
@@ -26,6 +29,7 @@ namespace esp {
 namespace {
 
 using namespace block_tile;
+typedef u32 uintx4 __attribute__((ext_vector_type(4)));
 
 struct BlockArgs {
     const uint8_t *qs;
@@ -47,11 +51,15 @@ __device__ __forceinline__ uint4 swap_middle(const uint4 &v) {
 }
 constexpr int pairs_of(int fmt) { return fmt == FMT_Q8_0 ? 2 : 1; }   // 64-byte stretches of a row in a step
 
-template <int TM, int NW>
-constexpr int block_buffers() { return 2 * (kWaves / NW) * 32 * TM * kRow * 2 <= 160 * 1024 ? 2 : 1; }
-template <int TM, int NW>
+// Weights through LDS on their way to the lanes of their rows
+constexpr bool turned(int fmt, int tm, int nw) { return fmt == FMT_Q8_0 && !(tm == 3 && nw == 2); }   // (that form has one buffer for its activations as it is, and was 2 to 5 % slower)
+constexpr int kTurn = 80;                          // bytes between the rows there
+constexpr size_t turn_bytes(int fmt, int tm, int nw) { return turned(fmt, tm, nw) ? (size_t)kWaves * 32 * kTurn : 0; }
+template <int FMT, int TM, int NW>
+constexpr int block_buffers() { return 2 * (kWaves / NW) * 32 * TM * kRow * 2 + turn_bytes(FMT, TM, NW) <= 160 * 1024 ? 2 : 1; }
+template <int FMT, int TM, int NW>
 constexpr size_t block_lds_bytes() {
-    const size_t x = (size_t)block_buffers<TM, NW>() * (kWaves / NW) * 32 * TM * kRow * 2, sums = kWaves / NW > 1 ? (size_t)kWaves * TM * 16 * 64 * 4 : 0;
+    const size_t x = (size_t)block_buffers<FMT, TM, NW>() * (kWaves / NW) * 32 * TM * kRow * 2 + turn_bytes(FMT, TM, NW), sums = kWaves / NW > 1 ? (size_t)kWaves * TM * 16 * 64 * 4 : 0;
     return x > sums ? x : sums;
 }
 
@@ -59,7 +67,7 @@ constexpr size_t block_lds_bytes() {
 template <int FMT, int TM, int NW, bool EXACT = false>
 __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     static_assert(!EXACT || FMT == FMT_Q8_0 || FMT == FMT_Q4_0, "formats of one scale per block");
-    constexpr int KW = kWaves / NW, MT = 32 * TM, GT = 64 * NW, BUFS = block_buffers<TM, NW>();
+    constexpr int KW = kWaves / NW, MT = 32 * TM, GT = 64 * NW, BUFS = block_buffers<FMT, TM, NW>();
     constexpr int XP = MT * (kStep / 8) / GT;       // sixteen-byte pieces of the activations per thread and step
     static_assert(MT * (kStep / 8) % GT == 0 && XP >= 1, "whole pieces");
     extern __shared__ uint4 smem[];
@@ -94,21 +102,43 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
             *reinterpret_cast<uint4 *>(xt + buf * MT * kRow + r * kRow + part * 8) = FMT == FMT_Q4_0 ? swap_middle(xv[i]) : xv[i];
         }
     };
-    // Weights (exchange_rows): each lane ends up with pieces 2 h and 2 h + 1 of row lane % 32
-    const int piece = EXACT ? 2 * ((lane >> 4) & 1) + h : lane >> 4;   // exact: pieces h and 2 + h
+    // Weights.  Turned: four neighbouring lanes load 64 bytes of a row, and a stretch of LDS of the wavefront's own brings each lane two pieces of row lane % 32.  Otherwise lanes sixteen apart, for
+    // exchange_rows.  Pieces 2 h and 2 h + 1; exact: h and 2 + h.
+    constexpr bool TURN = turned(FMT, TM, NW);
+    const int piece = TURN ? lane & 3 : EXACT ? 2 * ((lane >> 4) & 1) + h : lane >> 4, wrow = TURN ? lane >> 2 : lane & 15;
     const uint8_t *wbase = a.qs + (size_t)row0 * a.row_bytes;
-    const u32 wlo = (u32)row_of(lane & 15) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + (lane & 15)) * (u32)a.row_bytes + piece * 16;
+    const u32 wlo = (u32)row_of(wrow) * (u32)a.row_bytes + piece * 16, whi = (u32)row_of(16 + wrow) * (u32)a.row_bytes + piece * 16;
+    uint8_t *turn = reinterpret_cast<uint8_t *>(smem) + (size_t)BUFS * KW * MT * kRow * 2 + wave * 32 * kTurn, *turn_in = turn + wrow * kTurn + piece * 16;
+    const uint8_t *turn_out = turn + col * kTurn + (EXACT ? h : 2 * h) * 16;
     const uint16_t *sbase = a.scales + (size_t)row0 * (a.K / 32);
     const u32 so = (u32)row_of(col) * (u32)(a.K / 32) + (FMT == FMT_Q4_0 && !EXACT ? 2 * h : 0), ho = (u32)row_of(col) * (u32)a.row_bytes;
     constexpr int PAIRS = pairs_of(FMT);
-    uint4 raw[PAIRS][2], q[2];                  // the next step's stretches as they were loaded; the stretch in use, of the lane's own row
+    uintx4 raw[PAIRS][2], next_q[2];            // the next step's stretches as they were loaded; turned: the next stretch, of the lane's own row
+    uint4 q[2];                                 // the stretch in use
     auto load_pair = [&](int s, int j) __attribute__((always_inline)) {
         const uint8_t *from = wbase + (FMT == FMT_Q4_K ? (size_t)(at(s) >> 1) * 144 + 16 + (at(s) & 1) * 64 : (size_t)at(s) * (64 * PAIRS)) + 64 * j;
-        raw[j][0] = *reinterpret_cast<const uint4 *>(from + wlo);
-        raw[j][1] = *reinterpret_cast<const uint4 *>(from + whi);
+        raw[j][0] = *reinterpret_cast<const uintx4 *>(from + wlo);
+        raw[j][1] = *reinterpret_cast<const uintx4 *>(from + whi);
+    };
+    // turned: stretch j of the step in raw becomes the next one, step `then` goes on its way
+    auto turn_pair = [&](auto j_c, int then) __attribute__((always_inline)) {
+        constexpr int j = decltype(j_c)::value;
+        *reinterpret_cast<uintx4 *>(turn_in) = raw[j][0];
+        *reinterpret_cast<uintx4 *>(turn_in + 16 * kTurn) = raw[j][1];
+        load_pair(then, j);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // a wavefront's LDS operations keep their order
+        __builtin_amdgcn_wave_barrier();
+        next_q[0] = *reinterpret_cast<const uintx4 *>(turn_out);
+        next_q[1] = *reinterpret_cast<const uintx4 *>(turn_out + (EXACT ? 32 : 16));
     };
     auto use_pair = [&](int j) __attribute__((always_inline)) {
-        exchange_rows(raw[j], q);
+        if constexpr (TURN) {
+            q[0] = __builtin_bit_cast(uint4, next_q[0]);
+            q[1] = __builtin_bit_cast(uint4, next_q[1]);
+            return;
+        }
+        const uint4 loaded[2] = {__builtin_bit_cast(uint4, raw[j][0]), __builtin_bit_cast(uint4, raw[j][1])};
+        exchange_rows(loaded, q);
         if constexpr (EXACT && FMT == FMT_Q4_0) {   // each half of a wavefront holds a block; it needs bytes 8 h .. of both
 #pragma unroll
             for (int p = 0; p < 2; p++) {
@@ -148,6 +178,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     store_x(0);
     load_x(1);
     scale[1] = load_scales(1);
+    if constexpr (TURN) turn_pair(std::integral_constant<int, 0>{}, 1);
     __syncthreads();
 
     // eight weights of the lane's row as fp16
@@ -226,8 +257,9 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
             for (int i = 0; i < TM; i++) xf[g & 1][i] = *reinterpret_cast<const half8 *>(xb + 32 * i * kRow + koff(g));
             if (g % (8 / PAIRS) == 0) {   // a stretch is taken into use, the next step's goes on its way
                 use_pair(g / (8 / PAIRS));
-                load_pair(s + 1, g / (8 / PAIRS));
+                if constexpr (!TURN) load_pair(s + 1, g / (8 / PAIRS));
             }
+            if constexpr (TURN) if (PAIRS == 2 && g == 3) turn_pair(std::integral_constant<int, PAIRS - 1>{}, s + 1);
             wf[g & 1] = decode(hdr[H], scale[S], odd, g);
         };
         fragments(0);
@@ -250,6 +282,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 #pragma unroll
             for (int g = 0; g < 8; g++) {
                 if (g + 1 < 8) fragments(g + 1);
+                else if constexpr (TURN) turn_pair(std::integral_constant<int, 0>{}, s + 2);
 #pragma unroll
                 for (int i = 0; i < TM; i++) part[(g >> 1) & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][i], wf[g & 1], g & 1 ? part[(g >> 1) & 1][i] : zero16, 0, 0, 0);
                 if (g >= 2 && !(g & 1)) fold((g >> 1) - 1);
@@ -259,6 +292,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 #pragma unroll
         for (int g = 0; g < 8; g++) {
             if (g + 1 < 8) fragments(g + 1);
+            else if constexpr (TURN) turn_pair(std::integral_constant<int, 0>{}, s + 2);
 #pragma unroll
             for (int i = 0; i < TM; i++) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[g & 1][i], wf[g & 1], acc[i], 0, 0, 0);
             if (g + 1 < 8) {
@@ -332,7 +366,7 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
 template <int FMT, int TM, int NW, bool EXACT>
 hipError_t launch(const BlockArgs &a, hipStream_t stream) {
     static std::atomic<uint64_t> raised{0};
-    constexpr size_t lds = block_lds_bytes<TM, NW>();
+    constexpr size_t lds = block_lds_bytes<FMT, TM, NW>();
     const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT>), lds, raised);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW, EXACT>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
