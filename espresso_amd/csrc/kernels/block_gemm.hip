@@ -431,6 +431,8 @@ void block_gemm_set_form(int form) {
     g_block_gemm_form.store(known ? form : 0);
 }
 
+bool block_gemm_by_size() { return g_block_gemm_form.load() == 0; }
+
 // Products of 2048 columns and more that steps with exact weights ask for, in shares of K that the next kernel adds: up to 32 rows, and what is small (beyond it weights are
 // rounded).  Against rows_gemm.hip, whose wavefronts walk more of K each, 2560 x 2048, 4 / 31 / 93 rows: Q8_0 8.0 / 9.5 / 9.9 -> 6.2 / 6.4 / 7.8 us, Q4_0 6.8 / 8.2 / 8.4 -> 5.3 / 5.5 /
 // 6.7;  2048 x 2048, 64 / 128 rows: Q8_0 9.6 / 9.9 -> 6.5 / 7.7, Q4_0 8.2 / 8.5 -> 5.8 / 6.8.  Of what the launch gains the next kernel takes 1.5 to 2.5 us for the planes, so whole

@@ -28,6 +28,7 @@
 #include "block_gemm.h"
 #include "wide_gemm.h"
 #include "rows_gemm.h"
+#include "stream_gemm.h"
 #include <atomic>
 #include <type_traits>
 
@@ -586,6 +587,12 @@ hipError_t launch_gemm(const GemmParams &params, hipStream_t stream) {
     // single products of up to eight rows of Q4_0 keep their weights, whoever asks, and so may take either kernel that does (8 rows, in rows_gemm.hip -> with shares of K and
     // their sum: 768 x 768 3.9 -> 6.9 us, 2048 x 2048 6.7 -> 8.6, 2048 x 5632 10.3 -> 9.6)
     if (w.format == FMT_Q4_0 && p.rows <= 8 && w.cols % 128 == 0) p.unrounded = true;
+    if (stream_gemm_takes(p)) {
+        int shares = 1;
+        const hipError_t e = launch_stream_gemm(p, &shares, stream);
+        if (p.deferred_splits) *p.deferred_splits = shares;
+        return e;
+    }
     if (rows_gemm_takes(p)) return launch_rows_gemm(p, stream);
     GemmArgs a{};
     a.qs = w.qs; a.scales = w.scales; a.qs_row_bytes = w.qs_row_bytes; a.N = w.rows; a.K = w.cols; a.M = p.rows;

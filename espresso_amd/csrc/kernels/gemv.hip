@@ -41,6 +41,7 @@
 #include "block_split.h"
 #include "wide_split.h"
 #include "rows_gemm.h"
+#include "stream_gemm.h"
 #include "span_attention.h"
 
 #include <hip/hip_ext.h>
@@ -2905,6 +2906,7 @@ bool gemv_set_tuning(const char *key, int value) {
     if (k == "block_gemm_form") { block_gemm_set_form(value); return true; }
     if (k == "batch_gemv_form") { batch_gemv_set_form(value); return true; }
     if (k == "rows_gemm") { rows_gemm_set_mode(value); return true; }
+    if (k == "stream_gemm") { stream_gemm_set_mode(value); return true; }
     if (k == "dense_gemm_form") { dense_gemm_set_form(value); return true; }
     if (k == "wide_gemm_form") { wide_gemm_set_form(value); return true; }
     if (k == "block_split_form") { block_split_set_form(value); return true; }

@@ -302,6 +302,7 @@ static int rows_gemm_mode() {
     return g_rows_gemm_mode;
 }
 void rows_gemm_set_mode(int mode) { g_rows_gemm_mode = mode < 0 ? 1 : mode; }
+bool rows_gemm_by_size() { return rows_gemm_mode() == 1; }
 
 bool rows_gemm_takes(const GemmParams &p) {
     const DeviceMatrix &w = p.w;
