@@ -15,7 +15,7 @@ bool block_gemm_exact(const GemmParams &p);   // of a product that runs here
 bool block_gemm_exact(const DeviceMatrix &w, int rows);
 // Complete in p.y (+ residual) or p.swiglu_out where *splits is 1; otherwise *splits planes of sums in p.workspace, residual and SiLU left to whoever adds them.
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream);
-void block_gemm_set_form(int form);   // 0 by size (default), otherwise always: row tiles * 100 + wavefronts along the weights * 10 + shares of K
+void block_gemm_set_form(int form);   // 0 by size (default), otherwise always: row tiles * 100 + wavefronts along the weights * 10 + shares of K (+ long tiles * 1000, 64 rows each behind them)
 bool block_gemm_by_size();
 
 }  // namespace esp

@@ -42,6 +42,7 @@ struct BlockArgs {
     float *partial;
     uint16_t *swiglu_out;
     int per, splits, n_tiles, m_tiles;   // per: steps of one group of wavefronts
+    int long_tiles;                      // mixed heights: the first of the m_tiles have the kernel's height, the others the shorter one
 };
 
 __device__ __forceinline__ h2 splat_bits(u32 bits16) { return as_h2(__builtin_amdgcn_perm(bits16, bits16, 0x01000100u)); }
@@ -64,17 +65,15 @@ constexpr size_t block_lds_bytes() {
 }
 
 // EXACT (Q8_0, Q4_0; one row tile): integers go to the matrix cores, a block's scale to its sums.  Every product then contracts one block, each half of a wavefront holding half of it.
-template <int FMT, int TM, int NW, bool EXACT = false>
-__global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
+template <int FMT, int TM, int NW, bool EXACT>
+__device__ __forceinline__ void block_product(const BlockArgs &a, const int m0, const int n_tile, const int split, uint4 *smem) {
     static_assert(!EXACT || FMT == FMT_Q8_0 || FMT == FMT_Q4_0, "formats of one scale per block");
     constexpr int KW = kWaves / NW, MT = 32 * TM, GT = 64 * NW, BUFS = block_buffers<FMT, TM, NW>();
     constexpr int XP = MT * (kStep / 8) / GT;       // sixteen-byte pieces of the activations per thread and step
     static_assert(MT * (kStep / 8) % GT == 0 && XP >= 1, "whole pieces");
-    extern __shared__ uint4 smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, col = lane & 31;
     const int wn = wave % NW, wk = wave / NW, gtid = wn * 64 + lane;
-    const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
-    const int m0 = m_tile * MT, n0 = (n_tile * NW + wn) * 32, n = n0 + col;
+    const int n0 = (n_tile * NW + wn) * 32, n = n0 + col;
     const int row0 = n0 < a.N ? n0 : a.N - 1;
     auto row_of = [&](int r) { return row0 + r < a.N ? r : a.N - 1 - row0; };   // rows from row0 on, clamped: those beyond are never stored
     // every group of wavefronts passes the same barriers and has steps of its own
@@ -363,13 +362,32 @@ __global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
     }
 }
 
-template <int FMT, int TM, int NW, bool EXACT>
+// TS < TM: two heights of tiles in one launch, the long ones first (no shares of K).
+template <int FMT, int TM, int NW, bool EXACT = false, int TS = TM>
+__global__ __launch_bounds__(kThreads) void block_gemm_kernel(BlockArgs a) {
+    extern __shared__ uint4 smem[];
+    if constexpr (TS == TM) {
+        const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
+        block_product<FMT, TM, NW, EXACT>(a, m_tile * 32 * TM, n_tile, split, smem);
+    } else {
+        const int longs = a.long_tiles * a.n_tiles;
+        if ((int)blockIdx.x < longs) {
+            const auto [m_tile, n_tile, split] = place_of(a.long_tiles, a.n_tiles, blockIdx.x, longs);
+            block_product<FMT, TM, NW, EXACT>(a, m_tile * 32 * TM, n_tile, 0, smem);
+        } else {
+            const auto [m_tile, n_tile, split] = place_of(a.m_tiles - a.long_tiles, a.n_tiles, blockIdx.x - longs, gridDim.x - longs);
+            block_product<FMT, TS, NW, EXACT>(a, a.long_tiles * 32 * TM + m_tile * 32 * TS, n_tile, 0, smem);
+        }
+    }
+}
+
+template <int FMT, int TM, int NW, bool EXACT, int TS = TM>
 hipError_t launch(const BlockArgs &a, hipStream_t stream) {
     static std::atomic<uint64_t> raised{0};
-    constexpr size_t lds = block_lds_bytes<FMT, TM, NW>();
-    const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT>), lds, raised);
+    constexpr size_t one = block_lds_bytes<FMT, TM, NW>(), other = block_lds_bytes<FMT, TS, NW>(), lds = one > other ? one : other;
+    const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(block_gemm_kernel<FMT, TM, NW, EXACT, TS>), lds, raised);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW, EXACT>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL((block_gemm_kernel<FMT, TM, NW, EXACT, TS>), dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), lds, stream, a);
     return hipGetLastError();
 }
 
@@ -382,6 +400,7 @@ hipError_t launch_width(int nw, const BlockArgs &a, hipStream_t stream) {
 }
 template <int FMT>
 hipError_t launch_format(int tm, int nw, bool exact, const BlockArgs &a, hipStream_t stream) {
+    if (a.long_tiles) return tm == 4 ? launch<FMT, 4, 8, false, 2>(a, stream) : launch<FMT, 3, 8, false, 2>(a, stream);
     if constexpr (FMT == FMT_Q8_0 || FMT == FMT_Q4_0) if (exact) return launch_width<FMT, 1, true>(nw, a, stream);
     switch (tm) {
     case 1: return launch_width<FMT, 1>(nw, a, stream);
@@ -391,7 +410,7 @@ hipError_t launch_format(int tm, int nw, bool exact, const BlockArgs &a, hipStre
     }
 }
 
-struct Form { int tm = 0, nw = 0, per = 0, splits = 0; };
+struct Form { int tm = 0, nw = 0, per = 0, splits = 0, long_tiles = 0; };   // long_tiles: tiles of tm * 32 rows, tiles of 64 behind them
 std::atomic<int> g_block_gemm_form{0};
 
 // The form (rows of a tile, wavefronts along the weights, shares of K) by its expected time: rounds of one workgroup per compute unit, a step of a round growing with the tile's rows and
@@ -407,6 +426,7 @@ Form choose_form(const GemmParams &p, bool exact) {
     const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
     Form best;
     float best_us = 0.0f;
+    auto group = [&](int per, int tm, int kw) { return per * unit * (step + tm * (row_tile + staged * kw)) + fill + (kw > 1 ? join * tm : 0.0f); };   // one workgroup
     for (int tm = 1; tm <= (exact ? 1 : 4) && tm <= (M + 31) / 32; tm++)
         for (int nw = tm < 4 ? 2 : 4; nw <= 8; nw *= 2)
             for (int want : kSplits) {
@@ -416,18 +436,37 @@ Form choose_form(const GemmParams &p, bool exact) {
                 if (splits != want || (splits > 1 && (!p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
                 const long wgs = (long)((N + 32 * nw - 1) / (32 * nw)) * ((M + 32 * tm - 1) / (32 * tm)) * splits;
                 const float rounds = (float)((wgs + cus - 1) / cus);
-                float us = start + rounds * (per * unit * (step + tm * (row_tile + staged * kw)) + fill + (kw > 1 ? join * tm : 0.0f)) + plane_us * mb;
+                float us = start + rounds * group(per, tm, kw) + plane_us * mb;
                 if (splits > 1) us += again_us * mb + (p.swiglu_out ? 3.0f : p.deferred_splits ? 1.0f : 1.6f + 0.2f * splits);
                 if (!best.tm || us < best_us) { best = Form{tm, nw, per * unit, splits}; best_us = us; }
             }
+    // Several rounds of tiles whose last one is nearly empty: tiles of 64 rows at the end, which each compute unit takes as it comes free.  us, one height -> two: 16384 x 3072 Q4_K, 600 / 1200 / 1600 /
+    // 1777 rows 100.0 / 174.2 / 224.9 / 233.7 -> 92.2 / 162.1 / 213.2 / 225.4;  28672 x 4096 Q4_0, 300 / 600 / 1200 rows 116.7 / 196.7 / 339.7 -> 104.8 / 184.2 / 327.3;  6144 x 4096 Q4_0, 1400 / 1600 rows
+    // 105.5 / 117.8 -> 103.8 / 107.0.  Less than two per cent in the rule's own time is not taken.
+    for (int tm = 3; tm <= 4 && !exact && best.splits == 1; tm++) {
+        const int n_tiles = (N + 255) / 256;
+        const float along = group(units, tm, 1), ashort = group(units, 2, 1);
+        for (int longs = 1; 32 * tm * longs < M; longs++) {
+            int shorts = n_tiles * ((M - 32 * tm * longs + 63) / 64);
+            const int full = n_tiles * longs / cus, ahead = n_tiles * longs % cus;
+            float early = full * along, late = (full + (ahead ? 1 : 0)) * along;
+            for (; shorts > 0;) {
+                const bool at_early = early <= late || !ahead;
+                shorts -= at_early ? cus - ahead : ahead;
+                (at_early ? early : late) += ashort;
+            }
+            const float us = start + (early > late ? early : late) + plane_us * (float)M * (float)N * 4e-6f;
+            if (us < 0.98f * best_us) { best = Form{tm, 8, units * unit, 1, longs}; best_us = us; }
+        }
+    }
     return best;
 }
 
 }  // namespace
 
 void block_gemm_set_form(int form) {
-    const int tm = form / 100, nw = form / 10 % 10, shares = form % 10;
-    const bool known = tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
+    const int longs = form / 1000, tm = form / 100 % 10, nw = form / 10 % 10, shares = form % 10;
+    const bool known = (longs == 0 || (tm >= 3 && nw == 8 && shares == 1)) && tm >= 1 && tm <= 4 && (nw == 4 || nw == 8 || (nw == 2 && tm < 4)) && shares >= 1;
     g_block_gemm_form.store(known ? form : 0);
 }
 
@@ -471,8 +510,9 @@ bool block_gemm_takes(const GemmParams &p) {
 hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t stream) {
     bool exact = block_gemm_exact(p);
     Form f = choose_form(p, exact);
-    if (const int forced = g_block_gemm_form.load(); forced > 0) {   // tm * 100 + nw * 10 + shares of K
-        f.tm = forced / 100; f.nw = forced / 10 % 10;
+    if (const int forced = g_block_gemm_form.load(); forced > 0) {   // long tiles * 1000 + tm * 100 + nw * 10 + shares of K
+        f.tm = forced / 100 % 10; f.nw = forced / 10 % 10;
+        f.long_tiles = forced / 1000 * 32 * f.tm < p.rows ? forced / 1000 : 0;
         exact = exact && f.tm == 1;   // forms of more row tiles have no exact kernel
         const int unit = p.w.format == FMT_Q4_K ? 2 : 1;
         const Shares shares = shares_of(p.w.cols / (kStep * unit), f.nw, forced % 10);
@@ -480,7 +520,7 @@ hipError_t launch_block_gemm(const GemmParams &p, int *splits, hipStream_t strea
         if (f.splits > 1 && (!p.workspace || (size_t)f.splits * p.rows * p.w.rows > p.workspace_floats)) return hipErrorInvalidValue;
     }
     BlockArgs a{p.w.qs, p.w.scales, p.w.qs_row_bytes, p.w.rows, p.w.cols, p.rows, p.x, p.y, p.residual, p.workspace, f.splits == 1 && p.w.rows % 2 == 0 ? p.swiglu_out : nullptr, f.per, f.splits,
-                (p.w.rows + 32 * f.nw - 1) / (32 * f.nw), (p.rows + 32 * f.tm - 1) / (32 * f.tm)};
+                (p.w.rows + 32 * f.nw - 1) / (32 * f.nw), f.long_tiles ? f.long_tiles + (p.rows - 32 * f.tm * f.long_tiles + 63) / 64 : (p.rows + 32 * f.tm - 1) / (32 * f.tm), f.long_tiles};
     *splits = f.splits;
     switch (p.w.format) {
     case FMT_Q4_K: return launch_format<FMT_Q4_K>(f.tm, f.nw, false, a, stream);

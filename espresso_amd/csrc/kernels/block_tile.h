@@ -25,12 +25,13 @@ __device__ __forceinline__ float half_bits_to_float(u32 bits16) { return (float)
 // The workgroup's place among tiles of activation rows, tiles of weight rows and shares of K: workgroups of one die take neighbouring output tiles, the row tiles of one block of
 // weights first.
 struct Place { int m_tile, n_tile, split; };
-__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) {
-    const int total = gridDim.x, die = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-    const int unit = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
+__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles, int block, int total) {
+    const int die = block & 7, q8 = total >> 3, r8 = total & 7;
+    const int unit = die * q8 + (die < r8 ? die : r8) + (block >> 3);
     const int m_tile = unit % m_tiles, rest = unit / m_tiles, n_tile = rest % n_tiles, split = rest / n_tiles;
     return {m_tile, n_tile, split};
 }
+__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) { return place_of(m_tiles, n_tiles, blockIdx.x, gridDim.x); }
 
 // Lane 16 p + r loaded piece p of row r (raw[0]) and of row 16 + r (raw[1]), so that four lanes cover 64 bytes of a row; afterwards each lane holds two pieces of row lane % 32.
 __device__ __forceinline__ void exchange_rows(const uint4 (&raw)[2], uint4 (&q)[2]) {

@@ -40,7 +40,7 @@ int esp_gemv_stamps(const ESPMatrix *matrix, int batch, int launches, uint64_t *
  * "q4k_long_row_waves" (ESPRESSO_HIP_Q4K_LONG_ROW_WAVES): one activation row at 14336 columns: 0 (default) = the matrix-core
  * kernel, 8 or 4 = the dot-product kernel with that many wavefronts per workgroup (one or three workgroups per compute unit).
  * "block_gemm_form": blocks of rows with packed weights, rows of a tile / 32 * 100 + wavefronts along the weights * 10 + shares of K
- * (141, 282, ...), 0 (default) = by size.  "wide_gemm_form": products with fp16 matrices, rows of a tile * 10000 + weight rows * 10 + shares of K (641284, 2562561, ...), 0 (default) = by size, as is a form whose planes have no room.
+ * (141, 282, ...) (+ long tiles * 1000: tiles of 64 rows behind so many), 0 (default) = by size.  "wide_gemm_form": products with fp16 matrices, rows of a tile * 10000 + weight rows * 10 + shares of K (641284, 2562561, ...), 0 (default) = by size, as is a form whose planes have no room.
  * "dense_gemm_form": bf16 products of the layered models, the same numbers; shares of K stay by size.
  * "block_split_form": the same for exact Q4_K products of split rows, -1 = never this kernel.  "batch_gemv_form": steps of three to sixteen rows with Q4_K matrices, row blocks of a workgroup * 10 + shares of K, 0 (default) = by size.  "wide_split_shares": exact Q4_K products of split rows in whole tiles, shares of K (1, 2, 3, 4, 6, 8), 0 (default) = by size, -1 = never.
  * "rows_gemm" / "stream_gemm": small products with exact weights by those kernels, 0 = never, 1 (default) = by size, 2 = wherever they can.

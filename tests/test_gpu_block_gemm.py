@@ -254,3 +254,24 @@ def test_single_products_pay_for_no_launch_that_adds_shares(ops, fmt, rows, cols
         bound = bound + 4 * 2.0 ** -11 * np.abs(x).max(1).astype(np.float64)[:, None] * np.abs(w).max()
     assert (np.abs(default - x.astype(np.float64) @ w.T) <= bound).all()
     m.close()
+
+
+@pytest.mark.parametrize("fmt,rows,cols", [("q8_0", 300, 640), ("q4_0", 256, 1152), ("q4_k", 290, 1280)])
+@pytest.mark.parametrize("heights", [1481, 2481, 1381, 3381])
+def test_two_heights_of_tiles_are_the_same_product(ops, fmt, rows, cols, heights):
+    """Tiles of 64 rows behind long ones, at the edges of both: every sum in the order that tiles of one height have."""
+    f = lib.FORMAT_NAMES[fmt]
+    m = ops.Matrix(f, ops.synth_weights(f, rows + cols, 0.02, rows * cols), rows, cols)
+    rng = np.random.default_rng(cols)
+    first = heights // 1000 * 32 * (heights // 100 % 10)
+    try:
+        for batch in (first, first + 1, first + 64, first + 65, first + 190):
+            x = rng.normal(0, 1, (batch, cols)).astype(np.float16)
+            residual = rng.normal(0, 1, (batch, rows)).astype(np.float32)
+            ops.set_tuning("block_gemm_form", heights % 1000)
+            want = m.gemv(x, residual), m.layer_gate_up(x)
+            ops.set_tuning("block_gemm_form", heights)
+            assert np.array_equal(want[0], m.gemv(x, residual)) and np.array_equal(want[1], m.layer_gate_up(x)), batch
+    finally:
+        ops.set_tuning("block_gemm_form", 0)
+    m.close()
