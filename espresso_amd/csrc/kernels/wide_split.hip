@@ -9,7 +9,7 @@
 // Against the kernels these products had (gemm_q4k_split_regb_kernel behind a SiLU, block_split.hip otherwise), us with their planes added:
 //   28672 x 4096 behind a SiLU, 256 / 512 / 960 / 2048 rows 157 / 318 / 611 / 1099 -> 124 / 276 / 556 / 1029;  16384 x 2048, 512 / 2048 rows 82 / 368 -> 71 / 327;
 //   4096 x 14336, 512 / 960 / 2048 rows 140 / 282 / 636 -> 122 / 232 / 472;  4096 x 4096, 2048 rows 171 -> 134;  6144 x 4096, 512 rows 70 -> 68.
-// Kept out: tiles of 64 x 128, 64 x 256 and 128 x 128 (0.7 to 1.0 times as fast as what those sizes have).
+// Kept out: tiles of 64 x 128 and 128 x 128, and 64 x 256 alone (0.7 to 1.0 times as fast as what those sizes have).
 #include "../common.h"
 #include "silu.h"
 #include "split_rows.h"
@@ -37,6 +37,7 @@ struct WideSplitArgs {
     float *partial;
     uint16_t *sw_hi, *sw_lo, *sw_sums;
     int per, splits, n_tiles, m_tiles;   // per: super-blocks of a share
+    int long_tiles;                      // two heights: the first of the m_tiles have 128 rows, the others 64
 };
 
 __device__ __forceinline__ h2 as_h2(u32 v) { return __builtin_bit_cast(h2, v); }
@@ -92,16 +93,17 @@ struct Packed {
     }
 };
 
-constexpr int kWM = 2, kWN = 4, TM = 2, TN = 2, BM = 32 * kWM * TM, BN = 32 * kWN * TN;   // wavefronts, products of each, rows and weight rows of a tile
-constexpr int kBuffer = (2 * BM + BN) * kPitch, kLd = BN / 2 + 8;                           // kLd: units between the rows of the epilogue's planes
-constexpr size_t kLdsBytes = (size_t)2 * kBuffer * 2;
-static_assert(kLdsBytes <= 160 * 1024 && (size_t)2 * BM * kLd * 2 <= kLdsBytes, "LDS of a compute unit");
+constexpr int kWM = 2, kWN = 4, TN = 2, BN = 32 * kWN * TN, kLd = BN / 2 + 8;   // wavefronts, products of each, weight rows of a tile; units between the rows of the epilogue's planes
+constexpr int rows_of(int tm) { return 32 * kWM * tm; }
+constexpr int buffer_of(int tm) { return (2 * rows_of(tm) + BN) * kPitch; }
+constexpr int kLong = rows_of(2), kShort = rows_of(1);
+constexpr size_t kLdsBytes = (size_t)2 * buffer_of(2) * 2;
+static_assert(kLdsBytes <= 160 * 1024 && (size_t)2 * kLong * kLd * 2 <= kLdsBytes, "LDS of a compute unit");
 
-__global__ __launch_bounds__(kThreads) void wide_split_kernel(WideSplitArgs a) {
-    extern __shared__ uint4 smem[];
-    uint16_t *lds = reinterpret_cast<uint16_t *>(smem);
-    const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles);
-    const int m0 = m_tile * BM, n0 = n_tile * BN, sbs = a.K / 256, first = split * a.per, blocks = sbs - first < a.per ? sbs - first : a.per, steps = 4 * blocks;
+template <int TM>
+__device__ __forceinline__ void wide_split_tile(const WideSplitArgs &a, const int m0, const int n_tile, const int split, uint16_t *lds) {
+    constexpr int BM = rows_of(TM), kBuffer = buffer_of(TM);
+    const int n0 = n_tile * BN, sbs = a.K / 256, first = split * a.per, blocks = sbs - first < a.per ? sbs - first : a.per, steps = 4 * blocks;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave / kWN, wn = wave % kWN, h = lane >> 5, col = lane & 31;
     Plain<BM, 1> hi(a.xh, (size_t)a.K, m0, a.M, (size_t)first * 256, steps), lo(a.xl, (size_t)a.K, m0, a.M, (size_t)first * 256, steps);
     Packed<BN> w(a.qs, a.row_bytes, n0, a.N, first, steps);
@@ -314,6 +316,26 @@ __global__ __launch_bounds__(kThreads) void wide_split_kernel(WideSplitArgs a) {
         }
 }
 
+// TWO: two heights of tiles in one launch, the long ones first (no shares of K).
+template <bool TWO>
+__global__ __launch_bounds__(kThreads) void wide_split_kernel(WideSplitArgs a) {
+    extern __shared__ uint4 smem[];
+    uint16_t *lds = reinterpret_cast<uint16_t *>(smem);
+    if constexpr (!TWO) {
+        const auto [m_tile, n_tile, split] = place_of(a.m_tiles, a.n_tiles, blockIdx.x, gridDim.x);
+        wide_split_tile<2>(a, m_tile * kLong, n_tile, split, lds);
+    } else {
+        const int longs = a.long_tiles * a.n_tiles;
+        if ((int)blockIdx.x < longs) {
+            const auto [m_tile, n_tile, split] = place_of(a.long_tiles, a.n_tiles, blockIdx.x, longs);
+            wide_split_tile<2>(a, m_tile * kLong, n_tile, 0, lds);
+        } else {
+            const auto [m_tile, n_tile, split] = place_of(a.m_tiles - a.long_tiles, a.n_tiles, blockIdx.x - longs, gridDim.x - longs);
+            wide_split_tile<1>(a, a.long_tiles * kLong + m_tile * kShort, n_tile, 0, lds);
+        }
+    }
+}
+
 std::atomic<int> g_wide_split_shares{0};
 
 }  // namespace
@@ -330,26 +352,50 @@ WideSplitForm wide_split_form(const GemmSplitParams &p) {
     if (forced < 0 || (forced == 0 && M <= 64) || (swiglu && ((N / 2) % 32 != 0 || !p.swiglu.sums))) return best;
     const int kShares[] = {1, 2, 3, 4, 6, 8};
     for (int want : kShares) {
-        if (forced > 0 && want != (swiglu ? 1 : forced)) continue;
+        if (forced > 0 && want != (swiglu || forced >= 100 ? 1 : forced)) continue;
         const int per = (blocks + want - 1) / want, splits = (blocks + per - 1) / per;
         if ((splits != want && forced == 0) || (splits > 1 && (swiglu || !p.workspace || (size_t)splits * M * N > p.workspace_floats))) continue;
-        const long wgs = (long)((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits, rounds = (wgs + cus - 1) / cus;
+        const long wgs = (long)((N + BN - 1) / BN) * ((M + kLong - 1) / kLong) * splits, rounds = (wgs + cus - 1) / cus;
         float us = 1.3f + (float)per * (4.46f * (float)rounds + 2.93f * (float)wgs / (float)cus) + 5.5f * (float)rounds + 0.22f * (float)splits * (float)M * (float)N * (swiglu ? 2e-6f : 4e-6f);
         if (splits > 1) us += 1.75f + 0.35f * (float)splits;
         if (!best.per || us < best.us) best = WideSplitForm{per, splits, us};
     }
+    // Where the last round of tiles would be nearly empty, or the last tile: tiles of 64 rows at the end, which each compute unit takes as it comes free (0.65 of a tile's time, half of its power).  What the
+    // rule takes was the best of 159 launches' forms every time, 1.00 to 1.18 times as fast as tiles of one height; behind a SiLU, us: 28672 x 4096, 300 / 600 / 800 / 1777 rows 230 / 360 / 488 / 900 ->
+    // 194 / 334 / 421 / 871;  11264 x 2048, 800 / 1000 rows 121 / 125 -> 104 / 111;  16384 x 2048, 400 / 600 / 1777 rows 72 / 122 / 271 -> 68 / 107 / 258.  512 rows: tiles of one height, like 1000 and 1400 of
+    // the widest.
+    if (forced == 0 && best.per) {
+        const int n_tiles = (N + BN - 1) / BN;
+        float least = 0.98f * best.us;
+        for (int longs = 1; longs * kLong < M; longs++) {
+            const int shorts = n_tiles * ((M - longs * kLong + kShort - 1) / kShort), full = n_tiles * longs / cus, ahead = n_tiles * longs % cus;
+            float early = (float)full, late = (float)(full + (ahead ? 1 : 0));
+            for (int left = shorts; left > 0;) {
+                const bool at_early = early <= late || !ahead;
+                left -= at_early ? cus - ahead : ahead;
+                (at_early ? early : late) += 0.65f;
+            }
+            const float rounds = early > late ? early : late;
+            const float us = 1.3f + (float)blocks * (4.46f * rounds + 2.93f * ((float)(n_tiles * longs) + 0.5f * (float)shorts) / (float)cus) + 5.5f * rounds + 0.22f * (float)M * (float)N * (swiglu ? 2e-6f : 4e-6f);
+            if (us < least) { least = us; best = WideSplitForm{blocks, 1, us, longs}; }
+        }
+    }
     if (forced > 0) best.us = 0.0f;
+    if (forced >= 100 && forced / 100 * kLong < M) best.long_tiles = forced / 100;
     return best;
 }
 
 hipError_t launch_wide_split(const GemmSplitParams &p, const WideSplitForm &f, hipStream_t stream) {
     const WideSplitArgs a{p.w.qs, p.w.qs_row_bytes, p.w.rows, p.w.cols, p.rows, p.x.hi, p.x.lo, p.x.sums, p.y, p.residual, p.workspace, p.swiglu.hi, p.swiglu.lo, p.swiglu.sums,
-                          f.per, f.splits, (p.w.rows + BN - 1) / BN, (p.rows + BM - 1) / BM};
-    static std::atomic<uint64_t> raised{0};
-    const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(wide_split_kernel), kLdsBytes, raised);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(wide_split_kernel, dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), kLdsBytes, stream, a);
-    return hipGetLastError();
+                          f.per, f.splits, (p.w.rows + BN - 1) / BN, f.long_tiles ? f.long_tiles + (p.rows - f.long_tiles * kLong + kShort - 1) / kShort : (p.rows + kLong - 1) / kLong, f.long_tiles};
+    auto go = [&](auto kernel, std::atomic<uint64_t> &raised) {
+        const hipError_t err = raise_lds_limit(reinterpret_cast<const void *>(kernel), kLdsBytes, raised);
+        if (err != hipSuccess) return err;
+        hipLaunchKernelGGL(kernel, dim3(a.n_tiles * a.m_tiles * a.splits), dim3(kThreads), kLdsBytes, stream, a);
+        return hipGetLastError();
+    };
+    static std::atomic<uint64_t> raised_one{0}, raised_two{0};
+    return f.long_tiles ? go(wide_split_kernel<true>, raised_two) : go(wide_split_kernel<false>, raised_one);
 }
 
 }  // namespace esp

@@ -38,12 +38,13 @@ struct Tile {
 
 // The workgroup's place: workgroups of one die take neighbouring output tiles, the row tiles of one block of weights first.
 struct Place { int m_tile, n_tile, split; };
-__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) {
-    const int total = gridDim.x, die = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
-    const int unit = die * q8 + (die < r8 ? die : r8) + (blockIdx.x >> 3);
+__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles, int block, int total) {
+    const int die = block & 7, q8 = total >> 3, r8 = total & 7;
+    const int unit = die * q8 + (die < r8 ? die : r8) + (block >> 3);
     const int rest = unit / m_tiles;
     return {unit % m_tiles, rest % n_tiles, rest / n_tiles};
 }
+__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) { return place_of(m_tiles, n_tiles, blockIdx.x, gridDim.x); }
 
 // The limit of dynamic LDS, raised once per kernel and device (`raised`: the kernel's own).
 inline hipError_t raise_lds_limit(const void *kernel, size_t lds, std::atomic<uint64_t> &raised) {

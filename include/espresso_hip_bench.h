@@ -42,7 +42,7 @@ int esp_gemv_stamps(const ESPMatrix *matrix, int batch, int launches, uint64_t *
  * "block_gemm_form": blocks of rows with packed weights, rows of a tile / 32 * 100 + wavefronts along the weights * 10 + shares of K
  * (141, 282, ...) (+ long tiles * 1000: tiles of 64 rows behind so many), 0 (default) = by size.  "wide_gemm_form": products with fp16 matrices, rows of a tile * 10000 + weight rows * 10 + shares of K (641284, 2562561, ...), 0 (default) = by size, as is a form whose planes have no room.
  * "dense_gemm_form": bf16 products of the layered models, the same numbers; shares of K stay by size.
- * "block_split_form": the same for exact Q4_K products of split rows, -1 = never this kernel.  "batch_gemv_form": steps of three to sixteen rows with Q4_K matrices, row blocks of a workgroup * 10 + shares of K, 0 (default) = by size.  "wide_split_shares": exact Q4_K products of split rows in whole tiles, shares of K (1, 2, 3, 4, 6, 8), 0 (default) = by size, -1 = never.
+ * "block_split_form": the same for exact Q4_K products of split rows, -1 = never this kernel.  "batch_gemv_form": steps of three to sixteen rows with Q4_K matrices, row blocks of a workgroup * 10 + shares of K, 0 (default) = by size.  "wide_split_shares": exact Q4_K products of split rows in whole tiles, shares of K (1, 2, 3, 4, 6, 8), 100 * tiles of 128 rows with tiles of 64 behind them, 0 (default) = by size, -1 = never.
  * "rows_gemm" / "stream_gemm": small products with exact weights by those kernels, 0 = never, 1 (default) = by size, 2 = wherever they can.
  * "short_blocks": 0 = prompts of fewer than 32 tokens walk the steps, 1 (default) = a block where it is as exact and faster.
  * Runtimes that captured a step graph keep the kernels they captured. */

@@ -88,3 +88,23 @@ def test_blocks_by_rule_are_the_blocks_without(ops):
     # fp16 caches, whose last bit may fall either way
     for got in logits.values():
         assert np.abs(got - logits[-1]).max() <= 2.0 ** -9 * max(1.0, np.abs(logits[-1]).max())
+
+
+@pytest.mark.parametrize("rows,cols", [(288, 1280), (512, 512)])
+def test_two_heights_of_tiles_are_the_same_product(ops, rows, cols):
+    """Tiles of 64 rows behind tiles of 128, at the edges of both: every sum in the order that tiles of one height have."""
+    m, _ = matrix(ops, rows, cols)
+    rng = np.random.default_rng(cols)
+    try:
+        for tiles in (1, 2):
+            for batch in (128 * tiles + 1, 128 * tiles + 64, 128 * tiles + 65, 128 * tiles + 190):
+                x = rng.normal(0, 1, (batch, cols)).astype(np.float32)
+                residual = rng.normal(0, 1, (batch, rows)).astype(np.float32)
+                ops.set_tuning("wide_split_shares", 1)
+                want = m.matmul_f32(x, residual), m.matmul_f32_swiglu(x) if rows % 64 == 0 else None
+                ops.set_tuning("wide_split_shares", 100 * tiles)
+                assert np.array_equal(want[0], m.matmul_f32(x, residual)), (tiles, batch)
+                assert want[1] is None or np.array_equal(want[1], m.matmul_f32_swiglu(x)), (tiles, batch)
+    finally:
+        ops.set_tuning("wide_split_shares", 0)
+    m.close()
