@@ -24,6 +24,7 @@
 #include "../common.h"
 #include "attention_rows.h"
 #include "span_attention.h"
+#include "span_rows.h"
 #include <atomic>
 #include <type_traits>
 
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     uintx4 kr[KV_F16 ? KS : 1], vr[KV_F16 ? VP : 1];
     const uint32_t row_bytes = (uint32_t)kd * 2, k_row = (uint32_t)col * row_bytes, v_row = (uint32_t)(lane / VL) * row_bytes;
     auto first_row = [&](const void *cache, int t0) { return reinterpret_cast<const uint8_t *>(cache) + (base + (size_t)(t0 < t_max ? t0 : t_max) * kd) * 2; };
-    auto last_offset = [&](int t0) { return (uint32_t)(t0 < t_max ? t_max - t0 : 0) * row_bytes; };   // t_max's, from the tile's first row on (far tiles: beyond every lane's own)
+    auto last_offset = [&](int t0) { return last_row_offset(t_max - t0, row_bytes); };
     auto load_keys = [&](int t0) __attribute__((always_inline)) {
         const uint8_t *from = first_row(a.k_cache, t0);
         const uint32_t most = last_offset(t0), at = (k_row < most ? k_row : most) + 16 * half;
