@@ -12,8 +12,12 @@
 //     products: 8192 cycles per tile of 128 dims.
 //   * fp16 caches hold keys and values exactly, so only the fp32 operands are split, each into three fp16 parts that add up to its 24 bits: a query scaled
 //     by a power of two that takes its largest value to 2^14..2^15, a softmax weight times 2^15 (parts end at 2^-24, so what they leave is below
-//     2^-38 of the largest).  Three v_mfma_f32_32x32x16_f16 into one fp32 sum take 96 cycles where the fp32 form takes 512.  Values go through LDS as rows, whose transposed reads
+//     2^-38 of the largest).  Three v_mfma_f32_32x32x16_f16 take 96 cycles where the fp32 form takes 512.  Values go through LDS as rows, whose transposed reads
 //     (ds_read_b64_tr_b16) are the A operand.
+//     Every product rounds its sum, so the smaller parts of a score and of a tile's context are added up before the first ones, and a tile's context goes into the row's in one addition.  Root mean square
+//     error against 64 bits relative to the context, scores of 1 / 4 / 16 / 60, parts in turn into one sum for all tiles -> this: 300 rows of 8 heads (2 key/value heads) of 128 behind 200
+//     2.4 / 5.3 / 9.1 / 17.2e-7 -> 1.8 / 3.9 / 6.5 / 12.4e-7, 93 rows of 12 heads (4) of 64 behind 1500 2.3 / 4.9 / 8.3 / 16.5e-7 -> 1.7 / 3.6 / 6.3 / 12.1e-7.  Pairs of parts with rounded differences instead
+//     of exponents of differences, this kernel's forerunner: 2.3 / 5.3 / 9.3 / 17.4e-7 and 2.1 / 4.6 / 7.8 / 15.3e-7.  A correction term of the exponential changes less than 2 % of it.
 // A row whose result is not finite is done again from the keys it sees alone (plain_attention_row).
 // What bounds it (fp16 caches, 128 dims, a tile): 48 products, 0.78 us of a SIMD at the 2 GHz that the chip holds with all of them at work, beside 200 vector instructions: 1.5 us with two wavefronts a
 // SIMD; and a workgroup's way in and out, 9 us of 30 at 1777 rows.  Transposed two-byte writes of values, exponentials with a correction term, parts by rounding conversions, every wavefront reading every
@@ -213,18 +217,20 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             floatx16 s;
 #pragma unroll
             for (int r = 0; r < 16; r++) s[r] = 0.0f;
-            half8 qf[2][3];   // query parts of this step and the next: an LDS read takes as long as two steps' products
-            auto read_query = [&](int ks) __attribute__((always_inline)) {
-#pragma unroll
-                for (int p = 0; p < 3; p++) qf[ks & 1][p] = *reinterpret_cast<const half8 *>(q16 + (p * 32 + col) * LDQ + 16 * ks + 8 * half);
+            // The smaller parts of all queries first: their sums are small, and so is what rounds them.  Parts are read three products ahead.
+            half8 qf[4];
+            auto dims_of = [](int i) { return i < 2 * KS ? i / 2 : i - 2 * KS; };   // product i: of sixteen dims, with this part of the queries
+            auto read_part = [&](int i) __attribute__((always_inline)) {
+                const int part = i < 2 * KS ? 2 - i % 2 : 0;
+                qf[i & 3] = *reinterpret_cast<const half8 *>(q16 + (part * 32 + col) * LDQ + 16 * dims_of(i) + 8 * half);
             };
-            read_query(0);
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                if (ks + 1 < KS) read_query(ks + 1);
+            for (int i = 0; i < 3; i++) read_part(i);
 #pragma unroll
-                for (int p = 2; p >= 0; p--) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kr[ks]), qf[ks & 1][p], s, 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 3 * KS; i++) {
+                if (i + 3 < 3 * KS) read_part(i + 3);
+                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kr[dims_of(i)]), qf[i & 3], s, 0, 0, 0);
+                if (i % 3 == 2) __builtin_amdgcn_sched_barrier(0);
             }
             // values of this tile into LDS; nobody else reads this stretch, and a wavefront's LDS operations keep their order
 #pragma unroll
@@ -268,22 +274,29 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
                 for (int i = 0; i < 8; i += 2) split3(__fmul_rn(w[i], 32768.0f), __fmul_rn(w[i + 1], 32768.0f), p[j], i);
             };
             weights(0);
-            if (__any(alpha != 1.0f)) {   // the maximum has moved
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) o[mt][r] *= alpha;
-            }
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) v[1][mt] = read_value(1, mt);
             weights(1);
             l = __builtin_fmaf(l, alpha, psum);
+            // A tile's context by itself, the smaller parts of the weights first; then one addition, which takes the maximum's move along
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int mt = 0; mt < MT; mt += 2) {
+                floatx16 t[2];
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) t[u][r] = 0.0f;
 #pragma unroll
                 for (int i = 2; i >= 0; i--)
 #pragma unroll
-                    for (int mt = 0; mt < MT; mt++) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[j][mt], p[j][i], o[mt], 0, 0, 0);
+                    for (int j = 0; j < 2; j++)
+#pragma unroll
+                        for (int u = 0; u < 2; u++) t[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[j][mt + u], p[j][i], t[u], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[mt + u][r] = __builtin_fmaf(o[mt + u][r], alpha, t[u][r]);
+            }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
         }

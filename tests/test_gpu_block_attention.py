@@ -70,6 +70,37 @@ def test_span_attention_by_any_number_of_wavefronts(ops, rows, first, heads, kv_
     ops.set_tuning("prompt_attention_key_sets", 0)
 
 
+def in_steps(q, k, v):
+    """As exact(), but for scores that are fp32 sums of exact products of sixteen dims each."""
+    rows, heads, size = q.shape
+    first, share = k.shape[0] - rows, heads // k.shape[1]
+    out = np.empty(q.shape)
+    for h in range(heads):
+        s = np.zeros((rows, k.shape[0]), np.float32)
+        for d in range(0, size, 16):
+            s = (s + q[:, h, d:d + 16].astype(np.float64) @ k[:, h // share, d:d + 16].astype(np.float64).T).astype(np.float32)
+        s = s.astype(np.float64) / np.sqrt(size)
+        s[np.arange(k.shape[0])[None, :] > first + np.arange(rows)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = p / p.sum(1, keepdims=True) @ v[:, h // share].astype(np.float64)
+    return out
+
+
+@pytest.mark.parametrize("rows,first,heads,kv_heads,size", [(40, 700, 6, 2, 128), (300, 200, 8, 2, 128), (93, 1500, 12, 4, 64), (200, 900, 8, 4, 64)])
+def test_scores_round_as_sums_of_whole_products_do(ops, rows, first, heads, kv_heads, size):
+    """Scores of sixteen, where what rounds them outweighs the rest.  The matrix cores round twice in a product of sixteen dims: sqrt(2) of in_steps(), and a tenth for weights and sums.  Three parts of a
+    query one after the other into the same sum would be three times as many roundings."""
+    got = want = steps = []
+    for seed in (1, 2):
+        q, k, v = inputs(rows, first, heads, kv_heads, size, np.float16, seed, 16.0)
+        want = want + [exact(q, k, v)]
+        steps = steps + [in_steps(q, k, v)]
+        got = got + [ops.block_attention("span", q, k, v, split_rows=True)[0]]
+    def off(c):
+        return np.sqrt(np.mean((np.array(c) - np.array(want)) ** 2))
+    assert off(got) <= 1.1 * np.sqrt(2) * off(steps), off(got) / off(steps)
+
+
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("scale", [2.0 ** -40, 2.0 ** -12, 2.0 ** 14, 2.0 ** 60])
 def test_span_attention_takes_queries_of_any_size(ops, scale, dtype):
