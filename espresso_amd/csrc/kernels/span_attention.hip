@@ -23,7 +23,7 @@
 // SIMD; and a workgroup's way in and out, 9 us of 30 at 1777 rows.  Transposed two-byte writes of values, exponentials with a correction term, parts by rounding conversions, every wavefront reading every
 // query for its exponent and states handed on pairwise took: 1777 rows of 24 heads (8 key/value heads) 100 -> 79 us, 512 rows 21.6 -> 15.6, 93 rows of 32 heads of 64 behind 700 15.0 -> 10.4.  Against
 // attention_prompt_kernel with fp16 operands (and with pairs of them, inside a model), 32 heads, 8 key/value heads: 128 dims, 64 / 512 / 1500 rows 10.2 / 20.4 (38) / 93 (182) -> 8.3 / 17.3 / 75, 512 behind
-// 3000 85 -> 91; 64 dims, 128 / 1100 rows 7.8 / 35.5 -> 6.5 / 27.2: that kernel has 32-bit caches alone.  512 rows of 24 heads of 128 behind 1024 from fp32 caches: 137 us.
+// 3000 95 -> 92 with two parts; 64 dims, 128 / 1100 rows 7.8 / 35.5 -> 6.5 / 27.2: that kernel has 32-bit caches alone.  512 rows of 24 heads of 128 behind 1024 from fp32 caches: 137 us.
 // Query heads of a key/value head are x, x + kv_heads, ...: with eight key/value heads they share one L2.
 #include "../common.h"
 #include "attention_rows.h"
@@ -42,16 +42,17 @@ typedef short short4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// Two numbers of up to 2^15 as fp16 parts that add up to their 24 bits (each part cut off towards 0): elements e, e + 1 of p.
-__device__ __forceinline__ void split3(float v0, float v1, half8 (&p)[3], int e) {
+// Two numbers of up to 2^15 as fp16 parts, elements e, e + 1 of p: three, each cut off towards 0, add up to their 24 bits; two rounded ones leave 2^-23 of a number.
+template <int PARTS>
+__device__ __forceinline__ void split(float v0, float v1, half8 (&p)[PARTS], int e) {
     float minus = -1.0f;
     asm("" : "+v"(minus));   // v - part as one v_fma_mix: a conversion and a subtraction otherwise
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const half2 part = __builtin_bit_cast(half2, __builtin_amdgcn_cvt_pkrtz(v0, v1));
+    for (int i = 0; i < PARTS; i++) {
+        const half2 part = PARTS == 3 ? __builtin_bit_cast(half2, __builtin_amdgcn_cvt_pkrtz(v0, v1)) : half2{(_Float16)v0, (_Float16)v1};
         p[i][e] = part[0];
         p[i][e + 1] = part[1];
-        if (i == 2) break;
+        if (i == PARTS - 1) break;
         v0 = __builtin_fmaf((float)part[0], minus, v0);
         v1 = __builtin_fmaf((float)part[1], minus, v1);
     }
@@ -100,11 +101,12 @@ __device__ __forceinline__ float exp_weight(float x) {
 // than matrix work, and one wavefront's hides under the other's.
 constexpr int span_waves_per_simd(int hd, bool kv_f16, int kp) { return hd == 64 || (kv_f16 && kp > 1) ? 2 : 1; }
 
-template <int HD, bool KV_F16, int KP>
+// PARTS: of the 32-bit operands that meet fp16 caches
+template <int HD, bool KV_F16, int KP, int PARTS = 3>
 __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void span_attention_kernel(AttentionArgs a, int rows) {
     constexpr int KS = HD / 16, MT = HD / 32, LDV = HD + 16, VP = HD / 16;   // VP: 8-dim pieces of an fp16 value tile per lane; LDV: four keys' dims fall on all banks
     constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
-    constexpr int kQueryBytes = KV_F16 ? 3 * 32 * LDQ * 2 : 32 * LDQ * 4;
+    constexpr int kQueryBytes = KV_F16 ? PARTS * 32 * LDQ * 2 : 32 * LDQ * 4;
     constexpr int kWave = KV_F16 ? 32 * LDV * 2 : 0;                        // a value tile per wavefront
     constexpr int OWN = MT * 16 / KP, kMergeBytes = KP > 1 ? KP * (KP - 1) * OWN * 64 * 4 : 16;   // accumulators that a wavefront finishes
     __shared__ __attribute__((aligned(16))) unsigned char smem[kQueryBytes + KP * kWave > kMergeBytes ? kQueryBytes + KP * kWave : kMergeBytes];
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     // the queries (rows beyond the block repeat its last row, never stored)
     const size_t q_pitch = (size_t)a.n_head * HD;
     const float *queries = a.q + (size_t)m0 * q_pitch + (size_t)head * HD;
-    _Float16 *q16 = reinterpret_cast<_Float16 *>(query_mem);                   // [3][32][LDQ]
+    _Float16 *q16 = reinterpret_cast<_Float16 *>(query_mem);                   // [PARTS][32][LDQ]
     float *q32 = reinterpret_cast<float *>(query_mem);                         // [32][LDQ]
     if constexpr (KV_F16) {   // whole rows by neighbouring lanes, 32 / KP of them a wavefront
         constexpr int QL = HD / 4, QR = 64 / QL, PASSES = 32 / KP / QR;   // lanes of a row, rows of a load
@@ -174,11 +176,11 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             // where the power of two would not be a float (scores are 0 or beyond every type there), some other will do
             int q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
             q_exp = q_exp < -100 ? -100 : q_exp > 100 ? 100 : q_exp;
-            half8 p[3];
-            split3(__builtin_amdgcn_ldexpf(x[i].x, q_exp), __builtin_amdgcn_ldexpf(x[i].y, q_exp), p, 0);
-            split3(__builtin_amdgcn_ldexpf(x[i].z, q_exp), __builtin_amdgcn_ldexpf(x[i].w, q_exp), p, 2);
+            half8 p[PARTS];
+            split(__builtin_amdgcn_ldexpf(x[i].x, q_exp), __builtin_amdgcn_ldexpf(x[i].y, q_exp), p, 0);
+            split(__builtin_amdgcn_ldexpf(x[i].z, q_exp), __builtin_amdgcn_ldexpf(x[i].w, q_exp), p, 2);
 #pragma unroll
-            for (int k = 0; k < 3; k++) *reinterpret_cast<half4 *>(q16 + (k * 32 + r) * LDQ + 4 * (lane % QL)) = half4{p[k][0], p[k][1], p[k][2], p[k][3]};
+            for (int k = 0; k < PARTS; k++) *reinterpret_cast<half4 *>(q16 + (k * 32 + r) * LDQ + 4 * (lane % QL)) = half4{p[k][0], p[k][1], p[k][2], p[k][3]};
             if (lane % QL == 0) row_scale[r] = __builtin_amdgcn_ldexpf(__fmul_rn(1.0f / sqrtf((float)HD), 1.44269504f), -q_exp);
         }
     } else {
@@ -219,16 +221,17 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             for (int r = 0; r < 16; r++) s[r] = 0.0f;
             // The smaller parts of all queries first: their sums are small, and so is what rounds them.  Parts are read three products ahead.
             half8 qf[4];
-            auto dims_of = [](int i) { return i < 2 * KS ? i / 2 : i - 2 * KS; };   // product i: of sixteen dims, with this part of the queries
+            constexpr int SMALLER = KS * (PARTS - 1), ALL = KS * PARTS;
+            auto dims_of = [](int i) { return i < SMALLER ? i / (PARTS - 1) : i - SMALLER; };   // product i: of sixteen dims, with this part of the queries
             auto read_part = [&](int i) __attribute__((always_inline)) {
-                const int part = i < 2 * KS ? 2 - i % 2 : 0;
+                const int part = i < SMALLER ? PARTS - 1 - i % (PARTS - 1) : 0;
                 qf[i & 3] = *reinterpret_cast<const half8 *>(q16 + (part * 32 + col) * LDQ + 16 * dims_of(i) + 8 * half);
             };
 #pragma unroll
             for (int i = 0; i < 3; i++) read_part(i);
 #pragma unroll
-            for (int i = 0; i < 3 * KS; i++) {
-                if (i + 3 < 3 * KS) read_part(i + 3);
+            for (int i = 0; i < ALL; i++) {
+                if (i + 3 < ALL) read_part(i + 3);
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, kr[dims_of(i)]), qf[i & 3], s, 0, 0, 0);
                 if (i % 3 == 2) __builtin_amdgcn_sched_barrier(0);
             }
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
                 const half4 lo = read_transposed(vrow), hi = read_transposed(vrow + 8 * LDV);
                 return half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             };
-            half8 v[2][MT], p[2][3];
+            half8 v[2][MT], p[2][PARTS];
             float psum = 0.0f;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) v[0][mt] = read_value(0, mt);
@@ -271,7 +274,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
                     psum += w[i];
                 }
 #pragma unroll
-                for (int i = 0; i < 8; i += 2) split3(__fmul_rn(w[i], 32768.0f), __fmul_rn(w[i + 1], 32768.0f), p[j], i);
+                for (int i = 0; i < 8; i += 2) split(__fmul_rn(w[i], 32768.0f), __fmul_rn(w[i + 1], 32768.0f), p[j], i);
             };
             weights(0);
 #pragma unroll
@@ -287,7 +290,7 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
 #pragma unroll
                     for (int r = 0; r < 16; r++) t[u][r] = 0.0f;
 #pragma unroll
-                for (int i = 2; i >= 0; i--)
+                for (int i = PARTS - 1; i >= 0; i--)
 #pragma unroll
                     for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -408,9 +411,9 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             sums[r >> 4] = r % 16 == 0 ? s : sums[r >> 4] + s;
         }
         if (a.ctx_hi) {
-            constexpr int PARTS = OWN < 16 ? 16 / OWN : 1;   // wavefronts that share 32 dims
-            float *parts = reinterpret_cast<float *>(smem);  // [PARTS][32 queries] of every 32 dims; the merge is behind everybody
-            if constexpr (PARTS > 1) {
+            constexpr int SHARERS = OWN < 16 ? 16 / OWN : 1;   // wavefronts that share 32 dims
+            float *parts = reinterpret_cast<float *>(smem);  // [SHARERS][32 queries] of every 32 dims; the merge is behind everybody
+            if constexpr (SHARERS > 1) {
                 const float s = sums[0] + __shfl_xor(sums[0], 32);
                 if (half == 0) parts[phase * 32 + col] = s;
                 __syncthreads();
@@ -418,11 +421,11 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
 #pragma unroll
             for (int i = 0; i < (OWN < 16 ? 1 : OWN / 16); i++) {
                 float s = 0.0f;
-                if constexpr (PARTS > 1) {
+                if constexpr (SHARERS > 1) {
 #pragma unroll
-                    for (int w = 0; w < PARTS; w++) s += parts[(phase / PARTS * PARTS + w) * 32 + col];
+                    for (int w = 0; w < SHARERS; w++) s += parts[(phase / SHARERS * SHARERS + w) * 32 + col];
                 } else s = sums[i] + __shfl_xor(sums[i], 32);
-                if (phase % PARTS == 0 && half == 0 && col <= last_row) store_context_sum(a, row, a.n_head * HD, head * (HD / 32) + (phase * OWN >> 4) + i, s);
+                if (phase % SHARERS == 0 && half == 0 && col <= last_row) store_context_sum(a, row, a.n_head * HD, head * (HD / 32) + (phase * OWN >> 4) + i, s);
             }
         }
         return;
@@ -431,12 +434,17 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
 }
 
 template <int HD, bool KV_F16>
-void launch_shape(const AttentionArgs &a, int rows, int sets, hipStream_t s) {
+void launch_shape(const AttentionArgs &a, int rows, int sets, bool pairs, hipStream_t s) {
     const dim3 grid(a.n_head, a.tiles ? a.tile_count : (rows + 31) / 32);
     auto go = [&](auto waves) {
         constexpr int KP = decltype(waves)::value;
         hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, KP>), grid, dim3(64 * KP), 0, s, a, rows);
     };
+    if constexpr (HD == 128 && KV_F16)
+        if (pairs) {
+            hipLaunchKernelGGL((span_attention_kernel<HD, KV_F16, 4, 2>), grid, dim3(256), 0, s, a, rows);
+            return;
+        }
     if constexpr (!KV_F16) {
         if (sets == 1) return go(std::integral_constant<int, 1>{});
         if (sets == 2) return go(std::integral_constant<int, 2>{});
@@ -455,7 +463,7 @@ bool span_attention_supported(int n_head, int n_kv_head, int head_dim) {
     return n_kv_head > 0 && n_head % n_kv_head == 0 && (head_dim == 64 || head_dim == 128);
 }
 
-hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, bool kv_f16, hipStream_t s) {
+hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, bool kv_f16, hipStream_t s, bool pairs_do) {
     if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup, fp32 caches: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
@@ -470,12 +478,16 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
         const int forced = rows < 32 ? 0 : g_key_sets.load();   // (short blocks are by size whatever the key says)
         sets = forced ? 4 * forced : tiles >= 24 && groups <= cus ? 8 : 4;
     }
+    // Long walks over the keys are bound by the products (48 of a tile of 128 dims with three parts, 32 with two), and a context that is rounded to fp16 shows neither.  512 rows of 32 heads (8 key/value heads)
+    // behind 1500 / 2000 / 3000 / 6000 / 15000, fp16 operands / three parts / two, us: 58 / 57 / 54, 71 / 70 / 66, 95 / 99 / 92, 168 / 182 / 169, 382 / 409 / 379.  Up to 2048 keys three parts are no slower
+    // than fp16 operands were; nor are they where the workgroups are eight wavefronts (93 rows behind 3000 77 / 41) or heads are 64 dims (512 behind 8000 220 / 127).
+    const bool pairs = pairs_do && kv_f16 && a.head_dim == 128 && !a.ctx_hi && sets == 4 && keys > 2048;
     if (a.head_dim == 128) {
-        if (kv_f16) launch_shape<128, true>(a, rows, sets, s);
-        else launch_shape<128, false>(a, rows, sets, s);
+        if (kv_f16) launch_shape<128, true>(a, rows, sets, pairs, s);
+        else launch_shape<128, false>(a, rows, sets, false, s);
     } else {
-        if (kv_f16) launch_shape<64, true>(a, rows, sets, s);
-        else launch_shape<64, false>(a, rows, sets, s);
+        if (kv_f16) launch_shape<64, true>(a, rows, sets, false, s);
+        else launch_shape<64, false>(a, rows, sets, false, s);
     }
     return hipGetLastError();
 }

@@ -70,6 +70,21 @@ def test_span_attention_by_any_number_of_wavefronts(ops, rows, first, heads, kv_
     ops.set_tuning("prompt_attention_key_sets", 0)
 
 
+# prompts of more rows than one workgroup a compute unit (32 heads by 16 tiles of rows) up to 2048 keys, and behind them
+@pytest.mark.parametrize("rows,first", [(512, 1536), (512, 1537), (490, 1650), (481, 3000)])
+def test_prompts_behind_long_prefixes_are_as_exact_as_rows_alone(ops, rows, first):
+    for sharp in (1.0, 30.0):
+        q, k, v = inputs(rows, first, 32, 8, 128, np.float16, rows, sharp)
+        at = np.r_[0:3, 30:34, rows - 9:rows]
+        want = np.concatenate([exact(q[i:i + 1], k[:first + i + 1], v[:first + i + 1]) for i in at])
+        def off(c):
+            return np.sqrt(np.mean((c - want) ** 2))
+        one = ops.block_attention("single_row", q, k, v)[0][at]
+        for kernel in ("prompt", "span"):   # the same fp16 rounding of the context on all sides
+            assert off(ops.block_attention(kernel, q, k, v)[0][at]) <= 1.02 * off(one) + 1e-9, (kernel, sharp)
+        assert off(ops.block_attention("prompt", q, k, v, split_rows=True)[0][at]) <= 2.0 ** -24 * (np.sqrt(128) * sharp + 8) + 2.0 ** -22 * np.sqrt(np.mean(want ** 2))
+
+
 def in_steps(q, k, v):
     """As exact(), but for scores that are fp32 sums of exact products of sixteen dims each."""
     rows, heads, size = q.shape
