@@ -173,9 +173,8 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
         for (int i = 0; i < PASSES; i++) {
             const int r = phase * (32 / KP) + i * QR + lane / QL;
             const float most = row_max<QL>(fmaxf(fmaxf(fabsf(x[i].x), fabsf(x[i].y)), fmaxf(fabsf(x[i].z), fabsf(x[i].w))));
-            // where the power of two would not be a float (scores are 0 or beyond every type there), some other will do
-            int q_exp = 15 - __builtin_amdgcn_frexp_expf(most);
-            q_exp = q_exp < -100 ? -100 : q_exp > 100 ? 100 : q_exp;
+            // never below -113; where the power of two would not be a float (queries of 2^-86 and less: their scores are 0), some other will do
+            const int wanted = 15 - __builtin_amdgcn_frexp_expf(most), q_exp = wanted > 100 ? 100 : wanted;
             half8 p[PARTS];
             split(__builtin_amdgcn_ldexpf(x[i].x, q_exp), __builtin_amdgcn_ldexpf(x[i].y, q_exp), p, 0);
             split(__builtin_amdgcn_ldexpf(x[i].z, q_exp), __builtin_amdgcn_ldexpf(x[i].w, q_exp), p, 2);

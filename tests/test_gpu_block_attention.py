@@ -135,6 +135,18 @@ def test_span_attention_takes_queries_of_any_size(ops, scale, dtype):
         assert near[0] >= near[1] - 0.02 > 0.9
 
 
+@pytest.mark.parametrize("kernel,heads,size", [("span", 6, 128), ("span", 6, 64), ("prompt", 8, 128)])
+def test_the_largest_queries_meet_fp16_caches(ops, kernel, heads, size):
+    """Queries of up to 2^120, whose scores are still floats: one key takes everything, as above."""
+    q, k, v = inputs(40, 50, heads, 2, size, np.float16, 8)
+    q, k = q * np.float32(2.0 ** 118), (k / 64).astype(np.float16)
+    want = exact(q, k, v)
+    got, _ = ops.block_attention(kernel, q, k, v)
+    one, _ = ops.block_attention("single_row", q, k, v)
+    near = [(np.abs(c - want).max(-1) <= 2.0 ** -11 * np.abs(want).max(-1)).mean() for c in (got, one)]
+    assert near[0] >= near[1] - 0.02 > 0.9
+
+
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("magnitude", [3e-7, 1e-3, 3e4, 3e8])
 def test_span_attention_takes_values_of_any_size(ops, magnitude, dtype):
