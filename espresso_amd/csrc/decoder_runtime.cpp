@@ -358,7 +358,7 @@ int DecoderRuntime::head_rows(int count, uint32_t *tokens) {
 
 // One row at a time is a read of the head, a copy and a wait each: after sixteen prompts of an 8B Q4_K model (128256 x 4096) 1.2 ms, together 0.09.
 int DecoderRuntime::select_greedy_rows(int count, uint32_t *tokens) {
-    if (finalized_ && tokens && count >= 1 && count <= kMaxStepRows && count <= shape().max_sequences && head_is_as_exact_for_rows()) return select_rows(last_hidden_, count, tokens);
+    if (finalized_ && tokens && count >= 1 && count <= kMaxStepRows && count <= shape().max_sequences && head_is_as_exact_for_rows(count)) return select_rows(last_hidden_, count, tokens);
     for (int s = 0; s < count; s++) {
         const int rc = select_greedy(s, &tokens[s]);
         if (rc != ESP_OK) return rc;

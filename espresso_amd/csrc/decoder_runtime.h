@@ -131,8 +131,8 @@ class DecoderRuntime {
     // want_logits: the full-vocabulary logits are needed in logits_ (otherwise the head may store none)
     virtual int run_head(const float *hidden_rows, int count, bool want_logits = false) = 0;
     int select_rows(const float *hidden_rows, int count, uint32_t *tokens);   // run_head and its tokens
-    // Does run_head round the rows of a batch no more than a single one?
-    virtual bool head_is_as_exact_for_rows() const { return false; }
+    // Does run_head round no more for `count` rows than for a single one?
+    virtual bool head_is_as_exact_for_rows(int) const { return false; }
     // One greedy choice under capture: head over the sequence's kept state, the token into row 0 and the log, and what
     // enqueue_trunk(1, true) needs of its embedding.
     virtual int enqueue_greedy_token(int seq) = 0;

@@ -880,6 +880,21 @@ int LlamaRuntime::enqueue_device_head_candidates(HeadTokens *head) {
     return run_head_candidates(hidden_, 2, &head->blocks);
 }
 
+// More than two rows: one product, unless the weights are 32-bit or the caller keeps prompts from blocks.
+bool LlamaRuntime::head_in_one_product(int count) const { return count > 2 && matrix_prefill_ && lm_head_.format != FMT_F32 && lm_head_.cols % 64 == 0; }
+
+GemmParams LlamaRuntime::head_product(int count) const {
+    GemmParams m;
+    m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = gemm_workspace_floats_;
+    return m;
+}
+
+// Normed rows are fp16 and sums 32-bit either way, and so are weights as they are, but for products that round them to fp16: heads of 49152 x 576 (Q8_0, Q4_0) from three rows on, Q4_K ones from nine rows on
+// where neither launch for sixteen rows knows their width.
+bool LlamaRuntime::head_is_as_exact_for_rows(int count) const {
+    return !head_in_one_product(count) || gemv_takes_sixteen_rows(lm_head_, count) || gemm_keeps_weights(head_product(count));
+}
+
 int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits) {
     hipStream_t s = context().stream;
     if (count <= 2 && !want_logits && head_fuses_argmax()) {
@@ -888,7 +903,7 @@ int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits
         ESP_HIP_TRY(launch_argmax_final(argmax_scratch_, blocks, count, d_out_tokens_, s));
         return ESP_OK;
     }
-    if (count > 2 && matrix_prefill_ && lm_head_.format != FMT_F32 && lm_head_.cols % 64 == 0) {
+    if (head_in_one_product(count)) {
         // batched rows: final RMSNorm, then the head as one MFMA GEMM
         ESP_HIP_TRY(launch_rmsnorm(hidden_rows, final_norm_, c_.norm_eps, count, c_.d_model, xn_, nullptr, s));
         if (gemv_takes_sixteen_rows(lm_head_, count)) {
@@ -898,9 +913,7 @@ int LlamaRuntime::run_head(const float *hidden_rows, int count, bool want_logits
             ESP_HIP_TRY(launch_argmax(logits_, count, c_.vocab, d_out_tokens_, nullptr, argmax_scratch_, s));
             return ESP_OK;
         }
-        GemmParams m;
-        m.w = lm_head_; m.x = xn_; m.y = logits_; m.rows = count; m.unrounded = true; m.workspace = gemm_workspace_; m.workspace_floats = gemm_workspace_floats_;
-        ESP_HIP_TRY(launch_gemm(m, s));
+        ESP_HIP_TRY(launch_gemm(head_product(count), s));
         ESP_HIP_TRY(launch_argmax(logits_, count, c_.vocab, d_out_tokens_, nullptr, argmax_scratch_, s));
         return ESP_OK;
     }

@@ -86,7 +86,9 @@ class LlamaRuntime : public DecoderRuntime {
     int upload_vector(const HostTensor &t, size_t count, float **out, const char *what);
     // without want_logits one or two rows take the head whose epilogue is the arg-max and store none
     int run_head(const float *hidden_rows, int count, bool want_logits = false) override;
-    bool head_is_as_exact_for_rows() const override { return true; }   // normed rows to fp16, weights as they are, sums in 32 bits: either way
+    bool head_in_one_product(int count) const;
+    GemmParams head_product(int count) const;
+    bool head_is_as_exact_for_rows(int count) const override;
     int run_head_candidates(const float *hidden_rows, int count, int *blocks);   // head_fuses_argmax() only
     bool head_fuses_argmax() const { return fused_head_argmax_ && gemv_supports_argmax(lm_head_); }
     int enqueue_trunk(int rows, bool embedded = false, float *final_out = nullptr) override;

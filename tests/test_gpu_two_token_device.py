@@ -191,3 +191,47 @@ def test_first_tokens_of_a_batch_are_those_of_its_sequences(llama, fmt, n_seq):
         if top[1] - top[0] > 1e-3:
             assert got[s] == [rt.select_greedy(s)]
     rt.close()
+
+
+def near_head(fmt, rows, cols, seed):
+    """Blocks of a head whose rows are one row of large weights and a little noise: their logits lie as close as rounding the weights to fp16 moves them (0.02 of a step where the rows differ by one
+    or two), and sums of 32 bits do not."""
+    rng = np.random.default_rng(seed)
+    half = lambda x: np.asarray(x, np.float16).view(np.uint8).reshape(*np.shape(x), 2)  # noqa: E731
+    if fmt in (orc.FMT_Q8_0, orc.FMT_Q4_0):
+        n = cols // 32
+        d = np.broadcast_to(half(rng.uniform(0.001, 0.002, n)), (rows, n, 2))
+        if fmt == orc.FMT_Q8_0:
+            q = (rng.integers(64, 126, cols) * rng.choice([-1, 1], cols))[None] + rng.integers(-2, 3, (rows, cols), dtype=np.int8)
+            return np.concatenate([d, q.astype(np.int8).view(np.uint8).reshape(rows, n, 32)], -1).ravel()
+        q = np.where(rng.random(cols) < 0.5, rng.integers(0, 3, (rows, cols)), rng.integers(13, 16, (rows, cols))).astype(np.uint8).reshape(rows, n, 32)
+        return np.concatenate([d, q[..., :16] | q[..., 16:] << 4], -1).ravel()
+    n = cols // 256
+    sc, m = rng.integers(1, 64, (n, 8)).astype(np.uint8), rng.integers(32, 64, (n, 8)).astype(np.uint8)   # value sc d q - m dmin, the second part a hundred times the first one's step
+    head = np.concatenate([half(rng.uniform(1e-5, 2e-5, n)), half(rng.uniform(1e-3, 2e-3, n)), sc[:, :4] | sc[:, 4:] >> 4 << 6, m[:, :4] | m[:, 4:] >> 4 << 6, sc[:, 4:] & 15 | (m[:, 4:] & 15) << 4], -1)
+    return np.concatenate([np.broadcast_to(head, (rows, n, 16)), rng.integers(0, 256, (rows, n, 128), dtype=np.uint8)], -1).ravel()
+
+
+# a vocabulary and widths that no kernel with exact weights takes as a batch (Q4_K from nine rows on), and ones that one does
+@pytest.mark.parametrize("fmt,d_model,vocab,n_seq", [(orc.FMT_Q8_0, 576, 49152, 3), (orc.FMT_Q8_0, 576, 49152, 16), (orc.FMT_Q4_0, 576, 49152, 16), (orc.FMT_Q4_K, 1536, 32000, 9), (orc.FMT_Q4_K, 1536, 32000, 8),
+                                                     (orc.FMT_Q8_0, 768, 32000, 16), (orc.FMT_Q4_K, 1024, 32000, 16), (orc.FMT_Q4_0, 2048, 32000, 3)])
+def test_first_tokens_of_a_batch_hang_on_exact_heads(llama, fmt, d_model, vocab, n_seq):
+    kw = dict(n_layer=1, n_head=d_model // 64, n_kv_head=d_model // 64, d_model=d_model, head_dim=64, hidden_dim=512, max_seq=16)
+    packed = mu.pack_weights(mu.random_weights(orc.LlamaConfig(gemv_inputs_fp16=True, vocab=256, **kw), 5, std=0.05), fmt)[0]
+    packed["embedding"] = np.random.default_rng(6).normal(0, 1, (vocab, d_model)).astype(np.float16).view(np.uint8).ravel()
+    packed["lm_head"] = near_head(fmt, vocab, d_model, 7)
+    rt = llama.LlamaRuntime(llama.MultiModelConfig(vocab=vocab, **kw), max_sequences=n_seq)
+    llama.load_packed_weights(rt, packed, fmt)
+    rng = np.random.default_rng(n_seq)
+    checked = 0
+    for _ in range(max(2, 192 // n_seq)):
+        rt.reset()
+        got = llama.generate_batch(rt, [rng.integers(0, vocab, 3 + s % 4).astype(np.uint32) for s in range(n_seq)], 1)[0]
+        for s in range(n_seq):
+            logits = rt.logits(s)
+            top = np.sort(logits)[-2:]
+            if top[1] - top[0] > 1e-3 * logits.std():   # what a hidden row's own rounding to fp16 may move
+                assert got[s] == [rt.select_greedy(s)], s
+                checked += 1
+    assert checked > 100
+    rt.close()
