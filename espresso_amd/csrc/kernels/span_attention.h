@@ -14,6 +14,6 @@ inline hipError_t launch_prompt_attention(const AttentionArgs &a, int rows, int 
     if (!attention_prompt_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     return kv_f16 ? launch_span_attention(a, rows, keys, true, s, true) : launch_attention_prompt(a, rows, s);
 }
-void attention_prompt_set_key_sets(int sets);   // fp16 caches, 32 rows and more: 0 = wavefronts of a workgroup by size (default), 1 or 2 = always four or eight
+void attention_prompt_set_key_sets(int sets);   // fp16 caches: 0 = wavefronts of a workgroup by size (default), 1 or 2 = always four or eight
 
 }  // namespace esp

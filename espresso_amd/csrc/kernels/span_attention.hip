@@ -474,7 +474,7 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     if (!kv_f16) {
         while (sets < 8 && groups * sets < 1024 && sets * 2 <= tiles) sets *= 2;
     } else {
-        const int forced = rows < 32 ? 0 : g_key_sets.load();   // (short blocks are by size whatever the key says)
+        const int forced = g_key_sets.load();
         sets = forced ? 4 * forced : tiles >= 24 && groups <= cus ? 8 : 4;
     }
     // Long walks over the keys are bound by the products (48 of a tile of 128 dims with three parts, 32 with two), and a context that is rounded to fp16 shows neither.  512 rows of 32 heads (8 key/value heads)

@@ -56,9 +56,10 @@ def test_span_attention_is_as_exact_as_fp32(ops, rows, first, heads, kv_heads, s
             assert off(got) <= 1.02 * off(one) + 1e-9, sharp
 
 
-# four and eight wavefronts (1, 2) where some have no tile of keys, one, or one more than the others; the shares of dims that they finish, and their sums of 32
-@pytest.mark.parametrize("sets", [1, 2])
-@pytest.mark.parametrize("rows,first,heads,kv_heads,size", [(1, 0, 4, 4, 64), (1, 31, 2, 1, 128), (32, 1, 12, 4, 64), (33, 95, 2, 2, 128), (64, 193, 6, 2, 128), (31, 224, 4, 1, 64), (2, 255, 8, 2, 128)])
+# four and eight wavefronts (1, 2; 0: by size, eight from 24 tiles of keys on) where some have no tile of keys, one, or one more than the others; the shares of dims that they finish, and their sums of 32
+@pytest.mark.parametrize("sets", [0, 1, 2])
+@pytest.mark.parametrize("rows,first,heads,kv_heads,size", [(1, 0, 4, 4, 64), (1, 31, 2, 1, 128), (32, 1, 12, 4, 64), (33, 95, 2, 2, 128), (64, 193, 6, 2, 128), (31, 224, 4, 1, 64), (2, 255, 8, 2, 128), (31, 737, 4, 1, 64),
+                                                             (5, 731, 8, 2, 128), (1, 800, 12, 4, 64)])
 def test_span_attention_by_any_number_of_wavefronts(ops, rows, first, heads, kv_heads, size, sets):
     ops.set_tuning("prompt_attention_key_sets", sets)
     q, k, v = inputs(rows, first, heads, kv_heads, size, np.float16, rows + first, 4.0)
