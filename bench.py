@@ -523,7 +523,7 @@ def main() -> None:
                                       "all_gemv_frac_kernel_durations: over the kernels' own durations (kernel_us), as a kernel trace adds them up",
                      "all_gemv_frac_kernel_durations": gemv_bytes / gemv_kernel_us / 1e3 / HBM_PEAK_GBPS if gemv_kernel_us else 0.0,
                      "per_kernel": {k: {"mean_us": round(v["mean_us"], 2), "gbps": round(v["gbps"], 1), "launches": v["launches"]}
-                                    for k, v in kt.items()},
+                                    for k, v in kt.items() if v["launches"]},
                      "how": "achieved/mean_launch_us: the dominant kernel launched for each layer's matrix in turn, 8 rounds on the "
                             "library stream after the timed region, every launch with a pair of HIP events of its own that take the "
                             "kernel's start and end (hipExtLaunchKernel): the mean kernel duration, the figure a rocprofv3 kernel trace "
@@ -562,7 +562,7 @@ def main() -> None:
                    "steps": osteps, "ms_per_step": g2["elapsed"] / osteps * 1e3, "workload": other,
                    "weight_bytes_per_token": g2["weight_bytes"],
                    "frac_hbm_peak_whole_token": g2["weight_bytes"] / (g2["elapsed"] / osteps) / 1e9 / HBM_PEAK_GBPS,
-                   "per_kernel": {k: {"mean_us": round(v["mean_us"], 2), "gbps": round(v["gbps"], 1)} for k, v in g2["kernel_times"].items()},
+                   "per_kernel": {k: {"mean_us": round(v["mean_us"], 2), "gbps": round(v["gbps"], 1)} for k, v in g2["kernel_times"].items() if v["launches"]},
                    "per_kernel_note": "raw HIP-event means, event-pair overhead (see event_pair) included"}
             if not args.no_cpu_baseline:
                 sec["cpu_baseline"] = cpu_baseline(other, g2)

@@ -113,7 +113,9 @@ int LlamaRuntime::time_kernel_class(int kernel_class, int iters, double *mean_us
             if (wo_merges_attention(*L, 1)) { g.x = nullptr; g.merge_partials = attn_scratch_; g.merge_head_dim = c_.head_dim; }
             break;
         case K_GATE_UP:
-            g.w = L->w13; g.norm_x = hidden_; g.norm_w = L->rms_ffn; g.norm_eps = c_.norm_eps; g.out_f16 = act_; g.epilogue = EPI_SWIGLU_F16;
+            g.w = L->w13; g.norm_w = L->rms_ffn; g.norm_eps = c_.norm_eps; g.out_f16 = act_; g.epilogue = EPI_SWIGLU_F16;
+            if (projects_attention(*L, 1)) { g.norm_planes = gemm_workspace_; g.norm_plane_count = c_.n_head; g.norm_sum = gemm_workspace_ + (size_t)c_.n_head * c_.d_model; }
+            else g.norm_x = hidden_;
             g.split_out = split_activations_ && gemv_splits_activations(L->w2, 1);
             break;
         case K_DOWN: g.w = L->w2; g.x = act_; g.y = hidden_; g.residual = hidden_; g.epilogue = EPI_ADD_RESIDUAL; break;
@@ -129,16 +131,24 @@ int LlamaRuntime::time_kernel_class(int kernel_class, int iters, double *mean_us
         g.split_x = kernel_class != K_HEAD && !(g.x == ctx_ && kernel_class == K_WO) && split_activations_ && gemv_splits_activations(g.w, 1);
         return launch_gemv(g, s);
     };
+    std::vector<const Layer *> round;   // the class's launches of a step
+    if (kernel_class == K_HEAD) round.push_back(nullptr);
+    else
+        for (const Layer &L : layers_)
+            if (kernel_class != K_WO || !projects_attention(L, 1)) round.push_back(&L);
+    *mean_us = 0.0;
+    if (kernel_only_us) *kernel_only_us = 0.0;
+    if (round.empty()) return ESP_OK;
     StepRows rows{};
     rows.count = 1;
     ESP_HIP_TRY(launch_set_rows(rows, d_tokens_, d_pos_, d_seq_, s));
     hipEvent_t t0 = take_event(), t1 = take_event();
     if (!t0 || !t1) return fail(ESP_ERR_OUT_OF_MEMORY, "time_kernel_class: events");
-    const int per_round = kernel_class == K_HEAD ? 1 : (int)layers_.size();
-    for (int i = 0; i < per_round; i++) ESP_HIP_TRY(launch(kernel_class == K_HEAD ? nullptr : &layers_[(size_t)i]));   // warm-up round
+    const int per_round = (int)round.size();
+    for (const Layer *L : round) ESP_HIP_TRY(launch(L));   // warm-up round
     ESP_HIP_TRY(hipEventRecord(t0, s));
     for (int r = 0; r < iters; r++)
-        for (int i = 0; i < per_round; i++) ESP_HIP_TRY(launch(kernel_class == K_HEAD ? nullptr : &layers_[(size_t)i]));
+        for (const Layer *L : round) ESP_HIP_TRY(launch(L));
     ESP_HIP_TRY(hipEventRecord(t1, s));
     ESP_HIP_TRY(hipEventSynchronize(t1));
     float ms = 0.0f;
@@ -152,7 +162,7 @@ int LlamaRuntime::time_kernel_class(int kernel_class, int iters, double *mean_us
         for (hipEvent_t &e : ev) if (!(e = take_event())) return fail(ESP_ERR_OUT_OF_MEMORY, "time_kernel_class: events");
         for (int r = 0, k = 0; r < iters; r++)
             for (int i = 0; i < per_round; i++, k += 2)
-                ESP_HIP_TRY(launch(kernel_class == K_HEAD ? nullptr : &layers_[(size_t)i], ev[(size_t)k], ev[(size_t)k + 1]));
+                ESP_HIP_TRY(launch(round[(size_t)i], ev[(size_t)k], ev[(size_t)k + 1]));
         ESP_HIP_TRY(hipStreamSynchronize(s));
         double total = 0.0;
         for (size_t k = 0; k < ev.size(); k += 2) {
@@ -171,7 +181,7 @@ size_t LlamaRuntime::kernel_bytes(int kernel_class) const {
     auto io = [](const DeviceMatrix &m) { return m.bytes() + (size_t)m.cols * 2 + (size_t)m.rows * 4; };
     switch (kernel_class) {
     case K_QKV: return io(L.wqkv);
-    case K_WO: return io(L.wo);
+    case K_WO: return projects_attention(L, 1) ? 0 : io(L.wo);   // (no launch of its own there)
     case K_GATE_UP: return io(L.w13);
     case K_DOWN: return io(L.w2);
     case K_HEAD: return io(lm_head_) - (head_fuses_argmax() ? (size_t)lm_head_.rows * 4 : 0);   // the fused head stores no logits

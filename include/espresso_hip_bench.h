@@ -94,7 +94,8 @@ int esp_hbm_read_probe_pairs(size_t bytes_per_launch, int pair_bytes, int workgr
  * and reports, per kernel class, the summed elapsed microseconds, the launch count and the
  * algorithmic bytes of one batch-1 launch (packed weights + fp16 input + fp32 output).  Class
  * ESP_KERNEL_EVENT_PAIR brackets nothing, once per step: its mean is what an event pair itself adds to
- * every other class's mean. */
+ * every other class's mean.  Small models whose steps have attention and wo in one launch count it as
+ * attention: ESP_KERNEL_WO then has no launches, no bytes and, below, no time. */
 #define ESP_KERNEL_QKV 0
 #define ESP_KERNEL_WO 1
 #define ESP_KERNEL_GATE_UP 2

@@ -74,5 +74,8 @@ def test_attention_and_projection_in_one_launch_match_oracle(mods, n_head, n_kv,
         assert np.abs(o.logits() - g.logits()).max() <= 2e-2
     ll.set_kernel_timing(g, True)
     g.advance(0)
-    assert (ll.kernel_times(g)["wo"]["launches"] == 0) == (n_head <= 12 and max_seq <= 512)
+    times, joint = ll.kernel_times(g), n_head <= 12 and max_seq <= 512
+    assert (times["wo"]["launches"] == 0) == joint and (times["wo"]["bytes_per_launch"] == 0) == joint
+    for name in ("qkv", "wo", "gate_up", "down", "head"):   # launched by themselves: what a step launches and nothing else
+        assert (min(ll.time_kernel_dispatch(g, name, 1)) > 0) == (max(ll.time_kernel_dispatch(g, name, 1)) > 0) == (name != "wo" or not joint)
     g.close()
