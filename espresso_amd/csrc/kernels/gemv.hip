@@ -1109,6 +1109,9 @@ struct MfmaStage {
     uint4 v[MODE == 0 ? NBX : 1][K];
     float4 a0[MODE == 2 ? K : 1][kMergeSplits], a1[MODE == 2 ? K : 1][kMergeSplits];
     float2 ml[MODE == 2 ? K : 1][kMergeSplits];
+    // MODE 3: the norm of a sum of planes, four columns a thread, as gemv_kernel adds and norms them (KernelArgs::norm_planes)
+    static_assert(MODE != 3 || (GROUPS * 2 == THREADS && !Q40 && !SPLIT), "four columns for every thread");
+    float4 pv[MODE == 3 ? NB : 1][MODE == 3 ? kMaxNormPlanes : 1], pg;
 
     __device__ __forceinline__ int group(int k) const { return FULL || (int)threadIdx.x + k * THREADS < GROUPS ? (int)threadIdx.x + k * THREADS : 0; }
     __device__ __forceinline__ bool mine(int k) const { return FULL || (int)threadIdx.x + k * THREADS < GROUPS; }
@@ -1120,7 +1123,14 @@ struct MfmaStage {
         for (int k = 0; k < K; k++) merge_group_load(a, b, group(k), cols, ml[k], a0[k], a1[k]);
     }
     __device__ __forceinline__ void issue(const KernelArgs &a) {
-        if constexpr (MODE == 1) {
+        if constexpr (MODE == 3) {
+            const float4 *p4 = reinterpret_cast<const float4 *>(a.norm_planes);
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int k = 0; k < kMaxNormPlanes; k++) pv[b][k] = p4[(b * a.norm_plane_count + (k < a.norm_plane_count ? k : a.norm_plane_count - 1)) * (cols / 4) + (int)threadIdx.x];
+            pg = reinterpret_cast<const float4 *>(a.norm_w)[threadIdx.x];
+        } else if constexpr (MODE == 1) {
             const float4 *w4 = reinterpret_cast<const float4 *>(a.norm_w);
             const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -1151,7 +1161,34 @@ struct MfmaStage {
         }
     }
     __device__ __forceinline__ void finish(const KernelArgs &a, uint4 *xs4, float *xsum, float *red) {
-        if constexpr (MODE == 1) {
+        if constexpr (MODE == 3) {
+            const int tid = threadIdx.x;
+            float4 v[NB];
+            float s[NB];
+#pragma unroll
+            for (int b = 0; b < NB; b++) {   // the first plane, which holds the residual, last
+                v[b] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (int k = 1; k < kMaxNormPlanes; k++)
+                    if (k < a.norm_plane_count) { v[b].x += pv[b][k].x; v[b].y += pv[b][k].y; v[b].z += pv[b][k].z; v[b].w += pv[b][k].w; }
+                v[b].x += pv[b][0].x; v[b].y += pv[b][0].y; v[b].z += pv[b][0].z; v[b].w += pv[b][0].w;
+                s[b] = v[b].x * v[b].x + v[b].y * v[b].y + v[b].z * v[b].z + v[b].w * v[b].w;
+            }
+            workgroup_sums_waves<WAVES>(s, red);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const float inv = 1.0f / sqrtf(s[b] / (float)cols + a.norm_eps);
+                if (blockIdx.x == 0) reinterpret_cast<float4 *>(a.norm_sum)[b * (cols / 4) + tid] = v[b];
+                const u32 lo = pack_half2(__fmul_rn(__fmul_rn(v[b].x, inv), pg.x), __fmul_rn(__fmul_rn(v[b].y, inv), pg.y));
+                const u32 hi = pack_half2(__fmul_rn(__fmul_rn(v[b].z, inv), pg.z), __fmul_rn(__fmul_rn(v[b].w, inv), pg.w));
+                reinterpret_cast<uint2 *>(xs4)[b * (cols / 4) + tid] = make_uint2(__builtin_amdgcn_perm(hi, lo, 0x05040100u), __builtin_amdgcn_perm(hi, lo, 0x07060302u));
+                float t = ((float)as_h2(lo).x + (float)as_h2(lo).y) + ((float)as_h2(hi).x + (float)as_h2(hi).y);
+                t += dpp_term<0xB1, 0xF>(t);   // eight threads hold the fours of one 32
+                t += dpp_term<0x4E, 0xF>(t);
+                t += dpp_term<0x141, 0xF>(t);
+                if ((tid & 7) == 0) xsum[(size_t)b * (cols >> 5) + (tid >> 3)] = t;
+            }
+        } else if constexpr (MODE == 1) {
             float s[NB];
 #pragma unroll
             for (int b = 0; b < NB; b++) {
@@ -2045,7 +2082,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_q80_mfma_kernel(const uint8_t
     KernelArgs a = rest;
     a.rows = rows;
     if constexpr (MODE == 1) { a.norm_x = static_cast<const float *>(activations); a.norm_w = norm_w; a.norm_eps = norm_eps; }
-    else if constexpr (MODE == 2) a.merge_partials = static_cast<const float *>(activations);
+    else if constexpr (MODE == 3) {   // workgroups: the planes' number in the upper half
+        a.norm_planes = static_cast<const float *>(activations); a.norm_w = norm_w; a.norm_eps = norm_eps;
+        a.norm_plane_count = workgroups >> 16;
+        workgroups &= 0xFFFF;
+    } else if constexpr (MODE == 2) a.merge_partials = static_cast<const float *>(activations);
     else a.x = static_cast<const uint16_t *>(activations);
     constexpr int THREADS = WAVES * 64, cols = TPR * 256, IPR = cols / 64, S = TPR / KS, RB = WAVES / KS, GROUPS = cols / 8;
     constexpr int DEPTH = S % 4 == 0 ? 4 : (S % 2 == 0 ? 2 : 1);   // divides S: a step's slot in the ring is a constant
@@ -2796,8 +2837,9 @@ hipError_t launch_q80_mfma(const KernelArgs &a, hipStream_t stream, bool *launch
     const int grid = want < cap ? want : cap;
     const int iters = (want + grid - 1) / grid;
     if (KS > 1 && iters > kQ80Rounds) return hipSuccess;   // not launched: the caller takes the other kernel
-    const void *activations = MODE == 1 ? static_cast<const void *>(a.norm_x) : MODE == 2 ? static_cast<const void *>(a.merge_partials) : static_cast<const void *>(a.x);
-    launch_kernel(kernel, dim3(grid), dim3(THREADS), lds, stream, a.tiled, activations, a.norm_w, a.rows, iters, grid, a.norm_eps, a);
+    const void *activations = MODE == 3 ? static_cast<const void *>(a.norm_planes) : MODE == 1 ? static_cast<const void *>(a.norm_x) : MODE == 2 ? static_cast<const void *>(a.merge_partials) : static_cast<const void *>(a.x);
+    if (MODE == 3 && grid > 0xFFFF) return hipSuccess;
+    launch_kernel(kernel, dim3(grid), dim3(THREADS), lds, stream, a.tiled, activations, a.norm_w, a.rows, iters, MODE == 3 ? grid | (a.norm_plane_count << 16) : grid, a.norm_eps, a);
     *launched = true;
     return hipGetLastError();
 }
@@ -2816,8 +2858,12 @@ template <int NB, bool F16 = false>
 hipError_t try_q80_mfma(const KernelArgs &a, hipStream_t stream, bool *launched) {
     *launched = false;
     if (!a.tiled || q80_mfma_mode() == 0) return hipSuccess;
-    const int mode = a.merge_partials ? 2 : a.norm_x ? 1 : 0;
     const bool tall = a.rows > 8192;
+    if (a.norm_planes) {   // two rows of 4096 x 768 in fp16, 12 planes, in a trace: 5.8 us, 7.1 in gemv_kernel, whose workgroups are twice as many (each reads all planes); finished rows take 4.4
+        if constexpr (NB == 2) if (a.cols == 768 && !tall) return launch_q80_mfma<NB, 3, 3, 3, 3, F16>(a, stream, launched);
+        return hipSuccess;
+    }
+    const int mode = a.merge_partials ? 2 : a.norm_x ? 1 : 0;
 #define ESP_Q80_WIDTH(COLS_, W_)                                                                                       \
     if (a.cols == COLS_) {                                                                                            \
         if (tall) {                                                                                                   \
@@ -2839,7 +2885,7 @@ hipError_t try_q80_mfma(const KernelArgs &a, hipStream_t stream, bool *launched)
 // fp16 weights (768 and 2048 columns): the same rule
 template <int B>
 hipError_t launch_f16(const KernelArgs &a, hipStream_t stream) {
-    if (!a.norm_planes && (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192)))) {
+    if (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192))) {
         bool launched = false;
         const hipError_t e = try_q80_mfma<B, true>(a, stream, &launched);
         if (e != hipSuccess || launched) return e;
@@ -2852,7 +2898,7 @@ hipError_t launch_q80(const KernelArgs &a, hipStream_t stream) {
     // measured (us, dot-product / matrix cores): one row 2304 x 768 2.74 / 2.96, 4096 x 768 3.08 / 3.22, 768 x 2048 3.01 / 3.00, 4096 x 4096
     // 6.36 / 5.52, 32000 x 768 9.26 / 6.76, 32000 x 4096 31.5 / 26.9; two rows 3.36 / 3.17, 3.77 / 3.31, 3.47 / 3.36, 7.23 / 5.69, 12.1 / 6.8, 32.8 / 27.6:
     // two rows always, one row where the matrix is tall or wide ("q80_mfma" = 1: wherever an instantiation exists)
-    if (!a.norm_planes && (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192 || a.cols >= 4096)))) {
+    if (q80_mfma_mode() == 1 || (q80_mfma_mode() < 0 && (B >= 2 || a.rows > 8192 || a.cols >= 4096))) {
         bool launched = false;
         const hipError_t e = try_q80_mfma<B>(a, stream, &launched);
         if (e != hipSuccess || launched) return e;

@@ -3,6 +3,7 @@ candidates of one or many workgroups and heads that leave tokens, drafts that ar
 import numpy as np
 import pytest
 
+import espresso_amd._lib as lib
 import model_util as mu
 from oracle import oracle as orc
 
@@ -39,3 +40,35 @@ def test_two_token_stream_is_the_greedy_stream(ll, monkeypatch, fmt, width, head
             assert got == want
         draft.close()
     g.close()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "q8_0"])
+@pytest.mark.parametrize("n_head,hidden", [(12, 2048), (1, 64), (5, 1056), (2, 4096)])
+def test_two_rows_add_planes_on_the_matrix_cores(ll, fmt, n_head, hidden):
+    """768 columns, where attention and wo leave up to twelve planes a row to gate|up: the matrix-core kernel against the dot-product one, whose sums and norms these are, and both against single steps."""
+    import espresso_amd.ops as ops
+    import espresso_amd.synthetic as syn
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=n_head, n_kv_head=n_head, d_model=768, head_dim=64, hidden_dim=hidden, vocab=512, max_seq=64)
+    g, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=hidden, std=0.05)
+    tokens = np.random.default_rng(n_head).integers(0, cfg.vocab, 8)
+    want = []
+    for t in tokens:
+        g.advance(int(t))
+        want.append(np.concatenate([g.logits(), g.last_hidden()]))
+    got = {}
+    try:
+        ops.set_tuning("short_blocks", 0)
+        for mfma in (0, -1):
+            ops.set_tuning("q80_mfma", mfma)
+            g.reset()
+            got[mfma] = []
+            for i in range(0, 8, 2):
+                logits = g.append(tokens[i:i + 2], want=(0, 1))
+                got[mfma].append(np.concatenate([logits[1], g.last_hidden()]))
+    finally:
+        ops.set_tuning("short_blocks", 1)
+        ops.set_tuning("q80_mfma", -1)
+    g.close()
+    for i in range(4):   # other orders of fp32 sums; activations are rounded to fp16 in between
+        limit = 2.0 ** -9 * max(1.0, np.abs(want[2 * i + 1]).max())
+        assert np.abs(got[-1][i] - got[0][i]).max() <= limit and np.abs(got[-1][i] - want[2 * i + 1]).max() <= limit, i
