@@ -817,7 +817,6 @@ __global__ __launch_bounds__(WAVES * 64) void attention_partial_kernel(const flo
     }
 }
 
-constexpr int kProjectRows = 64;
 struct AttentionProject {
     size_t cache_seq_stride;
     const uint16_t *scales;
@@ -825,15 +824,15 @@ struct AttentionProject {
     float *planes;
     int rows;
 };
-// Attention and output projection of one row or two in one launch: grid (query heads, blocks of 64 rows of wo, rows).  A workgroup attends for its head over the whole prefix, as every other
+// Attention and output projection of one row or two in one launch: grid (query heads, blocks of 64 or 128 rows of wo, rows).  A workgroup attends for its head over the whole prefix, as every other
 // workgroup of the head does, and multiplies the context with its rows' 64 columns of that head; the heads' products are planes [row][heads][wo.rows] that the next norm adds
 // (GemvParams::norm_planes), the first with the residual in it.  The context is rounded to fp16 as in a block of rows, whose logits a step's are held to.  Bound by the launch, like everything beside it, and by its chain of memory trips: position ->
 // keys and values -> store; weights and residual are requested first.  In place of partial states and a GEMV that merges them, a step of 768 wide, 6 layers, Q8_0 went from 117 to 105 us, of 576
-// wide, 30 layers, fp16 from 580 to 528, and a speculative pass of the former (two rows) from 6.5 to 6.3 ms a generation of 64 tokens.
-template <bool KV_F16, int FMT, int WAVES, int U>
+// wide, 30 layers, fp16 from 580 to 528.  ROWS: of wo in a workgroup.
+template <bool KV_F16, int FMT, int WAVES, int U, int ROWS>
 __global__ __launch_bounds__(WAVES * 64) void attention_project_kernel(const float *q_rows, const void *k_cache, const void *v_cache, const int *pos, const int *seq, const uint8_t *qs, unsigned heads,
                                                                        unsigned row_bytes, AttentionProject p) {
-    constexpr int HD = 64, THREADS = WAVES * 64, LPR = FMT == FMT_F16 ? 8 : FMT == FMT_Q8_0 ? 4 : 2, PASS = THREADS / LPR, PASSES = (kProjectRows + PASS - 1) / PASS;   // LPR: lanes of a row's 64 columns
+    constexpr int HD = 64, THREADS = WAVES * 64, LPR = FMT == FMT_F16 ? 8 : FMT == FMT_Q8_0 ? 4 : 2, PASS = THREADS / LPR, PASSES = (ROWS + PASS - 1) / PASS;   // LPR: lanes of a row's 64 columns
     AttentionArgs a = {};
     a.q = q_rows; a.k_cache = k_cache; a.v_cache = v_cache; a.n_head = (int)(heads & 0xFFFFu); a.n_kv_head = (int)(heads >> 16); a.cache_seq_stride = p.cache_seq_stride;
     __shared__ float wm[WAVES], wl[WAVES], wacc[WAVES][HD], ctx[HD];
@@ -843,7 +842,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_project_kernel(const flo
     uint4 w[PASSES];
     uint16_t d[PASSES];
     float before[PASSES];
-    auto row_of = [&](int i) { const int r = (int)blockIdx.y * kProjectRows + i * PASS + tid / LPR; return r < p.rows ? r : p.rows - 1; };
+    auto row_of = [&](int i) { const int r = (int)blockIdx.y * ROWS + i * PASS + tid / LPR; return r < p.rows ? r : p.rows - 1; };
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
         const int r = row_of(i);
@@ -891,8 +890,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_project_kernel(const flo
         sum += dpp_get<0xB1>(sum);                          // quad_perm [1,0,3,2]
         if constexpr (LPR >= 4) sum += dpp_get<0x4E>(sum);  // quad_perm [2,3,0,1]
         if constexpr (LPR == 8) sum += dpp_get<0x141>(sum); // row_half_mirror
-        const int r = (int)blockIdx.y * kProjectRows + i * PASS + tid / LPR;
-        if (part == 0 && i * PASS + tid / LPR < kProjectRows && r < p.rows) p.planes[(size_t)(m * a.n_head + head) * p.rows + r] = head == 0 ? before[i] + sum : sum;
+        const int r = (int)blockIdx.y * ROWS + i * PASS + tid / LPR;
+        if (part == 0 && i * PASS + tid / LPR < ROWS && r < p.rows) p.planes[(size_t)(m * a.n_head + head) * p.rows + r] = head == 0 ? before[i] + sum : sum;
     }
 }
 
@@ -1570,12 +1569,25 @@ bool attention_project_supported(const DeviceMatrix &wo, int n_head, int n_kv_he
 
 template <bool KV_F16, int FMT>
 void launch_attention_project_format(const AttentionArgs &a, const DeviceMatrix &wo, const AttentionProject &p, int rows, hipStream_t s) {
-    const dim3 grid(a.n_head, (wo.rows + kProjectRows - 1) / kProjectRows, rows);
     const unsigned heads = (unsigned)a.n_head | ((unsigned)a.n_kv_head << 16);
+    auto go = [&](auto waves, auto block) {
+        constexpr int WAVES = decltype(waves)::value, ROWS = decltype(block)::value;
+        hipLaunchKernelGGL((attention_project_kernel<KV_F16, FMT, WAVES, 2, ROWS>), dim3(a.n_head, (wo.rows + ROWS - 1) / ROWS, rows), dim3(WAVES * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, wo.qs,
+                           heads, (unsigned)wo.qs_row_bytes, p);
+    };
+    typedef std::integral_constant<int, 4> Four;
+    typedef std::integral_constant<int, 8> Eight;
+    typedef std::integral_constant<int, 64> Narrow;
+    typedef std::integral_constant<int, 128> Wide;
     // Four wavefronts start and merge sooner, eight walk a longer prefix in fewer passes.  48 tokens, four / eight: 768 wide, 6 layers, Q8_0 from position 16 of 256 5.22 / 5.35 ms, from 200 of 256
     // 5.61 / 5.61; 576 wide, 30 layers, fp16 and 32-bit caches from 16 of 512 24.1 / 24.6, from 440 of 512 30.1 / 27.8 (sixteen: 28.9).
-    if (a.max_seq <= 256) hipLaunchKernelGGL((attention_project_kernel<KV_F16, FMT, 4, 2>), grid, dim3(256), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, wo.qs, heads, (unsigned)wo.qs_row_bytes, p);
-    else hipLaunchKernelGGL((attention_project_kernel<KV_F16, FMT, 8, 2>), grid, dim3(512), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, wo.qs, heads, (unsigned)wo.qs_row_bytes, p);
+    // Blocks of 128 rows of wo where those of 64 are more workgroups than compute units: each of them reads its head's keys and values, which bounds long prefixes.  Two rows of 768 wide, 6 layers, 64 tokens
+    // from position 16 / 200 / 440 of 512, attention and wo in launches of their own / blocks of 64 / of 128, ms: fp16 9.6 / 9.9 / 10.4, 8.9 / 9.6 / 10.7, 8.7 / 9.3 / 10.0; Q4_0 11.1 / 11.4 / 12.0,
+    // 10.8 / 11.6 / 12.7, 10.4 / 11.0 / 11.8.  576 wide (162 workgroups), 32 tokens from 16 / 430, fp16: 23.3 / 24.7, 20.7 / 23.3, 21.1 / 23.7.
+    const int cus = device_compute_units() > 0 ? device_compute_units() : 256;
+    if (a.max_seq <= 256) go(Four{}, Narrow{});
+    else if (rows * a.n_head * ((wo.rows + 63) / 64) <= cus) go(Eight{}, Narrow{});
+    else go(Eight{}, Wide{});
 }
 
 hipError_t launch_attention_project(const AttentionArgs &a, const DeviceMatrix &wo, int rows, const float *residual, float *planes, bool kv_f16, hipStream_t s) {

@@ -72,3 +72,27 @@ def test_two_rows_add_planes_on_the_matrix_cores(ll, fmt, n_head, hidden):
     for i in range(4):   # other orders of fp32 sums; activations are rounded to fp16 in between
         limit = 2.0 ** -9 * max(1.0, np.abs(want[2 * i + 1]).max())
         assert np.abs(got[-1][i] - got[0][i]).max() <= limit and np.abs(got[-1][i] - want[2 * i + 1]).max() <= limit, i
+
+
+@pytest.mark.parametrize("fmt,d_model,kv", [("f16", 704, "f32"), ("q8_0", 704, "f16"), ("q4_0", 768, "f32"), ("f16", 768, "f16")])
+def test_two_rows_of_many_heads_behind_long_prefixes(ll, fmt, d_model, kv):
+    """Contexts of more than 256 tokens and 12 heads: blocks of 128 rows of wo for two rows (704: the last one is half), of 64 for one."""
+    import espresso_amd.ops as ops
+    import espresso_amd.synthetic as syn
+    cfg = ll.MultiModelConfig(n_layer=2, n_head=12, n_kv_head=4, d_model=d_model, head_dim=64, hidden_dim=512, vocab=512, max_seq=300)
+    g, _ = syn.build_runtime(cfg, lib.FORMAT_NAMES[fmt], seed=d_model, std=0.05, kv_format=lib.FORMAT_F16 if kv == "f16" else lib.FORMAT_F32)
+    tokens = np.random.default_rng(d_model).integers(0, cfg.vocab, 280).astype(np.uint32)
+    try:
+        ops.set_tuning("short_blocks", 0)
+        for first in (2, 127, 271):
+            g.reset()
+            g.prefill(tokens[:first])
+            got = np.concatenate([g.append(tokens[i:i + 2], want=(0, 1)) for i in range(first, first + 8, 2)])
+            g.set_visible(first)
+            for i in range(8):
+                g.advance(int(tokens[first + i]))
+                want = g.logits()   # other orders of fp32 sums; activations are rounded to fp16 in between
+                assert np.abs(got[i] - want).max() <= 2.0 ** -9 * max(1.0, np.abs(want).max()), (first, i)
+    finally:
+        ops.set_tuning("short_blocks", 1)
+    g.close()
