@@ -607,18 +607,17 @@ int LlamaRuntime::prefill_shared_block(const PromptSpan *spans, int count) {
     return rc;
 }
 
-// Attention of a block: one prompt's rows (block_keys: the keys that the last of them sees), prompts that share it, or (neither) rows that attend alone.  Fewer than 32 rows of a prompt, and all rows of
-// models with fp16 caches, take 32-bit attention, as the steps they stand for.
+// Attention of a block: one prompt's rows (block_keys: the keys that the last of them sees), prompts that share it, or (neither) rows that attend alone.  Fewer than 32 rows of a prompt take 32-bit
+// attention, as the steps they stand for, and so do all rows of models with fp16 caches (behind more than 2048 keys as far as their fp16 contexts show it: launch_span_attention).
 int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_keys, int last) {
     hipStream_t s = context().stream;
     const bool kv16 = c_.kv_format == FMT_F16;
-    if (last > 0 && last < kMatrixPrefillMinTokens && finer_short_attention() && !kv16) {   // (fp16 caches: 32-bit attention for every row)
+    if (last > 0 && last < kMatrixPrefillMinTokens && finer_short_attention() && !kv16) {
         const int ahead = rows - last;
         const size_t at = (size_t)ahead * c_.attention_dim();
         ESP_HIP_TRY(launch_prompt_attention(aa, ahead, block_keys - last, kv16, s));
         aa.q += at; aa.pos += ahead; aa.seq += ahead;
-        if (aa.ctx_f16) aa.ctx_f16 += at;
-        if (aa.ctx_hi) { aa.ctx_hi += at; aa.ctx_lo += at; aa.ctx_sums += at / 16; }
+        aa.ctx_f16 += at;   // (split rows of so many belong to fp16 caches)
         ESP_HIP_TRY(launch_span_attention(aa, last, block_keys, kv16, s));
         return ESP_OK;
     }
@@ -640,9 +639,8 @@ int LlamaRuntime::enqueue_block_attention(AttentionArgs aa, int rows, int block_
 // The layer loop over `rows` rows whose embeddings sit in hidden_ and whose (position, sequence) sit in
 // d_pos_/d_seq_, every projection as one dequant-fused MFMA GEMM.  Rows that are one sequence at consecutive positions
 // (a prompt block) take a matrix-core attention kernel, others the single-query one.
-// Prompt blocks of Q4_K models: every projection with exact weights and split activations (launch_gemm_split), queries and softmax
-// weights as pairs (in short blocks, which single-row steps could walk as well, 32-bit) in the attention: the block then stays as close to the fp32 CPU walk as
-// the decode steps do.
+// Prompt blocks of Q4_K models: every projection with exact weights and split activations (launch_gemm_split), 32-bit attention: the block then stays as close to the fp32 CPU walk as the decode
+// steps do.
 bool LlamaRuntime::split_blocks_supported() const {
     return prompt_attention_ && c_.kv_format == FMT_F16 && splits_every_product();
 }
