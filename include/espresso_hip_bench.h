@@ -75,7 +75,8 @@ int esp_layer_gate_up(const ESPMatrix *matrix, const uint16_t *x_f16, int rows, 
  * as fp32: the fp16 context, or with split_rows the two fp16 planes added back together (hi + lo / 2048).  Host pointers.  `iters` launches;
  * *mean_us (may be NULL) is their mean time.  ESP_ERR_UNSUPPORTED for a shape the kernel is not written for. */
 #define ESP_ATTENTION_SINGLE_ROW 0   /* every row by itself */
-#define ESP_ATTENTION_PROMPT 1       /* prompt blocks, one, two or four query heads per key/value head */
+#define ESP_ATTENTION_PROMPT 1       /* prompt blocks, one, two or four query heads per key/value head; with fp16 caches the next one, which may then take
+                                        pairs of fp16 parts behind long prefixes */
 #define ESP_ATTENTION_SPAN 2         /* blocks of any head group */
 #define ESP_ATTENTION_STEP 3         /* up to 32 rows as a step of several sequences has them, the context as long as it is */
 int esp_block_attention(int kernel, const float *q, const void *k, const void *v, int kv_f16, int rows, int first, int heads, int kv_heads, int head_dim,

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("fmt,heads,kv_heads,kv_fp16,count", [
     (orc.FMT_Q8_0, 4, 2, True, 2049),    # a block of 2048 rows and one row in a block of its own
     (orc.FMT_Q8_0, 3, 1, False, 1999), (orc.FMT_Q4_0, 3, 1, True, 2304), (orc.FMT_F16, 4, 4, True, 1025),
-    (orc.FMT_Q4_K, 4, 1, True, 2111),    # exact products, queries and softmax weights as pairs
+    (orc.FMT_Q4_K, 4, 1, True, 2111),    # exact products of split rows
     (orc.FMT_Q4_K, 4, 2, False, 1537),
 ])
 def test_long_blocks_match_portions_and_steps(fmt, heads, kv_heads, kv_fp16, count):
@@ -103,7 +103,7 @@ def test_last_rows_are_as_exact_as_in_a_block_of_their_own(shape, fmt, kv, count
     got = rt.append(prompt, want=range(count - last, count))
     hidden = rt.last_hidden()
     # the same roundings, sums in another order: a last bit of an fp16 activation falls either way, up to 5.3e-4 of the logits' size; in a long block like its other rows they are 1.0 to 1.7e-3 off
-    # (products and attention of pairs of fp16: 0, and 2.3e-5)
+    # (512 wide: products of split rows, attention in 32 bits)
     assert rms_off(got, want) <= (2.0 ** -18 if shape["d_model"] == 512 else 3 * 2.0 ** -12)
     rt.reset()
     ll.generate_batch(rt, [prompt, prompt[:count - 3]], 1)
