@@ -511,8 +511,8 @@ typedef _Float16 attn_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 attn_half4 __attribute__((ext_vector_type(4)));
 typedef float attn_floatx16 __attribute__((ext_vector_type(16)));
 
-// Heads of 64 dims ask for two wavefronts per SIMD: without it the compiler spreads over accumulator registers past what two share (512 rows of 32
-// heads behind 512, split rows: 49 us, 44 with it).
+// Heads of 64 dims ask for two wavefronts per SIMD: without it the compiler spreads over accumulator registers past what two share.  512 rows behind 1536, without / with it, us: 12 heads of one query head
+// per key/value head 64.6 / 57.3, 16 of two 66.5 / 60.7, 32 of four 94.9 / 108.4 (100 rows behind 100: 10.1 / 9.4, 11.0 / 10.3, 14.8 / 15.5; 64 rows 5.4 / 5.3, 6.2 / 6.0, 8.2 / 7.9).
 template <int HD, int G>
 __global__ __launch_bounds__(G * 64, HD == 64 ? 2 : 1) void attention_prompt_kernel(AttentionArgs a, int rows) {
     constexpr int THREADS = G * 64, QT = 32, KS = HD / 16, MTILES = HD / 32, LDV = 32 + 8;   // LDV: fp16 per row of V^T
@@ -1560,8 +1560,11 @@ void launch_attention_partial_shape(const AttentionArgs &a, dim3 grid, bool kv_f
     else hipLaunchKernelGGL((attention_partial_kernel<HD, false, WAVES, U>), grid, dim3(WAVES * 64), 0, s, a.q, a.k_cache, a.v_cache, a.pos, a.seq, a.head_partials, (unsigned)a.cache_seq_stride, heads);
 }
 
-// Small models and short contexts.  Every block of rows repeats the head's attention, so its cost grows with wo.rows and the context: 12 heads of 768 rows and up to 512 positions were faster at every position
-// (below), 16 heads of 1024 rows faster from position 16 of 512 (12 layers of Q8_0, 48 tokens: 11.8 ms -> 11.4) and slower from 440 (12.5 -> 12.9, fp16 15.0 -> 15.9).
+// Small models and short contexts.  Every block of rows repeats the head's attention, so its cost grows with wo.rows and the context.  48 tokens from position 16 / 200 / 440 / 900 of 1024, in launches of their
+// own -> in this one, ms: 768 wide, 6 layers, Q8_0 and 32-bit caches 5.89 / 5.91 / 5.95 / 6.32 -> 5.24 / 5.47 / 5.94 / 6.72, fp16 and fp16 caches 5.89 / 5.97 / 5.95 / 6.24 -> 5.32 / 5.57 / 5.90 / 6.55;
+// 576 wide, 30 layers, fp16 and 32-bit caches 28.2 / 28.4 / 28.5 / 30.8 -> 24.4 / 25.6 / 28.0 / 32.6, Q8_0 and fp16 caches 26.2 / 26.3 / 26.3 / 27.5 -> 22.8 / 23.8 / 25.6 / 28.7.  They meet at 440 to 500 keys,
+// and a step is captured for its context's every position, so contexts end at 512.  16 heads of 1024 rows meet earlier: from position 16 of 512 (12 layers of Q8_0, 48 tokens) 11.8 -> 11.4, from 440 12.5 ->
+// 12.9 (fp16 15.0 -> 15.9).
 bool attention_project_supported(const DeviceMatrix &wo, int n_head, int n_kv_head, int head_dim, int max_seq) {
     return head_dim == 64 && n_kv_head > 0 && n_head % n_kv_head == 0 && n_head <= kMaxNormPlanes && wo.cols == n_head * 64 && wo.rows <= 768 && wo.rows % 8 == 0 && max_seq <= 512 &&
            wo.qs && wo.qs_row_bytes % 16 == 0 && wo.qs_row_bytes <= 0xFFFFFFFFull && (wo.format == FMT_F16 || ((wo.format == FMT_Q8_0 || wo.format == FMT_Q4_0) && wo.scales));
