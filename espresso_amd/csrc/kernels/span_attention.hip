@@ -183,12 +183,19 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             if (lane % QL == 0) row_scale[r] = __builtin_amdgcn_ldexpf(__fmul_rn(1.0f / sqrtf((float)HD), 1.44269504f), -q_exp);
         }
     } else {
+        // the wavefronts share the dims, 16 in turn; all of a wavefront's loads are on their way before the first store waits (33 rows of 24 heads of 128 dims, two wavefronts: 12.1 us, 11.9 so)
         const float *query = queries + (size_t)(col <= last_row ? col : last_row) * q_pitch;
+        constexpr int QS = (KS + KP - 1) / KP;
+        float4 x[QS][2];
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++)
-            if (ks % KP == phase)
+        for (int i = 0; i < QS; i++)
 #pragma unroll
-                for (int w = 0; w < 2; w++) *reinterpret_cast<float4 *>(q32 + col * LDQ + 16 * ks + 8 * half + 4 * w) = *reinterpret_cast<const float4 *>(query + 16 * ks + 8 * half + 4 * w);
+            for (int w = 0; w < 2; w++) x[i][w] = *reinterpret_cast<const float4 *>(query + 16 * (KS % KP == 0 || phase < KS ? i * KP + phase : 0) + 8 * half + 4 * w);
+        if (KS % KP == 0 || phase < KS)
+#pragma unroll
+            for (int i = 0; i < QS; i++)
+#pragma unroll
+                for (int w = 0; w < 2; w++) *reinterpret_cast<float4 *>(q32 + col * LDQ + 16 * (i * KP + phase) + 8 * half + 4 * w) = x[i][w];
     }
     if (threadIdx.x == 0) not_finite = 0;
     __syncthreads();
