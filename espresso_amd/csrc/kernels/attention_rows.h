@@ -39,7 +39,7 @@ __device__ __forceinline__ void store_context_sum(const AttentionArgs &a, size_t
 // split operand may be zero, or overflow, where the operand does not.  Rare, so nothing here is fast.
 template <int HD, bool KV_F16>
 __device__ void plain_attention_row(const AttentionArgs &a, int row, int head) {
-    const int lane = threadIdx.x & 63, kvh = head / (a.n_head / a.n_kv_head), kd = a.n_kv_head * HD;
+    const int lane = __lane_id(), kvh = head / (a.n_head / a.n_kv_head), kd = a.n_kv_head * HD;
     const size_t base = (size_t)a.seq[row] * a.cache_seq_stride + (size_t)kvh * HD;
     const float *q = a.q + (size_t)row * a.n_head * HD + (size_t)head * HD;
     const float scale = 1.0f / sqrtf((float)HD);

@@ -20,10 +20,11 @@
 //     of exponents of differences, this kernel's forerunner: 2.3 / 5.3 / 9.3 / 17.4e-7 and 2.1 / 4.6 / 7.8 / 15.3e-7.  A correction term of the exponential changes less than 2 % of it.
 // A row whose result is not finite is done again from the keys it sees alone (plain_attention_row).
 // What bounds it (fp16 caches, 128 dims, a tile): 48 products, 0.78 us of a SIMD at the 2 GHz that the chip holds with all of them at work, beside 200 vector instructions: 1.5 us with two wavefronts a
-// SIMD; and a workgroup's way in and out, 9 us of 30 at 1777 rows.  Transposed two-byte writes of values, exponentials with a correction term, parts by rounding conversions, every wavefront reading every
-// query for its exponent and states handed on pairwise took: 1777 rows of 24 heads (8 key/value heads) 100 -> 79 us, 512 rows 21.6 -> 15.6, 93 rows of 32 heads of 64 behind 700 15.0 -> 10.4.  Against
-// attention_prompt_kernel with fp16 operands (and with pairs of them, inside a model), 32 heads, 8 key/value heads: 128 dims, 64 / 512 / 1500 rows 10.2 / 20.4 (38) / 93 (182) -> 8.3 / 17.3 / 75, 512 behind
-// 3000 95 -> 92 with two parts; 64 dims, 128 / 1100 rows 7.8 / 35.5 -> 6.5 / 27.2: that kernel has 32-bit caches alone.  512 rows of 24 heads of 128 behind 1024 from fp32 caches: 137 us.
+// SIMD; and a workgroup's way in and out.  Transposed two-byte writes of values, exponentials with a correction term, parts by rounding conversions, every wavefront reading every
+// query for its exponent and states handed on pairwise took: 512 rows of 24 heads (8 key/value heads) 21.6 -> 15.4 us, 93 rows of 32 heads of 64 behind 700 15.0 -> 9.4.  Against
+// attention_prompt_kernel with fp16 operands (and with pairs of them, inside a model), 32 heads, 8 key/value heads: 128 dims, 64 / 512 rows 10.4 / 20.8 (38) -> 6.9 / 16.7, 512 behind
+// 3000 95 -> 92 with two parts; 64 dims, 128 rows 8.0 -> 5.4; slower alone for few heads that share nothing and few rows (33 rows of 12 heads of 64 4.0 -> 4.7): that kernel has 32-bit caches alone.
+// 512 rows of 24 heads of 128 behind 1024 from fp32 caches: 136 us.
 // Query heads of a key/value head are x, x + kv_heads, ...: with eight key/value heads they share one L2.
 #include "../common.h"
 #include "attention_rows.h"
@@ -97,6 +98,13 @@ __device__ __forceinline__ float exp_weight(float x) {
     return __builtin_fmaf(e, __fmul_rn(left, 0.693147181f), e);
 }
 
+// The lane, found again where it is used: three registers more through the loop over the keys are a spill.
+__device__ __forceinline__ int lane_again() {
+    uint32_t zero = 0;
+    asm volatile("" : "+v"(zero));
+    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 // Two wavefronts per SIMD where the registers (without copies to accumulator registers) and the LDS of one wavefront allow it: a tile of an fp16 cache is more vector work
 // than matrix work, and one wavefront's hides under the other's.
 constexpr int span_waves_per_simd(int hd, bool kv_f16, int kp) { return hd == 64 || (kv_f16 && kp > 1) ? 2 : 1; }
@@ -108,12 +116,13 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     constexpr int LDQ = KV_F16 ? HD + 8 : HD + 4;                           // elements between the queries' rows
     constexpr int kQueryBytes = KV_F16 ? PARTS * 32 * LDQ * 2 : 32 * LDQ * 4;
     constexpr int kWave = KV_F16 ? 32 * LDV * 2 : 0;                        // a value tile per wavefront
-    constexpr int OWN = MT * 16 / KP, kMergeBytes = KP > 1 ? KP * (KP - 1) * OWN * 64 * 4 : 16;   // accumulators that a wavefront finishes
+    constexpr int OWN = MT * 16 / KP, kMergeBytes = KP > 1 ? KP * KP * OWN * 64 * 4 : 16;   // accumulators that a wavefront finishes
     __shared__ __attribute__((aligned(16))) unsigned char smem[kQueryBytes + KP * kWave > kMergeBytes ? kQueryBytes + KP * kWave : kMergeBytes];
     unsigned char *const query_mem = smem;
     __shared__ int not_finite;
     __shared__ float state[KP][2][64], row_scale[32];
-    const int lane = threadIdx.x & 63, phase = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = lane >> 5, col = lane & 31;
+    const int phase = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
     const int group = a.n_head / a.n_kv_head, kvh = blockIdx.x % a.n_kv_head, head = kvh * group + blockIdx.x / a.n_kv_head;
     const int y = (int)(gridDim.y - 1 - blockIdx.y);                           // the row tiles with the most keys start first
     asm volatile("" ::"s"(a.tiles), "s"(a.pos), "s"(a.seq), "s"(a.q), "s"(a.k_cache), "s"(a.v_cache));   // fetched together, ahead of the branch
@@ -251,8 +260,9 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             // Accumulator r: key t0 + 8 (r / 4) + 4 half + r % 4 against query `col`.  Scores stay as they are summed: a weight is 2^((s - m) c) with c = scale log2(e), a subtraction, a product and
             // the hardware's 2^t.
             if (t0 + 31 > pos0) {
+                const int first = t0 + 4 * (lane_again() >> 5);
 #pragma unroll
-                for (int r = 0; r < 16; r++) s[r] = t0 + 8 * (r >> 2) + 4 * half + (r & 3) <= qpos ? s[r] : -INFINITY;
+                for (int r = 0; r < 16; r++) s[r] = first + 8 * (r >> 2) + (r & 3) <= qpos ? s[r] : -INFINITY;
             }
             float tile_max = s[0];
 #pragma unroll
@@ -355,7 +365,8 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             }
         }
     }
-    // The wavefronts' states meet: each leaves the others' accumulators in LDS and finishes OWN of its own, with factors that take every state to the largest maximum, sums in pairs.
+    if constexpr (KV_F16) { lane = lane_again(); half = lane >> 5; col = lane & 31; }
+    // The wavefronts' states meet: each leaves its accumulators in LDS and finishes OWN of everybody's, with factors that take every state to the largest maximum, sums in pairs.
     l += __shfl_xor(l, 32);
     float mine[OWN];
     if constexpr (KP > 1) {
@@ -379,20 +390,17 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
             return part[0];
         };
         l = total();
-        float *merge = reinterpret_cast<float *>(smem);   // [from][to, but for itself][OWN][64]
+        float *merge = reinterpret_cast<float *>(smem);   // [from][to][OWN][64], a wavefront's own share too: kept apart it was a branch for each accumulator, and a wait for each load (33 rows of
+                                                            // 24 heads of 128 7.9 us, 6.4 so; from fp32 caches, two wavefronts, 11.9 and 9.8)
 #pragma unroll
         for (int w = 0; w < KP; w++)
 #pragma unroll
-            for (int r = 0; r < OWN; r++) {
-                const float v = o[(w * OWN + r) >> 4][(w * OWN + r) & 15];
-                if (w == phase) mine[r] = v;
-                else merge[((phase * (KP - 1) + w - (w > phase)) * OWN + r) * 64 + lane] = v;
-            }
+            for (int r = 0; r < OWN; r++) merge[((phase * KP + w) * OWN + r) * 64 + lane] = o[(w * OWN + r) >> 4][(w * OWN + r) & 15];
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < OWN; r++) {
 #pragma unroll
-            for (int w = 0; w < KP; w++) part[w] = w == phase ? mine[r] : merge[((w * (KP - 1) + phase - (phase > w)) * OWN + r) * 64 + lane];
+            for (int w = 0; w < KP; w++) part[w] = merge[((w * KP + phase) * OWN + r) * 64 + lane];
             mine[r] = total();
         }
     } else {
@@ -402,9 +410,13 @@ __global__ __launch_bounds__(KP * 64, span_waves_per_simd(HD, KV_F16, KP)) void 
     float check = 0.0f;
 #pragma unroll
     for (int r = 0; r < OWN; r++) check = __builtin_fmaf(mine[r], 0.0f, check);
-    if (__any(!(check == 0.0f && l < INFINITY)) && lane == 0) not_finite = 1;   // NaN wherever an infinity or a NaN went in
-    __syncthreads();
-    if (!not_finite) {
+    bool finite = !__any(!(check == 0.0f && l < INFINITY));   // NaN wherever an infinity or a NaN went in
+    if constexpr (KP > 1) {
+        if (!finite && lane == 0) not_finite = 1;
+        __syncthreads();
+        finite = !not_finite;
+    }
+    if (finite) {
         const float inv = 1.0f / (KV_F16 ? __fmul_rn(l, 32768.0f) : l);   // key 0 is visible to every query: l > 0
         const size_t row = (size_t)(m0 + (col <= last_row ? col : last_row));
         float sums[OWN < 16 ? 1 : OWN / 16];   // of 32 dims each, or of this wavefront's share of them
@@ -473,9 +485,9 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     if (rows <= 0 || (a.tiles && a.tile_count <= 0) || !span_attention_supported(a.n_head, a.n_kv_head, a.head_dim)) return hipErrorInvalidValue;
     if (a.ctx_hi ? !a.ctx_lo || !a.ctx_sums || (a.n_head * a.head_dim) % 256 != 0 : !a.ctx_f16) return hipErrorInvalidValue;
     // Wavefronts per workgroup, fp32 caches: as many as it takes to give every SIMD one (256 compute units x 4), each with a tile of keys at least.
-    // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit, or eight where a workgroup has the compute unit to itself and keys for all of them.  Two wavefronts / four /
-    // eight, us: 1777 rows of 24 heads of 128 79 / 80 / 104, 512 rows 18.8 / 15.6 / 21.2, 64 rows 8.5 / 8.4 / 9.1, 93 rows behind 1000 31 / 21.9 / 20.5, 31 rows behind 4000 (32 heads) 87 / 51 / 49.5;
-    // heads of 64: 1100 rows of 32 heads 28.2 / 27.2 / 41, 128 rows 6.5 / 6.3 / 6.7, 93 rows behind 700 15.2 / 11.1 / 10.4, behind 1500 25 / 16.7 / 14.9, 512 rows behind 1024 33 / 23.8 / 28.
+    // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit, or eight where a workgroup has the compute unit to itself and keys for all of them.  Four / eight, us:
+    // 512 rows of 24 heads of 128 15.3 / 18.6, 64 rows 6.8 / 7.0, 93 rows behind 500 / 800 / 1000 14.9 / 13.3, 17.9 / 15.7, 20.8 / 17.8, 31 rows behind 300 / 500 / 4000 (32 heads) 10.9 / 10.5, 14.3 / 12.9, 52 / 45;
+    // heads of 64: 512 rows of 32 heads 9.7 / 13.0, 128 rows 5.3 / 5.6, 93 rows behind 300 / 500 / 700 / 1500 8.0 / 7.7, 9.0 / 8.2, 10.7 / 9.4, 16.4 / 13.3, 512 rows behind 1024 23.9 / 26.6.  Under 24 tiles of keys the sums of four stay, as they were when eight were no faster there.
     const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32), cus = device_compute_units() > 0 ? device_compute_units() : 256;
     int sets = 1;
     if (!kv_f16) {
@@ -485,8 +497,8 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
         sets = forced ? 4 * forced : tiles >= 24 && groups <= cus ? 8 : 4;
     }
     // Long walks over the keys are bound by the products (48 of a tile of 128 dims with three parts, 32 with two), and a context that is rounded to fp16 shows neither.  512 rows of 32 heads (8 key/value heads)
-    // behind 1500 / 2000 / 3000 / 6000 / 15000, fp16 operands / three parts / two, us: 58 / 57 / 54, 71 / 70 / 66, 95 / 99 / 92, 168 / 182 / 169, 382 / 409 / 379.  Up to 2048 keys three parts are no slower
-    // than fp16 operands were; nor are they where the workgroups are eight wavefronts (93 rows behind 3000 77 / 41) or heads are 64 dims (512 behind 8000 220 / 127).
+    // behind 1500 / 2000 / 3000 / 6000 / 15000, fp16 operands / three parts / two, us: 58 / 56 / 54, 71 / 73 / 67, 95 / 100 / 92, 168 / 180 / 164, 382 / 402 / 367.  Up to 2048 keys three parts are no slower
+    // than fp16 operands were; nor are they where the workgroups are eight wavefronts (93 rows behind 3000 77 / 37) or heads are 64 dims (512 behind 8000 220 / 127).
     const bool pairs = pairs_do && kv_f16 && a.head_dim == 128 && !a.ctx_hi && sets == 4 && keys > 2048;
     if (a.head_dim == 128) {
         if (kv_f16) launch_shape<128, true>(a, rows, sets, pairs, s);
