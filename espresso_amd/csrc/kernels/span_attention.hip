@@ -488,6 +488,7 @@ hipError_t launch_span_attention(const AttentionArgs &a, int rows, int keys, boo
     // fp16 caches: four, whose value tiles leave room for a second workgroup on the compute unit, or eight where a workgroup has the compute unit to itself and keys for all of them.  Four / eight, us:
     // 512 rows of 24 heads of 128 15.3 / 18.6, 64 rows 6.8 / 7.0, 93 rows behind 500 / 800 / 1000 14.9 / 13.3, 17.9 / 15.7, 20.8 / 17.8, 31 rows behind 300 / 500 / 4000 (32 heads) 10.9 / 10.5, 14.3 / 12.9, 52 / 45;
     // heads of 64: 512 rows of 32 heads 9.7 / 13.0, 128 rows 5.3 / 5.6, 93 rows behind 300 / 500 / 700 / 1500 8.0 / 7.7, 9.0 / 8.2, 10.7 / 9.4, 16.4 / 13.3, 512 rows behind 1024 23.9 / 26.6.  Under 24 tiles of keys the sums of four stay, as they were when eight were no faster there.
+    // One or two where there are no more tiles of keys than that: the same bits, and slower, since the queries are split by all wavefronts (16 rows 4.5 -> 4.9, of 24 heads of 128 6.1 -> 7.8; 64 rows 6.8 -> 7.1).
     const int tiles = (keys + 31) / 32, groups = a.n_head * (a.tiles ? a.tile_count : (rows + 31) / 32), cus = device_compute_units() > 0 ? device_compute_units() : 256;
     int sets = 1;
     if (!kv_f16) {
